@@ -57,7 +57,8 @@ struct moe_ctx {
   int* ids = nullptr;         // [T][id_stride]
   float* ws = nullptr;        // [T][id_stride]
   float* sh_logit = nullptr;  // [T]
-  float* rtol = nullptr;      // [min(T, small_max)]: per token, how far the small-batch router's logits can lie from the reference's
+  float* rtol = nullptr;      // [min(T, MOE_ROUTER_SPLIT_MAX)]: per token, how far the parallel routers' logits can lie from the reference's
+  double* gpart = nullptr;    // fp64 partial logits of the column-split router (33 .. MOE_ROUTER_SPLIT_MAX tokens)
   unsigned* ticket = nullptr; // block counter of the fused small-batch router launch (rests at 0)
   double* kpart = nullptr;    // partial tiles and per-row-group tickets (resting at 0) of the column-split router launch
   unsigned* ktickets = nullptr;
@@ -185,7 +186,7 @@ MOE_API int moe_destroy(moe_ctx* c) {
   if (c->side) (void)hipStreamDestroy(c->side);
   void* bufs[] = {c->logits, c->ids, c->ws, c->sh_logit, c->ticket, c->kpart, c->ktickets, c->xms, c->sample, c->hid32, c->xplanes, c->hplanes, c->xmeta, c->hmeta, c->x16, c->tokidx, c->pw, c->eoff,
                   c->pairids, c->tiles, c->ntiles, c->tiles_sh, c->ntiles_sh, c->hid16, c->pairs16, c->pairs32, c->rc_scratch,
-                  c->v2_zraw, c->v2_xplanes, c->v2_xmeta, c->v2_acc, c->v2_ey, c->v2_x16, c->v2_z16, c->pexp, c->span_tmp, c->rtol};
+                  c->v2_zraw, c->v2_xplanes, c->v2_xmeta, c->v2_acc, c->v2_ey, c->v2_x16, c->v2_z16, c->pexp, c->span_tmp, c->rtol, c->gpart};
   for (void* b : bufs)
     if (b) {
       hipError_t e = hipFree(b);
@@ -219,7 +220,7 @@ MOE_API int moe_create(const moe_config* cfg, moe_ctx** out) {
   if (e == hipSuccess) e = hipMalloc(&c->ws, T * S * 4);
   if (e == hipSuccess) e = hipMemset(c->ws, 0, T * S * 4);
   if (e == hipSuccess) e = hipMalloc(&c->sh_logit, T * 4);
-  if (e == hipSuccess) e = hipMalloc(&c->rtol, (T < (size_t)c->small_max ? T : (size_t)c->small_max) * 4);
+  if (e == hipSuccess) e = hipMalloc(&c->rtol, (T < (size_t)MOE_ROUTER_SPLIT_MAX ? T : (size_t)MOE_ROUTER_SPLIT_MAX) * 4);
   if (e == hipSuccess) e = hipMalloc(&c->ticket, 256);
   if (e == hipSuccess) e = hipMemset(c->ticket, 0, 256);
   if (e == hipSuccess) e = hipMalloc(&c->kpart, MOE_ROUTER_KPART_BYTES);
@@ -263,6 +264,7 @@ MOE_API int moe_create(const moe_config* cfg, moe_ctx** out) {
   if (e == hipSuccess && T > (size_t)c->small_max) {
     const size_t d = cfg->d, mid = cfg->mid;
     e = hipMalloc(&c->rc_scratch, moe_router_cand_scratch_bytes(cfg->max_tokens, cfg->experts, cfg->d));
+    if (e == hipSuccess) e = hipMalloc(&c->gpart, moe_router_split_scratch_bytes(cfg->max_tokens, cfg->experts, cfg->d));
     if (e == hipSuccess) e = hipMalloc(&c->x16, T * d * 2);
     const size_t pe_bytes = (size_t)cfg->layers * (2 * E + 2);
     if (e == hipSuccess) e = hipMalloc(&c->pexp, pe_bytes);
@@ -755,12 +757,8 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
       const int sh_first = sh ? P * g.topk : -1;
       const int max_tiles = P * g.topk + (sh ? (P + 3) / 4 : 0);  // tiles of <= 4 pairs
       if ((rc = stage(MOE_PROF_ROUTE, [&]() -> int {
-             if (moe_route_small_supported(P, g.topk, g.experts))  // permutation and tiles in one launch
-               return moe_launch_route_small(c->ids, c->ws, c->tokidx, c->pw, c->eoff, c->pairids, P, g.topk,
-                                             g.experts, g.id_stride, c->tiles, c->ntiles, 4, sh_first, st);
-             const int e = moe_routing_run(c->routing, c->ids, c->ws, c->tokidx, c->pw, c->eoff, c->pairids, P,
-                                           g.topk, g.experts, g.id_stride, st);
-             return e ? e : moe_launch_tiles_shared(c->eoff, c->tiles, c->ntiles, g.experts, 4, P, sh_first, c->tokidx, st);
+             return moe_launch_route(moe_routing_blockcnt(c->routing), c->ids, c->ws, c->tokidx, c->pw, c->eoff, c->pairids, P, g.topk, g.experts, g.id_stride,
+                                     c->tiles, c->ntiles, 4, sh_first, st);
            })))
         return rc;
       if ((rc = stage(MOE_PROF_UP, [&]() -> int {
@@ -831,12 +829,8 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
     const int sh_first = sh ? P * g.topk : -1;
     const int max_tiles = P * g.topk + (sh ? (P + cap - 1) / cap : 0);
     if ((rc = stage(MOE_PROF_ROUTE, [&]() -> int {
-           if (moe_route_small_supported(P, g.topk, g.experts))
-             return moe_launch_route_small(c->ids, c->ws, c->tokidx, c->pw, c->eoff, c->pairids, P, g.topk, g.experts,
-                                           g.id_stride, c->tiles, c->ntiles, cap, sh_first, st);
-           const int e = moe_routing_run(c->routing, c->ids, c->ws, c->tokidx, c->pw, c->eoff, c->pairids, P, g.topk,
-                                         g.experts, g.id_stride, st);
-           return e ? e : moe_launch_tiles_shared(c->eoff, c->tiles, c->ntiles, g.experts, cap, P, sh_first, c->tokidx, st);
+           return moe_launch_route(moe_routing_blockcnt(c->routing), c->ids, c->ws, c->tokidx, c->pw, c->eoff, c->pairids, P, g.topk, g.experts, g.id_stride,
+                                   c->tiles, c->ntiles, cap, sh_first, st);
          })))
       return rc;
     if ((rc = stage(MOE_PROF_UP, [&]() -> int {
@@ -1001,16 +995,15 @@ static int batch_x16_layout(const MoeLayer& L, const moe_config& g) {
   return gg_kinds(L, g).any_tuned() ? 2 : 0;
 }
 
-// Router of a batch: ids / ws, the shared-expert gate logit and (if asked) the per-token mean square of x.
-// By default through candidate selection (router_cand.hip); MOE_OPT_ROUTER_CANDIDATES = 0, or a shape it does not
-// take, runs the dense fp64 launch and the exact softmax / top-k over all experts.
-static int router_batch(moe_ctx* c, MoeLayer& L, const float* x, int P, float* out_xms, hipStream_t st) {
+// Router of a batch above MOE_ROUTER_SPLIT_MAX tokens: ids / ws.  By default through candidate selection
+// (router_cand.hip); MOE_OPT_ROUTER_CANDIDATES = 0, or a shape it does not take, runs the dense fp64 launch and the exact
+// softmax / top-k over all experts.
+static int router_batch(moe_ctx* c, MoeLayer& L, const float* x, int P, hipStream_t st) {
   const moe_config& g = c->cfg;
-  const moe_wview* wx = L.has_shared ? &L.sh_sg : nullptr;
-  if (c->router_cand && c->rc_scratch && moe_router_cand_supported(&L.router, wx, P, g.topk))
-    return moe_router_batch_cand(&L.router, L.router_bias, wx, x, P, c->logits, c->sh_logit, out_xms, c->ids, c->ws,
-                                 g.topk, g.id_stride, c->rc_scratch, st, L.router_bmax);
-  int rc = moe_router_logits_seq(&L.router, L.router_bias, wx, x, P, c->logits, c->sh_logit, out_xms, st);
+  if (c->router_cand && c->rc_scratch && moe_router_cand_supported(&L.router, P, g.topk))
+    return moe_router_batch_cand(&L.router, L.router_bias, x, P, c->logits, c->ids, c->ws, g.topk, g.id_stride, c->rc_scratch,
+                                 st, L.router_bmax);
+  int rc = moe_router_logits_seq(&L.router, L.router_bias, x, P, c->logits, st);
   if (!rc) rc = moe_router_topk(c->logits, c->ids, c->ws, P, g.experts, g.topk, g.id_stride, st);
   return rc;
 }
@@ -1157,7 +1150,12 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
                                 0, false, nat, pe_dn, pe_sdn);
   };
   const bool fused = c->fused_combine && !c->hc && !(q4k && !kd.r_dn) && !split && !v2;  // the HC write-back belongs to the ordered combine
-  const bool aside = v2 || (L.has_shared && (split || (c->shared_aside && !fused)));
+  // middle sizes: the router's column-split launches (router_split.hip); its first launch makes the f16 copy of x as well
+  const bool mid_router = c->router_cand && c->gpart && moe_router_split_supported(&L.router, L.has_shared ? &L.sh_sg : nullptr, P, g.topk);
+  // The shared expert in launches of its own, on the context's side stream: where its kernels differ from the routed
+  // experts', and for batches whose router takes long enough to hide them (at middle sizes they ride along: the
+  // router is two short launches there, and the shared expert's few tiles alone leave the chip idle).
+  const bool aside = v2 || (L.has_shared && (split || (c->shared_aside && !fused && !mid_router)));
   {
     const moe_comb cmb0{y, c->tokidx, c->pw, L.has_shared ? c->sh_logit : nullptr};
     int pre = MOE_OK;
@@ -1178,92 +1176,75 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   *enqueued = true;
   c->ev_n = 0;
   prof_mark(c, 0, st);
-  if (aside) {
-    // The shared expert does not depend on the routing: its two GEMMs run on the side stream from the start
-    // of the call, next to the fp64 router launch and the latency-bound top-k / permutation launches.  The
-    // side stream also makes what both streams need first: the per-token mean square of x (range guard) and
-    // the f16 copy of x.  Joins: in front of the routed gate/up GEMM (x16, xms) and in front of the combine.
-    const int sh_first = P * g.topk;
-    const int max_tiles_sh = (P + 127) / 128;
-    const int max_tiles = (P * g.topk + 127) / 128 + g.experts;
+  const int sh_first = P * g.topk;  // the shared expert's pair rows follow the routed ones
+  const bool sh_in = L.has_shared && !aside;  // ... and its tiles the routed tiles, where it rides along
+  const int max_tiles = (P * g.topk + 127) / 128 + g.experts + (sh_in ? (P + 127) / 128 : 0);
+  // what else is needed from x: f16 copy, mean square (range guard), the shared expert's gate logit
+  moe_row_extras ex{};
+  ex.x16 = c->x16_ext ? nullptr : c->x16;
+  ex.layout = xl;
+  ex.xms = c->xms;
+  if (L.has_shared) {
+    ex.wx = L.sh_sg.data;
+    ex.wx_bf16 = L.sh_sg.dtype == MOE_DT_BF16;
+    ex.out_x = c->sh_logit;
+  }
+  moe_rfix rf = router_fix(c, L, x, true);
+  if (mid_router) {
+    ex.tol = c->rtol;
+    ex.tol_scale = rf.tol_scale;
+    if ((rc = moe_router_batch_split(&L.router, x, P, c->ids, c->ws, g.topk, g.id_stride, c->gpart, ex, rf, st,
+                                     aside ? c->ev_fork : nullptr)))
+      return rc;
+  } else if (aside) {
     MOE_HIP(hipEventRecord(c->ev_fork, st));
+  }
+  int rs = MOE_OK;  // status of the side stream's launches
+  if (aside) {
+    // What does not depend on the routing runs on the side stream next to the router's launches: the passes over x that
+    // both streams need first (joined in front of the routed gate/up GEMM), then the shared expert's two GEMMs (joined
+    // in front of the combine).
     MOE_HIP(hipStreamWaitEvent(c->side, c->ev_fork, 0));
-    int rs = MOE_OK;
     if (v2) rs = moe_launch_v2_rot(x, (uint64_t)g.d, P, g.d, L.v2_su, nullptr, 1, c->v2_x16, (uint64_t)g.d, nullptr, 0, nullptr, nullptr, c->side);
-    if (!rs)
-      rs = c->x16_ext ? moe_launch_meansq_f16(xh, P, g.d, c->xms, c->side)
-                      : moe_launch_f16_rows_meansq(x, c->x16, P, g.d, xl, c->xms, c->side);
-    hipError_t ee = hipEventRecord(c->ev_x16, c->side);
+    if (!rs && !mid_router) rs = moe_launch_row_extras(x, P, g.d, ex, c->side);
+    const hipError_t ee = hipEventRecord(c->ev_x16, c->side);
     if (!rs && ee != hipSuccess) rs = (int)ee;
     if (L.has_shared) {
       if (!rs) rs = moe_launch_tiles_only_shared(c->tiles_sh, c->ntiles_sh, g.experts, moe_gemm_tile_cap(), P, sh_first, c->tokidx, c->side);
-      if (!rs) rs = gemm_up(true, c->tiles_sh, c->ntiles_sh, max_tiles_sh, c->side);
-      if (!rs) rs = gemm_dn(true, c->tiles_sh, c->ntiles_sh, max_tiles_sh, c->side, nullptr);
+      if (!rs) rs = gemm_up(true, c->tiles_sh, c->ntiles_sh, (P + 127) / 128, c->side);
+      if (!rs) rs = gemm_dn(true, c->tiles_sh, c->ntiles_sh, (P + 127) / 128, c->side, nullptr);
     }
-    // caller's stream: router, top-k, permutation, the routed experts' GEMMs
-    rc = router_batch(c, L, x, P, nullptr, st);
-    prof_mark(c, MOE_PROF_ROUTER, st);
-    if (!rc)
-      rc = moe_routing_run(c->routing, c->ids, c->ws, c->tokidx, c->pw, c->eoff, c->pairids, P, g.topk, g.experts,
-                           g.id_stride, st);
-    if (!rc) rc = moe_launch_tiles_shared(c->eoff, c->tiles, c->ntiles, g.experts, moe_gemm_tile_cap(), P, -1, c->tokidx, st);
-    ee = hipStreamWaitEvent(st, c->ev_x16, 0);
-    if (!rc && ee != hipSuccess) rc = (int)ee;
-    prof_mark(c, MOE_PROF_ROUTE, st);
-    if (!rc && !rs) rc = gemm_up(false, c->tiles, c->ntiles, max_tiles, st);
-    prof_mark(c, MOE_PROF_UP, st);
-    if (!rc && !rs) rc = gemm_dn(false, c->tiles, c->ntiles, max_tiles, st, nullptr);
-    // the side stream is joined on every path out of here (a capture on `st` must not end with it forked)
-    ee = hipEventRecord(c->ev_join, c->side);
-    if (ee == hipSuccess) ee = hipStreamWaitEvent(st, c->ev_join, 0);
-    prof_mark(c, MOE_PROF_DOWN, st);
-    if (rc) return rc;
-    if (rs) return rs;
-    if (ee != hipSuccess) return (int)ee;
-    rc = moe_launch_reduce(c->pairs16, true, c->pairids, c->pw, nullptr, L.has_shared ? c->sh_logit : nullptr,
-                           L.has_shared ? sh_first : -1, y, P, g.d, g.topk,
-                           hs, st, c->hc,
-                           v2 ? L.v2_svh_dn : nullptr);
-    prof_mark(c, MOE_PROF_REDUCE, st);
-    return rc;
   }
-  if ((rc = router_batch(c, L, x, P, c->xms, st))) return rc;
-  // x -> f16 (HBM-bound) on the side stream while top-k, counting, scan and scatter (small dependent
-  // launches that leave the memory system idle) run on the caller's stream
-  MOE_HIP(hipEventRecord(c->ev_fork, st));
-  MOE_HIP(hipStreamWaitEvent(c->side, c->ev_fork, 0));
-  int rc16 = c->x16_ext ? MOE_OK : moe_f32_to_f16(x, c->x16, (uint64_t)P * g.d, xl, c->side);
-  if (fused && !rc16) rc16 = moe_launch_zero_f32(y, (uint64_t)P * g.d, c->side);  // after the last read of x
-  // the side stream is joined on every path out of here (a capture on `st` must not end with it forked)
-  auto join = [&]() -> int {
-    hipError_t e = hipEventRecord(c->ev_join, c->side);
-    if (e == hipSuccess) e = hipStreamWaitEvent(st, c->ev_join, 0);
-    return (int)e;
-  };
-  const int sh_first = L.has_shared ? P * g.topk : -1;
-  rc = rc16;
+  // caller's stream: router, top-k, permutation, the routed experts' GEMMs
+  rc = MOE_OK;
+  if (!mid_router) {
+    rc = router_batch(c, L, x, P, st);
+    if (!rc && !aside) rc = moe_launch_row_extras(x, P, g.d, ex, st);
+  }
   prof_mark(c, MOE_PROF_ROUTER, st);
   if (!rc)
-    rc = moe_routing_run(c->routing, c->ids, c->ws, c->tokidx, c->pw, c->eoff, c->pairids, P, g.topk, g.experts,
-                         g.id_stride, st);
-  if (!rc) rc = moe_launch_tiles_shared(c->eoff, c->tiles, c->ntiles, g.experts, moe_gemm_tile_cap(), P, sh_first, c->tokidx, st);
-  const int jrc = join();
-  if (rc) return rc;
-  if (jrc) return jrc;
-  prof_mark(c, MOE_PROF_ROUTE, st);
-  const int max_tiles = (P * g.topk + 127) / 128 + g.experts + (L.has_shared ? (P + 127) / 128 : 0);
-  if ((rc = gemm_up(L.has_shared, c->tiles, c->ntiles, max_tiles, st))) return rc;
-  prof_mark(c, MOE_PROF_UP, st);
-  if (fused) {
-    const moe_comb cmb{y, c->tokidx, c->pw, L.has_shared ? c->sh_logit : nullptr};
-    rc = gemm_dn(L.has_shared, c->tiles, c->ntiles, max_tiles, st, &cmb);
-    prof_mark(c, MOE_PROF_DOWN, st);
-    return rc;
+    rc = moe_launch_route(moe_routing_blockcnt(c->routing), c->ids, c->ws, c->tokidx, c->pw, c->eoff, c->pairids, P, g.topk, g.experts, g.id_stride, c->tiles,
+                          c->ntiles, moe_gemm_tile_cap(), sh_in ? sh_first : -1, st);
+  if (!rc && fused) rc = moe_launch_zero_f32(y, (uint64_t)P * g.d, st);
+  if (aside) {
+    const hipError_t ee = hipStreamWaitEvent(st, c->ev_x16, 0);
+    if (!rc && ee != hipSuccess) rc = (int)ee;
   }
-  if ((rc = gemm_dn(L.has_shared, c->tiles, c->ntiles, max_tiles, st, nullptr))) return rc;
+  prof_mark(c, MOE_PROF_ROUTE, st);
+  if (!rc && !rs) rc = gemm_up(sh_in, c->tiles, c->ntiles, max_tiles, st);
+  prof_mark(c, MOE_PROF_UP, st);
+  const moe_comb cmb{y, c->tokidx, c->pw, L.has_shared ? c->sh_logit : nullptr};
+  if (!rc && !rs) rc = gemm_dn(sh_in, c->tiles, c->ntiles, max_tiles, st, fused ? &cmb : nullptr);
+  if (aside) {  // the side stream is joined on every path out of here (a capture on `st` must not end with it forked)
+    hipError_t ee = hipEventRecord(c->ev_join, c->side);
+    if (ee == hipSuccess) ee = hipStreamWaitEvent(st, c->ev_join, 0);
+    if (!rc && ee != hipSuccess) rc = (int)ee;
+  }
   prof_mark(c, MOE_PROF_DOWN, st);
+  if (rc || rs) return rc ? rc : rs;
+  if (fused) return MOE_OK;
   rc = moe_launch_reduce(c->pairs16, true, c->pairids, c->pw, nullptr, L.has_shared ? c->sh_logit : nullptr,
-                         sh_first, y, P, g.d, g.topk, hs, st, c->hc);
+                         L.has_shared ? sh_first : -1, y, P, g.d, g.topk, hs, st, c->hc, v2 ? L.v2_svh_dn : nullptr);
   prof_mark(c, MOE_PROF_REDUCE, st);
   return rc;
 }

@@ -94,30 +94,40 @@ int moe_gemm_tile_cap();
 int moe_launch_zero_f32(float* p, uint64_t n, hipStream_t st);
 int moe_launch_tiles_only_shared(moe_tile* tiles, int* ntiles, int E, int cap, int P, int sh_first, int* tokidx,
                                  hipStream_t st);
-int moe_launch_meansq_f16(const void* x16, int P, int d, float* xms, hipStream_t st);
-int moe_launch_f16_rows_meansq(const float* x, void* x16, int P, int d, int layout, float* xms, hipStream_t st);
-// permutation (+ tile list with tiles != nullptr) of a batch of at most 32 tokens in one launch
-bool moe_route_small_supported(int P, int k, int experts);
-int moe_launch_route_small(const int* ids, const float* ws, int* tokidx, float* pw, int* eoff, int* pairids,
-                           int P, int k, int experts, int id_stride, moe_tile* tiles, int* ntiles, int cap,
-                           int sh_first, hipStream_t st);
-int moe_launch_tiles_shared(const int* eoff, moe_tile* tiles, int* ntiles, int E, int cap, int P,
-                            int sh_first, int* tokidx, hipStream_t st);
+// permutation (+ tile list with tiles != nullptr) of any batch (route.hip)
+int* moe_routing_blockcnt(moe_routing* r);
+int moe_launch_route(int* blockcnt, const int* ids, const float* ws, int* tokidx, float* pw, int* eoff, int* pairids, int P,
+                     int k, int experts, int id_stride, moe_tile* tiles, int* ntiles, int cap, int sh_first, hipStream_t st);
 int moe_launch_reduce(const void* pairs, bool pairs_f16, const int* pairids, const float* pw,
                       const float* ey, const float* sg, int sh_first, float* out, int P, int D, int K,
                       moe_hscale hs, hipStream_t st, const moe_hc* hc, const float* rot_svh = nullptr);
-int moe_router_logits_seq(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x, int P,
-                          float* logits, float* out_x, float* out_xms, hipStream_t st);
-
-int moe_router_logits_seq_if(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x, int P,
-                             float* logits, float* out_x, float* out_xms, const int* run_if_above, int run_thr,
-                             hipStream_t st);
+// Router of 33 .. MOE_ROUTER_SPLIT_MAX tokens (router_split.hip): fp64 matrix pipe, columns split over waves and blocks, a
+// selecting block per token; what else a batch needs from x comes out of the first launch.
+constexpr int MOE_ROUTER_SPLIT_MAX = 1024, MOE_ROUTER_SPLIT_KS = 8;
+struct moe_row_extras {
+  void* x16;         // f16 copy of x in `layout` (moe_f32_to_f16), or nullptr
+  int layout;
+  float* xms;        // [P] mean square of each row, or nullptr
+  float* tol;        // [P] tol_scale * |row|, the selection's bound (moe_rfix), or nullptr
+  float tol_scale;
+  const void* wx;    // shared expert's gate vector, or nullptr
+  bool wx_bf16;
+  float* out_x;      // [P] its logit
+};
+int moe_launch_row_extras(const float* x, int P, int d, const moe_row_extras& R, hipStream_t st);  // (reduce.hip)
+bool moe_router_split_supported(const moe_wview* W, const moe_wview* Wx, int P, int k);
+size_t moe_router_split_scratch_bytes(int max_tokens, int experts, int d);
+int moe_router_batch_split(const moe_wview* W, const float* x, int P, int* ids, float* ws, int k,
+                           int id_stride, double* gpart, const moe_row_extras& R, const moe_rfix& RF, hipStream_t st,
+                           hipEvent_t after_rows = nullptr);  // recorded behind the first launch
+// sequential-order logits; run_if_above: only if *run_if_above > run_thr when the launch starts (device memory)
+int moe_router_logits_seq(const moe_wview* W, const float* bias, const float* x, int P, float* logits, hipStream_t st,
+                          const int* run_if_above = nullptr, int run_thr = 0);
 // batch router through candidate selection (router_cand.hip): bit-exact ids, weights within an ulp or two
-bool moe_router_cand_supported(const moe_wview* W, const moe_wview* Wx, int P, int k);
+bool moe_router_cand_supported(const moe_wview* W, int P, int k);
 size_t moe_router_cand_scratch_bytes(int max_tokens, int experts, int d);
-int moe_router_batch_cand(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x, int P,
-                          float* logits, float* out_x, float* out_xms, int* ids, float* ws, int k, int id_stride,
-                          void* scratch, hipStream_t st, float bias_max);
+int moe_router_batch_cand(const moe_wview* W, const float* bias, const float* x, int P, float* logits, int* ids, float* ws,
+                          int k, int id_stride, void* scratch, hipStream_t st, float bias_max);
 
 size_t moe_qvec_plane_bytes(int K);
 size_t moe_qvec_meta_bytes(int K);

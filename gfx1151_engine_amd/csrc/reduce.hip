@@ -5,6 +5,7 @@
 #include "common.h"
 #include "hv2.h"
 #include "internal.h"
+#include "rowx.h"
 
 namespace {
 
@@ -48,44 +49,15 @@ __global__ void __launch_bounds__(256) k_f32_to_f16_q4k(const float4* __restrict
   }
 }
 
-// The f16 copy of whole rows in layout 1 or 2 plus each row's mean square (the f16 range guard's input) in
-// one pass over x: a wave per row, lanes take the row's 8-element chunks in turn.
-template <int LAYOUT>
-__global__ void __launch_bounds__(256) k_f32_to_f16_rows(const float* __restrict__ x, uint4* __restrict__ y, int P,
-                                                         int d, float* __restrict__ xms) {
+__global__ void __launch_bounds__(256) k_row_extras(const float* __restrict__ x, int P, int d, moe_row_extras R) {
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (t >= P) return;
-  const float4* xr = (const float4*)(x + (size_t)t * d);
-  uint4* yr = y + (size_t)t * (d / 8);
-  float acc = 0.f;
-  for (int i = lane; i < d / 8; i += 64) {
-    float4 u, v;
-    __half2 a, b, c, e;
-    if (LAYOUT == 2) {
-      const int blk = i >> 3, w = i & 7;
-      u = xr[blk * 16 + w];
-      v = xr[blk * 16 + 8 + w];
-      a = __floats2half2_rn(u.x, u.z); b = __floats2half2_rn(v.x, v.z);
-      c = __floats2half2_rn(u.y, u.w); e = __floats2half2_rn(v.y, v.w);
-    } else if (LAYOUT == 0) {
-      u = xr[2 * i];
-      v = xr[2 * i + 1];
-      a = __floats2half2_rn(u.x, u.y); b = __floats2half2_rn(u.z, u.w);
-      c = __floats2half2_rn(v.x, v.y); e = __floats2half2_rn(v.z, v.w);
-    } else {
-      u = xr[2 * i];
-      v = xr[2 * i + 1];
-      a = __floats2half2_rn(u.x, v.x); b = __floats2half2_rn(u.y, v.y);
-      c = __floats2half2_rn(u.z, v.z); e = __floats2half2_rn(u.w, v.w);
-    }
-    acc += ((u.x * u.x + u.y * u.y) + (u.z * u.z + u.w * u.w)) + ((v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w));
-    uint4 o;
-    o.x = *(const uint32_t*)&a; o.y = *(const uint32_t*)&b; o.z = *(const uint32_t*)&c; o.w = *(const uint32_t*)&e;
-    yr[i] = o;
-  }
-#pragma unroll
-  for (int o = 32; o; o >>= 1) acc += __shfl_xor(acc, o, 64);
-  if (lane == 0) xms[t] = acc / (float)d;
+  float acc;
+  double gate;
+  row_extras_part(x, t, d, lane, 64, R, acc, gate);
+  acc = wave_sum(acc);
+  if (R.wx) gate = wave_sum(gate);
+  if (lane == 0) row_extras_out(t, d, R, acc, gate);
 }
 
 // out[t][c] = sum_{s<K} pw[pid_s] * pairs[pid_s][c]  (pid_s = pairids[t*K+s], ascending expert id)
@@ -221,54 +193,6 @@ __global__ void __launch_bounds__(128) k_reduce_pw_sg(const PT* __restrict__ pai
   o[1] = make_float4(sum[4], sum[5], sum[6], sum[7]);
 }
 
-// Tiles of the routed experts (expert order, <= cap pairs each) followed by the shared expert's
-// tiles: pairs [sh_first, sh_first + P) in runs of cap with expert id = n_experts; also fills
-// tokidx for those pairs with the identity.
-__global__ void __launch_bounds__(1024) k_tiles_shared(const int* __restrict__ eoff,
-                                                       moe_tile* __restrict__ tiles, int* __restrict__ total,
-                                                       int E, int cap, int P, int sh_first,
-                                                       int* __restrict__ tokidx) {
-  __shared__ int wsum[16];
-  __shared__ int routed_total;
-  const int e = threadIdx.x, lane = e & 63, w = e >> 6;
-  const int first = e < E ? eoff[e] : 0;
-  const int ne = e < E ? eoff[e + 1] - first : 0;
-  const int count = (ne + cap - 1) / cap;
-  int inc = count;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int v = __shfl_up(inc, o, 64);
-    if (lane >= o) inc += v;
-  }
-  if (lane == 63) wsum[w] = inc;
-  __syncthreads();
-  int base = 0;
-  for (int i = 0; i < w; i++) base += wsum[i];
-  const int begin = base + inc - count;
-  if (e == 1023) routed_total = begin + count;
-  for (int j = 0; j < count; j++) {
-    moe_tile t;
-    t.expert = e;
-    t.first = first + j * cap;
-    t.count = min(cap, ne - j * cap);
-    tiles[begin + j] = t;
-  }
-  __syncthreads();
-  const int nsh = sh_first >= 0 ? (P + cap - 1) / cap : 0;
-  for (int j = e; j < nsh; j += 1024) {
-    moe_tile t;
-    t.expert = E;
-    t.first = sh_first + j * cap;
-    t.count = min(cap, P - j * cap);
-    tiles[routed_total + j] = t;
-  }
-  if (e == 0) {
-    total[0] = routed_total + nsh;
-    total[1] = routed_total;
-  }
-  if (sh_first >= 0)
-    for (int i = e; i < P; i += 1024) tokidx[sh_first + i] = i;
-}
 // The shared expert's tile list on its own (it does not depend on the routing): tiles over pairs
 // [sh_first, sh_first + P) in runs of cap, expert id = n_experts, total = {tiles, 0 routed}; also the
 // identity tokidx entries of those pairs.
@@ -301,50 +225,12 @@ int moe_launch_tiles_only_shared(moe_tile* tiles, int* ntiles, int E, int cap, i
   return MOE_OK;
 }
 
-// x16 (layout 1 or 2) and the mean square of every row in one launch
-int moe_launch_f16_rows_meansq(const float* x, void* x16, int P, int d, int layout, float* xms, hipStream_t st) {
-  if (!x || !x16 || !xms || layout < 0 || layout > 2) return MOE_E_INVALID;
-  if (d % 8 || (layout == 2 && d % 64) || !moe_aligned(x, 16) || !moe_aligned(x16, 16)) return MOE_E_INVALID;
+// f16 copy, mean square, gate logit of every row in one launch
+int moe_launch_row_extras(const float* x, int P, int d, const moe_row_extras& R, hipStream_t st) {
+  if (!x || R.layout < 0 || R.layout > 2 || (R.wx && !R.out_x)) return MOE_E_INVALID;
+  if (d % 8 || (R.layout == 2 && d % 64) || !moe_aligned(x, 16) || !moe_aligned(R.x16, 16) || !moe_aligned(R.wx, 16)) return MOE_E_INVALID;
   if (P == 0) return MOE_OK;
-  if (layout == 0) k_f32_to_f16_rows<0><<<(P + 3) / 4, 256, 0, st>>>(x, (uint4*)x16, P, d, xms);
-  else if (layout == 2) k_f32_to_f16_rows<2><<<(P + 3) / 4, 256, 0, st>>>(x, (uint4*)x16, P, d, xms);
-  else k_f32_to_f16_rows<1><<<(P + 3) / 4, 256, 0, st>>>(x, (uint4*)x16, P, d, xms);
-  MOE_LAUNCH_CHECK();
-  return MOE_OK;
-}
-
-// per-token mean square from an f16 copy of x (any element order): one wave per token
-__global__ void __launch_bounds__(256) k_meansq_f16_rows(const uint4* __restrict__ x16, int P, int d,
-                                                         float* __restrict__ xms) {
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (t >= P) return;
-  const uint4* xr = x16 + (size_t)t * (d / 8);
-  float acc = 0.f;
-  for (int i = lane; i < d / 8; i += 64) {
-    const uint4 u = xr[i];
-    const __half2* h = (const __half2*)&u;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const float2 f = __half22float2(h[q]);
-      acc += f.x * f.x + f.y * f.y;
-    }
-  }
-#pragma unroll
-  for (int o = 32; o; o >>= 1) acc += __shfl_xor(acc, o, 64);
-  if (lane == 0) xms[t] = acc / (float)d;
-}
-
-int moe_launch_meansq_f16(const void* x16, int P, int d, float* xms, hipStream_t st) {
-  if (!x16 || !xms || d % 8 || !moe_aligned(x16, 16)) return MOE_E_INVALID;
-  if (P <= 0) return MOE_OK;
-  k_meansq_f16_rows<<<(P + 3) / 4, 256, 0, st>>>((const uint4*)x16, P, d, xms);
-  MOE_LAUNCH_CHECK();
-  return MOE_OK;
-}
-
-int moe_launch_tiles_shared(const int* eoff, moe_tile* tiles, int* ntiles, int E, int cap, int P,
-                            int sh_first, int* tokidx, hipStream_t st) {
-  k_tiles_shared<<<1, 1024, 0, st>>>(eoff, tiles, ntiles, E, cap, P, sh_first, tokidx);
+  k_row_extras<<<(P + 3) / 4, 256, 0, st>>>(x, P, d, R);
   MOE_LAUNCH_CHECK();
   return MOE_OK;
 }

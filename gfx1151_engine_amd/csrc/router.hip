@@ -25,19 +25,15 @@ __device__ __forceinline__ float load_w(const void* W, uint64_t i) {
 // are staged in LDS as f32 (k permuted so that one 16-byte read feeds four MFMAs) and widened in
 // registers; the next K slab is fetched into registers while the current one is consumed.
 // D layout: value r of lane l is token 4r + l/16, weight row l%16 of the 16 x 16 tile.
-// The shared-expert gate vector (Wx), if given, is one more plain FMA chain per token in the first
-// column block: its logit goes to out_x[t].  Block ids are dealt so that the column blocks of one
+// Block ids are dealt so that the column blocks of one
 // token tile run on the same XCD (ids that differ by 8) and share its L2 copy of the activations.
 typedef double double4v __attribute__((ext_vector_type(4)));
 constexpr int RS_E = 128, RS_K = 32, RS_PITCH = 36;
 template <bool BF16, int BT>
 __global__ void __launch_bounds__(256, 2) k_router_logits_seq(const void* __restrict__ W,
                                                            const float* __restrict__ bias,
-                                                           const void* __restrict__ Wx, bool wx_bf16,
                                                            const float* __restrict__ x, int P, int E,
-                                                           int d, float* __restrict__ logits,
-                                                           float* __restrict__ out_x,
-                                                           float* __restrict__ out_xms, int ncol, int ntt,
+                                                           int d, float* __restrict__ logits, int ncol, int ntt,
                                                            const int* __restrict__ run_if_above, int run_thr) {
   // (a launch that is only needed when many tokens were listed for an exact redo returns at once otherwise)
   if (run_if_above && *run_if_above <= run_thr) return;
@@ -46,15 +42,12 @@ __global__ void __launch_bounds__(256, 2) k_router_logits_seq(const void* __rest
   constexpr int WL = (RS_E * RS_K / 4) / 256; // (weights)
   __shared__ __attribute__((aligned(16))) float Xs[BT][RS_PITCH];
   __shared__ __attribute__((aligned(16))) float Ws[RS_E][RS_PITCH];
-  __shared__ float Wxs[RS_K];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int li = lane & 15, lg = lane >> 4, wm = wv >> 1, wn = wv & 1;
   const int b = blockIdx.x, xcd = b & 7, q = b >> 3;
   const int col = q % ncol, tt = (q / ncol) * 8 + xcd;
   if (tt >= ntt) return;
   const int e0 = col * RS_E, t0 = tt * BT;
-  const bool extra = Wx != nullptr && col == 0;
-  const bool want_ms = out_xms != nullptr && col == 0;
   const bool vec = (d % 4 == 0);
 
   auto fetch_x = [&](int c0, float4* v) {
@@ -102,11 +95,6 @@ __global__ void __launch_bounds__(256, 2) k_router_logits_seq(const void* __rest
       v[it] = f;
     }
   };
-  auto fetch_wx = [&](int c0) -> float {
-    const int cc = c0 + tid;
-    if (!extra || tid >= RS_K || cc >= d) return 0.f;
-    return wx_bf16 ? bf16_bits_to_f32(((const uint16_t*)Wx)[cc]) : ((const float*)Wx)[cc];
-  };
   // slab element k (0..31) of a row sits at [ (k & 3) * 8 + (k >> 2) ]: lane group g reads its
   // slices k = 4*kk + g for kk = 0..7 as two float4
   auto stage = [&](float (*dst)[RS_PITCH], const float4* v, int n) {
@@ -122,26 +110,18 @@ __global__ void __launch_bounds__(256, 2) k_router_logits_seq(const void* __rest
   for (int i = 0; i < MT; i++)
 #pragma unroll
     for (int j = 0; j < 4; j++) acc[i][j] = double4v{0.0, 0.0, 0.0, 0.0};
-  double accx = 0.0;
-  float accms = 0.f;
-  const bool do_x = extra && tid < BT;    // this thread also carries token t0 + tid of the gate row
-  const bool do_ms = want_ms && tid < BT;  // ... and that token's sum of squares
 
   float4 xr[XL], wr[WL];
-  float wxr;
   fetch_x(0, xr);
   fetch_w(0, wr);
-  wxr = fetch_wx(0);
   for (int c0 = 0; c0 < d; c0 += RS_K) {
     moe_lds_barrier();  // everybody is done reading the previous slab (LDS-only barriers: the next slab's loads stay in flight)
     stage(Xs, xr, XL);
     stage(Ws, wr, WL);
-    if (tid < RS_K) Wxs[tid] = wxr;
     moe_lds_barrier();
     if (c0 + RS_K < d) {
       fetch_x(c0 + RS_K, xr);
       fetch_w(c0 + RS_K, wr);
-      wxr = fetch_wx(c0 + RS_K);
     }
 #pragma unroll
     for (int half = 0; half < 2; half++) {
@@ -164,14 +144,6 @@ __global__ void __launch_bounds__(256, 2) k_router_logits_seq(const void* __rest
             acc[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[mt], bq[nt], acc[mt][nt], 0, 0, 0);
       }
     }
-    if (do_x) {
-#pragma unroll 8
-      for (int k = 0; k < RS_K; k++) accx = fma((double)Wxs[k], (double)Xs[tid][(k & 3) * 8 + (k >> 2)], accx);
-    }
-    if (do_ms) {
-#pragma unroll 8
-      for (int k = 0; k < RS_K; k++) accms = fmaf(Xs[tid][k], Xs[tid][k], accms);
-    }
   }
 #pragma unroll
   for (int mt = 0; mt < MT; mt++) {
@@ -189,8 +161,6 @@ __global__ void __launch_bounds__(256, 2) k_router_logits_seq(const void* __rest
       }
     }
   }
-  if (do_x && t0 + tid < P) out_x[t0 + tid] = (float)accx;
-  if (do_ms && t0 + tid < P) out_xms[t0 + tid] = accms / (float)d;
 }
 
 // The blocks past the rows of the small-batch router launches: the digit planes of x for the integer-dot decode
@@ -502,15 +472,14 @@ __global__ void __launch_bounds__(256) k_row_norm_max(const void* __restrict__ W
 
 // Launch of the sequential-order kernel: 128-token tiles when there are enough of them to fill the
 // chip, 64-token tiles otherwise.
-void launch_seq(const void* W, bool bf, const float* bias, const void* wx, bool xbf, const float* x, int P,
-                int E, int d, float* logits, float* out_x, float* out_xms, hipStream_t st,
+void launch_seq(const void* W, bool bf, const float* bias, const float* x, int P, int E, int d, float* logits, hipStream_t st,
                 const int* run_if_above = nullptr, int run_thr = 0) {
   const int ncol = (E + RS_E - 1) / RS_E;
   const bool big = (int64_t)((P + 127) / 128) * ncol >= 512;
   const int bt = big ? 128 : 64;
   const int ntt = (P + bt - 1) / bt;
   const unsigned grid = (unsigned)(((ntt + 7) / 8) * 8 * ncol);
-#define RS_GO(BF, BT) k_router_logits_seq<BF, BT><<<grid, 256, 0, st>>>(W, bias, wx, xbf, x, P, E, d, logits, out_x, out_xms, ncol, ntt, run_if_above, run_thr)
+#define RS_GO(BF, BT) k_router_logits_seq<BF, BT><<<grid, 256, 0, st>>>(W, bias, x, P, E, d, logits, ncol, ntt, run_if_above, run_thr)
   if (bf) { if (big) RS_GO(true, 128); else RS_GO(true, 64); }
   else { if (big) RS_GO(false, 128); else RS_GO(false, 64); }
 #undef RS_GO
@@ -680,31 +649,17 @@ MOE_API int moe_router_logits(const moe_wview* W, const float* bias, const float
     return moe_router_logits_small(W, bias, nullptr, x, P, logits, nullptr, nullptr, nullptr, false, nullptr, nullptr,
                                    nullptr, 0, 0, nullptr, moe_s(st), nullptr, nullptr);
   } else {
-    launch_seq(W->data, bf, bias, nullptr, false, x, P, E, d, logits, nullptr, nullptr, moe_s(st));
+    launch_seq(W->data, bf, bias, x, P, E, d, logits, moe_s(st));
   }
   MOE_LAUNCH_CHECK();
   return MOE_OK;
 }
 
-// Internal: sequential-order logits for any P (also used for the one-row shared-expert gate).
-int moe_router_logits_seq(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x, int P,
-                          float* logits, float* out_x, float* out_xms, hipStream_t st) {
-  const int E = (int)W->rows, d = (int)W->cols;
-  const bool xbf = Wx && Wx->dtype == MOE_DT_BF16;
-  const void* wx = Wx ? Wx->data : nullptr;
-  launch_seq(W->data, W->dtype == MOE_DT_BF16, bias, wx, xbf, x, P, E, d, logits, out_x, out_xms, st);
-  MOE_LAUNCH_CHECK();
-  return MOE_OK;
-}
-
-// Internal: the same launch, doing its work only if *run_if_above > run_thr when it starts (device memory).
-int moe_router_logits_seq_if(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x, int P,
-                             float* logits, float* out_x, float* out_xms, const int* run_if_above, int run_thr,
-                             hipStream_t st) {
-  const int E = (int)W->rows, d = (int)W->cols;
-  const bool xbf = Wx && Wx->dtype == MOE_DT_BF16;
-  launch_seq(W->data, W->dtype == MOE_DT_BF16, bias, Wx ? Wx->data : nullptr, xbf, x, P, E, d, logits, out_x, out_xms, st,
-             run_if_above, run_thr);
+// Internal: sequential-order logits for any P; with run_if_above the launch does its work only if *run_if_above > run_thr
+// when it starts (device memory).
+int moe_router_logits_seq(const moe_wview* W, const float* bias, const float* x, int P, float* logits, hipStream_t st,
+                          const int* run_if_above, int run_thr) {
+  launch_seq(W->data, W->dtype == MOE_DT_BF16, bias, x, P, (int)W->rows, (int)W->cols, logits, st, run_if_above, run_thr);
   MOE_LAUNCH_CHECK();
   return MOE_OK;
 }

@@ -42,7 +42,7 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 constexpr int RA_BT = 128, RA_BE = 128, RA_K = 32;
 constexpr int RA_PITCH = 80;   // bytes per LDS row: 32 f16 + 16 B of padding (the 16-byte fragment reads of 8 rows then cover all banks)
 constexpr int RA_CHUNK = 128;  // columns summed in the matrix pipe's f32 accumulators before they are added to the running sums
-constexpr int RC_SLOTS = 32;   // at most 31 candidates per token (+ the shared-expert gate row) in the exact pass
+constexpr int RC_SLOTS = 32;   // at most 31 candidates per token in the exact pass
 constexpr int RC_NC_ULP = 1 << 20;  // flag in nc[t]: one of the token's candidate logits may be an ulp off the reference's float
 
 // ---- 1. approximate logits: block = 128 tokens x 128 experts, 4 waves as 2 x 2, wave = 64 x 64 (2 x 2 MFMA tiles) ----
@@ -52,8 +52,8 @@ template <bool BF16>
 __global__ void __launch_bounds__(256, 2) k_router_approx(const void* __restrict__ W, const float* __restrict__ bias,
                                                          const float* __restrict__ x, int P, int E, int d,
                                                          float* __restrict__ alog, float* __restrict__ wnorm,
-                                                         float* __restrict__ xnorm, float* __restrict__ out_xms,
-                                                         int* __restrict__ counters, int ncol, int ntt) {
+                                                         float* __restrict__ xnorm, int* __restrict__ counters, int ncol,
+                                                         int ntt) {
   __shared__ __attribute__((aligned(16))) uint8_t Xs[RA_BT * RA_PITCH];
   __shared__ __attribute__((aligned(16))) uint8_t Ws[RA_BE * RA_PITCH];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -166,10 +166,7 @@ __global__ void __launch_bounds__(256, 2) k_router_approx(const void* __restrict
     }
     const int r = (tid + it * 256) / TPR;
     if (tid % TPR == 0) {
-      if (col == 0 && t0 + r < P) {
-        xnorm[t0 + r] = sqrtf(sx);
-        if (out_xms) out_xms[t0 + r] = sx / (float)d;
-      }
+      if (col == 0 && t0 + r < P) xnorm[t0 + r] = sqrtf(sx);
       if (tt == 0 && e0 + r < E) wnorm[e0 + r] = sqrtf(sw);
     }
   }
@@ -237,8 +234,7 @@ __device__ __forceinline__ float4 ld_stream4(const float* p) {
 }
 __global__ void __launch_bounds__(512, 1) k_router_approx2(const __half* __restrict__ W16, const float* __restrict__ bias,
                                                          const float* __restrict__ x, int P, int E, int d,
-                                                         float* __restrict__ alog, float* __restrict__ xnorm,
-                                                         float* __restrict__ out_xms) {
+                                                         float* __restrict__ alog, float* __restrict__ xnorm) {
   extern __shared__ __attribute__((aligned(16))) uint8_t r2sm[];
   uint8_t* const Wl = r2sm;
   uint8_t* const Xl = r2sm + R2_NBUF * R2_WBYTES;
@@ -378,10 +374,7 @@ __global__ void __launch_bounds__(512, 1) k_router_approx2(const __half* __restr
       v += __shfl_xor(v, 2, 64);
       v += __shfl_xor(v, 4, 64);
       const int f = (tid & 255) + 256 * j, row = f >> 3;
-      if (blockIdx.y == 0 && (f & 7) == 0 && xlive[j]) {
-        xnorm[t0 + row] = sqrtf(v);
-        if (out_xms) out_xms[t0 + row] = v / (float)d;
-      }
+      if (blockIdx.y == 0 && (f & 7) == 0 && xlive[j]) xnorm[t0 + row] = sqrtf(v);
     }
   }
 }
@@ -391,7 +384,7 @@ template <int NPL>
 __global__ void __launch_bounds__(1024) k_router_cand(const float* __restrict__ alog, const float* __restrict__ wnorm,
                                                      const float* __restrict__ xnorm, int P, int E, int k, float eps,
                                                      float dterm, uint32_t* __restrict__ pairs, int* __restrict__ nc,
-                                                     int* __restrict__ fb_list, int* __restrict__ counters, int gate_row) {
+                                                     int* __restrict__ fb_list, int* __restrict__ counters) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int t = blockIdx.x * 16 + wv;
   const bool tok = t < P;
@@ -445,11 +438,9 @@ __global__ void __launch_bounds__(1024) k_router_cand(const float* __restrict__ 
   }
   const int total = __shfl(inc, 63, 64);
   const bool ok = __all(fin) && total <= RC_SLOTS - 1 && total >= 1 && (maxU - thr) < 60.f && isfinite(tau);
-  // The rows whose exact dot products step 3 computes for this token: pairs[t][0 .. n), the shared-expert gate vector
-  // (row E) first where there is one, then the candidates; nc[t] = the number of candidates, -1 for a listed token.
+  // The rows whose exact dot products step 3 computes for this token: pairs[t][0 .. nc[t]); nc[t] = -1 for a listed token.
   if (!tok) return;
   uint32_t* mine_out = pairs + (size_t)t * RC_SLOTS;
-  if (gate_row && lane == 0) mine_out[0] = (uint32_t)E;
   if (!ok) {
     if (lane == 0) {
       nc[t] = -1;
@@ -457,7 +448,7 @@ __global__ void __launch_bounds__(1024) k_router_cand(const float* __restrict__ 
     }
     return;
   }
-  int pos = gate_row + inc - mine;
+  int pos = inc - mine;
 #pragma unroll
   for (int j = 0; j < NPL; j++)
     if (U[j] >= thr) mine_out[pos++] = (uint32_t)(NPL * lane + j);
@@ -617,11 +608,11 @@ __global__ void __launch_bounds__(64) k_router_exact_pairs(const void* __restric
 // current chunk is summed.  Two accumulators per lane, a three-step reduction; the order is fixed.
 template <bool BF16>
 __global__ void __launch_bounds__(256) k_router_pairs_token(const void* __restrict__ W, const float* __restrict__ bias,
-                                                            const void* __restrict__ Wx, const float* __restrict__ x,
+                                                            const float* __restrict__ x,
                                                             int P, int E, int d, const uint32_t* __restrict__ pairs,
-                                                            float* __restrict__ logits, float* __restrict__ out_x,
+                                                            float* __restrict__ logits,
                                                             const float* __restrict__ wnorm, const float* __restrict__ xnorm,
-                                                            int* __restrict__ nc, int gate_row) {
+                                                            int* __restrict__ nc) {
   constexpr int CH = 256;                    // columns of x per wave load
   constexpr int LINE = BF16 ? 64 : 32;       // columns per 128-byte line of a weight row
   constexpr int NL = CH / LINE;              // lines per chunk
@@ -633,7 +624,7 @@ __global__ void __launch_bounds__(256) k_router_pairs_token(const void* __restri
   const int t = blockIdx.x * 4 + wv;
   if (t >= P) return;
   const int ncv = nc[t];
-  const int cnt = (ncv < 0 ? 0 : ncv) + gate_row;  // (the marks of this launch are set after every wave's own read)
+  const int cnt = ncv < 0 ? 0 : ncv;  // (the marks of this launch are set after every wave's own read)
   const int slot = lane >> 3, j = lane & 7;
   const float* xrow = x + (size_t)t * d;
   const uint32_t* mine = pairs + (size_t)t * RC_SLOTS;
@@ -644,8 +635,7 @@ __global__ void __launch_bounds__(256) k_router_pairs_token(const void* __restri
   for (int p0 = 0; p0 < cnt; p0 += 8) {
     const bool live = p0 + slot < cnt;
     const int e = (int)mine[live ? p0 + slot : p0];  // idle slots repeat the pass's first row (no extra traffic)
-    const bool gate = e == E;
-    const uint8_t* wrow = gate ? (const uint8_t*)Wx : (const uint8_t*)W + (size_t)e * d * ESZ;
+    const uint8_t* wrow = (const uint8_t*)W + (size_t)e * d * ESZ;
     double a0 = 0.0, a1 = 0.0;
     uint4 wc[NL], wn[NL];
     auto load_w = [&](int g, uint4* w) {
@@ -700,14 +690,11 @@ __global__ void __launch_bounds__(256) k_router_pairs_token(const void* __restri
 #pragma unroll
     for (int o = 1; o < 8; o <<= 1) acc += __shfl_xor(acc, o, 64);
     if (live && j == 0) {
-      if (gate) out_x[t] = (float)acc;
-      else {
-        float v = (float)acc;
-        const double delta = (double)(2.f * (float)(d + 8) * 0x1p-53f * 1.01f) * (double)wnorm[e] * (double)xnorm[t];
-        if ((float)(acc - delta) != v || (float)(acc + delta) != v) atomicOr(&nc[t], RC_NC_ULP);
-        if (bias) v += bias[e];
-        logits[(size_t)t * E + e] = v;
-      }
+      float v = (float)acc;
+      const double delta = (double)(2.f * (float)(d + 8) * 0x1p-53f * 1.01f) * (double)wnorm[e] * (double)xnorm[t];
+      if ((float)(acc - delta) != v || (float)(acc + delta) != v) atomicOr(&nc[t], RC_NC_ULP);
+      if (bias) v += bias[e];
+      logits[(size_t)t * E + e] = v;
     }
   }
 }
@@ -816,11 +803,10 @@ __global__ void __launch_bounds__(256) k_router_topk_listed(const float* __restr
 
 }  // namespace
 
-bool moe_router_cand_supported(const moe_wview* W, const moe_wview* Wx, int P, int k) {
+bool moe_router_cand_supported(const moe_wview* W, int P, int k) {
   const int E = (int)W->rows, d = (int)W->cols;
   if (P < 1 || d % RA_K || d < RA_K || E > 512 || k + 1 > RC_SLOTS - 1 || k >= E) return false;
-  if (Wx && (Wx->dtype == MOE_DT_BF16) != (W->dtype == MOE_DT_BF16)) return false;
-  return moe_aligned(W->data, 16) && (!Wx || moe_aligned(Wx->data, 16));
+  return moe_aligned(W->data, 16);
 }
 
 static size_t rc_epad(int experts) { return ((size_t)experts + R2_BE - 1) / R2_BE * R2_BE; }
@@ -829,13 +815,11 @@ size_t moe_router_cand_scratch_bytes(int max_tokens, int experts, int d) {
   return (size_t)max_tokens * (RC_SLOTS * 4 + 4 + 4 + 4) + rc_epad(experts) * 4 + 64 + 256 + 256 + rc_epad(experts) * (size_t)d * 2;
 }
 
-// Internal: ids / ws (and the shared-expert gate logit, the per-token mean square of x) of a batch; `logits` ends
-// up holding exact values for each token's candidates and approximate ones elsewhere.
-int moe_router_batch_cand(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x, int P,
-                          float* logits, float* out_x, float* out_xms, int* ids, float* ws, int k, int id_stride,
-                          void* scratch, hipStream_t st, float bias_max) {
+// Internal: ids / ws of a batch; `logits` ends up holding exact values for each token's candidates and approximate ones elsewhere.
+int moe_router_batch_cand(const moe_wview* W, const float* bias, const float* x, int P, float* logits, int* ids, float* ws,
+                          int k, int id_stride, void* scratch, hipStream_t st, float bias_max) {
   const int E = (int)W->rows, d = (int)W->cols;
-  if (!moe_router_cand_supported(W, Wx, P, k) || !moe_aligned(x, 16)) return MOE_E_UNSUPPORTED;
+  if (!moe_router_cand_supported(W, P, k) || !moe_aligned(x, 16)) return MOE_E_UNSUPPORTED;
   uint8_t* sp = (uint8_t*)scratch;
   int* counters = (int*)sp; sp += 64;
   uint32_t* pairs = (uint32_t*)sp; sp += (size_t)P * RC_SLOTS * 4;
@@ -851,7 +835,6 @@ int moe_router_batch_cand(const moe_wview* W, const float* bias, const moe_wview
   const float eps = (0x1p-10f + (float)RA_CHUNK * 0x1p-22f + (float)(d / RA_CHUNK + 1) * 0x1p-23f) * 1.002f * 1.01f;
   const float dterm = 0x1p-25f * 1.01f * sqrtf((float)d);
   const int dense_above = P / 16;
-  const void* wx = Wx ? Wx->data : nullptr;
   const unsigned gtok = (unsigned)((P + 3) / 4), gtok16 = (unsigned)((P + 15) / 16);
   if (d % RA_CHUNK == 0) {
     // the router matrix as f16 once per call (a few microseconds), then the approximate logits with a token tile's
@@ -867,19 +850,18 @@ int moe_router_batch_cand(const moe_wview* W, const float* bias, const moe_wview
       moe_dev_done(attr_once, dev_now);
     }
     const dim3 g2((unsigned)((P + R2_BT - 1) / R2_BT), (unsigned)(Epad / R2_BE));
-    k_router_approx2<<<g2, 512, R2_SMEM, st>>>(W16, bias, x, P, E, d, logits, xnorm, out_xms);
+    k_router_approx2<<<g2, 512, R2_SMEM, st>>>(W16, bias, x, P, E, d, logits, xnorm);
   } else if (bf) {
-    k_router_approx<true><<<grid_a, 256, 0, st>>>(W->data, bias, x, P, E, d, logits, wnorm, xnorm, out_xms, counters, ncol, ntt);
+    k_router_approx<true><<<grid_a, 256, 0, st>>>(W->data, bias, x, P, E, d, logits, wnorm, xnorm, counters, ncol, ntt);
   } else {
-    k_router_approx<false><<<grid_a, 256, 0, st>>>(W->data, bias, x, P, E, d, logits, wnorm, xnorm, out_xms, counters, ncol, ntt);
+    k_router_approx<false><<<grid_a, 256, 0, st>>>(W->data, bias, x, P, E, d, logits, wnorm, xnorm, counters, ncol, ntt);
   }
   MOE_LAUNCH_CHECK();
-  k_router_cand<8><<<gtok16, 1024, 0, st>>>(logits, wnorm, xnorm, P, E, k, eps, dterm, pairs, nc, fb_list, counters,
-                                         wx ? 1 : 0);
+  k_router_cand<8><<<gtok16, 1024, 0, st>>>(logits, wnorm, xnorm, P, E, k, eps, dterm, pairs, nc, fb_list, counters);
   MOE_LAUNCH_CHECK();
-  // at most 32 rows per token (31 candidates + the gate row): a wave per token, eight rows a pass
-  if (bf) k_router_pairs_token<true><<<gtok, 256, 0, st>>>(W->data, bias, wx, x, P, E, d, pairs, logits, out_x, wnorm, xnorm, nc, wx ? 1 : 0);
-  else k_router_pairs_token<false><<<gtok, 256, 0, st>>>(W->data, bias, wx, x, P, E, d, pairs, logits, out_x, wnorm, xnorm, nc, wx ? 1 : 0);
+  // at most 31 rows per token: a wave per token, eight rows a pass
+  if (bf) k_router_pairs_token<true><<<gtok, 256, 0, st>>>(W->data, bias, x, P, E, d, pairs, logits, wnorm, xnorm, nc);
+  else k_router_pairs_token<false><<<gtok, 256, 0, st>>>(W->data, bias, x, P, E, d, pairs, logits, wnorm, xnorm, nc);
   MOE_LAUNCH_CHECK();
   k_router_topk_mixed<8><<<gtok, 256, 0, st>>>(logits, ids, ws, P, E, k, id_stride, nc, fb_list, counters, bias_max);
   MOE_LAUNCH_CHECK();
@@ -890,7 +872,7 @@ int moe_router_batch_cand(const moe_wview* W, const float* bias, const moe_wview
   if (bf) k_router_exact_pairs<true><<<glist, 64, 0, st>>>(W->data, bias, x, E, d, counters, logits, fb_list, dense_above, wpt);
   else k_router_exact_pairs<false><<<glist, 64, 0, st>>>(W->data, bias, x, E, d, counters, logits, fb_list, dense_above, wpt);
   MOE_LAUNCH_CHECK();
-  int rc = moe_router_logits_seq_if(W, bias, nullptr, x, P, logits, nullptr, nullptr, counters, dense_above, st);
+  const int rc = moe_router_logits_seq(W, bias, x, P, logits, st, counters, dense_above);
   if (rc) return rc;
   k_router_topk_listed<8><<<gtok, 256, 0, st>>>(logits, ids, ws, P, E, k, id_stride, fb_list, counters, dense_above);
   MOE_LAUNCH_CHECK();

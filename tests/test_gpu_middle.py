@@ -1,0 +1,82 @@
+"""Batches between the in-place kernels and the largest prefill chunks: the sizes at which the router, the permutation
+and the grouped GEMM change kernels, against the oracle."""
+import numpy as np
+import pytest
+
+from helpers import HostLayer, max_abs_rel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def capi():
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from gfx1151_engine_amd import capi as m
+    return m
+
+
+def gpu(a):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+# ---------- permutation: one block of tokens, its writers, several blocks ----------
+@pytest.mark.parametrize("P,E,k,stride", [(64, 512, 10, 16), (128, 512, 10, 16), (129, 64, 4, 16), (1024, 512, 10, 16),
+                                          (1025, 512, 10, 16), (2049, 8, 3, 4), (512, 1000, 12, 16), (513, 1000, 13, 16),
+                                          (700, 30, 17, 20), (1100, 30, 17, 17)])
+def test_routing_block_edges(capi, oracle, P, E, k, stride):
+    rng = np.random.default_rng(P + E)
+    ids = np.zeros((P, stride), np.int32)
+    ws = rng.random((P, stride)).astype(np.float32)
+    pr = 1.0 / (np.arange(E) + 1.0)
+    pr /= pr.sum()
+    for t in range(P):
+        ids[t, :k] = rng.choice(E, k, replace=False, p=pr)
+    to, po, eo, qo = oracle.route(ids, ws, k, E)
+    r = capi.Routing(P * k, E)
+    for got in (r.run(gpu(ids), gpu(ws), k), capi.routing_run_static(gpu(ids), gpu(ws), k, E)):
+        tokidx, pw, eoff, pairids = (a.cpu().numpy() for a in got)
+        assert (eoff == eo).all() and (tokidx == to).all() and (pw == po).all() and (pairids == qo).all()
+    r.close()
+
+
+# ---------- router: edges of its token and expert tiles, the last batch it takes and the first it does not ----------
+@pytest.mark.parametrize("T,E,k,d,dt", [(33, 512, 10, 3072, "bf16"), (64, 33, 5, 256, "f32"), (65, 512, 10, 2560, "f32"),
+                                        (515, 512, 10, 768, "bf16"), (1024, 520, 10, 384, "f32"), (1025, 512, 10, 384, "bf16")])
+def test_router_tiles(capi, oracle, T, E, k, d, dt):
+    rng = np.random.default_rng(T)
+    hl = HostLayer(rng, d, 256, E, k, router_dtype=dt)  # (the gate vector is f32 beside either type)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    x[T // 2] = x[0]
+    lo, io, wo = oracle.router(hl.oracle_layer().router, x, k)
+    m, dev = hl.to_gpu(max_tokens=T)
+    y = m.forward(0, gpu(x)).cpu().numpy()
+    assert m.last_path() == capi.PATH_BATCH
+    ids, ws = (a.cpu().numpy()[:, :k] for a in m.last_routing(T))
+    m.close()
+    assert (ids == io[:, :k]).all()
+    assert np.abs(ws - wo[:, :k]).max() <= 2.5e-7
+    sel = np.r_[0, T // 2, T - 1]
+    yo, _, _ = oracle.moe_layer(hl.oracle_layer(), x[sel])
+    assert max_abs_rel(y[sel], yo) <= 2e-3
+
+
+def test_router_ties_above_the_middle(capi, oracle):
+    """The candidate selection's redo of listed tokens, at a size only it takes: tied and nearly tied rows, a zero token."""
+    rng = np.random.default_rng(11)
+    E, k, d, T = 128, 10, 512, 1200
+    hl = HostLayer(rng, d, 256, E, k, shared=False)
+    hl.router[7] = hl.router[3]
+    hl.router[16] = hl.router[5] * np.float32(1 + 2 ** -22)
+    for zeros in (2, T - 30):  # few listed tokens; most of them (the dense launch takes over)
+        x = rng.standard_normal((T, d), dtype=np.float32)
+        x[:zeros] = 0.0
+        lo, io, wo = oracle.router(hl.oracle_layer().router, x, k)
+        m, dev = hl.to_gpu(max_tokens=T)
+        m.forward(0, gpu(x))
+        ids, ws = (a.cpu().numpy()[:, :k] for a in m.last_routing(T))
+        m.close()
+        assert (ids == io[:, :k]).all()
+        assert np.abs(ws - wo[:, :k]).max() <= 2.5e-7
