@@ -22,6 +22,8 @@ struct MoeLayer {
   int sh_dense = 0;  // != 0: gate/up/down of the shared expert are dense rows of this kind (dense.h), in launches of their own
   // every q4cp codebook of the layer is affine (cb[n] = a*n + b): the integer-dot decode kernels apply
   bool experts_affine = false, shared_affine = false;
+  // every expert of the tensor has a power of two for the scaled dequantisation (pexp below)
+  bool scaled_gu = false, scaled_dn = false, scaled_sgu = false, scaled_sdn = false;
   // f16 range guard of the batch path: typical |hid| (and |pair|) per unit mean-square activation,
   // estimated from sampled weight rows when the weights are registered
   moe_cmag c_routed{0.f, 0.f}, c_shared{0.f, 0.f};  // f16 range guard constants (common.h), 0 = no guard
@@ -42,7 +44,7 @@ static int codebook_affine(const moe_wview* w, bool* out) {
 }
 
 struct moe_ctx;
-static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_wview* a, const moe_wview* b, int n_experts);
+static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_wview* a, const moe_wview* b, int n_experts, bool* all);
 static int magnitude_constant(moe_ctx* c, int tgu, int tdn, const moe_wview* gate, uint64_t gate_stride,
                               const moe_wview* up, uint64_t up_first, const moe_wview* down, int n_experts,
                               moe_cmag* out);
@@ -134,7 +136,9 @@ struct moe_ctx {
 static int8_t* pexp_slot(moe_ctx* c, int layer, int slot0) {
   return c->pexp ? c->pexp + (size_t)layer * (2 * (size_t)c->cfg.experts + 2) + slot0 : nullptr;
 }
-static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_wview* a, const moe_wview* b, int n_experts) {
+// *all: every expert has one.
+static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_wview* a, const moe_wview* b, int n_experts, bool* all) {
+  *all = false;
   int8_t* dst = pexp_slot(c, layer, slot0);
   if (!dst) return MOE_OK;  // contexts for small batches only have no grouped GEMM
   std::vector<int8_t> out((size_t)n_experts, (int8_t)MOE_PEXP_NONE);
@@ -148,7 +152,11 @@ static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_wview* a, c
       if ((rc = moe_q4cp_scale_span(b, n_experts, c->span_tmp, nullptr))) return rc;
       MOE_HIP(hipMemcpy(sb.data(), c->span_tmp, sb.size(), hipMemcpyDeviceToHost));
     }
-    for (int e = 0; e < n_experts; e++) out[e] = (int8_t)moe_pexp_from_span(&sa[2 * e], b ? &sb[2 * e] : nullptr);
+    *all = true;
+    for (int e = 0; e < n_experts; e++) {
+      out[e] = (int8_t)moe_pexp_from_span(&sa[2 * e], b ? &sb[2 * e] : nullptr);
+      *all = *all && out[e] != (int8_t)MOE_PEXP_NONE;
+    }
   }
   MOE_HIP(hipMemcpy(dst, out.data(), out.size(), hipMemcpyHostToDevice));
   return MOE_OK;
@@ -239,6 +247,13 @@ MOE_API int moe_create(const moe_config* cfg, moe_ctx** out) {
     // expert-sorted permutation: the batch path, and small batches that de-duplicate shared experts
     const size_t batch_tiles = (T * cfg->topk + 127) / 128 + E + (T + 127) / 128, uq_tiles = Ts * cfg->topk + (Ts + 3) / 4;
     c->max_tiles = (int)(batch_tiles > uq_tiles ? batch_tiles : uq_tiles);
+    for (size_t p = 33; p <= T; p++) {  // middle-sized batches: smaller tiles
+      const int narrow = moe_stream_tile_cap((int)p, cfg->topk, (int)E, false);
+      const int cap = narrow ? narrow : moe_stream_tile_cap((int)p, cfg->topk, (int)E, true);
+      if (!cap) break;
+      const int n = (int)((p * cfg->topk + cap - 1) / cap + E + (p + cap - 1) / cap);
+      c->max_tiles = c->max_tiles > n ? c->max_tiles : n;
+    }
     int rc = moe_routing_create((int)(T * cfg->topk), cfg->experts, &c->routing);
     if (rc != MOE_OK) {
       moe_destroy(c);
@@ -326,8 +341,8 @@ MOE_API int moe_set_experts_q4cp(moe_ctx* c, int layer, const moe_wview* gu, con
   L->experts_affine = a1 && a2;
   if ((rc = magnitude_constant(c, 0, 0, gu, (uint64_t)2 * g.mid, gu, (uint64_t)g.mid, dn, g.experts, &L->c_routed)))
     return rc;
-  if ((rc = pexp_register(c, layer, 0, a1 ? gu : nullptr, nullptr, g.experts)) ||
-      (rc = pexp_register(c, layer, g.experts, a2 ? dn : nullptr, nullptr, g.experts)))
+  if ((rc = pexp_register(c, layer, 0, a1 ? gu : nullptr, nullptr, g.experts, &L->scaled_gu)) ||
+      (rc = pexp_register(c, layer, g.experts, a2 ? dn : nullptr, nullptr, g.experts, &L->scaled_dn)))
     return rc;
   L->gate_up = *gu;
   L->down = *dn;
@@ -441,13 +456,13 @@ MOE_API int moe_set_shared(moe_ctx* c, int layer, const moe_wview* g, const moe_
     int rc;
     if ((rc = codebook_affine(g, &a1)) || (rc = codebook_affine(u, &a2)) || (rc = codebook_affine(dn, &a3))) return rc;
     L->shared_affine = a1 && a2 && a3;
-    if ((rc = pexp_register(c, layer, 2 * cf.experts, a1 && a2 ? g : nullptr, u, 1)) ||
-        (rc = pexp_register(c, layer, 2 * cf.experts + 1, a3 ? dn : nullptr, nullptr, 1)))
+    if ((rc = pexp_register(c, layer, 2 * cf.experts, a1 && a2 ? g : nullptr, u, 1, &L->scaled_sgu)) ||
+        (rc = pexp_register(c, layer, 2 * cf.experts + 1, a3 ? dn : nullptr, nullptr, 1, &L->scaled_sdn)))
       return rc;
   } else {
     int rc;
-    if ((rc = pexp_register(c, layer, 2 * cf.experts, nullptr, nullptr, 1)) ||
-        (rc = pexp_register(c, layer, 2 * cf.experts + 1, nullptr, nullptr, 1)))
+    if ((rc = pexp_register(c, layer, 2 * cf.experts, nullptr, nullptr, 1, &L->scaled_sgu)) ||
+        (rc = pexp_register(c, layer, 2 * cf.experts + 1, nullptr, nullptr, 1, &L->scaled_sdn)))
       return rc;
   }
   L->c_shared = moe_cmag{0.f, 0.f};
@@ -995,6 +1010,34 @@ static int batch_x16_layout(const MoeLayer& L, const moe_config& g) {
   return gg_kinds(L, g).any_tuned() ? 2 : 0;
 }
 
+// Which of the streaming kernel's formats (gemm_stream.hip) a layer's routed experts take, up and down; -1: none, the layer
+// stays on the 128-pair kernels.  with_sh: the shared expert's tiles can ride in the same launches.
+struct StreamKinds {
+  int up, dn;
+  bool with_sh;
+};
+static StreamKinds stream_kinds(const MoeLayer& L, const moe_config& g) {
+  StreamKinds k{-1, -1, false};
+  const bool q4sh = L.has_shared && !L.sh_dense && L.sh_gguf_type == 0;
+  if (L.has_i4r) {
+    k.up = k.dn = MOE_STREAM_I4R;
+  } else if (L.has_q4cp) {
+    // (affine experts beside a table-coded shared expert, which is possible and unusual: one launch, one format)
+    if (L.experts_affine && q4sh && !L.shared_affine) return k;
+    k.up = !L.experts_affine ? MOE_STREAM_TABLE : L.scaled_gu && (!q4sh || L.scaled_sgu) ? MOE_STREAM_SCALED : MOE_STREAM_AFFINE;
+    k.dn = !L.experts_affine ? MOE_STREAM_TABLE : L.scaled_dn && (!q4sh || L.scaled_sdn) ? MOE_STREAM_SCALED : MOE_STREAM_AFFINE;
+    k.with_sh = q4sh;
+  } else if (L.has_gguf) {
+    const int up = L.gg.tgu == MOE_GGML_Q4_K ? MOE_STREAM_Q4K : L.gg.tgu == MOE_GGML_Q5_K ? MOE_STREAM_Q5K : -1;
+    const int dn = L.gg.tdn == MOE_GGML_Q4_K ? MOE_STREAM_Q4K : L.gg.tdn == MOE_GGML_Q8_0 ? MOE_STREAM_Q8_0 : -1;
+    if (up < 0 || dn < 0) return k;
+    k.up = up;
+    k.dn = dn;
+    k.with_sh = L.has_shared && !L.sh_dense && L.sh_gguf_type == L.gg.tgu && L.sh_gguf_type == L.gg.tdn;
+  }
+  return k;
+}
+
 // Router of a batch above MOE_ROUTER_SPLIT_MAX tokens: ids / ws.  By default through candidate selection
 // (router_cand.hip); MOE_OPT_ROUTER_CANDIDATES = 0, or a shape it does not take, runs the dense fp64 launch and the exact
 // softmax / top-k over all experts.
@@ -1030,7 +1073,14 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   // GGUF layers: each launch on the tuned kernel where it has a form for the block type, else on the general one
   const GgKinds kd = gg_kinds(L, g);
   const bool shd = L.has_shared && L.sh_dense;  // shared expert stored densely: the general GEMM, launches of its own
-  const bool split = shd || (q4k && !kd.uniform(L));  // routed and shared experts in launches of their own
+  const bool fused = c->fused_combine && !c->hc && !(q4k && !kd.r_dn) && !shd && !(q4k && !kd.uniform(L)) && !v2;  // the HC write-back belongs to the ordered combine
+  // middle sizes: tiles of few pairs, the weights streamed into registers
+  const StreamKinds sk = stream_kinds(L, g);
+  int cap = fused || sk.up < 0 ? 0 : moe_stream_tile_cap(P, g.topk, g.experts, moe_stream_wide(sk.up, sk.dn));
+  const int sxl = sk.up >= MOE_STREAM_Q4K ? 2 : sk.up == MOE_STREAM_TABLE ? 0 : 1;  // the order of activations it reads
+  if (c->x16_ext && sxl != batch_x16_layout(L, g)) cap = 0;
+  // routed and shared experts in launches of their own
+  bool split = shd || (q4k && !kd.uniform(L)) || (cap && L.has_shared && !sk.with_sh);
   if (L.has_shared && !shd && (L.sh_gguf_type != 0) != q4k) return MOE_E_UNSUPPORTED;  // one format family per layer
   if (q4k ? (g.d % 64 || g.mid % 64) : (g.d % 128 || g.mid % 128 || g.mid < 256 || g.d < 256))
     return MOE_E_UNSUPPORTED;  // the caller walks the batch through the small path
@@ -1063,7 +1113,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   int rc;
   const moe_hscale hs{c->xms, L.c_routed, L.c_shared};
   const __half* xh = c->x16_ext ? c->x16_ext : c->x16;  // f16 activations in the GEMM's order
-  const int xl = batch_x16_layout(L, g);       // that order (moe_f32_to_f16's layout)
+  int xl = cap ? sxl : batch_x16_layout(L, g);  // that order (moe_f32_to_f16's layout)
   const bool nat = batch_nat(L);               // table codebooks: natural K order, pair tables
   // scaled dequantisation (affine q4cp codebooks): the powers of two found when the weights were registered
   const bool pe_r = L.has_q4cp && !v2 && L.experts_affine, pe_s = L.has_shared && !shd && !q4k && L.shared_affine;
@@ -1076,8 +1126,16 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   // dry: the launchers run their shape / type / alignment checks and return in front of the launch (a tile capacity
   // of 0), so that every reason to decline is found before anything is enqueued
   bool dry = true;
-  auto gemm_up = [&](bool with_sh, const moe_tile* tl, const int* ntl, int mt, hipStream_t s2) -> int {
+  // (routed: the launch holds the routed experts' tiles -- with_sh then says that the shared expert's ride along)
+  auto gemm_up = [&](bool routed, bool with_sh, const moe_tile* tl, const int* ntl, int mt, hipStream_t s2) -> int {
     if (dry) mt = 0;
+    if (routed && cap) {
+      const moe_rotv rv{L.v2_svh_gu, L.v2_suh_dn};
+      moe_lutw gf = gu;
+      if (v2) gf.up_off = g.mid;
+      return moe_launch_stream(sk.up, true, cap, &gf, with_sh ? &sgu : nullptr, g.experts, v2 ? c->v2_x16 : xh, c->tokidx, tl, ntl,
+                               mt, c->hid16, g.mid, g.d, hs, s2, sh_cb_up, pe_gu, pe_sgu, v2 ? &rv : nullptr);
+    }
     if (shd && with_sh)  // the shared expert's own tile list
       return moe_launch_gemm_gg(true, L.sh_dense, L.sh_gate.data, L.sh_up.data, 0, nullptr, nullptr, g.experts, xh,
                                 c->tokidx, tl, ntl, mt, c->hid16, g.mid, g.d, hs, s2, xl);
@@ -1119,8 +1177,11 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
                                 g.mid, g.d, true, q4k, hs, s2, nullptr, sh_cb_up, 0, q4k && L.gg.tgu == MOE_GGML_Q5_K, nat,
                                 pe_gu, pe_sgu);
   };
-  auto gemm_dn = [&](bool with_sh, const moe_tile* tl, const int* ntl, int mt, hipStream_t s2, const moe_comb* cmb) -> int {
+  auto gemm_dn = [&](bool routed, bool with_sh, const moe_tile* tl, const int* ntl, int mt, hipStream_t s2, const moe_comb* cmb) -> int {
     if (dry) mt = 0;
+    if (routed && cap)
+      return moe_launch_stream(sk.dn, false, cap, &dn, with_sh ? &sdn : nullptr, g.experts, c->hid16, nullptr, tl, ntl, mt,
+                               c->pairs16, g.d, g.mid, hs, s2, nullptr, pe_dn, pe_sdn);
     if (shd && with_sh)  // (hid rows of the shared tiles were written in natural order by the launch above)
       return moe_launch_gemm_gg(false, L.sh_dense, L.sh_down.data, nullptr, 0, nullptr, nullptr, g.experts, c->hid16,
                                 nullptr, tl, ntl, mt, c->pairs16, g.d, g.mid, hs, s2, 0);
@@ -1149,7 +1210,19 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
                                 cmb ? (void*)cmb->y : (void*)c->pairs16, g.d, g.mid, cmb == nullptr, q4k, hs, s2, cmb, nullptr,
                                 0, false, nat, pe_dn, pe_sdn);
   };
-  const bool fused = c->fused_combine && !c->hc && !(q4k && !kd.r_dn) && !split && !v2;  // the HC write-back belongs to the ordered combine
+  if (cap) {
+    // what the streaming launches do not take (shapes, alignments) goes to the 128-pair kernels after all
+    int pre = gemm_up(true, false, c->tiles, c->ntiles, 0, st);
+    if (!pre) pre = gemm_dn(true, false, c->tiles, c->ntiles, 0, st, nullptr);
+    if (!pre && L.has_shared && !split) pre = gemm_up(true, true, c->tiles, c->ntiles, 0, st);
+    if (!pre && L.has_shared && !split) pre = gemm_dn(true, true, c->tiles, c->ntiles, 0, st, nullptr);
+    if (pre) {
+      cap = 0;
+      split = shd || (q4k && !kd.uniform(L));
+      xl = batch_x16_layout(L, g);
+    }
+  }
+  const int tile_cap = cap ? cap : moe_gemm_tile_cap();
   // middle sizes: the router's column-split launches (router_split.hip); its first launch makes the f16 copy of x as well
   const bool mid_router = c->router_cand && c->gpart && moe_router_split_supported(&L.router, L.has_shared ? &L.sh_sg : nullptr, P, g.topk);
   // The shared expert in launches of its own, on the context's side stream: where its kernels differ from the routed
@@ -1161,14 +1234,14 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
     int pre = MOE_OK;
     if (aside) {
       if (L.has_shared) {
-        pre = gemm_up(true, c->tiles_sh, c->ntiles_sh, 0, st);
-        if (!pre) pre = gemm_dn(true, c->tiles_sh, c->ntiles_sh, 0, st, nullptr);
+        pre = gemm_up(false, true, c->tiles_sh, c->ntiles_sh, 0, st);
+        if (!pre) pre = gemm_dn(false, true, c->tiles_sh, c->ntiles_sh, 0, st, nullptr);
       }
-      if (!pre) pre = gemm_up(false, c->tiles, c->ntiles, 0, st);
-      if (!pre) pre = gemm_dn(false, c->tiles, c->ntiles, 0, st, nullptr);
+      if (!pre) pre = gemm_up(true, false, c->tiles, c->ntiles, 0, st);
+      if (!pre) pre = gemm_dn(true, false, c->tiles, c->ntiles, 0, st, nullptr);
     } else {
-      pre = gemm_up(L.has_shared, c->tiles, c->ntiles, 0, st);
-      if (!pre) pre = gemm_dn(L.has_shared, c->tiles, c->ntiles, 0, st, fused ? &cmb0 : nullptr);
+      pre = gemm_up(true, L.has_shared, c->tiles, c->ntiles, 0, st);
+      if (!pre) pre = gemm_dn(true, L.has_shared, c->tiles, c->ntiles, 0, st, fused ? &cmb0 : nullptr);
     }
     if (pre) return pre;  // nothing has been enqueued
     dry = false;
@@ -1178,7 +1251,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   prof_mark(c, 0, st);
   const int sh_first = P * g.topk;  // the shared expert's pair rows follow the routed ones
   const bool sh_in = L.has_shared && !aside;  // ... and its tiles the routed tiles, where it rides along
-  const int max_tiles = (P * g.topk + 127) / 128 + g.experts + (sh_in ? (P + 127) / 128 : 0);
+  const int max_tiles = (P * g.topk + tile_cap - 1) / tile_cap + g.experts + (sh_in ? (P + tile_cap - 1) / tile_cap : 0);
   // what else is needed from x: f16 copy, mean square (range guard), the shared expert's gate logit
   moe_row_extras ex{};
   ex.x16 = c->x16_ext ? nullptr : c->x16;
@@ -1211,8 +1284,8 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
     if (!rs && ee != hipSuccess) rs = (int)ee;
     if (L.has_shared) {
       if (!rs) rs = moe_launch_tiles_only_shared(c->tiles_sh, c->ntiles_sh, g.experts, moe_gemm_tile_cap(), P, sh_first, c->tokidx, c->side);
-      if (!rs) rs = gemm_up(true, c->tiles_sh, c->ntiles_sh, (P + 127) / 128, c->side);
-      if (!rs) rs = gemm_dn(true, c->tiles_sh, c->ntiles_sh, (P + 127) / 128, c->side, nullptr);
+      if (!rs) rs = gemm_up(false, true, c->tiles_sh, c->ntiles_sh, (P + 127) / 128, c->side);
+      if (!rs) rs = gemm_dn(false, true, c->tiles_sh, c->ntiles_sh, (P + 127) / 128, c->side, nullptr);
     }
   }
   // caller's stream: router, top-k, permutation, the routed experts' GEMMs
@@ -1224,17 +1297,17 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   prof_mark(c, MOE_PROF_ROUTER, st);
   if (!rc)
     rc = moe_launch_route(moe_routing_blockcnt(c->routing), c->ids, c->ws, c->tokidx, c->pw, c->eoff, c->pairids, P, g.topk, g.experts, g.id_stride, c->tiles,
-                          c->ntiles, moe_gemm_tile_cap(), sh_in ? sh_first : -1, st);
+                          c->ntiles, tile_cap, sh_in ? sh_first : -1, st);
   if (!rc && fused) rc = moe_launch_zero_f32(y, (uint64_t)P * g.d, st);
   if (aside) {
     const hipError_t ee = hipStreamWaitEvent(st, c->ev_x16, 0);
     if (!rc && ee != hipSuccess) rc = (int)ee;
   }
   prof_mark(c, MOE_PROF_ROUTE, st);
-  if (!rc && !rs) rc = gemm_up(sh_in, c->tiles, c->ntiles, max_tiles, st);
+  if (!rc && !rs) rc = gemm_up(true, sh_in, c->tiles, c->ntiles, max_tiles, st);
   prof_mark(c, MOE_PROF_UP, st);
   const moe_comb cmb{y, c->tokidx, c->pw, L.has_shared ? c->sh_logit : nullptr};
-  if (!rc && !rs) rc = gemm_dn(sh_in, c->tiles, c->ntiles, max_tiles, st, fused ? &cmb : nullptr);
+  if (!rc && !rs) rc = gemm_dn(true, sh_in, c->tiles, c->ntiles, max_tiles, st, fused ? &cmb : nullptr);
   if (aside) {  // the side stream is joined on every path out of here (a capture on `st` must not end with it forked)
     hipError_t ee = hipEventRecord(c->ev_join, c->side);
     if (ee == hipSuccess) ee = hipStreamWaitEvent(st, c->ev_join, 0);

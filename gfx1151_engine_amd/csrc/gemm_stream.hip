@@ -1,0 +1,794 @@
+// Grouped expert GEMM for tiles of few pairs: the weights stream from memory straight into registers.
+// (same contract as gemm_q4cp.hip: src/gpu/parts/27_kernels_moe_lut.inc:660-821, 26_kernels_moe_gguf.inc:456-485)
+//
+// From a few dozen to about two thousand tokens every expert is read and none has many pairs: what bounds a launch is the
+// experts' bytes (1.4 / 0.7 GB per layer for gate/up / down).  gemm_q4cp.hip, made for 128-pair tiles, moves them through
+// LDS in 32-byte pieces of 256 rows, two 64-column stages ahead, and reaches 3.5 TB/s of the 6.3 that plain loads reach
+// on this chip (a load of 16 rows x 64 bytes per wave instruction, four or more in flight per wave; 32 rows x 32 bytes:
+// 4.4 .. 5.3).  Here:
+//   - a wave owns 16 weight rows twice (gate/up: 16 gate rows and their 16 up rows; down: 32 rows) and walks K in lines of
+//     256 columns.  v_mfma_f32_16x16x32_f16 takes the weights as A: lane (n, g) = row n, 16-byte chunks g and g + 4 of
+//     the line's 128 code bytes, so a load instruction covers 64 contiguous bytes of 16 rows and a chunk is one lane's
+//     operand for four MFMAs.  Which columns a lane group multiplies is free as long as the activations agree; a chunk
+//     is one scale group of 32 columns (q4cp), half of a 64-column run (Q4_K, Q5_K), a lane group's run (Q8_0).
+//   - gate/up keeps two lines per wave in flight, line by line; down, whose rows are three lines, requests a fragment's
+//     whole rows at once.  Rows start 64 bytes off the 128-byte cache lines (the codebook heads the tensor), so every line
+//     shares a cache line with the next one, and read a line at a time a third of the traffic is fetched twice (1.66 GB for
+//     1.26, at 6.15 TB/s); whole rows brought down from 6.9 to 5.3 M cache lines (of 5.0).  For gate/up the same, pairs of
+//     lines with four in registers, fetched 1.51 GB and was no faster (270 us either way, three waves per SIMD for four).
+//   - activations (16 pairs per MFMA, up to 64 per tile) go through LDS: gate/up one line at a time, double-buffered, one
+//     LDS-only barrier per line; down, where they are short, once per block, which then runs without barriers.
+//   - no branch stands around a load of the loops: the compiler counts outstanding loads exactly only along straight code
+//     (with branches every wait drained the pipeline: 332 against 270 us).
+// The weights' f16 values are those of gemm_q4cp.hip bit for bit; the sums run over the same columns in f32.
+// Pairs per tile: 16, 32 or 64 by the batch's average (moe_stream_tile_cap): a block's work is the weights whatever the
+// tile holds, so tiles should hold an expert's pairs as a rule, and larger ones cost LDS and registers.
+// Measured (512 experts, top-10, 3072 x 768, gate/up + down, us; in brackets the 128-pair kernels):
+//   130 tokens q4cp 270 + 137 (368 + 185)      48 table 208 + 110 (295 + 177)    515 Q4_K 356 + 176 (413 + 241)
+//   200 Q5_K / Q8_0 407 + 291 (501 + 471)     200 i4r 260 + 143 (338 + 190)      2048 q4cp 392 + 219 (437 + 238)
+#include <type_traits>
+
+#include "common.h"
+#include "hv2.h"
+#include "internal.h"
+
+namespace {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+// F_DN: affine q4cp codebooks whose experts all have a power of two for the scaled dequantisation (gemm_q4cp.hip, DN)
+enum { F_DN, F_AFF, F_TAB, F_I4R, F_Q4K, F_Q5K, F_Q80 };
+constexpr bool scale_plane(int FMT) { return FMT <= F_I4R; }
+// order of activations and hid (moe_f32_to_f16's layouts)
+constexpr int x_layout(int FMT) { return FMT == F_TAB ? 0 : FMT <= F_I4R ? 1 : 2; }
+
+constexpr int XROW = 512;  // bytes of a line of one pair row (256 f16)
+// copies of a pair table: lanes eight apart share one; gate/up with 64 pairs: four, so that two blocks fit a CU's LDS
+constexpr int tab_copies(bool UP, int MFX) { return UP && MFX == 4 ? 4 : 8; }
+
+struct SW {
+  const uint8_t *w, *w_up, *sc, *sc_up;
+  const float *cb, *cb_up;
+  int sstride, e_rows, up_off;
+  const int8_t* pexp;
+};
+
+union H8 {
+  half8 v;
+  uint32_t u[4];
+  half2v h[4];
+};
+__device__ __forceinline__ half2v h2(uint32_t u) {
+  union { uint32_t u; half2v h; } c;
+  c.u = u;
+  return c.h;
+}
+__device__ __forceinline__ uint32_t u2(half2v h) {
+  union { half2v h; uint32_t u; } c;
+  c.h = h;
+  return c.u;
+}
+__device__ __forceinline__ half2v both(float f) { return half2v{(_Float16)f, (_Float16)f}; }
+
+template <int FMT>
+__device__ __forceinline__ uint32_t row_bytes(int K) {
+  return FMT == F_Q4K ? K / 256 * 144 : FMT == F_Q5K ? K / 256 * 176 : FMT == F_Q80 ? K / 32 * 34 : K / 2;
+}
+constexpr int line_bytes(int FMT) { return FMT == F_Q4K ? 144 : FMT == F_Q5K ? 176 : FMT == F_Q80 ? 272 : 128; }
+
+// element of a group of 16 NW rows that output position 16 wv + i holds: the order the down launch reads hid in (layout 2
+// runs over 64-element blocks, four waves' groups)
+template <int LAYOUT>
+__device__ __forceinline__ int pos_elem(int wv, int i) {
+  if (LAYOUT == 1) return 16 * wv + (i & 8) + (((i & 1) << 2) | ((i & 7) >> 1));
+  if (LAYOUT == 2) {
+    const int p = 16 * (wv & 3) + i, w = p >> 3, r = p & 7;
+    return 64 * (wv >> 2) + 4 * w + ((r & 2) << 4) + ((r & 1) << 1) + (r >> 2);
+  }
+  return 16 * wv + i;
+}
+
+// ---- one line of one weight fragment (16 rows) in registers ----
+template <int FMT>
+struct Line {
+  uint4 c[FMT == F_Q80 ? 4 : 2];  // codes
+  uint4 hd[1], qh[1];             // K-quants: block header; Q5_K: this lane's fifth bits
+  uint32_t last;                  // Q8_0: the 17th word
+};
+// b: wave-uniform address of the line's first row, o: this lane's row offset, half: the second half does not exist
+template <int FMT>
+__device__ __forceinline__ void load_line(Line<FMT>& q, const uint8_t* b, uint32_t o, int g, bool half) {
+  if constexpr (FMT == F_Q80) {
+    // lane group g = columns 64 g .. of the line: two blocks, 68 bytes (4-byte aligned)
+    const uint8_t* s = b + (o + 68u * (half ? (uint32_t)(g & 1) : (uint32_t)g));
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t* d = (const uint32_t*)(s + 16 * k);
+      q.c[k] = make_uint4(d[0], d[1], d[2], d[3]);
+    }
+    q.last = *(const uint32_t*)(s + 64);
+  } else {
+    constexpr uint32_t C0 = FMT == F_Q4K ? 16 : FMT == F_Q5K ? 48 : 0;
+    if (FMT == F_Q4K || FMT == F_Q5K) q.hd[0] = *(const uint4*)(b + o);
+    if (FMT == F_Q5K) q.qh[0] = *(const uint4*)(b + (o + 16u + 16u * (uint32_t)(g & 1)));
+    q.c[0] = *(const uint4*)(b + (o + C0 + 16u * (uint32_t)g));
+    const uint8_t* b1 = b + (half ? 0 : 64);
+    q.c[1] = *(const uint4*)(b1 + (o + C0 + 16u * (uint32_t)g));
+  }
+}
+
+// What dequantisation needs beside the codes: per fragment the codebook's slope and offset or its pair table
+struct Consts {
+  float cb_a[2], cb_b[2];
+  const uint8_t* tabs;  // LDS
+  uint32_t tabo[2];
+  uint32_t selb;        // K-quants: this lane's two sub-blocks of four
+  int g;
+};
+
+// acc[f][mf] += line of fragment f x the line's activations.  f0: fragment 0's index into the constants; sw: this lane's two
+// scales of the line (scale planes); xb: the activations' line in LDS; xa: this lane's operand addresses of four steps
+// (Q8_0: eight)
+template <int FMT, int F, int MF, int XP, int TABC>
+__device__ __forceinline__ void line_mma(const Line<FMT> (&q)[F], const uint32_t (&sw)[F], const Consts& C, int f0,
+                                         const uint8_t* xb, const uint32_t* xa, bool half, floatx4 (&acc)[F][MF]) {
+  auto mma = [&](uint32_t xo, const H8 (&w)[F]) {
+#pragma unroll
+    for (int mf = 0; mf < MF; mf++) {
+      const half8 xf = *(const half8*)(xb + xo + 16 * mf * XP);
+#pragma unroll
+      for (int f = 0; f < F; f++) acc[f][mf] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[f].v, xf, acc[f][mf], 0, 0, 0);
+    }
+  };
+  if constexpr (FMT == F_Q80) {
+    half2v sc[F][2];
+    uint32_t cw[F][16];
+#pragma unroll
+    for (int f = 0; f < F; f++) {
+      const uint32_t w[17] = {q[f].c[0].x, q[f].c[0].y, q[f].c[0].z, q[f].c[0].w, q[f].c[1].x, q[f].c[1].y, q[f].c[1].z, q[f].c[1].w,
+                              q[f].c[2].x, q[f].c[2].y, q[f].c[2].z, q[f].c[2].w, q[f].c[3].x, q[f].c[3].y, q[f].c[3].z, q[f].c[3].w,
+                              q[f].last};
+      // bytes 0-1 the first block's scale, 2-33 its codes, 34-35 the second's scale, 36-67 its codes
+      sc[f][0] = h2(__builtin_amdgcn_perm(w[0], w[0], 0x01000100u));
+      sc[f][1] = h2(__builtin_amdgcn_perm(w[8], w[8], 0x03020302u));
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        cw[f][k] = __builtin_amdgcn_alignbyte(w[k + 1], w[k], 2) ^ 0x80808080u;
+        cw[f][8 + k] = w[9 + k] ^ 0x80808080u;
+      }
+      if (half && C.g >= 2) {  // (runs past K)
+        sc[f][0] = sc[f][1] = both(0.f);
+      }
+    }
+    // layout 2: chunk w of a run = columns 4w, 4w+2, 32+4w, 32+4w+2, 4w+1, 4w+3, 32+4w+1, 32+4w+3
+    const half2v k1152 = both(1152.f);  // 1024 + u with u = code + 128
+#pragma unroll
+    for (int w = 0; w < 8; w++) {
+      H8 a[F];
+#pragma unroll
+      for (int f = 0; f < F; f++) {
+        const uint32_t lo = cw[f][w], hi = cw[f][8 + w];
+        a[f].h[0] = (h2(__builtin_amdgcn_perm(0x64646464u, lo, 0x04020400u)) - k1152) * sc[f][0];
+        a[f].h[1] = (h2(__builtin_amdgcn_perm(0x64646464u, hi, 0x04020400u)) - k1152) * sc[f][1];
+        a[f].h[2] = (h2(__builtin_amdgcn_perm(0x64646464u, lo, 0x04030401u)) - k1152) * sc[f][0];
+        a[f].h[3] = (h2(__builtin_amdgcn_perm(0x64646464u, hi, 0x04030401u)) - k1152) * sc[f][1];
+      }
+      mma(xa[w], a);
+    }
+    return;
+  } else {
+    auto part = [&](auto ec) {
+      constexpr int E_ = decltype(ec)::value;
+      half2v as[F][2], bs[F][2];
+#pragma unroll
+      for (int f = 0; f < F; f++) {
+        if (FMT == F_Q4K || FMT == F_Q5K) {
+          // 6-bit (scale, min) fields of sub-blocks 0-3 (E_ = 0) or 4-7 as bytes, gguf scale_min_k4; d * sc and dmin * m as
+          // packed f16 products of exact integers
+          const uint4 hd = q[f].hd[0];
+          const uint32_t sc = E_ ? (hd.w & 0x0f0f0f0fu) | ((hd.y >> 2) & 0x30303030u) : hd.y & 0x3f3f3f3fu;
+          const uint32_t mn = E_ ? ((hd.w >> 4) & 0x0f0f0f0fu) | ((hd.z >> 2) & 0x30303030u) : hd.z & 0x3f3f3f3fu;
+          const half2v dd = h2(__builtin_amdgcn_perm(hd.x, hd.x, 0x01000100u));
+          const half2v dm = h2(__builtin_amdgcn_perm(hd.x, hd.x, 0x03020302u) ^ 0x80008000u);
+          const half2v k1024 = both(1024.f);
+          const half2v a = (h2(__builtin_amdgcn_perm(0x64646464u, sc, C.selb)) - k1024) * dd;
+          const half2v b = (h2(__builtin_amdgcn_perm(0x64646464u, mn, C.selb)) - k1024) * dm;
+          as[f][0] = half2v{a.x, a.x}; as[f][1] = half2v{a.y, a.y};
+          bs[f][0] = half2v{b.x, b.x}; bs[f][1] = half2v{b.y, b.y};
+        } else {
+          const half2v s2 = h2(sw[f]);
+          const _Float16 sh = E_ ? s2.y : s2.x;
+          if (FMT == F_TAB) {
+            as[f][0] = half2v{sh, sh};
+          } else {
+            const float s = (float)sh;
+            as[f][0] = both(C.cb_a[f0 + f] * s);
+            bs[f][0] = bs[f][1] = both(C.cb_b[f0 + f] * s);
+            as[f][1] = FMT == F_DN ? as[f][0] * both(0.0625f) : as[f][0];
+          }
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        H8 a[F];
+#pragma unroll
+        for (int f = 0; f < F; f++) {
+          const uint4 cq = q[f].c[E_];
+          const uint32_t w = s == 0 ? cq.x : s == 1 ? cq.y : s == 2 ? cq.z : cq.w;
+          if (FMT == F_TAB) {
+            // one look-up gives a code byte's two weights before scaling
+#pragma unroll
+            for (int b = 0; b < 4; b++)
+              a[f].h[b] = h2(*(const uint32_t*)(C.tabs + (((w >> (8 * b)) & 0xffu) * (4u * TABC) + C.tabo[f0 + f]))) * as[f][0];
+            continue;
+          }
+          const uint32_t w8 = w >> 8;
+          if (FMT == F_DN) {  // codes read as f16 denormals
+            a[f].h[0] = h2(w & 0x000f000fu) * as[f][0] + bs[f][0];
+            a[f].h[1] = h2(w & 0x00f000f0u) * as[f][1] + bs[f][0];
+            a[f].h[2] = h2(w8 & 0x000f000fu) * as[f][0] + bs[f][0];
+            a[f].h[3] = h2(w8 & 0x00f000f0u) * as[f][1] + bs[f][0];
+          } else {  // 0x6400 | n is the f16 1024 + n, 0x5400 | n << 4 is 64 + n
+            uint32_t t0 = (w & 0x000f000fu) | 0x64006400u, t1 = (w & 0x00f000f0u) | 0x54005400u;
+            uint32_t t2 = (w8 & 0x000f000fu) | 0x64006400u, t3 = (w8 & 0x00f000f0u) | 0x54005400u;
+            if (FMT == F_Q5K) {
+              // fifth bits: bit 2 jj (low nibbles) and 2 jj + 1 (high) of the qh byte, jj = g / 2 + 2 E_
+              const uint4 qq = q[f].qh[0];
+              const uint32_t qw = s == 0 ? qq.x : s == 1 ? qq.y : s == 2 ? qq.z : qq.w;
+              const uint32_t r = __builtin_amdgcn_alignbit(qw, qw, (uint32_t)((C.g & 2) + 4 * E_));
+              t0 |= (r << 4) & 0x00100010u;
+              t1 |= (r << 7) & 0x01000100u;
+              t2 |= (r >> 4) & 0x00100010u;
+              t3 |= (r >> 1) & 0x01000100u;
+            }
+            const half2v k1024 = both(1024.f), k64 = both(64.f);
+            a[f].h[0] = (h2(t0) - k1024) * as[f][0] + bs[f][0];
+            a[f].h[1] = (h2(t1) - k64) * as[f][1] + bs[f][1];
+            a[f].h[2] = (h2(t2) - k1024) * as[f][0] + bs[f][0];
+            a[f].h[3] = (h2(t3) - k64) * as[f][1] + bs[f][1];
+          }
+        }
+        mma(xa[s] + E_ * 256, a);
+      }
+    };
+    part(std::integral_constant<int, 0>{});
+    if (!half) part(std::integral_constant<int, 1>{});
+  }
+}
+
+// Scales of four lines of a row (64 bytes, i4r: 16) from line 4 qd on: lane group i fetches line i's, the exchange below
+// then hands every lane one word per line with its own two scales.  (Past the row's end: one address for all lanes.)
+template <int FMT>
+struct Raw { uint4 v; };
+template <int FMT>
+__device__ __forceinline__ Raw<FMT> load_scales(const uint8_t* b, uint32_t o, int qd, int g, int sstride) {
+  Raw<FMT> r;
+  if (FMT == F_I4R) {  // one word per line: both scales, the same for all lane groups
+    const uint32_t p = 4u * (uint32_t)(4 * qd + g);
+    r.v.x = *(const uint32_t*)(b + (p < (uint32_t)sstride ? o + p : 0u));
+  } else {
+    const uint32_t p = 16u * (uint32_t)(4 * qd + g);
+    r.v = *(const uint4*)(b + (p < (uint32_t)sstride ? o + p : 0u));
+  }
+  return r;
+}
+template <int FMT>
+__device__ __forceinline__ void take_scales(const Raw<FMT>& r, uint32_t (&sq)[4]) {
+  uint32_t p0 = r.v.x, p1 = p0, p2 = p0, p3 = p0;
+  if (FMT != F_I4R) {  // word k: (scale k, scale 4 + k), lane group k's chunks k and k + 4
+    p0 = __builtin_amdgcn_perm(r.v.z, r.v.x, 0x05040100u); p1 = __builtin_amdgcn_perm(r.v.z, r.v.x, 0x07060302u);
+    p2 = __builtin_amdgcn_perm(r.v.w, r.v.y, 0x05040100u); p3 = __builtin_amdgcn_perm(r.v.w, r.v.y, 0x07060302u);
+  }
+  // 4 x 4 transposition between lane groups and words
+  auto a = __builtin_amdgcn_permlane32_swap(p0, p2, false, false);
+  auto b = __builtin_amdgcn_permlane32_swap(p1, p3, false, false);
+  auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  sq[0] = c[0]; sq[1] = c[1]; sq[2] = d[0]; sq[3] = d[1];
+}
+
+template <int FMT, bool UP, int NT, int TABC>
+__device__ __forceinline__ Consts make_consts(const SW& L, int pexp, uint8_t* tabs, int tid, float& oscale) {
+  Consts C;
+  C.g = (tid & 63) >> 4;
+  C.selb = (C.g & 2) ? 0x04030402u : 0x04010400u;
+  C.cb_a[0] = C.cb_a[1] = 1.f;
+  C.cb_b[0] = C.cb_b[1] = -8.f;  // (i4r)
+  C.tabs = tabs;
+  C.tabo[0] = C.tabo[1] = 0u;
+  oscale = 1.f;
+  if (FMT == F_AFF || FMT == F_DN) {
+    C.cb_a[0] = L.cb[1] - L.cb[0]; C.cb_b[0] = L.cb[0];
+    C.cb_a[1] = UP ? L.cb_up[1] - L.cb_up[0] : C.cb_a[0]; C.cb_b[1] = UP ? L.cb_up[0] : C.cb_b[0];
+    if (FMT == F_DN) {  // in units of 2^pexp; slopes for codes read as f16 denormals
+      const float s24 = __builtin_ldexpf(1.f, 24 + pexp), sp = __builtin_ldexpf(1.f, pexp);
+      C.cb_a[0] *= s24; C.cb_a[1] *= s24; C.cb_b[0] *= sp; C.cb_b[1] *= sp;
+      oscale = __builtin_ldexpf(1.f, -pexp);
+    }
+  } else if (FMT == F_TAB) {
+    // TABC copies side by side: lanes that differ in their low bits never meet on a bank (with one copy the look-ups of a
+    // wave run into 3.5-way conflicts on average)
+    const bool two = UP && L.cb_up != L.cb;
+    for (int i = tid; i < 256 * TABC; i += NT) {
+      const int b = i / TABC;
+      ((uint32_t*)tabs)[i] = u2(half2v{(_Float16)L.cb[b & 15], (_Float16)L.cb[b >> 4]});
+      if (two) ((uint32_t*)tabs)[256 * TABC + i] = u2(half2v{(_Float16)L.cb_up[b & 15], (_Float16)L.cb_up[b >> 4]});
+    }
+    C.tabo[0] = (uint32_t)(tid & (TABC - 1)) * 4u;
+    C.tabo[1] = C.tabo[0] + (two ? 256u * TABC * 4u : 0u);
+  }
+  return C;
+}
+
+// this lane's operand address of step q: 16-byte chunk 16 e + 4 g + q of pair row n, XORed with the row against bank conflicts
+// (Q8_0: lane group g walks its run of 64 columns, chunks 8 g + w)
+template <int FMT, int XP>
+__device__ __forceinline__ void x_addrs(int n, int g, uint32_t (&xa)[8]) {
+#pragma unroll
+  for (int q = 0; q < 8; q++) xa[q] = (uint32_t)(n * XP + ((((FMT == F_Q80 ? 8 : 4) * g + q) ^ n) << 4));
+}
+
+// ---- gate/up ----
+// (The columns of a down launch that fits are whole pairs of lines here.  Said to the compiler, so that two lines become one
+// straight block without the checks below, it moves loads and operands further, spills and loses 20 us of 390 at 64 pairs.)
+// (Straight code of two lines, where K is known to be whole pairs of lines, gave the compiler room to move loads and operands
+// further and cost 20 us of 390 at 64 pairs (spills: up to 150): the branches around half and last lines stay.)
+template <int FMT, int MFX, int MF, bool ROT, int NW>
+__device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const moe_tile tile, int nb, const __half* __restrict__ x,
+                                        const int* __restrict__ tokidx, __half* __restrict__ out, int M, int K, int pexp,
+                                        const moe_hscale& hs, moe_cmag cmag, const moe_rotv& rot) {
+  constexpr int LAYOUT = x_layout(FMT), LB = line_bytes(FMT), NT = 64 * NW, UPR = 16 * NW;
+  constexpr int XBUF = MFX * 16 * XROW;
+  constexpr int DB = 2;  // lines in registers: one ahead of the line worked on
+  float* const rowscale = (float*)(smem + 2 * XBUF);
+  uint8_t* const tabs = smem + 2 * XBUF + 256;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  const uint32_t RB = row_bytes<FMT>(K);
+  const int nline = (K + 255) >> 8;
+  const bool tail = (K & 128) != 0;  // the last line is half a line
+
+  int r = nb * UPR + pos_elem<LAYOUT>(wv, n);
+  r = r < M ? r : M - 1;  // (loaded, never stored)
+  const uint8_t* wb[2];   // wave-uniform: the expert's gate and up rows
+  const uint8_t* sb[2];
+#pragma unroll
+  for (int f = 0; f < 2; f++) {
+    const size_t first = (size_t)e * L.e_rows + (f ? L.up_off : 0);
+    wb[f] = (f ? L.w_up : L.w) + first * RB;
+    sb[f] = scale_plane(FMT) ? (f ? L.sc_up : L.sc) + first * (size_t)L.sstride : nullptr;
+  }
+  const uint32_t wo = (uint32_t)r * RB, so = (uint32_t)r * (uint32_t)L.sstride;
+  Line<FMT> ln[DB][2];
+  auto load = [&](Line<FMT>(&q)[2], int i) {
+#pragma unroll
+    for (int f = 0; f < 2; f++) {
+      const bool past = i >= nline;  // (wave-uniform; one address for all lanes instead of a branch around the load)
+      load_line<FMT>(q[f], wb[f] + (past ? (size_t)0 : (size_t)i * LB), past ? 0u : wo, past ? 0 : g, tail && i >= nline - 1);
+    }
+  };
+  // ---- the pipeline's first requests: weights before the tile's row indices are needed ----
+  Raw<FMT> raw[2];
+  uint32_t sq[2][4];
+  if (scale_plane(FMT)) {
+#pragma unroll
+    for (int f = 0; f < 2; f++) raw[f] = load_scales<FMT>(sb[f], so, 0, g, L.sstride);
+  }
+#pragma unroll
+  for (int b = 0; b < DB; b++) load(ln[b], b);
+  // ---- activations: thread = 16-byte piece tid % 32 of pair rows tid / 32 + (NT / 32) l ----
+  // (rows past the tile's pairs repeat its first one: no branch around a load, and the lines are in L1)
+  constexpr int XL = MF * 16 * 32 / NT, XS = NT / 32;  // loads per thread and line, rows per load
+  static_assert(XL >= 1 && XL <= 4, "named registers below");
+  const int xc = tid & 31, xt = tid >> 5;
+  const __half* xr[XL];
+#pragma unroll
+  for (int l = 0; l < XL; l++) {
+    const int m = XS * l + xt;
+    const int row = tokidx[tile.first + (m < tile.count ? m : 0)];
+    xr[l] = x + (size_t)row * K + 8 * xc;
+    if (xc == 0) rowscale[m] = hs.xms ? moe_hid_scale(cmag, hs.xms[row]) : 1.f;
+  }
+  uint4 xv0, xv1, xv2, xv3;  // (named: an array here ends up in scratch memory)
+  auto fetch_x = [&](int i) {
+    i = i < nline ? i : nline - 1;
+    const bool half = tail && i == nline - 1;
+    const int o = i * 256 - (half && xc >= 16 ? 128 : 0);
+    xv0 = *(const uint4*)(xr[0] + o);
+    if constexpr (XL > 1) xv1 = *(const uint4*)(xr[1] + o);
+    if constexpr (XL > 2) xv2 = *(const uint4*)(xr[2] + o);
+    if constexpr (XL > 3) xv3 = *(const uint4*)(xr[3] + o);
+  };
+  auto put_x = [&](int buf) {
+    auto put = [&](int l, const uint4& v) {
+      const int m = XS * l + xt;
+      *(uint4*)(smem + buf * XBUF + m * XROW + ((xc ^ (m & 15)) << 4)) = v;
+    };
+    put(0, xv0);
+    if constexpr (XL > 1) put(1, xv1);
+    if constexpr (XL > 2) put(2, xv2);
+    if constexpr (XL > 3) put(3, xv3);
+  };
+  fetch_x(0);
+  float oscale;
+  const Consts C = make_consts<FMT, true, NT, tab_copies(true, MFX)>(L, pexp, tabs, tid, oscale);
+  uint32_t xa[8];
+  x_addrs<FMT, XROW>(n, g, xa);
+  floatx4 acc[2][MF];
+#pragma unroll
+  for (int f = 0; f < 2; f++)
+#pragma unroll
+    for (int mf = 0; mf < MF; mf++) acc[f][mf] = floatx4{0.f, 0.f, 0.f, 0.f};
+  put_x(0);
+
+  // stage V (mod 4): line i
+  auto stage = [&](auto vc, int i) {
+    constexpr int V = decltype(vc)::value, B = V & 1;
+    moe_lds_barrier();  // this line's activations are in LDS; the other buffer has been read
+    fetch_x(i + 1);
+    const uint32_t sw[2] = {sq[0][V], sq[1][V]};
+    line_mma<FMT, 2, MF, XROW, tab_copies(true, MFX)>(ln[B], sw, C, 0, smem + B * XBUF, xa, tail && i == nline - 1, acc);
+    load(ln[B], i + DB);
+    put_x(B ^ 1);
+  };
+  for (int i = 0;; i += 4) {
+    if (scale_plane(FMT)) {
+#pragma unroll
+      for (int f = 0; f < 2; f++) {
+        take_scales<FMT>(raw[f], sq[f]);
+        raw[f] = load_scales<FMT>(sb[f], so, (i >> 2) + 1, g, L.sstride);
+      }
+    }
+    stage(std::integral_constant<int, 0>{}, i);
+    if (i + 1 >= nline) break;
+    stage(std::integral_constant<int, 1>{}, i + 1);
+    if (i + 2 >= nline) break;
+    stage(std::integral_constant<int, 2>{}, i + 2);
+    if (i + 3 >= nline) break;
+    stage(std::integral_constant<int, 3>{}, i + 3);
+    if (i + 4 >= nline) break;
+  }
+
+  if constexpr (ROT) {
+    // hgn v2: the slot-wise middle on the block's 128 gate and 128 up sums of every pair (gemm_q4cp.hip, ROT)
+    static_assert(UPR == 128, "whole 128-blocks");
+    constexpr int BP = 2 * UPR * 2 + 16;
+    static_assert(MFX * 16 * BP <= 2 * XBUF, "the row scales stay");
+    moe_lds_barrier();
+    uint8_t* const patch = smem;  // (over the activations, which every wave has read)
+#pragma unroll
+    for (int mf = 0; mf < MF; mf++)
+#pragma unroll
+      for (int f = 0; f < 2; f++)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++) {
+          const int c = pos_elem<LAYOUT>(wv, 4 * g + r4);
+          *(__half*)(patch + (16 * mf + n) * BP + f * UPR * 2 + c * 2) = __float2half(acc[f][mf][r4]);
+        }
+    __syncthreads();
+    const int j = tid & 15, c = nb * UPR + 8 * j;
+    float fg[8], fu[8], sd[8];
+    {
+      const int cc = c < M ? c : 0;
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        fg[k] = rot.svh_gu[cc + k];
+        fu[k] = rot.svh_gu[M + cc + k];
+        sd[k] = rot.suh_dn[cc + k];
+      }
+    }
+    for (int m = tid >> 4; m < 16 * MF; m += NT / 16) {
+      const uint4 gq = *(const uint4*)(patch + m * BP + j * 16), uq = *(const uint4*)(patch + m * BP + UPR * 2 + j * 16);
+      const __half2* gh = (const __half2*)&gq;
+      const __half2* uh = (const __half2*)&uq;
+      float gv8[8], uv8[8], hv[8];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const float2 a = __half22float2(gh[k]), b = __half22float2(uh[k]);
+        gv8[2 * k] = a.x; gv8[2 * k + 1] = a.y; uv8[2 * k] = b.x; uv8[2 * k + 1] = b.y;
+      }
+      moe_fwht128_r8(gv8, lane);
+      moe_fwht128_r8(uv8, lane);
+      const float rs = rowscale[m];
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const float gg = gv8[k] * MOE_RS128 * fg[k], uu = uv8[k] * MOE_RS128 * fu[k];
+        hv[k] = gg * __builtin_amdgcn_rcpf(1.f + __expf(-gg)) * uu * (sd[k] * rs);
+      }
+      moe_fwht128_r8(hv, lane);
+#pragma unroll
+      for (int k = 0; k < 8; k++) hv[k] *= MOE_RS128;
+      if (m < tile.count && c < M) moe_st8_f16_ilv(out + (size_t)(tile.first + m) * M + c, hv);
+    }
+  } else {
+    const int col = nb * UPR + 16 * wv + 4 * g;
+#pragma unroll
+    for (int mf = 0; mf < MF; mf++) {
+      const int m = 16 * mf + n;
+      if (m < tile.count && col < M) {
+        const float rs = rowscale[m];
+        float h4[4];
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++) {
+          const float gv = acc[0][mf][r4] * oscale, uv = acc[1][mf][r4] * oscale;
+          h4[r4] = gv * __builtin_amdgcn_rcpf(1.f + __expf(-gv)) * uv * rs;
+        }
+        const __half2 a = __floats2half2_rn(h4[0], h4[1]), b = __floats2half2_rn(h4[2], h4[3]);
+        *(uint2*)(out + (size_t)(tile.first + m) * M + col) = make_uint2(*(const uint32_t*)&a, *(const uint32_t*)&b);
+      }
+    }
+  }
+}
+
+// ---- down: rows of at most three lines.  The tile's hid rows lie in LDS for the whole block; a wave takes 32 rows at a time,
+// requests a fragment's whole rows at once (neighbouring rows share their boundary cache lines as well) and the next
+// rows' as soon as the fragment's are used up; no barrier after the first.  ----
+constexpr int DN_LINES = 3, DN_XP = DN_LINES * XROW;
+template <int FMT, int MFX, int MF, int NW>
+__device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const moe_tile tile, int nb, int npass,
+                                        const __half* __restrict__ x, __half* __restrict__ out, int M, int K, int pexp) {
+  constexpr int LB = line_bytes(FMT), NT = 64 * NW, DNR = 32 * NW;
+  uint8_t* const tabs = smem + MFX * 16 * DN_XP;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  const uint32_t RB = row_bytes<FMT>(K);
+  const bool tail = (K & 128) != 0;
+  const uint8_t* const wb = L.w + (size_t)e * L.e_rows * RB;
+  const uint8_t* const sb = scale_plane(FMT) ? L.sc + (size_t)e * L.e_rows * (size_t)L.sstride : nullptr;
+  // fragment f, MFMA row i = weight row 8 (i / 4) + 4 f + i % 4 of the wave's 32: a lane's eight results are neighbours
+  Line<FMT> ln[2][DN_LINES];
+  Raw<FMT> raw[2];
+  auto load = [&](int f, int p) {
+    p = p < npass ? p : npass - 1;  // (past the end: the last rows again)
+    const int row0 = (nb + p) * DNR + 32 * wv;
+    const int r = 8 * (n >> 2) + 4 * f + (n & 3);
+    if (scale_plane(FMT)) raw[f] = load_scales<FMT>(sb + (size_t)row0 * L.sstride, (uint32_t)r * (uint32_t)L.sstride, 0, g, L.sstride);
+#pragma unroll
+    for (int i = 0; i < DN_LINES; i++)
+      load_line<FMT>(ln[f][i], wb + ((size_t)row0 * RB + i * LB), (uint32_t)r * RB, g, tail && i == DN_LINES - 1);
+  };
+  load(0, 0);
+  load(1, 0);
+  for (int c = tid; c < 16 * MF * (DN_XP / 16); c += NT) {
+    const int m = c / (DN_XP / 16), k = c % (DN_XP / 16);
+    const int kk = 8 * k < K ? k : 0;  // (a half line's second half: never multiplied)
+    const uint4 v = *(const uint4*)(x + (size_t)(tile.first + (m < tile.count ? m : 0)) * K + 8 * kk);
+    *(uint4*)(smem + m * DN_XP + ((k ^ (m & 15)) << 4)) = v;
+  }
+  float oscale;
+  const Consts C = make_consts<FMT, false, NT, tab_copies(false, MFX)>(L, pexp, tabs, tid, oscale);
+  uint32_t xa[8];
+  x_addrs<FMT, DN_XP>(n, g, xa);
+  moe_lds_barrier();
+  for (int p = 0; p < npass; p++) {
+    floatx4 acc[2][MF];
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+#pragma unroll
+      for (int mf = 0; mf < MF; mf++) acc[f][mf] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (MFX < 4) {
+#pragma unroll
+      for (int f = 0; f < 2; f++) {
+        asm volatile("" ::: "memory");  // (the activations are the same for all rows: hoisted out of the loop they would fill the registers)
+        uint32_t sq[4] = {0u, 0u, 0u, 0u};
+        if (scale_plane(FMT)) take_scales<FMT>(raw[f], sq);
+        floatx4 a1[1][MF];
+#pragma unroll
+        for (int mf = 0; mf < MF; mf++) a1[0][mf] = acc[f][mf];
+#pragma unroll
+        for (int i = 0; i < DN_LINES; i++) {
+          const Line<FMT> q1[1] = {ln[f][i]};
+          const uint32_t sw[1] = {sq[i]};
+          line_mma<FMT, 1, MF, DN_XP, tab_copies(false, MFX)>(q1, sw, C, 0, smem + i * XROW, xa, tail && i == DN_LINES - 1, a1);
+        }
+#pragma unroll
+        for (int mf = 0; mf < MF; mf++) acc[f][mf] = a1[0][mf];
+        load(f, p + 1);
+      }
+    } else {  // (64 pairs: both fragments share an activation operand's trip out of LDS)
+      asm volatile("" ::: "memory");
+      uint32_t sq[2][4];
+      if (scale_plane(FMT)) {
+#pragma unroll
+        for (int f = 0; f < 2; f++) take_scales<FMT>(raw[f], sq[f]);
+      }
+#pragma unroll
+      for (int i = 0; i < DN_LINES; i++) {
+        const Line<FMT> q2[2] = {ln[0][i], ln[1][i]};
+        const uint32_t sw[2] = {sq[0][i], sq[1][i]};
+        line_mma<FMT, 2, MF, DN_XP, tab_copies(false, MFX)>(q2, sw, C, 0, smem + i * XROW, xa, tail && i == DN_LINES - 1, acc);
+      }
+      load(0, p + 1);
+      load(1, p + 1);
+    }
+    const int col = (nb + p) * DNR + 32 * wv + 8 * g;
+#pragma unroll
+    for (int mf = 0; mf < MF; mf++) {
+      const int m = 16 * mf + n;
+      if (m < tile.count) {
+        uint4 o;
+        __half2 h[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) h[k] = __floats2half2_rn(oscale * acc[k >> 1][mf][2 * (k & 1)], oscale * acc[k >> 1][mf][2 * (k & 1) + 1]);
+        o.x = *(uint32_t*)&h[0]; o.y = *(uint32_t*)&h[1]; o.z = *(uint32_t*)&h[2]; o.w = *(uint32_t*)&h[3];
+        *(uint4*)(out + (size_t)(tile.first + m) * M + col) = o;
+      }
+    }
+  }
+}
+
+// Waves of a block.  Four: several blocks to a CU pass their prologues, barriers and epilogues independently.  Eight for
+// rotated experts, whose epilogue works on 128 rows, and where 64 pairs' activations fill the LDS (down: sixteen).
+constexpr int block_waves(int FMT, bool UP, int MFX) { return MFX == 4 ? (UP ? 8 : 16) : UP && FMT == F_I4R ? 8 : 4; }
+// waves per SIMD asked for: what the registers of the lines in flight leave
+constexpr int simd_waves(int FMT, bool UP, int MFX) {
+  if (UP) return 4;
+  return MFX == 4 ? 4 : FMT == F_Q80 || FMT == F_Q4K ? 3 : 4;
+}
+constexpr size_t smem_bytes(int FMT, bool UP, int MFX) {
+  const size_t tab = FMT == F_TAB ? (size_t)(UP ? 2 : 1) * 256 * tab_copies(UP, MFX) * 4 : 0;
+  return UP ? (size_t)2 * MFX * 16 * XROW + 256 + tab : (size_t)MFX * 16 * DN_XP + tab;
+}
+
+template <int FMT, bool UP, int MFX>
+__global__ void __launch_bounds__(64 * block_waves(FMT, UP, MFX), simd_waves(FMT, UP, MFX))
+k_moe_stream(SW R, SW Sh, int n_experts, const __half* __restrict__ x, const int* __restrict__ tokidx,
+             const moe_tile* __restrict__ tiles, const int* __restrict__ ntiles, __half* __restrict__ out, int M, int K,
+             int nblk_n, int split, int npass, moe_hscale hs, moe_rotv rot) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  constexpr int NW = block_waves(FMT, UP, MFX);
+  // XCD-aware order as in gemm_q4cp.hip: consecutive workgroup ids go round-robin over the XCDs; each takes a contiguous
+  // run of tiles, routed and shared ones dealt separately
+  const int nt = ntiles[0], nr = split ? ntiles[1] : nt;
+  const int wg = blockIdx.x, xcd = wg & 7, j = wg >> 3;
+  const int per_r = (nr + 7) >> 3, per_s = (nt - nr + 7) >> 3;
+  const int tl = j / nblk_n, nb = (j - tl * nblk_n) * npass;
+  int ti;
+  if (tl < per_r) {
+    ti = xcd * per_r + tl;
+    if (ti >= nr) return;
+  } else {
+    const int k2 = tl - per_r;
+    ti = nr + xcd * per_s + k2;
+    if (k2 >= per_s || ti >= nt) return;
+  }
+  const moe_tile tile = tiles[ti];
+  const bool shared = tile.expert >= n_experts;
+  SW L;
+  L.w = shared ? Sh.w : R.w;
+  L.w_up = shared ? Sh.w_up : R.w_up;
+  L.sc = shared ? Sh.sc : R.sc;
+  L.sc_up = shared ? Sh.sc_up : R.sc_up;
+  L.cb = shared ? Sh.cb : R.cb;
+  L.cb_up = shared ? Sh.cb_up : R.cb_up;
+  L.sstride = shared ? Sh.sstride : R.sstride;
+  L.e_rows = shared ? Sh.e_rows : R.e_rows;
+  L.up_off = shared ? Sh.up_off : R.up_off;
+  L.pexp = shared ? Sh.pexp : R.pexp;
+  const int e = shared ? 0 : tile.expert;
+  const int pexp = FMT == F_DN ? (int)L.pexp[e] : 0;
+  const moe_cmag cmag = shared ? hs.c_shared : hs.c_routed;
+  const int mfn = (tile.count + 15) >> 4;
+#define ST_GO(MF)                                                                                              \
+  do {                                                                                                         \
+    if constexpr (UP) up_tile<FMT, MFX, MF, FMT == F_I4R, NW>(smem, L, e, tile, nb, x, tokidx, out, M, K, pexp, hs, cmag, rot); \
+    else dn_tile<FMT, MFX, MF, NW>(smem, L, e, tile, nb, npass, x, out, M, K, pexp);                           \
+  } while (0)
+  if (MFX == 1 || mfn <= 1) ST_GO(1);
+  else if (MFX == 2 || mfn <= 2) ST_GO(2);
+  else if constexpr (MFX > 2) ST_GO(4);
+#undef ST_GO
+}
+
+SW to_dev(const moe_lutw* p, const float* cb_up, const int8_t* pexp) {
+  SW d{};
+  d.pexp = pexp;
+  if (p) {
+    d.w = p->w; d.w_up = p->w_up; d.sc = p->sc; d.sc_up = p->sc_up; d.cb = p->cb;
+    d.cb_up = cb_up ? cb_up : p->cb;
+    d.sstride = p->sstride; d.e_rows = p->e_rows; d.up_off = p->up_off;
+  }
+  return d;
+}
+
+template <int FMT, bool UP, int MFX>
+int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* tokidx, const moe_tile* tiles,
+           const int* ntiles, int max_tiles, __half* out, int m, int k, int split, moe_hscale hs, const moe_rotv* rot,
+           hipStream_t st) {
+  constexpr int NW = block_waves(FMT, UP, MFX);
+  constexpr size_t lds = smem_bytes(FMT, UP, MFX);
+  static moe_dev_once once;
+  int dev;
+  if (moe_dev_pending(once, &dev)) {
+    MOE_HIP(hipFuncSetAttribute((const void*)k_moe_stream<FMT, UP, MFX>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    moe_dev_done(once, dev);
+  }
+  int nblk = UP ? (m + 16 * NW - 1) / (16 * NW) : m / (32 * NW), npass = 1;
+  // Down: a block walks several groups of rows behind one staging of the activations; the longest walk that leaves twelve
+  // blocks per CU (64 pairs: two.  Staging is most of a short walk there: 2048 tokens i4r 205 us, with six blocks 223, with
+  // twelve 300)
+  if (!UP)
+    for (int c = 1; c <= nblk; c++)
+      if (nblk % c == 0 && (int64_t)max_tiles * (nblk / c) >= (MFX == 4 ? 512 : 3072)) npass = c;
+  nblk /= npass;
+  const int per_xcd = (max_tiles + 7) / 8 + 1;
+  k_moe_stream<FMT, UP, MFX><<<(unsigned)(per_xcd * nblk * 8), 64 * NW, lds, st>>>(
+      R, S, n_experts, x, tokidx, tiles, ntiles, out, m, k, nblk, split, npass, hs, rot ? *rot : moe_rotv{nullptr, nullptr});
+  MOE_LAUNCH_CHECK();
+  return MOE_OK;
+}
+
+}  // namespace
+
+// Pairs per tile for a batch of P tokens, 0 = the batch belongs to the 128-pair kernels.
+// The lines: an expert's pairs spread by about the root of their mean, so 16 and 32 hold nearly all experts in one tile up
+// to 10 and 22; 64-pair tiles at an average of 25 against 32-pair ones: 797 -> 779 us per layer (q4cp), 740 -> 738 (i4r).
+// At 44 a tenth of the experts takes a second tile and the 128-pair kernels draw level (2300 tokens, average 45: 945 against
+// 940 us; 2048: 855 against 924).  Q5_K and Q8_0 fragments leave no registers for 64 pairs: 32-pair tiles win up to about
+// 40 (1700 tokens, average 33: 1248 against 1339 us; 2600, 51: 1542 against 1451).
+int moe_stream_tile_cap(int P, int k, int experts, bool wide) {
+  const float avg = (float)P * (float)k / (float)experts;
+  if (avg <= 10.f) return 16;
+  return wide ? (avg <= 22.f ? 32 : avg <= 44.f ? 64 : 0) : avg <= 38.f ? 32 : 0;
+}
+bool moe_stream_wide(int fmt_up, int fmt_dn) { return fmt_up != F_Q5K && fmt_dn != F_Q80; }
+
+// fmt: MOE_STREAM_*; the views as for moe_launch_gemm_q4cp.  max_tiles == 0: checks only.
+int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const moe_lutw* sh, int n_experts, const __half* x,
+                      const int* tokidx, const moe_tile* tiles, const int* ntiles, int max_tiles, __half* out, int m, int k,
+                      moe_hscale hs, hipStream_t st, const float* sh_cb_up, const int8_t* pexp_routed,
+                      const int8_t* pexp_sh, const moe_rotv* rot) {
+  if (!x || !tiles || !ntiles || !out || max_tiles < 0 || !routed || (up && !tokidx)) return MOE_E_INVALID;
+  const bool plane = fmt <= F_I4R;
+  auto ok = [&](const moe_lutw* p) {
+    if (!p->w || (up && !p->w_up)) return false;
+    if (!moe_aligned(p->w, fmt == F_Q80 ? 4 : 16) || (up && !moe_aligned(p->w_up, 16))) return false;
+    if (plane) {
+      const int a = fmt == F_I4R ? 4 : 16;
+      if (!p->sc || !p->cb || !moe_aligned(p->sc, a) || p->sstride % a || p->sstride < k / (fmt == F_I4R ? 128 : 32) * 2) return false;
+      if (up && (!p->sc_up || !moe_aligned(p->sc_up, a))) return false;
+    }
+    return true;
+  };
+  if (!ok(routed) || (sh && !ok(sh))) return MOE_E_UNSUPPORTED;
+  if (k % 128 || ((fmt == F_Q4K || fmt == F_Q5K || fmt == F_I4R) && k % 256)) return MOE_E_UNSUPPORTED;
+  // (down: rows of three lines, and whole groups of rows for sixteen waves)
+  if (up ? k < 256 : (k + 255) / 256 != DN_LINES || m % 512) return MOE_E_UNSUPPORTED;
+  if (up && (m % 16 || (fmt >= F_Q4K && m % 64) || (fmt == F_I4R && m % 128))) return MOE_E_UNSUPPORTED;
+  if ((up && fmt == F_Q80) || (!up && fmt == F_Q5K) || (cap > 32 && (fmt == F_Q5K || fmt == F_Q80))) return MOE_E_UNSUPPORTED;
+  if (fmt == F_I4R && up != (rot != nullptr)) return MOE_E_INVALID;
+  if (rot && (!rot->svh_gu || !rot->suh_dn)) return MOE_E_INVALID;
+  if (fmt == F_DN && (!pexp_routed || (sh && !pexp_sh))) return MOE_E_INVALID;
+  if (!moe_aligned(x, 16) || !moe_aligned(out, 16)) return MOE_E_INVALID;
+  if (max_tiles == 0) return MOE_OK;
+  const SW R = to_dev(routed, nullptr, pexp_routed), S = to_dev(sh ? sh : routed, sh ? sh_cb_up : nullptr, sh ? pexp_sh : pexp_routed);
+  const int split = sh ? 1 : 0;
+#define ST_ARGS R, S, n_experts, x, tokidx, tiles, ntiles, max_tiles, out, m, k, split, hs, rot, st
+#define ST_CAP(F, U)                                \
+  do {                                              \
+    if (cap == 16) return launch<F, U, 1>(ST_ARGS); \
+    if (cap == 32) return launch<F, U, 2>(ST_ARGS); \
+    if constexpr (F != F_Q5K && F != F_Q80) return launch<F, U, 4>(ST_ARGS); \
+    return MOE_E_UNSUPPORTED;                       \
+  } while (0)
+#define ST_DIR(F)            \
+  do {                       \
+    if (up) ST_CAP(F, true); \
+    ST_CAP(F, false);        \
+  } while (0)
+  switch (fmt) {
+    case F_DN: ST_DIR(F_DN);
+    case F_AFF: ST_DIR(F_AFF);
+    case F_TAB: ST_DIR(F_TAB);
+    case F_I4R: ST_DIR(F_I4R);
+    case F_Q4K: ST_DIR(F_Q4K);
+    case F_Q5K: ST_CAP(F_Q5K, true);
+    case F_Q80: ST_CAP(F_Q80, false);
+    default: return MOE_E_INVALID;
+  }
+#undef ST_ARGS
+#undef ST_CAP
+#undef ST_DIR
+}

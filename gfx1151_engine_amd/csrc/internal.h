@@ -78,6 +78,14 @@ int moe_launch_gemm_q4cp(bool up, const moe_lutw* routed, const moe_lutw* sh, in
                          hipStream_t st, const moe_comb* comb, const float* sh_cb_up = nullptr, int gs = 0,
                          bool q5k = false, bool nat = false, const int8_t* pexp_routed = nullptr,
                          const int8_t* pexp_sh = nullptr, const moe_rotv* rot = nullptr);
+// Grouped GEMM for tiles of few pairs, weights streamed into registers (gemm_stream.hip)
+enum { MOE_STREAM_SCALED, MOE_STREAM_AFFINE, MOE_STREAM_TABLE, MOE_STREAM_I4R, MOE_STREAM_Q4K, MOE_STREAM_Q5K, MOE_STREAM_Q8_0 };
+int moe_stream_tile_cap(int P, int k, int experts, bool wide);
+bool moe_stream_wide(int fmt_up, int fmt_dn);
+int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const moe_lutw* sh, int n_experts, const __half* x,
+                      const int* tokidx, const moe_tile* tiles, const int* ntiles, int max_tiles, __half* out, int m, int k,
+                      moe_hscale hs, hipStream_t st, const float* sh_cb_up = nullptr, const int8_t* pexp_routed = nullptr,
+                      const int8_t* pexp_sh = nullptr, const moe_rotv* rot = nullptr);
 // Scaled dequantisation of the grouped GEMM (affine q4cp codebooks): per expert the power of two P with
 // |cb slope| * (largest scale of the expert) * 2^(24+P) in [2^14, 2^15), or MOE_PEXP_NONE where the form does not apply
 // (a scale that is not finite, a zero slope, rows whose largest scale lies more than 2^5 below the expert's: their

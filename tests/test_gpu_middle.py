@@ -80,3 +80,33 @@ def test_router_ties_above_the_middle(capi, oracle):
         m.close()
         assert (ids == io[:, :k]).all()
         assert np.abs(ws - wo[:, :k]).max() <= 2.5e-7
+
+
+# ---------- grouped GEMM over tiles of few pairs: every format, tile size and side of a line between them ----------
+TABLE = np.array([-1.0, -0.7, -0.53, -0.4, -0.28, -0.18, -0.09, 0.0, 0.08, 0.16, 0.25, 0.34, 0.44, 0.56, 0.72, 1.0], np.float32)
+
+
+@pytest.mark.parametrize("T", [33, 40, 41, 88, 89, 152, 153, 176, 177])
+@pytest.mark.parametrize("kind,kw,d,mid", [
+    ("q4cp", dict(fmt="q4cp"), 512, 640), ("q4cp-affine", dict(fmt="q4cp"), 1024, 768),
+    ("q4cp-table", dict(fmt="q4cp", codebook=TABLE), 512, 640),
+    ("q4cp-tables", dict(fmt="q4cp", codebook=TABLE, shared_codebooks=[TABLE, TABLE[::-1].copy(), TABLE * 0.5]), 1024, 768),
+    ("i4r", dict(fmt="i4r"), 512, 768), ("q4k", dict(fmt="q4k"), 512, 768), ("q4k-alone", dict(fmt="q4k", shared=False), 1024, 768),
+    ("q5k-q8_0", dict(fmt="q4k", gg_types=(13, 8, 13)), 512, 768), ("q4k-q8_0", dict(fmt="q4k", gg_types=(12, 8, 8)), 1024, 768)])
+def test_tiles_of_few_pairs(capi, oracle, kind, kw, d, mid, T):
+    rng = np.random.default_rng(T + d)
+    E, k = 16, 4  # (averages of 10, 22, 38 and 44 pairs per expert at 40, 88, 152 and 176 tokens)
+    hl = HostLayer(rng, d, mid, E, k, bias=np.linspace(0, 0.5, E, dtype=np.float32), **kw)
+    if kind == "q4cp-affine":  # one expert's row with a scale 2^6 below its others: no scaled dequantisation
+        sc = hl.gate_up[64 + E * 2 * mid * d // 2:].view(np.float16).reshape(E * 2 * mid, -1)
+        sc[3, :] = np.float16(np.abs(sc).max() / 128)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    m, dev = hl.to_gpu(max_tokens=T)
+    y = m.forward(0, gpu(x)).cpu().numpy()
+    again = m.forward(0, gpu(x)).cpu().numpy()
+    assert m.last_path() == capi.PATH_BATCH
+    m.close()
+    assert (y == again).all()
+    sel = np.r_[0, 1, T // 2, T - 2, T - 1]
+    yo, _, _ = oracle.moe_layer(hl.oracle_layer(), x[sel])
+    assert max_abs_rel(y[sel], yo) <= 2e-3
