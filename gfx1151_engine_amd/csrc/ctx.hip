@@ -59,7 +59,7 @@ struct moe_ctx {
   int* ids = nullptr;         // [T][id_stride]
   float* ws = nullptr;        // [T][id_stride]
   float* sh_logit = nullptr;  // [T]
-  float* rtol = nullptr;      // [min(T, MOE_ROUTER_SPLIT_MAX)]: per token, how far the parallel routers' logits can lie from the reference's
+  float* rtol = nullptr;      // [T]: per token, how far the parallel routers' logits can lie from the reference's
   double* gpart = nullptr;    // fp64 partial logits of the column-split router (33 .. MOE_ROUTER_SPLIT_MAX tokens)
   unsigned* ticket = nullptr; // block counter of the fused small-batch router launch (rests at 0)
   double* kpart = nullptr;    // partial tiles and per-row-group tickets (resting at 0) of the column-split router launch
@@ -228,7 +228,7 @@ MOE_API int moe_create(const moe_config* cfg, moe_ctx** out) {
   if (e == hipSuccess) e = hipMalloc(&c->ws, T * S * 4);
   if (e == hipSuccess) e = hipMemset(c->ws, 0, T * S * 4);
   if (e == hipSuccess) e = hipMalloc(&c->sh_logit, T * 4);
-  if (e == hipSuccess) e = hipMalloc(&c->rtol, (T < (size_t)MOE_ROUTER_SPLIT_MAX ? T : (size_t)MOE_ROUTER_SPLIT_MAX) * 4);
+  if (e == hipSuccess) e = hipMalloc(&c->rtol, T * 4);
   if (e == hipSuccess) e = hipMalloc(&c->ticket, 256);
   if (e == hipSuccess) e = hipMemset(c->ticket, 0, 256);
   if (e == hipSuccess) e = hipMalloc(&c->kpart, MOE_ROUTER_KPART_BYTES);
@@ -1038,19 +1038,6 @@ static StreamKinds stream_kinds(const MoeLayer& L, const moe_config& g) {
   return k;
 }
 
-// Router of a batch above MOE_ROUTER_SPLIT_MAX tokens: ids / ws.  By default through candidate selection
-// (router_cand.hip); MOE_OPT_ROUTER_CANDIDATES = 0, or a shape it does not take, runs the dense fp64 launch and the exact
-// softmax / top-k over all experts.
-static int router_batch(moe_ctx* c, MoeLayer& L, const float* x, int P, hipStream_t st) {
-  const moe_config& g = c->cfg;
-  if (c->router_cand && c->rc_scratch && moe_router_cand_supported(&L.router, P, g.topk))
-    return moe_router_batch_cand(&L.router, L.router_bias, x, P, c->logits, c->ids, c->ws, g.topk, g.id_stride, c->rc_scratch,
-                                 st, L.router_bmax);
-  int rc = moe_router_logits_seq(&L.router, L.router_bias, x, P, c->logits, st);
-  if (!rc) rc = moe_router_topk(c->logits, c->ids, c->ws, P, g.experts, g.topk, g.id_stride, st);
-  return rc;
-}
-
 // Batches: expert-sorted permutation, MFMA grouped GEMMs over <=128-pair tiles (the shared expert
 // rides along as expert index E over all tokens), f16 pair buffer, deterministic weighted combine.
 // Returns MOE_E_UNSUPPORTED (before enqueuing anything) for shapes / formats the GEMM does not cover.
@@ -1223,8 +1210,12 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
     }
   }
   const int tile_cap = cap ? cap : moe_gemm_tile_cap();
-  // middle sizes: the router's column-split launches (router_split.hip); its first launch makes the f16 copy of x as well
-  const bool mid_router = c->router_cand && c->gpart && moe_router_split_supported(&L.router, L.has_shared ? &L.sh_sg : nullptr, P, g.topk);
+  // router: column-split fp64 launches for middle sizes (router_split.hip), above candidate selection (router_cand.hip); their
+  // first launches make the f16 copy of x as well.  MOE_OPT_ROUTER_CANDIDATES = 0, or a shape they do not take: the dense
+  // fp64 launch and the exact softmax / top-k over all experts.
+  const moe_wview* const wx = L.has_shared ? &L.sh_sg : nullptr;
+  const bool cand_router = P >= MOE_ROUTER_CAND_MIN && c->router_cand && c->rc_scratch && moe_router_cand_supported(&L.router, wx, P, g.topk);
+  const bool mid_router = !cand_router && c->router_cand && c->gpart && moe_router_split_supported(&L.router, wx, P, g.topk);
   // The shared expert in launches of its own, on the context's side stream: where its kernels differ from the routed
   // experts', and for batches whose router takes long enough to hide them (at middle sizes they ride along: the
   // router is two short launches there, and the shared expert's few tiles alone leave the chip idle).
@@ -1254,7 +1245,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   const int max_tiles = (P * g.topk + tile_cap - 1) / tile_cap + g.experts + (sh_in ? (P + tile_cap - 1) / tile_cap : 0);
   // what else is needed from x: f16 copy, mean square (range guard), the shared expert's gate logit
   moe_row_extras ex{};
-  ex.x16 = c->x16_ext ? nullptr : c->x16;
+  ex.x16 = c->x16_ext && !cand_router ? nullptr : c->x16;  // (the candidates' bound is on this library's own rounding)
   ex.layout = xl;
   ex.xms = c->xms;
   if (L.has_shared) {
@@ -1263,9 +1254,15 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
     ex.out_x = c->sh_logit;
   }
   moe_rfix rf = router_fix(c, L, x, true);
-  if (mid_router) {
+  if (mid_router || cand_router) {
     ex.tol = c->rtol;
     ex.tol_scale = rf.tol_scale;
+  }
+  if (cand_router) {
+    if ((rc = moe_router_batch_cand(&L.router, x, P, c->logits, c->ids, c->ws, g.topk, g.id_stride, c->rc_scratch, ex, rf, L.router_bmax,
+                                    st, aside ? c->ev_fork : nullptr)))
+      return rc;
+  } else if (mid_router) {
     if ((rc = moe_router_batch_split(&L.router, x, P, c->ids, c->ws, g.topk, g.id_stride, c->gpart, ex, rf, st,
                                      aside ? c->ev_fork : nullptr)))
       return rc;
@@ -1279,7 +1276,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
     // in front of the combine).
     MOE_HIP(hipStreamWaitEvent(c->side, c->ev_fork, 0));
     if (v2) rs = moe_launch_v2_rot(x, (uint64_t)g.d, P, g.d, L.v2_su, nullptr, 1, c->v2_x16, (uint64_t)g.d, nullptr, 0, nullptr, nullptr, c->side);
-    if (!rs && !mid_router) rs = moe_launch_row_extras(x, P, g.d, ex, c->side);
+    if (!rs && !mid_router && !cand_router) rs = moe_launch_row_extras(x, P, g.d, ex, c->side);
     const hipError_t ee = hipEventRecord(c->ev_x16, c->side);
     if (!rs && ee != hipSuccess) rs = (int)ee;
     if (L.has_shared) {
@@ -1290,8 +1287,9 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   }
   // caller's stream: router, top-k, permutation, the routed experts' GEMMs
   rc = MOE_OK;
-  if (!mid_router) {
-    rc = router_batch(c, L, x, P, st);
+  if (!mid_router && !cand_router) {
+    rc = moe_router_logits_seq(&L.router, L.router_bias, x, P, c->logits, st);
+    if (!rc) rc = moe_router_topk(c->logits, c->ids, c->ws, P, g.experts, g.topk, g.id_stride, st);
     if (!rc && !aside) rc = moe_launch_row_extras(x, P, g.d, ex, st);
   }
   prof_mark(c, MOE_PROF_ROUTER, st);

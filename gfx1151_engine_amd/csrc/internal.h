@@ -112,6 +112,9 @@ int moe_launch_reduce(const void* pairs, bool pairs_f16, const int* pairids, con
 // Router of 33 .. MOE_ROUTER_SPLIT_MAX tokens (router_split.hip): fp64 matrix pipe, columns split over waves and blocks, a
 // selecting block per token; what else a batch needs from x comes out of the first launch.
 constexpr int MOE_ROUTER_SPLIT_MAX = 1024, MOE_ROUTER_SPLIT_KS = 8;
+// ... and the size from which the candidate selection (router_cand.hip) goes first: the layer at 400 tokens 536 us with the one,
+// 549 with the other; 515: 568 and 566; 800: 630 and 609
+constexpr int MOE_ROUTER_CAND_MIN = 513;
 struct moe_row_extras {
   void* x16;         // f16 copy of x in `layout` (moe_f32_to_f16), or nullptr
   int layout;
@@ -128,14 +131,15 @@ size_t moe_router_split_scratch_bytes(int max_tokens, int experts, int d);
 int moe_router_batch_split(const moe_wview* W, const float* x, int P, int* ids, float* ws, int k,
                            int id_stride, double* gpart, const moe_row_extras& R, const moe_rfix& RF, hipStream_t st,
                            hipEvent_t after_rows = nullptr);  // recorded behind the first launch
-// sequential-order logits; run_if_above: only if *run_if_above > run_thr when the launch starts (device memory)
-int moe_router_logits_seq(const moe_wview* W, const float* bias, const float* x, int P, float* logits, hipStream_t st,
-                          const int* run_if_above = nullptr, int run_thr = 0);
-// batch router through candidate selection (router_cand.hip): bit-exact ids, weights within an ulp or two
-bool moe_router_cand_supported(const moe_wview* W, int P, int k);
+// sequential-order logits
+int moe_router_logits_seq(const moe_wview* W, const float* bias, const float* x, int P, float* logits, hipStream_t st);
+// Router of larger batches through candidate selection (router_cand.hip): bit-exact ids, weights within an ulp or two.  Its
+// first launch leaves what else a batch needs from x; R.x16 is required.
+bool moe_router_cand_supported(const moe_wview* W, const moe_wview* Wx, int P, int k);
 size_t moe_router_cand_scratch_bytes(int max_tokens, int experts, int d);
-int moe_router_batch_cand(const moe_wview* W, const float* bias, const float* x, int P, float* logits, int* ids, float* ws,
-                          int k, int id_stride, void* scratch, hipStream_t st, float bias_max);
+int moe_router_batch_cand(const moe_wview* W, const float* x, int P, float* logits, int* ids, float* ws, int k, int id_stride,
+                          void* scratch, const moe_row_extras& R, const moe_rfix& RF, float bias_max, hipStream_t st,
+                          hipEvent_t after_rows = nullptr);  // recorded behind the first launch
 
 size_t moe_qvec_plane_bytes(int K);
 size_t moe_qvec_meta_bytes(int K);

@@ -33,10 +33,7 @@ template <bool BF16, int BT>
 __global__ void __launch_bounds__(256, 2) k_router_logits_seq(const void* __restrict__ W,
                                                            const float* __restrict__ bias,
                                                            const float* __restrict__ x, int P, int E,
-                                                           int d, float* __restrict__ logits, int ncol, int ntt,
-                                                           const int* __restrict__ run_if_above, int run_thr) {
-  // (a launch that is only needed when many tokens were listed for an exact redo returns at once otherwise)
-  if (run_if_above && *run_if_above <= run_thr) return;
+                                                           int d, float* __restrict__ logits, int ncol, int ntt) {
   constexpr int MT = BT / 32;                 // 16-token MFMA tiles per wave
   constexpr int XL = (BT * RS_K / 4) / 256;   // float4 loads per thread and slab (activations)
   constexpr int WL = (RS_E * RS_K / 4) / 256; // (weights)
@@ -472,14 +469,13 @@ __global__ void __launch_bounds__(256) k_row_norm_max(const void* __restrict__ W
 
 // Launch of the sequential-order kernel: 128-token tiles when there are enough of them to fill the
 // chip, 64-token tiles otherwise.
-void launch_seq(const void* W, bool bf, const float* bias, const float* x, int P, int E, int d, float* logits, hipStream_t st,
-                const int* run_if_above = nullptr, int run_thr = 0) {
+void launch_seq(const void* W, bool bf, const float* bias, const float* x, int P, int E, int d, float* logits, hipStream_t st) {
   const int ncol = (E + RS_E - 1) / RS_E;
   const bool big = (int64_t)((P + 127) / 128) * ncol >= 512;
   const int bt = big ? 128 : 64;
   const int ntt = (P + bt - 1) / bt;
   const unsigned grid = (unsigned)(((ntt + 7) / 8) * 8 * ncol);
-#define RS_GO(BF, BT) k_router_logits_seq<BF, BT><<<grid, 256, 0, st>>>(W, bias, x, P, E, d, logits, ncol, ntt, run_if_above, run_thr)
+#define RS_GO(BF, BT) k_router_logits_seq<BF, BT><<<grid, 256, 0, st>>>(W, bias, x, P, E, d, logits, ncol, ntt)
   if (bf) { if (big) RS_GO(true, 128); else RS_GO(true, 64); }
   else { if (big) RS_GO(false, 128); else RS_GO(false, 64); }
 #undef RS_GO
@@ -655,11 +651,9 @@ MOE_API int moe_router_logits(const moe_wview* W, const float* bias, const float
   return MOE_OK;
 }
 
-// Internal: sequential-order logits for any P; with run_if_above the launch does its work only if *run_if_above > run_thr
-// when it starts (device memory).
-int moe_router_logits_seq(const moe_wview* W, const float* bias, const float* x, int P, float* logits, hipStream_t st,
-                          const int* run_if_above, int run_thr) {
-  launch_seq(W->data, W->dtype == MOE_DT_BF16, bias, x, P, (int)W->rows, (int)W->cols, logits, st, run_if_above, run_thr);
+// Internal: sequential-order logits for any P.
+int moe_router_logits_seq(const moe_wview* W, const float* bias, const float* x, int P, float* logits, hipStream_t st) {
+  launch_seq(W->data, W->dtype == MOE_DT_BF16, bias, x, P, (int)W->rows, (int)W->cols, logits, st);
   MOE_LAUNCH_CHECK();
   return MOE_OK;
 }

@@ -1,11 +1,11 @@
-// Router of middle-sized batches (33 .. MOE_ROUTER_SPLIT_MAX tokens): fp64 logits on the f64 matrix pipe with the columns
+// Router of middle-sized batches (33 .. MOE_ROUTER_CAND_MIN - 1 tokens, up to MOE_ROUTER_SPLIT_MAX where the candidate selection
+// does not apply): fp64 logits on the f64 matrix pipe with the columns
 // split over the waves of a block and over blocks, then one selecting block per token.  Two launches.
 // (reference arithmetic: src/ref.cpp:68-77,565-594)
 //
-// The candidate selection of router_cand.hip pays off once its eight dependent launches are small against the fp64 work
-// they save.  At a few hundred tokens they are not: 130 tokens took 150 us in those launches (the f16 pass alone 75 us,
-// three blocks of 64 tokens walking all columns), while all 130 x 512 sums are 0.2 G fp64 FMAs, 5 us of the chip's f64
-// matrix rate.  What this needs is enough waves, so columns are dealt out: a block is 32 tokens x 32 experts x one of KS
+// The candidate selection of router_cand.hip pays off once its third launch, a chain of about 30 us, is small against the
+// fp64 work it saves.  At a few hundred tokens it is not: all 130 x 512 sums are 0.2 G fp64 FMAs, 5 us of the chip's f64
+// matrix rate.  What that needs is enough waves, so columns are dealt out: a block is 32 tokens x 32 experts x one of KS
 // column shares, its eight waves take an eighth of the share each and their partial tiles are added in wave order through
 // LDS; the KS shares' fp64 partial sums go to memory and the selecting block of a token adds them in share order.  Every
 // order is fixed, so results do not depend on timing.
@@ -15,12 +15,12 @@
 // The launch's spare blocks read x anyway, so they leave what else a batch needs from it: the f16 copy in the grouped
 // GEMM's order, the mean square (f16 range guard), |x| as the selection's error bound and the shared expert's gate logit.
 // Measured (512 experts, d = 3072, bf16 router): 10.7 + 7.6 us at 48 tokens, 25 + 7.7 us at 130 (f32), 53 + 7.2 us at 515; the
-// dense fp64 launch that such layers took before (the router and its gate vector of different types) 395 us, the candidate
-// selection's eight launches 150 us.
+// dense fp64 launch that such layers took before (the router and its gate vector of different types) 395 us, the others
+// 150 us in the candidate selection of then.
 #include "common.h"
 #include "internal.h"
+#include "router_chain.h"
 #include "rowx.h"
-#include "topk.h"
 
 namespace {
 
@@ -144,53 +144,8 @@ __global__ void __launch_bounds__(512, 2) k_router_split(const void* __restrict_
   }
 }
 
-// One logit's fp64 sum as the reference's sequential chain (src/ref.cpp:70-77), by one wave: the lanes widen 256 columns
-// at a time into LDS (a single thread's 2 d quarter-rate conversions and its dependent loads took 110 us), then every lane
-// runs the same chain over them.  buf: 512 doubles of LDS owned by the wave.
-__device__ double exact_chain_wave(const moe_rfix& R, int t, int e, double* buf) {
-  const int lane = threadIdx.x & 63;
-  const float* xr = R.x + (size_t)t * R.d;
-  double acc = 0.0;
-  float4 w, xv;
-  auto load = [&](int c) {
-    w = xv = float4{0.f, 0.f, 0.f, 0.f};
-    if (c >= R.d) return;
-    xv = *(const float4*)(xr + c);
-    if (R.bf16) {
-      const uint2 u = *(const uint2*)((const uint16_t*)R.W + (size_t)e * R.d + c);
-      w = float4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
-                 __uint_as_float(u.y & 0xffff0000u)};
-    } else {
-      w = *(const float4*)((const float*)R.W + (size_t)e * R.d + c);
-    }
-  };
-  load(4 * lane);
-  for (int c = 0; c < R.d; c += 256) {
-    double* const q = buf + 8 * lane;  // (w, x) pairs of this lane's four columns
-    q[0] = (double)w.x; q[1] = (double)xv.x; q[2] = (double)w.y; q[3] = (double)xv.y;
-    q[4] = (double)w.z; q[5] = (double)xv.z; q[6] = (double)w.w; q[7] = (double)xv.w;
-    load(c + 256 + 4 * lane);
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wave's own LDS writes
-    __builtin_amdgcn_wave_barrier();
-    const int n = R.d - c < 256 ? R.d - c : 256;  // (a multiple of 32)
-    for (int i = 0; i < n; i += 16) {
-#pragma unroll
-      for (int j = 0; j < 16; j++) {
-        const double2 p = *(const double2*)(buf + 2 * (i + j));
-        acc = fma(p.x, p.y, acc);
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-  }
-  return acc;
-}
-
 // The selecting block of a token: the column shares' sums in share order, + bias, softmax / top-k.
-// Its fp64 sums differ from the reference's sequential ones by at most tol, so a logit is the reference's float unless a
-// rounding boundary lies within tol of the sum.  No such logit (two tokens in three): the selection is the reference's as
-// it stands.  Otherwise the k + 1 best must be further apart than the doubt (topk.h), and where they are not, the
-// doubtful logits alone are redone as the reference's chains -- which leaves none in doubt.  (Redoing all 512 logits of
-// such a token, as the launches for up to 32 tokens do, takes 70 us; one batch of 515 tokens in ten has one.)
+// Its fp64 sums differ from the reference's sequential ones by at most tol; select_listed makes the ids certain.
 template <int NPL>
 __global__ void __launch_bounds__(256) k_router_split_topk(const double* __restrict__ gpart, int KS, int* __restrict__ ids,
                                                            float* __restrict__ ws, int P, int E, int k, int id_stride,
@@ -203,12 +158,11 @@ __global__ void __launch_bounds__(256) k_router_split_topk(const double* __restr
   __shared__ int list[64 * NPL], nlist;
   const int t = blockIdx.x, tid = threadIdx.x;
   if (tid == 0) nlist = 0;
+  __syncthreads();
   const float tol = RF.tol[t];
-  bool doubt[NV], any = false;
 #pragma unroll
   for (int j = 0; j < NV; j++) {
     const int e = tid + 256 * j;
-    doubt[j] = false;
     if (e < E) {
       const double* p = gpart + (size_t)t * E + e;
       double v[MOE_ROUTER_SPLIT_KS];
@@ -217,29 +171,12 @@ __global__ void __launch_bounds__(256) k_router_split_topk(const double* __restr
       double sum = v[0];
 #pragma unroll
       for (int s = 1; s < MOE_ROUTER_SPLIT_KS; s++) sum += v[s];
-      doubt[j] = !((float)(sum - (double)tol) == (float)(sum + (double)tol));  // (true for NaNs and an infinite tol)
+      if (logit_doubtful(sum, tol)) list[atomicAdd(&nlist, 1)] = e;
       lg[e] = (float)sum + (RF.bias ? RF.bias[e] : 0.f);
     }
-    any = any || doubt[j];
-  }
-  const bool some = __syncthreads_or(any);
-  float slack = INFINITY;
-  if (some) slack = topk_block<NPL, false, 256, true>(lg, sel_ids, sel_ws, E, k);
-  else (void)topk_block<NPL, false, 256>(lg, sel_ids, sel_ws, E, k);
-  if (some && (!(slack > 2.f * tol) || !topk_fast_handled<NPL>(lg, E, k))) {  // block-uniform
-#pragma unroll
-    for (int j = 0; j < NV; j++)
-      if (doubt[j]) list[atomicAdd(&nlist, 1)] = tid + 256 * j;
-    __syncthreads();
-    for (int i = tid >> 6; i < nlist; i += 4) {
-      const int e = list[i];
-      const float v = (float)exact_chain_wave(RF, t, e, chain[tid >> 6]) + (RF.bias ? RF.bias[e] : 0.f);
-      if ((tid & 63) == 0) lg[e] = v;
-    }
-    __syncthreads();
-    (void)topk_block<NPL, false, 256>(lg, sel_ids, sel_ws, E, k);
   }
   __syncthreads();
+  select_listed<NPL>(lg, list, nlist, tol, RF, t, E, k, sel_ids, sel_ws, chain);
   if (tid < k) {
     ids[(size_t)t * id_stride + tid] = sel_ids[tid];
     ws[(size_t)t * id_stride + tid] = sel_ws[tid];

@@ -3,6 +3,28 @@
 #include "common.h"
 #include "internal.h"
 
+// the chunk's two float4: neighbours, or (layout 2) elements 4w.. and 32 + 4w.. of the 64-block
+__device__ __forceinline__ void f16_chunk_src(int layout, int i, int& ia, int& ib) {
+  ia = layout == 2 ? (i >> 3) * 16 + (i & 7) : 2 * i;
+  ib = layout == 2 ? ia + 8 : ia + 1;
+}
+__device__ __forceinline__ uint4 f16_chunk(int layout, const float4& u, const float4& v) {
+  __half2 a, b, c, e;
+  if (layout == 2) {
+    a = __floats2half2_rn(u.x, u.z); b = __floats2half2_rn(v.x, v.z);
+    c = __floats2half2_rn(u.y, u.w); e = __floats2half2_rn(v.y, v.w);
+  } else if (layout == 0) {
+    a = __floats2half2_rn(u.x, u.y); b = __floats2half2_rn(u.z, u.w);
+    c = __floats2half2_rn(v.x, v.y); e = __floats2half2_rn(v.z, v.w);
+  } else {
+    a = __floats2half2_rn(u.x, v.x); b = __floats2half2_rn(u.y, v.y);
+    c = __floats2half2_rn(u.z, v.z); e = __floats2half2_rn(u.w, v.w);
+  }
+  uint4 o;
+  o.x = *(const uint32_t*)&a; o.y = *(const uint32_t*)&b; o.z = *(const uint32_t*)&c; o.w = *(const uint32_t*)&e;
+  return o;
+}
+
 // the f16 copy (layout as moe_f32_to_f16's), the mean square, the selection's error bound and the shared expert's gate
 // logit (fp64 sum) of row t; each is left out where its pointer is null
 // (chunks of 8 columns i0, i0 + step, ...: this thread's part of the row's sums in acc and gate)
@@ -14,24 +36,11 @@ __device__ __forceinline__ void row_extras_part(const float* __restrict__ x, int
   gate = 0.0;
 #pragma unroll 2
   for (int i = i0; i < d / 8; i += step) {
-    // the chunk's two float4: neighbours, or (layout 2) elements 4w.. and 32 + 4w.. of the 64-block
-    const int ia = R.layout == 2 ? (i >> 3) * 16 + (i & 7) : 2 * i, ib = R.layout == 2 ? ia + 8 : ia + 1;
+    int ia, ib;
+    f16_chunk_src(R.layout, i, ia, ib);
     const float4 u = xr[ia], v = xr[ib];
     if (yr) {
-      __half2 a, b, c, e;
-      if (R.layout == 2) {
-        a = __floats2half2_rn(u.x, u.z); b = __floats2half2_rn(v.x, v.z);
-        c = __floats2half2_rn(u.y, u.w); e = __floats2half2_rn(v.y, v.w);
-      } else if (R.layout == 0) {
-        a = __floats2half2_rn(u.x, u.y); b = __floats2half2_rn(u.z, u.w);
-        c = __floats2half2_rn(v.x, v.y); e = __floats2half2_rn(v.z, v.w);
-      } else {
-        a = __floats2half2_rn(u.x, v.x); b = __floats2half2_rn(u.y, v.y);
-        c = __floats2half2_rn(u.z, v.z); e = __floats2half2_rn(u.w, v.w);
-      }
-      uint4 o;
-      o.x = *(const uint32_t*)&a; o.y = *(const uint32_t*)&b; o.z = *(const uint32_t*)&c; o.w = *(const uint32_t*)&e;
-      yr[i] = o;
+      yr[i] = f16_chunk(R.layout, u, v);
     }
     acc += ((u.x * u.x + u.y * u.y) + (u.z * u.z + u.w * u.w)) + ((v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w));
     if (R.wx) {

@@ -82,6 +82,31 @@ def test_router_ties_above_the_middle(capi, oracle):
         assert np.abs(ws - wo[:, :k]).max() <= 2.5e-7
 
 
+# ---------- router, candidate selection: tiles and column shares of its f16 launch, ragged experts, ties, doubt, padding ----------
+@pytest.mark.parametrize("T,E,k,d,dt,fmt", [(513, 512, 10, 3072, "bf16", "q4cp"), (600, 500, 10, 512, "f32", "q4cp"), (700, 43, 15, 256, "f32", "q4cp"),
+                                            (777, 128, 4, 320, "f32", "q8_0"), (2600, 512, 10, 256, "bf16", "q4cp"), (2689, 510, 8, 384, "f32", "q4cp")])
+def test_router_candidates(capi, oracle, T, E, k, d, dt, fmt):
+    rng = np.random.default_rng(T)
+    kw = dict(fmt="q4k", gg_types=(8, 8, 8)) if fmt == "q8_0" else {}
+    hl = HostLayer(rng, d, 256, E, k, router_dtype=dt, shared=False, **kw)
+    hl.router[E - 1] = hl.router[2]          # a tie for every token, in and out of the selection
+    if dt == "f32":
+        hl.router[E // 2] = hl.router[1] * np.float32(1 + 2 ** -22)  # logits an ulp apart: tokens for the redo
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    x[5] = 0.0                               # padding, a value past f16's range, a spread that underflows probabilities
+    x[T - 1] = 0.0
+    x[6, 3] = 1e6
+    x[7] *= 300.0
+    lo, io, wo = oracle.router(hl.oracle_layer().router, x, k)
+    m, dev = hl.to_gpu(max_tokens=T)
+    m.forward(0, gpu(x))
+    assert m.last_path() == capi.PATH_BATCH
+    ids, ws = (a.cpu().numpy()[:, :k] for a in m.last_routing(T))
+    m.close()
+    assert (ids == io[:, :k]).all()
+    assert np.abs(ws - wo[:, :k]).max() <= 2.5e-7
+
+
 # ---------- grouped GEMM over tiles of few pairs: every format, tile size and side of a line between them ----------
 TABLE = np.array([-1.0, -0.7, -0.53, -0.4, -0.28, -0.18, -0.09, 0.0, 0.08, 0.16, 0.25, 0.34, 0.44, 0.56, 0.72, 1.0], np.float32)
 
