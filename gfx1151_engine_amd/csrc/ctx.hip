@@ -750,12 +750,10 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
   //  block takes the norm of x itself)
   const moe_rfix rf = router_fix(c, L, x, P <= 4);
   if ((rc = stage(MOE_PROF_ROUTER, [&]() -> int {
-         bool fused = false;
          // (the selection runs in launches of its own here, so that it can be made certain: no top-k inside the logits launch)
          int e = moe_router_logits_small(&L.router, L.router_bias, L.has_shared ? &L.sh_sg : nullptr, x, P, c->logits,
                                          c->sh_logit, (use_int || use_int4k || use_intgg) ? c->xplanes : nullptr, c->xmeta,
-                                         use_int4k || use_intgg, nullptr, c->ids, c->ws, g.topk,
-                                         g.id_stride, &fused, st, c->kpart, c->ktickets, nullptr, P <= 4 && rf.W ? c->rtol : nullptr,
+                                         use_int4k || use_intgg, st, c->kpart, c->ktickets, nullptr, P <= 4 && rf.W ? c->rtol : nullptr,
                                          rf.tol_scale);
          if (!e && !gu_topk)
            e = moe_launch_router_topk_small(c->logits, c->ids, c->ws, P, g.experts, g.topk, g.id_stride, &rf, st);
@@ -937,13 +935,11 @@ static int forward_small_v2(moe_ctx* c, MoeLayer& L, const float* x, int P, floa
   const bool gu_topk = P <= c->gu_topk_max;
   const moe_rfix rf = router_fix(c, L, x, P <= 4);
   if ((rc = stage(MOE_PROF_ROUTER, [&]() -> int {
-         bool fused = false;
          // (the planes of rot_in(x, su) ride in the router launch's spare blocks)
          const moe_rot_planes rot{L.v2_su, c->v2_xplanes, c->v2_xmeta};
          int e = moe_router_logits_small(&L.router, L.router_bias, L.has_shared ? &L.sh_sg : nullptr, x, P, c->logits,
                                          c->sh_logit, sh ? c->xplanes : nullptr, c->xmeta, false,
-                                         nullptr, c->ids, c->ws, g.topk, g.id_stride, &fused, st,
-                                         c->kpart, c->ktickets, &rot, P <= 4 && rf.W ? c->rtol : nullptr, rf.tol_scale);
+                                         st, c->kpart, c->ktickets, &rot, P <= 4 && rf.W ? c->rtol : nullptr, rf.tol_scale);
          if (!e && !gu_topk) e = moe_launch_router_topk_small(c->logits, c->ids, c->ws, P, g.experts, g.topk, g.id_stride, &rf, st);
          return e;
        })))

@@ -48,8 +48,7 @@ struct moe_rot_planes {
 };
 int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x,
                             int P, float* logits, float* out_x, uint32_t* planes, float2* meta,
-                            bool planes_natural, unsigned* counter, int* ids, float* ws, int k, int id_stride, bool* fused_topk,
-                            hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rot = nullptr,
+                            bool planes_natural, hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rot = nullptr,
                             float* tol_out = nullptr, float tol_scale = 0.f);
 // scratch of the column-split router launch (5..32 tokens): fp64 partial tiles of up to 8 splits x 32 tokens
 // for at most MOE_ROUTER_KSPLIT_ROWS rows, and one ticket counter (resting at 0) per 16 rows

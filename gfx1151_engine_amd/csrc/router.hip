@@ -198,124 +198,128 @@ __device__ __forceinline__ void router_plane_blocks(int q, int bs, int tid, cons
   moe_st8_planes(v, tid, R.planes, R.meta, (size_t)t * G + (c8 >> 2), live);
 }
 
-// ---- lane-parallel order for small P: one wave per weight row (four rows per block), lanes stride
-// the columns, four independent fp64 chains per lane and token, fixed combination order.  The fp64
+// ---- lane-parallel order for 1..4 tokens: one wave per weight row (two rows per block, so that 513 rows cover every CU),
+// lanes stride the columns, four independent fp64 chains per lane and token, fixed combination order.  The fp64
 // sum differs from the sequential one only in its last bits, so the f32 logit differs with
 // probability ~1e-8 per value.  Row E (if Wx given) is the shared-expert gate vector: out_x[t] =
 // its logit.  Blocks past the rows (if planes given) turn x into the digit planes of the
 // integer-dot decode kernels, so that work rides along instead of costing a launch.
-// If `counter` is given, the block that finishes last (an atomic ticket per row block; the logits
-// cross as device-scope stores that have completed before the ticket, and device-scope loads after
-// it) runs the softmax / top-k of every token as well and re-arms the counter: one launch instead
-// of two on the latency-bound decode path.
-template <bool BF16, int TT, int NPL>
-__global__ void __launch_bounds__(256) k_router_small(const void* __restrict__ W,
-                                                      const float* __restrict__ bias,
-                                                      const void* __restrict__ Wx, bool wx_bf16,
-                                                      const float* __restrict__ x, int P, int E, int d,
-                                                      float* __restrict__ logits, float* __restrict__ out_x,
-                                                      int nrows, uint32_t* __restrict__ planes,
-                                                      float2* __restrict__ meta, bool planes_natural,
-                                                      unsigned* counter, int* __restrict__ ids,
-                                                      float* __restrict__ ws, int k, int id_stride, moe_rot_planes rot,
-                                                      float* __restrict__ tol_out, float tol_scale) {
-  __shared__ int s_last;
-  // the wave index as a scalar: row, weight type and base address are then wave-uniform values
-  // and the bf16 / f32 choice below is a scalar branch, not a divergent one around every load
-  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int rpb = blockDim.x >> 6;  // rows per block: one per wave
-  const int nrb = (nrows + rpb - 1) / rpb;
-  if ((int)blockIdx.x >= nrb) {
-    router_plane_blocks((int)blockIdx.x - nrb, (int)blockDim.x, (int)threadIdx.x, x, P, d, planes, meta, planes_natural, rot);
-    return;
+// What bounds it is one trip to memory: a wave's twelve loads of its row (3072 columns) are requested before anything
+// is used, with nothing conditional between them.  The weight type and the token count are therefore template
+// arguments, and the next token's activations are requested while one token is summed: with the type tested in the loop (the gate vector may differ from the matrix) and tokens tested per
+// column step, each step waited for its own loads (512 experts, 3072 columns, bf16 matrix and f32 gate vector: one token 8.4 us,
+// three tokens 16.2; now 4.0 and 5.9).  One token on an f32 matrix, where the compiler had untangled the loop: 4.1 before and
+// now; with all weights requested ahead of all activations instead of pair by pair 4.5.
+constexpr int RSM_IT = 12;  // column steps of 256 requested together
+template <bool BF>
+struct RsmW {
+  typedef float4 T;
+};
+template <>
+struct RsmW<true> {
+  typedef uint2 T;
+};
+template <bool BF, int TT>
+__device__ __forceinline__ void router_small_row(const void* __restrict__ Wr, const float* __restrict__ x, int d, int lane,
+                                                 bool norms, double (&sum)[TT], float (&n2)[TT]) {
+  typedef typename RsmW<BF>::T WT;
+  double acc[TT][4];
+  float xs[TT];
+#pragma unroll
+  for (int i = 0; i < TT; i++) {
+    xs[i] = 0.f;
+#pragma unroll
+    for (int q = 0; q < 4; q++) acc[i][q] = 0.0;
   }
-  const int row = blockIdx.x * rpb + wv;
-  if (row < nrows) {
-    const bool extra = row == E;
-    const void* Wr = extra ? Wx : W;
-    const uint64_t base = extra ? 0 : (uint64_t)row * d;
-    const bool bf = extra ? wx_bf16 : BF16;
-    // the wave of row 0 also takes |x|^2 of every token: the selection that follows needs a bound on how far these
-    // sums (lanes, then a tree) can lie from the reference's sequential ones, tol_scale * |x|
-    const bool norms = tol_out && row == 0;
-    for (int t0 = 0; t0 < P; t0 += TT) {
-      double acc[TT][4];
-      float xs[TT];
+  for (int c0 = 0; c0 < d; c0 += 256 * RSM_IT) {
+    WT w[RSM_IT];
+    float4 xv[2][RSM_IT];  // a token's activations, and the next one's
+    auto load_x = [&](int i, int j) {
+      const int c = c0 + 256 * j + 4 * lane;
+      xv[i & 1][j] = *(const float4*)(x + (size_t)i * d + (c < d ? c : 0));
+    };
 #pragma unroll
-      for (int i = 0; i < TT; i++) {
-        xs[i] = 0.f;
+    for (int j = 0; j < RSM_IT; j++) {
+      const int c = c0 + 256 * j + 4 * lane;
+      w[j] = *(const WT*)((const uint8_t*)Wr + (size_t)(c < d ? c : 0) * (BF ? 2 : 4));  // (past the row: its head, not used)
+      load_x(0, j);  // (in the order of use: the sums start when the first pair is there)
+    }
 #pragma unroll
-        for (int q = 0; q < 4; q++) acc[i][q] = 0.0;
-      }
-#pragma unroll 12
-      for (int c = lane * 4; c < d; c += 256) {
-        float w[4];
-        if (bf) {
-          const uint2 u = *(const uint2*)((const uint16_t*)Wr + base + c);
-          w[0] = __uint_as_float(u.x << 16);
-          w[1] = __uint_as_float(u.x & 0xffff0000u);
-          w[2] = __uint_as_float(u.y << 16);
-          w[3] = __uint_as_float(u.y & 0xffff0000u);
+    for (int i = 0; i < TT; i++) {
+#pragma unroll
+      for (int j = 0; j < RSM_IT; j++)
+        if (i + 1 < TT) load_x(i + 1, j);
+      __builtin_amdgcn_sched_barrier(0);  // the loads are issued here, not next to their uses
+#pragma unroll
+      for (int j = 0; j < RSM_IT; j++) {
+        // (columns past the row count as zeros: selects, where a branch would make the step wait for its own loads)
+        const bool in = c0 + 256 * j + 4 * lane < d;
+        float4 wf, xf = xv[i & 1][j];
+        if constexpr (BF) {
+          wf.x = __uint_as_float(w[j].x << 16);
+          wf.y = __uint_as_float(w[j].x & 0xffff0000u);
+          wf.z = __uint_as_float(w[j].y << 16);
+          wf.w = __uint_as_float(w[j].y & 0xffff0000u);
         } else {
-          const float4 f = *(const float4*)((const float*)Wr + base + c);
-          w[0] = f.x; w[1] = f.y; w[2] = f.z; w[3] = f.w;
+          wf = w[j];
         }
-#pragma unroll
-        for (int i = 0; i < TT; i++) {
-          if (t0 + i < P) {
-            const float4 xv = *(const float4*)(x + (size_t)(t0 + i) * d + c);
-            acc[i][0] = fma((double)w[0], (double)xv.x, acc[i][0]);
-            acc[i][1] = fma((double)w[1], (double)xv.y, acc[i][1]);
-            acc[i][2] = fma((double)w[2], (double)xv.z, acc[i][2]);
-            acc[i][3] = fma((double)w[3], (double)xv.w, acc[i][3]);
-            if (norms) xs[i] += xv.x * xv.x + xv.y * xv.y + xv.z * xv.z + xv.w * xv.w;
-          }
-        }
-      }
-      if (norms) {
-#pragma unroll
-        for (int i = 0; i < TT; i++) {
-          const float n2 = wave_sum(xs[i]);
-          if (lane == 0 && t0 + i < P) {
-            float tl = tol_scale * sqrtf(n2) * 1.01f;
-            tol_out[t0 + i] = tl >= 0.f ? tl : INFINITY;  // (NaN: nothing is certain)
-          }
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < TT; i++) {
-        const double sum = wave_sum((acc[i][0] + acc[i][1]) + (acc[i][2] + acc[i][3]));
-        if (lane == 0 && t0 + i < P) {
-          float v = (float)sum;
-          if (extra) out_x[t0 + i] = v;
-          else {
-            if (bias) v += bias[row];
-            // device-scope store: written through to where every XCD's loads of that scope see it
-            __hip_atomic_store(&logits[(size_t)(t0 + i) * E + row], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          }
-        }
+        wf = in ? wf : float4{0.f, 0.f, 0.f, 0.f};
+        xf = in ? xf : float4{0.f, 0.f, 0.f, 0.f};
+        acc[i][0] = fma((double)wf.x, (double)xf.x, acc[i][0]);
+        acc[i][1] = fma((double)wf.y, (double)xf.y, acc[i][1]);
+        acc[i][2] = fma((double)wf.z, (double)xf.z, acc[i][2]);
+        acc[i][3] = fma((double)wf.w, (double)xf.w, acc[i][3]);
+        xs[i] += xf.x * xf.x + xf.y * xf.y + xf.z * xf.z + xf.w * xf.w;
       }
     }
   }
-  if (!counter) return;
-  // Hand-over to the block that draws the last ticket (possibly on another XCD).  The logits above are
-  // device-scope atomic stores (written through to the device's coherence point, not left in this XCD's
-  // L2), and every storing wave waits here until the memory system has acknowledged all of them
-  // (vmcnt = 0) before it reaches the barrier; only then does thread 0 take the ticket.  The reader
-  // (topk_block<.., true>) uses device-scope atomic loads issued after its own ticket came back, which
-  // read at that same point.  No cache-wide write-back or invalidate is involved on either side.
-  __builtin_amdgcn_s_waitcnt(0);
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const unsigned ticket = atomicAdd(counter, 1u);
-    s_last = ticket == (unsigned)nrb - 1u;
+#pragma unroll
+  for (int i = 0; i < TT; i++) {
+    sum[i] = wave_sum((acc[i][0] + acc[i][1]) + (acc[i][2] + acc[i][3]));
+    n2[i] = norms ? wave_sum(xs[i]) : 0.f;
   }
-  __syncthreads();
-  if (!s_last) return;
-  for (int t = 0; t < P; t++)
-    topk_block<NPL, true>(logits + (size_t)t * E, ids + (size_t)t * id_stride, ws + (size_t)t * id_stride, E, k);
-  if (threadIdx.x == 0) *counter = 0u;  // re-armed for the next launch on the stream
+}
+
+template <bool BF16, int TT>
+__global__ void __launch_bounds__(128) k_router_small(const void* __restrict__ W, const float* __restrict__ bias,
+                                                      const void* __restrict__ Wx, bool wx_bf16,
+                                                      const float* __restrict__ x, int E, int d,
+                                                      float* __restrict__ logits, float* __restrict__ out_x,
+                                                      int nrows, uint32_t* __restrict__ planes,
+                                                      float2* __restrict__ meta, bool planes_natural, moe_rot_planes rot,
+                                                      float* __restrict__ tol_out, float tol_scale) {
+  // the wave index as a scalar: row, weight type and base address are then wave-uniform values
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int nrb = (nrows + 1) / 2;
+  if ((int)blockIdx.x >= nrb) {
+    router_plane_blocks((int)blockIdx.x - nrb, (int)blockDim.x, (int)threadIdx.x, x, TT, d, planes, meta, planes_natural, rot);
+    return;
+  }
+  const int row = blockIdx.x * 2 + wv;
+  if (row >= nrows) return;
+  const bool extra = row == E;
+  // the wave of row 0 also takes |x|^2 of every token: the selection that follows needs a bound on how far these
+  // sums (lanes, then a tree) can lie from the reference's sequential ones, tol_scale * |x|
+  const bool norms = tol_out && row == 0;
+  double sum[TT];
+  float n2[TT];
+  if (extra && wx_bf16 != BF16) router_small_row<!BF16, TT>(Wx, x, d, lane, false, sum, n2);
+  else router_small_row<BF16, TT>(extra ? Wx : (const void*)((const uint8_t*)W + (uint64_t)row * d * (BF16 ? 2 : 4)), x, d, lane, norms, sum, n2);
+  if (lane != 0) return;
+#pragma unroll
+  for (int i = 0; i < TT; i++) {
+    if (norms) {
+      const float tl = tol_scale * sqrtf(n2[i]) * 1.01f;
+      tol_out[i] = tl >= 0.f ? tl : INFINITY;  // (NaN: nothing is certain)
+    }
+    float v = (float)sum[i];
+    if (extra) {
+      out_x[i] = v;
+    } else {
+      if (bias) v += bias[row];
+      logits[(size_t)i * E + row] = v;
+    }
+  }
 }
 
 // ---- lane-parallel order for 5..32 tokens: four weight rows per block (a wave each); the tokens'
@@ -642,8 +646,8 @@ MOE_API int moe_router_logits(const moe_wview* W, const float* bias, const float
   const bool bf = W->dtype == MOE_DT_BF16;
   const bool par = mode == 0 && P <= 32 && d % 4 == 0 && moe_aligned(x, 16) && moe_aligned(W->data, 16);
   if (par) {
-    return moe_router_logits_small(W, bias, nullptr, x, P, logits, nullptr, nullptr, nullptr, false, nullptr, nullptr,
-                                   nullptr, 0, 0, nullptr, moe_s(st), nullptr, nullptr);
+    return moe_router_logits_small(W, bias, nullptr, x, P, logits, nullptr, nullptr, nullptr, false, moe_s(st), nullptr,
+                                   nullptr);
   } else {
     launch_seq(W->data, bf, bias, x, P, E, d, logits, moe_s(st));
   }
@@ -659,12 +663,10 @@ int moe_router_logits_seq(const moe_wview* W, const float* bias, const float* x,
 }
 
 // Internal: small-P logits plus the shared-expert gate row (and, if planes != nullptr, the digit
-// planes of x for the integer-dot decode kernels) in the same launch.  With a counter (device
-// memory holding 0) and P <= 4 the launch also does the softmax / top-k: *fused_topk says so.
+// planes of x for the integer-dot decode kernels) in the same launch.
 int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x,
                             int P, float* logits, float* out_x, uint32_t* planes, float2* meta,
-                            bool planes_natural, unsigned* counter, int* ids, float* ws, int k, int id_stride, bool* fused_topk,
-                            hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rotp,
+                            bool planes_natural, hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rotp,
                             float* tol_out, float tol_scale) {
   const int E = (int)W->rows, d = (int)W->cols;
   moe_rot_planes rot{nullptr, nullptr, nullptr};
@@ -690,10 +692,9 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
     // two launches of at most 16 tokens read the router matrix twice (L2 / MALL) and are faster
     const int P0 = 16, G = d / 32;
     const size_t pdw = planes_natural ? QV_GROUP_DW : QV4_GROUP_DW;
-    int rc = moe_router_logits_small(W, bias, Wx, x, P0, logits, out_x, planes, meta, planes_natural, nullptr, nullptr,
-                                     nullptr, k, id_stride, nullptr, st, nullptr, nullptr, rotp);
+    int rc = moe_router_logits_small(W, bias, Wx, x, P0, logits, out_x, planes, meta, planes_natural, st, nullptr,
+                                     nullptr, rotp);
     if (rc) return rc;
-    if (fused_topk) *fused_topk = false;
     moe_rot_planes rot2 = rot;
     if (rotp) {
       rot2.planes += (size_t)P0 * G * QV4_GROUP_DW;
@@ -701,27 +702,25 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
     }
     return moe_router_logits_small(W, bias, Wx, x + (size_t)P0 * d, P - P0, logits + (size_t)P0 * E,
                                    out_x ? out_x + P0 : nullptr, planes ? planes + (size_t)P0 * G * pdw : nullptr,
-                                   meta ? meta + (size_t)P0 * G : nullptr, planes_natural, nullptr, nullptr, nullptr, k,
-                                   id_stride, nullptr, st, nullptr, nullptr, rotp ? &rot2 : nullptr);
+                                   meta ? meta + (size_t)P0 * G : nullptr, planes_natural, st, nullptr, nullptr,
+                                   rotp ? &rot2 : nullptr);
   }
   const bool bf = W->dtype == MOE_DT_BF16;
   const bool xbf = Wx && Wx->dtype == MOE_DT_BF16;
   const int nrows = E + (Wx ? 1 : 0);
-  const bool fuse = counter && ids && ws && P <= 4 && E <= 1024;
-  if (fused_topk) *fused_topk = fuse;
-  unsigned* cn = fuse ? counter : nullptr;
-  // one token, no top-k in this launch: two rows per block so that the rows cover every CU
-  // (the fused top-k needs its 256 threads)
-  const int bs = (P == 1 && !fuse && E <= 512) ? 128 : 256, rpb = bs / 64;
+  const int bs = P <= 4 ? 128 : 256, rpb = bs / 64;  // rows per block: one per wave
   const int qblocks = (planes ? P * ((d / 32 + bs - 1) / bs) : 0) + (rot.planes ? P * ((d / 8 + bs - 1) / bs) : 0);
   dim3 g((nrows + rpb - 1) / rpb + qblocks);
   const void* wx = Wx ? Wx->data : nullptr;
-#define RSM_GO(BF, TT, NPL) k_router_small<BF, TT, NPL><<<g, bs, 0, st>>>(W->data, bias, wx, xbf, x, P, E, d, logits, out_x, nrows, planes, meta, planes_natural, cn, ids, ws, k, id_stride, rot, tol_out, tol_scale)
-  if (P == 1 && E <= 512) {
-    if (bf) RSM_GO(true, 1, 8); else RSM_GO(false, 1, 8);
-  } else if (P <= 4) {
-    if (E <= 512) { if (bf) RSM_GO(true, 4, 8); else RSM_GO(false, 4, 8); }
-    else { if (bf) RSM_GO(true, 4, 16); else RSM_GO(false, 4, 16); }
+  if (P <= 4) {
+#define RSM_GO(BF, TT) k_router_small<BF, TT><<<g, bs, 0, st>>>(W->data, bias, wx, xbf, x, E, d, logits, out_x, nrows, planes, meta, planes_natural, rot, tol_out, tol_scale)
+#define RSM_T(TT) do { if (bf) RSM_GO(true, TT); else RSM_GO(false, TT); } while (0)
+    if (P == 1) RSM_T(1);
+    else if (P == 2) RSM_T(2);
+    else if (P == 3) RSM_T(3);
+    else RSM_T(4);
+#undef RSM_T
+#undef RSM_GO
   } else {
     if (mfma_ok) {
       // the f64 matrix pipe: 16 rows per block, columns split over KS blocks and their eight waves
@@ -746,7 +745,6 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
     else { if (bf) RMD_GO(true, 24); else RMD_GO(false, 24); }  // P <= 24 (larger batches were split above)
 #undef RMD_GO
   }
-#undef RSM_GO
   MOE_LAUNCH_CHECK();
   return MOE_OK;
 }

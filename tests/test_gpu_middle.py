@@ -42,6 +42,36 @@ def test_routing_block_edges(capi, oracle, P, E, k, stride):
     r.close()
 
 
+# ---------- router of 1 .. 4 tokens: rows of less than a column step, of ragged steps, of more than one pass over the columns ----------
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("P,E,d", [(1, 33, 4), (2, 9, 252), (3, 512, 2560), (4, 40, 3076), (1, 17, 6400), (3, 8, 3072)])
+def test_router_rows_of_a_few_tokens(capi, oracle, P, E, d, dt):
+    from gfx1151_engine_amd import synth as S
+    rng = np.random.default_rng(100 * P + d)
+    W = rng.standard_normal((E, d), dtype=np.float32) * 0.02
+    x = rng.standard_normal((P, d), dtype=np.float32)
+    if dt == "bf16":
+        W = S.f32_to_bf16_bits(W)
+    lo, _, _ = oracle.router(oracle.Mat(oracle.BF16 if dt == "bf16" else oracle.F32, W, E, d), x, 4)
+    lg = capi.router_logits(capi.wview(gpu(W.view(np.int16) if dt == "bf16" else W), capi.BF16 if dt == "bf16" else capi.F32, E, d),
+                            gpu(x), None, 0).cpu().numpy()
+    assert np.abs(lg - lo).max() <= 2.4e-7 * np.abs(lo).max()  # fp64 sums in another order: at most the last f32 bit
+
+
+@pytest.mark.parametrize("T", [1, 2, 3, 4])
+def test_router_and_gate_vector_of_two_types(capi, oracle, T):
+    rng = np.random.default_rng(T)
+    hl = HostLayer(rng, 768, 256, 33, 5, router_dtype="bf16")  # (the gate vector is f32)
+    x = rng.standard_normal((T, 768), dtype=np.float32)
+    yo, io, _ = oracle.moe_layer(hl.oracle_layer(), x)
+    m, dev = hl.to_gpu(max_tokens=T)
+    y = m.forward(0, gpu(x)).cpu().numpy()
+    ids = m.last_routing(T)[0].cpu().numpy()[:, :5]
+    m.close()
+    assert (ids == io[:, :5]).all()
+    assert max_abs_rel(y, yo) <= 2e-3
+
+
 # ---------- router: edges of its token and expert tiles, the last batch it takes and the first it does not ----------
 @pytest.mark.parametrize("T,E,k,d,dt", [(33, 512, 10, 3072, "bf16"), (64, 33, 5, 256, "f32"), (65, 512, 10, 2560, "f32"),
                                         (515, 512, 10, 768, "bf16"), (1024, 520, 10, 384, "f32"), (1025, 512, 10, 384, "bf16")])
