@@ -94,7 +94,7 @@ struct moe_ctx {
   bool fused_combine = false; // batch path: the down GEMM adds its weighted rows into y with f32 atomics (no pairs buffer, no reduce launch)
   int uq_min = 24;            // > 0: small batches of at least this many tokens read every distinct expert once
   int lut_max = 5;            // q4cp layers off the integer-dot kernels: batches up to this size take the register-resident f32 down kernel
-  int gu_topk_max = 4;        // batches up to this size run the softmax / top-k inside the gate/up launch (else in the router's launches)
+  int gu_topk_max = -1;       // batches up to this size run the softmax / top-k inside the gate/up launch (else in the router's launches); -1: by kernel
   bool uq_gguf = false;       // the same for GGUF layers (off: their per-token kernels measure faster unless most tokens share experts)
   // per-stage timing (the reference's KP("moe:route|up|down|reduce") tags, 07_kprof.inc)
   bool profile = false;
@@ -744,7 +744,12 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
                          (!sh || L.sh_gguf_type != 0);
   // integer-dot kernels: the gate/up launch runs the softmax / top-k itself (one launch less on the
   // latency-bound path than a top-k kernel, no last-block ticket in the logits launch)
-  const bool gu_topk = (((use_int && !use_uq) || ((use_int4k || use_intgg) && !use_uq_gg) || use_lut || use_f32a) && P <= c->gu_topk_max) &&
+  // -- as long as its blocks run in one round: each repeats the selection, 3 .. 4 us, where a launch of its own costs 7.
+  // Two layers, us, in the gate/up launch and aside: look-up kernels (a block per CU) 112 and 101 at 2 tokens, 182 and 154
+  // at 4; GGUF mixes 84.7 and 84.4 at 2, 122 and 119 at 3, 153 and 148 at 4; Q4_K 83.6 and 85.3 at 3, 113 and 108 at 4; q4cp
+  // 73.7 and 76.4 at 3, 100 and 97 at 4
+  const int topk_max = c->gu_topk_max >= 0 ? c->gu_topk_max : use_lut ? 1 : use_intgg ? 2 : use_f32a ? 4 : 3;
+  const bool gu_topk = (((use_int && !use_uq) || ((use_int4k || use_intgg) && !use_uq_gg) || use_lut || use_f32a) && P <= topk_max) &&
                        moe_dec_gu_topk_supported(g.experts, g.topk);
   // (up to 4 tokens the router launch leaves each token's bound for the selection; larger batches: the selecting
   //  block takes the norm of x itself)
@@ -932,7 +937,7 @@ static int forward_small_v2(moe_ctx* c, MoeLayer& L, const float* x, int P, floa
   const bool sh = L.has_shared && !L.sh_dense;  // a q4cp shared expert rides in these kernels as one more slot
   if (sh && (L.sh_gguf_type != 0 || !L.shared_affine)) return MOE_E_UNSUPPORTED;
   const int nslots_d = g.topk + (sh ? 1 : 0);
-  const bool gu_topk = P <= c->gu_topk_max;
+  const bool gu_topk = P <= (c->gu_topk_max >= 0 ? c->gu_topk_max : 4);  // (105 us either way at 4 tokens, two layers)
   const moe_rfix rf = router_fix(c, L, x, P <= 4);
   if ((rc = stage(MOE_PROF_ROUTER, [&]() -> int {
          // (the planes of rot_in(x, su) ride in the router launch's spare blocks)

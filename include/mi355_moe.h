@@ -309,7 +309,7 @@ int moe_forward_x16(moe_ctx* ctx, int layer, const float* x, const void* x16, in
  * tokens has run on the context.  The difference between the times of a loop of calls without and with the skip is
  * that stage's cost inside the pipelined stream, without the dispatch latency that an event pair around a 10 us
  * kernel adds. */
-/* MOE_OPT_GU_TOPK_MAX_TOKENS (default 4: the measured crossover on every weight format): batches of at most this many tokens run the softmax / top-k inside the gate/up launch
+/* MOE_OPT_GU_TOPK_MAX_TOKENS (default: the measured crossover of the kernels a layer takes, 1 .. 4): batches of at most this many tokens run the softmax / top-k inside the gate/up launch
  * (every block of a routed slot selects its token's experts itself: one launch less on the latency-bound path);
  * larger batches of the integer-dot kernels take the ids from the router's launches, so that the thousands of blocks
  * of such a launch do not each repeat the selection. */
