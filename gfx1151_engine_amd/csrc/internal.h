@@ -111,9 +111,10 @@ int moe_launch_reduce(const void* pairs, bool pairs_f16, const int* pairids, con
 // Router of 33 .. MOE_ROUTER_SPLIT_MAX tokens (router_split.hip): fp64 matrix pipe, columns split over waves and blocks, a
 // selecting block per token; what else a batch needs from x comes out of the first launch.
 constexpr int MOE_ROUTER_SPLIT_MAX = 1024, MOE_ROUTER_SPLIT_KS = 8;
-// ... and the size from which the candidate selection (router_cand.hip) goes first: the layer at 400 tokens 536 us with the one,
-// 549 with the other; 515: 568 and 566; 800: 630 and 609
-constexpr int MOE_ROUTER_CAND_MIN = 513;
+// ... and the size from which the candidate selection (router_cand.hip) goes first.  The layer, us, with the one and the other:
+// q4cp 200 tokens 482 and 500, 260 509 and 510, 330 526 and 521, 500 567 and 549; i4r 330 493 and 479; table codebook 330 575
+// and 562; Q5_K / Q8_0 200 740 and 742, 330 783 and 773
+constexpr int MOE_ROUTER_CAND_MIN = 257;
 struct moe_row_extras {
   void* x16;         // f16 copy of x in `layout` (moe_f32_to_f16), or nullptr
   int layout;

@@ -7,7 +7,7 @@
 //                     from it: the f16 copy in the grouped GEMM's order (the router matrix is written in the same order), the
 //                     mean square, the error bound of fp64 sums, the shared expert's gate logit;
 //   2. k_router_f16   all T x E logits from the two f16 copies on the matrix pipe (f32 accumulation);
-//   3. k_router_pick  a wave per token.  A RIGOROUS error bound B_e on each approximate logit (below) gives an interval
+//   3. k_router_pick  a wave per token (small batches: four).  A RIGOROUS error bound B_e on each approximate logit (below) gives an interval
 //                     [a_e - B_e, a_e + B_e] that holds the exact logit; tau = the k-th largest lower end; every expert whose
 //                     upper end reaches tau - 1e-5 is a candidate (the true top k are among them: at least k exact logits are
 //                     >= tau, and a true top-k logit is >= the k-th largest exact one).  The candidates' logits (typically
@@ -198,16 +198,17 @@ __global__ void __launch_bounds__(256, 2) k_router_f16(const __half* __restrict_
 // conversions run at a quarter of the FMA rate and are what bounds this: a lane would otherwise convert activations that
 // 63 others convert too, and does where two rows do not share them).  The next chunk's weights are requested before the
 // current chunk is summed; short chunks, so that four waves fit a SIMD.  Two accumulators per lane and row, a three-step
-// reduction; the order is fixed.
+// reduction; the order is fixed.  Columns c0 .. c0 + d - 1 of rows of ld (multiples of 64, d > 0).
 constexpr int DR_CH = 128;
 template <bool BF16, bool TWO>
-__device__ __forceinline__ void dot_rows(const void* __restrict__ W, const float* __restrict__ xrow, int d, int ra, int rb, int lane,
-                                         double (*xl)[DR_CH], double& sa, double& sb) {
+__device__ __forceinline__ void dot_rows(const void* __restrict__ W, const float* __restrict__ xrow, int ld, int c0, int d, int ra, int rb,
+                                         int lane, double (*xl)[DR_CH], double& sa, double& sb) {
   constexpr int LINE = BF16 ? 64 : 32;  // columns per 128-byte line of a weight row
   constexpr int NL = DR_CH / LINE;      // lines per chunk
   constexpr int ESZ = BF16 ? 2 : 4, NR = TWO ? 2 : 1;
   const int j = lane & 7;
-  const uint8_t* const wrow[2] = {(const uint8_t*)W + (size_t)ra * d * ESZ + 16 * j, (const uint8_t*)W + (size_t)rb * d * ESZ + 16 * j};
+  const uint8_t* const wrow[2] = {(const uint8_t*)W + ((size_t)ra * ld + c0) * ESZ + 16 * j, (const uint8_t*)W + ((size_t)rb * ld + c0) * ESZ + 16 * j};
+  xrow += c0;
   const int nchunk = (d + DR_CH - 1) / DR_CH;
   double a[NR][2];
 #pragma unroll
@@ -289,7 +290,9 @@ struct PickLds {
   int sel_ids[64], redo[4], nlist, nredo;
 };
 
-template <bool BF16>
+// WPT: waves per token (1, 4).  With four, each wave takes a quarter of the columns of the exact dot products; all else runs
+// in every wave alike, so that they agree on every branch.
+template <bool BF16, int WPT>
 __device__ __forceinline__ bool pick_token(PickLds& S, const float* __restrict__ alog, int KS, const float* __restrict__ wnorm, int P,
                                            int E, int d, int k, float eps, float dterm, float bias_max, float xms, int t, int lane,
                                            int wv, int* __restrict__ ids, float* __restrict__ ws, const moe_rfix& RF) {
@@ -391,20 +394,27 @@ __device__ __forceinline__ bool pick_token(PickLds& S, const float* __restrict__
     const int s = p0 + (lane >> 3);
     const int ea = S.cid[wv][s < cnt ? s : p0], eb = S.cid[wv][s + 8 < cnt ? s + 8 : p0];
     double va, vb = 0.0;
-    if (cnt - p0 > 8) dot_rows<BF16, true>(RF.W, xrow, d, ea, eb, lane, S.xl[wv], va, vb);
-    else dot_rows<BF16, false>(RF.W, xrow, d, ea, eb, lane, S.xl[wv], va, vb);
+    const int c0 = WPT == 1 ? 0 : d / 64 * wv / 4 * 64, c1 = WPT == 1 ? d : d / 64 * (wv + 1) / 4 * 64;
+    if (c1 == c0) va = 0.0;  // (fewer than four runs of 64 columns)
+    else if (cnt - p0 > 8) dot_rows<BF16, true>(RF.W, xrow, d, c0, c1 - c0, ea, eb, lane, S.xl[wv], va, vb);
+    else dot_rows<BF16, false>(RF.W, xrow, d, c0, c1 - c0, ea, eb, lane, S.xl[wv], va, vb);
     if ((lane & 7) == 0) {
       S.part[wv][lane >> 3] = va;
       S.part[wv][8 + (lane >> 3)] = vb;
     }
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    __builtin_amdgcn_wave_barrier();
+    if (WPT == 1) {
+      __builtin_amdgcn_s_waitcnt(0xC07F);
+      __builtin_amdgcn_wave_barrier();
+    } else {
+      __syncthreads();
+    }
     const int i = lane - p0;
     if (i >= 0 && i < 16 && lane < cnt) {
-      const double v = S.part[wv][i];
+      const double v = WPT == 1 ? S.part[wv][i] : (S.part[0][i] + S.part[1][i]) + (S.part[2][i] + S.part[3][i]);
       doubt = logit_doubtful(v, tol);
       cv = (float)v + (RF.bias ? RF.bias[S.cid[wv][lane]] : 0.f);
     }
+    if (WPT > 1) __syncthreads();  // (S.part has been read)
   }
   doubt = __any(doubt);
   // rank
@@ -450,27 +460,34 @@ __device__ __forceinline__ bool pick_token(PickLds& S, const float* __restrict__
   const float sc = (float)((double)term / se);
   double wsum = 0.0;
   for (int r = 0; r < k; r++) wsum += (double)__int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc), r));  // selection order, as the reference's loop
-  if (lane < k) {
+  if (lane < k && (WPT == 1 || wv == 0)) {
     ids[lane] = ia;
     ws[lane] = (float)((double)sc / wsum);
   }
   return true;
 }
 
-template <bool BF16>
+// Batches up to this size give a token to four waves: with one, the chip holds a wave or less per SIMD that walks the 3072
+// columns in 24 dependent steps, 37 us whatever the number of tokens.  In four waves the walk is six steps, 21 us at 515
+// tokens, but each repeats the selection around it, which counts as soon as the SIMDs are full (three blocks per CU: 768
+// tokens).  The layer with one wave and with four, us: 600 tokens 568 and 558, 900 616 and 610, 1200 648 and 648, 1500 685 and
+// 695.
+constexpr int PICK_SPLIT_MAX = 1024;
+
+template <bool BF16, int WPT>
 __global__ void __launch_bounds__(256, 3) k_router_pick(const float* __restrict__ alog, int KS, const float* __restrict__ wnorm,
                                                         const float* __restrict__ xms, int P, int E, int d, int k, float eps, float dterm,
                                                         float bias_max, int* __restrict__ ids, float* __restrict__ ws, int id_stride,
                                                         moe_rfix RF) {
   __shared__ __attribute__((aligned(16))) PickLds S;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int t = blockIdx.x * 4 + wv;
+  const int t = WPT == 1 ? blockIdx.x * 4 + wv : blockIdx.x;
   if (tid == 0) S.nredo = 0;
   __syncthreads();
   if (t < P) {
-    const bool ok = pick_token<BF16>(S, alog, KS, wnorm, P, E, d, k, eps, dterm, bias_max, xms[t], t, lane, wv,
+    const bool ok = pick_token<BF16, WPT>(S, alog, KS, wnorm, P, E, d, k, eps, dterm, bias_max, xms[t], t, lane, wv,
                                      ids + (size_t)t * id_stride, ws + (size_t)t * id_stride, RF);
-    if (!ok && lane == 0) S.redo[atomicAdd(&S.nredo, 1)] = t;
+    if (!ok && lane == 0 && (WPT == 1 || wv == 0)) S.redo[atomicAdd(&S.nredo, 1)] = t;
   }
   __syncthreads();
   const int nredo = S.nredo;
@@ -487,7 +504,7 @@ __global__ void __launch_bounds__(256, 3) k_router_pick(const float* __restrict_
     for (int e0 = zero ? E : 16 * wv; e0 < E; e0 += 64) {
       const int ea = e0 + (lane >> 3), eb = ea + 8;
       double va, vb;
-      dot_rows<BF16, true>(RF.W, RF.x + (size_t)tr * d, d, ea < E ? ea : E - 1, eb < E ? eb : E - 1, lane, S.xl[wv], va, vb);
+      dot_rows<BF16, true>(RF.W, RF.x + (size_t)tr * d, d, 0, d, ea < E ? ea : E - 1, eb < E ? eb : E - 1, lane, S.xl[wv], va, vb);
       if ((lane & 7) == 0) {
         if (ea < E) {
           if (logit_doubtful(va, tol)) S.list[atomicAdd(&S.nlist, 1)] = ea;
@@ -564,8 +581,15 @@ int moe_router_batch_cand(const moe_wview* W, const float* x, int P, float* logi
   if (s.mt == 2) k_router_f16<2><<<g2, 256, 0, st>>>(W16, (const __half*)R.x16, P, E, d, alog, s.ncol, s.ntt, s.ks);
   else k_router_f16<1><<<g2, 256, 0, st>>>(W16, (const __half*)R.x16, P, E, d, alog, s.ncol, s.ntt, s.ks);
   MOE_LAUNCH_CHECK();
-  if (bf) k_router_pick<true><<<g3, 256, 0, st>>>(alog, s.ks, wnorm, R.xms, P, E, d, k, eps, dterm, bias_max, ids, ws, id_stride, RF);
-  else k_router_pick<false><<<g3, 256, 0, st>>>(alog, s.ks, wnorm, R.xms, P, E, d, k, eps, dterm, bias_max, ids, ws, id_stride, RF);
+#define PICK_GO(BF, WPT) k_router_pick<BF, WPT><<<WPT == 1 ? g3 : (unsigned)P, 256, 0, st>>>(alog, s.ks, wnorm, R.xms, P, E, d, k, eps, dterm, bias_max, ids, ws, id_stride, RF)
+  if (P <= PICK_SPLIT_MAX) {
+    if (bf) PICK_GO(true, 4);
+    else PICK_GO(false, 4);
+  } else {
+    if (bf) PICK_GO(true, 1);
+    else PICK_GO(false, 1);
+  }
+#undef PICK_GO
   MOE_LAUNCH_CHECK();
   return MOE_OK;
 }

@@ -3,8 +3,8 @@
 // split over the waves of a block and over blocks, then one selecting block per token.  Two launches.
 // (reference arithmetic: src/ref.cpp:68-77,565-594)
 //
-// The candidate selection of router_cand.hip pays off once its third launch, a chain of about 30 us, is small against the
-// fp64 work it saves.  At a few hundred tokens it is not: all 130 x 512 sums are 0.2 G fp64 FMAs, 5 us of the chip's f64
+// The candidate selection of router_cand.hip pays off once its third launch, a chain of 15 .. 20 us, is small against the
+// fp64 work it saves.  At 130 tokens it is not: all 130 x 512 sums are 0.2 G fp64 FMAs, 5 us of the chip's f64
 // matrix rate.  What that needs is enough waves, so columns are dealt out: a block is 32 tokens x 32 experts x one of KS
 // column shares, its eight waves take an eighth of the share each and their partial tiles are added in wave order through
 // LDS; the KS shares' fp64 partial sums go to memory and the selecting block of a token adds them in share order.  Every

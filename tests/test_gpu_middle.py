@@ -137,6 +137,33 @@ def test_router_candidates(capi, oracle, T, E, k, d, dt, fmt):
     assert np.abs(ws - wo[:, :k]).max() <= 2.5e-7
 
 
+# ... at the sizes where four waves share a token: the smallest and largest, rows of fewer runs than waves, uneven shares, a
+# second pass over the candidates (many close logits)
+@pytest.mark.parametrize("T,E,k,d,dt,fmt,std", [(257, 512, 10, 3072, "f32", "q4cp", 0.02), (258, 43, 15, 192, "bf16", "q8_0", 0.02),
+                                                (300, 512, 10, 320, "f32", "q8_0", 0.02), (301, 300, 15, 512, "bf16", "q4cp", 0.0005),
+                                                (1024, 128, 4, 128, "f32", "q8_0", 0.02), (1025, 128, 4, 128, "f32", "q8_0", 0.02)])
+def test_router_candidates_of_small_batches(capi, oracle, T, E, k, d, dt, fmt, std):
+    rng = np.random.default_rng(T)
+    kw = dict(fmt="q4k", gg_types=(8, 8, 8)) if fmt == "q8_0" else {}
+    hl = HostLayer(rng, d, 256, E, k, router_dtype=dt, router_std=std, shared=False, **kw)
+    hl.router[E - 1] = hl.router[2]
+    if dt == "f32":
+        hl.router[E // 2] = hl.router[1] * np.float32(1 + 2 ** -22)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    x[5] = 0.0
+    x[6, 3] = 1e6
+    x[7] *= 300.0
+    x[T - 1] = x[0]
+    lo, io, wo = oracle.router(hl.oracle_layer().router, x, k)
+    m, dev = hl.to_gpu(max_tokens=T)
+    m.forward(0, gpu(x))
+    assert m.last_path() == capi.PATH_BATCH
+    ids, ws = (a.cpu().numpy()[:, :k] for a in m.last_routing(T))
+    m.close()
+    assert (ids == io[:, :k]).all()
+    assert np.abs(ws - wo[:, :k]).max() <= 2.5e-7
+
+
 # ---------- grouped GEMM over tiles of few pairs: every format, tile size and side of a line between them ----------
 TABLE = np.array([-1.0, -0.7, -0.53, -0.4, -0.28, -0.18, -0.09, 0.0, 0.08, 0.16, 0.25, 0.34, 0.44, 0.56, 0.72, 1.0], np.float32)
 
