@@ -1,7 +1,5 @@
 // Router: logits with the CPU path's fp64 accumulation, fp64 softmax, top-k, renormalised weights.
 // (reference: src/ref.cpp:68-77,565-594; src/gpu/parts/20_kernels_gemv.inc:1433-1562)
-#include <type_traits>
-
 #include "common.h"
 #include "hv2.h"
 #include "internal.h"
@@ -233,19 +231,17 @@ __device__ __forceinline__ void router_small_row(const void* __restrict__ Wr, co
 #pragma unroll
     for (int q = 0; q < 4; q++) acc[i][q] = 0.0;
   }
-  // FULL: every step lies inside the row
-  auto steps = [&](auto fullc, int c0) {
-    constexpr bool FULL = decltype(fullc)::value;
+  for (int c0 = 0; c0 < d; c0 += 256 * RSM_IT) {
     WT w[RSM_IT];
     float4 xv[2][RSM_IT];  // a token's activations, and the next one's
     auto load_x = [&](int i, int j) {
       const int c = c0 + 256 * j + 4 * lane;
-      xv[i & 1][j] = *(const float4*)(x + (size_t)i * d + (FULL || c < d ? c : 0));
+      xv[i & 1][j] = *(const float4*)(x + (size_t)i * d + (c < d ? c : 0));
     };
 #pragma unroll
     for (int j = 0; j < RSM_IT; j++) {
       const int c = c0 + 256 * j + 4 * lane;
-      w[j] = *(const WT*)((const uint8_t*)Wr + (size_t)(FULL || c < d ? c : 0) * (BF ? 2 : 4));  // (past the row: its head, not used)
+      w[j] = *(const WT*)((const uint8_t*)Wr + (size_t)(c < d ? c : 0) * (BF ? 2 : 4));  // (past the row: its head, not used)
       load_x(0, j);  // (in the order of use: the sums start when the first pair is there)
     }
 #pragma unroll
@@ -257,7 +253,7 @@ __device__ __forceinline__ void router_small_row(const void* __restrict__ Wr, co
 #pragma unroll
       for (int j = 0; j < RSM_IT; j++) {
         // (columns past the row count as zeros: selects, where a branch would make the step wait for its own loads)
-        const bool in = FULL || c0 + 256 * j + 4 * lane < d;
+        const bool in = c0 + 256 * j + 4 * lane < d;
         float4 wf, xf = xv[i & 1][j];
         if constexpr (BF) {
           wf.x = __uint_as_float(w[j].x << 16);
@@ -276,15 +272,6 @@ __device__ __forceinline__ void router_small_row(const void* __restrict__ Wr, co
         xs[i] += xf.x * xf.x + xf.y * xf.y + xf.z * xf.z + xf.w * xf.w;
       }
     }
-  };
-  for (int c0 = 0; c0 < d; c0 += 256 * RSM_IT) {
-    if constexpr (TT < 4) {  // (four tokens: two copies of the body, and the compiler spills)
-      if (c0 + 256 * RSM_IT <= d) {
-        steps(std::true_type{}, c0);
-        continue;
-      }
-    }
-    steps(std::false_type{}, c0);
   }
 #pragma unroll
   for (int i = 0; i < TT; i++) {
