@@ -210,7 +210,15 @@ __device__ __forceinline__ void router_plane_blocks(int q, int bs, int tid, cons
 // column step, each step waited for its own loads (512 experts, 3072 columns, bf16 matrix and f32 gate vector: one token 8.4 us,
 // three tokens 16.2; now 4.0 and 5.9).  One token on an f32 matrix, where the compiler had untangled the loop: 4.1 before and
 // now; with all weights requested ahead of all activations instead of pair by pair 4.5.
-constexpr int RSM_IT = 12;  // column steps of 256 requested together
+// Four tokens take 306 of the 512 registers a wave can have (AGPRs among them).  One body serves rows of any length: with a
+// second copy for passes that lie wholly inside the row, without the selects below, three tokens of 3072 columns gain 1 us
+// of 120 in two layers, and the compiler keeps 415 registers of the four-token kernel in scratch: 98 -> 130 us (q4cp), 150 ->
+// 190 (Q5_K / Q8_0).
+// Column steps of 256 requested together: what registers and one trip allow.  Steps past the row's end load its head again.
+// Two q4cp layers of 1 / 2 / 3 / 4 tokens, us, against one load in flight per step: 1024 columns 34 / 39 / 48 / 58 (34 / 42 /
+// 53 / 60), 2048 37 / 53 / 63 / 78 (42 / 60 / 74 / 93), 2560 38 / 46 / 63 / 80 (45 / 57 / 78 / 94), 4096 86 / 130 / 127 / 148 (93 / 148 / 149 /
+// 178), 5120 99 / 134 / 165 / 200 (109 / 158 / 206 / 257).
+constexpr int RSM_IT = 12;
 template <bool BF>
 struct RsmW {
   typedef float4 T;
