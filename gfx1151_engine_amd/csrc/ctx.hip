@@ -1214,9 +1214,8 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   // router: column-split fp64 launches for middle sizes (router_split.hip), above candidate selection (router_cand.hip); their
   // first launches make the f16 copy of x as well.  MOE_OPT_ROUTER_CANDIDATES = 0, or a shape they do not take: the dense
   // fp64 launch and the exact softmax / top-k over all experts.
-  const moe_wview* const wx = L.has_shared ? &L.sh_sg : nullptr;
-  const bool cand_router = P >= MOE_ROUTER_CAND_MIN && c->router_cand && c->rc_scratch && moe_router_cand_supported(&L.router, wx, P, g.topk);
-  const bool mid_router = !cand_router && c->router_cand && c->gpart && moe_router_split_supported(&L.router, wx, P, g.topk);
+  const bool cand_router = P >= MOE_ROUTER_CAND_MIN && c->router_cand && c->rc_scratch && moe_router_cand_supported(&L.router, P, g.topk);
+  const bool mid_router = !cand_router && c->router_cand && c->gpart && moe_router_split_supported(&L.router, P, g.topk);
   // The shared expert in launches of its own, on the context's side stream: where its kernels differ from the routed
   // experts', and for batches whose router takes long enough to hide them (at middle sizes they ride along: the
   // router is two short launches there, and the shared expert's few tiles alone leave the chip idle).

@@ -126,7 +126,7 @@ struct moe_row_extras {
   float* out_x;      // [P] its logit
 };
 int moe_launch_row_extras(const float* x, int P, int d, const moe_row_extras& R, hipStream_t st);  // (reduce.hip)
-bool moe_router_split_supported(const moe_wview* W, const moe_wview* Wx, int P, int k);
+bool moe_router_split_supported(const moe_wview* W, int P, int k);
 size_t moe_router_split_scratch_bytes(int max_tokens, int experts, int d);
 int moe_router_batch_split(const moe_wview* W, const float* x, int P, int* ids, float* ws, int k,
                            int id_stride, double* gpart, const moe_row_extras& R, const moe_rfix& RF, hipStream_t st,
@@ -135,7 +135,7 @@ int moe_router_batch_split(const moe_wview* W, const float* x, int P, int* ids, 
 int moe_router_logits_seq(const moe_wview* W, const float* bias, const float* x, int P, float* logits, hipStream_t st);
 // Router of larger batches through candidate selection (router_cand.hip): bit-exact ids, weights within an ulp or two.  Its
 // first launch leaves what else a batch needs from x; R.x16 is required.
-bool moe_router_cand_supported(const moe_wview* W, const moe_wview* Wx, int P, int k);
+bool moe_router_cand_supported(const moe_wview* W, int P, int k);
 size_t moe_router_cand_scratch_bytes(int max_tokens, int experts, int d);
 int moe_router_batch_cand(const moe_wview* W, const float* x, int P, float* logits, int* ids, float* ws, int k, int id_stride,
                           void* scratch, const moe_row_extras& R, const moe_rfix& RF, float bias_max, hipStream_t st,

@@ -228,7 +228,7 @@ int moe_launch_tiles_only_shared(moe_tile* tiles, int* ntiles, int E, int cap, i
 // f16 copy, mean square, gate logit of every row in one launch
 int moe_launch_row_extras(const float* x, int P, int d, const moe_row_extras& R, hipStream_t st) {
   if (!x || R.layout < 0 || R.layout > 2 || (R.wx && !R.out_x)) return MOE_E_INVALID;
-  if (d % 8 || (R.layout == 2 && d % 64) || !moe_aligned(x, 16) || !moe_aligned(R.x16, 16) || !moe_aligned(R.wx, 16)) return MOE_E_INVALID;
+  if (d % 8 || (R.layout == 2 && d % 64) || !moe_aligned(x, 16) || !moe_aligned(R.x16, 16)) return MOE_E_INVALID;
   if (P == 0) return MOE_OK;
   k_row_extras<<<(P + 3) / 4, 256, 0, st>>>(x, P, d, R);
   MOE_LAUNCH_CHECK();

@@ -4,6 +4,7 @@
 #include "hv2.h"
 #include "internal.h"
 #include "qvec.h"
+#include "rowx.h"
 #include "topk.h"
 
 namespace {
@@ -221,11 +222,11 @@ __device__ __forceinline__ void router_plane_blocks(int q, int bs, int tid, cons
 constexpr int RSM_IT = 12;
 template <bool BF>
 struct RsmW {
-  typedef float4 T;
+  typedef gate_f32x4 T;
 };
 template <>
 struct RsmW<true> {
-  typedef uint2 T;
+  typedef gate_bf16x4 T;
 };
 template <bool BF, int TT>
 __device__ __forceinline__ void router_small_row(const void* __restrict__ Wr, const float* __restrict__ x, int d, int lane,
@@ -269,7 +270,7 @@ __device__ __forceinline__ void router_small_row(const void* __restrict__ Wr, co
           wf.z = __uint_as_float(w[j].y << 16);
           wf.w = __uint_as_float(w[j].y & 0xffff0000u);
         } else {
-          wf = w[j];
+          wf = float4{w[j].x, w[j].y, w[j].z, w[j].w};
         }
         wf = in ? wf : float4{0.f, 0.f, 0.f, 0.f};
         xf = in ? xf : float4{0.f, 0.f, 0.f, 0.f};
@@ -377,8 +378,8 @@ __global__ void __launch_bounds__(256) k_router_mid(const void* __restrict__ W, 
     const int cc = c < d ? c : 0;
     // two 32-bit loads in either format (bf16: the same word twice), so no branch surrounds them
     const uint8_t* p0 = (const uint8_t*)Wr + (base + cc) * (bf ? 2 : 4);
-    wr[j].x = *(const uint32_t*)p0;
-    wr[j].y = *(const uint32_t*)(p0 + (bf ? 0 : 4));
+    wr[j].x = *(const gate_bf16x2*)p0;
+    wr[j].y = *(const gate_bf16x2*)(p0 + (bf ? 0 : 4));
   };
   auto weights = [&](int j, int c0, double& w0, double& w1) {
     const float m = c0 + 2 * lane < d ? 1.f : 0.f;
@@ -545,7 +546,7 @@ __global__ void __launch_bounds__(512, 2) k_router_mfma(const void* __restrict__
     const int c = k0 + 16 * (it < nit ? it : nit - 1);  // past the end: a repeat that is never used
     // 16 bytes in either format (bf16: 8 bytes twice), so no branch surrounds the load
     const uint8_t* p = wrow + (size_t)c * (wbf ? 2 : 4);
-    const uint2 lo = *(const uint2*)p, hi = *(const uint2*)(p + (wbf ? 0 : 8));
+    const gate_bf16x4 lo = *(const gate_bf16x4*)p, hi = *(const gate_bf16x4*)(p + (wbf ? 0 : 8));
     wr[j] = make_uint4(lo.x, lo.y, hi.x, hi.y);
 #pragma unroll
     for (int tt = 0; tt < NTT; tt++) xr[j][tt] = *(const float4*)(xrow[tt] + c);

@@ -545,10 +545,10 @@ F16Shape f16_shape(int P, int E, int d) {
 
 }  // namespace
 
-bool moe_router_cand_supported(const moe_wview* W, const moe_wview* Wx, int P, int k) {
+bool moe_router_cand_supported(const moe_wview* W, int P, int k) {
   const int E = (int)W->rows, d = (int)W->cols;
   if (P < 1 || d % 64 || d < 64 || E > 512 || k + 1 > RC_SLOTS - 1 || k >= E) return false;
-  return moe_aligned(W->data, 16) && (!Wx || moe_aligned(Wx->data, 16));
+  return moe_aligned(W->data, 16);
 }
 
 static size_t rc_wnorm_bytes(int experts) { return ((size_t)experts * 4 + 255) / 256 * 256; }
@@ -563,7 +563,7 @@ int moe_router_batch_cand(const moe_wview* W, const float* x, int P, float* logi
                           void* scratch, const moe_row_extras& R, const moe_rfix& RF, float bias_max, hipStream_t st,
                           hipEvent_t after_rows) {
   const int E = (int)W->rows, d = (int)W->cols;
-  if (!moe_router_cand_supported(W, nullptr, P, k) || !moe_aligned(x, 16) || !R.x16 || !R.xms || !R.tol) return MOE_E_UNSUPPORTED;
+  if (!moe_router_cand_supported(W, P, k) || !moe_aligned(x, 16) || !R.x16 || !R.xms || !R.tol) return MOE_E_UNSUPPORTED;
   float* wnorm = (float*)scratch;
   __half* W16 = (__half*)((uint8_t*)scratch + rc_wnorm_bytes(E));
   const F16Shape s = f16_shape(P, E, d);

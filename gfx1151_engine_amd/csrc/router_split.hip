@@ -203,9 +203,8 @@ int split_shares(int P, int E, int d) {
 
 }  // namespace
 
-bool moe_router_split_supported(const moe_wview* W, const moe_wview* Wx, int P, int k) {
-  return P >= 1 && P <= MOE_ROUTER_SPLIT_MAX && W->rows <= 1024 && k <= 63 && W->cols % 32 == 0 && moe_aligned(W->data, 16) &&
-         (!Wx || moe_aligned(Wx->data, 16));
+bool moe_router_split_supported(const moe_wview* W, int P, int k) {
+  return P >= 1 && P <= MOE_ROUTER_SPLIT_MAX && W->rows <= 1024 && k <= 63 && W->cols % 32 == 0 && moe_aligned(W->data, 16);
 }
 
 size_t moe_router_split_scratch_bytes(int max_tokens, int experts, int d) {

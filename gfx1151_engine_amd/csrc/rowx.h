@@ -25,6 +25,12 @@ __device__ __forceinline__ uint4 f16_chunk(int layout, const float4& u, const fl
   return o;
 }
 
+// Four (two) values of the gate vector, which may start at any element (moe_set_shared asks for no more; the loads are the same single
+// instructions as for aligned ones).
+typedef float gate_f32x4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t gate_bf16x4 __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t gate_bf16x2 __attribute__((aligned(2)));
+
 // the f16 copy (layout as moe_f32_to_f16's), the mean square, the selection's error bound and the shared expert's gate
 // logit (fp64 sum) of row t; each is left out where its pointer is null
 // (chunks of 8 columns i0, i0 + step, ...: this thread's part of the row's sums in acc and gate)
@@ -46,13 +52,13 @@ __device__ __forceinline__ void row_extras_part(const float* __restrict__ x, int
     if (R.wx) {
       float g[8];
       if (R.wx_bf16) {
-        const uint2 p = ((const uint2*)R.wx)[ia], q = ((const uint2*)R.wx)[ib];
+        const gate_bf16x4 p = ((const gate_bf16x4*)R.wx)[ia], q = ((const gate_bf16x4*)R.wx)[ib];
         g[0] = __uint_as_float(p.x << 16); g[1] = __uint_as_float(p.x & 0xffff0000u);
         g[2] = __uint_as_float(p.y << 16); g[3] = __uint_as_float(p.y & 0xffff0000u);
         g[4] = __uint_as_float(q.x << 16); g[5] = __uint_as_float(q.x & 0xffff0000u);
         g[6] = __uint_as_float(q.y << 16); g[7] = __uint_as_float(q.y & 0xffff0000u);
       } else {
-        const float4 p = ((const float4*)R.wx)[ia], q = ((const float4*)R.wx)[ib];
+        const gate_f32x4 p = ((const gate_f32x4*)R.wx)[ia], q = ((const gate_f32x4*)R.wx)[ib];
         g[0] = p.x; g[1] = p.y; g[2] = p.z; g[3] = p.w; g[4] = q.x; g[5] = q.y; g[6] = q.z; g[7] = q.w;
       }
       gate = fma((double)g[0], (double)u.x, gate); gate = fma((double)g[1], (double)u.y, gate);

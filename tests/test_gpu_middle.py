@@ -72,6 +72,29 @@ def test_router_and_gate_vector_of_two_types(capi, oracle, T):
     assert max_abs_rel(y, yo) <= 2e-3
 
 
+# ---------- the shared expert's gate vector may start at any element, whatever router a batch takes ----------
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("T,candidates", [(1, 1), (4, 1), (6, 1), (20, 1), (32, 1), (40, 1), (256, 1), (300, 1), (40, 0), (300, 0)])
+def test_gate_vector_at_any_element(capi, T, candidates, dt):
+    import torch
+    rng = np.random.default_rng(T)
+    d, mid = 512, 256
+    hl = HostLayer(rng, d, mid, 32, 4, router_dtype=dt)
+    m, dev = hl.to_gpu(max_tokens=T)
+    m.set_option(capi.OPT_ROUTER_CANDIDATES, candidates)
+    gate = dev["shsg"].reshape(-1).to(torch.bfloat16 if dt == "bf16" else torch.float32)
+    x = gpu(rng.standard_normal((T, d), dtype=np.float32))
+    ys = []
+    for off in (0, 1, 3):
+        room = torch.zeros(d + 8, dtype=gate.dtype, device="cuda")
+        room[off:off + d] = gate
+        m.set_shared(0, *(capi.wview(dev[n], capi.Q4CP, r, c) for n, r, c in (("shg", mid, d), ("shu", mid, d), ("shd", d, mid))),
+                     capi.wview(room[off:], capi.BF16 if dt == "bf16" else capi.F32, 1, d))
+        ys.append(m.forward(0, x).cpu())
+    m.close()
+    assert torch.equal(ys[0], ys[1]) and torch.equal(ys[0], ys[2])
+
+
 # ---------- router: edges of its token and expert tiles, the last batch it takes and the first it does not ----------
 @pytest.mark.parametrize("T,E,k,d,dt", [(33, 512, 10, 3072, "bf16"), (64, 33, 5, 256, "f32"), (65, 512, 10, 2560, "f32"),
                                         (515, 512, 10, 768, "bf16"), (1024, 520, 10, 384, "f32"), (1025, 512, 10, 384, "bf16")])
