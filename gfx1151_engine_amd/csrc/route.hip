@@ -27,8 +27,19 @@ constexpr int RT_MAXE = 1024;
 //  at 16384)
 // KV: a token's picks as KV 16-byte loads (k <= 4 KV, rows of ids aligned for it); 0 = any k, read one by one.
 enum { ROUTE_ONE, ROUTE_COUNT, ROUTE_PLACE };
-int route_block_tokens(int E) { return E <= 512 ? 1024 : 512; }  // tokens of a block: the masks fit its LDS
-size_t route_lds_bytes(int E, int waves) { return (size_t)waves * E * 10 + (size_t)E * 4; }
+constexpr int route_block_tokens(int E) { return E <= 512 ? 1024 : 512; }  // tokens of a block: the masks fit its LDS
+constexpr size_t route_lds_bytes(int E, int waves) { return (size_t)waves * E * 10 + (size_t)E * 4; }
+// the most a launch asks for (1024 experts, 512 tokens: 86016 bytes; 512 experts, 1024 tokens: 83968)
+constexpr size_t route_lds_most() {
+  size_t most = 0;
+  for (int E = 1; E <= RT_MAXE; E++) {
+    const size_t n = route_lds_bytes(E, route_block_tokens(E) / 64);
+    most = n > most ? n : most;
+  }
+  return most;
+}
+constexpr size_t ROUTE_LDS_MOST = route_lds_most();
+static_assert(ROUTE_LDS_MOST + 4096 <= 160 * 1024, "a CU's LDS");
 // A block writes the pairs of an eighth of its tokens only (RT_SUB blocks per token block, each building the same masks):
 // the scattered stores are single lanes' cache lines, 1024 tokens' worth of them kept one CU busy for 17 us.
 constexpr int RT_SUB = 8;
@@ -222,7 +233,7 @@ static int route_launch(unsigned grid, size_t lds, hipStream_t st, const int* id
   static moe_dev_once once;
   int dev;
   if (moe_dev_pending(once, &dev)) {
-    MOE_HIP(hipFuncSetAttribute((const void*)k_route<KV, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)route_lds_bytes(512, 16)));
+    MOE_HIP(hipFuncSetAttribute((const void*)k_route<KV, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ROUTE_LDS_MOST));
     moe_dev_done(once, dev);
   }
   k_route<KV, MODE><<<grid, RT_MAXE, lds, st>>>(ids, ws, P, k, E, id_stride, tpb, blockcnt, tokidx, pw, eoff, pairids, tiles,

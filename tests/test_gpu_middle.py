@@ -25,6 +25,7 @@ def gpu(a):
 # ---------- permutation: one block of tokens, its writers, several blocks ----------
 @pytest.mark.parametrize("P,E,k,stride", [(64, 512, 10, 16), (128, 512, 10, 16), (129, 64, 4, 16), (1024, 512, 10, 16),
                                           (1025, 512, 10, 16), (2049, 8, 3, 4), (512, 1000, 12, 16), (513, 1000, 13, 16),
+                                          (512, 1024, 10, 16), (600, 1024, 15, 16), (1024, 513, 10, 16),
                                           (700, 30, 17, 20), (1100, 30, 17, 17)])
 def test_routing_block_edges(capi, oracle, P, E, k, stride):
     rng = np.random.default_rng(P + E)
