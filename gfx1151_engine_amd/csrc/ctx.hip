@@ -14,7 +14,7 @@ struct MoeLayer {
   moe_wview router{};
   const float* router_bias = nullptr;
   float router_wmax = 0.f;  // the largest row norm of the router matrix (the bound of the small-batch selection, moe_rfix)
-  float router_bmax = 0.f;  // the largest |bias| (how far a logit's dot product can lie above the logit itself)
+  float router_bmax = 0.f;  // the largest |bias| (how far a logit's dot product can lie above the logit itself; experts switched off by a bias of minus infinity aside)
   moe_wview gate_up{}, down{};
   moe_gg_experts gg{};
   moe_wview sh_gate{}, sh_up{}, sh_down{}, sh_sg{};
@@ -319,7 +319,8 @@ MOE_API int moe_set_router(moe_ctx* c, int layer, const moe_wview* w, const floa
   if (bias) {
     std::vector<float> hb((size_t)w->rows);
     MOE_HIP(hipMemcpy(hb.data(), bias, hb.size() * 4, hipMemcpyDeviceToHost));
-    for (float b : hb) L->router_bmax = fmaxf(L->router_bmax, fabsf(b));
+    for (float b : hb)
+      if (b != -INFINITY) L->router_bmax = fmaxf(L->router_bmax, fabsf(b));
   }
   L->router = *w;
   L->router_bias = bias;

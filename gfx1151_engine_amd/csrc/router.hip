@@ -442,7 +442,7 @@ template <int NPL>
 __global__ void __launch_bounds__(256) k_router_topk(const float* __restrict__ logits,
                                                      int* __restrict__ ids, float* __restrict__ ws,
                                                      int P, int E, int k, int id_stride) {
-  __shared__ float pbuf[4][64 * NPL];
+  __shared__ __attribute__((aligned(16))) float pbuf[4][64 * NPL];
   const int wv = threadIdx.x >> 6;
   const int tok = blockIdx.x * 4 + wv;
   if (tok >= P) return;

@@ -1,4 +1,5 @@
-// Batch router without the dense fp64 pass: bit-exact expert ids at a fraction of the fp64 work.  Three launches.
+// Batch router without the dense fp64 pass: bit-exact expert ids at a fraction of the fp64 work.  Three launches, and a
+// fourth for the tokens that the selection cannot settle, whose blocks return at once where there are none.
 //
 // The reference's router (src/ref.cpp:565-594) needs every logit as a sequential fp64 sum, but only the k
 // best logits of a token decide its experts and weights; the other ~500 enter through the softmax
@@ -18,14 +19,15 @@
 //                     logit is the reference's order by f32 probability and the ids are final; the weights use these logits
 //                     and a normaliser in which the non-candidates' terms are approximate, which moves a renormalised weight
 //                     by an ulp or two at most.  Tokens that fail any test (near ties, a logit range where probabilities
-//                     underflow, more candidates than slots, non-finite values) are redone by their whole block: all E
-//                     logits as fp64 sums, the doubtful ones as the reference's chains (router_chain.h).
+//                     underflow, more candidates than slots, non-finite values) are listed; rows of zeros (padding) are
+//                     settled by their block, which knows their sums;
+//   4. k_router_listed  listed tokens, sixteen at a time, as the reference's chains on the f64 matrix pipe.
 // Error bound.  a~ = fl32(sum of f16(x_c) * f16(w_c)): |f16(v) - v| <= 2^-11 |v| + 2^-25 (the second term covers
 // f16 subnormals), so sum |x~ w~ - x w| <= 1.001 (2^-10 |x||w| + 2^-25 sqrt(d) (|x| + |w|)) by Cauchy-Schwarz, and
 // the accumulation adds at most (RA_CHUNK * 2^-22 + (d / RA_CHUNK + RA_KS) * 2^-23) * 1.001 |x||w|: inside a chunk of RA_CHUNK
 // columns however the matrix pipe orders and rounds its partial sums (twice the IEEE bound per addition, one addition
 // charged per product), plus one IEEE f32 addition per chunk for the running sum and per column share.  Non-finite
-// approximations (overflow of the f16 conversions) send the token to the redo.
+// approximations (overflow of the f16 conversions) put the token on the list.
 // Measured (512 experts, top-10; prep + f16 + pick, us): 2048 tokens, d = 2560, f32 router 12 + 17 + 35; 3001, d = 3072 17 + 24 + 48;
 // 16384 61 + 85 + 225 -- against 209, 223 and 690 for the eight launches that were here before (W and x converted by the f16
 // launch, which had 32 blocks at 2048 tokens; candidates, exact pairs, ranking and three launches for the redo, 60 us when
@@ -45,13 +47,18 @@ constexpr int RA_CHUNK = 128;  // columns summed in the matrix pipe's f32 accumu
 constexpr int RA_KS = 4;       // column shares at most
 constexpr int RA_NBUF = 4;     // slabs in LDS
 constexpr int RC_SLOTS = 32;   // candidates per token at most
+constexpr int RL_T = 16;       // listed tokens of a group
 
 // ---- 1. a wave per row: first the router matrix's, then x's ----
 template <bool BF16>
 __global__ void __launch_bounds__(256) k_router_prep(const void* __restrict__ W, int E, int d, __half* __restrict__ W16,
-                                                     float* __restrict__ wnorm, const float* __restrict__ x, int P,
-                                                     moe_row_extras R) {
+                                                     float* __restrict__ wnorm, int* __restrict__ hard,
+                                                     const float* __restrict__ x, int P, moe_row_extras R) {
   const int lane = threadIdx.x & 63, nwb = (E + 3) >> 2;
+  {  // the list's count and its tickets (first used two launches on)
+    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
+    if (i <= (P + RL_T - 1) / RL_T) hard[i] = 0;
+  }
   if ((int)blockIdx.x < nwb) {
     const int e = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (e >= E) return;
@@ -279,15 +286,12 @@ __device__ __forceinline__ void dot_rows(const void* __restrict__ W, const float
 
 // ---- 3. candidates, their exact logits, ids and weights ----
 struct PickLds {
-  union {
-    double xl[4][2][DR_CH];  // [wave]: activations of a chunk
-    double chain[4][512];    // a redone token: operands of the chains
-  };
-  float lg[512];
-  int list[512], cid[4][RC_SLOTS], sid[4][RC_SLOTS];
+  double xl[4][2][DR_CH];  // [wave]: activations of a chunk
+  __attribute__((aligned(16))) float lg[512];
+  int cid[4][RC_SLOTS], sid[4][RC_SLOTS];
   double part[4][16];
   float sval[4][RC_SLOTS], sel_ws[64];
-  int sel_ids[64], redo[4], nlist, nredo;
+  int sel_ids[64], zero[4], nzero;
 };
 
 // WPT: waves per token (1, 4).  With four, each wave takes a quarter of the columns of the exact dot products; all else runs
@@ -332,7 +336,9 @@ __device__ __forceinline__ bool pick_token(PickLds& S, const float* __restrict__
   for (int j = 0; j < 8; j++) {
     const int e = 8 * lane + j;
     a[j] = U[j] = L[j] = -INFINITY;
-    if (e < E) {
+    // (an expert whose bias is minus infinity is switched off: its logit is the same minus infinity whatever the sum, its
+    //  softmax term zero, and it is no candidate)
+    if (e < E && !(bi8[j] == -INFINITY && isfinite(v8[j]))) {
       const float av = v8[j] + bi8[j];
       const float B = eps * xn * wn8[j] + dterm * (xn + wn8[j]) + 1e-6f * (1.f + fabsf(av));
       fin = fin && isfinite(av) && isfinite(B);
@@ -474,56 +480,178 @@ __device__ __forceinline__ bool pick_token(PickLds& S, const float* __restrict__
 // 695.
 constexpr int PICK_SPLIT_MAX = 1024;
 
+// The list of tokens for k_router_listed, ints: [0] their number, [1 + g] the tickets of group g, then the tokens.
+__host__ __device__ constexpr int hard_first(int P) { return 1 + (P + RL_T - 1) / RL_T; }
+
 template <bool BF16, int WPT>
 __global__ void __launch_bounds__(256, 3) k_router_pick(const float* __restrict__ alog, int KS, const float* __restrict__ wnorm,
                                                         const float* __restrict__ xms, int P, int E, int d, int k, float eps, float dterm,
                                                         float bias_max, int* __restrict__ ids, float* __restrict__ ws, int id_stride,
-                                                        moe_rfix RF) {
+                                                        int* __restrict__ hard, moe_rfix RF) {
   __shared__ __attribute__((aligned(16))) PickLds S;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int t = WPT == 1 ? blockIdx.x * 4 + wv : blockIdx.x;
-  if (tid == 0) S.nredo = 0;
+  if (tid == 0) S.nzero = 0;
   __syncthreads();
   if (t < P) {
     const bool ok = pick_token<BF16, WPT>(S, alog, KS, wnorm, P, E, d, k, eps, dterm, bias_max, xms[t], t, lane, wv,
                                      ids + (size_t)t * id_stride, ws + (size_t)t * id_stride, RF);
-    if (!ok && lane == 0 && (WPT == 1 || wv == 0)) S.redo[atomicAdd(&S.nredo, 1)] = t;
+    if (!ok && lane == 0 && (WPT == 1 || wv == 0)) {
+      // an all-zero row (padding): every dot product is zero.  (A mean square that underflows: |dot| < 1e-17, no softmax term
+      // moves.)
+      if (xms[t] == 0.f) S.zero[atomicAdd(&S.nzero, 1)] = t;
+      else hard[hard_first(P) + atomicAdd(hard, 1)] = t;
+    }
   }
   __syncthreads();
-  const int nredo = S.nredo;
-  for (int i = 0; i < nredo; i++) {
-    const int tr = S.redo[i];
-    if (tid == 0) S.nlist = 0;
-    __syncthreads();
-    const float tol = RF.tol[tr];
-    // an all-zero row (padding): every dot product is zero.  (A mean square that underflows: |dot| < 1e-17, no softmax term
-    // moves.)
-    const bool zero = xms[tr] == 0.f;
-    if (zero)
-      for (int e = tid; e < E; e += 256) S.lg[e] = RF.bias ? RF.bias[e] : 0.f;
-    for (int e0 = zero ? E : 16 * wv; e0 < E; e0 += 64) {
-      const int ea = e0 + (lane >> 3), eb = ea + 8;
-      double va, vb;
-      dot_rows<BF16, true>(RF.W, RF.x + (size_t)tr * d, d, 0, d, ea < E ? ea : E - 1, eb < E ? eb : E - 1, lane, S.xl[wv], va, vb);
-      if ((lane & 7) == 0) {
-        if (ea < E) {
-          if (logit_doubtful(va, tol)) S.list[atomicAdd(&S.nlist, 1)] = ea;
-          S.lg[ea] = (float)va + (RF.bias ? RF.bias[ea] : 0.f);
+  const int nzero = S.nzero;
+  if (nzero == 0) return;
+  // (one selection for all of them: their logits are the biases)
+  for (int e = tid; e < E; e += 256) S.lg[e] = RF.bias ? RF.bias[e] : 0.f;
+  __syncthreads();
+  (void)topk_block<8, false, 256>(S.lg, S.sel_ids, S.sel_ws, E, k);
+  __syncthreads();
+  for (int i = 0; i < nzero; i++)
+    if (tid < k) {
+      ids[(size_t)S.zero[i] * id_stride + tid] = S.sel_ids[tid];
+      ws[(size_t)S.zero[i] * id_stride + tid] = S.sel_ws[tid];
+    }
+}
+
+// ---- 4. listed tokens: all E logits as the reference's chains, in groups of sixteen tokens x 64 experts to a block ----
+// v_mfma_f64_16x16x4_f64 adds its four k slices one after the other (router.hip), so MFMAs over ascending columns are the
+// reference's sums bit for bit and nothing is left in doubt.  A lane's 16-byte load holds four neighbouring columns of a row; the
+// 4 x 4 exchange between lane groups and words turns them into the order of the slices: word q of lane group g = column
+// 4 q + g of sixteen.  The block that draws a group's last ticket runs its softmax and top-k, a wave per token (hand-over of the
+// logits as in k_router_mfma).
+// A few tokens wait for one wave's chain of d / 4 dependent MFMAs, so a wave takes one tile (all 512 experts in one block: 280 us
+// for one group).  Long lists are bound by the f64 pipe, where an operand's conversion from f32 counts for half an MFMA:
+// there a wave takes 2 x 4 tiles, 6 conversions to 8 MFMAs for 2 to 1 (from RL_LONG tokens; all of 8192 tokens: 1050 -> 540 us).
+// The router's launches, us (512 experts, d = 3072, f32; in brackets redone by the tokens' own blocks, and by the dense launch that
+// was here before): one token of 300 130 (330, 224) where none takes 46 (43, 239); one of 2048 160 (364, 250); 40 of 2048 190
+// (358, 264); all of 1024 190 (645, 442), of 2048 345 (1285, 470), of 8192 810 (3830, 1000), of 16384 1580 (-, 1560).  Nothing
+// listed: 2.4 us.
+constexpr int RL_E = 64, RL_GRID = 512, RL_LONG = 2560;
+__device__ __forceinline__ void group_transpose(const float4& f, float (&o)[4]) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(f.x), __float_as_uint(f.z), false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(f.y), __float_as_uint(f.w), false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const auto e = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  o[0] = __uint_as_float(c[0]); o[1] = __uint_as_float(c[1]); o[2] = __uint_as_float(e[0]); o[3] = __uint_as_float(e[1]);
+}
+// NT x NE: a wave's tiles of sixteen tokens and sixteen experts; RD: 16-column steps in flight.
+template <bool BF16, int NT, int NE, int RD>
+__device__ __forceinline__ void listed_groups(float (*lg)[512], float (*pbuf)[512], int* s_last, int* __restrict__ hard, int P, int E, int d,
+                                              int k, float* logits, int* __restrict__ ids, float* __restrict__ ws, int id_stride,
+                                              const moe_rfix& RF) {
+  typedef double double4v __attribute__((ext_vector_type(4)));
+  constexpr int T = RL_T * NT, EB = 64 * NE;  // tokens and experts of a block
+  const int n = hard[0];
+  const int* const list = hard + hard_first(P);
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15, g = lane >> 4, nst = d / 16;
+  const int nrb = (E + EB - 1) / EB, nitem = (n + T - 1) / T * nrb;
+  for (int item = blockIdx.x; item < nitem; item += gridDim.x) {
+    const int grp = item / nrb, i0 = grp * T, e0 = (item % nrb) * EB + 16 * NE * wv + li;
+    // rows past the end: the group's first token, the matrix's last row; not stored
+    const float* xp[NT];
+#pragma unroll
+    for (int m = 0; m < NT; m++) xp[m] = RF.x + (size_t)list[i0 + 16 * m + li < n ? i0 + 16 * m + li : i0] * d + 4 * g;
+    const uint8_t* wp[NE];
+#pragma unroll
+    for (int q = 0; q < NE; q++) wp[q] = (const uint8_t*)RF.W + ((size_t)(e0 + 16 * q < E ? e0 + 16 * q : E - 1) * d + 4 * g) * (BF16 ? 2 : 4);
+    float4 xr[RD][NT], wr[RD][NE];
+    auto fetch = [&](int j, int s) {
+      s = s < nst ? s : nst - 1;  // (past the end: a repeat that is never used)
+#pragma unroll
+      for (int m = 0; m < NT; m++) xr[j][m] = *(const float4*)(xp[m] + (size_t)s * 16);
+#pragma unroll
+      for (int q = 0; q < NE; q++) {
+        if (BF16) {
+          const uint2 u = *(const uint2*)(wp[q] + (size_t)s * 32);
+          wr[j][q].x = __uint_as_float(u.x); wr[j][q].y = __uint_as_float(u.y);
+        } else {
+          wr[j][q] = *(const float4*)(wp[q] + (size_t)s * 64);
         }
-        if (eb < E) {
-          if (logit_doubtful(vb, tol)) S.list[atomicAdd(&S.nlist, 1)] = eb;
-          S.lg[eb] = (float)vb + (RF.bias ? RF.bias[eb] : 0.f);
+      }
+    };
+    double4v acc[NT][NE];
+#pragma unroll
+    for (int m = 0; m < NT; m++)
+#pragma unroll
+      for (int q = 0; q < NE; q++) acc[m][q] = double4v{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int j = 0; j < RD; j++) fetch(j, j);
+    for (int sb = 0; sb < nst; sb += RD) {
+#pragma unroll
+      for (int j = 0; j < RD; j++) {
+        if (sb + j < nst) {
+          float xt[NT][4], wt[NE][4];
+#pragma unroll
+          for (int m = 0; m < NT; m++) group_transpose(xr[j][m], xt[m]);
+#pragma unroll
+          for (int q = 0; q < NE; q++) {
+            float4 f = wr[j][q];
+            if (BF16) {
+              const uint32_t u = __float_as_uint(f.x), v = __float_as_uint(f.y);
+              f = float4{__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u), __uint_as_float(v << 16), __uint_as_float(v & 0xffff0000u)};
+            }
+            group_transpose(f, wt[q]);
+          }
+          fetch(j, sb + j + RD);
+#pragma unroll
+          for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int m = 0; m < NT; m++)
+#pragma unroll
+              for (int q = 0; q < NE; q++)
+                acc[m][q] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xt[m][c], (double)wt[q][c], acc[m][q], 0, 0, 0);
         }
       }
     }
+    // D value r of lane l = [token 4r + l/16][expert l%16]
+#pragma unroll
+    for (int m = 0; m < NT; m++)
+#pragma unroll
+      for (int q = 0; q < NE; q++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int i = i0 + 16 * m + 4 * r + g, e = e0 + 16 * q;
+          if (i < n && e < E)
+            __hip_atomic_store(&logits[(size_t)i * E + e], (float)acc[m][q][r] + (RF.bias ? RF.bias[e] : 0.f), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __syncthreads();
-    select_listed<8>(S.lg, S.list, S.nlist, tol, RF, tr, E, k, S.sel_ids, S.sel_ws, S.chain);
-    if (tid < k) {
-      ids[(size_t)tr * id_stride + tid] = S.sel_ids[tid];
-      ws[(size_t)tr * id_stride + tid] = S.sel_ws[tid];
+    if (tid == 0) *s_last = __hip_atomic_fetch_add(&hard[1 + grp], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nrb - 1;
+    __syncthreads();
+    if (!*s_last) continue;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    for (int h = 0; h < NT; h++) {
+      const int ih = i0 + 16 * h, nt = n - ih < RL_T ? n - ih : RL_T;
+      for (int j = tid; j < nt * 512; j += 256)
+        if ((j & 511) < E)
+          lg[j >> 9][j & 511] = __hip_atomic_load(&logits[(size_t)(ih + (j >> 9)) * E + (j & 511)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+#pragma unroll 1
+      for (int i = wv; i < nt; i += 4) {
+        const size_t row = (size_t)list[ih + i] * id_stride;
+        topk_wave<8>(lg[i], ids + row, ws + row, E, k, pbuf[wv]);
+      }
+      __syncthreads();  // (before the next logits)
     }
-    __syncthreads();
   }
+}
+template <bool BF16>
+__global__ void __launch_bounds__(256, 2) k_router_listed(int* __restrict__ hard, int P, int E, int d, int k, float* logits,
+                                                       int* __restrict__ ids, float* __restrict__ ws, int id_stride, moe_rfix RF) {
+  __shared__ __attribute__((aligned(16))) float lg[RL_T][512];
+  __shared__ __attribute__((aligned(16))) float pbuf[4][512];
+  __shared__ int s_last;
+  const int n = hard[0];
+  if (n == 0) return;
+  if (n < RL_LONG) listed_groups<BF16, 1, 1, 6>(lg, pbuf, &s_last, hard, P, E, d, k, logits, ids, ws, id_stride, RF);
+  else listed_groups<BF16, 2, 4, 3>(lg, pbuf, &s_last, hard, P, E, d, k, logits, ids, ws, id_stride, RF);
 }
 
 // Tiles of the f16 launch, and column shares as far as two blocks per CU.  Either tile moves 10.5 TB/s out of the L2s, so the
@@ -551,11 +679,13 @@ bool moe_router_cand_supported(const moe_wview* W, int P, int k) {
   return moe_aligned(W->data, 16);
 }
 
+static size_t rc_hard_bytes(int tokens) { return ((size_t)(hard_first(tokens) + tokens) * 4 + 255) / 256 * 256; }
 static size_t rc_wnorm_bytes(int experts) { return ((size_t)experts * 4 + 255) / 256 * 256; }
 size_t moe_router_cand_scratch_bytes(int max_tokens, int experts, int d) {
   // wnorm [E], the router matrix as f16, the column shares' partial logits (as long as there are shares: at most RA_SLOTS tiles)
   const size_t tiles = (size_t)RA_SLOTS * 128 * 128 * 4, all = (size_t)RA_KS * max_tokens * experts * 4;
-  return rc_wnorm_bytes(experts) + (size_t)experts * d * 2 + 256 + (all < tiles ? all : tiles);
+  // and the list of hard tokens in front of all
+  return rc_hard_bytes(max_tokens) + rc_wnorm_bytes(experts) + (size_t)experts * d * 2 + 256 + (all < tiles ? all : tiles);
 }
 
 // Internal: ids / ws of a batch; `logits` [P][E] is scratch.
@@ -564,8 +694,9 @@ int moe_router_batch_cand(const moe_wview* W, const float* x, int P, float* logi
                           hipEvent_t after_rows) {
   const int E = (int)W->rows, d = (int)W->cols;
   if (!moe_router_cand_supported(W, P, k) || !moe_aligned(x, 16) || !R.x16 || !R.xms || !R.tol) return MOE_E_UNSUPPORTED;
-  float* wnorm = (float*)scratch;
-  __half* W16 = (__half*)((uint8_t*)scratch + rc_wnorm_bytes(E));
+  int* const hard = (int*)scratch;
+  float* wnorm = (float*)((uint8_t*)scratch + rc_hard_bytes(P));
+  __half* W16 = (__half*)((uint8_t*)wnorm + rc_wnorm_bytes(E));
   const F16Shape s = f16_shape(P, E, d);
   float* alog = s.ks == 1 ? logits : (float*)((uint8_t*)W16 + ((size_t)E * d * 2 + 255) / 256 * 256);
   // 1.002: second-order terms; 1.01: the f32 norms' own rounding
@@ -574,14 +705,14 @@ int moe_router_batch_cand(const moe_wview* W, const float* x, int P, float* logi
   const bool bf = W->dtype == MOE_DT_BF16;
   const unsigned g1 = (unsigned)((E + 3) / 4 + (P + 3) / 4), g3 = (unsigned)((P + 3) / 4);
   const unsigned g2 = (unsigned)((s.ntt + 7) / 8 * 8 * s.ncol * s.ks);
-  if (bf) k_router_prep<true><<<g1, 256, 0, st>>>(W->data, E, d, W16, wnorm, x, P, R);
-  else k_router_prep<false><<<g1, 256, 0, st>>>(W->data, E, d, W16, wnorm, x, P, R);
+  if (bf) k_router_prep<true><<<g1, 256, 0, st>>>(W->data, E, d, W16, wnorm, hard, x, P, R);
+  else k_router_prep<false><<<g1, 256, 0, st>>>(W->data, E, d, W16, wnorm, hard, x, P, R);
   MOE_LAUNCH_CHECK();
   if (after_rows) MOE_HIP(hipEventRecord(after_rows, st));
   if (s.mt == 2) k_router_f16<2><<<g2, 256, 0, st>>>(W16, (const __half*)R.x16, P, E, d, alog, s.ncol, s.ntt, s.ks);
   else k_router_f16<1><<<g2, 256, 0, st>>>(W16, (const __half*)R.x16, P, E, d, alog, s.ncol, s.ntt, s.ks);
   MOE_LAUNCH_CHECK();
-#define PICK_GO(BF, WPT) k_router_pick<BF, WPT><<<WPT == 1 ? g3 : (unsigned)P, 256, 0, st>>>(alog, s.ks, wnorm, R.xms, P, E, d, k, eps, dterm, bias_max, ids, ws, id_stride, RF)
+#define PICK_GO(BF, WPT) k_router_pick<BF, WPT><<<WPT == 1 ? g3 : (unsigned)P, 256, 0, st>>>(alog, s.ks, wnorm, R.xms, P, E, d, k, eps, dterm, bias_max, ids, ws, id_stride, hard, RF)
   if (P <= PICK_SPLIT_MAX) {
     if (bf) PICK_GO(true, 4);
     else PICK_GO(false, 4);
@@ -590,6 +721,11 @@ int moe_router_batch_cand(const moe_wview* W, const float* x, int P, float* logi
     else PICK_GO(false, 1);
   }
 #undef PICK_GO
+  MOE_LAUNCH_CHECK();
+  const int items = (P + RL_T - 1) / RL_T * ((E + RL_E - 1) / RL_E);
+  const unsigned g4 = (unsigned)(items < RL_GRID ? items : RL_GRID);
+  if (bf) k_router_listed<true><<<g4, 256, 0, st>>>(hard, P, E, d, k, logits, ids, ws, id_stride, RF);
+  else k_router_listed<false><<<g4, 256, 0, st>>>(hard, P, E, d, k, logits, ids, ws, id_stride, RF);
   MOE_LAUNCH_CHECK();
   return MOE_OK;
 }

@@ -220,7 +220,7 @@ __device__ __forceinline__ bool topk_fast_handled(const float* lg, int E, int k)
 
 // The softmax / top-k of one token by one wave (E <= 64 * NPL): lane l holds experts NPL*l .. NPL*l + NPL - 1
 // (lane-major), so that among equal keys the lowest expert sits in the lowest lane and register, and the
-// selection can pre-sort each lane's keys.  pbuf: 64 * NPL floats of LDS owned by this wave.
+// selection can pre-sort each lane's keys.  pbuf: 64 * NPL floats of LDS owned by this wave, 16-byte aligned.
 template <int NPL>
 __device__ __forceinline__ void topk_wave(const float* __restrict__ lg, int* __restrict__ ids_row,
                                           float* __restrict__ ws_row, int E, int k, float* pbuf) {
@@ -256,8 +256,16 @@ __device__ __forceinline__ void topk_wave(const float* __restrict__ lg, int* __r
     __builtin_amdgcn_s_waitcnt(0);
     __builtin_amdgcn_wave_barrier();
     double s = 0.0;
-    if (lane == 0)
-      for (int e = 0; e < E; e++) s += (double)pbuf[e];
+    if (lane == 0) {  // (16-byte reads, eight in flight: one by one each addition waited for its own; zeros past E)
+#pragma unroll 8
+      for (int e = 0; e < 64 * NPL; e += 4) {
+        const float4 q = *(const float4*)(pbuf + e);
+        s += (double)q.x;
+        s += (double)q.y;
+        s += (double)q.z;
+        s += (double)q.w;
+      }
+    }
     se = __shfl(s, 0, 64);
   }
   // probabilities are >= 0, so their bit patterns order like unsigned integers; key = bits + 1

@@ -118,13 +118,13 @@ def test_router_tiles(capi, oracle, T, E, k, d, dt):
 
 
 def test_router_ties_above_the_middle(capi, oracle):
-    """The candidate selection's redo of listed tokens, at a size only it takes: tied and nearly tied rows, a zero token."""
+    """Tokens that the candidate selection lists, at a size only it takes: tied and nearly tied rows, a zero token."""
     rng = np.random.default_rng(11)
     E, k, d, T = 128, 10, 512, 1200
     hl = HostLayer(rng, d, 256, E, k, shared=False)
     hl.router[7] = hl.router[3]
     hl.router[16] = hl.router[5] * np.float32(1 + 2 ** -22)
-    for zeros in (2, T - 30):  # few listed tokens; most of them (the dense launch takes over)
+    for zeros in (2, T - 30):  # few tokens to redo; most of them (padding: their sums are known)
         x = rng.standard_normal((T, d), dtype=np.float32)
         x[:zeros] = 0.0
         lo, io, wo = oracle.router(hl.oracle_layer().router, x, k)
@@ -186,6 +186,77 @@ def test_router_candidates_of_small_batches(capi, oracle, T, E, k, d, dt, fmt, s
     m.close()
     assert (ids == io[:, :k]).all()
     assert np.abs(ws - wo[:, :k]).max() <= 2.5e-7
+
+
+# ---------- routers of 33 tokens and more: tokens that the fast selection cannot settle, few and many of them ----------
+def route_and_compare(capi, oracle, hl, x, k):
+    T = len(x)
+    _, io, wo = oracle.router(hl.oracle_layer().router, x, k, bias=hl.bias)
+    m, dev = hl.to_gpu(max_tokens=T)
+    m.profile(True)
+    xg = gpu(x)
+    ms = []
+    for _ in range(4):
+        m.forward(0, xg)
+        ms.append(m.profile_read()["router"])
+    assert m.last_path() == capi.PATH_BATCH
+    ids, ws = (a.cpu().numpy()[:, :k] for a in m.last_routing(T))
+    m.close()
+    assert (ids == io[:, :k]).all(), np.where((ids != io[:, :k]).any(1))
+    wo = wo[:, :k]
+    ok = np.isfinite(wo)
+    assert (np.isfinite(ws) == ok).all()
+    assert np.abs(ws[ok] - wo[ok]).max(initial=0.0) <= 2.5e-7
+    return min(ms)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("T,E,d", [(130, 512, 512), (300, 512, 512), (1200, 500, 384), (2600, 128, 256), (2700, 500, 256)])
+@pytest.mark.parametrize("kind", ["one off", "most off", "all but k off", "too many off", "wide", "some wide", "a nan", "infinities"])
+def test_tokens_the_selection_cannot_settle(capi, oracle, kind, T, E, d, dt):
+    rng = np.random.default_rng(T)
+    k = 10
+    bias = None
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    if "off" in kind:  # experts switched off by a bias of minus infinity (too many: k reaches into them)
+        n = {"one off": 1, "most off": E - 40, "all but k off": E - k, "too many off": E - k + 3}[kind]
+        bias = rng.standard_normal(E).astype(np.float32) * 0.1
+        bias[rng.permutation(E)[:n]] = -np.inf
+    elif kind == "wide":        # probabilities underflow: every token has to be redone
+        x *= 400.0
+    elif kind == "some wide":   # a part of the batch, a ragged last group, padding between them
+        x[::4] *= 400.0
+        x[1::8] = 0.0
+    elif kind == "a nan":
+        x[T // 2, 3] = np.nan
+    else:
+        x[5, 7] = np.inf
+        x[::9, 1] = -np.inf
+        x[9, 2] = np.inf
+    hl = HostLayer(rng, d, 256, E, k, router_dtype=dt, shared=False, bias=bias)
+    route_and_compare(capi, oracle, hl, x, k)
+
+
+# ... and what they cost: a batch of ordinary tokens and the same with an expert off, with one NaN, with nothing but tokens to
+# redo.  Measured at 2048 tokens of 3072 columns: 0.08 ms ordinary and with an expert off, 0.16 with one NaN, 0.35 with all
+# tokens to redo; with each of them redone by its own block 0.8, 9.7 and 1.3 .. 41 ms.
+@pytest.mark.parametrize("T", [130, 2048])
+def test_cost_of_tokens_the_selection_cannot_settle(capi, oracle, T):
+    rng = np.random.default_rng(5)
+    E, d, k = 512, 1024, 10
+    hl = HostLayer(rng, d, 256, E, k, shared=False)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    plain = route_and_compare(capi, oracle, hl, x, k)
+    hl.bias = np.zeros(E, np.float32)
+    hl.bias[17] = -np.inf
+    assert route_and_compare(capi, oracle, hl, x, k) <= 1.5 * plain + 0.02
+    hl.bias = None
+    nan = x.copy()
+    nan[T // 2, 3] = np.nan
+    assert route_and_compare(capi, oracle, hl, nan, k) <= 1.5 * plain + 0.2
+    nan[:, 3] = np.nan
+    assert route_and_compare(capi, oracle, hl, nan, k) <= 1.5 * plain + 0.4
+    assert route_and_compare(capi, oracle, hl, x * np.float32(300.0), k) <= 1.5 * plain + 0.4
 
 
 # ---------- grouped GEMM over tiles of few pairs: every format, tile size and side of a line between them ----------
