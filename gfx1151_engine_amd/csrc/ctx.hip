@@ -114,6 +114,7 @@ struct moe_ctx {
   const __half* x16_ext = nullptr;  // set for the duration of moe_forward_x16: the caller's f16 copy of x
   bool shared_aside = true;
   bool v2_fused_mid = true;   // hgn v2 batches: the slot-wise middle in the gate/up launch's epilogue
+  bool stream_gemm = true;    // batches of few pairs per expert: the streaming GEMMs
   bool pair_tables = true;    // table codebooks, 6..32 tokens: look-ups through pair tables
   int last_path = MOE_PATH_NONE;  // which path the last successful moe_forward* call took (moe_last_path)
   // batch router through candidate selection (exact ids at a fraction of the fp64 work); its scratch
@@ -613,6 +614,7 @@ MOE_API int moe_set_option(moe_ctx* c, int option, int value) {
     case MOE_OPT_ROUTER_CANDIDATES: c->router_cand = value != 0; return MOE_OK;
     case MOE_OPT_UNIQUE_GGUF: c->uq_gguf = value != 0; return MOE_OK;
     case MOE_OPT_V2_FUSED_MIDDLE: c->v2_fused_mid = value != 0; return MOE_OK;
+    case MOE_OPT_STREAM_GEMM: c->stream_gemm = value != 0; return MOE_OK;
     case MOE_OPT_PAIR_TABLES: c->pair_tables = value != 0; return MOE_OK;
     case MOE_OPT_F32_DECODE_MAX_TOKENS:
       if (value < 0 || value > c->small_max) return MOE_E_INVALID;
@@ -1030,7 +1032,10 @@ static StreamKinds stream_kinds(const MoeLayer& L, const moe_config& g) {
     k.dn = !L.experts_affine ? MOE_STREAM_TABLE : L.scaled_dn && (!q4sh || L.scaled_sdn) ? MOE_STREAM_SCALED : MOE_STREAM_AFFINE;
     k.with_sh = q4sh;
   } else if (L.has_gguf) {
-    const int up = L.gg.tgu == MOE_GGML_Q4_K ? MOE_STREAM_Q4K : L.gg.tgu == MOE_GGML_Q5_K ? MOE_STREAM_Q5K : -1;
+    // (layers whose gate/up rows the general kernel takes otherwise, which rounds a weight once: no less here)
+    const bool once = !gg_kinds(L, g).r_gu;
+    const int up = L.gg.tgu == MOE_GGML_Q4_K ? (once ? MOE_STREAM_Q4K_ONCE : MOE_STREAM_Q4K)
+                   : L.gg.tgu == MOE_GGML_Q5_K ? (once ? MOE_STREAM_Q5K_ONCE : MOE_STREAM_Q5K) : -1;
     const int dn = L.gg.tdn == MOE_GGML_Q4_K ? MOE_STREAM_Q4K : L.gg.tdn == MOE_GGML_Q8_0 ? MOE_STREAM_Q8_0 : -1;
     if (up < 0 || dn < 0) return k;
     k.up = up;
@@ -1065,7 +1070,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   const bool fused = c->fused_combine && !c->hc && !(q4k && !kd.r_dn) && !shd && !(q4k && !kd.uniform(L)) && !v2;  // the HC write-back belongs to the ordered combine
   // middle sizes: tiles of few pairs, the weights streamed into registers
   const StreamKinds sk = stream_kinds(L, g);
-  int cap = fused || sk.up < 0 ? 0 : moe_stream_tile_cap(P, g.topk, g.experts, moe_stream_wide(sk.up, sk.dn));
+  int cap = fused || sk.up < 0 || !c->stream_gemm ? 0 : moe_stream_tile_cap(P, g.topk, g.experts, moe_stream_wide(sk.up, sk.dn));
   const int sxl = sk.up >= MOE_STREAM_Q4K ? 2 : sk.up == MOE_STREAM_TABLE ? 0 : 1;  // the order of activations it reads
   if (c->x16_ext && sxl != batch_x16_layout(L, g)) cap = 0;
   // routed and shared experts in launches of their own

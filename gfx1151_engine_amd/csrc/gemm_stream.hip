@@ -20,7 +20,13 @@
 //     LDS-only barrier per line; down, where they are short, once per block, which then runs without barriers.
 //   - no branch stands around a load of the loops: the compiler counts outstanding loads exactly only along straight code
 //     (with branches every wait drained the pipeline: 332 against 270 us).
-// The weights' f16 values are those of gemm_q4cp.hip bit for bit; the sums run over the same columns in f32.
+// The weights' f16 values are those of gemm_q4cp.hip's form of the same name (scaled, plain, table, K-quant) bit for bit; the sums
+// run over the same columns in f32.  Q4_K and Q5_K layers that gemm_q4cp.hip does not take (widths that are no multiples of
+// 256) go to the general kernel of gguf_types.hip otherwise, which rounds a weight once, from its exact value; so does
+// their form here (F_Q4E, F_Q5E: three instructions for two weights where the packed f16 arithmetic of F_Q4K and F_Q5K, which
+// rounds d * sc and dmin * m as well, takes two.  Error of a 2560 x 640 layer's output against fp64 4.9e-4, with the packed
+// arithmetic 5.5e-4; 130 / 515 / 1500 tokens 544 / 612 / 796 us, with it 522 / 581 / 760, on the general kernel 1855 / 1968 /
+// 2060).
 // Pairs per tile: 16, 32 or 64 by the batch's average (moe_stream_tile_cap): a block's work is the weights whatever the
 // tile holds, so tiles should hold an expert's pairs as a rule, and larger ones cost LDS and registers.
 // Measured (512 experts, top-10, 3072 x 768, gate/up + down, us; in brackets the 128-pair kernels):
@@ -39,7 +45,11 @@ typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // F_DN: affine q4cp codebooks whose experts all have a power of two for the scaled dequantisation (gemm_q4cp.hip, DN)
-enum { F_DN, F_AFF, F_TAB, F_I4R, F_Q4K, F_Q5K, F_Q80 };
+// F_Q4E, F_Q5E: Q4_K and Q5_K weights rounded to f16 once, from their exact values
+enum { F_DN, F_AFF, F_TAB, F_I4R, F_Q4K, F_Q5K, F_Q80, F_Q4E, F_Q5E };
+constexpr bool q4(int FMT) { return FMT == F_Q4K || FMT == F_Q4E; }
+constexpr bool q5(int FMT) { return FMT == F_Q5K || FMT == F_Q5E; }
+constexpr bool once_rounded(int FMT) { return FMT == F_Q4E || FMT == F_Q5E; }
 constexpr bool scale_plane(int FMT) { return FMT <= F_I4R; }
 // order of activations and hid (moe_f32_to_f16's layouts)
 constexpr int x_layout(int FMT) { return FMT == F_TAB ? 0 : FMT <= F_I4R ? 1 : 2; }
@@ -74,9 +84,9 @@ __device__ __forceinline__ half2v both(float f) { return half2v{(_Float16)f, (_F
 
 template <int FMT>
 __device__ __forceinline__ uint32_t row_bytes(int K) {
-  return FMT == F_Q4K ? K / 256 * 144 : FMT == F_Q5K ? K / 256 * 176 : FMT == F_Q80 ? K / 32 * 34 : K / 2;
+  return q4(FMT) ? K / 256 * 144 : q5(FMT) ? K / 256 * 176 : FMT == F_Q80 ? K / 32 * 34 : K / 2;
 }
-constexpr int line_bytes(int FMT) { return FMT == F_Q4K ? 144 : FMT == F_Q5K ? 176 : FMT == F_Q80 ? 272 : 128; }
+constexpr int line_bytes(int FMT) { return q4(FMT) ? 144 : q5(FMT) ? 176 : FMT == F_Q80 ? 272 : 128; }
 
 // element of a group of 16 NW rows that output position 16 wv + i holds: the order the down launch reads hid in (layout 2
 // runs over 64-element blocks, four waves' groups)
@@ -110,9 +120,9 @@ __device__ __forceinline__ void load_line(Line<FMT>& q, const uint8_t* b, uint32
     }
     q.last = *(const uint32_t*)(s + 64);
   } else {
-    constexpr uint32_t C0 = FMT == F_Q4K ? 16 : FMT == F_Q5K ? 48 : 0;
-    if (FMT == F_Q4K || FMT == F_Q5K) q.hd[0] = *(const uint4*)(b + o);
-    if (FMT == F_Q5K) q.qh[0] = *(const uint4*)(b + (o + 16u + 16u * (uint32_t)(g & 1)));
+    constexpr uint32_t C0 = q4(FMT) ? 16 : q5(FMT) ? 48 : 0;
+    if (q4(FMT) || q5(FMT)) q.hd[0] = *(const uint4*)(b + o);
+    if (q5(FMT)) q.qh[0] = *(const uint4*)(b + (o + 16u + 16u * (uint32_t)(g & 1)));
     q.c[0] = *(const uint4*)(b + (o + C0 + 16u * (uint32_t)g));
     const uint8_t* b1 = b + (half ? 0 : 64);
     q.c[1] = *(const uint4*)(b1 + (o + C0 + 16u * (uint32_t)g));
@@ -182,21 +192,32 @@ __device__ __forceinline__ void line_mma(const Line<FMT> (&q)[F], const uint32_t
     auto part = [&](auto ec) {
       constexpr int E_ = decltype(ec)::value;
       half2v as[F][2], bs[F][2];
+      float ka[F][2], kb[F][2];
+      constexpr bool ONCE = once_rounded(FMT);
 #pragma unroll
       for (int f = 0; f < F; f++) {
-        if (FMT == F_Q4K || FMT == F_Q5K) {
-          // 6-bit (scale, min) fields of sub-blocks 0-3 (E_ = 0) or 4-7 as bytes, gguf scale_min_k4; d * sc and dmin * m as
-          // packed f16 products of exact integers
+        if (q4(FMT) || q5(FMT)) {
+          // 6-bit (scale, min) fields of sub-blocks 0-3 (E_ = 0) or 4-7 as bytes, gguf scale_min_k4
           const uint4 hd = q[f].hd[0];
           const uint32_t sc = E_ ? (hd.w & 0x0f0f0f0fu) | ((hd.y >> 2) & 0x30303030u) : hd.y & 0x3f3f3f3fu;
           const uint32_t mn = E_ ? ((hd.w >> 4) & 0x0f0f0f0fu) | ((hd.z >> 2) & 0x30303030u) : hd.z & 0x3f3f3f3fu;
-          const half2v dd = h2(__builtin_amdgcn_perm(hd.x, hd.x, 0x01000100u));
-          const half2v dm = h2(__builtin_amdgcn_perm(hd.x, hd.x, 0x03020302u) ^ 0x80008000u);
           const half2v k1024 = both(1024.f);
-          const half2v a = (h2(__builtin_amdgcn_perm(0x64646464u, sc, C.selb)) - k1024) * dd;
-          const half2v b = (h2(__builtin_amdgcn_perm(0x64646464u, mn, C.selb)) - k1024) * dm;
-          as[f][0] = half2v{a.x, a.x}; as[f][1] = half2v{a.y, a.y};
-          bs[f][0] = half2v{b.x, b.x}; bs[f][1] = half2v{b.y, b.y};
+          const half2v s2 = h2(__builtin_amdgcn_perm(0x64646464u, sc, C.selb)) - k1024;
+          const half2v m2 = h2(__builtin_amdgcn_perm(0x64646464u, mn, C.selb)) - k1024;
+          if (ONCE) {
+            // d * sc and dmin * m are exact in f32, and so to 2^-14 of a step is what the codes' offsets (below) add
+            const half2v dd = h2(hd.x);
+            ka[f][0] = (float)s2.x * (float)dd.x;
+            ka[f][1] = (float)s2.y * (float)dd.x;
+            kb[f][0] = -fmaf(1024.f, ka[f][0], (float)m2.x * (float)dd.y);
+            kb[f][1] = -fmaf(64.f, ka[f][1], (float)m2.y * (float)dd.y);
+          } else {  // d * sc and dmin * m as packed f16 products of exact integers
+            const half2v dd = h2(__builtin_amdgcn_perm(hd.x, hd.x, 0x01000100u));
+            const half2v dm = h2(__builtin_amdgcn_perm(hd.x, hd.x, 0x03020302u) ^ 0x80008000u);
+            const half2v a = s2 * dd, b = m2 * dm;
+            as[f][0] = half2v{a.x, a.x}; as[f][1] = half2v{a.y, a.y};
+            bs[f][0] = half2v{b.x, b.x}; bs[f][1] = half2v{b.y, b.y};
+          }
         } else {
           const half2v s2 = h2(sw[f]);
           const _Float16 sh = E_ ? s2.y : s2.x;
@@ -233,7 +254,7 @@ __device__ __forceinline__ void line_mma(const Line<FMT> (&q)[F], const uint32_t
           } else {  // 0x6400 | n is the f16 1024 + n, 0x5400 | n << 4 is 64 + n
             uint32_t t0 = (w & 0x000f000fu) | 0x64006400u, t1 = (w & 0x00f000f0u) | 0x54005400u;
             uint32_t t2 = (w8 & 0x000f000fu) | 0x64006400u, t3 = (w8 & 0x00f000f0u) | 0x54005400u;
-            if (FMT == F_Q5K) {
+            if (q5(FMT)) {
               // fifth bits: bit 2 jj (low nibbles) and 2 jj + 1 (high) of the qh byte, jj = g / 2 + 2 E_
               const uint4 qq = q[f].qh[0];
               const uint32_t qw = s == 0 ? qq.x : s == 1 ? qq.y : s == 2 ? qq.z : qq.w;
@@ -242,6 +263,17 @@ __device__ __forceinline__ void line_mma(const Line<FMT> (&q)[F], const uint32_t
               t1 |= (r << 7) & 0x01000100u;
               t2 |= (r >> 4) & 0x00100010u;
               t3 |= (r >> 1) & 0x01000100u;
+            }
+            if (ONCE) {
+              auto once = [&](uint32_t t, int i) {
+                const half2v n = h2(t);
+                return half2v{(_Float16)fmaf((float)n.x, ka[f][i], kb[f][i]), (_Float16)fmaf((float)n.y, ka[f][i], kb[f][i])};
+              };
+              a[f].h[0] = once(t0, 0);
+              a[f].h[1] = once(t1, 1);
+              a[f].h[2] = once(t2, 0);
+              a[f].h[3] = once(t3, 1);
+              continue;
             }
             const half2v k1024 = both(1024.f), k64 = both(64.f);
             a[f].h[0] = (h2(t0) - k1024) * as[f][0] + bs[f][0];
@@ -733,7 +765,7 @@ int moe_stream_tile_cap(int P, int k, int experts, bool wide) {
   if (avg <= 10.f) return 16;
   return wide ? (avg <= 22.f ? 32 : avg <= 44.f ? 64 : 0) : avg <= 38.f ? 32 : 0;
 }
-bool moe_stream_wide(int fmt_up, int fmt_dn) { return fmt_up != F_Q5K && fmt_dn != F_Q80; }
+bool moe_stream_wide(int fmt_up, int fmt_dn) { return !q5(fmt_up) && fmt_dn != F_Q80; }
 
 // fmt: MOE_STREAM_*; the views as for moe_launch_gemm_q4cp.  max_tiles == 0: checks only.
 int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const moe_lutw* sh, int n_experts, const __half* x,
@@ -753,11 +785,11 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
     return true;
   };
   if (!ok(routed) || (sh && !ok(sh))) return MOE_E_UNSUPPORTED;
-  if (k % 128 || ((fmt == F_Q4K || fmt == F_Q5K || fmt == F_I4R) && k % 256)) return MOE_E_UNSUPPORTED;
+  if (k % 128 || ((q4(fmt) || q5(fmt) || fmt == F_I4R) && k % 256)) return MOE_E_UNSUPPORTED;
   // (down: rows of three lines, and whole groups of rows for sixteen waves)
   if (up ? k < 256 : (k + 255) / 256 != DN_LINES || m % 512) return MOE_E_UNSUPPORTED;
   if (up && (m % 16 || (fmt >= F_Q4K && m % 64) || (fmt == F_I4R && m % 128))) return MOE_E_UNSUPPORTED;
-  if ((up && fmt == F_Q80) || (!up && fmt == F_Q5K) || (cap > 32 && (fmt == F_Q5K || fmt == F_Q80))) return MOE_E_UNSUPPORTED;
+  if ((up && fmt == F_Q80) || (!up && (q5(fmt) || once_rounded(fmt))) || (cap > 32 && (q5(fmt) || fmt == F_Q80))) return MOE_E_UNSUPPORTED;
   if (fmt == F_I4R && up != (rot != nullptr)) return MOE_E_INVALID;
   if (rot && (!rot->svh_gu || !rot->suh_dn)) return MOE_E_INVALID;
   if (fmt == F_DN && (!pexp_routed || (sh && !pexp_sh))) return MOE_E_INVALID;
@@ -770,7 +802,7 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
   do {                                              \
     if (cap == 16) return launch<F, U, 1>(ST_ARGS); \
     if (cap == 32) return launch<F, U, 2>(ST_ARGS); \
-    if constexpr (F != F_Q5K && F != F_Q80) return launch<F, U, 4>(ST_ARGS); \
+    if constexpr (!q5(F) && F != F_Q80) return launch<F, U, 4>(ST_ARGS); \
     return MOE_E_UNSUPPORTED;                       \
   } while (0)
 #define ST_DIR(F)            \
@@ -785,6 +817,8 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
     case F_I4R: ST_DIR(F_I4R);
     case F_Q4K: ST_DIR(F_Q4K);
     case F_Q5K: ST_CAP(F_Q5K, true);
+    case F_Q4E: ST_CAP(F_Q4E, true);
+    case F_Q5E: ST_CAP(F_Q5E, true);
     case F_Q80: ST_CAP(F_Q80, false);
     default: return MOE_E_INVALID;
   }

@@ -287,3 +287,36 @@ def test_tiles_of_few_pairs(capi, oracle, kind, kw, d, mid, T):
     sel = np.r_[0, 1, T // 2, T - 2, T - 1]
     yo, _, _ = oracle.moe_layer(hl.oracle_layer(), x[sel])
     assert max_abs_rel(y[sel], yo) <= 2e-3
+
+
+# ---------- ... against the 128-pair kernels ----------
+STREAM_KINDS = [("q4cp", dict(fmt="q4cp"), 512, 640), ("q4cp-affine", dict(fmt="q4cp"), 512, 768),
+                ("q4cp-table", dict(fmt="q4cp", codebook=TABLE), 512, 640), ("q4k", dict(fmt="q4k"), 512, 768),
+                ("q5k-q8_0", dict(fmt="q4k", gg_types=(13, 8, 8)), 512, 768), ("q4k-q8_0", dict(fmt="q4k", gg_types=(12, 8, 8)), 512, 768)]
+
+
+def both_kernels(capi, hl, x):
+    m, dev = hl.to_gpu(max_tokens=len(x))
+    ys = []
+    for on in (1, 0):
+        m.set_option(capi.OPT_STREAM_GEMM, on)
+        ys.append(m.forward(0, gpu(x)).cpu().numpy())
+        assert m.last_path() == capi.PATH_BATCH
+    m.close()
+    return ys
+
+
+@pytest.mark.parametrize("T", [40, 88, 152])
+@pytest.mark.parametrize("kind,kw,d,mid", STREAM_KINDS + [("i4r", dict(fmt="i4r"), 512, 768),
+                                                          ("q5k-q8_0", dict(fmt="q4k", gg_types=(13, 8, 8)), 512, 640),
+                                                          ("q4k-q8_0", dict(fmt="q4k", gg_types=(12, 8, 8)), 512, 640)])
+def test_few_pair_tiles_are_no_less_exact(capi, oracle, kind, kw, d, mid, T):
+    """All rows, dense activations: the 2-norm error against the oracle is that of the 128-pair kernel the layer would take
+    otherwise (roundings of x, hid and pairs to f16 and of the weights, 3 .. 6e-4; another order of the f32 sums moves it
+    by less than a hundredth).  The last two layers take the general kernel there, which rounds a weight once."""
+    rng = np.random.default_rng(T + mid)
+    hl = HostLayer(rng, d, mid, 16, 4, bias=np.linspace(0, 0.5, 16, dtype=np.float32), **kw)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    yo = oracle.moe_layer(hl.oracle_layer(), x)[0].astype(np.float64)
+    e1, e0 = (np.linalg.norm(y - yo) / np.linalg.norm(yo) for y in both_kernels(capi, hl, x))
+    assert e1 <= 1.02 * e0 <= 1e-3, (e1, e0)
