@@ -307,6 +307,34 @@ def both_kernels(capi, hl, x):
 
 
 @pytest.mark.parametrize("T", [40, 88, 152])
+@pytest.mark.parametrize("kind,kw,d,mid", STREAM_KINDS)
+def test_few_pair_tiles_multiply_the_same_weights(capi, kind, kw, d, mid, T):
+    """Tokens with one column, experts with one row of up_proj: every sum has one term, so that both kernels' results are
+    products of the same f16 weights, bit for bit."""
+    rng = np.random.default_rng(T + mid)
+    E, k = 16, 4
+    hl = HostLayer(rng, d, mid, E, k, shared=False, bias=np.linspace(0, 0.5, E, dtype=np.float32), **kw)
+    keep = np.r_[0, 1, 31, 32, 33, 100, 127, 128, 191, 255, 256, 300, 383, 511, mid - 129, mid - 1]  # row of expert 0, 1, ...
+    if hl.fmt == "q4cp":
+        up = hl.gate_up[64:64 + E * 2 * mid * d // 2].reshape(E, 2, mid, d // 2)[:, 1]
+        zero = 0x77 if "table" in kind else 0x88
+        if kind == "q4cp-affine":  # every expert has a row with scales 2^6 below the others: no scaled dequantisation
+            hl.gate_up[64 + E * 2 * mid * d // 2:].view(np.float16).reshape(E, 2 * mid, -1)[:, 3, :] = np.float16(1e-5)
+    else:
+        up = hl.up.reshape(E, mid, -1)
+        zero = 0
+    for e in range(E):
+        row = up[e, keep[e]].copy()
+        up[e] = zero
+        up[e, keep[e]] = row
+    x = np.zeros((T, d), np.float32)
+    x[np.arange(T), rng.integers(0, d, T)] = rng.choice([-2.0, 1.0, 0.5], T) * 16
+    y1, y0 = both_kernels(capi, hl, x)
+    assert np.abs(y0).max() > 0
+    assert (y1 == y0).all()
+
+
+@pytest.mark.parametrize("T", [40, 88, 152])
 @pytest.mark.parametrize("kind,kw,d,mid", STREAM_KINDS + [("i4r", dict(fmt="i4r"), 512, 768),
                                                           ("q5k-q8_0", dict(fmt="q4k", gg_types=(13, 8, 8)), 512, 640),
                                                           ("q4k-q8_0", dict(fmt="q4k", gg_types=(12, 8, 8)), 512, 640)])
