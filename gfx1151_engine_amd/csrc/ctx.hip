@@ -249,8 +249,7 @@ MOE_API int moe_create(const moe_config* cfg, moe_ctx** out) {
     const size_t batch_tiles = (T * cfg->topk + 127) / 128 + E + (T + 127) / 128, uq_tiles = Ts * cfg->topk + (Ts + 3) / 4;
     c->max_tiles = (int)(batch_tiles > uq_tiles ? batch_tiles : uq_tiles);
     for (size_t p = 33; p <= T; p++) {  // middle-sized batches: smaller tiles
-      const int narrow = moe_stream_tile_cap((int)p, cfg->topk, (int)E, false);
-      const int cap = narrow ? narrow : moe_stream_tile_cap((int)p, cfg->topk, (int)E, true);
+      const int cap = moe_stream_tile_cap_least((int)p, cfg->topk, (int)E);
       if (!cap) break;
       const int n = (int)((p * cfg->topk + cap - 1) / cap + E + (p + cap - 1) / cap);
       c->max_tiles = c->max_tiles > n ? c->max_tiles : n;
@@ -1070,7 +1069,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   const bool fused = c->fused_combine && !c->hc && !(q4k && !kd.r_dn) && !shd && !(q4k && !kd.uniform(L)) && !v2;  // the HC write-back belongs to the ordered combine
   // middle sizes: tiles of few pairs, the weights streamed into registers
   const StreamKinds sk = stream_kinds(L, g);
-  int cap = fused || sk.up < 0 || !c->stream_gemm ? 0 : moe_stream_tile_cap(P, g.topk, g.experts, moe_stream_wide(sk.up, sk.dn));
+  int cap = fused || sk.up < 0 || !c->stream_gemm ? 0 : moe_stream_tile_cap(P, g.topk, g.experts, sk.up, sk.dn, g.mid);
   const int sxl = sk.up >= MOE_STREAM_Q4K ? 2 : sk.up == MOE_STREAM_TABLE ? 0 : 1;  // the order of activations it reads
   if (c->x16_ext && sxl != batch_x16_layout(L, g)) cap = 0;
   // routed and shared experts in launches of their own

@@ -6,13 +6,13 @@
 // LDS in 32-byte pieces of 256 rows, two 64-column stages ahead, and reaches 3.5 TB/s of the 6.3 that plain loads reach
 // on this chip (a load of 16 rows x 64 bytes per wave instruction, four or more in flight per wave; 32 rows x 32 bytes:
 // 4.4 .. 5.3).  Here:
-//   - a wave owns 16 weight rows twice (gate/up: 16 gate rows and their 16 up rows; down: 32 rows) and walks K in lines of
-//     256 columns.  v_mfma_f32_16x16x32_f16 takes the weights as A: lane (n, g) = row n, 16-byte chunks g and g + 4 of
+//   - a wave owns 16 weight rows twice (gate/up: 16 gate rows and their 16 up rows; down: 32 rows) and walks K, any multiple of
+//     128 (K-quants and i4r: 256), in lines of 256 columns.  v_mfma_f32_16x16x32_f16 takes the weights as A: lane (n, g) = row n, 16-byte chunks g and g + 4 of
 //     the line's 128 code bytes, so a load instruction covers 64 contiguous bytes of 16 rows and a chunk is one lane's
 //     operand for four MFMAs.  Which columns a lane group multiplies is free as long as the activations agree; a chunk
 //     is one scale group of 32 columns (q4cp), half of a 64-column run (Q4_K, Q5_K), a lane group's run (Q8_0).
-//   - gate/up keeps two lines per wave in flight, line by line; down, whose rows are three lines, requests a fragment's
-//     whole rows at once.  Rows start 64 bytes off the 128-byte cache lines (the codebook heads the tensor), so every line
+//   - gate/up keeps two lines per wave in flight, line by line; down requests a fragment's whole rows at once where they are
+//     three lines, else two lines at a time.  Rows start 64 bytes off the 128-byte cache lines (the codebook heads the tensor), so every line
 //     shares a cache line with the next one, and read a line at a time a third of the traffic is fetched twice (1.66 GB for
 //     1.26, at 6.15 TB/s); whole rows brought down from 6.9 to 5.3 M cache lines (of 5.0).  For gate/up the same, pairs of
 //     lines with four in registers, fetched 1.51 GB and was no faster (270 us either way, three waves per SIMD for four).
@@ -32,6 +32,10 @@
 // Measured (512 experts, top-10, 3072 x 768, gate/up + down, us; in brackets the 128-pair kernels):
 //   130 tokens q4cp 270 + 137 (368 + 185)      48 table 208 + 110 (295 + 177)    515 Q4_K 356 + 176 (413 + 241)
 //   200 Q5_K / Q8_0 407 + 291 (501 + 471)     200 i4r 260 + 143 (338 + 190)      2048 q4cp 392 + 219 (437 + 238)
+// The layer at other widths, us (128-pair kernels in brackets), 48 / 515 / 1200 tokens, d = 3072: mid 256 q4cp 162 / 258 / 331 (207 / 307 /
+// 361), Q5_K / Q8_0 240 / 351 / 450 (353 / 523 / 560); 512 q4cp 245 / 401 / 474 (312 / 491 / 549), table 272 / 434 / 535 (392 / 610 / 639),
+// Q4_K 257 / 428 / 513 (339 / 544 / 602), i4r 245 / 378 / 467 (318 / 478 / 542); 1024 q4cp 429 / 719 / 827 (520 / 851 / 942), table 471 /
+// 781 / 930 (645 / 1074 / 1143); d = 2048: 1536 q4cp 419 / 759 / 891 (518 / 833 / 896), 2048 545 / 969 / 1083 (669 / 1083 / 1148).
 #include <type_traits>
 
 #include "common.h"
@@ -55,6 +59,7 @@ constexpr bool scale_plane(int FMT) { return FMT <= F_I4R; }
 constexpr int x_layout(int FMT) { return FMT == F_TAB ? 0 : FMT <= F_I4R ? 1 : 2; }
 
 constexpr int XROW = 512;  // bytes of a line of one pair row (256 f16)
+constexpr size_t LDS_MOST = 160 * 1024;  // of a CU
 // copies of a pair table: lanes eight apart share one; gate/up with 64 pairs: four, so that two blocks fit a CU's LDS
 constexpr int tab_copies(bool UP, int MFX) { return UP && MFX == 4 ? 4 : 8; }
 
@@ -290,18 +295,18 @@ __device__ __forceinline__ void line_mma(const Line<FMT> (&q)[F], const uint32_t
   }
 }
 
-// Scales of four lines of a row (64 bytes, i4r: 16) from line 4 qd on: lane group i fetches line i's, the exchange below
-// then hands every lane one word per line with its own two scales.  (Past the row's end: one address for all lanes.)
+// Scales of four lines of a row (64 bytes, i4r: 16) from line `first` on: lane group i fetches line first + i's, the exchange
+// below then hands every lane one word per line with its own two scales.  (Past the row's end: one address for all lanes.)
 template <int FMT>
 struct Raw { uint4 v; };
 template <int FMT>
-__device__ __forceinline__ Raw<FMT> load_scales(const uint8_t* b, uint32_t o, int qd, int g, int sstride) {
+__device__ __forceinline__ Raw<FMT> load_scales(const uint8_t* b, uint32_t o, int first, int g, int sstride) {
   Raw<FMT> r;
   if (FMT == F_I4R) {  // one word per line: both scales, the same for all lane groups
-    const uint32_t p = 4u * (uint32_t)(4 * qd + g);
+    const uint32_t p = 4u * (uint32_t)(first + g);
     r.v.x = *(const uint32_t*)(b + (p < (uint32_t)sstride ? o + p : 0u));
   } else {
-    const uint32_t p = 16u * (uint32_t)(4 * qd + g);
+    const uint32_t p = 16u * (uint32_t)(first + g);
     r.v = *(const uint4*)(b + (p < (uint32_t)sstride ? o + p : 0u));
   }
   return r;
@@ -363,8 +368,6 @@ __device__ __forceinline__ void x_addrs(int n, int g, uint32_t (&xa)[8]) {
 }
 
 // ---- gate/up ----
-// (The columns of a down launch that fits are whole pairs of lines here.  Said to the compiler, so that two lines become one
-// straight block without the checks below, it moves loads and operands further, spills and loses 20 us of 390 at 64 pairs.)
 // (Straight code of two lines, where K is known to be whole pairs of lines, gave the compiler room to move loads and operands
 // further and cost 20 us of 390 at 64 pairs (spills: up to 150): the branches around half and last lines stay.)
 template <int FMT, int MFX, int MF, bool ROT, int NW>
@@ -470,7 +473,7 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
 #pragma unroll
       for (int f = 0; f < 2; f++) {
         take_scales<FMT>(raw[f], sq[f]);
-        raw[f] = load_scales<FMT>(sb[f], so, (i >> 2) + 1, g, L.sstride);
+        raw[f] = load_scales<FMT>(sb[f], so, i + 4, g, L.sstride);
       }
     }
     stage(std::integral_constant<int, 0>{}, i);
@@ -554,15 +557,17 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
   }
 }
 
-// ---- down: rows of at most three lines.  The tile's hid rows lie in LDS for the whole block; a wave takes 32 rows at a time,
-// requests a fragment's whole rows at once (neighbouring rows share their boundary cache lines as well) and the next
-// rows' as soon as the fragment's are used up; no barrier after the first.  ----
-constexpr int DN_LINES = 3, DN_XP = DN_LINES * XROW;
-template <int FMT, int MFX, int MF, int NW>
+// ---- down.  The tile's hid rows lie in LDS for the whole block (ONE: row by row, else line by line: strides the compiler knows);
+// a wave takes 32 rows at a time, a piece of LN
+// lines of both fragments in registers, and requests a fragment's next piece as soon as this one is used up; no barrier after
+// the first.  Rows of three lines are one piece (ONE: neighbouring rows then share their boundary cache lines as well); rows of
+// any other length go two lines at a time. ----
+template <int FMT, int MFX, int MF, int NW, int LN, bool ONE>
 __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const moe_tile tile, int nb, int npass,
                                         const __half* __restrict__ x, __half* __restrict__ out, int M, int K, int pexp) {
-  constexpr int LB = line_bytes(FMT), NT = 64 * NW, DNR = 32 * NW;
-  uint8_t* const tabs = smem + MFX * 16 * DN_XP;
+  constexpr int LB = line_bytes(FMT), NT = 64 * NW, DNR = 32 * NW, XP = ONE ? LN * XROW : XROW, XLINE = ONE ? XROW : MFX * 16 * XROW;
+  const int nline = ONE ? LN : (K + 255) >> 8, np = ONE ? 1 : (nline + LN - 1) / LN;
+  uint8_t* const tabs = smem + nline * MFX * 16 * XROW;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, g = lane >> 4;
   const uint32_t RB = row_bytes<FMT>(K);
@@ -570,29 +575,36 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
   const uint8_t* const wb = L.w + (size_t)e * L.e_rows * RB;
   const uint8_t* const sb = scale_plane(FMT) ? L.sc + (size_t)e * L.e_rows * (size_t)L.sstride : nullptr;
   // fragment f, MFMA row i = weight row 8 (i / 4) + 4 f + i % 4 of the wave's 32: a lane's eight results are neighbours
-  Line<FMT> ln[2][DN_LINES];
+  Line<FMT> ln[2][LN];
   Raw<FMT> raw[2];
-  auto load = [&](int f, int p) {
-    p = p < npass ? p : npass - 1;  // (past the end: the last rows again)
-    const int row0 = (nb + p) * DNR + 32 * wv;
-    const int r = 8 * (n >> 2) + 4 * f + (n & 3);
-    if (scale_plane(FMT)) raw[f] = load_scales<FMT>(sb + (size_t)row0 * L.sstride, (uint32_t)r * (uint32_t)L.sstride, 0, g, L.sstride);
-#pragma unroll
-    for (int i = 0; i < DN_LINES; i++)
-      load_line<FMT>(ln[f][i], wb + ((size_t)row0 * RB + i * LB), (uint32_t)r * RB, g, tail && i == DN_LINES - 1);
+  auto first_row = [&](int p) {
+    const int r = (nb + p) * DNR + 32 * wv;
+    return r < M ? r : M - 32;  // (loaded, never stored)
   };
-  load(0, 0);
-  load(1, 0);
-  for (int c = tid; c < 16 * MF * (DN_XP / 16); c += NT) {
-    const int m = c / (DN_XP / 16), k = c % (DN_XP / 16);
-    const int kk = 8 * k < K ? k : 0;  // (a half line's second half: never multiplied)
-    const uint4 v = *(const uint4*)(x + (size_t)(tile.first + (m < tile.count ? m : 0)) * K + 8 * kk);
-    *(uint4*)(smem + m * DN_XP + ((k ^ (m & 15)) << 4)) = v;
-  }
+  // fragment f, pass p, piece q (past the end: the last rows again)
+  auto load = [&](int f, int p, int q) {
+    const int row0 = first_row(p < npass ? p : npass - 1);
+    const int r = 8 * (n >> 2) + 4 * f + (n & 3);
+    if (scale_plane(FMT)) raw[f] = load_scales<FMT>(sb + (size_t)row0 * L.sstride, (uint32_t)r * (uint32_t)L.sstride, q * LN, g, L.sstride);
+#pragma unroll
+    for (int i = 0; i < LN; i++) {
+      const int l = ONE || q * LN + i < nline ? q * LN + i : nline - 1;
+      load_line<FMT>(ln[f][i], wb + ((size_t)row0 * RB + l * LB), (uint32_t)r * RB, g, tail && l == nline - 1);
+    }
+  };
+  load(0, 0, 0);
+  load(1, 0, 0);
+  for (int l = 0; l < nline; l++)
+    for (int c = tid; c < 16 * MF * 32; c += NT) {
+      const int m = c >> 5, k = 32 * l + (c & 31);
+      const int kk = 8 * k < K ? k : 0;  // (a half line's second half: never multiplied)
+      const uint4 v = *(const uint4*)(x + (size_t)(tile.first + (m < tile.count ? m : 0)) * K + 8 * kk);
+      *(uint4*)(smem + l * XLINE + m * XP + (((c & 31) ^ (m & 15)) << 4)) = v;
+    }
   float oscale;
   const Consts C = make_consts<FMT, false, NT, tab_copies(false, MFX)>(L, pexp, tabs, tid, oscale);
   uint32_t xa[8];
-  x_addrs<FMT, DN_XP>(n, g, xa);
+  x_addrs<FMT, XP>(n, g, xa);
   moe_lds_barrier();
   for (int p = 0; p < npass; p++) {
     floatx4 acc[2][MF];
@@ -600,46 +612,53 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
     for (int f = 0; f < 2; f++)
 #pragma unroll
       for (int mf = 0; mf < MF; mf++) acc[f][mf] = floatx4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (MFX < 4) {
+    for (int q = 0; q < np; q++) {
+      const int pn = q + 1 < np ? p : p + 1, qn = q + 1 < np ? q + 1 : 0;  // the piece after this one
+      if constexpr (MFX < 4) {
 #pragma unroll
-      for (int f = 0; f < 2; f++) {
-        asm volatile("" ::: "memory");  // (the activations are the same for all rows: hoisted out of the loop they would fill the registers)
-        uint32_t sq[4] = {0u, 0u, 0u, 0u};
-        if (scale_plane(FMT)) take_scales<FMT>(raw[f], sq);
-        floatx4 a1[1][MF];
+        for (int f = 0; f < 2; f++) {
+          asm volatile("" ::: "memory");  // (the activations are the same for all rows: hoisted out of the loop they would fill the registers)
+          uint32_t sq[4] = {0u, 0u, 0u, 0u};
+          if (scale_plane(FMT)) take_scales<FMT>(raw[f], sq);
+          floatx4 a1[1][MF];
 #pragma unroll
-        for (int mf = 0; mf < MF; mf++) a1[0][mf] = acc[f][mf];
+          for (int mf = 0; mf < MF; mf++) a1[0][mf] = acc[f][mf];
 #pragma unroll
-        for (int i = 0; i < DN_LINES; i++) {
-          const Line<FMT> q1[1] = {ln[f][i]};
-          const uint32_t sw[1] = {sq[i]};
-          line_mma<FMT, 1, MF, DN_XP, tab_copies(false, MFX)>(q1, sw, C, 0, smem + i * XROW, xa, tail && i == DN_LINES - 1, a1);
+          for (int i = 0; i < LN; i++) {
+            const int l = q * LN + i;
+            if (!ONE && l >= nline) break;
+            const Line<FMT> q1[1] = {ln[f][i]};
+            const uint32_t sw[1] = {sq[i]};
+            line_mma<FMT, 1, MF, XP, tab_copies(false, MFX)>(q1, sw, C, 0, smem + l * XLINE, xa, tail && l == nline - 1, a1);
+          }
+#pragma unroll
+          for (int mf = 0; mf < MF; mf++) acc[f][mf] = a1[0][mf];
+          load(f, pn, qn);
+        }
+      } else {  // (64 pairs: both fragments share an activation operand's trip out of LDS)
+        asm volatile("" ::: "memory");
+        uint32_t sq[2][4];
+        if (scale_plane(FMT)) {
+#pragma unroll
+          for (int f = 0; f < 2; f++) take_scales<FMT>(raw[f], sq[f]);
         }
 #pragma unroll
-        for (int mf = 0; mf < MF; mf++) acc[f][mf] = a1[0][mf];
-        load(f, p + 1);
+        for (int i = 0; i < LN; i++) {
+          const int l = q * LN + i;
+          if (!ONE && l >= nline) break;
+          const Line<FMT> q2[2] = {ln[0][i], ln[1][i]};
+          const uint32_t sw[2] = {sq[0][i], sq[1][i]};
+          line_mma<FMT, 2, MF, XP, tab_copies(false, MFX)>(q2, sw, C, 0, smem + l * XLINE, xa, tail && l == nline - 1, acc);
+        }
+        load(0, pn, qn);
+        load(1, pn, qn);
       }
-    } else {  // (64 pairs: both fragments share an activation operand's trip out of LDS)
-      asm volatile("" ::: "memory");
-      uint32_t sq[2][4];
-      if (scale_plane(FMT)) {
-#pragma unroll
-        for (int f = 0; f < 2; f++) take_scales<FMT>(raw[f], sq[f]);
-      }
-#pragma unroll
-      for (int i = 0; i < DN_LINES; i++) {
-        const Line<FMT> q2[2] = {ln[0][i], ln[1][i]};
-        const uint32_t sw[2] = {sq[0][i], sq[1][i]};
-        line_mma<FMT, 2, MF, DN_XP, tab_copies(false, MFX)>(q2, sw, C, 0, smem + i * XROW, xa, tail && i == DN_LINES - 1, acc);
-      }
-      load(0, p + 1);
-      load(1, p + 1);
     }
-    const int col = (nb + p) * DNR + 32 * wv + 8 * g;
+    const int row0 = (nb + p) * DNR + 32 * wv, col = row0 + 8 * g;
 #pragma unroll
     for (int mf = 0; mf < MF; mf++) {
       const int m = 16 * mf + n;
-      if (m < tile.count) {
+      if (m < tile.count && row0 < M) {
         uint4 o;
         __half2 h[4];
 #pragma unroll
@@ -652,25 +671,29 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
 }
 
 // Waves of a block.  Four: several blocks to a CU pass their prologues, barriers and epilogues independently.  Eight for
-// rotated experts, whose epilogue works on 128 rows, and where 64 pairs' activations fill the LDS (down: sixteen).
-constexpr int block_waves(int FMT, bool UP, int MFX) { return MFX == 4 ? (UP ? 8 : 16) : UP && FMT == F_I4R ? 8 : 4; }
+// rotated experts' gate/up, whose epilogue works on 128 rows; more as well where a tile's activations leave a CU's LDS to one or
+// two blocks (64 pairs: gate/up eight, down sixteen; down with 32 pairs and rows of more than four lines: sixteen.  us of a layer with
+// four, eight and sixteen there, q4cp, 2048 x 1536: 130 tokens 585, 620, 621, with 32 pairs to a tile 515 tokens 779, 749, 740, 800
+// 880, 805, 792; 3072 x 512: 515 tokens 401, 404, 435).
+constexpr int DN_ONE = 3;  // lines of the rows that a wave takes whole
+constexpr int up_waves(int FMT, int MFX) { return MFX == 4 || FMT == F_I4R ? 8 : 4; }
 // waves per SIMD asked for: what the registers of the lines in flight leave
-constexpr int simd_waves(int FMT, bool UP, int MFX) {
+constexpr int simd_waves(int FMT, bool UP, int MFX, int NW) {
   if (UP) return 4;
-  return MFX == 4 ? 4 : FMT == F_Q80 || FMT == F_Q4K ? 3 : 4;
+  return NW == 16 ? 4 : FMT == F_Q80 || FMT == F_Q4K ? 3 : 4;
 }
-constexpr size_t smem_bytes(int FMT, bool UP, int MFX) {
+constexpr size_t smem_bytes(int FMT, bool UP, int MFX, int nline) {
   const size_t tab = FMT == F_TAB ? (size_t)(UP ? 2 : 1) * 256 * tab_copies(UP, MFX) * 4 : 0;
-  return UP ? (size_t)2 * MFX * 16 * XROW + 256 + tab : (size_t)MFX * 16 * DN_XP + tab;
+  return UP ? (size_t)2 * MFX * 16 * XROW + 256 + tab : (size_t)MFX * 16 * XROW * nline + tab;
 }
 
-template <int FMT, bool UP, int MFX>
-__global__ void __launch_bounds__(64 * block_waves(FMT, UP, MFX), simd_waves(FMT, UP, MFX))
+// LN: lines of a piece (down)
+template <int FMT, bool UP, int MFX, int LN, int NW>
+__global__ void __launch_bounds__(64 * NW, simd_waves(FMT, UP, MFX, NW))
 k_moe_stream(SW R, SW Sh, int n_experts, const __half* __restrict__ x, const int* __restrict__ tokidx,
              const moe_tile* __restrict__ tiles, const int* __restrict__ ntiles, __half* __restrict__ out, int M, int K,
              int nblk_n, int split, int npass, moe_hscale hs, moe_rotv rot) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  constexpr int NW = block_waves(FMT, UP, MFX);
   // XCD-aware order as in gemm_q4cp.hip: consecutive workgroup ids go round-robin over the XCDs; each takes a contiguous
   // run of tiles, routed and shared ones dealt separately
   const int nt = ntiles[0], nr = split ? ntiles[1] : nt;
@@ -706,7 +729,7 @@ k_moe_stream(SW R, SW Sh, int n_experts, const __half* __restrict__ x, const int
 #define ST_GO(MF)                                                                                              \
   do {                                                                                                         \
     if constexpr (UP) up_tile<FMT, MFX, MF, FMT == F_I4R, NW>(smem, L, e, tile, nb, x, tokidx, out, M, K, pexp, hs, cmag, rot); \
-    else dn_tile<FMT, MFX, MF, NW>(smem, L, e, tile, nb, npass, x, out, M, K, pexp);                           \
+    else dn_tile<FMT, MFX, MF, NW, LN, LN == DN_ONE>(smem, L, e, tile, nb, npass, x, out, M, K, pexp);                           \
   } while (0)
   if (MFX == 1 || mfn <= 1) ST_GO(1);
   else if (MFX == 2 || mfn <= 2) ST_GO(2);
@@ -725,19 +748,19 @@ SW to_dev(const moe_lutw* p, const float* cb_up, const int8_t* pexp) {
   return d;
 }
 
-template <int FMT, bool UP, int MFX>
+template <int FMT, bool UP, int MFX, int LN, int NW>
 int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* tokidx, const moe_tile* tiles,
            const int* ntiles, int max_tiles, __half* out, int m, int k, int split, moe_hscale hs, const moe_rotv* rot,
            hipStream_t st) {
-  constexpr int NW = block_waves(FMT, UP, MFX);
-  constexpr size_t lds = smem_bytes(FMT, UP, MFX);
+  const size_t lds = smem_bytes(FMT, UP, MFX, (k + 255) / 256);
   static moe_dev_once once;
   int dev;
   if (moe_dev_pending(once, &dev)) {
-    MOE_HIP(hipFuncSetAttribute((const void*)k_moe_stream<FMT, UP, MFX>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    MOE_HIP(hipFuncSetAttribute((const void*)k_moe_stream<FMT, UP, MFX, LN, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)(LN == 0 || LN == DN_ONE ? lds : LDS_MOST)));
     moe_dev_done(once, dev);
   }
-  int nblk = UP ? (m + 16 * NW - 1) / (16 * NW) : m / (32 * NW), npass = 1;
+  int nblk = UP ? (m + 16 * NW - 1) / (16 * NW) : (m + 32 * NW - 1) / (32 * NW), npass = 1;
   // Down: a block walks several groups of rows behind one staging of the activations; the longest walk that leaves twelve
   // blocks per CU (64 pairs: two.  Staging is most of a short walk there: 2048 tokens i4r 205 us, with six blocks 223, with
   // twelve 300)
@@ -746,7 +769,7 @@ int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* 
       if (nblk % c == 0 && (int64_t)max_tiles * (nblk / c) >= (MFX == 4 ? 512 : 3072)) npass = c;
   nblk /= npass;
   const int per_xcd = (max_tiles + 7) / 8 + 1;
-  k_moe_stream<FMT, UP, MFX><<<(unsigned)(per_xcd * nblk * 8), 64 * NW, lds, st>>>(
+  k_moe_stream<FMT, UP, MFX, LN, NW><<<(unsigned)(per_xcd * nblk * 8), 64 * NW, lds, st>>>(
       R, S, n_experts, x, tokidx, tiles, ntiles, out, m, k, nblk, split, npass, hs, rot ? *rot : moe_rotv{nullptr, nullptr});
   MOE_LAUNCH_CHECK();
   return MOE_OK;
@@ -760,12 +783,22 @@ int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* 
 // At 44 a tenth of the experts takes a second tile and the 128-pair kernels draw level (2300 tokens, average 45: 945 against
 // 940 us; 2048: 855 against 924).  Q5_K and Q8_0 fragments leave no registers for 64 pairs: 32-pair tiles win up to about
 // 40 (1700 tokens, average 33: 1248 against 1339 us; 2600, 51: 1542 against 1451).
-int moe_stream_tile_cap(int P, int k, int experts, bool wide) {
+// Rows of more than four lines of hid (mid > 1024) leave no LDS for 64 pairs: 32-pair tiles as well, level earlier (2048 x 1536, us
+// with the 128-pair kernels and with these, at averages of 23: q4cp 896 891, Q4_K 967 912; 29: q4cp 923 967, Q4_K 996 1038, table
+// 1149 1139, Q5_K / Q8_0 1519 1434; 37: table 1248 1409, Q5_K / Q8_0 1612 1741).
+constexpr float ONCE_LINE = 38.f;
+int moe_stream_tile_cap(int P, int k, int experts, int fmt_up, int fmt_dn, int mid) {
   const float avg = (float)P * (float)k / (float)experts;
+  const bool small = q5(fmt_up) || fmt_dn == F_Q80, lone = mid > 1024;
+  const float line = once_rounded(fmt_up) ? ONCE_LINE : small ? (lone ? 32.f : 38.f) : fmt_up == F_TAB ? (lone ? 29.f : 44.f) : lone ? 25.f : 44.f;
   if (avg <= 10.f) return 16;
-  return wide ? (avg <= 22.f ? 32 : avg <= 44.f ? 64 : 0) : avg <= 38.f ? 32 : 0;
+  return avg > line ? 0 : small || lone || avg <= 22.f ? 32 : 64;
 }
-bool moe_stream_wide(int fmt_up, int fmt_dn) { return !q5(fmt_up) && fmt_dn != F_Q80; }
+// The smallest that any layer takes (0 above the last line): what the tile list is sized for.
+int moe_stream_tile_cap_least(int P, int k, int experts) {
+  const float avg = (float)P * (float)k / (float)experts;
+  return avg <= 10.f ? 16 : avg <= 38.f ? 32 : avg <= 44.f ? 64 : 0;
+}
 
 // fmt: MOE_STREAM_*; the views as for moe_launch_gemm_q4cp.  max_tiles == 0: checks only.
 int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const moe_lutw* sh, int n_experts, const __half* x,
@@ -786,8 +819,8 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
   };
   if (!ok(routed) || (sh && !ok(sh))) return MOE_E_UNSUPPORTED;
   if (k % 128 || ((q4(fmt) || q5(fmt) || fmt == F_I4R) && k % 256)) return MOE_E_UNSUPPORTED;
-  // (down: rows of three lines, and whole groups of rows for sixteen waves)
-  if (up ? k < 256 : (k + 255) / 256 != DN_LINES || m % 512) return MOE_E_UNSUPPORTED;
+  // (down: groups of 32 rows, and a tile's hid rows in LDS)
+  if (up ? k < 256 : k < 128 || m % 32 || smem_bytes(fmt, false, cap / 16, (k + 255) / 256) > LDS_MOST) return MOE_E_UNSUPPORTED;
   if (up && (m % 16 || (fmt >= F_Q4K && m % 64) || (fmt == F_I4R && m % 128))) return MOE_E_UNSUPPORTED;
   if ((up && fmt == F_Q80) || (!up && (q5(fmt) || once_rounded(fmt))) || (cap > 32 && (q5(fmt) || fmt == F_Q80))) return MOE_E_UNSUPPORTED;
   if (fmt == F_I4R && up != (rot != nullptr)) return MOE_E_INVALID;
@@ -798,17 +831,34 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
   const SW R = to_dev(routed, nullptr, pexp_routed), S = to_dev(sh ? sh : routed, sh ? sh_cb_up : nullptr, sh ? pexp_sh : pexp_routed);
   const int split = sh ? 1 : 0;
 #define ST_ARGS R, S, n_experts, x, tokidx, tiles, ntiles, max_tiles, out, m, k, split, hs, rot, st
-#define ST_CAP(F, U)                                \
-  do {                                              \
-    if (cap == 16) return launch<F, U, 1>(ST_ARGS); \
-    if (cap == 32) return launch<F, U, 2>(ST_ARGS); \
-    if constexpr (!q5(F) && F != F_Q80) return launch<F, U, 4>(ST_ARGS); \
-    return MOE_E_UNSUPPORTED;                       \
+#define ST_UP(F)                                                                        \
+  do {                                                                                  \
+    if (cap == 16) return launch<F, true, 1, 0, up_waves(F, 1)>(ST_ARGS);               \
+    if (cap == 32) return launch<F, true, 2, 0, up_waves(F, 2)>(ST_ARGS);               \
+    if constexpr (!q5(F)) return launch<F, true, 4, 0, up_waves(F, 4)>(ST_ARGS);        \
+    return MOE_E_UNSUPPORTED;                                                           \
   } while (0)
-#define ST_DIR(F)            \
-  do {                       \
-    if (up) ST_CAP(F, true); \
-    ST_CAP(F, false);        \
+  // (Q4_K with 64 pairs has no registers for whole rows of three lines: 21 in scratch, and 743 us for 733 at 1500 tokens, 815
+  //  for 805 at 2000; the other formats lose 1 .. 2 % with pieces of two)
+  const int nline = (k + 255) / 256;
+#define ST_DN(F)                                                                        \
+  do {                                                                                  \
+    if (nline == DN_ONE && !(F == F_Q4K && cap > 32)) {                                 \
+      if (cap == 16) return launch<F, false, 1, DN_ONE, 4>(ST_ARGS);                    \
+      if (cap == 32) return launch<F, false, 2, DN_ONE, 4>(ST_ARGS);                    \
+      if constexpr (F != F_Q80 && F != F_Q4K) return launch<F, false, 4, DN_ONE, 16>(ST_ARGS); \
+      return MOE_E_UNSUPPORTED;                                                         \
+    }                                                                                   \
+    if (cap == 16) return launch<F, false, 1, 2, 4>(ST_ARGS);                           \
+    if (cap == 32 && nline <= 4) return launch<F, false, 2, 2, 4>(ST_ARGS);             \
+    if (cap == 32) return launch<F, false, 2, 2, 16>(ST_ARGS);                          \
+    if constexpr (F != F_Q80) return launch<F, false, 4, 2, 16>(ST_ARGS);               \
+    return MOE_E_UNSUPPORTED;                                                           \
+  } while (0)
+#define ST_DIR(F)      \
+  do {                 \
+    if (up) ST_UP(F);  \
+    ST_DN(F);          \
   } while (0)
   switch (fmt) {
     case F_DN: ST_DIR(F_DN);
@@ -816,13 +866,14 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
     case F_TAB: ST_DIR(F_TAB);
     case F_I4R: ST_DIR(F_I4R);
     case F_Q4K: ST_DIR(F_Q4K);
-    case F_Q5K: ST_CAP(F_Q5K, true);
-    case F_Q4E: ST_CAP(F_Q4E, true);
-    case F_Q5E: ST_CAP(F_Q5E, true);
-    case F_Q80: ST_CAP(F_Q80, false);
+    case F_Q5K: ST_UP(F_Q5K);
+    case F_Q4E: ST_UP(F_Q4E);
+    case F_Q5E: ST_UP(F_Q5E);
+    case F_Q80: ST_DN(F_Q80);
     default: return MOE_E_INVALID;
   }
 #undef ST_ARGS
-#undef ST_CAP
+#undef ST_UP
+#undef ST_DN
 #undef ST_DIR
 }
