@@ -778,26 +778,33 @@ int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* 
 }  // namespace
 
 // Pairs per tile for a batch of P tokens, 0 = the batch belongs to the 128-pair kernels.
-// The lines: an expert's pairs spread by about the root of their mean, so 16 and 32 hold nearly all experts in one tile up
-// to 10 and 22; 64-pair tiles at an average of 25 against 32-pair ones: 797 -> 779 us per layer (q4cp), 740 -> 738 (i4r).
-// At 44 a tenth of the experts takes a second tile and the 128-pair kernels draw level (2300 tokens, average 45: 945 against
-// 940 us; 2048: 855 against 924).  Q5_K and Q8_0 fragments leave no registers for 64 pairs: 32-pair tiles win up to about
-// 40 (1700 tokens, average 33: 1248 against 1339 us; 2600, 51: 1542 against 1451).
-// Rows of more than four lines of hid (mid > 1024) leave no LDS for 64 pairs: 32-pair tiles as well, level earlier (2048 x 1536, us
-// with the 128-pair kernels and with these, at averages of 23: q4cp 896 891, Q4_K 967 912; 29: q4cp 923 967, Q4_K 996 1038, table
-// 1149 1139, Q5_K / Q8_0 1519 1434; 37: table 1248 1409, Q5_K / Q8_0 1612 1741).
-constexpr float ONCE_LINE = 38.f;
+// An expert's pairs spread by about the root of their mean, so tiles of 16 and 32 hold nearly all experts in one up to averages of 10
+// and 22; 64-pair tiles at an average of 25 against 32-pair ones: 797 -> 779 us per layer (q4cp), 740 -> 738 (i4r).  Above, more
+// and more experts take a second tile and the 128-pair kernels draw level; the line lies where they do, for each kind of
+// layer with its own kernels, at even and at Zipf-skewed routing.  Layers, us, 128-pair kernels and these (3072 x 768):
+//   average pairs        44, even / skewed            49                         59
+//   q4cp                 867 791 / 885 840            888 871 / 920 875          932 935 / 982 950
+//   Q4_K                 933 840 / 943 913            956 941 / 994 957          1000 1013 / 1045 1046
+//   i4r                  869 794 / 886 854            887 869 / 928 894          956 953 / 994 995
+//   table                1047 930 / 1068 991          1069 1013 / 1102 1046      1134 1114 / 1187 1139
+//   Q5_K / Q8_0          29: 1268 1052 / 1296 1079    37: 1324 1270 / 1342 1204  44: 1344 1390 / 1384 1328
+// Q5_K and Q8_0 fragments leave no registers for 64 pairs (32-pair tiles above 22).  Rows of more than four lines of hid (mid >
+// 1024) leave no LDS for them: 32-pair tiles as well, level earlier (2048 x 1536, even: 23 q4cp 896 891, Q4_K 967 912; 29 q4cp
+// 923 967, Q4_K 996 1038, table 1149 1139, Q5_K / Q8_0 1519 1434; 37 table 1248 1409, Q5_K / Q8_0 1612 1741).
+// Layers that go to the general kernel otherwise (F_Q4E, F_Q5E): as far as was measured (2560 x 640: 59 1979 1245 / 2153 1257; 160
+// 3888 2682 / 3480 2691; 2048 x 1152: 160 5146 4036 / 4570 4035).
+constexpr float ONCE_LINE = 160.f;
 int moe_stream_tile_cap(int P, int k, int experts, int fmt_up, int fmt_dn, int mid) {
   const float avg = (float)P * (float)k / (float)experts;
   const bool small = q5(fmt_up) || fmt_dn == F_Q80, lone = mid > 1024;
-  const float line = once_rounded(fmt_up) ? ONCE_LINE : small ? (lone ? 32.f : 38.f) : fmt_up == F_TAB ? (lone ? 29.f : 44.f) : lone ? 25.f : 44.f;
+  const float line = once_rounded(fmt_up) ? ONCE_LINE : small ? (lone ? 32.f : 38.f) : fmt_up == F_TAB ? (lone ? 29.f : 60.f) : lone ? 25.f : 50.f;
   if (avg <= 10.f) return 16;
   return avg > line ? 0 : small || lone || avg <= 22.f ? 32 : 64;
 }
 // The smallest that any layer takes (0 above the last line): what the tile list is sized for.
 int moe_stream_tile_cap_least(int P, int k, int experts) {
   const float avg = (float)P * (float)k / (float)experts;
-  return avg <= 10.f ? 16 : avg <= 38.f ? 32 : avg <= 44.f ? 64 : 0;
+  return avg <= 10.f ? 16 : avg <= ONCE_LINE ? 32 : 0;
 }
 
 // fmt: MOE_STREAM_*; the views as for moe_launch_gemm_q4cp.  max_tiles == 0: checks only.

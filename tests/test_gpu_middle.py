@@ -361,3 +361,25 @@ def test_few_pair_tiles_are_no_less_exact(capi, oracle, kind, kw, d, mid, T):
     e1, e0 = (np.linalg.norm(y - yo) / np.linalg.norm(yo) for y in (y1, y0))
     assert e1 <= 1.02 * e0 <= 1e-3, (e1, e0)
     assert (y1 != y0).any() or (mid > 1024 and T > 100)  # (two kernels; longer rows leave them earlier)
+
+
+@pytest.mark.parametrize("kind,kw,d,mid,last", [("q4cp", dict(fmt="q4cp"), 512, 640, 50), ("q4cp", dict(fmt="q4cp"), 384, 1152, 25),
+                                                ("table", dict(fmt="q4cp", codebook=TABLE), 512, 768, 60), ("i4r", dict(fmt="i4r"), 512, 768, 50),
+                                                ("table", dict(fmt="q4cp", codebook=TABLE), 384, 1152, 29), ("q4k", dict(fmt="q4k"), 512, 768, 50),
+                                                ("q5k-q8_0", dict(fmt="q4k", gg_types=(13, 8, 8)), 512, 768, 38),
+                                                ("q5k-q8_0", dict(fmt="q4k", gg_types=(13, 8, 8)), 512, 1280, 32),
+                                                ("q5k-q8_0", dict(fmt="q4k", gg_types=(13, 8, 8)), 512, 640, 160)])
+def test_where_the_few_pair_tiles_end(capi, oracle, kind, kw, d, mid, last):
+    """The largest batch that each kind of layer runs on them, and the next one on the 128-pair kernels."""
+    E, k = 16, 4
+    T = last * E // k
+    rng = np.random.default_rng(T + mid)
+    hl = HostLayer(rng, d, mid, E, k, **kw)
+    x = rng.standard_normal((T + 1, d), dtype=np.float32)
+    sel = np.r_[0, T // 2, T - 1]
+    yo, _, _ = oracle.moe_layer(hl.oracle_layer(), x[sel])
+    y1, y0 = both_kernels(capi, hl, x[:T])
+    assert (y1 != y0).any()
+    assert max_abs_rel(y1[sel], yo) <= 2e-3
+    y1, y0 = both_kernels(capi, hl, x)
+    assert (y1 == y0).all()
