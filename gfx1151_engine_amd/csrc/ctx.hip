@@ -1126,7 +1126,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
       const moe_rotv rv{L.v2_svh_gu, L.v2_suh_dn};
       moe_lutw gf = gu;
       if (v2) gf.up_off = g.mid;
-      return moe_launch_stream(sk.up, true, cap, &gf, with_sh ? &sgu : nullptr, g.experts, v2 ? c->v2_x16 : xh, c->tokidx, tl, ntl,
+      return moe_launch_stream(sk.up, true, cap, &gf, with_sh ? &sgu : nullptr, g.experts, v2 ? c->v2_x16 : xh, P, c->tokidx, tl, ntl,
                                mt, c->hid16, g.mid, g.d, hs, s2, sh_cb_up, pe_gu, pe_sgu, v2 ? &rv : nullptr);
     }
     if (shd && with_sh)  // the shared expert's own tile list
@@ -1173,7 +1173,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   auto gemm_dn = [&](bool routed, bool with_sh, const moe_tile* tl, const int* ntl, int mt, hipStream_t s2, const moe_comb* cmb) -> int {
     if (dry) mt = 0;
     if (routed && cap)
-      return moe_launch_stream(sk.dn, false, cap, &dn, with_sh ? &sdn : nullptr, g.experts, c->hid16, nullptr, tl, ntl, mt,
+      return moe_launch_stream(sk.dn, false, cap, &dn, with_sh ? &sdn : nullptr, g.experts, c->hid16, 0, nullptr, tl, ntl, mt,
                                c->pairs16, g.d, g.mid, hs, s2, nullptr, pe_dn, pe_sdn);
     if (shd && with_sh)  // (hid rows of the shared tiles were written in natural order by the launch above)
       return moe_launch_gemm_gg(false, L.sh_dense, L.sh_down.data, nullptr, 0, nullptr, nullptr, g.experts, c->hid16,

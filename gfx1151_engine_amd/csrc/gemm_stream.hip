@@ -224,12 +224,11 @@ __device__ __forceinline__ void line_mma(const Line<FMT> (&q)[F], const uint32_t
             bs[f][0] = half2v{b.x, b.x}; bs[f][1] = half2v{b.y, b.y};
           }
         } else {
-          const half2v s2 = h2(sw[f]);
-          const _Float16 sh = E_ ? s2.y : s2.x;
+          const half2v s2 = h2(__builtin_amdgcn_perm(sw[f], sw[f], E_ ? 0x03020302u : 0x01000100u));
           if (FMT == F_TAB) {
-            as[f][0] = half2v{sh, sh};
+            as[f][0] = s2;
           } else {
-            const float s = (float)sh;
+            const float s = (float)s2.x;
             as[f][0] = both(C.cb_a[f0 + f] * s);
             bs[f][0] = bs[f][1] = both(C.cb_b[f0 + f] * s);
             as[f][1] = FMT == F_DN ? as[f][0] * both(0.0625f) : as[f][0];
@@ -418,23 +417,24 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
   constexpr int XL = MF * 16 * 32 / NT, XS = NT / 32;  // loads per thread and line, rows per load
   static_assert(XL >= 1 && XL <= 4, "named registers below");
   const int xc = tid & 31, xt = tid >> 5;
-  const __half* xr[XL];
+  uint32_t xr[XL];  // (32-bit byte offsets: moe_launch_stream)
 #pragma unroll
   for (int l = 0; l < XL; l++) {
     const int m = XS * l + xt;
     const int row = tokidx[tile.first + (m < tile.count ? m : 0)];
-    xr[l] = x + (size_t)row * K + 8 * xc;
+    xr[l] = ((uint32_t)row * (uint32_t)K + 8u * (uint32_t)xc) * 2u;
     if (xc == 0) rowscale[m] = hs.xms ? moe_hid_scale(cmag, hs.xms[row]) : 1.f;
   }
   uint4 xv0, xv1, xv2, xv3;  // (named: an array here ends up in scratch memory)
   auto fetch_x = [&](int i) {
     i = i < nline ? i : nline - 1;
     const bool half = tail && i == nline - 1;
-    const int o = i * 256 - (half && xc >= 16 ? 128 : 0);
-    xv0 = *(const uint4*)(xr[0] + o);
-    if constexpr (XL > 1) xv1 = *(const uint4*)(xr[1] + o);
-    if constexpr (XL > 2) xv2 = *(const uint4*)(xr[2] + o);
-    if constexpr (XL > 3) xv3 = *(const uint4*)(xr[3] + o);
+    const uint8_t* const xb = (const uint8_t*)x + 512 * (size_t)i;
+    const uint32_t back = half && xc >= 16 ? 256u : 0u;
+    xv0 = *(const uint4*)(xb + (xr[0] - back));
+    if constexpr (XL > 1) xv1 = *(const uint4*)(xb + (xr[1] - back));
+    if constexpr (XL > 2) xv2 = *(const uint4*)(xb + (xr[2] - back));
+    if constexpr (XL > 3) xv3 = *(const uint4*)(xb + (xr[3] - back));
   };
   auto put_x = [&](int buf) {
     auto put = [&](int l, const uint4& v) {
@@ -672,14 +672,19 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
 
 // Waves of a block.  Four: several blocks to a CU pass their prologues, barriers and epilogues independently.  Eight for
 // rotated experts' gate/up, whose epilogue works on 128 rows; more as well where a tile's activations leave a CU's LDS to one or
-// two blocks (64 pairs: gate/up eight, down sixteen; down with 32 pairs and rows of more than four lines: sixteen.  us of a layer with
+// two blocks (64 pairs: gate/up eight, down sixteen; down with 32 pairs and rows of more than four lines: sixteen, Q8_0 with its
+// registers eight.  us of a layer with
 // four, eight and sixteen there, q4cp, 2048 x 1536: 130 tokens 585, 620, 621, with 32 pairs to a tile 515 tokens 779, 749, 740, 800
 // 880, 805, 792; 3072 x 512: 515 tokens 401, 404, 435).
 constexpr int DN_ONE = 3;  // lines of the rows that a wave takes whole
 constexpr int up_waves(int FMT, int MFX) { return MFX == 4 || FMT == F_I4R ? 8 : 4; }
-// waves per SIMD asked for: what the registers of the lines in flight leave
+// waves per SIMD asked for: what the registers of the lines in flight leave.  (Gate/up with Q5_K rounded once, 32 pairs: three; with
+// four 21 registers went to scratch inside the loop, 757 us for 702 at 1200 tokens of 2560 x 640.  A few kernels keep 1 .. 4
+// registers of their prologue in scratch until the epilogue, F_DN's down launch with 64 pairs an address once per pass:
+// gate/up F_DN and F_AFF with 64 pairs, F_Q5K with 32; down F_DN and F_TAB with 64.  F_Q5K with three waves has none and is no
+// faster: 808 us for 799 at 515 tokens, 1159 for 1152 at 1700.)
 constexpr int simd_waves(int FMT, bool UP, int MFX, int NW) {
-  if (UP) return 4;
+  if (UP) return FMT == F_Q5E && MFX == 2 ? 3 : 4;
   return NW == 16 ? 4 : FMT == F_Q80 || FMT == F_Q4K ? 3 : 4;
 }
 constexpr size_t smem_bytes(int FMT, bool UP, int MFX, int nline) {
@@ -807,8 +812,8 @@ int moe_stream_tile_cap_least(int P, int k, int experts) {
   return avg <= 10.f ? 16 : avg <= ONCE_LINE ? 32 : 0;
 }
 
-// fmt: MOE_STREAM_*; the views as for moe_launch_gemm_q4cp.  max_tiles == 0: checks only.
-int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const moe_lutw* sh, int n_experts, const __half* x,
+// fmt: MOE_STREAM_*; the views as for moe_launch_gemm_q4cp; x_rows: rows of x.  max_tiles == 0: checks only.
+int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const moe_lutw* sh, int n_experts, const __half* x, int x_rows,
                       const int* tokidx, const moe_tile* tiles, const int* ntiles, int max_tiles, __half* out, int m, int k,
                       moe_hscale hs, hipStream_t st, const float* sh_cb_up, const int8_t* pexp_routed,
                       const int8_t* pexp_sh, const moe_rotv* rot) {
@@ -827,6 +832,7 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
   if (!ok(routed) || (sh && !ok(sh))) return MOE_E_UNSUPPORTED;
   if (k % 128 || ((q4(fmt) || q5(fmt) || fmt == F_I4R) && k % 256)) return MOE_E_UNSUPPORTED;
   // (down: groups of 32 rows, and a tile's hid rows in LDS)
+  if (up && (uint64_t)x_rows * (uint64_t)k * 2 >= 1ull << 32) return MOE_E_UNSUPPORTED;  // (32-bit byte offsets into x)
   if (up ? k < 256 : k < 128 || m % 32 || smem_bytes(fmt, false, cap / 16, (k + 255) / 256) > LDS_MOST) return MOE_E_UNSUPPORTED;
   if (up && (m % 16 || (fmt >= F_Q4K && m % 64) || (fmt == F_I4R && m % 128))) return MOE_E_UNSUPPORTED;
   if ((up && fmt == F_Q80) || (!up && (q5(fmt) || once_rounded(fmt))) || (cap > 32 && (q5(fmt) || fmt == F_Q80))) return MOE_E_UNSUPPORTED;
@@ -842,7 +848,7 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
   do {                                                                                  \
     if (cap == 16) return launch<F, true, 1, 0, up_waves(F, 1)>(ST_ARGS);               \
     if (cap == 32) return launch<F, true, 2, 0, up_waves(F, 2)>(ST_ARGS);               \
-    if constexpr (!q5(F)) return launch<F, true, 4, 0, up_waves(F, 4)>(ST_ARGS);        \
+    if constexpr (!q5(F) && !once_rounded(F)) return launch<F, true, 4, 0, up_waves(F, 4)>(ST_ARGS); \
     return MOE_E_UNSUPPORTED;                                                           \
   } while (0)
   // (Q4_K with 64 pairs has no registers for whole rows of three lines: 21 in scratch, and 743 us for 733 at 1500 tokens, 815
@@ -858,7 +864,7 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
     }                                                                                   \
     if (cap == 16) return launch<F, false, 1, 2, 4>(ST_ARGS);                           \
     if (cap == 32 && nline <= 4) return launch<F, false, 2, 2, 4>(ST_ARGS);             \
-    if (cap == 32) return launch<F, false, 2, 2, 16>(ST_ARGS);                          \
+    if (cap == 32) return launch<F, false, 2, 2, F == F_Q80 ? 8 : 16>(ST_ARGS);         \
     if constexpr (F != F_Q80) return launch<F, false, 4, 2, 16>(ST_ARGS);               \
     return MOE_E_UNSUPPORTED;                                                           \
   } while (0)
