@@ -1394,7 +1394,8 @@ MOE_API int moe_x16_layout(moe_ctx* c, int layer) {
 }
 
 // moe_forward for a batch whose f16 copy the caller has already made (its HC-read epilogue can write it next to
-// the f32 rows, src/gpu/parts/40_model.inc:2556-2565,4817): the library's own conversion pass is left out.
+// the f32 rows, src/gpu/parts/40_model.inc:2556-2565,4817): the GEMMs read it, and up to 256 tokens the library makes no
+// copy of its own (above, the candidate selection writes one with its own rounding in any case).
 MOE_API int moe_forward_x16(moe_ctx* c, int layer, const float* x, const void* x16, int P, float* y, moe_stream_t st) {
   MoeLayer* L = layer_of(c, layer);
   if (!L || !x || !x16 || !y || P < 0) return MOE_E_INVALID;

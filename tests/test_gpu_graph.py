@@ -87,3 +87,40 @@ def test_other_paths_under_graph_capture(oracle, variant, T):
             torch.cuda.synchronize()
             assert torch.equal(y, eager[1 - i])
     m.close()
+
+
+def test_listed_tokens_under_graph_capture(oracle):
+    """A batch whose router lists tokens: none, a few and all of them from replay to replay of one graph (the list, its
+    count and its tickets are the call's own)."""
+    import torch
+    rng = np.random.default_rng(9)
+    d, mid, E, k, T = 512, 256, 64, 4, 300
+    hl = HostLayer(rng, d, mid, E, k)
+    m, dev = hl.to_gpu(max_tokens=T)
+    base = rng.standard_normal((T, d), dtype=np.float32)
+    few = base.copy()
+    few[::37] *= 400.0
+    xs = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (base, few, base * np.float32(400.0))]
+    x, y = torch.empty_like(xs[0]), torch.empty_like(xs[0])
+    eager = []
+    for xi in xs:
+        x.copy_(xi)
+        m.forward(0, x, y)
+        eager.append((y.clone(), m.last_routing(T)[0]))
+        io = oracle.router(hl.oracle_layer().router, xi.cpu().numpy(), k)[1]
+        assert (eager[-1][1].cpu().numpy()[:, :k] == io[:, :k]).all()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        m.forward(0, x, y)
+    for rep in range(3):
+        for i in (0, 2, 1, 2, 0):
+            x.copy_(xs[i])
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y.nan_to_num(), eager[i][0].nan_to_num()), (rep, i)
+            assert torch.equal(m.last_routing(T)[0], eager[i][1])
+            m.forward(0, xs[(i + 1) % 3], y)
+            torch.cuda.synchronize()
+            assert torch.equal(y.nan_to_num(), eager[(i + 1) % 3][0].nan_to_num())
+    m.close()

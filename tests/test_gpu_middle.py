@@ -383,3 +383,17 @@ def test_where_the_few_pair_tiles_end(capi, oracle, kind, kw, d, mid, last):
     assert max_abs_rel(y1[sel], yo) <= 2e-3
     y1, y0 = both_kernels(capi, hl, x)
     assert (y1 == y0).all()
+
+
+@pytest.mark.parametrize("fmt,T", [("q4cp", 40), ("q4cp", 300), ("q4k", 300), ("q4cp", 1100)])
+def test_the_callers_f16_copy_at_every_router(capi, fmt, T):
+    """moe_forward_x16 against moe_forward, bit for bit; the router of 257 tokens and more makes its own copy all the same."""
+    rng = np.random.default_rng(T)
+    hl = HostLayer(rng, 512, 256, 16, 4, fmt=fmt)
+    m, dev = hl.to_gpu(max_tokens=T)
+    x = gpu(rng.standard_normal((T, 512), dtype=np.float32))
+    y0 = m.forward(0, x).cpu().numpy()
+    i0 = m.last_routing(T)[0].cpu().numpy()
+    y1 = m.forward_x16(0, x, capi.f32_to_f16(x, layout=m.x16_layout(0))).cpu().numpy()
+    assert (y0 == y1).all() and (m.last_routing(T)[0].cpu().numpy() == i0).all()
+    m.close()
