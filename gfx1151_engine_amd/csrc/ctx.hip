@@ -14,7 +14,9 @@ struct MoeLayer {
   moe_wview router{};
   const float* router_bias = nullptr;
   float router_wmax = 0.f;  // the largest row norm of the router matrix (the bound of the small-batch selection, moe_rfix)
-  float router_bmax = 0.f;  // the largest |bias| (how far a logit's dot product can lie above the logit itself; experts switched off by a bias of minus infinity aside)
+  // the largest |bias| (how far a logit's dot product can lie above the logit itself), experts switched off by a bias of
+  // minus infinity aside
+  float router_bmax = 0.f;
   moe_wview gate_up{}, down{};
   moe_gg_experts gg{};
   moe_wview sh_gate{}, sh_up{}, sh_down{}, sh_sg{};

@@ -7,15 +7,17 @@
 // on this chip (a load of 16 rows x 64 bytes per wave instruction, four or more in flight per wave; 32 rows x 32 bytes:
 // 4.4 .. 5.3).  Here:
 //   - a wave owns 16 weight rows twice (gate/up: 16 gate rows and their 16 up rows; down: 32 rows) and walks K, any multiple of
-//     128 (K-quants and i4r: 256), in lines of 256 columns.  v_mfma_f32_16x16x32_f16 takes the weights as A: lane (n, g) = row n, 16-byte chunks g and g + 4 of
-//     the line's 128 code bytes, so a load instruction covers 64 contiguous bytes of 16 rows and a chunk is one lane's
-//     operand for four MFMAs.  Which columns a lane group multiplies is free as long as the activations agree; a chunk
-//     is one scale group of 32 columns (q4cp), half of a 64-column run (Q4_K, Q5_K), a lane group's run (Q8_0).
+//     128 (K-quants and i4r: 256), in lines of 256 columns.  v_mfma_f32_16x16x32_f16 takes the weights as A: lane (n, g) = row
+//     n, 16-byte chunks g and g + 4 of the line's 128 code bytes, so a load instruction covers 64 contiguous bytes of 16 rows
+//     and a chunk is one lane's operand for four MFMAs.  Which columns a lane group multiplies is free as long as the
+//     activations agree; a chunk is one scale group of 32 columns (q4cp), half of a 64-column run (Q4_K, Q5_K), a lane group's
+//     run (Q8_0).
 //   - gate/up keeps two lines per wave in flight, line by line; down requests a fragment's whole rows at once where they are
-//     three lines, else two lines at a time.  Rows start 64 bytes off the 128-byte cache lines (the codebook heads the tensor), so every line
-//     shares a cache line with the next one, and read a line at a time a third of the traffic is fetched twice (1.66 GB for
-//     1.26, at 6.15 TB/s); whole rows brought down from 6.9 to 5.3 M cache lines (of 5.0).  For gate/up the same, pairs of
-//     lines with four in registers, fetched 1.51 GB and was no faster (270 us either way, three waves per SIMD for four).
+//     three lines, else two lines at a time.  Rows start 64 bytes off the 128-byte cache lines (the codebook heads the tensor),
+//     so every line shares a cache line with the next one, and read a line at a time a third of the traffic is fetched twice
+//     (1.66 GB for 1.26, at 6.15 TB/s); whole rows brought down from 6.9 to 5.3 M cache lines (of 5.0).  For gate/up the same,
+//     pairs of lines with four in registers, fetched 1.51 GB and was no faster (270 us either way, three waves per SIMD for
+//     four).
 //   - activations (16 pairs per MFMA, up to 64 per tile) go through LDS: gate/up one line at a time, double-buffered, one
 //     LDS-only barrier per line; down, where they are short, once per block, which then runs without barriers.
 //   - no branch stands around a load of the loops: the compiler counts outstanding loads exactly only along straight code
@@ -802,7 +804,10 @@ constexpr float ONCE_LINE = 160.f;
 int moe_stream_tile_cap(int P, int k, int experts, int fmt_up, int fmt_dn, int mid) {
   const float avg = (float)P * (float)k / (float)experts;
   const bool small = q5(fmt_up) || fmt_dn == F_Q80, lone = mid > 1024;
-  const float line = once_rounded(fmt_up) ? ONCE_LINE : small ? (lone ? 32.f : 38.f) : fmt_up == F_TAB ? (lone ? 29.f : 60.f) : lone ? 25.f : 50.f;
+  const float line = once_rounded(fmt_up) ? ONCE_LINE
+                     : small              ? (lone ? 32.f : 38.f)
+                     : fmt_up == F_TAB    ? (lone ? 29.f : 60.f)
+                                          : (lone ? 25.f : 50.f);
   if (avg <= 10.f) return 16;
   return avg > line ? 0 : small || lone || avg <= 22.f ? 32 : 64;
 }

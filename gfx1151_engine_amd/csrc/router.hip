@@ -217,8 +217,8 @@ __device__ __forceinline__ void router_plane_blocks(int q, int bs, int tid, cons
 // 190 (Q5_K / Q8_0).
 // Column steps of 256 requested together: what registers and one trip allow.  Steps past the row's end load its head again.
 // Two q4cp layers of 1 / 2 / 3 / 4 tokens, us, against one load in flight per step: 1024 columns 34 / 39 / 48 / 58 (34 / 42 /
-// 53 / 60), 2048 37 / 53 / 63 / 78 (42 / 60 / 74 / 93), 2560 38 / 46 / 63 / 80 (45 / 57 / 78 / 94), 4096 86 / 130 / 127 / 148 (93 / 148 / 149 /
-// 178), 5120 99 / 134 / 165 / 200 (109 / 158 / 206 / 257).
+// 53 / 60), 2048 37 / 53 / 63 / 78 (42 / 60 / 74 / 93), 2560 38 / 46 / 63 / 80 (45 / 57 / 78 / 94), 4096 86 / 130 / 127 /
+// 148 (93 / 148 / 149 / 178), 5120 99 / 134 / 165 / 200 (109 / 158 / 206 / 257).
 constexpr int RSM_IT = 12;
 template <bool BF>
 struct RsmW {

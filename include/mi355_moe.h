@@ -272,9 +272,10 @@ int moe_forward_hc(moe_ctx* ctx, int layer, const float* x, int P, const float* 
  * moe_q4w_run / moe_gguf convert once more, :1762, :1703).  x16: f16 [P][d] as moe_f32_to_f16(x, ., layout) makes it,
  * layout = moe_x16_layout(ctx, layer) (q4cp experts: 1, or 0 = natural order when their codebook is a table rather than
  * a*n + b; GGUF layers: 2 when the launches that read x run Q4_K / Q5_K tensors on the tuned kernel, else 0).  x (f32) is still read by the router.
- * The GEMMs read the caller's copy.  Up to 256 tokens (at any size with more than 512 experts or MOE_OPT_ROUTER_CANDIDATES = 0) the library makes none of its
- * own; above, the router's selection is certain of its expert ids only from a copy with this library's rounding, which its
- * first launch writes on its way over x whether or not one is handed over: nothing is saved there.  P > 32 only (MOE_E_UNSUPPORTED below: the small-batch kernels do
+ * The GEMMs read the caller's copy.  Up to 256 tokens (at any size with more than 512 experts or with
+ * MOE_OPT_ROUTER_CANDIDATES = 0) the library makes none of its own; above, the router's selection is certain of its expert ids
+ * only from a copy with this library's rounding, which its first launch writes on its way over x whether or not one is
+ * handed over: nothing is saved there.  P > 32 only (MOE_E_UNSUPPORTED below: the small-batch kernels do
  * not use an f16 copy; call moe_forward there), and a format outside the grouped GEMM returns MOE_E_UNSUPPORTED. */
 int moe_x16_layout(moe_ctx* ctx, int layer);
 int moe_forward_x16(moe_ctx* ctx, int layer, const float* x, const void* x16, int P, float* y, moe_stream_t st);
@@ -299,9 +300,10 @@ int moe_forward_x16(moe_ctx* ctx, int layer, const float* x, const void* x16, in
  * expert's tiles ride in the routed experts' launches.  Same arithmetic either way. */
 /* MOE_OPT_ROUTER_CANDIDATES (default 1): batches over 32 tokens find each token's experts without the dense fp64
  * pass over all experts: approximate logits on the f16 matrix pipe with a rigorous error bound select the experts
- * that can be among the k best, whose logits are then computed as fp64 sums; tokens that those cannot settle (near ties, a logit
- * range in which probabilities underflow, values that are not finite) are redone with the reference's sequential sums
- * (src/ref.cpp:70-77) over all experts.  Up to 256 tokens all logits are fp64 sums, the doubtful ones the reference's.  Expert ids and their order are the reference's bit for bit; the renormalised
+ * that can be among the k best, whose logits are then computed as fp64 sums; tokens that those cannot settle (near ties, a
+ * logit range in which probabilities underflow, values that are not finite) are redone with the reference's sequential
+ * sums (src/ref.cpp:70-77) over all experts.  Up to 256 tokens all logits are fp64 sums, the doubtful ones the
+ * reference's.  Expert ids and their order are the reference's bit for bit; the renormalised
  * weights can differ from it in the last bit or two (the softmax normaliser, which cancels in them up to rounding,
  * contains approximate terms for the experts that were not candidates).  0 = dense fp64 logits and exact weights. */
 /* MOE_OPT_TIMING_SKIP_STAGE (default 0): NOT in the library's default build, where it returns MOE_E_UNSUPPORTED; only a
@@ -331,7 +333,8 @@ int moe_forward_x16(moe_ctx* ctx, int layer, const float* x, const void* x16, in
 /* MOE_OPT_PAIR_TABLES (default 1): q4cp layers whose codebook is a table (not a*n + b), batches above
  * MOE_OPT_F32_DECODE_MAX_TOKENS and up to 32 tokens: the f32 kernels look two neighbouring weights up at a time in
  * 256-entry pair tables (one per code byte); 0 = one look-up per weight in the 16-entry table, as at a few tokens. */
-/* MOE_OPT_STREAM_GEMM (default 1): batches in which an expert has few pairs (33 tokens up to an average of 38 or 44 pairs) run the
+/* MOE_OPT_STREAM_GEMM (default 1): batches in which an expert has few pairs (33 tokens up to an average of 25 to 160 pairs,
+ * by kind of layer) run the
  * routed experts' two GEMMs on tiles of 16 to 64 pairs with the weights streamed into registers; 0 = the 128-pair
  * kernels at every size.  The same f16 weights and f32 sums, in another order. */
 enum { MOE_OPT_INT_DECODE = 1, MOE_OPT_UNIQUE_MIN_TOKENS = 2, MOE_OPT_FUSED_COMBINE = 3, MOE_OPT_SHARED_ASIDE = 4,
