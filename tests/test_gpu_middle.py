@@ -249,7 +249,7 @@ def test_cost_of_tokens_the_selection_cannot_settle(capi, oracle, T):
     plain = route_and_compare(capi, oracle, hl, x, k)
     hl.bias = np.zeros(E, np.float32)
     hl.bias[17] = -np.inf
-    assert route_and_compare(capi, oracle, hl, x, k) <= 1.5 * plain + 0.02
+    assert route_and_compare(capi, oracle, hl, x, k) <= 1.5 * plain + 0.06
     hl.bias = None
     nan = x.copy()
     nan[T // 2, 3] = np.nan
