@@ -33,7 +33,7 @@
 // tile holds, so tiles should hold an expert's pairs as a rule, and larger ones cost LDS and registers.
 // Measured (512 experts, top-10, 3072 x 768, gate/up + down, us; in brackets the 128-pair kernels):
 //   130 tokens q4cp 270 + 137 (368 + 185)      48 table 208 + 110 (295 + 177)    515 Q4_K 356 + 176 (413 + 241)
-//   200 Q5_K / Q8_0 407 + 291 (501 + 471)     200 i4r 260 + 143 (338 + 190)      2048 q4cp 392 + 219 (437 + 238)
+//   200 Q5_K / Q8_0 407 + 291 (501 + 471)     200 i4r 260 + 143 (338 + 190)      2048 q4cp 371 + 209 (437 + 238)
 // The layer at other widths, us (128-pair kernels in brackets), 48 / 515 / 1200 tokens, d = 3072: mid 256 q4cp 162 / 258 / 331 (207 / 307 /
 // 361), Q5_K / Q8_0 240 / 351 / 450 (353 / 523 / 560); 512 q4cp 245 / 401 / 474 (312 / 491 / 549), table 272 / 434 / 535 (392 / 610 / 639),
 // Q4_K 257 / 428 / 513 (339 / 544 / 602), i4r 245 / 378 / 467 (318 / 478 / 542); 1024 q4cp 429 / 719 / 827 (520 / 851 / 942), table 471 /
@@ -62,8 +62,9 @@ constexpr int x_layout(int FMT) { return FMT == F_TAB ? 0 : FMT <= F_I4R ? 1 : 2
 
 constexpr int XROW = 512;  // bytes of a line of one pair row (256 f16)
 constexpr size_t LDS_MOST = 160 * 1024;  // of a CU
-// copies of a pair table: lanes eight apart share one; gate/up with 64 pairs: four, so that two blocks fit a CU's LDS
-constexpr int tab_copies(bool UP, int MFX) { return UP && MFX == 4 ? 4 : 8; }
+// copies of a pair table: lanes eight apart share one; with 64 pairs four (gate/up: so that two blocks fit a CU's LDS; down: for
+// the registers, 246 us with eight copies, 237 with four at 2048 tokens)
+constexpr int tab_copies(bool, int MFX) { return MFX == 4 ? 4 : 8; }
 
 struct SW {
   const uint8_t *w, *w_up, *sc, *sc_up;
@@ -296,6 +297,88 @@ __device__ __forceinline__ void line_mma(const Line<FMT> (&q)[F], const uint32_t
   }
 }
 
+// ---- half a line (128 columns) of F q4cp fragments ----
+// slopes and offsets of half E_'s scale
+template <int F>
+struct Deq {
+  half2v as[F][2], bs[F];
+};
+template <int FMT, int F, int E_>
+__device__ __forceinline__ Deq<F> make_deq(const uint32_t (&sw)[F], const Consts& C) {
+  static_assert(FMT == F_DN || FMT == F_AFF || FMT == F_TAB, "");
+  Deq<F> D;
+#pragma unroll
+  for (int f = 0; f < F; f++) {
+    const half2v s2 = h2(__builtin_amdgcn_perm(sw[f], sw[f], E_ ? 0x03020302u : 0x01000100u));
+    if (FMT == F_TAB) {
+      D.as[f][0] = s2;
+    } else {
+      const float s = (float)s2.x;
+      D.as[f][0] = both(C.cb_a[f] * s);
+      D.bs[f] = both(C.cb_b[f] * s);
+      D.as[f][1] = FMT == F_DN ? D.as[f][0] * both(0.0625f) : D.as[f][0];
+    }
+  }
+  return D;
+}
+__device__ __forceinline__ uint32_t word(const uint4& q, int s) { return s == 0 ? q.x : s == 1 ? q.y : s == 2 ? q.z : q.w; }
+
+// acc[f][mf] += half line E_ of fragment f x the line's activations (line_mma's arguments and its sums, in its order).
+// A step's MFMAs run while the next step's operands are made: every (step, 16 pairs) is an item of F MFMAs, one activation
+// operand is read two items ahead, and the next step's weights are dequantised in equal parts next to the step's items.
+// The fences keep that order: left alone the compiler reads every activation operand into the same four registers and
+// waits a trip through LDS for each, and puts a step's dequantisation into one clump (a SIMD takes eight 16x16x32 MFMAs and 32
+// vector operations in 199 cycles side by side, in 219 clump behind clump).
+template <int FMT, int F, int MF, int XP, int TABC, int E_>
+__device__ __forceinline__ void half_mma(const uint4 (&c)[F], const Deq<F>& D, const Consts& C, const uint8_t* xb, const uint32_t* xa,
+                                         floatx4 (&acc)[F][MF]) {
+  constexpr int N = 4 * MF, AHEAD = 2;
+  half8 xf[AHEAD + 1];
+  auto ldx = [&](int t) { xf[t % (AHEAD + 1)] = *(const half8*)(xb + xa[t / MF] + E_ * 256 + 16 * (t % MF) * XP); };
+  H8 a[2][F];
+  uint32_t lut[4 * F];
+  auto look = [&](int s) {  // table codebooks: the two weights of every code byte before scaling
+#pragma unroll
+    for (int u = 0; u < 4 * F; u++)
+      lut[u] = *(const uint32_t*)(C.tabs + (((word(c[u >> 2], s) >> (8 * (u & 3))) & 0xffu) * (4u * TABC) + C.tabo[u >> 2]));
+  };
+  auto unit = [&](int s, int u) {  // a pair of step s's weights (line_mma's forms)
+    const int f = u >> 2, b = u & 3, i = b & 1;
+    H8& o = a[s & 1][f];
+    if constexpr (FMT == F_TAB) {
+      o.h[b] = h2(lut[u]) * D.as[f][0];
+    } else {
+      const uint32_t w = word(c[f], s), n = (b & 2 ? w >> 8 : w) & (i ? 0x00f000f0u : 0x000f000fu);
+      if constexpr (FMT == F_DN) o.h[b] = h2(n) * D.as[f][i] + D.bs[f];
+      else o.h[b] = (h2(n | (i ? 0x54005400u : 0x64006400u)) - both(i ? 64.f : 1024.f)) * D.as[f][i] + D.bs[f];
+    }
+  };
+#pragma unroll
+  for (int t = 0; t < AHEAD; t++) ldx(t);
+  if constexpr (FMT == F_TAB) look(0);
+#pragma unroll
+  for (int u = 0; u < 4 * F; u++) unit(0, u);
+#pragma unroll
+  for (int t = 0; t < N; t++) {
+    const int st = t / MF, mf = t % MF;
+    if constexpr (FMT == F_TAB) {
+      if (mf == 0 && st < 3) look(st + 1);
+    }
+    if (t + AHEAD < N) ldx(t + AHEAD);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int f = 0; f < F; f++) {
+      acc[f][mf] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[st & 1][f].v, xf[t % (AHEAD + 1)], acc[f][mf], 0, 0, 0);
+      if (st < 3) {
+        const int slot = F * mf + f;
+#pragma unroll
+        for (int u = slot * 4 / MF; u < (slot + 1) * 4 / MF; u++) unit(st + 1, u);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 // Scales of four lines of a row (64 bytes, i4r: 16) from line `first` on: lane group i fetches line first + i's, the exchange
 // below then hands every lane one word per line with its own two scales.  (Past the row's end: one address for all lanes.)
 template <int FMT>
@@ -360,24 +443,44 @@ __device__ __forceinline__ Consts make_consts(const SW& L, int pexp, uint8_t* ta
   return C;
 }
 
-// this lane's operand address of step q: 16-byte chunk 16 e + 4 g + q of pair row n, XORed with the row against bank conflicts
-// (Q8_0: lane group g walks its run of 64 columns, chunks 8 g + w)
+// Where a pair row's line has its 16-byte chunk c (16 e + 4 g + q: lane group g's step q of half e; Q8_0: 8 g + q) in LDS: the
+// bits of q above those of g, the low four XORed with the row.  A 128-bit read goes through the 64 banks sixteen lanes at
+// a time, lanes 0-3, 12-15 and 20-27 first: rows 4-11 come from the next lane group there, so a group bit may not meet the
+// rows' bits 2 and 3 (with chunks in order, g at bit 2, every read took twice as long).
+template <int FMT>
+__device__ __forceinline__ int x_slot(int c, int row) {
+  const int lo = FMT == F_Q80 ? ((c & 7) << 1) | ((c >> 3) & 1) : ((c & 3) << 2) | ((c >> 2) & 3);
+  return (c & 16) | (lo ^ (row & 15));
+}
+// this lane's operand address of step q of pair row n
 template <int FMT, int XP>
 __device__ __forceinline__ void x_addrs(int n, int g, uint32_t (&xa)[8]) {
 #pragma unroll
-  for (int q = 0; q < 8; q++) xa[q] = (uint32_t)(n * XP + ((((FMT == F_Q80 ? 8 : 4) * g + q) ^ n) << 4));
+  for (int q = 0; q < 8; q++) xa[q] = (uint32_t)(n * XP + (x_slot<FMT>((FMT == F_Q80 ? 8 : 4) * g + q, n) << 4));
 }
 
 // ---- gate/up ----
+// HALVES (64 pairs of q4cp codes): the codes go through registers in half lines, the next line's activations in two parts, and
+// half_mma orders the rest.  Else whole lines, one ahead of the line worked on, in the compiler's order.  What either is
+// bound by is traffic first: 16.6 M cache lines for the 10.6 M that 2048 tokens' gate/up rows and scales have (q4cp; rows are
+// visited a line, their scales four lines at a time, and what a visit leaves of a cache line is gone from L2 before the
+// next), 345 us of 386 at the 6.15 TB/s that plain loads reach; half lines need 15.2 M.  us of the launch, whole lines and
+// halves: 2048 tokens q4cp 386 371, table 483 432; but 515 q4cp (32 pairs) 312 320, 1500 Q4_K 404 425, 2048 i4r 401 406.
+// Tried beside it: lines that begin where the cache lines do (rows rotated by half a line: no fewer cache lines, +20 us),
+// a row's scales all at once (registers: spills at 64 pairs), non-temporal loads (21 M cache lines), 32 gate and 32 up rows to
+// a wave with two waves per SIMD (half the LDS reads, +12 us), and x in registers with the waves of a block splitting K, which
+// reads 9.8 M cache lines for 9.75 M at 130 tokens but leaves two waves per SIMD whose arithmetic does not hide (280 us for 268).
 // (Straight code of two lines, where K is known to be whole pairs of lines, gave the compiler room to move loads and operands
 // further and cost 20 us of 390 at 64 pairs (spills: up to 150): the branches around half and last lines stay.)
+constexpr bool up_halves(int FMT, int MFX) { return MFX == 4 && FMT <= F_TAB; }
 template <int FMT, int MFX, int MF, bool ROT, int NW>
 __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const moe_tile tile, int nb, const __half* __restrict__ x,
                                         const int* __restrict__ tokidx, __half* __restrict__ out, int M, int K, int pexp,
                                         const moe_hscale& hs, moe_cmag cmag, const moe_rotv& rot) {
   constexpr int LAYOUT = x_layout(FMT), LB = line_bytes(FMT), NT = 64 * NW, UPR = 16 * NW;
   constexpr int XBUF = MFX * 16 * XROW;
-  constexpr int DB = 2;  // lines in registers: one ahead of the line worked on
+  constexpr bool HALVES = up_halves(FMT, MFX);
+  constexpr int DB = HALVES ? 1 : 2;  // lines of codes in registers
   float* const rowscale = (float*)(smem + 2 * XBUF);
   uint8_t* const tabs = smem + 2 * XBUF + 256;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -397,13 +500,21 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
     sb[f] = scale_plane(FMT) ? (f ? L.sc_up : L.sc) + first * (size_t)L.sstride : nullptr;
   }
   const uint32_t wo = (uint32_t)r * RB, so = (uint32_t)r * (uint32_t)L.sstride;
-  Line<FMT> ln[DB][2];
+  Line<FMT> ln[HALVES ? 1 : DB][2];
+  uint4 cd[HALVES ? DB : 1][2][2];  // line, half, fragment
+  // (past the last line: one address for all lanes instead of a branch around the load)
   auto load = [&](Line<FMT>(&q)[2], int i) {
 #pragma unroll
     for (int f = 0; f < 2; f++) {
-      const bool past = i >= nline;  // (wave-uniform; one address for all lanes instead of a branch around the load)
+      const bool past = i >= nline;
       load_line<FMT>(q[f], wb[f] + (past ? (size_t)0 : (size_t)i * LB), past ? 0u : wo, past ? 0 : g, tail && i >= nline - 1);
     }
+  };
+  auto load_half = [&](uint4(&q)[2], int i, int E) {
+    const bool past = i >= nline;
+    const size_t at = past ? (size_t)0 : (size_t)i * LB + (E && !(tail && i == nline - 1) ? 64 : 0);
+#pragma unroll
+    for (int f = 0; f < 2; f++) q[f] = *(const uint4*)(wb[f] + at + (past ? 0u : wo + 16u * (uint32_t)g));
   };
   // ---- the pipeline's first requests: weights before the tile's row indices are needed ----
   Raw<FMT> raw[2];
@@ -413,11 +524,19 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
     for (int f = 0; f < 2; f++) raw[f] = load_scales<FMT>(sb[f], so, 0, g, L.sstride);
   }
 #pragma unroll
-  for (int b = 0; b < DB; b++) load(ln[b], b);
-  // ---- activations: thread = 16-byte piece tid % 32 of pair rows tid / 32 + (NT / 32) l ----
+  for (int b = 0; b < DB; b++) {
+    if constexpr (HALVES) {
+      load_half(cd[b][0], b, 0);
+      load_half(cd[b][1], b, 1);
+    } else {
+      load(ln[b], b);
+    }
+  }
+  // ---- activations: thread = 16-byte chunk tid % 32 of pair rows tid / 32 + (NT / 32) l ----
   // (rows past the tile's pairs repeat its first one: no branch around a load, and the lines are in L1)
   constexpr int XL = MF * 16 * 32 / NT, XS = NT / 32;  // loads per thread and line, rows per load
-  static_assert(XL >= 1 && XL <= 4, "named registers below");
+  constexpr int XH = HALVES ? (XL + 1) / 2 : XL;       // loads of a part of the line
+  static_assert(XL >= 1 && XL * NT == MF * 16 * 32 && XH <= 4, "whole loads, named registers below");
   const int xc = tid & 31, xt = tid >> 5;
   uint32_t xr[XL];  // (32-bit byte offsets: moe_launch_stream)
 #pragma unroll
@@ -428,27 +547,35 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
     if (xc == 0) rowscale[m] = hs.xms ? moe_hid_scale(cmag, hs.xms[row]) : 1.f;
   }
   uint4 xv0, xv1, xv2, xv3;  // (named: an array here ends up in scratch memory)
-  auto fetch_x = [&](int i) {
+  auto fetch_x = [&](int i, auto part) {
+    constexpr int h = XH * decltype(part)::value;
     i = i < nline ? i : nline - 1;
     const bool half = tail && i == nline - 1;
     const uint8_t* const xb = (const uint8_t*)x + 512 * (size_t)i;
     const uint32_t back = half && xc >= 16 ? 256u : 0u;
-    xv0 = *(const uint4*)(xb + (xr[0] - back));
-    if constexpr (XL > 1) xv1 = *(const uint4*)(xb + (xr[1] - back));
-    if constexpr (XL > 2) xv2 = *(const uint4*)(xb + (xr[2] - back));
-    if constexpr (XL > 3) xv3 = *(const uint4*)(xb + (xr[3] - back));
+    if constexpr (h < XL) xv0 = *(const uint4*)(xb + (xr[h] - back));
+    if constexpr (XH > 1 && h + 1 < XL) xv1 = *(const uint4*)(xb + (xr[h + 1] - back));
+    if constexpr (XH > 2 && h + 2 < XL) xv2 = *(const uint4*)(xb + (xr[h + 2] - back));
+    if constexpr (XH > 3 && h + 3 < XL) xv3 = *(const uint4*)(xb + (xr[h + 3] - back));
   };
-  auto put_x = [&](int buf) {
+  auto put_x = [&](int buf, auto part) {
+    constexpr int h = XH * decltype(part)::value;
     auto put = [&](int l, const uint4& v) {
       const int m = XS * l + xt;
-      *(uint4*)(smem + buf * XBUF + m * XROW + ((xc ^ (m & 15)) << 4)) = v;
+      *(uint4*)(smem + buf * XBUF + m * XROW + (x_slot<FMT>(xc, m) << 4)) = v;
     };
-    put(0, xv0);
-    if constexpr (XL > 1) put(1, xv1);
-    if constexpr (XL > 2) put(2, xv2);
-    if constexpr (XL > 3) put(3, xv3);
+    if constexpr (h < XL) put(h, xv0);
+    if constexpr (XH > 1 && h + 1 < XL) put(h + 1, xv1);
+    if constexpr (XH > 2 && h + 2 < XL) put(h + 2, xv2);
+    if constexpr (XH > 3 && h + 3 < XL) put(h + 3, xv3);
   };
-  fetch_x(0);
+  constexpr std::integral_constant<int, 0> P0{};
+  constexpr std::integral_constant<int, 1> P1{};
+  fetch_x(0, P0);
+  if constexpr (HALVES) {
+    put_x(0, P0);
+    fetch_x(0, P1);
+  }
   float oscale;
   const Consts C = make_consts<FMT, true, NT, tab_copies(true, MFX)>(L, pexp, tabs, tid, oscale);
   uint32_t xa[8];
@@ -458,20 +585,46 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
   for (int f = 0; f < 2; f++)
 #pragma unroll
     for (int mf = 0; mf < MF; mf++) acc[f][mf] = floatx4{0.f, 0.f, 0.f, 0.f};
-  put_x(0);
+  if constexpr (HALVES) put_x(0, P1);
+  else put_x(0, P0);
 
   // stage V (mod 4): line i
   auto stage = [&](auto vc, int i) {
-    constexpr int V = decltype(vc)::value, B = V & 1;
+    constexpr int V = decltype(vc)::value, B = V & 1, S = V % DB;
     moe_lds_barrier();  // this line's activations are in LDS; the other buffer has been read
-    fetch_x(i + 1);
-    const uint32_t sw[2] = {sq[0][V], sq[1][V]};
-    line_mma<FMT, 2, MF, XROW, tab_copies(true, MFX)>(ln[B], sw, C, 0, smem + B * XBUF, xa, tail && i == nline - 1, acc);
-    load(ln[B], i + DB);
-    put_x(B ^ 1);
+    fetch_x(i + 1, P0);
+    if constexpr (HALVES) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (V == 0) {
+#pragma unroll
+        for (int f = 0; f < 2; f++) take_scales<FMT>(raw[f], sq[f]);
+      }
+      const uint32_t sw[2] = {sq[0][V], sq[1][V]};
+      half_mma<FMT, 2, MF, XROW, tab_copies(true, MFX), 0>(cd[S][0], make_deq<FMT, 2, 0>(sw, C), C, smem + B * XBUF, xa, acc);
+      const Deq<2> d1 = make_deq<FMT, 2, 1>(sw, C);
+      put_x(B ^ 1, P0);
+      fetch_x(i + 1, P1);
+      load_half(cd[S][0], i + DB, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (!(tail && i == nline - 1))
+        half_mma<FMT, 2, MF, XROW, tab_copies(true, MFX), 1>(cd[S][1], d1, C, smem + B * XBUF, xa, acc);
+      __builtin_amdgcn_sched_barrier(0);
+      put_x(B ^ 1, P1);
+      load_half(cd[S][1], i + DB, 1);
+      if (V == 2) {  // (the next four lines')
+#pragma unroll
+        for (int f = 0; f < 2; f++) raw[f] = load_scales<FMT>(sb[f], so, i + 2, g, L.sstride);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    } else {
+      const uint32_t sw[2] = {sq[0][V], sq[1][V]};
+      line_mma<FMT, 2, MF, XROW, tab_copies(true, MFX)>(ln[S], sw, C, 0, smem + B * XBUF, xa, tail && i == nline - 1, acc);
+      load(ln[S], i + DB);
+      put_x(B ^ 1, P0);
+    }
   };
   for (int i = 0;; i += 4) {
-    if (scale_plane(FMT)) {
+    if (scale_plane(FMT) && !HALVES) {
 #pragma unroll
       for (int f = 0; f < 2; f++) {
         take_scales<FMT>(raw[f], sq[f]);
@@ -601,7 +754,7 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
       const int m = c >> 5, k = 32 * l + (c & 31);
       const int kk = 8 * k < K ? k : 0;  // (a half line's second half: never multiplied)
       const uint4 v = *(const uint4*)(x + (size_t)(tile.first + (m < tile.count ? m : 0)) * K + 8 * kk);
-      *(uint4*)(smem + l * XLINE + m * XP + (((c & 31) ^ (m & 15)) << 4)) = v;
+      *(uint4*)(smem + l * XLINE + m * XP + (x_slot<FMT>(c & 31, m) << 4)) = v;
     }
   float oscale;
   const Consts C = make_consts<FMT, false, NT, tab_copies(false, MFX)>(L, pexp, tabs, tid, oscale);
@@ -683,7 +836,7 @@ constexpr int up_waves(int FMT, int MFX) { return MFX == 4 || FMT == F_I4R ? 8 :
 // waves per SIMD asked for: what the registers of the lines in flight leave.  (Gate/up with Q5_K rounded once, 32 pairs: three; with
 // four 21 registers went to scratch inside the loop, 757 us for 702 at 1200 tokens of 2560 x 640.  A few kernels keep 1 .. 4
 // registers of their prologue in scratch until the epilogue, F_DN's down launch with 64 pairs an address once per pass:
-// gate/up F_DN and F_AFF with 64 pairs, F_Q5K with 32; down F_DN and F_TAB with 64.  F_Q5K with three waves has none and is no
+// gate/up F_Q5K with 32 pairs; down F_DN and F_TAB with 64.  F_Q5K with three waves has none and is no
 // faster: 808 us for 799 at 515 tokens, 1159 for 1152 at 1700.)
 constexpr int simd_waves(int FMT, bool UP, int MFX, int NW) {
   if (UP) return FMT == F_Q5E && MFX == 2 ? 3 : 4;
@@ -738,9 +891,13 @@ k_moe_stream(SW R, SW Sh, int n_experts, const __half* __restrict__ x, const int
     if constexpr (UP) up_tile<FMT, MFX, MF, FMT == F_I4R, NW>(smem, L, e, tile, nb, x, tokidx, out, M, K, pexp, hs, cmag, rot); \
     else dn_tile<FMT, MFX, MF, NW, LN, LN == DN_ONE>(smem, L, e, tile, nb, npass, x, out, M, K, pexp);                           \
   } while (0)
+  // (33 .. 48 pairs as three groups instead of four: 2048 tokens q4cp, 755 -> 720 us a layer)
   if (MFX == 1 || mfn <= 1) ST_GO(1);
   else if (MFX == 2 || mfn <= 2) ST_GO(2);
-  else if constexpr (MFX > 2) ST_GO(4);
+  else if constexpr (MFX > 2) {
+    if (mfn <= 3) ST_GO(3);
+    else ST_GO(4);
+  }
 #undef ST_GO
 }
 

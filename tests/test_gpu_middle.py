@@ -397,3 +397,25 @@ def test_the_callers_f16_copy_at_every_router(capi, fmt, T):
     y1 = m.forward_x16(0, x, capi.f32_to_f16(x, layout=m.x16_layout(0))).cpu().numpy()
     assert (y0 == y1).all() and (m.last_routing(T)[0].cpu().numpy() == i0).all()
     m.close()
+
+
+@pytest.mark.parametrize("pairs", [(33, 33), (32, 48), (49, 47), (48, 16), (63, 17), (64, 33), (65, 31)])
+@pytest.mark.parametrize("kind,kw,d,mid", [("q4cp", dict(fmt="q4cp"), 1152, 640), ("q4cp-affine", dict(fmt="q4cp"), 512, 256),
+                                           ("q4cp-table", dict(fmt="q4cp", codebook=TABLE), 640, 640), ("i4r", dict(fmt="i4r"), 512, 256),
+                                           ("q4k", dict(fmt="q4k"), 768, 256)])
+def test_tiles_of_33_to_64_pairs(capi, oracle, kind, kw, d, mid, pairs):
+    """Whole tiles and the edges of their 16-pair groups, lines of d that are four, one more, and half of one: two experts
+    that share the batch by the sign of one column.  All rows against the oracle, the grouped GEMM's tolerance."""
+    rng = np.random.default_rng(sum(pairs) + d)
+    hl = HostLayer(rng, d, mid, 4, 1, shared=False, bias=np.float32([0, 0, -90, -90]), **kw)
+    hl.router[:] = 0
+    hl.router[0, 0], hl.router[1, 0] = 40, -40
+    if kind == "q4cp-affine":  # no scaled dequantisation
+        hl.gate_up[64 + 8 * mid * d // 2:].view(np.float16).reshape(4, 2 * mid, -1)[:, 3, :] = np.float16(1e-5)
+    x = rng.standard_normal((sum(pairs), d), dtype=np.float32)
+    x[:, 0] = rng.permutation(np.repeat(np.float32([1, -1]), pairs))
+    yo, io, _ = oracle.moe_layer(hl.oracle_layer(), x)
+    assert np.bincount(io[:, 0]).tolist() == list(pairs)
+    y1, y0 = both_kernels(capi, hl, x)
+    assert max_abs_rel(y1, yo) <= 2e-3
+    assert (y1 != y0).any()  # (its own kernel)
