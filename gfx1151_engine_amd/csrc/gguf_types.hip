@@ -875,6 +875,8 @@ int moe_launch_gemm_gg(bool up, int type, const uint8_t* w, const uint8_t* w_up,
     return MOE_E_INVALID;
   if (!up && (m % 8 || !moe_aligned(out, 16))) return MOE_E_UNSUPPORTED;  // (down results leave as 16-byte pieces)
   if (max_tiles == 0) return MOE_OK;
+  if (moe_wide_takes(up, type, w, w_up, tsh, sh_w, sh_w_up, m, k, a_layout))
+    return moe_launch_wide(up, type, w, w_up, sh_w, sh_w_up, n_experts, x16, tokidx, tiles, ntiles, max_tiles, out, m, k, hs, st, a_layout);
   GgGemmW R{w, w_up, type}, S{sh_w ? sh_w : w, sh_w ? sh_w_up : w_up, sh_w ? tsh : type};
   const dim3 grid((unsigned)(up ? (m + 63) / 64 : (m + GG_BN - 1) / GG_BN), (unsigned)max_tiles);
   static moe_dev_once attr_once;

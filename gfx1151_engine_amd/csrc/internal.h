@@ -229,6 +229,12 @@ int moe_launch_gemm_gg(bool up, int type, const uint8_t* w, const uint8_t* w_up,
                        const uint8_t* sh_w_up, int n_experts, const __half* x16, const int* tokidx,
                        const moe_tile* tiles, const int* ntiles, int max_tiles, __half* out, int m, int k,
                        moe_hscale hs, hipStream_t st, int a_layout = 0);
+// Grouped GEMM for 8-bit codes (gemm_wide.hip): what moe_launch_gemm_gg hands over, its arguments checked
+bool moe_wide_takes(bool up, int type, const uint8_t* w, const uint8_t* w_up, int tsh, const uint8_t* sh_w, const uint8_t* sh_w_up,
+                    int m, int k, int a_layout);
+int moe_launch_wide(bool up, int type, const uint8_t* w, const uint8_t* w_up, const uint8_t* sh_w, const uint8_t* sh_w_up, int n_experts,
+                    const __half* x16, const int* tokidx, const moe_tile* tiles, const int* ntiles, int max_tiles, __half* out, int m,
+                    int k, moe_hscale hs, hipStream_t st, int a_layout);
 // shared expert stored densely (bf16 / f32 / q8g64; type codes of dense.h)
 bool moe_dense_shared_supported(int type, int d, int mid);
 int moe_launch_dense_shared_small(int type, const uint8_t* g, const uint8_t* u, const uint8_t* dn, const float* sh_logit,

@@ -419,3 +419,31 @@ def test_tiles_of_33_to_64_pairs(capi, oracle, kind, kw, d, mid, pairs):
     y1, y0 = both_kernels(capi, hl, x)
     assert max_abs_rel(y1, yo) <= 2e-3
     assert (y1 != y0).any()  # (its own kernel)
+
+
+# ---------- 8-bit codes from memory into registers (gemm_wide.hip): tiles of 1 .. 128 pairs, stages of 128 columns ----------
+@pytest.mark.parametrize("pairs", [(1, 32), (33, 64), (65, 96), (97, 128), (129, 31)])
+@pytest.mark.parametrize("kind,kw,d,mid", [
+    ("q5k-q8_0", dict(fmt="q4k", gg_types=(13, 8, 8)), 512, 768), ("q8_0", dict(fmt="q4k", gg_types=(8, 8, 8)), 384, 128),
+    ("q8_0-narrow", dict(fmt="q4k", gg_types=(8, 8, 8)), 640, 320), ("q4k-q8_0", dict(fmt="q4k", gg_types=(12, 8, 8)), 512, 640),
+    ("q8g32", dict(fmt="q4cp", shared_dense="q8g32"), 512, 640), ("q8g32-table", dict(fmt="q4cp", codebook=TABLE, shared_dense="q8g32"), 384, 256),
+    ("q8g32-i4r", dict(fmt="i4r", shared_dense="q8g32"), 256, 768)])
+def test_8_bit_codes_in_tiles_of_every_size(capi, oracle, kind, kw, d, mid, pairs):
+    """Two experts that share the batch by the sign of one column (the shared expert has all of it), groups of 32 pairs and
+    one more or less; columns of one stage to six, rows that are no whole blocks; widths that the general kernel keeps (320).
+    Tolerance: that of the grouped GEMMs."""
+    rng = np.random.default_rng(sum(pairs) + d)
+    hl = HostLayer(rng, d, mid, 4, 1, bias=np.float32([0, 0, -90, -90]), **kw)
+    hl.router[:] = 0
+    hl.router[0, 0], hl.router[1, 0] = 40, -40
+    T = sum(pairs)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    x[:, 0] = rng.permutation(np.repeat(np.float32([1, -1]), pairs))
+    yo, io, _ = oracle.moe_layer(hl.oracle_layer(), x)
+    assert np.bincount(io[:, 0]).tolist() == list(pairs)
+    m, dev = hl.to_gpu(max_tokens=T)
+    m.set_option(capi.OPT_STREAM_GEMM, 0)
+    y = m.forward(0, gpu(x)).cpu().numpy()
+    assert m.last_path() == capi.PATH_BATCH
+    m.close()
+    assert max_abs_rel(y, yo) <= 2e-3
