@@ -94,7 +94,8 @@ __device__ __forceinline__ void wide_tile(uint8_t* smem, const WideW& L, int e, 
         ld(0);
         ld(LX == 2 ? 2 : 1);
         if (G32)
-          last[S][f] = *(const uint32_t*)((UP && f ? L.w_up : L.w) + L.sc + ((fr * (size_t)(K >> 5) + 4 * s) * 2 + (lrow * (uint32_t)(K >> 5) + 2u * (uint32_t)h) * 2u));
+          last[S][f] = *(const uint32_t*)((UP && f ? L.w_up : L.w) + L.sc +
+                                          ((fr * (size_t)(K >> 5) + 4 * s) * 2 + (lrow * (uint32_t)(K >> 5) + 2u * (uint32_t)h) * 2u));
       } else {
         ld(LX == 2 ? 1 : 2);
         ld(3);
@@ -199,7 +200,8 @@ __device__ __forceinline__ void wide_tile(uint8_t* smem, const WideW& L, int e, 
       t = __builtin_amdgcn_perm(0x64646464u, code(S, f, blk, 2 * (w & 3) + (b >> 1)), b & 1 ? 0x04030402u : 0x04010400u);
     } else {  // columns 0, 4, 1, 5, 2, 6, 3, 7 of the chunk
       blk = w >> 2;
-      t = __builtin_amdgcn_perm(code(S, f, blk, 2 * (w & 3) + 1), code(S, f, blk, 2 * (w & 3)), 0x0c040c00u + 0x00010001u * (uint32_t)b) | 0x64006400u;
+      t = __builtin_amdgcn_perm(code(S, f, blk, 2 * (w & 3) + 1), code(S, f, blk, 2 * (w & 3)),
+                                0x0c040c00u + 0x00010001u * (uint32_t)b) | 0x64006400u;
     }
     a[w & 1][f].h[b] = (h2(t) - k1152) * (blk ? sB[f] : sA[f]);
   };
@@ -228,7 +230,9 @@ __device__ __forceinline__ void wide_tile(uint8_t* smem, const WideW& L, int e, 
     moe_lds_barrier();  // this stage's activations are in LDS; the other buffer has been read
     fetch_x(nst + 1, P0);
     half8 xf[AHEAD + 1];
-    auto ldx = [&](int t) { xf[t % (AHEAD + 1)] = *(const half8*)(smem + (xa0 ^ (uint32_t)(t / MF << 4)) + (B * XBUF + 32 * (t % MF) * XROW)); };
+    auto ldx = [&](int t) {
+      xf[t % (AHEAD + 1)] = *(const half8*)(smem + (xa0 ^ (uint32_t)(t / MF << 4)) + (B * XBUF + 32 * (t % MF) * XROW));
+    };
 #pragma unroll
     for (int t = 0; t < AHEAD; t++) ldx(t);
 #pragma unroll
@@ -296,7 +300,7 @@ __device__ __forceinline__ void wide_tile(uint8_t* smem, const WideW& L, int e, 
 #pragma unroll
           for (int i = 0; i < 8; i++) {
             const float gv = acc[0][mf][8 * k + i], uv = acc[1][mf][8 * k + i];
-            v[i] = gv * __builtin_amdgcn_rcpf(1.f + __expf(-gv)) * uv * rs;
+            v[i] = gv / (1.f + __expf(-gv)) * uv * rs;
           }
           put8(8 * k, v);
         } else {
