@@ -683,19 +683,21 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
     if (!rotp->pre || !rotp->planes || !rotp->meta || d % 128 || !moe_aligned(rotp->pre, 16) || !moe_aligned(x, 16)) return MOE_E_INVALID;
     rot = *rotp;
   }
-  // The f64 matrix pipe kernel (d a multiple of 128, one weight format).  With the caller's scratch for
+  // The f64 matrix pipe kernel (d a multiple of 128).  With the caller's scratch for
   // partial tiles the columns are split over up to eight blocks per 16 rows and it serves 5..32 tokens;
   // without it one block per 16 rows leaves most CUs idle (38 us at 32 tokens), which only beats
-  // k_router_mid above 24 tokens.
-  const bool one_fmt = !Wx || (Wx->dtype == MOE_DT_BF16) == (W->dtype == MOE_DT_BF16);
+  // k_router_mid above 24 tokens.  A shared-expert gate row in the other format (checkpoints: a bf16 matrix, an f32 row)
+  // makes no difference to it: a lane loads its row in that row's own format.  With such a row, the router's
+  // launches (logits, top-k) with k_router_mid and with this, us: 5 tokens 25 and 20, 11 tokens 32 and 22, 20 tokens 40 and
+  // 25, 32 tokens 57 and 26.
   int KS = 1;
-  if (kpart && ktickets && one_fmt && P > 4 && E + 1 <= MOE_ROUTER_KSPLIT_ROWS)
+  if (kpart && ktickets && P > 4 && E + 1 <= MOE_ROUTER_KSPLIT_ROWS)
     for (int s = 8; s > 1; s >>= 1)
       if (d % (128 * s) == 0) {
         KS = s;
         break;
       }
-  const bool mfma_ok = (P > 24 || KS > 1) && d % 128 == 0 && one_fmt;
+  const bool mfma_ok = (P > 24 || KS > 1) && d % 128 == 0;
   if (P > 24 && !mfma_ok) {
     // more than 24 tokens per block cost the kernel its second wave per SIMD (accumulators):
     // two launches of at most 16 tokens read the router matrix twice (L2 / MALL) and are faster

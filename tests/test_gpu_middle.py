@@ -73,6 +73,36 @@ def test_router_and_gate_vector_of_two_types(capi, oracle, T):
     assert max_abs_rel(y, yo) <= 2e-3
 
 
+# The launches of 5 .. 32 tokens: a gate vector of the matrix's own type and one of the other type (off any alignment) meet in
+# the same kernel, so layers that differ in nothing but the type their equal values are stored in give equal results.
+@pytest.mark.parametrize("T,E,d", [(5, 512, 3072), (16, 33, 768), (17, 520, 2560), (24, 48, 128), (25, 33, 640), (32, 512, 3072)])
+def test_gate_vector_of_the_other_type(capi, oracle, T, E, d):
+    import torch
+    rng = np.random.default_rng(T)
+    hl = HostLayer(rng, d, 256, E, 5, router_dtype="bf16")
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    m, dev = hl.to_gpu(max_tokens=T)
+    bits = dev["router"].view(torch.bfloat16).reshape(E, d)
+    gate = dev["shsg"].reshape(-1).to(torch.bfloat16)
+    got = {}
+    for rt in (torch.bfloat16, torch.float32):
+        r = bits.to(rt).contiguous()
+        m.set_router(0, capi.wview(r, capi.BF16 if rt == torch.bfloat16 else capi.F32, E, d))
+        for gt in (torch.bfloat16, torch.float32):
+            room = torch.zeros(d + 8, dtype=gt, device="cuda")
+            room[1:1 + d] = gate
+            m.set_shared(0, *(capi.wview(dev[n], capi.Q4CP, a, b) for n, a, b in (("shg", 256, d), ("shu", 256, d), ("shd", d, 256))),
+                         capi.wview(room[1:], capi.BF16 if gt == torch.bfloat16 else capi.F32, 1, d))
+            got[rt, gt] = m.forward(0, gpu(x)).cpu()
+    ids = m.last_routing(T)[0].cpu().numpy()[:, :5]
+    m.close()
+    lo, io, _ = oracle.router(hl.oracle_layer().router, x, 5)
+    assert (ids == io[:, :5]).all()
+    ref = got[torch.float32, torch.float32]
+    for y in got.values():
+        assert torch.equal(y, ref)
+
+
 # ---------- the shared expert's gate vector may start at any element, whatever router a batch takes ----------
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 @pytest.mark.parametrize("T,candidates", [(1, 1), (4, 1), (6, 1), (20, 1), (32, 1), (40, 1), (256, 1), (300, 1), (40, 0), (300, 0)])
