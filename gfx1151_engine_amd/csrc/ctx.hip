@@ -726,8 +726,8 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
                          (!sh || L.sh_gguf_type == MOE_GGML_Q4_K) && moe_dec4k_supported(g.d, g.mid, nslots_d);
   // q4cp codebooks that are not affine (the reference converter's fixed table, trained tables): the same launch
   // structure with look-up arithmetic
-  // (the gate/up launch at every small-batch size -- 138 against 151 us at 20 tokens --, the down launch up to
-  //  lut_max tokens: 35 against 38 us at 4 tokens, but 135 against 91 at 20)
+  // (the gate/up launch at every small-batch size -- 104 against 151 us at 20 tokens --, the down launch up to
+  //  lut_max tokens: 35 us at 5 tokens; the other kernel 37 at 6, 39 at 8)
   const bool use_lut = L.has_q4cp && c->int_decode && !use_int && (!sh || L.sh_gguf_type == 0) &&
                        moe_dec_supported(g.d, g.mid, nslots_d) && moe_dec_gu_topk_supported(g.experts, g.topk);
   // the integer-dot kernels switched off: for a*n + b codebooks the same launches with f32 arithmetic (every weight a
@@ -749,8 +749,7 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
   // integer-dot kernels: the gate/up launch runs the softmax / top-k itself (one launch less on the
   // latency-bound path than a top-k kernel, no last-block ticket in the logits launch)
   // -- as long as its blocks run in one round: each repeats the selection, 3 .. 4 us, where a launch of its own costs 7.
-  // Two layers, us, in the gate/up launch and aside: look-up kernels (a block per CU) 112 and 101 at 2 tokens, 182 and 154
-  // at 4; GGUF mixes 84.7 and 84.4 at 2, 122 and 119 at 3, 153 and 148 at 4; Q4_K 83.6 and 85.3 at 3, 113 and 108 at 4; q4cp
+  // Two layers, us, in the gate/up launch and aside: look-up kernels 95.4 and 88.7 at 2 tokens; GGUF mixes 84.7 and 84.4 at 2, 122 and 119 at 3, 153 and 148 at 4; Q4_K 83.6 and 85.3 at 3, 113 and 108 at 4; q4cp
   // 73.7 and 76.4 at 3, 100 and 97 at 4
   const int topk_max = c->gu_topk_max >= 0 ? c->gu_topk_max : use_lut ? 1 : use_intgg ? 2 : use_f32a ? 4 : 3;
   const bool gu_topk = (((use_int && !use_uq) || ((use_int4k || use_intgg) && !use_uq_gg) || use_lut || use_f32a) && P <= topk_max) &&

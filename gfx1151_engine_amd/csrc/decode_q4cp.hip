@@ -99,11 +99,20 @@ struct DecW {  // one q4cp tensor's planes
 
 // ---- codebooks that are not a*n + b (the reference converter's fixed non-uniform table, trained tables): the same
 // kernels with a look-up instead of the integer dots, all in f32 (no quantised activations: the result differs
-// from the f32 GEMV kernels only by the order of the additions).  The 16 codebook entries lie in LDS 32 times
-// side by side (entry n, copy c at dword 32 n + c), so that lane l always reads bank l % 32: no conflicts,
-// whatever the codes are.  A weight costs one bit-field extract, one address operation, one LDS read and one
-// FMA; a lane keeps the 32 activations of the group it is working on in registers.
-constexpr int LUT_DW = 16 * 32;  // dwords per table (2 KB)
+// from the f32 GEMV kernels only by the order of the additions).  What bounds them up to about ten tokens is the vector
+// instructions of the look-ups, so these are few: the 16 entries lie in LDS 64 times side by side (entry n at byte
+// 256 n, a copy per lane: no conflicts, whatever the codes are) at a multiple of the table's size, so that an address is
+// bytes put together.  Two masks turn a code word's nibbles into bytes with the table's place in them, and a weight
+// costs one byte permute, one LDS read and one FMA, 2.4 vector instructions with its share of the masks (a bit-field extract
+// and an address operation per weight, 32 copies: 3).  One layer of 20 tokens, gate/up: 117 -> 104 us; a 256-entry table of
+// pairs (64 KB) reads at 6 TB/s there, 95, but gains 1 us at 2 tokens and does not fit beside the selection at 1.
+// A lane keeps the 32 activations of the group it is working on in registers.
+constexpr int LUT_BYTES = 16 * 256;
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+// LDS byte address: the first multiple of LUT_BYTES from p on
+__device__ __forceinline__ uint32_t lut_at(const void* p) {
+  return ((uint32_t)(uintptr_t)p + (LUT_BYTES - 1)) & ~(uint32_t)(LUT_BYTES - 1);
+}
 
 struct XF {  // one group's activations
   float v[32];
@@ -116,14 +125,14 @@ __device__ __forceinline__ void load_xf(XF& x, const float* src) {  // src: glob
     x.v[4 * i] = f.x; x.v[4 * i + 1] = f.y; x.v[4 * i + 2] = f.z; x.v[4 * i + 3] = f.w;
   }
 }
-// the block fills one table
-__device__ __forceinline__ void build_lut(float* lut, const float* __restrict__ cb) {
-  for (int i = threadIdx.x; i < LUT_DW; i += blockDim.x) lut[i] = cb[i >> 5];
+// piece i of a table (16 copies of an entry); 256 pieces
+__device__ __forceinline__ void lut_put(uint32_t lut, int i, float v) {
+  *(__attribute__((address_space(3))) floatx4*)(uintptr_t)(lut + 16u * (uint32_t)i) = floatx4{v, v, v, v};
 }
-// sum_k cb[n_k] * x_k over one group (16 code bytes, low nibble = the earlier element); lut_lane = table + (lane & 31)
-__device__ __forceinline__ float lut_dot(const uint4 cw, const XF& x, const float* lut_lane) {
+// sum_k cb[n_k] * x_k over one group (16 code bytes, low nibble = the earlier element); lut4 = the table's address >> 8 in
+// each byte, lane4 = 4 * lane
+__device__ __forceinline__ float lut_dot(const uint4 cw, const XF& x, uint32_t lut4, uint32_t lane4) {
   const uint32_t w[4] = {cw.x, cw.y, cw.z, cw.w};
-  const uint32_t base = (uint32_t)(uintptr_t)lut_lane;  // LDS byte address of this lane's copy of entry 0
   float a0 = 0.f, a1 = 0.f;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
@@ -131,19 +140,15 @@ __device__ __forceinline__ float lut_dot(const uint4 cw, const XF& x, const floa
     // addresses of a whole launch's look-ups ahead of the first one and spills hundreds of registers)
     uint32_t wi = w[i];
     asm volatile("" : "+v"(wi));
+    const uint32_t lo = (wi & 0x0f0f0f0fu) | lut4, hi = ((wi >> 4) & 0x0f0f0f0fu) | lut4;
 #pragma unroll
-    for (int j = 0; j < 8; j += 2) {
-      // entry n of this lane's copy: base + 128 n, two instructions (left to itself the compiler takes three:
-      // shift, mask, add)
-      uint32_t n_lo, n_hi, a_lo, a_hi;
-      asm("v_bfe_u32 %0, %1, %2, 4" : "=v"(n_lo) : "v"(wi), "n"(4 * j));
-      asm("v_bfe_u32 %0, %1, %2, 4" : "=v"(n_hi) : "v"(wi), "n"(4 * j + 4));
-      asm("v_lshl_add_u32 %0, %1, 7, %2" : "=v"(a_lo) : "v"(n_lo), "v"(base));
-      asm("v_lshl_add_u32 %0, %1, 7, %2" : "=v"(a_hi) : "v"(n_hi), "v"(base));
+    for (int j = 0; j < 4; j++) {
+      const uint32_t sel = 0x0c0c0000u | (uint32_t)(4 + j) << 8;
+      const uint32_t a_lo = __builtin_amdgcn_perm(lo, lane4, sel), a_hi = __builtin_amdgcn_perm(hi, lane4, sel);
       const float t0 = *(const __attribute__((address_space(3))) float*)(uintptr_t)a_lo;
       const float t1 = *(const __attribute__((address_space(3))) float*)(uintptr_t)a_hi;
-      a0 = fmaf(t0, x.v[8 * i + j], a0);
-      a1 = fmaf(t1, x.v[8 * i + j + 1], a1);
+      a0 = fmaf(t0, x.v[8 * i + 2 * j], a0);
+      a1 = fmaf(t1, x.v[8 * i + 2 * j + 1], a1);
     }
     if (i & 1) __builtin_amdgcn_sched_barrier(0);  // sixteen look-ups in flight at a time, not a whole row's
   }
@@ -181,9 +186,9 @@ __device__ __forceinline__ float xf_sum(const XF& x) {
 }
 // MODE 1: the look-up (any codebook); MODE 2: cb[n] = a n + b0 in f32, sx = the sum of the group's activations
 template <int MODE>
-__device__ __forceinline__ float f32_dot(const uint4 cw, const XF& x, const float* lut_lane, float a, float b0, float sx) {
+__device__ __forceinline__ float f32_dot(const uint4 cw, const XF& x, uint32_t lut4, float a, float b0, float sx) {
   if (MODE == 2) return fmaf(a, aff_dot(cw, x), b0 * sx);
-  return lut_dot(cw, x, lut_lane);
+  return lut_dot(cw, x, lut4, 4u * (threadIdx.x & 63));
 }
 
 struct GuArgs2 {
@@ -210,12 +215,16 @@ struct GuArgs2 {
 // ids and weights in every block; cheaper than a last-block ticket in the router launch plus a
 // dependent load of the ids here) and block (0, 0, token) writes ids / weights out for the down
 // kernel.  The shared expert's blocks skip it and have the CU to themselves meanwhile.
-// LUT = 1 (not with UQ): table look-up arithmetic (above) for any codebook; xf32 = the tokens' activations [P][d],
-// dynamic LDS = two tables (gate rows', up rows') and the token's d activations, hid goes out as f32 only.
+// LUT = 1 (not with UQ): table look-up arithmetic (above) for any codebook; blocks of 16 rows and 256 threads; xf32 = the
+// tokens' activations [P][d], dynamic LDS = the token's d activations and two tables (gate rows', up rows'), hid goes out as
+// f32 only.
 // LUT = 2: the same data flow with f32 arithmetic for codebooks a*n + b (no tables).
 constexpr int GU2_ROWS = 32;
+// (LUT = 1: four waves, 16 rows.  A block is tens of thousands of vector instructions there, and one token's 264 blocks of
+// eight waves leave the CUs that get a second one with twice the work: four layers 129 -> 119 us)
+constexpr int gu2_threads(int lut) { return lut == 1 ? 256 : 512; }
 template <bool UQ, int NPL, int LUT>
-__global__ void __launch_bounds__(512, 4) k_dec_gu(GuArgs2 A, const uint32_t* __restrict__ xplanes,
+__global__ void __launch_bounds__(gu2_threads(LUT), 4) k_dec_gu(GuArgs2 A, const uint32_t* __restrict__ xplanes,
                                                 const float2* __restrict__ xmeta,
                                                 const int* __restrict__ ids, int id_stride, int kpt, int d,
                                                 int mid, uint32_t* __restrict__ hplanes,
@@ -224,8 +233,9 @@ __global__ void __launch_bounds__(512, 4) k_dec_gu(GuArgs2 A, const uint32_t* __
                                                 const int* __restrict__ tokidx, int n_experts,
                                                 const float* __restrict__ logits, int* __restrict__ ids_out,
                                                 float* __restrict__ ws_out, const float* __restrict__ xf32, moe_rfix RF) {
+  constexpr int NT = gu2_threads(LUT), ROWS = NT / 16;
   extern __shared__ float lutmem[];
-  __shared__ float gs[GU2_ROWS], us[GU2_ROWS];
+  __shared__ float gs[ROWS], us[ROWS];
   __shared__ uint32_t pk[QV4_GROUP_DW];
   __shared__ int sel_ids[64];
   __shared__ float sel_ws[64];
@@ -236,7 +246,7 @@ __global__ void __launch_bounds__(512, 4) k_dec_gu(GuArgs2 A, const uint32_t* __
     // one block of the extra grid row: the exact softmax / top-k (ids, renormalised weights) for the down
     // launch, next to the blocks that stream the weights and only need the ids
     if (blockIdx.x == 0) {
-      select_certain<NPL ? NPL : 8, 512>(logits + (size_t)blockIdx.z * n_experts, RF, (int)blockIdx.z, sel_ids, sel_ws, n_experts, kpt, true);
+      select_certain<NPL ? NPL : 8, NT>(logits + (size_t)blockIdx.z * n_experts, RF, (int)blockIdx.z, sel_ids, sel_ws, n_experts, kpt, true);
       __syncthreads();
       if ((int)threadIdx.x < kpt) {
         ids_out[(size_t)blockIdx.z * id_stride + threadIdx.x] = sel_ids[threadIdx.x];
@@ -244,6 +254,30 @@ __global__ void __launch_bounds__(512, 4) k_dec_gu(GuArgs2 A, const uint32_t* __
       }
     }
     return;
+  }
+  // Look-up tables and the token's activations: requested here, next to the selection's loads, and put into LDS behind the
+  // weights' requests
+  const bool sh_blk = !UQ && s >= kpt;
+  const float* const cbg = sh_blk ? A.shg.cb : A.gu.cb;
+  const float* const cbu = sh_blk ? A.shu.cb : A.gu.cb;
+  const bool two_tabs = LUT == 1 && cbu != cbg;  // (block-uniform) the shared expert's up_proj is a tensor with a codebook of its own
+  constexpr int XL = (96 * 8 + NT - 1) / NT;  // (d <= 3072)
+  static_assert(XL <= 3 && (LUT != 1 || NT == 256), "a thread stages at most three pieces of x and one of a table");
+  float4 x0, x1, x2;
+  float cg0 = 0.f, cu0 = 0.f;
+  if (LUT) {
+    const float4* xr = (const float4*)(xf32 + (size_t)blockIdx.z * d);
+    auto ld = [&](int i) {
+      const int c = (int)threadIdx.x + NT * i;
+      return xr[c < d / 4 ? c : 0];
+    };
+    x0 = ld(0);
+    x1 = ld(1);
+    if (XL > 2) x2 = ld(2);
+    if (LUT == 1) {
+      cg0 = cbg[threadIdx.x >> 4];
+      cu0 = cbu[threadIdx.x >> 4];
+    }
   }
   bool shared;
   if (UQ) {
@@ -259,39 +293,24 @@ __global__ void __launch_bounds__(512, 4) k_dec_gu(GuArgs2 A, const uint32_t* __
       // the ids by logit order (no exps, no sums); the exact selection only when two of the best logits
       // are too close for that to be certain
       const float* lg = logits + (size_t)blockIdx.z * n_experts;
-      if (!select_certain<NPL ? NPL : 8, 512>(lg, RF, (int)blockIdx.z, sel_ids, sel_ws, n_experts, kpt, false)) __syncthreads();
+      if (!select_certain<NPL ? NPL : 8, NT>(lg, RF, (int)blockIdx.z, sel_ids, sel_ws, n_experts, kpt, false)) __syncthreads();
       e = sel_ids[s];
     }
   } else {
     shared = s >= kpt;
     e = shared ? 0 : ids[(size_t)blockIdx.z * id_stride + s];
   }
+  const DecW Wg = shared ? A.shg : A.gu;  // block-uniform choice, by value
+  const DecW Wu = shared ? A.shu : A.gu;
   // the expert number is the same in every lane: as a scalar, the row and byte offsets that follow from it are scalar
   // arithmetic instead of 64-bit products per lane (quarter-rate instructions between the selection and the first load)
   e = __builtin_amdgcn_readfirstlane(e);
-  const DecW Wg = shared ? A.shg : A.gu;  // block-uniform choice, by value
-  const DecW Wu = shared ? A.shu : A.gu;
-  const float *lutg = lutmem + (lane & 31), *lutu = lutg;
-  if (LUT) {
-    if (LUT == 1) {
-      build_lut(lutmem, Wg.cb);
-      if (Wu.cb != Wg.cb) {  // (block-uniform) the shared expert's up_proj is a tensor with a codebook of its own
-        build_lut(lutmem + LUT_DW, Wu.cb);
-        lutu += LUT_DW;
-      }
-    }
-    // the token's activations, staged once per block: a lane fetches a group's 32 values when it starts on it.
-    // A group's 128 bytes lie at a pitch of 144: lanes read different groups 16 bytes at a time, and at a pitch of
-    // 128 every lane of such a read would sit on the same four banks (measured: 6.4 times the LDS time of this pitch).
-    const float4* xr = (const float4*)(xf32 + (size_t)blockIdx.z * d);
-    for (int i = threadIdx.x; i < d / 4; i += blockDim.x)
-      ((float4*)(lutmem + (LUT == 1 ? 2 * LUT_DW : 0)))[(i >> 3) * (XF_PITCH / 4) + (i & 7)] = xr[i];
-    __syncthreads();
-  }
-  const float* xs = lutmem + (LUT == 1 ? 2 * LUT_DW : 0);
+  const uint32_t lut_g = lut_at(lutmem + d / 32 * XF_PITCH), lut_u = lut_g + (two_tabs ? LUT_BYTES : 0);
+  const uint32_t lutg = (lut_g >> 8) * 0x01010101u, lutu = (lut_u >> 8) * 0x01010101u;
+  const float* xs = lutmem;
   const uint64_t grow0 = shared ? 0 : (uint64_t)e * 2 * mid;
   const uint64_t urow0 = shared ? 0 : (uint64_t)e * 2 * mid + mid;
-  const int r0 = blockIdx.x * GU2_ROWS + 4 * wv;  // first of this wave's 4 gate rows
+  const int r0 = blockIdx.x * ROWS + 4 * wv;  // first of this wave's 4 gate rows
 
   // Branch-free loads: a lane whose group lies past the row reads group 0 instead and gets a zero
   // scale.  (Loads inside divergent branches make the compiler wait for each of them where it is
@@ -330,6 +349,23 @@ __global__ void __launch_bounds__(512, 4) k_dec_gu(GuArgs2 A, const uint32_t* __
     st[p] = *(const __half*)(s0 + trow * W.ss + (gB >> W.gsh) * 2);
   }
   __builtin_amdgcn_sched_barrier(0);  // every load above is issued before the first dot product
+  if (LUT) {
+    // A group's 128 bytes lie at a pitch of 144: lanes read different groups 16 bytes at a time, and at a pitch of
+    // 128 every lane of such a read would sit on the same four banks (measured: 6.4 times the LDS time of this pitch).
+    auto put = [&](int i, const float4& v) {
+      const int c = (int)threadIdx.x + NT * i;
+      if (c < d / 4) ((float4*)lutmem)[(c >> 3) * (XF_PITCH / 4) + (c & 7)] = v;
+    };
+    put(0, x0);
+    put(1, x1);
+    if (XL > 2) put(2, x2);
+    if (LUT == 1) {
+      lut_put(lut_g, threadIdx.x, cg0);
+      if (two_tabs) lut_put(lut_u, threadIdx.x, cu0);
+    }
+    moe_lds_barrier();  // (the weights stay in flight)
+    __builtin_amdgcn_sched_barrier(0);
+  }
   for (int pi = 0; pi < npairs; pi++) {
   const int tok = UQ ? tokidx[first + pi] : (int)blockIdx.z;
   if (UQ) {
@@ -347,7 +383,7 @@ __global__ void __launch_bounds__(512, 4) k_dec_gu(GuArgs2 A, const uint32_t* __
     float sx = LUT == 2 ? xf_sum(xf) : 0.f;
 #pragma unroll
     for (int p = 0; p < 4; p++) {
-      const float* lt = p >= 2 ? lutu : lutg;
+      const uint32_t lt = p >= 2 ? lutu : lutg;
       const float a = p >= 2 ? ua : ga, b0 = p >= 2 ? u0 : g0;
       acc[2 * p] = __half2float(sa[p]) * mA * f32_dot<LUT>(ca[p], xf, lt, a, b0, sx);
       acc[2 * p + 1] = __half2float(sb[p]) * mA * f32_dot<LUT>(cb[p], xf, lt, a, b0, sx);
@@ -388,7 +424,7 @@ __global__ void __launch_bounds__(512, 4) k_dec_gu(GuArgs2 A, const uint32_t* __
   __syncthreads();
   if (raw) {
     if (threadIdx.x < 32) {
-      float* zr = A.zraw + ((size_t)tok * kpt + s) * 2 * mid + blockIdx.x * GU2_ROWS + threadIdx.x;
+      float* zr = A.zraw + ((size_t)tok * kpt + s) * 2 * mid + blockIdx.x * ROWS + threadIdx.x;
       zr[0] = gs[threadIdx.x];
       zr[mid] = us[threadIdx.x];
     }
@@ -396,11 +432,11 @@ __global__ void __launch_bounds__(512, 4) k_dec_gu(GuArgs2 A, const uint32_t* __
   }
   // SwiGLU on the block's 32 rows = one group of the down projection's input; quantise it
   if (wv == 0) {
-    const int j = lane & 31;
+    const int j = lane & (ROWS - 1);
     const float g = gs[j], u = us[j];
     const float hv = g / (1.f + expf(-g)) * u;
     const size_t slot = UQ ? (size_t)(first + pi) : (size_t)tok * nslots + s;
-    if (hid_f32 && lane < 32) hid_f32[slot * mid + blockIdx.x * GU2_ROWS + j] = hv;
+    if (hid_f32 && lane < ROWS) hid_f32[slot * mid + blockIdx.x * ROWS + j] = hv;
     if (LUT) return;  // (the down kernel of this arithmetic reads hid as f32)
     int p0, p1, p2, p3;
     float q, qsx;
@@ -459,11 +495,14 @@ __global__ void __launch_bounds__(512) k_dec_dn(DnArgs2 A, const uint32_t* __res
   const int G = mid / 32, half = lane >> 5;
   const int r0 = blockIdx.x * ROWS;
   const size_t rb = (size_t)mid / 2;
+  // (the tables' entries are requested first and written behind the weights' requests)
+  const float* const tcb = has_shared ? A.shd.cb : A.dn.cb;
+  float c0 = 0.f, c1 = 0.f;
   if (LUT == 1) {
-    build_lut(lutmem, A.dn.cb);
-    if (has_shared) build_lut(lutmem + LUT_DW, A.shd.cb);
-    __syncthreads();
+    c0 = A.dn.cb[threadIdx.x >> 4 & 15];
+    c1 = tcb[threadIdx.x >> 4 & 15];
   }
+  const uint32_t lut_r = lut_at(lutmem), lut_s = lut_r + LUT_BYTES;
   // combine weights of the token, fetched while the weight rows are in flight
   float wmine = 0.f;
   if ((int)threadIdx.x < nslots)
@@ -492,7 +531,7 @@ __global__ void __launch_bounds__(512) k_dec_dn(DnArgs2 A, const uint32_t* __res
     XF xh;
     if (LUT) load_xf(xh, hid_f32 + ((size_t)tok * nslots + s) * mid + (size_t)g * 32);
     else load_xg(x, hplanes, hmeta, (size_t)((tok * nslots + s) * G + g));
-    const float* lt = lutmem + (shared ? LUT_DW : 0) + (lane & 31);
+    const uint32_t lt = ((shared ? lut_s : lut_r) >> 8) * 0x01010101u;
     const float a = wcb[1] - wcb[0], b = fmaf(8.f, a, wcb[0]);
     const uint32_t row0 = e * (uint32_t)d + (uint32_t)r0;  // < experts * d: the launcher checks that it fits
     const uint8_t* cp = wcodes + (uint64_t)row0 * (uint32_t)rb + (uint32_t)g * 16;
@@ -512,6 +551,18 @@ __global__ void __launch_bounds__(512) k_dec_dn(DnArgs2 A, const uint32_t* __res
       }
     }
     __builtin_amdgcn_sched_barrier(0);  // every load is issued before the first dot product
+    if (LUT == 1) {
+      if (threadIdx.x < 256) {
+        lut_put(lut_r, threadIdx.x, c0);
+        lut_put(lut_s, threadIdx.x, c1);
+      }
+      for (int i = threadIdx.x + blockDim.x; i < 256; i += blockDim.x) {  // (blocks of fewer than four waves)
+        lut_put(lut_r, i, A.dn.cb[i >> 4]);
+        lut_put(lut_s, i, tcb[i >> 4]);
+      }
+      moe_lds_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+    }
     const float b0 = LUT == 2 ? wcb[0] : 0.f, sxh = LUT == 2 ? xf_sum(xh) : 0.f;
 #pragma unroll
     for (int r = 0; r < ROWS; r++) {
@@ -692,11 +743,12 @@ int moe_launch_dec_gu_lut(const moe_wview* gu, const moe_wview* sh_gate, const m
   A.gu = decw(gu);
   A.shg = decw(sh_gate);
   A.shu = decw(sh_up);
-  dim3 grid(mid / GU2_ROWS, kpt + (sh_gate ? 1 : 0) + (logits ? 1 : 0), P);
-  const int lds = (affine ? 0 : 2 * LUT_DW * 4) + d / 32 * XF_PITCH * 4;
-  if (lds > 64 * 1024) return MOE_E_UNSUPPORTED;
+  if (d > 3072) return MOE_E_UNSUPPORTED;
+  const int nt = gu2_threads(affine ? 2 : 1);
+  dim3 grid(mid / (nt / 16), kpt + (sh_gate ? 1 : 0) + (logits ? 1 : 0), P);
+  const int lds = (affine ? 0 : 3 * LUT_BYTES) + d / 32 * XF_PITCH * 4;  // (a table's worth for the tables' alignment)
 #define DEC_GU_F32(NPL, MODE)                                                                                          \
-  k_dec_gu<false, NPL, MODE><<<grid, 512, lds, st>>>(A, nullptr, nullptr, NPL ? nullptr : ids, id_stride, kpt, d, mid, nullptr, \
+  k_dec_gu<false, NPL, MODE><<<grid, nt, lds, st>>>(A, nullptr, nullptr, NPL ? nullptr : ids, id_stride, kpt, d, mid, nullptr, \
                                                      nullptr, hid_f32, nullptr, nullptr, nullptr, n_experts, logits, ids, ws, x, RFV)
   if (!logits) {
     if (affine) DEC_GU_F32(0, 2);
@@ -722,7 +774,7 @@ int moe_launch_dec_dn_lut(const moe_wview* dn, const moe_wview* sh_down, const f
   A.sh_logit = sh_logit;
   if (dn->rows > 0xffffffffull) return MOE_E_UNSUPPORTED;  // (row numbers are 32-bit in the kernel)
   const int nslots = kpt + (sh_down ? 1 : 0), bs = 64 * ((nslots + 1) / 2);
-  constexpr int lds = 2 * LUT_DW * 4;
+  constexpr int lds = 3 * LUT_BYTES;  // (one for the tables' alignment)
 #define DEC_DN_F32(ROWS, MODE)                                                                                          \
   k_dec_dn<ROWS, MODE><<<dim3(d / ROWS, P), bs, MODE == 1 ? lds : 0, st>>>(A, nullptr, nullptr, ids, ws, id_stride, kpt, d, mid, \
                                                                            out, out_stride, hid_f32)

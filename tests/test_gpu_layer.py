@@ -445,3 +445,24 @@ def test_small_batch_ids_when_summation_orders_disagree(oracle, fmt, T, int_deco
     assert (ids[:, :k] == io[:, :k]).all(), (ids[:, :k], io[:, :k])
     assert np.isfinite(y.cpu().numpy()).all()
     m.close()
+
+
+# ---------- few tokens, codebooks by look-up: where its blocks, tables and selection end ----------
+# (one slot: a down block of a single wave fills the tables in four turns; 1000 experts: the selection keeps twice the LDS;
+# a gate codebook and an up codebook of the shared expert: two tables; groups past the lanes of a row: d = 3072)
+@pytest.mark.parametrize("d,mid,E,k,shared,T", [(3072, 64, 20, 10, "own", 1), (32, 32, 8, 1, None, 1), (64, 32, 8, 1, "same", 3),
+                                                (2080, 96, 1000, 4, "own", 1), (1024, 992, 24, 14, "own", 2), (96, 64, 40, 7, None, 5),
+                                                (3072, 96, 530, 2, "same", 4), (2048, 32, 16, 3, "own", 6)])
+def test_look_up_blocks(oracle, d, mid, E, k, shared, T):
+    rng = np.random.default_rng(d + mid + T)
+    own = [np.sort(rng.uniform(-2, 2, 16)).astype(np.float32) for _ in range(3)]
+    hl = HostLayer(rng, d, mid, E, k, codebook=rng.uniform(-2, 2, 16).astype(np.float32), shared=shared is not None,
+                   shared_codebooks=own if shared == "own" else None, scale_std=0.05)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    yo, io, _ = oracle.moe_layer(hl.oracle_layer(), x)
+    m, dev = hl.to_gpu(max_tokens=T)
+    y = m.forward(0, gpu(x)).cpu().numpy()
+    ids = m.last_routing(T)[0].cpu().numpy()[:, :k]
+    m.close()
+    assert (ids == io[:, :k]).all()
+    assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= TOL_LUT
