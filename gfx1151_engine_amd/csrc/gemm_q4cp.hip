@@ -26,10 +26,12 @@
 //
 // Q5 (with Q4K): raw GGUF Q5_K super-blocks (176 B: the Q4_K header, 32 bytes qh, 128 code bytes; src/gguf.h:421-441):
 // the same stages with a fifth bit per code -- bit 2jj of qh byte l for the low nibble of code byte l in stage jj of the
-// super-block, bit 2jj+1 for the high nibble.  A lane fetches the 16 qh bytes of its half of each fragment row straight
-// into registers, together with the header's load one super-block ahead (through LDS they would take 8 KB more, one
-// block per CU instead of two), keeps them for the four stages and ORs the bit into the magic-number form of each code
-// pair (1024 + n and 64 + n stay exact for n < 32).
+// super-block, bit 2jj+1 for the high nibble.  The 32 qh bytes of a fragment's rows go straight into registers, one
+// super-block ahead with the header's load (through LDS they would take 8 KB more, one block per CU instead of two), two
+// neighbouring lanes to a row -- a lane each for its own row's half made 64 cache lines of every load -- and change lanes
+// when their super-block begins.  Codes become bytes of five bits, four at a time (a rotated qh word gives four fifth
+// bits), and then the magic-number form, pair by pair: 19 vector operations per code word, 22 with the bits ORed into
+// each pair.  Both, gate/up of one layer, us: 2000 tokens 650 -> 569, 4096 (skewed) 812 -> 709, 8192 1254 -> 1183.
 //
 // GS = 2: one scale per 128 columns instead of 32 (hgn v2 i4r experts, reference kI4R,
 // src/gpu/parts/27_kernels_moe_lut.inc:23-29): the four stages between two scale refreshes span exactly two scales,
@@ -188,11 +190,10 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
   const uint32_t* const ptab = (const uint32_t*)(smem + SMEM_BYTES);
   constexpr int KBLK = Q5 ? 176 : 144;   // bytes per super-block
   constexpr int KQS = Q5 ? 48 : 16;      // offset of the code bytes in it
-  // loads per row group behind the scale buffer's: the header's 16 bytes go to LDS; Q5_K adds two 8-byte register loads
-  // per weight fragment of the lane (its half of the row's 32 qh bytes; pairs of registers are easier to place than
-  // quadruples in a kernel this close to the register limit), issued in the same place so that the count of outstanding
+  // loads per row group behind the scale buffer's: the header's 16 bytes go to LDS; Q5_K adds a register load per weight
+  // fragment (the rows' 32 qh bytes, two lanes to a row), issued in the same place so that the count of outstanding
   // loads the waits rely on is the same for every wave
-  constexpr int SP = Q5 ? 1 + 2 * NF : 1;
+  constexpr int SP = Q5 ? 1 + NF : 1;
   static_assert(!Q5 || (WROWS / 64 + NW - 1) / NW == 1, "Q5_K: one row group per wave in the scale buffer");
   uint8_t* const A0 = smem;
   uint8_t* const W0 = smem + NBUF * A_BYTES;
@@ -248,7 +249,7 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
   // tensors and the activation rows stay below 4 GB): the registers that saves are what lets two blocks share a CU.
   // A wave's code and header rows lie in one half of the block's rows: gate rows for the first NW / 2 waves, up rows
   // for the others.
-  uint32_t a_off[Q5 ? A_LOADS : 1], w_off[Q5 ? W_LOADS : 1], s_off = 0, qh_off0 = 0, qh_off1 = 0;
+  uint32_t a_off[Q5 ? A_LOADS : 1], w_off[Q5 ? W_LOADS : 1], s_off = 0, qh_off = 0;
   const uint8_t* const wave_w = Q5 ? (wv >= NW / 2 ? L.w_up : L.w) : nullptr;
   auto wrow_off = [&](int lr) -> uint32_t {  // Q5_K gate/up: byte offset of LDS row lr's weight row in its tensor
     int r = nb * HALF + (lr & (HALF - 1));
@@ -285,13 +286,13 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
     else wrow[nf] = (nf / NH) * HALF + 32 * NH * wv + 32 * (nf % NH) + n;
   }
 
-  // Q5_K: the lane's half (code bytes 16 h .. 16 h + 15) of its fragment rows' 32 qh bytes, fetched into registers one
-  // super-block ahead
+  // Q5_K: the 32 qh bytes of the wave's fragment rows, fetched into registers one super-block ahead: lane 2 n + h holds what
+  // lane (n, h) needs.  Gate and up rows lie at the same offset from their wave-uniform bases.
   static_assert(!Q5 || (UP && NF == 2 && W_LOADS * 32 * (NW / 2) == HALF), "Q5_K: gate/up, a gate and an up fragment per wave");
-  uint2 qhn[4] = {{0u, 0u}, {0u, 0u}, {0u, 0u}, {0u, 0u}};
+  uint4 qhn[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
   if (Q5) {
-    qh_off0 = wrow_off(wrow[0]) + 16 + 16 * h;        // fragment 0: a gate row (base L.w)
-    qh_off1 = wrow_off(wrow[NF - 1]) + 16 + 16 * h;   // fragment 1: the matching up row (base L.w_up)
+    const int nq = lane >> 1, q0 = 64 * (wv >> 1) + 16 * (wv & 1) + (nq & 15) + 2 * (nq & 16);
+    qh_off = wrow_off(q0) + 16 + 16 * (lane & 1);  // of a gate row (base L.w); its up row lies L.up_off rows on in L.w_up
   }
   const int nstage = K / BK, ngroups = K / 32;
   constexpr int NLOADS = A_LOADS + W_LOADS;  // per stage (+S_LOADS scale loads on every fourth stage)
@@ -315,14 +316,10 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
       int g0 = 2 * s;
       g0 = g0 + 8 <= ngroups ? g0 : ngroups - 8;
       const size_t off = (Q4K ? (size_t)(s >> 2) * KBLK : (size_t)g0 * 2) + ps;
-      if (Q5 && pc == 1)  // this lane's 16 qh bytes of each fragment, into registers
-        qhn[0] = *(const uint2*)(L.w + (qh_off0 + (uint32_t)off));
+      if (Q5 && pc == 1)
+        qhn[0] = *(const uint4*)(L.w + (qh_off + (uint32_t)off));
       else if (Q5 && pc == 2)
-        qhn[1] = *(const uint2*)(L.w + (qh_off0 + (uint32_t)off + 8u));
-      else if (Q5 && pc == 3)
-        qhn[2] = *(const uint2*)(L.w_up + (qh_off1 + (uint32_t)off));
-      else if (Q5 && pc == 4)
-        qhn[3] = *(const uint2*)(L.w_up + (qh_off1 + (uint32_t)off + 8u));
+        qhn[1] = *(const uint4*)(L.w_up + (qh_off + ((uint32_t)L.up_off * (uint32_t)(K / 256 * KBLK) + (uint32_t)off)));
       else if (Q5)
         g2l16(wave_w + (s_off + (uint32_t)off), S0 + wv * 1024);
       else if (GS == 2)  // the two scales of stages s..s+3 (s % 4 == 0: columns 64 s .. 64 s + 255), [row][4 B]
@@ -399,6 +396,7 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
   float scf[NF];
   uint4 hdr[NF];
   uint4 qh4[Q5 ? NF : 1];  // Q5_K: this lane's 16 qh bytes of the current super-block (code bytes 16 h .. 16 h + 15)
+  uint32_t c5[Q5 ? NF : 1][2];  // Q5_K: the four low / high codes of a word, a byte each
   int q5sh = 0;            // Q5_K: 2 * (stage within the super-block) = the bit of a qh byte that belongs to the stage's low nibbles
   uint32_t k4w[Q4K ? NF : 1][6];  // Q4_K: the current super-block's scale / min fields and (d, d), (-dmin, -dmin)
   const uint8_t* Ab = A0;
@@ -428,7 +426,15 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
         if (Q4K) {
           if ((s & 3) == 0) {
             hdr[nf] = *(const uint4*)(Sb + wrow[nf] * 16);
-            if (Q5) qh4[nf] = uint4{qhn[2 * nf].x, qhn[2 * nf].y, qhn[2 * nf + 1].x, qhn[2 * nf + 1].y};  // (requested with the header's load, two stages ago)
+            if (Q5) {  // (requested with the header's load, two stages ago; `l` opaque: a register less over the K loop)
+              uint32_t l = lane;
+              asm volatile("" : "+v"(l));
+              const int from = (int)(8 * (l & 31) + 4 * (l >> 5));
+              qh4[nf].x = __builtin_amdgcn_ds_bpermute(from, qhn[nf].x);
+              qh4[nf].y = __builtin_amdgcn_ds_bpermute(from, qhn[nf].y);
+              qh4[nf].z = __builtin_amdgcn_ds_bpermute(from, qhn[nf].z);
+              qh4[nf].w = __builtin_amdgcn_ds_bpermute(from, qhn[nf].w);
+            }
           }
         } else {
           if (GS == 2) {
@@ -518,28 +524,26 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
       const uint32_t ws = part >= 2 ? w8 : w;
       if ((part & 1) == 0) dst[nf].h[part] = as_h2(ws & 0x000f000fu) * as2[nf][0] + bs2[nf][0];
       else dst[nf].h[part] = as_h2(ws & 0x00f000f0u) * as20[DN ? nf : 0] + bs2[nf][0];
+    } else if (Q5) {
+      // five-bit codes as bytes, the low nibbles' (parts 0, 2) and the high nibbles' (1, 3): parts 0 and 1 make them.  Bit
+      // 2 jj / 2 jj + 1 of each byte of the qh word goes to bit 4
+      if (part < 2) {
+        const uint32_t qw = q == 0 ? qh4[nf].x : q == 1 ? qh4[nf].y : q == 2 ? qh4[nf].z : qh4[nf].w;
+        const uint32_t fifth = __builtin_amdgcn_alignbit(qw, qw, (uint32_t)(q5sh + part - 4) & 31u) & 0x10101010u;
+        c5[nf][part] = ((part ? w >> 4 : w) & 0x0f0f0f0fu) | fifth;
+      }
+      const uint32_t t = __builtin_amdgcn_perm(0x64646464u, c5[nf][part & 1], part >= 2 ? 0x04030401u : 0x04020400u);
+      dst[nf].h[part] = (as_h2(t) - half2v{(_Float16)1024.f, (_Float16)1024.f}) * as2[nf][part & (NS - 1)] + bs2[nf][part & (NS - 1)];
     } else if (AFFINE) {
-      // (Q5_K shifts on the spot: it has no registers to spare for the shifted copies)
-      const uint32_t w8 = Q5 ? w >> 8 : q == 0 ? cw8[nf].x : q == 1 ? cw8[nf].y : q == 2 ? cw8[nf].z : cw8[nf].w;
+      const uint32_t w8 = q == 0 ? cw8[nf].x : q == 1 ? cw8[nf].y : q == 2 ? cw8[nf].z : cw8[nf].w;
       const uint32_t ws = part >= 2 ? w8 : w;
       const int ss = Q4K ? (part & 1) : 0;  // Q4_K: odd parts are the high nibbles = the stage's second sub-block
       uint32_t t;
-      // Q5_K: the qh word of these four code bytes; the pair's two fifth bits go to bit 4 / 20 (low nibbles: value 16
-      // on top of 1024 + n) or bit 8 / 24 (high nibbles: 16 on top of 64 + n, whose unit is bit 4)
-      uint32_t q5 = 0;
-      if (Q5) {
-        const uint32_t qw = q == 0 ? qh4[nf].x : q == 1 ? qh4[nf].y : q == 2 ? qh4[nf].z : qh4[nf].w;
-        // bytes 0, 2 (parts 0, 1) or 1, 3 (parts 2, 3); bit 2 jj (low nibbles) or 2 jj + 1 (high nibbles) of each
-        const int from = (part >= 2 ? 8 : 0) + q5sh + (part & 1), to = (part & 1) ? 8 : 4;
-        q5 = __builtin_amdgcn_alignbit(qw, qw, (uint32_t)(from - to) & 31u);  // rotate: the mask below drops the rest
-      }
       if ((part & 1) == 0) {
         asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t) : "v"(ws), "s"(0x000f000fu), "v"(0x64006400u));
-        if (Q5) asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t) : "v"(q5), "s"(0x00100010u), "v"(t));
         dst[nf].h[part] = (as_h2(t) - half2v{(_Float16)1024.f, (_Float16)1024.f}) * as2[nf][ss] + bs2[nf][ss];
       } else {
         asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t) : "v"(ws), "s"(0x00f000f0u), "v"(0x54005400u));
-        if (Q5) asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t) : "v"(q5), "s"(0x01000100u), "v"(t));
         dst[nf].h[part] = (as_h2(t) - half2v{(_Float16)64.f, (_Float16)64.f}) * as2[nf][ss] + bs2[nf][ss];
       }
     } else {

@@ -477,3 +477,18 @@ def test_8_bit_codes_in_tiles_of_every_size(capi, oracle, kind, kw, d, mid, pair
     assert m.last_path() == capi.PATH_BATCH
     m.close()
     assert max_abs_rel(y, yo) <= 2e-3
+
+
+# ---------- Q5_K in 128-pair tiles: rows that end inside a block, one super-block and several, tiles of every size ----------
+@pytest.mark.parametrize("d,mid,E,T", [(256, 320, 8, 40), (512, 192, 2, 150), (768, 64, 3, 200), (1024, 960, 4, 70)])
+def test_fifth_bits_of_part_filled_row_blocks(capi, oracle, d, mid, E, T):
+    rng = np.random.default_rng(d + mid)
+    hl = HostLayer(rng, d, mid, E, 2, fmt="q4k", gg_types=(13, 8, 8))
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    yo, io, _ = oracle.moe_layer(hl.oracle_layer(), x)
+    m, dev = hl.to_gpu(max_tokens=T)
+    m.set_option(capi.OPT_STREAM_GEMM, 0)
+    y = m.forward(0, gpu(x)).cpu().numpy()
+    assert m.last_path() == capi.PATH_BATCH
+    m.close()
+    assert max_abs_rel(y, yo) <= 2e-3
