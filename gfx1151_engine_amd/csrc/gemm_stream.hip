@@ -62,9 +62,11 @@ constexpr int x_layout(int FMT) { return FMT == F_TAB ? 0 : FMT <= F_I4R ? 1 : 2
 
 constexpr int XROW = 512;  // bytes of a line of one pair row (256 f16)
 constexpr size_t LDS_MOST = 160 * 1024;  // of a CU
-// copies of a pair table: lanes eight apart share one; with 64 pairs four (gate/up: so that two blocks fit a CU's LDS; down: for
-// the registers, 246 us with eight copies, 237 with four at 2048 tokens)
-constexpr int tab_copies(bool, int MFX) { return MFX == 4 ? 4 : 8; }
+// copies of a pair table: lanes eight (four) apart share one.  Gate/up: what lets four blocks of up to 32 pairs, two of 64, share
+// a CU's LDS with one table (515 tokens, 32 pairs, eight copies and four 346 -> 340 us; 2048, 64 pairs, four and eight
+// 324 -> 317; 16 pairs have room for sixteen, which take longer to fill than they save: 197 -> 208); down with 64 pairs: four
+// for the registers (246 us with eight copies, 237 with four at 2048 tokens)
+constexpr int tab_copies(bool UP, int MFX) { return MFX == 4 ? (UP ? 8 : 4) : UP && MFX == 2 ? 4 : 8; }
 
 struct SW {
   const uint8_t *w, *w_up, *sc, *sc_up;
@@ -410,8 +412,30 @@ __device__ __forceinline__ void take_scales(const Raw<FMT>& r, uint32_t (&sq)[4]
   sq[0] = c[0]; sq[1] = c[1]; sq[2] = d[0]; sq[3] = d[1];
 }
 
+// Pair tables: a thread's entry of each, as f32.  Requested before the first weights -- loads come back in order -- and written
+// (make_consts) when the activations are, four copies at a time.  Entries that were fetched one copy at a time behind the
+// weights kept a block from its first line: 48 tokens, gate/up 215 -> 196 and down 115 -> 105 us one by one, the layer, whose
+// launches overlap less, 353.5 -> 350.5; 300 tokens of 2560 x 640 418 -> 411, 515 599 -> 589.
+struct TabEntry {
+  float lo[2], hi[2];
+};
+template <int NT, int TABC>
+constexpr int tab_pieces() { return 64 * TABC > NT ? 64 * TABC / NT : 1; }  // 16-byte pieces (four copies) of a thread
+template <int NT, int TABC>
+__device__ __forceinline__ int tab_index(int tid) { return tid * tab_pieces<NT, TABC>() / (TABC / 4); }
 template <int FMT, bool UP, int NT, int TABC>
-__device__ __forceinline__ Consts make_consts(const SW& L, int pexp, uint8_t* tabs, int tid, float& oscale) {
+__device__ __forceinline__ TabEntry load_entry(const SW& L, int tid) {
+  TabEntry t{};
+  if (FMT == F_TAB) {
+    static_assert(tab_pieces<NT, TABC>() <= TABC / 4, "one entry per thread");
+    const int b = tab_index<NT, TABC>(tid) & 255;
+    t.lo[0] = L.cb[b & 15]; t.hi[0] = L.cb[b >> 4];
+    if (UP) { t.lo[1] = L.cb_up[b & 15]; t.hi[1] = L.cb_up[b >> 4]; }
+  }
+  return t;
+}
+template <int FMT, bool UP, int NT, int TABC>
+__device__ __forceinline__ Consts make_consts(const SW& L, int pexp, const TabEntry& te, uint8_t* tabs, int tid, float& oscale) {
   Consts C;
   C.g = (tid & 63) >> 4;
   C.selb = (C.g & 2) ? 0x04030402u : 0x04010400u;
@@ -432,10 +456,15 @@ __device__ __forceinline__ Consts make_consts(const SW& L, int pexp, uint8_t* ta
     // TABC copies side by side: lanes that differ in their low bits never meet on a bank (with one copy the look-ups of a
     // wave run into 3.5-way conflicts on average)
     const bool two = UP && L.cb_up != L.cb;
-    for (int i = tid; i < 256 * TABC; i += NT) {
-      const int b = i / TABC;
-      ((uint32_t*)tabs)[i] = u2(half2v{(_Float16)L.cb[b & 15], (_Float16)L.cb[b >> 4]});
-      if (two) ((uint32_t*)tabs)[256 * TABC + i] = u2(half2v{(_Float16)L.cb_up[b & 15], (_Float16)L.cb_up[b >> 4]});
+    constexpr int PT = tab_pieces<NT, TABC>();
+    if (64 * TABC >= NT || tid < 64 * TABC) {
+#pragma unroll
+      for (int t = 0; t < 2; t++) {
+        if (t && !two) break;
+        const uint32_t v = u2(half2v{(_Float16)te.lo[t], (_Float16)te.hi[t]});
+#pragma unroll
+        for (int i = 0; i < PT; i++) ((uint4*)tabs)[64 * TABC * t + PT * tid + i] = make_uint4(v, v, v, v);
+      }
     }
     C.tabo[0] = (uint32_t)(tid & (TABC - 1)) * 4u;
     C.tabo[1] = C.tabo[0] + (two ? 256u * TABC * 4u : 0u);
@@ -517,6 +546,8 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
     for (int f = 0; f < 2; f++) q[f] = *(const uint4*)(wb[f] + at + (past ? 0u : wo + 16u * (uint32_t)g));
   };
   // ---- the pipeline's first requests: weights before the tile's row indices are needed ----
+  TabEntry te;
+  if constexpr (MFX < 4) te = load_entry<FMT, true, NT, tab_copies(true, MFX)>(L, tid);
   Raw<FMT> raw[2];
   uint32_t sq[2][4];
   if (scale_plane(FMT)) {
@@ -577,7 +608,8 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
     fetch_x(0, P1);
   }
   float oscale;
-  const Consts C = make_consts<FMT, true, NT, tab_copies(true, MFX)>(L, pexp, tabs, tid, oscale);
+  if constexpr (MFX == 4) te = load_entry<FMT, true, NT, tab_copies(true, MFX)>(L, tid);  // (no registers for it any earlier)
+  const Consts C = make_consts<FMT, true, NT, tab_copies(true, MFX)>(L, pexp, te, tabs, tid, oscale);
   uint32_t xa[8];
   x_addrs<FMT, XROW>(n, g, xa);
   floatx4 acc[2][MF];
@@ -747,6 +779,8 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
       load_line<FMT>(ln[f][i], wb + ((size_t)row0 * RB + l * LB), (uint32_t)r * RB, g, tail && l == nline - 1);
     }
   };
+  TabEntry te;
+  if constexpr (MFX < 4) te = load_entry<FMT, false, NT, tab_copies(false, MFX)>(L, tid);
   load(0, 0, 0);
   load(1, 0, 0);
   for (int l = 0; l < nline; l++)
@@ -757,7 +791,8 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
       *(uint4*)(smem + l * XLINE + m * XP + (x_slot<FMT>(c & 31, m) << 4)) = v;
     }
   float oscale;
-  const Consts C = make_consts<FMT, false, NT, tab_copies(false, MFX)>(L, pexp, tabs, tid, oscale);
+  if constexpr (MFX == 4) te = load_entry<FMT, false, NT, tab_copies(false, MFX)>(L, tid);
+  const Consts C = make_consts<FMT, false, NT, tab_copies(false, MFX)>(L, pexp, te, tabs, tid, oscale);
   uint32_t xa[8];
   x_addrs<FMT, XP>(n, g, xa);
   moe_lds_barrier();
@@ -842,8 +877,9 @@ constexpr int simd_waves(int FMT, bool UP, int MFX, int NW) {
   if (UP) return FMT == F_Q5E && MFX == 2 ? 3 : 4;
   return NW == 16 ? 4 : FMT == F_Q80 || FMT == F_Q4K ? 3 : 4;
 }
-constexpr size_t smem_bytes(int FMT, bool UP, int MFX, int nline) {
-  const size_t tab = FMT == F_TAB ? (size_t)(UP ? 2 : 1) * 256 * tab_copies(UP, MFX) * 4 : 0;
+// tabs: pair tables (gate/up: two where an up tensor has a codebook of its own)
+constexpr size_t smem_bytes(int FMT, bool UP, int MFX, int nline, int tabs) {
+  const size_t tab = FMT == F_TAB ? (size_t)tabs * 256 * tab_copies(UP, MFX) * 4 : 0;
   return UP ? (size_t)2 * MFX * 16 * XROW + 256 + tab : (size_t)MFX * 16 * XROW * nline + tab;
 }
 
@@ -916,12 +952,12 @@ template <int FMT, bool UP, int MFX, int LN, int NW>
 int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* tokidx, const moe_tile* tiles,
            const int* ntiles, int max_tiles, __half* out, int m, int k, int split, moe_hscale hs, const moe_rotv* rot,
            hipStream_t st) {
-  const size_t lds = smem_bytes(FMT, UP, MFX, (k + 255) / 256);
+  const size_t lds = smem_bytes(FMT, UP, MFX, (k + 255) / 256, UP && (R.cb != R.cb_up || S.cb != S.cb_up) ? 2 : 1);
   static moe_dev_once once;
   int dev;
   if (moe_dev_pending(once, &dev)) {
     MOE_HIP(hipFuncSetAttribute((const void*)k_moe_stream<FMT, UP, MFX, LN, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(LN == 0 || LN == DN_ONE ? lds : LDS_MOST)));
+                                (int)(LN == 0 || LN == DN_ONE ? (UP ? smem_bytes(FMT, UP, MFX, 0, 2) : lds) : LDS_MOST)));
     moe_dev_done(once, dev);
   }
   int nblk = UP ? (m + 16 * NW - 1) / (16 * NW) : (m + 32 * NW - 1) / (32 * NW), npass = 1;
@@ -995,7 +1031,7 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
   if (k % 128 || ((q4(fmt) || q5(fmt) || fmt == F_I4R) && k % 256)) return MOE_E_UNSUPPORTED;
   // (down: groups of 32 rows, and a tile's hid rows in LDS)
   if (up && (uint64_t)x_rows * (uint64_t)k * 2 >= 1ull << 32) return MOE_E_UNSUPPORTED;  // (32-bit byte offsets into x)
-  if (up ? k < 256 : k < 128 || m % 32 || smem_bytes(fmt, false, cap / 16, (k + 255) / 256) > LDS_MOST) return MOE_E_UNSUPPORTED;
+  if (up ? k < 256 : k < 128 || m % 32 || smem_bytes(fmt, false, cap / 16, (k + 255) / 256, 1) > LDS_MOST) return MOE_E_UNSUPPORTED;
   if (up && (m % 16 || (fmt >= F_Q4K && m % 64) || (fmt == F_I4R && m % 128))) return MOE_E_UNSUPPORTED;
   if ((up && fmt == F_Q80) || (!up && (q5(fmt) || once_rounded(fmt))) || (cap > 32 && (q5(fmt) || fmt == F_Q80))) return MOE_E_UNSUPPORTED;
   if (fmt == F_I4R && up != (rot != nullptr)) return MOE_E_INVALID;
