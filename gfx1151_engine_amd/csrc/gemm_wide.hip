@@ -49,7 +49,9 @@ __device__ __forceinline__ uint32_t word(const uint4& q, int s) { return s == 0 
 
 constexpr int XROW = 256;              // bytes of a stage (128 columns) of one pair row
 constexpr int XBUF = 128 * XROW;       // of a tile
+constexpr int PROW = 128 + 16;         // down: bytes of a pair row in a wave's patch of results (64 f16 and padding)
 constexpr int SMEM = 2 * XBUF + 1024;  // + row scales and gate/up's row offsets
+constexpr int SMEM_DN = 2 * XBUF + 4 * 16 * PROW;
 
 // LX: order of the activations (moe_f32_to_f16's layouts); MF: groups of 32 pairs
 template <int FMT, bool UP, int LX, int MF>
@@ -281,36 +283,69 @@ __device__ __forceinline__ void wide_tile(uint8_t* smem, const WideW& L, int e, 
   auto finish = [&](int p) {
     const int r0 = (nb + p) * 4 * WR + WR * wv;
     if (r0 >= M) return;
+    auto pack8 = [&](const float* v) {
+      union { __half2 h[4]; uint4 q; } u;
+#pragma unroll
+      for (int k = 0; k < 4; k++) u.h[k] = __floats2half2_rn(v[2 * k], v[2 * k + 1]);
+      return u.q;
+    };
+    if constexpr (!UP) {
+      // sixteen pairs at a time through the wave's patch, so that eight lanes store a line: as 16-byte pieces of 64 lines the
+      // stores took the address unit 64 cycles each (8192 tokens 835 -> 814 us, 4096 543 -> 541)
+      uint32_t ln = lane;
+      asm volatile("" : "+v"(ln));  // (opaque: addresses made here instead of held through the stages)
+      uint8_t* const patch = smem + 2 * XBUF + wv * 16 * PROW;
+      const uint32_t wr = (ln & 15) * PROW + 64 * (ln >> 5), rd = (ln >> 3) * PROW + 16 * (ln & 7);
+      const uint32_t low = ln & 16;
+      int m = (int)(ln >> 3);
+      __half* o = out + (size_t)(tile.first + m) * M + r0 + 8 * (ln & 7);
+#pragma unroll
+      for (int mf = 0; mf < MF; mf++) {
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+          if ((low != 0) == (q != 0)) {
+#pragma unroll
+            for (int f = 0; f < 2; f++)
+#pragma unroll
+              for (int k = 0; k < 2; k++) {
+                float v[8];
+#pragma unroll
+                for (int i = 0; i < 8; i++) v[i] = acc[f][mf][8 * k + i];
+                *(uint4*)(patch + wr + 32 * f + 16 * k) = pack8(v);
+              }
+          }
+          __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the patch is the wave's own
+          __builtin_amdgcn_wave_barrier();
+#pragma unroll
+          for (int j = 0; j < 2; j++) {
+            const uint4 v = *(const uint4*)(patch + rd + 8 * j * PROW);
+            if (m < tile.count) *(uint4*)o = v;
+            m += 8;
+            o += 8 * (size_t)M;
+            asm volatile("" : "+v"(m), "+v"(o));
+          }
+          __builtin_amdgcn_s_waitcnt(0xC07F);
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int mf = 0; mf < MF; mf++) {
       const int m = 32 * mf + n;
       if (m >= tile.count) continue;
-      __half* const o = out + (size_t)(tile.first + m) * M + r0 + (UP ? 16 : 32) * h;
-      auto put8 = [&](int at, const float* v) {
-        union { __half2 h[4]; uint4 q; } u;
-#pragma unroll
-        for (int k = 0; k < 4; k++) u.h[k] = __floats2half2_rn(v[2 * k], v[2 * k + 1]);
-        *(uint4*)(o + at) = u.q;
-      };
+      __half* const o = out + (size_t)(tile.first + m) * M + r0 + 16 * h;
 #pragma unroll
       for (int k = 0; k < 2; k++) {
         float v[8];
-        if constexpr (UP) {
-          const float rs = rowscale[m];
+        const float rs = rowscale[m];
 #pragma unroll
-          for (int i = 0; i < 8; i++) {
-            const float gv = acc[0][mf][8 * k + i], uv = acc[1][mf][8 * k + i];
-            v[i] = gv / (1.f + __expf(-gv)) * uv * rs;
-          }
-          put8(8 * k, v);
-        } else {
-#pragma unroll
-          for (int f = 0; f < 2; f++) {
-#pragma unroll
-            for (int i = 0; i < 8; i++) v[i] = acc[f][mf][8 * k + i];
-            put8(16 * f + 8 * k, v);
-          }
+        for (int i = 0; i < 8; i++) {
+          const float gv = acc[0][mf][8 * k + i], uv = acc[1][mf][8 * k + i];
+          v[i] = gv / (1.f + __expf(-gv)) * uv * rs;
         }
+        *(uint4*)(o + 8 * k) = pack8(v);
       }
     }
   };
@@ -362,10 +397,11 @@ k_moe_wide(WideW R, WideW Sh, int n_experts, const __half* __restrict__ x, const
 template <int FMT, bool UP, int LX>
 int launch(const WideW& R, const WideW& S, int n_experts, const __half* x, const int* tokidx, const moe_tile* tiles, const int* ntiles,
            int max_tiles, __half* out, int m, int k, moe_hscale hs, hipStream_t st) {
+  constexpr int LDS = UP ? SMEM : SMEM_DN;
   static moe_dev_once once;
   int dev;
   if (moe_dev_pending(once, &dev)) {
-    MOE_HIP(hipFuncSetAttribute((const void*)k_moe_wide<FMT, UP, LX>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM));
+    MOE_HIP(hipFuncSetAttribute((const void*)k_moe_wide<FMT, UP, LX>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
     moe_dev_done(once, dev);
   }
   const int rows = UP ? 128 : 256;
@@ -376,7 +412,7 @@ int launch(const WideW& R, const WideW& S, int n_experts, const __half* x, const
       if (nblk % w == 0 && (int64_t)max_tiles * (nblk / w) >= 1024) npass = w;
   nblk /= npass;
   const int per = (max_tiles + 7) / 8;
-  k_moe_wide<FMT, UP, LX><<<(unsigned)(per * nblk * 8), 256, SMEM, st>>>(R, S, n_experts, x, tokidx, tiles, ntiles, out, m, k, nblk,
+  k_moe_wide<FMT, UP, LX><<<(unsigned)(per * nblk * 8), 256, LDS, st>>>(R, S, n_experts, x, tokidx, tiles, ntiles, out, m, k, nblk,
                                                                         npass, hs);
   MOE_LAUNCH_CHECK();
   return MOE_OK;
