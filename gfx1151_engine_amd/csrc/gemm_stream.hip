@@ -1002,7 +1002,10 @@ int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* 
 //   Q4_K                 933 840 / 943 913            956 941 / 994 957          1000 1013 / 1045 1046
 //   i4r                  869 794 / 886 854            887 869 / 928 894          956 953 / 994 995
 //   table                1047 930 / 1068 991          1069 1013 / 1102 1046      1134 1114 / 1187 1139
-//   Q5_K / Q8_0          29: 1268 1052 / 1296 1079    37: 1324 1270 / 1342 1204  44: 1344 1390 / 1384 1328
+//   Q5_K / Q8_0          25: 1039 964 / 1099 1032     29: 1061 1033 / -          33: 1091 1148 / 1139 1134
+// Q5_K / Q8_0 at even routing and other sizes: 3072 x 768 of 256 experts 30: 578 565, 34: 609 634; of 128 345 365, 351 374; of 64
+// 210 212, 211 246; 2048 x 768 of 512 29: 713 716, 33: 732 792.  With fewer experts neither has the blocks to fill the chip and the two are
+// level (16 experts, 512 x 768, 30, 34 and 38: 80 80, 79 81, 79 80): their line lies where it did with slower 128-pair kernels.
 // Q5_K and Q8_0 fragments leave no registers for 64 pairs (32-pair tiles above 22).  Rows of more than four lines of hid (mid >
 // 1024) leave no LDS for them: 32-pair tiles as well, level earlier (2048 x 1536, even: 23 q4cp 896 891, Q4_K 967 912; 29 q4cp
 // 923 967, Q4_K 996 1038, table 1149 1139, Q5_K / Q8_0 1519 1434; 37 table 1248 1409, Q5_K / Q8_0 1612 1741).
@@ -1013,7 +1016,7 @@ int moe_stream_tile_cap(int P, int k, int experts, int fmt_up, int fmt_dn, int m
   const float avg = (float)P * (float)k / (float)experts;
   const bool small = q5(fmt_up) || fmt_dn == F_Q80, lone = mid > 1024;
   const float line = once_rounded(fmt_up) ? ONCE_LINE
-                     : small              ? (lone ? 32.f : 38.f)
+                     : small              ? (lone ? 32.f : q5(fmt_up) && experts >= 64 ? 31.f : 38.f)
                      : fmt_up == F_TAB    ? (lone ? 29.f : 60.f)
                                           : (lone ? 25.f : 50.f);
   if (avg <= 10.f) return 16;

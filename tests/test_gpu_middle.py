@@ -415,6 +415,23 @@ def test_where_the_few_pair_tiles_end(capi, oracle, kind, kw, d, mid, last):
     assert (y1 == y0).all()
 
 
+@pytest.mark.parametrize("E,last", [(63, 38), (64, 31)])
+def test_where_the_few_pair_tiles_of_many_q5k_experts_end(capi, oracle, E, last):
+    """Q5_K / Q8_0: with experts that fill the chip in 128-pair tiles the line lies lower."""
+    k, d, mid = 3, 512, 256
+    T = last * E // k
+    rng = np.random.default_rng(E)
+    hl = HostLayer(rng, d, mid, E, k, fmt="q4k", gg_types=(13, 8, 8))
+    x = rng.standard_normal((T + 1, d), dtype=np.float32)
+    sel = np.r_[0, T // 2, T]
+    yo, _, _ = oracle.moe_layer(hl.oracle_layer(), x[sel])
+    y1, y0 = both_kernels(capi, hl, x[:T])
+    assert (y1 != y0).any()
+    y1, y0 = both_kernels(capi, hl, x)
+    assert (y1 == y0).all()
+    assert max_abs_rel(y1[sel], yo) <= 2e-3
+
+
 @pytest.mark.parametrize("fmt,T", [("q4cp", 40), ("q4cp", 300), ("q4k", 300), ("q4cp", 1100)])
 def test_the_callers_f16_copy_at_every_router(capi, fmt, T):
     """moe_forward_x16 against moe_forward, bit for bit; the router of 257 tokens and more makes its own copy all the same."""
