@@ -997,11 +997,14 @@ int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* 
 // and 22; 64-pair tiles at an average of 25 against 32-pair ones: 797 -> 779 us per layer (q4cp), 740 -> 738 (i4r).  Above, more
 // and more experts take a second tile and the 128-pair kernels draw level; the line lies where they do, for each kind of
 // layer with its own kernels, at even and at Zipf-skewed routing.  Layers, us, 128-pair kernels and these (3072 x 768):
-//   average pairs        44, even / skewed            49                         59
-//   q4cp                 867 791 / 885 840            888 871 / 920 875          932 935 / 982 950
-//   Q4_K                 933 840 / 943 913            956 941 / 994 957          1000 1013 / 1045 1046
-//   i4r                  869 794 / 886 854            887 869 / 928 894          956 953 / 994 995
-//   table                1047 930 / 1068 991          1069 1013 / 1102 1046      1134 1114 / 1187 1139
+//   average pairs        51, even / skewed            59                         62, table 66           66, table 70
+//   q4cp                 907 833 / 935 855            949 896 / 999 922          984 948 / 1047 951     1015 1033 / 1070 981
+//   Q4_K                 966 927 / 1012 950           1005 995 / 1062 982 (55)   1043 1053 / 1115 1058
+//   i4r                  921 862 / 940 884            967 938 / 1016 967         1001 1000 / 1068 1005  1042 1088 / 1089 1038
+//   table                                             1183 1063 / 1247 1080 (60) 1232 1204              1265 1272 / 1348 1215
+// That is of layers whose weights are many: d x mid x experts of 3 * 2^28, 2048 x 768 of 512 experts (62: 675 676; 2560 x 640, 62: q4cp 733
+// 716, 70: table 931 926).  With fewer the 128-pair kernels draw level earlier (3072 x 768 of 256 experts 59: i4r 531 535, 56: Q4_K 535
+// 544; of 64, 55: q4cp 176 190; 1024 x 768 of 512, 59: i4r 403 412), and the lines are where 16 experts have them.
 //   Q5_K / Q8_0          25: 1039 964 / 1099 1032     29: 1061 1033 / -          33: 1091 1148 / 1139 1134
 // Q5_K / Q8_0 at even routing and other sizes: 3072 x 768 of 256 experts 30: 578 565, 34: 609 634; of 128 345 365, 351 374; of 64
 // 210 212, 211 246; 2048 x 768 of 512 29: 713 716, 33: 732 792.  With fewer experts neither has the blocks to fill the chip and the two are
@@ -1012,13 +1015,13 @@ int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* 
 // Layers that go to the general kernel otherwise (F_Q4E, F_Q5E): as far as was measured (2560 x 640: 59 1979 1245 / 2153 1257; 160
 // 3888 2682 / 3480 2691; 2048 x 1152: 160 5146 4036 / 4570 4035).
 constexpr float ONCE_LINE = 160.f;
-int moe_stream_tile_cap(int P, int k, int experts, int fmt_up, int fmt_dn, int mid) {
+int moe_stream_tile_cap(int P, int k, int experts, int fmt_up, int fmt_dn, int d, int mid) {
   const float avg = (float)P * (float)k / (float)experts;
-  const bool small = q5(fmt_up) || fmt_dn == F_Q80, lone = mid > 1024;
+  const bool small = q5(fmt_up) || fmt_dn == F_Q80, lone = mid > 1024, big = (int64_t)d * mid * experts >= (int64_t)3 << 28;
   const float line = once_rounded(fmt_up) ? ONCE_LINE
                      : small              ? (lone ? 32.f : q5(fmt_up) && experts >= 64 ? 31.f : 38.f)
-                     : fmt_up == F_TAB    ? (lone ? 29.f : 60.f)
-                                          : (lone ? 25.f : 50.f);
+                     : fmt_up == F_TAB    ? (lone ? 29.f : big ? 70.f : 60.f)
+                                          : (lone ? 25.f : !big ? 50.f : fmt_up == F_DN || fmt_up == F_AFF ? 62.f : 60.f);
   if (avg <= 10.f) return 16;
   return avg > line ? 0 : small || lone || avg <= 22.f ? 32 : 64;
 }

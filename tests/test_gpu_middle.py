@@ -432,6 +432,28 @@ def test_where_the_few_pair_tiles_of_many_q5k_experts_end(capi, oracle, E, last)
     assert max_abs_rel(y1[sel], yo) <= 2e-3
 
 
+@pytest.mark.parametrize("fmt,codebook,last", [("q4cp", "zp8", 62), ("q4cp", "universal", 70), ("q4k", "zp8", 60), ("i4r", "zp8", 60)])
+def test_where_the_few_pair_tiles_of_many_weights_end(capi, fmt, codebook, last):
+    """512 experts of 2048 x 768: the lines of layers whose weights are many.  The two kernels' outputs are each within 6e-4 of
+    the exact ones in the 2-norm (test_few_pair_tiles_are_no_less_exact)."""
+    import torch
+    from gfx1151_engine_amd import workloads as W
+    d, mid, E, k = 2048, 768, 512, 10
+    T = last * E // k
+    L = W.DeviceLayer(5, d, mid, E, k, fmt, codebook=codebook)
+    m = capi.Moe(d, mid, E, k, max_tokens=T + 1)
+    L.register(m, 0)
+    x = torch.randn((T + 1, d), device="cuda", generator=torch.Generator(device="cuda").manual_seed(T))
+    for n, same in ((T, False), (T + 1, True)):
+        ys = []
+        for on in (1, 0):
+            m.set_option(capi.OPT_STREAM_GEMM, on)
+            ys.append(m.forward(0, x[:n].contiguous()).double())
+        assert torch.equal(ys[0], ys[1]) == same
+        assert float((ys[0] - ys[1]).norm() / ys[1].norm()) <= 1.2e-3
+    m.close()
+
+
 @pytest.mark.parametrize("fmt,T", [("q4cp", 40), ("q4cp", 300), ("q4k", 300), ("q4cp", 1100)])
 def test_the_callers_f16_copy_at_every_router(capi, fmt, T):
     """moe_forward_x16 against moe_forward, bit for bit; the router of 257 tokens and more makes its own copy all the same."""
