@@ -63,9 +63,9 @@ constexpr int x_layout(int FMT) { return FMT == F_TAB ? 0 : FMT <= F_I4R ? 1 : 2
 constexpr int XROW = 512;  // bytes of a line of one pair row (256 f16)
 constexpr size_t LDS_MOST = 160 * 1024;  // of a CU
 // copies of a pair table: lanes eight (four) apart share one.  Gate/up: what lets four blocks of up to 32 pairs, two of 64, share
-// a CU's LDS with one table (515 tokens, 32 pairs, eight copies and four 346 -> 340 us; 2048, 64 pairs, four and eight
-// 324 -> 317; 16 pairs have room for sixteen, which take longer to fill than they save: 197 -> 208); down with 64 pairs: four
-// for the registers (246 us with eight copies, 237 with four at 2048 tokens)
+// a CU's LDS, with two tables as well (smem_bytes; 515 tokens, 32 pairs, eight copies and four 346 -> 340 us; 2048, 64 pairs,
+// four and eight 324 -> 317; 16 pairs have room for sixteen, which take longer to fill than they save: 197 -> 208); down with
+// 64 pairs: four for the registers (246 us with eight copies, 237 with four at 2048 tokens)
 constexpr int tab_copies(bool UP, int MFX) { return MFX == 4 ? (UP ? 8 : 4) : UP && MFX == 2 ? 4 : 8; }
 
 struct SW {
@@ -502,16 +502,23 @@ __device__ __forceinline__ void x_addrs(int n, int g, uint32_t (&xa)[8]) {
 // (Straight code of two lines, where K is known to be whole pairs of lines, gave the compiler room to move loads and operands
 // further and cost 20 us of 390 at 64 pairs (spills: up to 150): the branches around half and last lines stay.)
 constexpr bool up_halves(int FMT, int MFX) { return MFX == 4 && FMT <= F_TAB; }
+// Bytes of LDS for the tile's row scales.  None beside two pair tables: those and the activations fill half of a CU's LDS (64
+// pairs) or a quarter (32) to the byte, so the epilogue reads the scales' sources again.  us of the layer, table codebook with a
+// shared expert of its own tables, 64 experts, top-8, with the scales behind them (one block fewer per CU) and without: 3072 x 768
+// 100 tokens (32 pairs) 128.3 126.6, 200 (64 pairs) 143.0 135.7, 256 146.4 140.7; 2560 x 640 200 123.5 116.2.  With one table there
+// is room, and reading again costs: 200 tokens without a shared expert 126.6 127.9
+constexpr size_t up_scales(int FMT, int tabs) { return FMT == F_TAB && tabs == 2 ? 0 : 256; }
 template <int FMT, int MFX, int MF, bool ROT, int NW>
 __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const moe_tile tile, int nb, const __half* __restrict__ x,
                                         const int* __restrict__ tokidx, __half* __restrict__ out, int M, int K, int pexp,
-                                        const moe_hscale& hs, moe_cmag cmag, const moe_rotv& rot) {
+                                        const moe_hscale& hs, moe_cmag cmag, const moe_rotv& rot, bool two_tabs) {
   constexpr int LAYOUT = x_layout(FMT), LB = line_bytes(FMT), NT = 64 * NW, UPR = 16 * NW;
   constexpr int XBUF = MFX * 16 * XROW;
   constexpr bool HALVES = up_halves(FMT, MFX);
   constexpr int DB = HALVES ? 1 : 2;  // lines of codes in registers
   float* const rowscale = (float*)(smem + 2 * XBUF);
-  uint8_t* const tabs = smem + 2 * XBUF + 256;
+  const bool scales = !(FMT == F_TAB && two_tabs);  // (up_scales)
+  uint8_t* const tabs = smem + 2 * XBUF + up_scales(FMT, scales ? 1 : 2);
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, g = lane >> 4;
   const uint32_t RB = row_bytes<FMT>(K);
@@ -590,7 +597,7 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
     const int m = XS * l + xt;
     const int row = xrow[l];
     xr[l] = ((uint32_t)row * (uint32_t)K + 8u * (uint32_t)xc) * 2u;
-    if (xc == 0) rowscale[m] = hs.xms ? moe_hid_scale(cmag, hs.xms[row]) : 1.f;
+    if (scales && xc == 0) rowscale[m] = hs.xms ? moe_hid_scale(cmag, hs.xms[row]) : 1.f;
   }
   uint4 xv0, xv1, xv2, xv3;  // (named: an array here ends up in scratch memory)
   auto fetch_x = [&](int i, auto part) {
@@ -741,11 +748,18 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
     }
   } else {
     const int col = nb * UPR + 16 * wv + 4 * g;
+    float rsv[MF];
+#pragma unroll
+    for (int mf = 0; mf < MF; mf++) {
+      const int m = 16 * mf + n;
+      if (scales) rsv[mf] = rowscale[m];
+      else rsv[mf] = hs.xms ? hs.xms[tokidx[tile.first + (m < tile.count ? m : 0)]] : 0.f;
+    }
 #pragma unroll
     for (int mf = 0; mf < MF; mf++) {
       const int m = 16 * mf + n;
       if (m < tile.count && col < M) {
-        const float rs = rowscale[m];
+        const float rs = scales ? rsv[mf] : hs.xms ? moe_hid_scale(cmag, rsv[mf]) : 1.f;
         float h4[4];
 #pragma unroll
         for (int r4 = 0; r4 < 4; r4++) {
@@ -895,8 +909,11 @@ constexpr int simd_waves(int FMT, bool UP, int MFX, int NW) {
 // tabs: pair tables (gate/up: two where an up tensor has a codebook of its own)
 constexpr size_t smem_bytes(int FMT, bool UP, int MFX, int nline, int tabs) {
   const size_t tab = FMT == F_TAB ? (size_t)tabs * 256 * tab_copies(UP, MFX) * 4 : 0;
-  return UP ? (size_t)2 * MFX * 16 * XROW + 256 + tab : (size_t)MFX * 16 * XROW * nline + tab;
+  return UP ? (size_t)2 * MFX * 16 * XROW + up_scales(FMT, tabs) + tab : (size_t)MFX * 16 * XROW * nline + tab;
 }
+// (gate/up keeps with two tables the blocks that a CU has with one)
+static_assert(2 * smem_bytes(F_TAB, true, 4, 0, 2) <= LDS_MOST && 4 * smem_bytes(F_TAB, true, 2, 0, 2) <= LDS_MOST &&
+              4 * smem_bytes(F_TAB, true, 1, 0, 2) <= LDS_MOST, "blocks per CU");
 
 // LN: lines of a piece (down)
 template <int FMT, bool UP, int MFX, int LN, int NW>
@@ -937,9 +954,10 @@ k_moe_stream(SW R, SW Sh, int n_experts, const __half* __restrict__ x, const int
   const int pexp = FMT == F_DN ? (int)L.pexp[e] : 0;
   const moe_cmag cmag = shared ? hs.c_shared : hs.c_routed;
   const int mfn = (tile.count + 15) >> 4;
+  const bool two_tabs = R.cb != R.cb_up || Sh.cb != Sh.cb_up;  // (launch)
 #define ST_GO(MF)                                                                                              \
   do {                                                                                                         \
-    if constexpr (UP) up_tile<FMT, MFX, MF, FMT == F_I4R, NW>(smem, L, e, tile, nb, x, tokidx, out, M, K, pexp, hs, cmag, rot); \
+    if constexpr (UP) up_tile<FMT, MFX, MF, FMT == F_I4R, NW>(smem, L, e, tile, nb, x, tokidx, out, M, K, pexp, hs, cmag, rot, two_tabs); \
     else dn_tile<FMT, MFX, MF, NW, LN, LN == DN_ONE>(smem, L, e, tile, nb, npass, x, out, M, K, pexp);                           \
   } while (0)
   // (33 .. 48 pairs as three groups instead of four: 2048 tokens q4cp, 755 -> 720 us a layer)

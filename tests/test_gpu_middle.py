@@ -490,6 +490,24 @@ def test_tiles_of_33_to_64_pairs(capi, oracle, kind, kw, d, mid, pairs):
     assert (y1 != y0).any()  # (its own kernel)
 
 
+@pytest.mark.parametrize("T", [40, 88, 152])
+@pytest.mark.parametrize("shared", ["its own tables", "the same values", "none"])
+def test_row_scales_beside_one_table_and_two(capi, oracle, shared, T):
+    """Table codebooks, tiles of 16, 32 and 64 pairs: with two pair tables the row scales of hid are read in the epilogue, with one
+    they wait in LDS.  Rows of a thousandth to three hundred times the usual size, so that a tile's scales differ; every row against
+    the oracle by its own size, the layer's tolerance."""
+    rng = np.random.default_rng(T)
+    kw = {"its own tables": dict(shared_codebooks=[TABLE, TABLE[::-1].copy(), TABLE * 0.5]), "the same values": {}, "none": dict(shared=False)}
+    hl = HostLayer(rng, 512, 384, 16, 4, fmt="q4cp", codebook=TABLE, **kw[shared])
+    x = rng.standard_normal((T, 512), dtype=np.float32) * np.float32(10) ** rng.uniform(-3, 2.5, (T, 1)).astype(np.float32)
+    yo, _, _ = oracle.moe_layer(hl.oracle_layer(), x)
+    m, dev = hl.to_gpu(max_tokens=T)
+    y = m.forward(0, gpu(x)).cpu().numpy()
+    assert m.last_path() == capi.PATH_BATCH
+    m.close()
+    assert (np.abs(y - yo).max(1) <= 2e-3 * np.abs(yo).max(1)).all()
+
+
 # ---------- 8-bit codes from memory into registers (gemm_wide.hip): tiles of 1 .. 128 pairs, stages of 128 columns ----------
 @pytest.mark.parametrize("pairs", [(1, 32), (33, 64), (65, 96), (97, 128), (129, 31)])
 @pytest.mark.parametrize("kind,kw,d,mid", [
