@@ -334,9 +334,7 @@ __host__ __device__ constexpr uint64_t ggu_row_bytes(int t, uint64_t k) {
 
 __device__ __forceinline__ int iq4_lookup4(uint32_t q, int shift) { return (int)moe_iq4_lookup4<0>(q, shift); }
 // rows in flight together: four (eight Q4_K rows of nine registers spill next to the kernel's other state and measured
-// 1.4 us slower per token than two batches of four).  In the launches below a row that has been multiplied makes place for
-// the one four on, so that a wave's loads never run dry; in two batches, each waited for, four layers of one token took
-// 120 us instead of 117, two layers of two tokens 88 instead of 84.5
+// 1.4 us slower per token than two batches of four)
 template <int T> constexpr int ggu_batch() { return 4; }
 
 template <int T>
@@ -501,24 +499,51 @@ __device__ __forceinline__ float ggu_dot(const GgU<T>& o, int jj, const XU& x) {
   }
 }
 
+// How a wave of the gate/up launch walks its eight rows: as a ring, in which a row that has been multiplied makes place for the one
+// four on, or as two batches of four, each waited for.  The ring keeps loads in flight all the time, and its fences keep the
+// compiler from interleaving two rows' arithmetic, which Q5_K's, Q8_0's and Q5_1's rows (the longest) need once there are
+// tokens enough to hide the loads: the layer at 3072 x 768, us, ring and batches, gate/up / down types, 8, 20 and 32 tokens Q8_0 /
+// Q8_0 136.4 134.8, 299.2 292.3, 462.9 451.2; Q5_K / Q8_0 118.3 117.8, 252.3 250.0, 387.0 382.4; Q5_1 / Q8_0 117.2 117.3, 250.3
+// 249.1, 382.7 380.7; Q5_K / Q5_K 107.2 106.0, 227.5 225.0, 355.9 353.2.
+// Q4_K and IQ4 rows are level or better in the ring (20 tokens, batches and ring: Q4_K 231.0 231.5, IQ4_NL 227.4 226.0, IQ4_XS
+// 232.1 231.5; 1 token, four layers: Q4_K 112.8 111.5); one and two tokens of any type are within 1 % either way (FEW).  Down rows are better in the ring for every type (ggu_dn_rows; 1 token, four
+// layers: Q5_K / Q8_0 117.5 115.6, Q4_K / Q8_0 111.5 107.9, Q8_0 132.5 129.6, Q5_1 112.4 111.4, IQ4_NL 115.4 114.9).
+template <int T, bool FEW>
+constexpr bool ggu_gu_ring() { return FEW || T == MOE_GGML_Q4_K || T == MOE_GGML_IQ4_NL || T == MOE_GGML_IQ4_XS; }
 // eight rows of one wave (gate/up launch: four gate rows and the matching up rows): acc[i] = wave sum of row i
-template <int T>
+template <int T, bool FEW>
 __device__ __forceinline__ void ggu_gu_rows(const uint8_t* gbase, const uint8_t* ubase, int r0, int d, int ul,
                                             float mlive, const XU& x, float (&acc)[8]) {
   constexpr int RB = ggu_batch<T>();
   const uint64_t rb = ggu_row_bytes(T, (uint64_t)d);
   const int jj = ul & 3;
-  GgU<T> u[RB];
-  auto fetch = [&](int i) { ggu_fetch<T>((i < 4 ? gbase : ubase) + (uint64_t)(r0 + (i & 3)) * rb, ul, u[i % RB]); };
+  if constexpr (ggu_gu_ring<T, FEW>()) {
+    GgU<T> u[RB];
+    auto fetch = [&](int i) { ggu_fetch<T>((i < 4 ? gbase : ubase) + (uint64_t)(r0 + (i & 3)) * rb, ul, u[i % RB]); };
 #pragma unroll
-  for (int i = 0; i < RB; i++) fetch(i);
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    acc[i] = sum64(ggu_dot<T>(u[i % RB], jj, x) * mlive);
-    __builtin_amdgcn_sched_barrier(0);  // rows are consumed in arrival order
-    if (i + RB < 8) fetch(i + RB);
+    for (int i = 0; i < RB; i++) fetch(i);
     __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      acc[i] = sum64(ggu_dot<T>(u[i % RB], jj, x) * mlive);
+      __builtin_amdgcn_sched_barrier(0);  // rows are consumed in arrival order
+      if (i + RB < 8) fetch(i + RB);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+#pragma unroll
+    for (int h = 0; h < 8; h += RB) {
+      GgU<T> u[RB];
+#pragma unroll
+      for (int i = 0; i < RB; i++)
+        ggu_fetch<T>(((i + h) < 4 ? gbase : ubase) + (uint64_t)(r0 + ((i + h) & 3)) * rb, ul, u[i]);
+      __builtin_amdgcn_sched_barrier(0);  // every load of the batch is issued before the first dot product
+#pragma unroll
+      for (int i = 0; i < RB; i++) {
+        acc[i + h] = sum64(ggu_dot<T>(u[i], jj, x) * mlive);
+        if (i & 1) __builtin_amdgcn_sched_barrier(0);  // rows are consumed in arrival order
+      }
+    }
   }
 }
 
@@ -586,7 +611,7 @@ __global__ void __launch_bounds__(512, 4) k_decgg_gu(GuGgArgs A, const uint32_t*
   XU x;
   load_xu(x, xplanes, xmeta, ((size_t)tok * U + ul) * 2);
   float acc[8];
-  GGU_SWITCH(t, ggu_gu_rows<T>(gbase, ubase, r0, d, ul, mlive, x, acc));
+  GGU_SWITCH(t, (ggu_gu_rows<T, (NPL > 0)>(gbase, ubase, r0, d, ul, mlive, x, acc)));
   if (lane == 0) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {

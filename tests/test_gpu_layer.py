@@ -263,6 +263,26 @@ def test_gguf_mixed_types(oracle, tgu, tdn, tsh, T):
     m.close()
 
 
+@pytest.mark.parametrize("tgu", [12, 13, 7, 8, 20, 23])
+def test_gguf_gate_up_rows_in_both_orders(oracle, tgu):
+    """Every gate/up type (the shared expert's as well) in the launch that selects the experts itself, whose waves take their rows
+    as a ring, and in the one that is given them, where longer rows go in two batches: the same sums, bit for bit."""
+    from gfx1151_engine_amd import capi
+    rng = np.random.default_rng(tgu)
+    T, d, mid = 5, 768, 256
+    hl = HostLayer(rng, d, mid, 12, 4, fmt="q4k", gg_types=(tgu, 8, tgu))
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    yo, _, _ = oracle.moe_layer(hl.oracle_layer(), x)
+    m, dev = hl.to_gpu(max_tokens=T)
+    ys = []
+    for most in (T, 0):
+        m.set_option(capi.OPT_GU_TOPK_MAX_TOKENS, most)
+        ys.append(m.forward(0, gpu(x)).cpu().numpy())
+    m.close()
+    assert (ys[0] == ys[1]).all()
+    assert max_abs_rel(ys[0], yo) <= TOL_INT_Q4K
+
+
 @pytest.mark.parametrize("share", [0.3, 1.0])
 def test_unique_expert_path(oracle, share):
     """MOE_OPT_UNIQUE_MIN_TOKENS: a verify-size batch through the expert-sorted pair lists (every distinct
