@@ -1020,9 +1020,16 @@ int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* 
 //   Q4_K                 966 927 / 1012 950           1005 995 / 1062 982 (55)   1043 1053 / 1115 1058
 //   i4r                  921 862 / 940 884            967 938 / 1016 967         1001 1000 / 1068 1005  1042 1088 / 1089 1038
 //   table                                             1183 1063 / 1247 1080 (60) 1232 1204              1265 1272 / 1348 1215
-// That is of layers whose weights are many: d x mid x experts of 3 * 2^28, 2048 x 768 of 512 experts (62: 675 676; 2560 x 640, 62: q4cp 733
-// 716, 70: table 931 926).  With fewer the 128-pair kernels draw level earlier (3072 x 768 of 256 experts 59: i4r 531 535, 56: Q4_K 535
-// 544; of 64, 55: q4cp 176 190; 1024 x 768 of 512, 59: i4r 403 412), and the lines are where 16 experts have them.
+// That is of layers whose weights are many.  With fewer the 128-pair kernels draw level earlier: a launch is then one or two rounds
+// of blocks, and a second tile of some experts is a round more.  d x mid x experts tells the layers apart better than either
+// width or the number of experts does.  q4cp, even / skewed, averages of 50, 56 and 62 (change against the 128-pair kernels, %):
+//   3072 x 768 of 384 (906 M)  -9 / -11, -8, 0 / -6      of 256 (604 M)  -7 / -8, -6, -3 / -7       of 128 (302 M)  -6 / -6, 0, +1 / -2
+//   4096 x 1024 of 128 (537 M) -6 / -9, -3, -1 / -4      2048 x 1024 of 256 (537 M) -3 / -4, -2, +2 / -3
+//   1024 x 512 of 1000 (524 M) -3 / -4, -3, 0 / -3       2048 x 768 of 256 (403 M)  0 / -4, 0, +2 / -4
+//   1024 x 768 of 512 (403 M)  0 / -5, +1, +3 / -1       3072 x 768 of 64 (151 M)   +9 / -1, +10, +15 / -3
+// (Q4_K and i4r 1 .. 2 % less throughout; table codebooks 2048 x 768 of 256 at 62 and 70 -3, 0, 3072 x 768 of 256 -3, +2.)  The
+// line between many and few lies between 403 and 524 M.
+constexpr int64_t MANY_WEIGHTS = (int64_t)7 << 26;
 //   Q5_K / Q8_0          25: 1039 964 / 1099 1032     29: 1061 1033 / -          33: 1091 1148 / 1139 1134
 // Q5_K / Q8_0 at even routing and other sizes: 3072 x 768 of 256 experts 30: 578 565, 34: 609 634; of 128 345 365, 351 374; of 64
 // 210 212, 211 246; 2048 x 768 of 512 29: 713 716, 33: 732 792.  With fewer experts neither has the blocks to fill the chip and the two are
@@ -1035,7 +1042,7 @@ int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* 
 constexpr float ONCE_LINE = 160.f;
 int moe_stream_tile_cap(int P, int k, int experts, int fmt_up, int fmt_dn, int d, int mid) {
   const float avg = (float)P * (float)k / (float)experts;
-  const bool small = q5(fmt_up) || fmt_dn == F_Q80, lone = mid > 1024, big = (int64_t)d * mid * experts >= (int64_t)3 << 28;
+  const bool small = q5(fmt_up) || fmt_dn == F_Q80, lone = mid > 1024, big = (int64_t)d * mid * experts >= MANY_WEIGHTS;
   const float line = once_rounded(fmt_up) ? ONCE_LINE
                      : small              ? (lone ? 32.f : q5(fmt_up) && experts >= 64 ? 31.f : 38.f)
                      : fmt_up == F_TAB    ? (lone ? 29.f : big ? 70.f : 60.f)

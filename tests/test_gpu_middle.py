@@ -454,6 +454,31 @@ def test_where_the_few_pair_tiles_of_many_weights_end(capi, fmt, codebook, last)
     m.close()
 
 
+def ends_at(capi, L, d, mid, E, k, T):
+    """T tokens are the largest batch of layer L on the few-pair tiles.  The two kernels' outputs are each within 6e-4 of the exact
+    ones in the 2-norm (test_few_pair_tiles_are_no_less_exact)."""
+    import torch
+    m = capi.Moe(d, mid, E, k, max_tokens=T + 1)
+    L.register(m, 0)
+    x = torch.randn((T + 1, d), device="cuda", generator=torch.Generator(device="cuda").manual_seed(T))
+    for n, same in ((T, False), (T + 1, True)):
+        ys = []
+        for on in (1, 0):
+            m.set_option(capi.OPT_STREAM_GEMM, on)
+            ys.append(m.forward(0, x[:n].contiguous()).double())
+        assert torch.equal(ys[0], ys[1]) == same
+        assert float((ys[0] - ys[1]).norm() / ys[1].norm()) <= 1.2e-3
+    m.close()
+
+
+@pytest.mark.parametrize("fmt,codebook,d,mid,E,last", [("q4cp", "zp8", 3072, 768, 256, 62), ("q4cp", "zp8", 2048, 768, 256, 50),
+                                                       ("q4cp", "universal", 1024, 512, 1000, 70), ("q4cp", "universal", 1024, 768, 256, 60),
+                                                       ("q4k", "zp8", 2048, 1024, 256, 60), ("i4r", "zp8", 3072, 768, 192, 50)])
+def test_which_layers_have_many_weights(capi, fmt, codebook, d, mid, E, last):
+    from gfx1151_engine_amd import workloads as W
+    ends_at(capi, W.DeviceLayer(6, d, mid, E, 8, fmt, codebook=codebook), d, mid, E, 8, last * E // 8)
+
+
 @pytest.mark.parametrize("fmt,T", [("q4cp", 40), ("q4cp", 300), ("q4k", 300), ("q4cp", 1100)])
 def test_the_callers_f16_copy_at_every_router(capi, fmt, T):
     """moe_forward_x16 against moe_forward, bit for bit; the router of 257 tokens and more makes its own copy all the same."""
