@@ -1030,23 +1030,34 @@ int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* 
 // (Q4_K and i4r 1 .. 2 % less throughout; table codebooks 2048 x 768 of 256 at 62 and 70 -3, 0, 3072 x 768 of 256 -3, +2.)  The
 // line between many and few lies between 403 and 524 M.
 constexpr int64_t MANY_WEIGHTS = (int64_t)7 << 26;
-//   Q5_K / Q8_0          25: 1039 964 / 1099 1032     29: 1061 1033 / -          33: 1091 1148 / 1139 1134
-// Q5_K / Q8_0 at even routing and other sizes: 3072 x 768 of 256 experts 30: 578 565, 34: 609 634; of 128 345 365, 351 374; of 64
-// 210 212, 211 246; 2048 x 768 of 512 29: 713 716, 33: 732 792.  With fewer experts neither has the blocks to fill the chip and the two are
-// level (16 experts, 512 x 768, 30, 34 and 38: 80 80, 79 81, 79 80): their line lies where it did with slower 128-pair kernels.
-// Q5_K and Q8_0 fragments leave no registers for 64 pairs (32-pair tiles above 22).  Rows of more than four lines of hid (mid >
-// 1024) leave no LDS for them: 32-pair tiles as well, level earlier (2048 x 1536, even: 23 q4cp 896 891, Q4_K 967 912; 29 q4cp
-// 923 967, Q4_K 996 1038, table 1149 1139, Q5_K / Q8_0 1519 1434; 37 table 1248 1409, Q5_K / Q8_0 1612 1741).
-// Layers that go to the general kernel otherwise (F_Q4E, F_Q5E): as far as was measured (2560 x 640: 59 1979 1245 / 2153 1257; 160
-// 3888 2682 / 3480 2691; 2048 x 1152: 160 5146 4036 / 4570 4035).
+// Q8_0 down rows beside Q4_K or Q5_K: the 128-pair kernels are k_moe_wide's, 32-pair tiles are the largest here.  Averages of 25, 28, 31
+// and 34, %, Q4_K | Q5_K gate/up: 3072 x 768 of 512 -9 -6 -1 +3 | (29) -3, (33) +5; of 384 -9 -5 -1 +3 | -7 -2 +2 +7; of 256 -11
+// -7 -2 0 | -9 -4 +1 +3; of 192 (453 M) -13 -9 -4 -3 | -10 -6 -1 -1; 2048 x 768 of 512 -8 -4 0 +4 | -4 -1 +5 +8; of 256 (403 M) -6 -3
+// +3 +5 | -3 0 +6 +10; 4096 x 1024 of 256 -8 -4 -1 +4 | -5 0 +2 +7; skewed, 28: -3 .. -10 | +2 .. -7.  With fewer weights, 22, 25, 28
+// and 31: 3072 x 768 of 128 0 +1 +1 +8 | -1 +2 +2 +9; of 64 +1 +1 +1 +4 | +2 +4 +2 +7; 2048 x 768 of 128 (201 M) +2 +1 +6 +8 | +2 +1
+// +7 +10; 1024 x 512 of 128 (67 M) -1 -3 -2 +3 | +3 -1 +1 +6; 4096 x 1024 of 32 +1 +1 +1 +5 | +5 +4 +2 +5.  Below 34 M the two are
+// level at any average up to 38 (16 .. 64 experts of 512 x 256 .. 1024 x 768: 75 .. 95 us either way), and the line lies where
+// it did with slower 128-pair kernels.
+// Rows of more than four lines of hid (mid > 1024) leave no LDS for 64 pairs: 32-pair tiles as well, level earlier (2048 x 1536, even:
+// 23 q4cp 896 891, Q4_K 967 912; 29 q4cp 923 967, Q4_K 996 1038, table 1149 1139; 37 table 1248 1409).  Beside Q8_0, averages of 23,
+// 26, 29 and 32, Q4_K | Q5_K: 512 experts -5 -4 +2 +6 | -2 0 +6 +11; 128 0 +2 +9 +11 | +2 +5 +12 +16; 64 -4 -5 -3 +1 | -1 -1 +1 +9;
+// 16 -7 -4 +1 +5 | -8 -5 -4 +2.
+// (Q5_K with Q4_K down rows: 25, 28 and 31 3072 x 768 of 512 -7 -6 +1, of 256 -9 -5 0, 2048 x 768 of 256 -4 0 +8, 3072 x 768 of 64 -1 +1
+// +13: the same lines.)
+// Layers that go to the general kernel otherwise (F_Q4E, F_Q5E): as far as was measured (2560 x 640 of 512, Q5_K / Q8_0: 60 1912 1273; 100
+// 2220 1869 / 2541 1863; 160 3676 2688; Q4_K / Q8_0: 100 2154 1646 / 2464 1636; 160 3562 2390; of 64, Q5_K: 60 367 236, 160 578 413; of
+// 16: 179 126, 198 169).
 constexpr float ONCE_LINE = 160.f;
 int moe_stream_tile_cap(int P, int k, int experts, int fmt_up, int fmt_dn, int d, int mid) {
   const float avg = (float)P * (float)k / (float)experts;
-  const bool small = q5(fmt_up) || fmt_dn == F_Q80, lone = mid > 1024, big = (int64_t)d * mid * experts >= MANY_WEIGHTS;
-  const float line = once_rounded(fmt_up) ? ONCE_LINE
-                     : small              ? (lone ? 32.f : q5(fmt_up) && experts >= 64 ? 31.f : 38.f)
-                     : fmt_up == F_TAB    ? (lone ? 29.f : big ? 70.f : 60.f)
-                                          : (lone ? 25.f : !big ? 50.f : fmt_up == F_DN || fmt_up == F_AFF ? 62.f : 60.f);
+  const int64_t weights = (int64_t)d * mid * experts;
+  const bool small = q5(fmt_up) || fmt_dn == F_Q80, lone = mid > 1024, big = weights >= MANY_WEIGHTS, five = q5(fmt_up);
+  float line;
+  if (once_rounded(fmt_up)) line = ONCE_LINE;
+  else if (small && lone) line = !five ? 28.f : experts >= 64 ? 26.f : 32.f;
+  else if (small) line = weights >= (int64_t)3 << 27 ? (five ? 29.f : 31.f) : weights >= 1 << 25 ? (five ? 22.f : 26.f) : five && experts >= 64 ? 31.f : 38.f;
+  else if (fmt_up == F_TAB) line = lone ? 29.f : big ? 70.f : 60.f;
+  else line = lone ? 25.f : !big ? 50.f : fmt_up == F_DN || fmt_up == F_AFF ? 62.f : 60.f;
   if (avg <= 10.f) return 16;
   return avg > line ? 0 : small || lone || avg <= 22.f ? 32 : 64;
 }

@@ -333,7 +333,7 @@ int moe_forward_x16(moe_ctx* ctx, int layer, const float* x, const void* x16, in
 /* MOE_OPT_PAIR_TABLES (default 1): q4cp layers whose codebook is a table (not a*n + b), batches above
  * MOE_OPT_F32_DECODE_MAX_TOKENS and up to 32 tokens: the f32 kernels look two neighbouring weights up at a time in
  * 256-entry pair tables (one per code byte); 0 = one look-up per weight in the 16-entry table, as at a few tokens. */
-/* MOE_OPT_STREAM_GEMM (default 1): batches in which an expert has few pairs (33 tokens up to an average of 25 to 160 pairs,
+/* MOE_OPT_STREAM_GEMM (default 1): batches in which an expert has few pairs (33 tokens up to an average of 22 to 160 pairs,
  * by kind of layer) run the
  * routed experts' two GEMMs on tiles of 16 to 64 pairs with the weights streamed into registers; 0 = the 128-pair
  * kernels at every size.  The same f16 weights and f32 sums, in another order. */

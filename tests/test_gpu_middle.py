@@ -479,6 +479,14 @@ def test_which_layers_have_many_weights(capi, fmt, codebook, d, mid, E, last):
     ends_at(capi, W.DeviceLayer(6, d, mid, E, 8, fmt, codebook=codebook), d, mid, E, 8, last * E // 8)
 
 
+@pytest.mark.parametrize("types,d,mid,E,last", [((12, 8, 8), 2048, 768, 256, 31), ((13, 8, 8), 2048, 768, 256, 29), ((12, 8, 8), 1024, 768, 64, 26),
+                                                ((13, 8, 12), 1024, 768, 64, 22), ((12, 8, 8), 512, 512, 32, 38), ((13, 8, 8), 512, 512, 32, 38),
+                                                ((12, 8, 8), 768, 1536, 64, 28), ((13, 8, 8), 768, 1536, 64, 26)])
+def test_where_the_few_pair_tiles_beside_8_bit_down_rows_end(capi, types, d, mid, E, last):
+    from gfx1151_engine_amd import workloads as W
+    ends_at(capi, W.DeviceLayer(7, d, mid, E, 8, "q4k", gg_types=types), d, mid, E, 8, last * E // 8)
+
+
 @pytest.mark.parametrize("fmt,T", [("q4cp", 40), ("q4cp", 300), ("q4k", 300), ("q4cp", 1100)])
 def test_the_callers_f16_copy_at_every_router(capi, fmt, T):
     """moe_forward_x16 against moe_forward, bit for bit; the router of 257 tokens and more makes its own copy all the same."""
