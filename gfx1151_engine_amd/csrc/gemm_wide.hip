@@ -373,10 +373,15 @@ k_moe_wide(WideW R, WideW Sh, int n_experts, const __half* __restrict__ x, const
            const moe_tile* __restrict__ tiles, const int* __restrict__ ntiles, __half* __restrict__ out, int M, int K, int nblk,
            int npass, moe_hscale hs) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  // consecutive workgroup ids go round-robin over the XCDs: each takes a contiguous run of tiles (gemm_q4cp.hip)
+  // consecutive workgroup ids go round-robin over the XCDs: each takes a contiguous run of tiles (gemm_q4cp.hip).  With no more
+  // tiles than XCDs their blocks are dealt out one by one instead: all of a shared expert's on the first XCD, beside the routed
+  // experts' launches, slowed that XCD's share of those (512 experts, 3072 x 768 Q5_K / Q8_0, 33 tokens 377 -> 368 us, 96 631 -> 622;
+  // 2560 x 640 q4cp with a q8g32 shared expert 33 237 -> 226, 130 380 -> 371; 128 experts, 3072 x 768, 33 253 -> 239.  Up to 31 or 63
+  // tiles dealt out: up to 14 % slower, blocks of a tile fetch its activations through every L2)
   const int nt = ntiles[0], per = (nt + 7) >> 3;
-  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3, tl = j / nblk, ti = xcd * per + tl;
-  if (tl >= per || ti >= nt) return;
+  const bool spread = nt <= 8;
+  const int xcd = blockIdx.x & 7, j = spread ? blockIdx.x : blockIdx.x >> 3, tl = j / nblk, ti = spread ? tl : xcd * per + tl;
+  if ((!spread && tl >= per) || ti >= nt) return;
   const moe_tile tile = tiles[ti];
   const bool shared = tile.expert >= n_experts;
   WideW L;

@@ -569,6 +569,21 @@ def test_8_bit_codes_in_tiles_of_every_size(capi, oracle, kind, kw, d, mid, pair
     assert max_abs_rel(y, yo) <= 2e-3
 
 
+@pytest.mark.parametrize("E", [5, 7, 8, 16, 17])
+def test_8_bit_codes_on_few_tiles_and_more(capi, oracle, E):
+    """Six tiles to eighteen, the shared expert's among them: up to eight are dealt out to the XCDs block by block."""
+    rng = np.random.default_rng(E)
+    hl = HostLayer(rng, 512, 384, E, E // 2, fmt="q4k", gg_types=(8, 8, 8))
+    x = rng.standard_normal((60, 512), dtype=np.float32)
+    yo, io, _ = oracle.moe_layer(hl.oracle_layer(), x)
+    assert (np.bincount(io[:, :E // 2].ravel(), minlength=E) > 0).all()
+    m, dev = hl.to_gpu(max_tokens=60)
+    y = m.forward(0, gpu(x)).cpu().numpy()
+    assert m.last_path() == capi.PATH_BATCH
+    m.close()
+    assert max_abs_rel(y, yo) <= 2e-3
+
+
 # ---------- Q5_K in 128-pair tiles: rows that end inside a block, one super-block and several, tiles of every size ----------
 @pytest.mark.parametrize("d,mid,E,T", [(256, 320, 8, 40), (512, 192, 2, 150), (768, 64, 3, 200), (1024, 960, 4, 70)])
 def test_fifth_bits_of_part_filled_row_blocks(capi, oracle, d, mid, E, T):
