@@ -1121,6 +1121,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   // of 0), so that every reason to decline is found before anything is enqueued
   bool dry = true;
   // (routed: the launch holds the routed experts' tiles -- with_sh then says that the shared expert's ride along)
+  const int each = (P * g.topk + g.experts - 1) / g.experts;  // pairs of a routed expert
   auto gemm_up = [&](bool routed, bool with_sh, const moe_tile* tl, const int* ntl, int mt, hipStream_t s2) -> int {
     if (dry) mt = 0;
     if (routed && cap) {
@@ -1132,7 +1133,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
     }
     if (shd && with_sh)  // the shared expert's own tile list
       return moe_launch_gemm_gg(true, L.sh_dense, L.sh_gate.data, L.sh_up.data, 0, nullptr, nullptr, g.experts, xh,
-                                c->tokidx, tl, ntl, mt, c->hid16, g.mid, g.d, hs, s2, xl);
+                                c->tokidx, tl, ntl, mt, c->hid16, g.mid, g.d, hs, s2, xl, P, true);
     if (q4k && split) {  // one class per launch: the shared expert's tiles (with_sh) or the routed experts'
       if (with_sh ? kd.s_gu : kd.r_gu)
         return moe_launch_gemm_q4cp(true, with_sh ? &sgu : &gu, with_sh ? &sgu : nullptr, g.experts, xh, c->tokidx, tl, ntl,
@@ -1140,14 +1141,14 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
                                     (with_sh ? L.sh_gguf_type : L.gg.tgu) == MOE_GGML_Q5_K);
       return with_sh ? moe_launch_gemm_gg(true, L.sh_gguf_type, L.sh_gate.data, L.sh_up.data, L.sh_gguf_type,
                                           L.sh_gate.data, L.sh_up.data, g.experts, xh, c->tokidx, tl, ntl, mt, c->hid16,
-                                          g.mid, g.d, hs, s2, xl)
+                                          g.mid, g.d, hs, s2, xl, P, true)
                      : moe_launch_gemm_gg(true, L.gg.tgu, L.gg.gate, L.gg.up, 0, nullptr, nullptr, g.experts, xh,
-                                          c->tokidx, tl, ntl, mt, c->hid16, g.mid, g.d, hs, s2, xl);
+                                          c->tokidx, tl, ntl, mt, c->hid16, g.mid, g.d, hs, s2, xl, each, false);
     }
     if (q4k && !kd.r_gu)
       return moe_launch_gemm_gg(true, L.gg.tgu, L.gg.gate, L.gg.up, L.sh_gguf_type, with_sh ? L.sh_gate.data : nullptr,
                                 with_sh ? L.sh_up.data : nullptr, g.experts, xh, c->tokidx, tl, ntl, mt, c->hid16, g.mid,
-                                g.d, hs, s2, xl);
+                                g.d, hs, s2, xl, routed ? each : P, !routed);
     if (v2 && !with_sh) {
       // the routed experts' tiles: gate rows and their up rows in one block, the slot-wise middle (rotation back,
       // SwiGLU, rotation for down_proj) in the launch's epilogue
@@ -1178,7 +1179,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
                                c->pairs16, g.d, g.mid, hs, s2, nullptr, pe_dn, pe_sdn);
     if (shd && with_sh)  // (hid rows of the shared tiles were written in natural order by the launch above)
       return moe_launch_gemm_gg(false, L.sh_dense, L.sh_down.data, nullptr, 0, nullptr, nullptr, g.experts, c->hid16,
-                                nullptr, tl, ntl, mt, c->pairs16, g.d, g.mid, hs, s2, 0);
+                                nullptr, tl, ntl, mt, c->pairs16, g.d, g.mid, hs, s2, 0, P, true);
     if (q4k && split) {
       // (hid rows are in the tuned kernel's order where its gate/up form wrote them, else in natural order)
       if (with_sh ? kd.s_dn : kd.r_dn)
@@ -1186,14 +1187,14 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
                                     ntl, mt, c->pairs16, g.d, g.mid, true, true, hs, s2, nullptr);
       return with_sh ? moe_launch_gemm_gg(false, L.sh_gguf_type, L.sh_down.data, nullptr, L.sh_gguf_type, L.sh_down.data,
                                           nullptr, g.experts, c->hid16, nullptr, tl, ntl, mt, c->pairs16, g.d, g.mid, hs, s2,
-                                          kd.s_gu ? 2 : 0)
+                                          kd.s_gu ? 2 : 0, P, true)
                      : moe_launch_gemm_gg(false, L.gg.tdn, L.gg.down, nullptr, 0, nullptr, nullptr, g.experts, c->hid16,
-                                          nullptr, tl, ntl, mt, c->pairs16, g.d, g.mid, hs, s2, kd.r_gu ? 2 : 0);
+                                          nullptr, tl, ntl, mt, c->pairs16, g.d, g.mid, hs, s2, kd.r_gu ? 2 : 0, each, false);
     }
     if (q4k && !kd.r_dn)
       return moe_launch_gemm_gg(false, L.gg.tdn, L.gg.down, nullptr, L.sh_gguf_type, with_sh ? L.sh_down.data : nullptr,
                                 nullptr, g.experts, c->hid16, nullptr, tl, ntl, mt, c->pairs16, g.d, g.mid, hs, s2,
-                                kd.r_gu ? 2 : 0);
+                                kd.r_gu ? 2 : 0, routed ? each : P, !routed);
     if (v2 && !with_sh)
       return moe_launch_gemm_q4cp(false, &dn, nullptr, g.experts, c->hid16, nullptr, tl, ntl, mt, c->pairs16, g.d, g.mid,
                                   true, false, moe_hscale{nullptr, 0.f, 0.f}, s2, nullptr, nullptr, 2);

@@ -426,15 +426,31 @@ int launch(const WideW& R, const WideW& S, int n_experts, const __half* x, const
 }  // namespace
 
 // The launches of moe_launch_gemm_gg that k_moe_wide takes: every tensor Q8_0 or every tensor q8g32, whole stages of 128
-// columns, whole waves of rows.
+// columns, whole waves of rows.  each: pairs that an expert has on average; alone: the launch is the shared expert's
 bool moe_wide_takes(bool up, int type, const uint8_t* w, const uint8_t* w_up, int tsh, const uint8_t* sh_w, const uint8_t* sh_w_up,
-                    int m, int k, int a_layout) {
+                    int m, int k, int a_layout, int n_experts, int max_tiles, int each, bool alone) {
   if (type != MOE_GGML_Q8_0 && type != MOE_T_Q8G32) return false;
   if (sh_w && tsh != type) return false;
   const size_t al = type == MOE_GGML_Q8_0 ? 4 : 16;
   for (const uint8_t* p : {w, up ? w_up : w, sh_w ? sh_w : w, sh_w && up ? sh_w_up : w})
     if (!moe_aligned(p, al)) return false;
   if (k % 128 || m % (up ? 32 : 64)) return false;
+  // Q8_0 on few blocks: the general kernel has twice as many, and there the tile's weights take less of a wave's time.  (q8g32: it
+  // has no such form, and takes 25 .. 45 % longer at any size.)  us of a layer, here and there, Q5_K / Q8_0, Q8_0 shared expert:
+  //   up to four tiles of more than 64 tokens   3072 x 768 of 16 experts 130 138 125, 300 155 130, 400 163 141, 515 (five) 154 149; of
+  //     32 130 150 135, 400 181 161, 700 (six) 214 221; of 64 256 216 190, 700 243 274; of 128 400 340 333, 1000 (eight) 381 397
+  //   one tile of at most 64, next to a launch of many weights   3072 x 768 of 64 (151 M) 33 185 167, 64 189 171; 2048 x 1536 of 64 191
+  //     185; 2560 x 640 of 64 (105 M) 144 138; of 512 experts level; with fewer weights the shared expert is waited for, and is done
+  //     sooner here: 3072 x 768 of 32 (75 M) 48 127 132; 1024 x 768 of 64 93 99
+  //   routed gate/up, more than 64 pairs, fewer than 128 blocks   all Q8_0, top-2 of 8, 2560 x 640 1000 tokens 141 120, 4096 x 1024 400
+  //     194 187, 700 (152 blocks) 154 162
+  if (type == MOE_GGML_Q8_0) {
+    if (each <= 64) {
+      if (alone && (int64_t)m * k * n_experts >= (int64_t)3 << 25) return false;
+    } else if (alone ? max_tiles <= 4 : up && max_tiles * ((m + 127) / 128) < 128) {
+      return false;
+    }
+  }
   return a_layout == 0 || (type == MOE_GGML_Q8_0 && a_layout == 2) || (type == MOE_T_Q8G32 && up && a_layout == 1);
 }
 int moe_launch_wide(bool up, int type, const uint8_t* w, const uint8_t* w_up, const uint8_t* sh_w, const uint8_t* sh_w_up, int n_experts,

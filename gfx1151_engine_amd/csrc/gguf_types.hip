@@ -861,10 +861,11 @@ int moe_launch_ggx_gemv(int phase, int tgu, int tdn, int tsh, const uint8_t* gat
 // `type` / `tsh` may also be a dense code of dense.h (bf16 / f32 / q8g64 rows).
 // up: gate/up + SwiGLU -> hid f16 [pairs][m]; else down -> pairs f16 [pairs][m].  x / hid: f16, natural order
 // (a_layout = 1 / 2: x is in the q4cp / Q4_K GEMM's order and is put back in natural order on its way into LDS).
+// each: pairs that an expert of the launch has on average; alone: all tiles are the shared expert's (moe_wide_takes).
 int moe_launch_gemm_gg(bool up, int type, const uint8_t* w, const uint8_t* w_up, int tsh, const uint8_t* sh_w,
                        const uint8_t* sh_w_up, int n_experts, const __half* x16, const int* tokidx,
                        const moe_tile* tiles, const int* ntiles, int max_tiles, __half* out, int m, int k,
-                       moe_hscale hs, hipStream_t st, int a_layout) {
+                       moe_hscale hs, hipStream_t st, int a_layout, int each, bool alone) {
   if (!w || (up && !w_up) || !x16 || !tiles || !ntiles || !out || max_tiles < 0) return MOE_E_INVALID;
   auto type_ok = [&](int t) { return moe_is_dense_type(t) ? k % 64 == 0 : gg_type_ok(t, k); };
   auto align_of = [&](int t) -> size_t { return moe_is_dense_type(t) ? 16 : gg_align(t); };
@@ -875,7 +876,7 @@ int moe_launch_gemm_gg(bool up, int type, const uint8_t* w, const uint8_t* w_up,
     return MOE_E_INVALID;
   if (!up && (m % 8 || !moe_aligned(out, 16))) return MOE_E_UNSUPPORTED;  // (down results leave as 16-byte pieces)
   if (max_tiles == 0) return MOE_OK;
-  if (moe_wide_takes(up, type, w, w_up, tsh, sh_w, sh_w_up, m, k, a_layout))
+  if (moe_wide_takes(up, type, w, w_up, tsh, sh_w, sh_w_up, m, k, a_layout, n_experts, max_tiles, each, alone))
     return moe_launch_wide(up, type, w, w_up, sh_w, sh_w_up, n_experts, x16, tokidx, tiles, ntiles, max_tiles, out, m, k, hs, st, a_layout);
   GgGemmW R{w, w_up, type}, S{sh_w ? sh_w : w, sh_w ? sh_w_up : w_up, sh_w ? tsh : type};
   const dim3 grid((unsigned)(up ? (m + 63) / 64 : (m + GG_BN - 1) / GG_BN), (unsigned)max_tiles);

@@ -228,10 +228,10 @@ int moe_launch_i4r_mid(const void* z, bool z_f16, uint64_t zs, int nslots, int m
 int moe_launch_gemm_gg(bool up, int type, const uint8_t* w, const uint8_t* w_up, int tsh, const uint8_t* sh_w,
                        const uint8_t* sh_w_up, int n_experts, const __half* x16, const int* tokidx,
                        const moe_tile* tiles, const int* ntiles, int max_tiles, __half* out, int m, int k,
-                       moe_hscale hs, hipStream_t st, int a_layout = 0);
+                       moe_hscale hs, hipStream_t st, int a_layout, int each, bool alone);
 // Grouped GEMM for 8-bit codes (gemm_wide.hip): what moe_launch_gemm_gg hands over, its arguments checked
 bool moe_wide_takes(bool up, int type, const uint8_t* w, const uint8_t* w_up, int tsh, const uint8_t* sh_w, const uint8_t* sh_w_up,
-                    int m, int k, int a_layout);
+                    int m, int k, int a_layout, int n_experts, int max_tiles, int each, bool alone);
 int moe_launch_wide(bool up, int type, const uint8_t* w, const uint8_t* w_up, const uint8_t* sh_w, const uint8_t* sh_w_up, int n_experts,
                     const __half* x16, const int* tokidx, const moe_tile* tiles, const int* ntiles, int max_tiles, __half* out, int m,
                     int k, moe_hscale hs, hipStream_t st, int a_layout);

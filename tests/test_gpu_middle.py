@@ -584,6 +584,21 @@ def test_8_bit_codes_on_few_tiles_and_more(capi, oracle, E):
     assert max_abs_rel(y, yo) <= 2e-3
 
 
+@pytest.mark.parametrize("types,T", [((13, 8, 8), 64), ((13, 8, 8), 65), ((13, 8, 8), 512), ((13, 8, 8), 513), ((8, 8, 8), 257), ((8, 8, 8), 520)])
+def test_8_bit_shared_experts_alone(capi, oracle, types, T):
+    """A shared expert's own launches on either side of the line between the kernels (one tile of 64, five of 128), and all-Q8_0 layers
+    whose routed gate/up has few blocks."""
+    rng = np.random.default_rng(T)
+    hl = HostLayer(rng, 512, 256, 4, 2, fmt="q4k", gg_types=types)
+    x = rng.standard_normal((T, 512), dtype=np.float32)
+    yo, _, _ = oracle.moe_layer(hl.oracle_layer(), x)
+    m, dev = hl.to_gpu(max_tokens=T)
+    y = m.forward(0, gpu(x)).cpu().numpy()
+    assert m.last_path() == capi.PATH_BATCH
+    m.close()
+    assert max_abs_rel(y, yo) <= 2e-3
+
+
 # ---------- Q5_K in 128-pair tiles: rows that end inside a block, one super-block and several, tiles of every size ----------
 @pytest.mark.parametrize("d,mid,E,T", [(256, 320, 8, 40), (512, 192, 2, 150), (768, 64, 3, 200), (1024, 960, 4, 70)])
 def test_fifth_bits_of_part_filled_row_blocks(capi, oracle, d, mid, E, T):
