@@ -37,13 +37,12 @@
 // src/gpu/parts/27_kernels_moe_lut.inc:23-29): the four stages between two scale refreshes span exactly two scales,
 // fetched as one 4-byte load per row.
 #include "common.h"
+#include "half.h"
 #include "hv2.h"
 #include "internal.h"
 
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 #ifndef MOE_GEMM_NF
@@ -90,18 +89,6 @@ struct LutDev {
   const int8_t* pexp;
 };
 
-union H8 {
-  half8 v;
-  uint32_t u[4];
-  half2v h[4];
-};
-
-__device__ __forceinline__ half2v as_h2(uint32_t u) {
-  union { uint32_t u; half2v h; } c;
-  c.u = u;
-  return c.h;
-}
-
 // 8 codes of one 32-bit word -> 8 f16 weights (a*n + b) * s, order [n0,n4,n1,n5,n2,n6,n3,n7].
 // 0x6400|n is the f16 1024+n, 0x5400|(n<<4) is 64+n: subtracting the magic leaves n exactly;
 // for the zero-point-8 codebook (a=1, b=-8) fma(n, s, -8s) rounds (n-8)*s once.
@@ -109,10 +96,10 @@ __device__ __forceinline__ half8 deq8_affine(uint32_t w, half2v as2, half2v bs2)
   const half2v k1024 = {(_Float16)1024.f, (_Float16)1024.f}, k64 = {(_Float16)64.f, (_Float16)64.f};
   H8 r;
   const uint32_t w8 = w >> 8;
-  r.h[0] = (as_h2((w & 0x000f000fu) | 0x64006400u) - k1024) * as2 + bs2;
-  r.h[1] = (as_h2((w & 0x00f000f0u) | 0x54005400u) - k64) * as2 + bs2;
-  r.h[2] = (as_h2((w8 & 0x000f000fu) | 0x64006400u) - k1024) * as2 + bs2;
-  r.h[3] = (as_h2((w8 & 0x00f000f0u) | 0x54005400u) - k64) * as2 + bs2;
+  r.h[0] = (h2((w & 0x000f000fu) | 0x64006400u) - k1024) * as2 + bs2;
+  r.h[1] = (h2((w & 0x00f000f0u) | 0x54005400u) - k64) * as2 + bs2;
+  r.h[2] = (h2((w8 & 0x000f000fu) | 0x64006400u) - k1024) * as2 + bs2;
+  r.h[3] = (h2((w8 & 0x00f000f0u) | 0x54005400u) - k64) * as2 + bs2;
   return r.v;
 }
 // any codebook: 16-entry f32 table in LDS, w = f16(cb[n] * s)
@@ -488,15 +475,15 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
         }
         const uint32_t wsc = jj < 2 ? k4w[nf][0] : k4w[nf][1], wmn = jj < 2 ? k4w[nf][2] : k4w[nf][3];
         const half2v k1024 = half2v{(_Float16)1024.f, (_Float16)1024.f};
-        const half2v sc = as_h2(__builtin_amdgcn_perm(0x64646464u, wsc, selb)) - k1024;
-        const half2v mn = as_h2(__builtin_amdgcn_perm(0x64646464u, wmn, selb)) - k1024;
+        const half2v sc = h2(__builtin_amdgcn_perm(0x64646464u, wsc, selb)) - k1024;
+        const half2v mn = h2(__builtin_amdgcn_perm(0x64646464u, wmn, selb)) - k1024;
         union { half2v h; uint32_t u; } a, b;
-        a.h = sc * as_h2(k4w[nf][4]);
-        b.h = mn * as_h2(k4w[nf][5]);
-        as2[nf][0] = as_h2(__builtin_amdgcn_perm(a.u, a.u, 0x01000100u));
-        bs2[nf][0] = as_h2(__builtin_amdgcn_perm(b.u, b.u, 0x01000100u));
-        as2[nf][NS - 1] = as_h2(__builtin_amdgcn_perm(a.u, a.u, 0x03020302u));
-        bs2[nf][NS - 1] = as_h2(__builtin_amdgcn_perm(b.u, b.u, 0x03020302u));
+        a.h = sc * h2(k4w[nf][4]);
+        b.h = mn * h2(k4w[nf][5]);
+        as2[nf][0] = h2(__builtin_amdgcn_perm(a.u, a.u, 0x01000100u));
+        bs2[nf][0] = h2(__builtin_amdgcn_perm(b.u, b.u, 0x01000100u));
+        as2[nf][NS - 1] = h2(__builtin_amdgcn_perm(a.u, a.u, 0x03020302u));
+        bs2[nf][NS - 1] = h2(__builtin_amdgcn_perm(b.u, b.u, 0x03020302u));
       }
     } else {
 #pragma unroll
@@ -522,8 +509,8 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
     if (DN) {
       const uint32_t w8 = q == 0 ? cw8[nf].x : q == 1 ? cw8[nf].y : q == 2 ? cw8[nf].z : cw8[nf].w;
       const uint32_t ws = part >= 2 ? w8 : w;
-      if ((part & 1) == 0) dst[nf].h[part] = as_h2(ws & 0x000f000fu) * as2[nf][0] + bs2[nf][0];
-      else dst[nf].h[part] = as_h2(ws & 0x00f000f0u) * as20[DN ? nf : 0] + bs2[nf][0];
+      if ((part & 1) == 0) dst[nf].h[part] = h2(ws & 0x000f000fu) * as2[nf][0] + bs2[nf][0];
+      else dst[nf].h[part] = h2(ws & 0x00f000f0u) * as20[DN ? nf : 0] + bs2[nf][0];
     } else if (Q5) {
       // five-bit codes as bytes, the low nibbles' (parts 0, 2) and the high nibbles' (1, 3): parts 0 and 1 make them.  Bit
       // 2 jj / 2 jj + 1 of each byte of the qh word goes to bit 4
@@ -533,7 +520,7 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
         c5[nf][part] = ((part ? w >> 4 : w) & 0x0f0f0f0fu) | fifth;
       }
       const uint32_t t = __builtin_amdgcn_perm(0x64646464u, c5[nf][part & 1], part >= 2 ? 0x04030401u : 0x04020400u);
-      dst[nf].h[part] = (as_h2(t) - half2v{(_Float16)1024.f, (_Float16)1024.f}) * as2[nf][part & (NS - 1)] + bs2[nf][part & (NS - 1)];
+      dst[nf].h[part] = (h2(t) - half2v{(_Float16)1024.f, (_Float16)1024.f}) * as2[nf][part & (NS - 1)] + bs2[nf][part & (NS - 1)];
     } else if (AFFINE) {
       const uint32_t w8 = q == 0 ? cw8[nf].x : q == 1 ? cw8[nf].y : q == 2 ? cw8[nf].z : cw8[nf].w;
       const uint32_t ws = part >= 2 ? w8 : w;
@@ -541,10 +528,10 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
       uint32_t t;
       if ((part & 1) == 0) {
         asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t) : "v"(ws), "s"(0x000f000fu), "v"(0x64006400u));
-        dst[nf].h[part] = (as_h2(t) - half2v{(_Float16)1024.f, (_Float16)1024.f}) * as2[nf][ss] + bs2[nf][ss];
+        dst[nf].h[part] = (h2(t) - half2v{(_Float16)1024.f, (_Float16)1024.f}) * as2[nf][ss] + bs2[nf][ss];
       } else {
         asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t) : "v"(ws), "s"(0x00f000f0u), "v"(0x54005400u));
-        dst[nf].h[part] = (as_h2(t) - half2v{(_Float16)64.f, (_Float16)64.f}) * as2[nf][ss] + bs2[nf][ss];
+        dst[nf].h[part] = (h2(t) - half2v{(_Float16)64.f, (_Float16)64.f}) * as2[nf][ss] + bs2[nf][ss];
       }
     } else {
       if (NAT) {
@@ -552,7 +539,7 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
         // f16(cb), one packed product applies the scale: w = f16(f16(cb[n]) * scale), the reference kernel's contract
         // (src/gpu/parts/27_kernels_moe_lut.inc:16)
         const uint32_t* pt = (UP && nf >= NH) ? ptab + 256 : ptab;
-        dst[nf].h[part] = as_h2(pt[(w >> (8 * part)) & 0xffu]) * as2[nf][0];
+        dst[nf].h[part] = h2(pt[(w >> (8 * part)) & 0xffu]) * as2[nf][0];
       } else {
         half2v hv;
         const float* tb = (UP && nf >= NH) ? cbs + 16 : cbs;

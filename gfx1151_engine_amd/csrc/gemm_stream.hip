@@ -41,13 +41,12 @@
 #include <type_traits>
 
 #include "common.h"
+#include "half.h"
 #include "hv2.h"
 #include "internal.h"
 
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // F_DN: affine q4cp codebooks whose experts all have a power of two for the scaled dequantisation (gemm_q4cp.hip, DN)
@@ -75,21 +74,6 @@ struct SW {
   const int8_t* pexp;
 };
 
-union H8 {
-  half8 v;
-  uint32_t u[4];
-  half2v h[4];
-};
-__device__ __forceinline__ half2v h2(uint32_t u) {
-  union { uint32_t u; half2v h; } c;
-  c.u = u;
-  return c.h;
-}
-__device__ __forceinline__ uint32_t u2(half2v h) {
-  union { half2v h; uint32_t u; } c;
-  c.h = h;
-  return c.u;
-}
 __device__ __forceinline__ half2v both(float f) { return half2v{(_Float16)f, (_Float16)f}; }
 
 template <int FMT>
@@ -323,7 +307,6 @@ __device__ __forceinline__ Deq<F> make_deq(const uint32_t (&sw)[F], const Consts
   }
   return D;
 }
-__device__ __forceinline__ uint32_t word(const uint4& q, int s) { return s == 0 ? q.x : s == 1 ? q.y : s == 2 ? q.z : q.w; }
 
 // acc[f][mf] += half line E_ of fragment f x the line's activations (line_mma's arguments and its sums, in its order).
 // A step's MFMAs run while the next step's operands are made: every (step, 16 pairs) is an item of F MFMAs, one activation

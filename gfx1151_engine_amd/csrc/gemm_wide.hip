@@ -21,12 +21,11 @@
 
 #include "common.h"
 #include "dense.h"
+#include "half.h"
 #include "internal.h"
 
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 enum { W_Q80, W_G32 };
@@ -35,17 +34,6 @@ struct WideW {
   const uint8_t *w, *w_up;
   uint64_t sc;  // q8g32: byte offset of the scale plane
 };
-
-union H8 {
-  half8 v;
-  half2v h[4];
-};
-__device__ __forceinline__ half2v h2(uint32_t u) {
-  union { uint32_t u; half2v h; } c;
-  c.u = u;
-  return c.h;
-}
-__device__ __forceinline__ uint32_t word(const uint4& q, int s) { return s == 0 ? q.x : s == 1 ? q.y : s == 2 ? q.z : q.w; }
 
 constexpr int XROW = 256;              // bytes of a stage (128 columns) of one pair row
 constexpr int XBUF = 128 * XROW;       // of a tile
