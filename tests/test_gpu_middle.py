@@ -584,6 +584,21 @@ def test_8_bit_codes_on_few_tiles_and_more(capi, oracle, E):
     assert max_abs_rel(y, yo) <= 2e-3
 
 
+@pytest.mark.parametrize("d,mid,E", [(2560, 128, 205), (2560, 256, 205), (1536, 128, 512)])
+def test_8_bit_down_blocks_of_several_row_groups(capi, oracle, d, mid, E):
+    """Down blocks that walk two neighbouring groups of 256 rows (of ten) and three (of six), one stage of columns to a pass and two:
+    what a pass leaves behind for the next one."""
+    rng = np.random.default_rng(d + mid)
+    hl = HostLayer(rng, d, mid, E, 4, fmt="q4k", gg_types=(8, 8, 8))
+    x = rng.standard_normal((33, d), dtype=np.float32)
+    yo, _, _ = oracle.moe_layer(hl.oracle_layer(), x)
+    m, dev = hl.to_gpu(max_tokens=33)
+    y = m.forward(0, gpu(x)).cpu().numpy()
+    assert m.last_path() == capi.PATH_BATCH
+    m.close()
+    assert max_abs_rel(y, yo) <= 2e-3
+
+
 @pytest.mark.parametrize("types,T", [((13, 8, 8), 64), ((13, 8, 8), 65), ((13, 8, 8), 512), ((13, 8, 8), 513), ((8, 8, 8), 257), ((8, 8, 8), 520)])
 def test_8_bit_shared_experts_alone(capi, oracle, types, T):
     """A shared expert's own launches on either side of the line between the kernels (one tile of 64, five of 128), and all-Q8_0 layers
