@@ -402,7 +402,7 @@ __device__ __forceinline__ float ggu_dot(const GgU<T>& o, int jj, const XU& x) {
     int a0 = 0, a1 = 0, b0 = 0, b1 = 0;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      // (the unit's two bits rotated to bit 4 of each byte: 2 operations of 20 per word less, 117 -> 116 us)
+      // (the unit's two bits rotated to bit 4 of each byte: 2 operations of 20 per word less)
       const int lo = (int)((w[i] & 0x0f0f0f0fu) | (__builtin_amdgcn_alignbit(qh[i], qh[i], to4) & 0x10101010u));
       const int hi = (int)(((w[i] >> 4) & 0x0f0f0f0fu) | (__builtin_amdgcn_alignbit(qh[i], qh[i], to4h) & 0x10101010u));
       a0 = __builtin_amdgcn_sdot4(lo, (int)x.a[0][i], a0, false);
@@ -506,8 +506,9 @@ __device__ __forceinline__ float ggu_dot(const GgU<T>& o, int jj, const XU& x) {
 // Q8_0 136.4 134.8, 299.2 292.3, 462.9 451.2; Q5_K / Q8_0 118.3 117.8, 252.3 250.0, 387.0 382.4; Q5_1 / Q8_0 117.2 117.3, 250.3
 // 249.1, 382.7 380.7; Q5_K / Q5_K 107.2 106.0, 227.5 225.0, 355.9 353.2.
 // Q4_K and IQ4 rows are level or better in the ring (20 tokens, batches and ring: Q4_K 231.0 231.5, IQ4_NL 227.4 226.0, IQ4_XS
-// 232.1 231.5; 1 token, four layers: Q4_K 112.8 111.5); one and two tokens of any type are within 1 % either way (FEW).  Down rows are better in the ring for every type (ggu_dn_rows; 1 token, four
-// layers: Q5_K / Q8_0 117.5 115.6, Q4_K / Q8_0 111.5 107.9, Q8_0 132.5 129.6, Q5_1 112.4 111.4, IQ4_NL 115.4 114.9).
+// 232.1 231.5; 1 token, four layers: Q4_K 112.8 111.5); one and two tokens of any type are within 1 % either way (FEW).  Down
+// rows are better in the ring for every type (ggu_dn_rows; 1 token, four layers: Q5_K / Q8_0 117.5 115.6, Q4_K / Q8_0 111.5
+// 107.9, Q8_0 132.5 129.6, Q5_1 112.4 111.4, IQ4_NL 115.4 114.9).
 template <int T, bool FEW>
 constexpr bool ggu_gu_ring() { return FEW || T == MOE_GGML_Q4_K || T == MOE_GGML_IQ4_NL || T == MOE_GGML_IQ4_XS; }
 // eight rows of one wave (gate/up launch: four gate rows and the matching up rows): acc[i] = wave sum of row i

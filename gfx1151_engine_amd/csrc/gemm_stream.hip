@@ -32,10 +32,10 @@
 // Pairs per tile: 16, 32 or 64 by the batch's average (moe_stream_tile_cap): a block's work is the weights whatever the
 // tile holds, so tiles should hold an expert's pairs as a rule, and larger ones cost LDS and registers.
 // Measured (512 experts, top-10, 3072 x 768, gate/up + down, us; in brackets the 128-pair kernels):
-//   130 tokens q4cp 270 + 137 (368 + 185)      48 table 208 + 110 (295 + 177)    515 Q4_K 356 + 176 (413 + 241)
-//   200 Q5_K / Q8_0 407 + 291 (501 + 471)     200 i4r 260 + 143 (338 + 190)      2048 q4cp 371 + 209 (437 + 238)
+//   130 tokens q4cp 264 + 134 (354 + 178)      48 table 205 + 106 (298 + 170)    515 Q4_K 341 + 163 (431 + 234)
+//   200 Q5_K / Q8_0 396 + 282 (487 + 357)     200 i4r 266 + 135 (369 + 191)      2048 q4cp 357 + 206 (444 + 239)
 // The layer at other widths, us (128-pair kernels in brackets), 48 / 515 / 1200 tokens, d = 3072: mid 256 q4cp 162 / 258 / 331 (207 / 307 /
-// 361), Q5_K / Q8_0 240 / 351 / 450 (353 / 523 / 560); 512 q4cp 245 / 401 / 474 (312 / 491 / 549), table 272 / 434 / 535 (392 / 610 / 639),
+// 361), Q5_K / Q8_0 214 / 343 / 437 (261 / 409 / 461); 512 q4cp 245 / 401 / 474 (312 / 491 / 549), table 272 / 434 / 535 (392 / 610 / 639),
 // Q4_K 257 / 428 / 513 (339 / 544 / 602), i4r 245 / 378 / 467 (318 / 478 / 542); 1024 q4cp 429 / 719 / 827 (520 / 851 / 942), table 471 /
 // 781 / 930 (645 / 1074 / 1143); d = 2048: 1536 q4cp 419 / 759 / 891 (518 / 833 / 896), 2048 545 / 969 / 1083 (669 / 1083 / 1148).
 #include <type_traits>
@@ -536,8 +536,8 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
     for (int f = 0; f < 2; f++) q[f] = *(const uint4*)(wb[f] + at + (past ? 0u : wo + 16u * (uint32_t)g));
   };
   // ---- the pipeline's first requests.  Loads come back in order: the tile's row indices, which the activations' addresses wait
-  // for, go ahead of the weights (after them: 48 tokens table 350 -> 348 us, 130 i4r 436.5 -> 433.5, 300 Q5_K 770 -> 766, 515 Q4_K
-  // 578 -> 575.5) ----
+  // for, go ahead of the weights (after them 0.4 .. 0.7 % slower with both timed in turn -- 130 tokens i4r 436.5 433.5 us, 300 Q5_K 770 766,
+  // 515 Q4_K 578 575.5 --, little more than two runs differ) ----
   constexpr int XL = MF * 16 * 32 / NT, XS = NT / 32;  // loads per thread and line, rows per load
   constexpr int XH = HALVES ? (XL + 1) / 2 : XL;       // loads of a part of the line
   static_assert(XL >= 1 && XL * NT == MF * 16 * 32 && XH <= 4, "whole loads, named registers below");

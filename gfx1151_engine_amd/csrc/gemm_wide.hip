@@ -11,10 +11,12 @@
 // leaves room for six vector operations; dequantisation takes 30 per step of 2 .. 8 MFMAs.  The order of a step is fixed by hand:
 // an item of two MFMAs reads one activation operand two items ahead and dequantises a part of the next step's weights.
 // Two blocks to a CU (65 KB of LDS, 256 registers): their barriers, prologues and epilogues are independent.
-// us, general kernel and this one: a shared expert of 2000 tokens, 3072 x 768 Q8_0, alone: 91 + 110 and 56 + 23; beside the
-// routed launches, q8g32 2560 x 640, a layer of 2048 tokens: 668 and 632.  Routed Q8_0 down: 2000 tokens 520 and 427, 4096
-// (skewed) 648 and 551, 8192 930 and 788.  What bounds that is the loads: 16 bytes of every row and half per lane are 100 cycles of the
-// address unit each (busy 85 % of the launch), and rows are visited 136 bytes at a time, 1.6 times the lines that they have.
+// us, general kernel and this one (3072 x 768, 512 experts): routed Q8_0 down, 2000 tokens 541 and 423, 4096 (skewed) 656 and 538,
+// 8192 (skewed / even) 938 / 1065 and 767 / 806; the Q8_0 shared expert's two launches beside the router's, 4096 tokens 92 + 66 and 84
+// + 45, 8192 219 + 87 and 137 + 120; layers with a q8g32 shared expert, 2560 x 640 2000 tokens 614 and 594, 3072 x 768 of 64 experts
+// 130 tokens 219 and 155; all-Q8_0 layers 130 tokens 1460 and 1062, 2000 1755 and 1323, 8192 3600 and 2727.  What bounds it is the
+// loads: 16 bytes of every row and half per lane are 100 cycles of the address unit each (busy 85 % of the launch), and rows are
+// visited 136 bytes at a time, 1.6 times the lines that they have.  (Few blocks: moe_wide_takes.)
 // (All of a stage's loads in a row instead of half of them half a stage later, so that a line's second load finds it in L1:
 // 466 -> 427; two stages in registers instead of one, by itself: no change.)
 #include <type_traits>
@@ -279,7 +281,7 @@ __device__ __forceinline__ void wide_tile(uint8_t* smem, const WideW& L, int e, 
     };
     if constexpr (!UP) {
       // sixteen pairs at a time through the wave's patch, so that eight lanes store a line: as 16-byte pieces of 64 lines the
-      // stores took the address unit 64 cycles each (8192 tokens 835 -> 814 us, 4096 543 -> 541)
+      // stores took the address unit 64 cycles each (8192 tokens, even, 835 -> 814 us; 4096, skewed, level)
       uint32_t ln = lane;
       asm volatile("" : "+v"(ln));  // (opaque: addresses made here instead of held through the stages)
       uint8_t* const patch = smem + 2 * XBUF + wv * 16 * PROW;
