@@ -1038,7 +1038,9 @@ int moe_stream_tile_cap(int P, int k, int experts, int fmt_up, int fmt_dn, int d
   float line;
   if (once_rounded(fmt_up)) line = ONCE_LINE;
   else if (small && lone) line = !five ? 28.f : experts >= 64 ? 26.f : 32.f;
-  else if (small) line = weights >= (int64_t)3 << 27 ? (five ? 29.f : 31.f) : weights >= 1 << 25 ? (five ? 22.f : 26.f) : five && experts >= 64 ? 31.f : 38.f;
+  else if (small && weights >= (int64_t)3 << 27) line = five ? 29.f : 31.f;
+  else if (small && weights >= 1 << 25) line = five ? 22.f : 26.f;
+  else if (small) line = five && experts >= 64 ? 31.f : 38.f;
   else if (fmt_up == F_TAB) line = lone ? 29.f : big ? 70.f : 60.f;
   else line = lone ? 25.f : !big ? 50.f : fmt_up == F_DN || fmt_up == F_AFF ? 62.f : 60.f;
   if (avg <= 10.f) return 16;

@@ -425,8 +425,9 @@ bool moe_wide_takes(bool up, int type, const uint8_t* w, const uint8_t* w_up, in
   for (const uint8_t* p : {w, up ? w_up : w, sh_w ? sh_w : w, sh_w && up ? sh_w_up : w})
     if (!moe_aligned(p, al)) return false;
   if (k % 128 || m % (up ? 32 : 64)) return false;
-  // Q8_0 on few blocks: the general kernel has twice as many, and there the tile's weights take less of a wave's time.  (q8g32: it
-  // has no such form, and takes 25 .. 45 % longer at any size.)  us of a layer, here and there, Q5_K / Q8_0, Q8_0 shared expert:
+  // Q8_0 on few blocks: the launch takes as long as a block does, and the general kernel's have half the rows.  (q8g32: it has no
+  // pipelined form for that, a layer takes up to 45 % longer with it and is level at best.)  us of a layer, here and there, Q5_K /
+  // Q8_0 with a Q8_0 shared expert:
   //   up to four tiles of more than 64 tokens   3072 x 768 of 16 experts 130 138 125, 300 155 130, 400 163 141, 515 (five) 154 149; of
   //     32 130 150 135, 400 181 161, 700 (six) 214 221; of 64 256 216 190, 700 243 274; of 128 400 340 333, 1000 (eight) 381 397
   //   one tile of at most 64, next to a launch of many weights   3072 x 768 of 64 (151 M) 33 185 167, 64 189 171; 2048 x 1536 of 64 191
