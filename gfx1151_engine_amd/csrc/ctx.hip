@@ -46,7 +46,10 @@ static int codebook_affine(const moe_wview* w, bool* out) {
 }
 
 struct moe_ctx;
-static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_wview* a, const moe_wview* b, int n_experts, bool* all);
+static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_lutw* a, const moe_lutw* b, int kq, int rows, int cols,
+                         int n_experts, bool* all);
+static int pexp_register_gguf(moe_ctx* c, int layer, int slot0, int type, const uint8_t* a, const uint8_t* b, int rows, int cols,
+                              int n_experts, bool* all);
 static int magnitude_constant(moe_ctx* c, int tgu, int tdn, const moe_wview* gate, uint64_t gate_stride,
                               const moe_wview* up, uint64_t up_first, const moe_wview* down, int n_experts,
                               moe_cmag* out);
@@ -139,30 +142,42 @@ struct moe_ctx {
 static int8_t* pexp_slot(moe_ctx* c, int layer, int slot0) {
   return c->pexp ? c->pexp + (size_t)layer * (2 * (size_t)c->cfg.experts + 2) + slot0 : nullptr;
 }
-// *all: every expert has one.
-static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_wview* a, const moe_wview* b, int n_experts, bool* all) {
+// rows, cols: of one expert; kq as for moe_scale_span.  *all: every expert has one.
+static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_lutw* a, const moe_lutw* b, int kq, int rows, int cols,
+                         int n_experts, bool* all) {
   *all = false;
   int8_t* dst = pexp_slot(c, layer, slot0);
   if (!dst) return MOE_OK;  // contexts for small batches only have no grouped GEMM
   std::vector<int8_t> out((size_t)n_experts, (int8_t)MOE_PEXP_NONE);
   if (a) {
     std::vector<int8_t> sa((size_t)2 * n_experts), sb;
-    int rc = moe_q4cp_scale_span(a, n_experts, c->span_tmp, nullptr);
+    int rc = moe_scale_span(a, kq, n_experts, rows, cols, c->span_tmp, nullptr);
     if (rc) return rc;
     MOE_HIP(hipMemcpy(sa.data(), c->span_tmp, sa.size(), hipMemcpyDeviceToHost));
     if (b) {
       sb.resize(sa.size());
-      if ((rc = moe_q4cp_scale_span(b, n_experts, c->span_tmp, nullptr))) return rc;
+      if ((rc = moe_scale_span(b, kq, n_experts, rows, cols, c->span_tmp, nullptr))) return rc;
       MOE_HIP(hipMemcpy(sb.data(), c->span_tmp, sb.size(), hipMemcpyDeviceToHost));
     }
     *all = true;
     for (int e = 0; e < n_experts; e++) {
-      out[e] = (int8_t)moe_pexp_from_span(&sa[2 * e], b ? &sb[2 * e] : nullptr);
+      out[e] = (int8_t)moe_pexp_from_span(&sa[2 * e], b ? &sb[2 * e] : nullptr, kq >= 144);
       *all = *all && out[e] != (int8_t)MOE_PEXP_NONE;
     }
   }
   MOE_HIP(hipMemcpy(dst, out.data(), out.size(), hipMemcpyHostToDevice));
   return MOE_OK;
+}
+
+// Raw GGUF rows: of the types that gemm_q4cp.hip takes, Q4_K has the form (Q5_K's fifth bits leave no registers for it: 739 us
+// without and 750 with it, gate/up at 4096 tokens)
+static int pexp_register_gguf(moe_ctx* c, int layer, int slot0, int type, const uint8_t* a, const uint8_t* b, int rows, int cols,
+                              int n_experts, bool* all) {
+  const bool ok = type == MOE_GGML_Q4_K && cols % 256 == 0 && moe_aligned(a, 16) && (!b || moe_aligned(b, 16));
+  moe_lutw va{}, vb{};
+  va.w = a;
+  vb.w = b;
+  return pexp_register(c, layer, slot0, ok ? &va : nullptr, b ? &vb : nullptr, 144, rows, cols, n_experts, all);
 }
 
 static void prof_mark(moe_ctx* c, int stage_done, hipStream_t st) {
@@ -344,8 +359,11 @@ MOE_API int moe_set_experts_q4cp(moe_ctx* c, int layer, const moe_wview* gu, con
   L->experts_affine = a1 && a2;
   if ((rc = magnitude_constant(c, 0, 0, gu, (uint64_t)2 * g.mid, gu, (uint64_t)g.mid, dn, g.experts, &L->c_routed)))
     return rc;
-  if ((rc = pexp_register(c, layer, 0, a1 ? gu : nullptr, nullptr, g.experts, &L->scaled_gu)) ||
-      (rc = pexp_register(c, layer, g.experts, a2 ? dn : nullptr, nullptr, g.experts, &L->scaled_dn)))
+  moe_lutw vg, vd;
+  moe_lut_q4cp_view(gu->data, gu->rows, gu->cols, gu->scale_stride, 2 * g.mid, g.mid, &vg);
+  moe_lut_q4cp_view(dn->data, dn->rows, dn->cols, dn->scale_stride, g.d, 0, &vd);
+  if ((rc = pexp_register(c, layer, 0, a1 ? &vg : nullptr, nullptr, 32, 2 * g.mid, g.d, g.experts, &L->scaled_gu)) ||
+      (rc = pexp_register(c, layer, g.experts, a2 ? &vd : nullptr, nullptr, 32, g.d, g.mid, g.experts, &L->scaled_dn)))
     return rc;
   L->gate_up = *gu;
   L->down = *dn;
@@ -393,6 +411,14 @@ MOE_API int moe_set_experts_i4r(moe_ctx* c, int layer, const moe_wview* gu, cons
       return (int)e;
     }
   }
+  {
+    moe_lutw vg, vd;
+    int rc = moe_lut_i4r_view(gu->data, gu->rows, gu->cols, 2 * g.mid, g.mid, &vg);
+    if (!rc) rc = moe_lut_i4r_view(dn->data, dn->rows, dn->cols, g.d, 0, &vd);
+    if (!rc) rc = pexp_register(c, layer, 0, &vg, nullptr, 128, 2 * g.mid, g.d, g.experts, &L->scaled_gu);
+    if (!rc) rc = pexp_register(c, layer, g.experts, &vd, nullptr, 128, g.d, g.mid, g.experts, &L->scaled_dn);
+    if (rc) return rc;
+  }
   L->gate_up = *gu;
   L->down = *dn;
   L->v2_su = su; L->v2_svh_gu = svh_gu; L->v2_suh_dn = suh_dn; L->v2_svh_dn = svh_dn;
@@ -426,6 +452,9 @@ MOE_API int moe_set_experts_gguf(moe_ctx* c, int layer, const moe_gg_experts* gg
     moe_wview dv{0, gg->down, (uint64_t)g.experts * g.d, (uint64_t)g.mid, 0};
     int rc = magnitude_constant(c, gg->tgu, gg->tdn, &gv, (uint64_t)g.mid, &uv, 0, &dv, g.experts, &L->c_routed);
     if (rc) return rc;
+    if ((rc = pexp_register_gguf(c, layer, 0, gg->tgu, gg->gate, gg->up, g.mid, g.d, g.experts, &L->scaled_gu)) ||
+        (rc = pexp_register_gguf(c, layer, g.experts, gg->tdn, gg->down, nullptr, g.d, g.mid, g.experts, &L->scaled_dn)))
+      return rc;
   }
   L->gg = *gg;
   L->has_gguf = true;
@@ -459,13 +488,18 @@ MOE_API int moe_set_shared(moe_ctx* c, int layer, const moe_wview* g, const moe_
     int rc;
     if ((rc = codebook_affine(g, &a1)) || (rc = codebook_affine(u, &a2)) || (rc = codebook_affine(dn, &a3))) return rc;
     L->shared_affine = a1 && a2 && a3;
-    if ((rc = pexp_register(c, layer, 2 * cf.experts, a1 && a2 ? g : nullptr, u, 1, &L->scaled_sgu)) ||
-        (rc = pexp_register(c, layer, 2 * cf.experts + 1, a3 ? dn : nullptr, nullptr, 1, &L->scaled_sdn)))
+    moe_lutw vg, vu, vd;
+    moe_lut_q4cp_view(g->data, g->rows, g->cols, g->scale_stride, cf.mid, 0, &vg);
+    moe_lut_q4cp_view(u->data, u->rows, u->cols, u->scale_stride, cf.mid, 0, &vu);
+    moe_lut_q4cp_view(dn->data, dn->rows, dn->cols, dn->scale_stride, cf.d, 0, &vd);
+    if ((rc = pexp_register(c, layer, 2 * cf.experts, a1 && a2 ? &vg : nullptr, &vu, 32, cf.mid, cf.d, 1, &L->scaled_sgu)) ||
+        (rc = pexp_register(c, layer, 2 * cf.experts + 1, a3 ? &vd : nullptr, nullptr, 32, cf.d, cf.mid, 1, &L->scaled_sdn)))
       return rc;
   } else {
+    const int t = dense ? 0 : sh_gguf_type;
     int rc;
-    if ((rc = pexp_register(c, layer, 2 * cf.experts, nullptr, nullptr, 1, &L->scaled_sgu)) ||
-        (rc = pexp_register(c, layer, 2 * cf.experts + 1, nullptr, nullptr, 1, &L->scaled_sdn)))
+    if ((rc = pexp_register_gguf(c, layer, 2 * cf.experts, t, g->data, u->data, cf.mid, cf.d, 1, &L->scaled_sgu)) ||
+        (rc = pexp_register_gguf(c, layer, 2 * cf.experts + 1, t, dn->data, nullptr, cf.d, cf.mid, 1, &L->scaled_sdn)))
       return rc;
   }
   L->c_shared = moe_cmag{0.f, 0.f};
@@ -1024,7 +1058,8 @@ static StreamKinds stream_kinds(const MoeLayer& L, const moe_config& g) {
   StreamKinds k{-1, -1, false};
   const bool q4sh = L.has_shared && !L.sh_dense && L.sh_gguf_type == 0;
   if (L.has_i4r) {
-    k.up = k.dn = MOE_STREAM_I4R;
+    k.up = L.scaled_gu ? MOE_STREAM_I4R_SCALED : MOE_STREAM_I4R;
+    k.dn = L.scaled_dn ? MOE_STREAM_I4R_SCALED : MOE_STREAM_I4R;
   } else if (L.has_q4cp) {
     // (affine experts beside a table-coded shared expert, which is possible and unusual: one launch, one format)
     if (L.experts_affine && q4sh && !L.shared_affine) return k;
@@ -1109,8 +1144,8 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   const __half* xh = c->x16_ext ? c->x16_ext : c->x16;  // f16 activations in the GEMM's order
   int xl = cap ? sxl : batch_x16_layout(L, g);  // that order (moe_f32_to_f16's layout)
   const bool nat = batch_nat(L);               // table codebooks: natural K order, pair tables
-  // scaled dequantisation (affine q4cp codebooks): the powers of two found when the weights were registered
-  const bool pe_r = L.has_q4cp && !v2 && L.experts_affine, pe_s = L.has_shared && !shd && !q4k && L.shared_affine;
+  // scaled dequantisation (affine codebooks, Q4_K): the powers of two found when the weights were registered
+  const bool pe_r = L.experts_affine || L.has_gguf, pe_s = L.has_shared && !shd && (q4k || L.shared_affine);
   const int8_t* pe_gu = pe_r ? pexp_slot(c, (int)(&L - c->layers.data()), 0) : nullptr;
   const int8_t* pe_dn = pe_r ? pexp_slot(c, (int)(&L - c->layers.data()), g.experts) : nullptr;
   const int8_t* pe_sgu = pe_s ? pexp_slot(c, (int)(&L - c->layers.data()), 2 * g.experts) : nullptr;
@@ -1138,7 +1173,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
       if (with_sh ? kd.s_gu : kd.r_gu)
         return moe_launch_gemm_q4cp(true, with_sh ? &sgu : &gu, with_sh ? &sgu : nullptr, g.experts, xh, c->tokidx, tl, ntl,
                                     mt, c->hid16, g.mid, g.d, true, true, hs, s2, nullptr, nullptr, 0,
-                                    (with_sh ? L.sh_gguf_type : L.gg.tgu) == MOE_GGML_Q5_K);
+                                    (with_sh ? L.sh_gguf_type : L.gg.tgu) == MOE_GGML_Q5_K, false, with_sh ? pe_sgu : pe_gu, pe_sgu);
       return with_sh ? moe_launch_gemm_gg(true, L.sh_gguf_type, L.sh_gate.data, L.sh_up.data, L.sh_gguf_type,
                                           L.sh_gate.data, L.sh_up.data, g.experts, xh, c->tokidx, tl, ntl, mt, c->hid16,
                                           g.mid, g.d, hs, s2, xl, P, true)
@@ -1157,11 +1192,12 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
         gf.up_off = g.mid;
         const moe_rotv rv{L.v2_svh_gu, L.v2_suh_dn};
         return moe_launch_gemm_q4cp(true, &gf, nullptr, g.experts, c->v2_x16, c->tokidx, tl, ntl, mt, c->hid16, g.mid, g.d,
-                                    true, false, hs, s2, nullptr, nullptr, 2, false, false, nullptr, nullptr, &rv);
+                                    true, false, hs, s2, nullptr, nullptr, 2, false, false, pe_gu, nullptr, &rv);
       }
       // (the earlier form: plain rows of the fused tensor as f16 sums, then the middle as a launch of its own)
       const int e = moe_launch_gemm_q4cp(false, &gu, nullptr, g.experts, c->v2_x16, c->tokidx, tl, ntl, mt, c->v2_z16,
-                                         2 * g.mid, g.d, true, false, moe_hscale{nullptr, 0.f, 0.f}, s2, nullptr, nullptr, 2);
+                                         2 * g.mid, g.d, true, false, moe_hscale{nullptr, 0.f, 0.f}, s2, nullptr, nullptr, 2,
+                                         false, false, pe_gu);
       return e || dry ? e : moe_launch_i4r_mid(c->v2_z16, true, (uint64_t)2 * g.mid, P * g.topk, g.mid, L.v2_svh_gu, L.v2_suh_dn,
                                         1, c->hid16, (uint64_t)g.mid, 1, 1, nullptr, nullptr, s2, c->xms, L.c_routed, c->tokidx);
     }
@@ -1184,7 +1220,8 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
       // (hid rows are in the tuned kernel's order where its gate/up form wrote them, else in natural order)
       if (with_sh ? kd.s_dn : kd.r_dn)
         return moe_launch_gemm_q4cp(false, with_sh ? &sdn : &dn, with_sh ? &sdn : nullptr, g.experts, c->hid16, nullptr, tl,
-                                    ntl, mt, c->pairs16, g.d, g.mid, true, true, hs, s2, nullptr);
+                                    ntl, mt, c->pairs16, g.d, g.mid, true, true, hs, s2, nullptr, nullptr, 0, false, false,
+                                    with_sh ? pe_sdn : pe_dn, pe_sdn);
       return with_sh ? moe_launch_gemm_gg(false, L.sh_gguf_type, L.sh_down.data, nullptr, L.sh_gguf_type, L.sh_down.data,
                                           nullptr, g.experts, c->hid16, nullptr, tl, ntl, mt, c->pairs16, g.d, g.mid, hs, s2,
                                           kd.s_gu ? 2 : 0, P, true)
@@ -1197,7 +1234,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
                                 kd.r_gu ? 2 : 0, routed ? each : P, !routed);
     if (v2 && !with_sh)
       return moe_launch_gemm_q4cp(false, &dn, nullptr, g.experts, c->hid16, nullptr, tl, ntl, mt, c->pairs16, g.d, g.mid,
-                                  true, false, moe_hscale{nullptr, 0.f, 0.f}, s2, nullptr, nullptr, 2);
+                                  true, false, moe_hscale{nullptr, 0.f, 0.f}, s2, nullptr, nullptr, 2, false, false, pe_dn);
     if (v2)
       return moe_launch_gemm_q4cp(false, &sdn, &sdn, g.experts, c->hid16, nullptr, tl, ntl, mt, c->pairs16, g.d, g.mid,
                                   true, false, hs, s2, nullptr, nullptr, 0, false, false, pe_sdn, pe_sdn);

@@ -51,9 +51,13 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // F_DN: affine q4cp codebooks whose experts all have a power of two for the scaled dequantisation (gemm_q4cp.hip, DN)
 // F_Q4E, F_Q5E: Q4_K and Q5_K weights rounded to f16 once, from their exact values
-enum { F_DN, F_AFF, F_TAB, F_I4R, F_Q4K, F_Q5K, F_Q80, F_Q4E, F_Q5E };
+// F_I4D: i4r with the scaled dequantisation (3001 skewed tokens, gate/up 509 -> 459 us, down 284 -> 266; 130: 239 -> 227, 134 -> 129.
+// Q4_K gained half a per cent of a layer with it and Q5_K lost 15 at 1200 tokens, both short of registers.)
+enum { F_DN, F_AFF, F_TAB, F_I4D, F_I4R, F_Q4K, F_Q5K, F_Q80, F_Q4E, F_Q5E };
 constexpr bool q4(int FMT) { return FMT == F_Q4K || FMT == F_Q4E; }
 constexpr bool q5(int FMT) { return FMT == F_Q5K || FMT == F_Q5E; }
+constexpr bool i4(int FMT) { return FMT == F_I4D || FMT == F_I4R; }
+constexpr bool scaled(int FMT) { return FMT == F_DN || FMT == F_I4D; }
 constexpr bool once_rounded(int FMT) { return FMT == F_Q4E || FMT == F_Q5E; }
 constexpr bool scale_plane(int FMT) { return FMT <= F_I4R; }
 // order of activations and hid (moe_f32_to_f16's layouts)
@@ -220,7 +224,7 @@ __device__ __forceinline__ void line_mma(const Line<FMT> (&q)[F], const uint32_t
             const float s = (float)s2.x;
             as[f][0] = both(C.cb_a[f0 + f] * s);
             bs[f][0] = bs[f][1] = both(C.cb_b[f0 + f] * s);
-            as[f][1] = FMT == F_DN ? as[f][0] * both(0.0625f) : as[f][0];
+            as[f][1] = scaled(FMT) ? as[f][0] * both(0.0625f) : as[f][0];
           }
         }
       }
@@ -239,7 +243,7 @@ __device__ __forceinline__ void line_mma(const Line<FMT> (&q)[F], const uint32_t
             continue;
           }
           const uint32_t w8 = w >> 8;
-          if (FMT == F_DN) {  // codes read as f16 denormals
+          if (scaled(FMT)) {  // codes read as f16 denormals
             a[f].h[0] = h2(w & 0x000f000fu) * as[f][0] + bs[f][0];
             a[f].h[1] = h2(w & 0x00f000f0u) * as[f][1] + bs[f][0];
             a[f].h[2] = h2(w8 & 0x000f000fu) * as[f][0] + bs[f][0];
@@ -371,7 +375,7 @@ struct Raw { uint4 v; };
 template <int FMT>
 __device__ __forceinline__ Raw<FMT> load_scales(const uint8_t* b, uint32_t o, int first, int g, int sstride) {
   Raw<FMT> r;
-  if (FMT == F_I4R) {  // one word per line: both scales, the same for all lane groups
+  if (i4(FMT)) {  // one word per line: both scales, the same for all lane groups
     const uint32_t p = 4u * (uint32_t)(first + g);
     r.v.x = *(const uint32_t*)(b + (p < (uint32_t)sstride ? o + p : 0u));
   } else {
@@ -383,7 +387,7 @@ __device__ __forceinline__ Raw<FMT> load_scales(const uint8_t* b, uint32_t o, in
 template <int FMT>
 __device__ __forceinline__ void take_scales(const Raw<FMT>& r, uint32_t (&sq)[4]) {
   uint32_t p0 = r.v.x, p1 = p0, p2 = p0, p3 = p0;
-  if (FMT != F_I4R) {  // word k: (scale k, scale 4 + k), lane group k's chunks k and k + 4
+  if (!i4(FMT)) {  // word k: (scale k, scale 4 + k), lane group k's chunks k and k + 4
     p0 = __builtin_amdgcn_perm(r.v.z, r.v.x, 0x05040100u); p1 = __builtin_amdgcn_perm(r.v.z, r.v.x, 0x07060302u);
     p2 = __builtin_amdgcn_perm(r.v.w, r.v.y, 0x05040100u); p3 = __builtin_amdgcn_perm(r.v.w, r.v.y, 0x07060302u);
   }
@@ -427,10 +431,12 @@ __device__ __forceinline__ Consts make_consts(const SW& L, int pexp, const TabEn
   C.tabs = tabs;
   C.tabo[0] = C.tabo[1] = 0u;
   oscale = 1.f;
-  if (FMT == F_AFF || FMT == F_DN) {
-    C.cb_a[0] = L.cb[1] - L.cb[0]; C.cb_b[0] = L.cb[0];
-    C.cb_a[1] = UP ? L.cb_up[1] - L.cb_up[0] : C.cb_a[0]; C.cb_b[1] = UP ? L.cb_up[0] : C.cb_b[0];
-    if (FMT == F_DN) {  // in units of 2^pexp; slopes for codes read as f16 denormals
+  if (FMT == F_AFF || scaled(FMT)) {
+    if (FMT != F_I4D) {
+      C.cb_a[0] = L.cb[1] - L.cb[0]; C.cb_b[0] = L.cb[0];
+      C.cb_a[1] = UP ? L.cb_up[1] - L.cb_up[0] : C.cb_a[0]; C.cb_b[1] = UP ? L.cb_up[0] : C.cb_b[0];
+    }
+    if (scaled(FMT)) {  // in units of 2^pexp; slopes for codes read as f16 denormals
       const float s24 = __builtin_ldexpf(1.f, 24 + pexp), sp = __builtin_ldexpf(1.f, pexp);
       C.cb_a[0] *= s24; C.cb_a[1] *= s24; C.cb_b[0] *= sp; C.cb_b[1] *= sp;
       oscale = __builtin_ldexpf(1.f, -pexp);
@@ -692,7 +698,7 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
 #pragma unroll
         for (int r4 = 0; r4 < 4; r4++) {
           const int c = pos_elem<LAYOUT>(wv, 4 * g + r4);
-          *(__half*)(patch + (16 * mf + n) * BP + f * UPR * 2 + c * 2) = __float2half(acc[f][mf][r4]);
+          *(__half*)(patch + (16 * mf + n) * BP + f * UPR * 2 + c * 2) = __float2half(acc[f][mf][r4] * oscale);
         }
     __syncthreads();
     const int j = tid & 15, c = nb * UPR + 8 * j;
@@ -879,7 +885,7 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
 // four, eight and sixteen there, q4cp, 2048 x 1536: 130 tokens 585, 620, 621, with 32 pairs to a tile 515 tokens 779, 749, 740, 800
 // 880, 805, 792; 3072 x 512: 515 tokens 401, 404, 435).
 constexpr int DN_ONE = 3;  // lines of the rows that a wave takes whole
-constexpr int up_waves(int FMT, int MFX) { return MFX == 4 || FMT == F_I4R ? 8 : 4; }
+constexpr int up_waves(int FMT, int MFX) { return MFX == 4 || i4(FMT) ? 8 : 4; }
 // waves per SIMD asked for: what the registers of the lines in flight leave.  (Gate/up with Q5_K rounded once, 32 pairs: three; with
 // four 21 registers went to scratch inside the loop, 757 us for 702 at 1200 tokens of 2560 x 640.  A few kernels keep 1 .. 4
 // registers of their prologue in scratch until the epilogue, F_DN's down launch with 64 pairs an address once per pass:
@@ -934,13 +940,13 @@ k_moe_stream(SW R, SW Sh, int n_experts, const __half* __restrict__ x, const int
   L.up_off = shared ? Sh.up_off : R.up_off;
   L.pexp = shared ? Sh.pexp : R.pexp;
   const int e = shared ? 0 : tile.expert;
-  const int pexp = FMT == F_DN ? (int)L.pexp[e] : 0;
+  const int pexp = scaled(FMT) ? (int)L.pexp[e] : 0;
   const moe_cmag cmag = shared ? hs.c_shared : hs.c_routed;
   const int mfn = (tile.count + 15) >> 4;
   const bool two_tabs = R.cb != R.cb_up || Sh.cb != Sh.cb_up;  // (launch)
 #define ST_GO(MF)                                                                                              \
   do {                                                                                                         \
-    if constexpr (UP) up_tile<FMT, MFX, MF, FMT == F_I4R, NW>(smem, L, e, tile, nb, x, tokidx, out, M, K, pexp, hs, cmag, rot, two_tabs); \
+    if constexpr (UP) up_tile<FMT, MFX, MF, i4(FMT), NW>(smem, L, e, tile, nb, x, tokidx, out, M, K, pexp, hs, cmag, rot, two_tabs); \
     else dn_tile<FMT, MFX, MF, NW, LN, LN == DN_ONE>(smem, L, e, tile, nb, npass, x, out, M, K, pexp);                           \
   } while (0)
   // (33 .. 48 pairs as three groups instead of four: 2048 tokens q4cp, 755 -> 720 us a layer)
@@ -1058,27 +1064,27 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
                       moe_hscale hs, hipStream_t st, const float* sh_cb_up, const int8_t* pexp_routed,
                       const int8_t* pexp_sh, const moe_rotv* rot) {
   if (!x || !tiles || !ntiles || !out || max_tiles < 0 || !routed || (up && !tokidx)) return MOE_E_INVALID;
-  const bool plane = fmt <= F_I4R;
+  const bool plane = scale_plane(fmt);
   auto ok = [&](const moe_lutw* p) {
     if (!p->w || (up && !p->w_up)) return false;
     if (!moe_aligned(p->w, fmt == F_Q80 ? 4 : 16) || (up && !moe_aligned(p->w_up, 16))) return false;
     if (plane) {
-      const int a = fmt == F_I4R ? 4 : 16;
-      if (!p->sc || !p->cb || !moe_aligned(p->sc, a) || p->sstride % a || p->sstride < k / (fmt == F_I4R ? 128 : 32) * 2) return false;
+      const int a = i4(fmt) ? 4 : 16;
+      if (!p->sc || !p->cb || !moe_aligned(p->sc, a) || p->sstride % a || p->sstride < k / (i4(fmt) ? 128 : 32) * 2) return false;
       if (up && (!p->sc_up || !moe_aligned(p->sc_up, a))) return false;
     }
     return true;
   };
   if (!ok(routed) || (sh && !ok(sh))) return MOE_E_UNSUPPORTED;
-  if (k % 128 || ((q4(fmt) || q5(fmt) || fmt == F_I4R) && k % 256)) return MOE_E_UNSUPPORTED;
+  if (k % 128 || ((q4(fmt) || q5(fmt) || i4(fmt)) && k % 256)) return MOE_E_UNSUPPORTED;
   // (down: groups of 32 rows, and a tile's hid rows in LDS)
   if (up && (uint64_t)x_rows * (uint64_t)k * 2 >= 1ull << 32) return MOE_E_UNSUPPORTED;  // (32-bit byte offsets into x)
   if (up ? k < 256 : k < 128 || m % 32 || smem_bytes(fmt, false, cap / 16, (k + 255) / 256, 1) > LDS_MOST) return MOE_E_UNSUPPORTED;
-  if (up && (m % 16 || (fmt >= F_Q4K && m % 64) || (fmt == F_I4R && m % 128))) return MOE_E_UNSUPPORTED;
+  if (up && (m % 16 || (fmt >= F_Q4K && m % 64) || (i4(fmt) && m % 128))) return MOE_E_UNSUPPORTED;
   if ((up && fmt == F_Q80) || (!up && (q5(fmt) || once_rounded(fmt))) || (cap > 32 && (q5(fmt) || fmt == F_Q80))) return MOE_E_UNSUPPORTED;
-  if (fmt == F_I4R && up != (rot != nullptr)) return MOE_E_INVALID;
+  if (i4(fmt) && up != (rot != nullptr)) return MOE_E_INVALID;
   if (rot && (!rot->svh_gu || !rot->suh_dn)) return MOE_E_INVALID;
-  if (fmt == F_DN && (!pexp_routed || (sh && !pexp_sh))) return MOE_E_INVALID;
+  if (scaled(fmt) && (!pexp_routed || (sh && !pexp_sh))) return MOE_E_INVALID;
   if (!moe_aligned(x, 16) || !moe_aligned(out, 16)) return MOE_E_INVALID;
   if (max_tiles == 0) return MOE_OK;
   const SW R = to_dev(routed, nullptr, pexp_routed), S = to_dev(sh ? sh : routed, sh ? sh_cb_up : nullptr, sh ? pexp_sh : pexp_routed);
@@ -1117,6 +1123,7 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
     case F_DN: ST_DIR(F_DN);
     case F_AFF: ST_DIR(F_AFF);
     case F_TAB: ST_DIR(F_TAB);
+    case F_I4D: ST_DIR(F_I4D);
     case F_I4R: ST_DIR(F_I4R);
     case F_Q4K: ST_DIR(F_Q4K);
     case F_Q5K: ST_UP(F_Q5K);

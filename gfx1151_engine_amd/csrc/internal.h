@@ -78,7 +78,7 @@ int moe_launch_gemm_q4cp(bool up, const moe_lutw* routed, const moe_lutw* sh, in
                          bool q5k = false, bool nat = false, const int8_t* pexp_routed = nullptr,
                          const int8_t* pexp_sh = nullptr, const moe_rotv* rot = nullptr);
 // Grouped GEMM for tiles of few pairs, weights streamed into registers (gemm_stream.hip)
-enum { MOE_STREAM_SCALED, MOE_STREAM_AFFINE, MOE_STREAM_TABLE, MOE_STREAM_I4R, MOE_STREAM_Q4K, MOE_STREAM_Q5K, MOE_STREAM_Q8_0,
+enum { MOE_STREAM_SCALED, MOE_STREAM_AFFINE, MOE_STREAM_TABLE, MOE_STREAM_I4R_SCALED, MOE_STREAM_I4R, MOE_STREAM_Q4K, MOE_STREAM_Q5K, MOE_STREAM_Q8_0,
        MOE_STREAM_Q4K_ONCE, MOE_STREAM_Q5K_ONCE };
 int moe_stream_tile_cap(int P, int k, int experts, int fmt_up, int fmt_dn, int d, int mid);
 int moe_stream_tile_cap_least(int P, int k, int experts);
@@ -86,14 +86,15 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
                       const int* tokidx, const moe_tile* tiles, const int* ntiles, int max_tiles, __half* out, int m, int k,
                       moe_hscale hs, hipStream_t st, const float* sh_cb_up = nullptr, const int8_t* pexp_routed = nullptr,
                       const int8_t* pexp_sh = nullptr, const moe_rotv* rot = nullptr);
-// Scaled dequantisation of the grouped GEMM (affine q4cp codebooks): per expert the power of two P with
-// |cb slope| * (largest scale of the expert) * 2^(24+P) in [2^14, 2^15), or MOE_PEXP_NONE where the form does not apply
-// (a scale that is not finite, a zero slope, rows whose largest scale lies more than 2^5 below the expert's: their
-// weights would fall into the f16 denormals of the scaled units).  moe_q4cp_scale_span fills one (hi, lo) pair of
-// exponents per expert for a tensor; moe_pexp_from_span combines the spans of the tensors one launch reads.
+// Scaled dequantisation of the grouped GEMMs (affine q4cp codebooks, i4r, Q4_K): per expert the power of two P with
+// |cb slope| * (largest scale of the expert) * 2^(24+P) in [2^15, 2^16), or MOE_PEXP_NONE where the form does not apply
+// (a scale that is not finite, a zero slope, rows whose largest scale lies more than 2^6 below the expert's: their
+// weights would fall into the f16 denormals of the scaled units).  moe_scale_span fills one (hi, lo) pair of exponents per
+// expert for a tensor; moe_pexp_from_span combines the spans of the tensors one launch reads.
 constexpr int MOE_PEXP_NONE = -128;
-int moe_q4cp_scale_span(const moe_wview* w, int n_experts, int8_t* span_dev, hipStream_t st);
-int moe_pexp_from_span(const int8_t* hi_lo_a, const int8_t* hi_lo_b);
+// kq: columns per scale of the view's scale plane (32, 128), or the bytes of a K-quant block (144)
+int moe_scale_span(const moe_lutw* w, int kq, int n_experts, int rows, int cols, int8_t* span_dev, hipStream_t st);
+int moe_pexp_from_span(const int8_t* hi_lo_a, const int8_t* hi_lo_b, bool kq);
 // The Q5_K form addresses weights and activations with 32-bit byte offsets: true when a tensor of `rows` rows of k
 // columns and an activation buffer of `x_rows` rows of k f16 values both stay below 4 GB (the caller of
 // moe_launch_gemm_q4cp(q5k = true) checks it; other layers take the general kernel)
