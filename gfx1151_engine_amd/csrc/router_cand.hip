@@ -12,7 +12,7 @@
 //                     [a_e - B_e, a_e + B_e] that holds the exact logit; tau = the k-th largest lower end; every expert whose
 //                     upper end reaches tau - 1e-5 is a candidate (the true top k are among them: at least k exact logits are
 //                     >= tau, and a true top-k logit is >= the k-th largest exact one).  The candidates' logits (typically
-//                     12-18 of 512) are taken as fp64 dot products, in another order than the reference's sequential one:
+//                     10-12 of 512) are taken as fp64 dot products, in another order than the reference's sequential one:
 //                     the reference's float, or in rare cases (a rounding boundary within tol of the sum) its neighbour.  If
 //                     every gap between neighbours among the k + 1 best exceeds what can make two probabilities round to one
 //                     float, plus two ulps where a logit is in doubt, and all lie within 70 of the maximum, the order by
@@ -22,16 +22,20 @@
 //                     underflow, more candidates than slots, non-finite values) are listed; rows of zeros (padding) are
 //                     settled by their block, which knows their sums;
 //   4. k_router_listed  listed tokens, sixteen at a time, as the reference's chains on the f64 matrix pipe.
-// Error bound.  a~ = fl32(sum of f16(x_c) * f16(w_c)): |f16(v) - v| <= 2^-11 |v| + 2^-25 (the second term covers
-// f16 subnormals), so sum |x~ w~ - x w| <= 1.001 (2^-10 |x||w| + 2^-25 sqrt(d) (|x| + |w|)) by Cauchy-Schwarz, and
-// the accumulation adds at most (RA_CHUNK * 2^-22 + (d / RA_CHUNK + RA_KS) * 2^-23) * 1.001 |x||w|: inside a chunk of RA_CHUNK
+// Error bound.  a~ = fl32(sum of x~_c * w~_c) with x~ = f16(x), w~ = f16(w).  |x.w - x~.w~| <= |x - x~||w| + |x~||w - w~| by
+// Cauchy-Schwarz; prep, which makes the copies, leaves the norms of what their rounding changed (a bound from the format alone,
+// 2^-10 |x||w|, is five times as wide for an f32 router beside activations that came from bf16, thirty times where the router
+// is bf16 too and nothing rounds: 13 candidates of 512 instead of 10.8 and 10.1).  The accumulation adds at most (RA_CHUNK *
+// 2^-22 + (d / RA_CHUNK + RA_KS) * 2^-23) * 1.001 |x~||w~|: inside a chunk of RA_CHUNK
 // columns however the matrix pipe orders and rounds its partial sums (twice the IEEE bound per addition, one addition
 // charged per product), plus one IEEE f32 addition per chunk for the running sum and per column share.  Non-finite
 // approximations (overflow of the f16 conversions) put the token on the list.
-// Measured (512 experts, top-10; prep + f16 + pick, us): 2048 tokens, d = 2560, f32 router 12 + 17 + 35; 3001, d = 3072 17 + 24 + 48;
-// 16384 61 + 85 + 225 -- against 209, 223 and 690 for the eight launches that were here before (W and x converted by the f16
-// launch, which had 32 blocks at 2048 tokens; candidates, exact pairs, ranking and three launches for the redo, 60 us when
-// one token was in it).  The f16 launch and the dot products run at the L2s' rate, 10.5 TB/s; prep at the memory's.
+// Measured (512 experts, d = 3072, top-10, nothing beside them; prep + f16 + pick, us): 515 tokens, f32 router 12 + 12 + 20; 2048 16 + 21 + 35,
+// bf16 16 + 22 + 30; 4096 bf16 22 + 34 + 55; 16384 f32 62 + 90 + 190.  The f16 launch and the dot products of an f32 router (which two
+// XCDs' L2s together could hold, one cannot) run at the L2s' rate, 10.5 TB/s; prep at the memory's.  (With the format's bound, eight lanes
+// to a row, sixteen rows a pass whatever their number, x handed round through LDS and v_cvt_f64_f32, pick took 25, 41, 40, 65 and 222.)
+#include <type_traits>
+
 #include "common.h"
 #include "internal.h"
 #include "router_chain.h"
@@ -40,7 +44,6 @@
 namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef double double2v __attribute__((ext_vector_type(2)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int RA_CHUNK = 128;  // columns summed in the matrix pipe's f32 accumulators before they are added to the running sums
@@ -49,10 +52,14 @@ constexpr int RA_NBUF = 4;     // slabs in LDS
 constexpr int RC_SLOTS = 32;   // candidates per token at most
 constexpr int RL_T = 16;       // listed tokens of a group
 
+// Norm of a row's rounding errors from the sum of their squares; what underflow dropped from that is below the smallest normal
+// float a column.
+__device__ __forceinline__ float f16_err_norm(float sum2, int d) { return sqrtf(sum2 + (float)d * 1.2e-38f); }
+
 // ---- 1. a wave per row: first the router matrix's, then x's ----
 template <bool BF16>
 __global__ void __launch_bounds__(256) k_router_prep(const void* __restrict__ W, int E, int d, __half* __restrict__ W16,
-                                                     float* __restrict__ wnorm, int* __restrict__ hard,
+                                                     float* __restrict__ wnorm, float* __restrict__ xerr, int* __restrict__ hard,
                                                      const float* __restrict__ x, int P, moe_row_extras R) {
   const int lane = threadIdx.x & 63, nwb = (E + 3) >> 2;
   {  // the list's count and its tickets (first used two launches on)
@@ -63,7 +70,7 @@ __global__ void __launch_bounds__(256) k_router_prep(const void* __restrict__ W,
     const int e = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (e >= E) return;
     uint4* dst = (uint4*)W16 + (size_t)e * (d / 8);
-    float s2 = 0.f;
+    float s2 = 0.f, r2 = 0.f;
     for (int i = lane; i < d / 8; i += 64) {
       int ia, ib;
       f16_chunk_src(R.layout, i, ia, ib);
@@ -79,20 +86,29 @@ __global__ void __launch_bounds__(256) k_router_prep(const void* __restrict__ W,
         v = w[ib];
       }
       s2 += ((u.x * u.x + u.y * u.y) + (u.z * u.z + u.w * u.w)) + ((v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w));
+      r2 += f16_err2(u) + f16_err2(v);
       dst[i] = f16_chunk(R.layout, u, v);
     }
     s2 = wave_sum(s2);
-    if (lane == 0) wnorm[e] = sqrtf(s2);
+    r2 = wave_sum(r2);
+    if (lane == 0) {
+      wnorm[e] = sqrtf(s2);
+      wnorm[E + e] = f16_err_norm(r2, d);
+    }
     return;
   }
   const int t = ((int)blockIdx.x - nwb) * 4 + (threadIdx.x >> 6);
   if (t >= P) return;
-  float acc;
+  float acc, err = 0.f;
   double gate;
-  row_extras_part(x, t, d, lane, 64, R, acc, gate);
+  row_extras_part(x, t, d, lane, 64, R, acc, gate, &err);
   acc = wave_sum(acc);
+  err = wave_sum(err);
   if (R.wx) gate = wave_sum(gate);
-  if (lane == 0) row_extras_out(t, d, R, acc, gate);
+  if (lane == 0) {
+    row_extras_out(t, d, R, acc, gate);
+    xerr[t] = f16_err_norm(err, d);
+  }
 }
 
 // ---- 2. approximate logits: block = 64 MT tokens x 64 MT experts x one column share, 4 waves as 2 x 2 ----
@@ -199,115 +215,139 @@ __global__ void __launch_bounds__(256, 2) k_router_f16(const __half* __restrict_
     }
 }
 
-// fp64 dot products of row x with weight rows ra (and rb): lane j of a group of eight takes the 16-byte piece j of every
-// 128-byte line of the group's row, so that a load instruction covers eight whole lines.  The activations are the same for all
-// groups: the wave fetches them once, DR_CH columns per load, and hands them round through LDS, widened to f64 (f32 -> f64
-// conversions run at a quarter of the FMA rate and are what bounds this: a lane would otherwise convert activations that
-// 63 others convert too, and does where two rows do not share them).  The next chunk's weights are requested before the
-// current chunk is summed; short chunks, so that four waves fit a SIMD.  Two accumulators per lane and row, a three-step
-// reduction; the order is fixed.  Columns c0 .. c0 + d - 1 of rows of ld (multiples of 64, d > 0).
-constexpr int DR_CH = 128;
-template <bool BF16, bool TWO>
-__device__ __forceinline__ void dot_rows(const void* __restrict__ W, const float* __restrict__ xrow, int ld, int c0, int d, int ra, int rb,
-                                         int lane, double (*xl)[DR_CH], double& sa, double& sb) {
-  constexpr int LINE = BF16 ? 64 : 32;  // columns per 128-byte line of a weight row
-  constexpr int NL = DR_CH / LINE;      // lines per chunk
-  constexpr int ESZ = BF16 ? 2 : 4, NR = TWO ? 2 : 1;
-  const int j = lane & 7;
-  const uint8_t* const wrow[2] = {(const uint8_t*)W + ((size_t)ra * ld + c0) * ESZ + 16 * j, (const uint8_t*)W + ((size_t)rb * ld + c0) * ESZ + 16 * j};
-  xrow += c0;
-  const int nchunk = (d + DR_CH - 1) / DR_CH;
-  double a[NR][2];
+// fp64 dot products of row x with up to sixteen weight rows (ids: lane i's register holds row i's index, n of them; the lanes
+// past n repeat the last), columns c0 .. c1 - 1 of rows of ld (multiples of 64).  The wave keeps a panel of x in registers, four
+// columns of every 256 to a lane, widened once, and lets the rows go past it two at a time, the next two requested before
+// these are summed: a load covers 1 KB (bf16 512 bytes) of one row, no activation passes through LDS, and no more rows are
+// multiplied than there are candidates (one more where their number is odd).  A lane's sums wait in LDS between panels.
+// What bounds it is widening the weights -- v_cvt_f64_f32 takes four times as long as an FMA -- next to the L2s' rate.  A float's
+// exponent and mantissa shifted into a double's places are the value times 2^-896, zeros and subnormals included, so the
+// weights are widened with shifts and x carries the 2^896 (|x| < 2^128: no overflow; infinities and NaNs never get here).
+// The order of the sums is fixed.
+constexpr int DR_ROWS = 16, DR_PITCH = 65;  // rows of a pass; doubles of a row's sums in LDS
+__device__ __forceinline__ double widen_m896(uint32_t u) {
+  union { double d; uint32_t i[2]; } r;
+  r.i[0] = u << 29;
+  r.i[1] = (u & 0x80000000u) | ((u >> 3) & 0x0fffffffu);
+  return r.d;
+}
+__device__ __forceinline__ double widen_m896_hi(uint32_t u) {  // (a bf16 in the upper half; the lower half is zero)
+  union { double d; uint32_t i[2]; } r;
+  r.i[0] = 0u;
+  r.i[1] = (u & 0x80000000u) | ((u >> 3) & 0x0fffffffu);
+  return r.d;
+}
+// sums: DR_ROWS x DR_PITCH doubles of LDS owned by the wave.  Returns row lane % 16's sum.  PP: pieces of 256 columns in a panel.
+template <bool BF16, int PP>
+__device__ __forceinline__ double dot_rows(__amdgpu_buffer_rsrc_t W, const float* __restrict__ xrow, int ld, int c0, int c1, int ids, int n,
+                                           int lane, double* sums) {
+  constexpr int ESZ = BF16 ? 2 : 4, WPL = BF16 ? 2 : 4;  // words of four weights
+  double* const mine = sums + lane;
+  for (int p0 = c0; p0 < c1; p0 += 256 * PP) {
+    int off[PP];
+    float4 xv[PP];
 #pragma unroll
-  for (int r = 0; r < NR; r++) a[r][0] = a[r][1] = 0.0;
-  uint4 w0[NR][NL], w1[NR][NL];
-  float2 xn;
-  // chunk g (past the end: the last one again, unused; lines past the row's end: its last line, which meets zeros)
-  auto load = [&](int g, uint4 (&w)[NR][NL]) {
-    const int c = (g < nchunk ? g : nchunk - 1) * DR_CH;
+    for (int i = 0; i < PP; i++) {  // (past the end: the first columns again, times zero)
+      const int c = p0 + 256 * i + 4 * lane;
+      off[i] = (c < c1 ? c : c0) * ESZ;
+      xv[i] = *(const float4*)(xrow + (c < c1 ? c : c0));
+    }
+    uint32_t w[2][2][PP][WPL];  // [pair][row][piece]
+    auto load = [&](int r, uint32_t(&q)[2][PP][WPL]) {
 #pragma unroll
-    for (int r = 0; r < NR; r++)
+      for (int h = 0; h < 2; h++) {
+        const int at = __builtin_amdgcn_readlane(ids, r + h < DR_ROWS ? r + h : DR_ROWS - 1) * (ld * ESZ);
 #pragma unroll
-      for (int l = 0; l < NL; l++) {
-        const int cl = c + l * LINE;
-        w[r][l] = *(const uint4*)(wrow[r] + (cl < d ? cl : d - LINE) * ESZ);
-      }
-    const int cx = c + 2 * lane;
-    xn = *(const float2*)(xrow + (cx < d ? cx : 0));
-    if (cx >= d) xn = float2{0.f, 0.f};
-  };
-  auto put_x = [&](int buf) { *(double2v*)(xl[buf] + 2 * lane) = double2v{(double)xn.x, (double)xn.y}; };
-  auto sum = [&](const uint4 (&w)[NR][NL], const double* xs) {
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wave's own LDS writes
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int l = 0; l < NL; l++) {
-      double xv[BF16 ? 8 : 4];
-#pragma unroll
-      for (int i = 0; i < (BF16 ? 4 : 2); i++) {
-        const double2v v = *(const double2v*)(xs + l * LINE + (BF16 ? 8 : 4) * j + 2 * i);
-        xv[2 * i] = v.x;
-        xv[2 * i + 1] = v.y;
-      }
-#pragma unroll
-      for (int r = 0; r < NR; r++) {
-        double& acc = a[r][l & 1];
-        const uint32_t u[4] = {w[r][l].x, w[r][l].y, w[r][l].z, w[r][l].w};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < PP; i++) {
           if constexpr (BF16) {
-            acc = fma((double)__uint_as_float(u[i] << 16), xv[2 * i], acc);
-            acc = fma((double)__uint_as_float(u[i] & 0xffff0000u), xv[2 * i + 1], acc);
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(W, off[i], at, 0);
+            q[h][i][0] = v[0]; q[h][i][1] = v[1];
           } else {
-            acc = fma((double)__uint_as_float(u[i]), xv[i], acc);
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(W, off[i], at, 0);
+            q[h][i][0] = v[0]; q[h][i][1] = v[1]; q[h][i][2] = v[2]; q[h][i][3] = v[3];
           }
         }
       }
-    }
-  };
-  load(0, w0);
-  for (int g = 0; g < nchunk; g += 2) {
-    put_x(0);
-    load(g + 1, w1);
-    sum(w0, xl[0]);
-    if (g + 1 >= nchunk) break;
-    put_x(1);
-    load(g + 2, w0);
-    sum(w1, xl[1]);
-  }
-  sa = a[0][0] + a[0][1];
-  sb = TWO ? a[NR - 1][0] + a[NR - 1][1] : 0.0;
+    };
+    load(0, w[0]);
+    double x[PP][4];
 #pragma unroll
-  for (int o = 1; o < 8; o <<= 1) {
-    sa += __shfl_xor(sa, o, 64);
-    if (TWO) sb += __shfl_xor(sb, o, 64);
+    for (int i = 0; i < PP; i++) {
+      const float f[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
+      const double s = p0 + 256 * i + 4 * lane < c1 ? 0x1p896 : 0.0;
+#pragma unroll
+      for (int k = 0; k < 4; k++) x[i][k] = (double)f[k] * s;
+    }
+    const bool first = p0 == c0;
+    auto sum = [&](int r, const uint32_t(&q)[2][PP][WPL]) {
+      double a[2];
+#pragma unroll
+      for (int h = 0; h < 2; h++) a[h] = first ? 0.0 : mine[(r + h) * DR_PITCH];
+#pragma unroll
+      for (int i = 0; i < PP; i++)
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+          for (int h = 0; h < 2; h++) {
+            double wd;
+            if constexpr (BF16) wd = widen_m896_hi(k & 1 ? q[h][i][k >> 1] & 0xffff0000u : q[h][i][k >> 1] << 16);
+            else wd = widen_m896(q[h][i][k]);
+            a[h] = fma(wd, x[i][k], a[h]);
+          }
+#pragma unroll
+      for (int h = 0; h < 2; h++) mine[(r + h) * DR_PITCH] = a[h];
+    };
+#pragma unroll 1
+    for (int r = 0; r < n; r += 4) {
+      load(r + 2, w[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      sum(r, w[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      load(r + 4, w[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (r + 2 < n) sum(r + 2, w[1]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wave's own LDS writes
+  __builtin_amdgcn_wave_barrier();
+  // lane group g adds sixteen lanes' sums of row lane % 16, two more steps add the groups'
+  const double* const q = sums + (lane & 15) * DR_PITCH + (lane >> 4) * 16;
+  double v = 0.0;
+  if (c1 > c0) {
+#pragma unroll
+    for (int i = 0; i < 16; i++) v += q[i];
+  }
+  v += __shfl_xor(v, 16, 64);
+  v += __shfl_xor(v, 32, 64);
+  __builtin_amdgcn_wave_barrier();
+  return v;
 }
 
 // ---- 3. candidates, their exact logits, ids and weights ----
 struct PickLds {
-  double xl[4][2][DR_CH];  // [wave]: activations of a chunk
   __attribute__((aligned(16))) float lg[512];
   int cid[4][RC_SLOTS], sid[4][RC_SLOTS];
-  double part[4][16];
+  double sums[4][DR_ROWS * DR_PITCH], part[4][DR_ROWS];  // [wave]
   float sval[4][RC_SLOTS], sel_ws[64];
   int sel_ids[64], zero[4], nzero;
 };
 
 // WPT: waves per token (1, 4).  With four, each wave takes a quarter of the columns of the exact dot products; all else runs
 // in every wave alike, so that they agree on every branch.
-template <bool BF16, int WPT>
+template <bool BF16, int WPT, int PP>
 __device__ __forceinline__ bool pick_token(PickLds& S, const float* __restrict__ alog, int KS, const float* __restrict__ wnorm, int P,
-                                           int E, int d, int k, float eps, float dterm, float bias_max, float xms, int t, int lane,
+                                           int E, int d, int k, float eps, float bias_max, float xms, float xerr, int t, int lane,
                                            int wv, int* __restrict__ ids, float* __restrict__ ws, const moe_rfix& RF) {
-  const float xn = sqrtf(xms * (float)d);
+  // |x| of what the matrix pipe has seen at most; a weight row's norm and error norm count (below) with cw and ce
+  const float xn = sqrtf(xms * (float)d) + xerr, cw = 1.01f * (xerr + eps * xn), ce = 1.02f * xn;
   // lane l holds experts 8 l .. 8 l + 7
   float a[8], U[8], L[8];
   bool fin = isfinite(xn);
   float maxU = -INFINITY, maxB = 0.f;
-  float v8[8], wn8[8], bi8[8];
+  float v8[8], wn8[8], we8[8], bi8[8];
 #pragma unroll
-  for (int j = 0; j < 8; j++) v8[j] = wn8[j] = bi8[j] = 0.f;
+  for (int j = 0; j < 8; j++) v8[j] = wn8[j] = we8[j] = bi8[j] = 0.f;
   if (E % 8 == 0) {  // whole lanes, aligned rows
     if (8 * lane < E) {
       auto ld8 = [&](const float* p, float (&o)[8], bool add) {
@@ -317,6 +357,7 @@ __device__ __forceinline__ bool pick_token(PickLds& S, const float* __restrict__
         for (int j = 0; j < 8; j++) o[j] = add ? o[j] + q[j] : q[j];
       };
       ld8(wnorm + 8 * lane, wn8, false);
+      ld8(wnorm + E + 8 * lane, we8, false);
       for (int s = 0; s < KS; s++) ld8(alog + ((size_t)s * P + t) * E + 8 * lane, v8, s > 0);
     }
   } else {
@@ -325,6 +366,7 @@ __device__ __forceinline__ bool pick_token(PickLds& S, const float* __restrict__
       const int e = 8 * lane + j;
       if (e < E) {
         wn8[j] = wnorm[e];
+        we8[j] = wnorm[E + e];
         for (int s = 0; s < KS; s++) v8[j] = s ? v8[j] + alog[((size_t)s * P + t) * E + e] : alog[(size_t)t * E + e];
       }
     }
@@ -340,7 +382,7 @@ __device__ __forceinline__ bool pick_token(PickLds& S, const float* __restrict__
     //  softmax term zero, and it is no candidate)
     if (e < E && !(bi8[j] == -INFINITY && isfinite(v8[j]))) {
       const float av = v8[j] + bi8[j];
-      const float B = eps * xn * wn8[j] + dterm * (xn + wn8[j]) + 1e-6f * (1.f + fabsf(av));
+      const float B = cw * wn8[j] + ce * we8[j] + 1e-6f * (1.f + fabsf(av));
       fin = fin && isfinite(av) && isfinite(B);
       a[j] = av;
       maxB = fmaxf(maxB, B);
@@ -352,24 +394,26 @@ __device__ __forceinline__ bool pick_token(PickLds& S, const float* __restrict__
   maxU = wave_fmax_dpp(maxU);
   maxB = wave_fmax_dpp(maxB);
   if (!__all(fin)) return false;
-  // tau = the k-th largest lower end
+  // tau = the k-th largest lower end: each lane's eight sorted, then k rounds of the largest head
+#pragma unroll
+  for (int pass = 0; pass < 8; pass++)
+#pragma unroll
+    for (int j = pass & 1; j + 1 < 8; j += 2) {
+      const float p = L[j], q = L[j + 1];
+      L[j] = fmaxf(p, q);
+      L[j + 1] = fminf(p, q);
+    }
   float tau = -INFINITY;
   for (int r = 0; r < k; r++) {
-    float m = L[0];
+    tau = wave_fmax_dpp(L[0]);
+    const bool me = lane == (int)__builtin_ctzll(__ballot(L[0] == tau) | (1ull << 63));  // drop one instance
 #pragma unroll
-    for (int j = 1; j < 8; j++) m = fmaxf(m, L[j]);
-    const float wmx = wave_fmax_dpp(m);
-    const int owner = __builtin_ctzll(__ballot(m == wmx) | (1ull << 63));
-    tau = wmx;
-    if (lane == owner) {  // drop one instance
-      bool done = false;
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const bool hit = !done && L[j] == wmx;
-        L[j] = hit ? -INFINITY : L[j];
-        done = done || hit;
-      }
+    for (int j = 0; j < 7; j++) {
+      const float cur = L[j], nxt = L[j + 1];
+      L[j] = me ? nxt : cur;
     }
+    const float last = L[7];
+    L[7] = me ? -INFINITY : last;
   }
   const float thr = tau - 1e-5f;
   // the candidates' rows, by expert index
@@ -394,20 +438,14 @@ __device__ __forceinline__ bool pick_token(PickLds& S, const float* __restrict__
   // exact logits, sixteen rows a pass
   const float tol = RF.tol[t];
   const float* xrow = RF.x + (size_t)t * d;
+  const __amdgpu_buffer_rsrc_t W = __builtin_amdgcn_make_buffer_rsrc((void*)RF.W, 0, E * d * (BF16 ? 2 : 4), 0x00027000);
   bool doubt = false;
   float cv = -INFINITY;  // lane i < cnt: candidate i's logit
-  for (int p0 = 0; p0 < cnt; p0 += 16) {
-    const int s = p0 + (lane >> 3);
-    const int ea = S.cid[wv][s < cnt ? s : p0], eb = S.cid[wv][s + 8 < cnt ? s + 8 : p0];
-    double va, vb = 0.0;
-    const int c0 = WPT == 1 ? 0 : d / 64 * wv / 4 * 64, c1 = WPT == 1 ? d : d / 64 * (wv + 1) / 4 * 64;
-    if (c1 == c0) va = 0.0;  // (fewer than four runs of 64 columns)
-    else if (cnt - p0 > 8) dot_rows<BF16, true>(RF.W, xrow, d, c0, c1 - c0, ea, eb, lane, S.xl[wv], va, vb);
-    else dot_rows<BF16, false>(RF.W, xrow, d, c0, c1 - c0, ea, eb, lane, S.xl[wv], va, vb);
-    if ((lane & 7) == 0) {
-      S.part[wv][lane >> 3] = va;
-      S.part[wv][8 + (lane >> 3)] = vb;
-    }
+  for (int p0 = 0; p0 < cnt; p0 += DR_ROWS) {
+    const int left = cnt - p0 < DR_ROWS ? cnt - p0 : DR_ROWS, s = lane & (DR_ROWS - 1);
+    const int c0 = WPT == 1 ? 0 : d / 64 * wv / 4 * 64, c1 = WPT == 1 ? d : d / 64 * (wv + 1) / 4 * 64;  // (WPT 4: may be none)
+    const double dot = dot_rows<BF16, PP>(W, xrow, d, c0, c1, S.cid[wv][p0 + (s < left ? s : left - 1)], left, lane, S.sums[wv]);
+    if (lane < DR_ROWS) S.part[wv][lane] = dot;
     if (WPT == 1) {
       __builtin_amdgcn_s_waitcnt(0xC07F);
       __builtin_amdgcn_wave_barrier();
@@ -415,7 +453,7 @@ __device__ __forceinline__ bool pick_token(PickLds& S, const float* __restrict__
       __syncthreads();
     }
     const int i = lane - p0;
-    if (i >= 0 && i < 16 && lane < cnt) {
+    if (i >= 0 && i < DR_ROWS && lane < cnt) {
       const double v = WPT == 1 ? S.part[wv][i] : (S.part[0][i] + S.part[1][i]) + (S.part[2][i] + S.part[3][i]);
       doubt = logit_doubtful(v, tol);
       cv = (float)v + (RF.bias ? RF.bias[S.cid[wv][lane]] : 0.f);
@@ -474,19 +512,18 @@ __device__ __forceinline__ bool pick_token(PickLds& S, const float* __restrict__
 }
 
 // Batches up to this size give a token to four waves: with one, the chip holds a wave or less per SIMD that walks the 3072
-// columns in 24 dependent steps, 37 us whatever the number of tokens.  In four waves the walk is six steps, 21 us at 515
-// tokens, but each repeats the selection around it, which counts as soon as the SIMDs are full (three blocks per CU: 768
-// tokens).  The layer with one wave and with four, us: 600 tokens 568 and 558, 900 616 and 610, 1200 648 and 648, 1500 685 and
-// 695.
-constexpr int PICK_SPLIT_MAX = 1024;
+// columns of all candidates by itself.  Four walk a quarter each, but each repeats the selection around it, which counts as
+// soon as the SIMDs are full (three blocks per CU: 768 tokens).  The layer with one wave and with four, us, f32 router: 420 tokens 535
+// and 530, 600 565 and 558, 700 572 and 567, 800 584.5 and 591, 1020 618 and 629; bf16: 300 553 and 551, 900 639 and 646.
+constexpr int PICK_SPLIT_MAX = 768;
 
 // The list of tokens for k_router_listed, ints: [0] their number, [1 + g] the tickets of group g, then the tokens.
 __host__ __device__ constexpr int hard_first(int P) { return 1 + (P + RL_T - 1) / RL_T; }
 
-template <bool BF16, int WPT>
+template <bool BF16, int WPT, int PP>
 __global__ void __launch_bounds__(256, 3) k_router_pick(const float* __restrict__ alog, int KS, const float* __restrict__ wnorm,
-                                                        const float* __restrict__ xms, int P, int E, int d, int k, float eps, float dterm,
-                                                        float bias_max, int* __restrict__ ids, float* __restrict__ ws, int id_stride,
+                                                        const float* __restrict__ xms, const float* __restrict__ xerr, int P, int E, int d,
+                                                        int k, float eps, float bias_max, int* __restrict__ ids, float* __restrict__ ws, int id_stride,
                                                         int* __restrict__ hard, moe_rfix RF) {
   __shared__ __attribute__((aligned(16))) PickLds S;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -494,7 +531,7 @@ __global__ void __launch_bounds__(256, 3) k_router_pick(const float* __restrict_
   if (tid == 0) S.nzero = 0;
   __syncthreads();
   if (t < P) {
-    const bool ok = pick_token<BF16, WPT>(S, alog, KS, wnorm, P, E, d, k, eps, dterm, bias_max, xms[t], t, lane, wv,
+    const bool ok = pick_token<BF16, WPT, PP>(S, alog, KS, wnorm, P, E, d, k, eps, bias_max, xms[t], xerr[t], t, lane, wv,
                                      ids + (size_t)t * id_stride, ws + (size_t)t * id_stride, RF);
     if (!ok && lane == 0 && (WPT == 1 || wv == 0)) {
       // an all-zero row (padding): every dot product is zero.  (A mean square that underflows: |dot| < 1e-17, no softmax term
@@ -680,12 +717,13 @@ bool moe_router_cand_supported(const moe_wview* W, int P, int k) {
 }
 
 static size_t rc_hard_bytes(int tokens) { return ((size_t)(hard_first(tokens) + tokens) * 4 + 255) / 256 * 256; }
-static size_t rc_wnorm_bytes(int experts) { return ((size_t)experts * 4 + 255) / 256 * 256; }
+static size_t rc_wnorm_bytes(int experts) { return ((size_t)experts * 8 + 255) / 256 * 256; }
+static size_t rc_xerr_bytes(int tokens) { return ((size_t)tokens * 4 + 255) / 256 * 256; }
 size_t moe_router_cand_scratch_bytes(int max_tokens, int experts, int d) {
-  // wnorm [E], the router matrix as f16, the column shares' partial logits (as long as there are shares: at most RA_SLOTS tiles)
+  // the rows' norms and error norms (W 2 E, x), the router matrix as f16, the column shares' partial logits (as long as there are shares: at most RA_SLOTS tiles)
   const size_t tiles = (size_t)RA_SLOTS * 128 * 128 * 4, all = (size_t)RA_KS * max_tokens * experts * 4;
   // and the list of hard tokens in front of all
-  return rc_hard_bytes(max_tokens) + rc_wnorm_bytes(experts) + (size_t)experts * d * 2 + 256 + (all < tiles ? all : tiles);
+  return rc_hard_bytes(max_tokens) + rc_wnorm_bytes(experts) + rc_xerr_bytes(max_tokens) + (size_t)experts * d * 2 + 256 + (all < tiles ? all : tiles);
 }
 
 // Internal: ids / ws of a batch; `logits` [P][E] is scratch.
@@ -696,23 +734,34 @@ int moe_router_batch_cand(const moe_wview* W, const float* x, int P, float* logi
   if (!moe_router_cand_supported(W, P, k) || !moe_aligned(x, 16) || !R.x16 || !R.xms || !R.tol) return MOE_E_UNSUPPORTED;
   int* const hard = (int*)scratch;
   float* wnorm = (float*)((uint8_t*)scratch + rc_hard_bytes(P));
-  __half* W16 = (__half*)((uint8_t*)wnorm + rc_wnorm_bytes(E));
+  float* xerr = (float*)((uint8_t*)wnorm + rc_wnorm_bytes(E));
+  __half* W16 = (__half*)((uint8_t*)xerr + rc_xerr_bytes(P));
   const F16Shape s = f16_shape(P, E, d);
   float* alog = s.ks == 1 ? logits : (float*)((uint8_t*)W16 + ((size_t)E * d * 2 + 255) / 256 * 256);
   // 1.002: second-order terms; 1.01: the f32 norms' own rounding
-  const float eps = (0x1p-10f + (float)RA_CHUNK * 0x1p-22f + (float)(d / RA_CHUNK + 1 + RA_KS) * 0x1p-23f) * 1.002f * 1.01f;
-  const float dterm = 0x1p-25f * 1.01f * sqrtf((float)d);
+  const float eps = ((float)RA_CHUNK * 0x1p-22f + (float)(d / RA_CHUNK + 1 + RA_KS) * 0x1p-23f) * 1.002f * 1.01f;
   const bool bf = W->dtype == MOE_DT_BF16;
   const unsigned g1 = (unsigned)((E + 3) / 4 + (P + 3) / 4), g3 = (unsigned)((P + 3) / 4);
   const unsigned g2 = (unsigned)((s.ntt + 7) / 8 * 8 * s.ncol * s.ks);
-  if (bf) k_router_prep<true><<<g1, 256, 0, st>>>(W->data, E, d, W16, wnorm, hard, x, P, R);
-  else k_router_prep<false><<<g1, 256, 0, st>>>(W->data, E, d, W16, wnorm, hard, x, P, R);
+  if (bf) k_router_prep<true><<<g1, 256, 0, st>>>(W->data, E, d, W16, wnorm, xerr, hard, x, P, R);
+  else k_router_prep<false><<<g1, 256, 0, st>>>(W->data, E, d, W16, wnorm, xerr, hard, x, P, R);
   MOE_LAUNCH_CHECK();
   if (after_rows) MOE_HIP(hipEventRecord(after_rows, st));
   if (s.mt == 2) k_router_f16<2><<<g2, 256, 0, st>>>(W16, (const __half*)R.x16, P, E, d, alog, s.ncol, s.ntt, s.ks);
   else k_router_f16<1><<<g2, 256, 0, st>>>(W16, (const __half*)R.x16, P, E, d, alog, s.ncol, s.ntt, s.ks);
   MOE_LAUNCH_CHECK();
-#define PICK_GO(BF, WPT) k_router_pick<BF, WPT><<<WPT == 1 ? g3 : (unsigned)P, 256, 0, st>>>(alog, s.ks, wnorm, R.xms, P, E, d, k, eps, dterm, bias_max, ids, ws, id_stride, hard, RF)
+  // panels of three, four or five pieces: what leaves the fewest empty pieces (3001 tokens, d = 3072, f32: four 41.5 us, three 42.2)
+  const int pieces = ((P <= PICK_SPLIT_MAX ? (d / 64 + 3) / 4 * 64 : d) + 255) / 256;
+  int pp = 4;
+  for (int i = 3; i <= 5; i += 2)
+    if ((pieces + i - 1) / i * i < (pieces + pp - 1) / pp * pp) pp = i;
+#define PICK_PP(BF, WPT, PP) k_router_pick<BF, WPT, PP><<<WPT == 1 ? g3 : (unsigned)P, 256, 0, st>>>(alog, s.ks, wnorm, R.xms, xerr, P, E, d, k, eps, bias_max, ids, ws, id_stride, hard, RF)
+#define PICK_GO(BF, WPT)                    \
+  do {                                      \
+    if (pp == 3) PICK_PP(BF, WPT, 3);       \
+    else if (pp == 4) PICK_PP(BF, WPT, 4);  \
+    else PICK_PP(BF, WPT, 5);               \
+  } while (0)
   if (P <= PICK_SPLIT_MAX) {
     if (bf) PICK_GO(true, 4);
     else PICK_GO(false, 4);
@@ -720,6 +769,7 @@ int moe_router_batch_cand(const moe_wview* W, const float* x, int P, float* logi
     if (bf) PICK_GO(true, 1);
     else PICK_GO(false, 1);
   }
+#undef PICK_PP
 #undef PICK_GO
   MOE_LAUNCH_CHECK();
   const int items = (P + RL_T - 1) / RL_T * ((E + RL_E - 1) / RL_E);

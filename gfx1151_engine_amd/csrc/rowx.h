@@ -33,9 +33,15 @@ typedef uint32_t gate_bf16x2 __attribute__((aligned(2)));
 
 // the f16 copy (layout as moe_f32_to_f16's), the mean square, the selection's error bound and the shared expert's gate
 // logit (fp64 sum) of row t; each is left out where its pointer is null
-// (chunks of 8 columns i0, i0 + step, ...: this thread's part of the row's sums in acc and gate)
+// (chunks of 8 columns i0, i0 + step, ...: this thread's part of the row's sums in acc and gate; err: of the squares of what
+// rounding to f16 changes)
+__device__ __forceinline__ float f16_err2(const float4& u) {
+  const float a = u.x - __half2float(__float2half_rn(u.x)), b = u.y - __half2float(__float2half_rn(u.y));
+  const float c = u.z - __half2float(__float2half_rn(u.z)), e = u.w - __half2float(__float2half_rn(u.w));
+  return (a * a + b * b) + (c * c + e * e);
+}
 __device__ __forceinline__ void row_extras_part(const float* __restrict__ x, int t, int d, int i0, int step, const moe_row_extras& R,
-                                                float& acc, double& gate) {
+                                                float& acc, double& gate, float* err = nullptr) {
   const float4* xr = (const float4*)(x + (size_t)t * d);
   uint4* yr = R.x16 ? (uint4*)R.x16 + (size_t)t * (d / 8) : nullptr;
   acc = 0.f;
@@ -49,6 +55,7 @@ __device__ __forceinline__ void row_extras_part(const float* __restrict__ x, int
       yr[i] = f16_chunk(R.layout, u, v);
     }
     acc += ((u.x * u.x + u.y * u.y) + (u.z * u.z + u.w * u.w)) + ((v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w));
+    if (err) *err += f16_err2(u) + f16_err2(v);
     if (R.wx) {
       float g[8];
       if (R.wx_bf16) {

@@ -218,6 +218,34 @@ def test_router_candidates_of_small_batches(capi, oracle, T, E, k, d, dt, fmt, s
     assert np.abs(ws - wo[:, :k]).max() <= 2.5e-7
 
 
+# ... and at the widths of the exact dot products' panels (three, four and five pieces of 256 columns, whole and cut short, one
+# panel and several), on both sides of the line between four waves and one, with odd numbers of candidates and with more
+# than one pass of sixteen takes; weights that are zero or subnormal (the products are widened by shifting)
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("T,E,k,d,std", [(768, 512, 10, 3072, 0.02), (769, 512, 10, 3072, 0.02), (300, 512, 9, 2560, 0.02), (770, 512, 9, 2560, 0.02),
+                                         (771, 300, 15, 832, 0.0005), (900, 128, 4, 1280, 0.02), (800, 64, 5, 64, 0.02), (780, 40, 11, 1600, 0.02)])
+def test_router_candidates_exact_products(capi, oracle, T, E, k, d, std, dt):
+    rng = np.random.default_rng(T + d)
+    kw = dict(fmt="q4k", gg_types=(8, 8, 8)) if d % 128 else {}
+    hl = HostLayer(rng, d, 256, E, k, router_dtype=dt, router_std=std, shared=False, **kw)
+    w = hl.router
+    w[:, ::7] = 0
+    w[1, ::3] = np.float32(1e-40) if dt == "f32" else w.dtype.type(1)  # (the smallest bf16)
+    w[2, 1::5] = np.float32(-1e-41) if dt == "f32" else w.dtype.type(0x8001)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    x[::2] = x[::2].astype(np.float16)       # exact in f16 (no rounding error to bound), and not
+    x[8] = 0.0
+    x[9, 0] = 3e4
+    lo, io, wo = oracle.router(hl.oracle_layer().router, x, k)
+    m, dev = hl.to_gpu(max_tokens=T)
+    m.forward(0, gpu(x))
+    assert m.last_path() == capi.PATH_BATCH
+    ids, ws = (a.cpu().numpy()[:, :k] for a in m.last_routing(T))
+    m.close()
+    assert (ids == io[:, :k]).all()
+    assert np.abs(ws - wo[:, :k]).max() <= 2.5e-7
+
+
 # ---------- routers of 33 tokens and more: tokens that the fast selection cannot settle, few and many of them ----------
 def route_and_compare(capi, oracle, hl, x, k):
     T = len(x)
