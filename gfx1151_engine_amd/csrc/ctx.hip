@@ -46,10 +46,8 @@ static int codebook_affine(const moe_wview* w, bool* out) {
 }
 
 struct moe_ctx;
-static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_lutw* a, const moe_lutw* b, int kq, int rows, int cols,
+static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_lutw* a, const moe_lutw* b, int group, int rows, int cols,
                          int n_experts, bool* all);
-static int pexp_register_gguf(moe_ctx* c, int layer, int slot0, int type, const uint8_t* a, const uint8_t* b, int rows, int cols,
-                              int n_experts, bool* all);
 static int magnitude_constant(moe_ctx* c, int tgu, int tdn, const moe_wview* gate, uint64_t gate_stride,
                               const moe_wview* up, uint64_t up_first, const moe_wview* down, int n_experts,
                               moe_cmag* out);
@@ -142,8 +140,8 @@ struct moe_ctx {
 static int8_t* pexp_slot(moe_ctx* c, int layer, int slot0) {
   return c->pexp ? c->pexp + (size_t)layer * (2 * (size_t)c->cfg.experts + 2) + slot0 : nullptr;
 }
-// rows, cols: of one expert; kq as for moe_scale_span.  *all: every expert has one.
-static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_lutw* a, const moe_lutw* b, int kq, int rows, int cols,
+// rows, cols: of one expert; group: columns of a scale.  *all: every expert has one.
+static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_lutw* a, const moe_lutw* b, int group, int rows, int cols,
                          int n_experts, bool* all) {
   *all = false;
   int8_t* dst = pexp_slot(c, layer, slot0);
@@ -151,33 +149,22 @@ static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_lutw* a, co
   std::vector<int8_t> out((size_t)n_experts, (int8_t)MOE_PEXP_NONE);
   if (a) {
     std::vector<int8_t> sa((size_t)2 * n_experts), sb;
-    int rc = moe_scale_span(a, kq, n_experts, rows, cols, c->span_tmp, nullptr);
+    int rc = moe_scale_span(a, group, n_experts, rows, cols, c->span_tmp, nullptr);
     if (rc) return rc;
     MOE_HIP(hipMemcpy(sa.data(), c->span_tmp, sa.size(), hipMemcpyDeviceToHost));
     if (b) {
       sb.resize(sa.size());
-      if ((rc = moe_scale_span(b, kq, n_experts, rows, cols, c->span_tmp, nullptr))) return rc;
+      if ((rc = moe_scale_span(b, group, n_experts, rows, cols, c->span_tmp, nullptr))) return rc;
       MOE_HIP(hipMemcpy(sb.data(), c->span_tmp, sb.size(), hipMemcpyDeviceToHost));
     }
     *all = true;
     for (int e = 0; e < n_experts; e++) {
-      out[e] = (int8_t)moe_pexp_from_span(&sa[2 * e], b ? &sb[2 * e] : nullptr, kq >= 144);
+      out[e] = (int8_t)moe_pexp_from_span(&sa[2 * e], b ? &sb[2 * e] : nullptr);
       *all = *all && out[e] != (int8_t)MOE_PEXP_NONE;
     }
   }
   MOE_HIP(hipMemcpy(dst, out.data(), out.size(), hipMemcpyHostToDevice));
   return MOE_OK;
-}
-
-// Raw GGUF rows: of the types that gemm_q4cp.hip takes, Q4_K has the form (Q5_K's fifth bits leave no registers for it: 739 us
-// without and 750 with it, gate/up at 4096 tokens)
-static int pexp_register_gguf(moe_ctx* c, int layer, int slot0, int type, const uint8_t* a, const uint8_t* b, int rows, int cols,
-                              int n_experts, bool* all) {
-  const bool ok = type == MOE_GGML_Q4_K && cols % 256 == 0 && moe_aligned(a, 16) && (!b || moe_aligned(b, 16));
-  moe_lutw va{}, vb{};
-  va.w = a;
-  vb.w = b;
-  return pexp_register(c, layer, slot0, ok ? &va : nullptr, b ? &vb : nullptr, 144, rows, cols, n_experts, all);
 }
 
 static void prof_mark(moe_ctx* c, int stage_done, hipStream_t st) {
@@ -452,9 +439,6 @@ MOE_API int moe_set_experts_gguf(moe_ctx* c, int layer, const moe_gg_experts* gg
     moe_wview dv{0, gg->down, (uint64_t)g.experts * g.d, (uint64_t)g.mid, 0};
     int rc = magnitude_constant(c, gg->tgu, gg->tdn, &gv, (uint64_t)g.mid, &uv, 0, &dv, g.experts, &L->c_routed);
     if (rc) return rc;
-    if ((rc = pexp_register_gguf(c, layer, 0, gg->tgu, gg->gate, gg->up, g.mid, g.d, g.experts, &L->scaled_gu)) ||
-        (rc = pexp_register_gguf(c, layer, g.experts, gg->tdn, gg->down, nullptr, g.d, g.mid, g.experts, &L->scaled_dn)))
-      return rc;
   }
   L->gg = *gg;
   L->has_gguf = true;
@@ -496,10 +480,9 @@ MOE_API int moe_set_shared(moe_ctx* c, int layer, const moe_wview* g, const moe_
         (rc = pexp_register(c, layer, 2 * cf.experts + 1, a3 ? &vd : nullptr, nullptr, 32, cf.d, cf.mid, 1, &L->scaled_sdn)))
       return rc;
   } else {
-    const int t = dense ? 0 : sh_gguf_type;
     int rc;
-    if ((rc = pexp_register_gguf(c, layer, 2 * cf.experts, t, g->data, u->data, cf.mid, cf.d, 1, &L->scaled_sgu)) ||
-        (rc = pexp_register_gguf(c, layer, 2 * cf.experts + 1, t, dn->data, nullptr, cf.d, cf.mid, 1, &L->scaled_sdn)))
+    if ((rc = pexp_register(c, layer, 2 * cf.experts, nullptr, nullptr, 32, cf.mid, cf.d, 1, &L->scaled_sgu)) ||
+        (rc = pexp_register(c, layer, 2 * cf.experts + 1, nullptr, nullptr, 32, cf.d, cf.mid, 1, &L->scaled_sdn)))
       return rc;
   }
   L->c_shared = moe_cmag{0.f, 0.f};
@@ -1144,8 +1127,8 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   const __half* xh = c->x16_ext ? c->x16_ext : c->x16;  // f16 activations in the GEMM's order
   int xl = cap ? sxl : batch_x16_layout(L, g);  // that order (moe_f32_to_f16's layout)
   const bool nat = batch_nat(L);               // table codebooks: natural K order, pair tables
-  // scaled dequantisation (affine codebooks, Q4_K): the powers of two found when the weights were registered
-  const bool pe_r = L.experts_affine || L.has_gguf, pe_s = L.has_shared && !shd && (q4k || L.shared_affine);
+  // scaled dequantisation (affine codebooks): the powers of two found when the weights were registered
+  const bool pe_r = L.experts_affine, pe_s = L.has_shared && !shd && !q4k && L.shared_affine;
   const int8_t* pe_gu = pe_r ? pexp_slot(c, (int)(&L - c->layers.data()), 0) : nullptr;
   const int8_t* pe_dn = pe_r ? pexp_slot(c, (int)(&L - c->layers.data()), g.experts) : nullptr;
   const int8_t* pe_sgu = pe_s ? pexp_slot(c, (int)(&L - c->layers.data()), 2 * g.experts) : nullptr;
@@ -1173,7 +1156,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
       if (with_sh ? kd.s_gu : kd.r_gu)
         return moe_launch_gemm_q4cp(true, with_sh ? &sgu : &gu, with_sh ? &sgu : nullptr, g.experts, xh, c->tokidx, tl, ntl,
                                     mt, c->hid16, g.mid, g.d, true, true, hs, s2, nullptr, nullptr, 0,
-                                    (with_sh ? L.sh_gguf_type : L.gg.tgu) == MOE_GGML_Q5_K, false, with_sh ? pe_sgu : pe_gu, pe_sgu);
+                                    (with_sh ? L.sh_gguf_type : L.gg.tgu) == MOE_GGML_Q5_K);
       return with_sh ? moe_launch_gemm_gg(true, L.sh_gguf_type, L.sh_gate.data, L.sh_up.data, L.sh_gguf_type,
                                           L.sh_gate.data, L.sh_up.data, g.experts, xh, c->tokidx, tl, ntl, mt, c->hid16,
                                           g.mid, g.d, hs, s2, xl, P, true)
@@ -1220,8 +1203,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
       // (hid rows are in the tuned kernel's order where its gate/up form wrote them, else in natural order)
       if (with_sh ? kd.s_dn : kd.r_dn)
         return moe_launch_gemm_q4cp(false, with_sh ? &sdn : &dn, with_sh ? &sdn : nullptr, g.experts, c->hid16, nullptr, tl,
-                                    ntl, mt, c->pairs16, g.d, g.mid, true, true, hs, s2, nullptr, nullptr, 0, false, false,
-                                    with_sh ? pe_sdn : pe_dn, pe_sdn);
+                                    ntl, mt, c->pairs16, g.d, g.mid, true, true, hs, s2, nullptr);
       return with_sh ? moe_launch_gemm_gg(false, L.sh_gguf_type, L.sh_down.data, nullptr, L.sh_gguf_type, L.sh_down.data,
                                           nullptr, g.experts, c->hid16, nullptr, tl, ntl, mt, c->pairs16, g.d, g.mid, hs, s2,
                                           kd.s_gu ? 2 : 0, P, true)

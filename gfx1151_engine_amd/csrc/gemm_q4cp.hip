@@ -141,18 +141,16 @@ __device__ __forceinline__ void g2l4(const void* g, uint8_t* lds_base) {
 // MF = live 32-row fragments of the tile (1 .. 4); AFFINE = codebook a*n+b.
 // NF = weight fragments (32 rows) per wave: the block's 16 fragments are split over NW = 16/NF
 // waves, each wave multiplying all MF pair fragments with its own NF weight fragments.
-// DN (affine q4cp codebooks, i4r and Q4_K, a power of two P known for the expert): two instructions per weight pair instead
-// of three.
+// DN (affine q4cp codebooks and i4r, a power of two P known for the expert): two instructions per weight pair instead of three.
 // A masked code pair IS a pair of f16 denormals, n * 2^-24 (nibbles at bits 0-3) or n * 2^-20 (bits 4-7), so one packed
 // FMA with a = f16(cb_a * scale) * 2^(24+P) (or 2^(20+P)) and b = f16(cb_b * scale) * 2^P gives 2^P * f16(n*a' + b'):
 // the weights of the three-instruction form times 2^P, bit for bit wherever the scaled weight is a normal f16 (the
 // product is exact inside the FMA, one rounding).  P is chosen when the weights are registered, from the expert's
 // largest scale, so that the scaled slope stays below 2^15 (an f16 can hold it); the accumulators carry the factor
-// 2^P and the epilogue takes it out (exact).  v_pk_fma_f16 takes denormal operands at full rate on gfx950.  Q4_K: d and
-// dmin are brought into the scaled units once per super-block (2^(12+P), then 2^12 or 2^8), a sub-block's min is read as a
-// denormal too.  us, with three instructions and two: i4r 8192 tokens (skewed) gate/up 1141 1098, down 558 531; Q4_K 8192
-// gate/up 1038 1003, 4096 569 561 (down rows of three super-blocks whose scales are drawn independently span more than 2^6 in
-// most experts, which keeps them on three).
+// 2^P and the epilogue takes it out (exact).  v_pk_fma_f16 takes denormal operands at full rate on gfx950.  us, with three instructions
+// and two: i4r 8192 tokens (skewed) gate/up 1141 1098, down 558 531.  (Q4_K gained two per cent of a layer of 4096 tokens and more with it,
+// d and dmin brought into the scaled units, but products of theirs that are subnormal as f16 were then rounded otherwise than
+// in the streaming GEMM; Q5_K's fifth bits leave no registers for it: 739 us without and 750 with it.)
 constexpr bool NH_OK = NF == 2;
 template <bool UP, bool F16OUT, int MF, bool AFFINE, bool Q4K, int GS, bool Q5, bool NAT = false, bool DN = false, bool ROT = false>
 __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e, const moe_tile tile, int nb,
@@ -168,9 +166,8 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
   // uses the stage buffer that the pipeline has just left.
   constexpr bool WALK = !UP && F16OUT && !Q5 && AHEAD == 2;
   if (!WALK) npass = 1;
-  static_assert(!DN || (AFFINE && !NAT && !Q5), "scaled dequantisation: codes of four bits that stand for a * n + b");
-  const uint32_t kq12 = DN && Q4K ? (uint32_t)(27 + pexp) * 0x04000400u : 0u;  // K-quants: (2^(12+P), 2^(12+P))
-  if (DN && !Q4K) {  // the codebook in the scaled units
+  static_assert(!DN || (AFFINE && !NAT && !Q4K), "scaled dequantisation: codes of four bits that stand for a * n + b");
+  if (DN) {  // the codebook in the scaled units
     const float s24 = __builtin_ldexpf(1.f, 24 + pexp);
     const float sp = __builtin_ldexpf(1.f, pexp);
     cb_a *= s24; cb_a_up *= s24;
@@ -477,20 +474,13 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
           k4w[nf][1] = (hd.w & 0x0f0f0f0fu) | ((hd.y >> 2) & 0x30303030u);
           k4w[nf][2] = hd.z & 0x3f3f3f3fu;
           k4w[nf][3] = ((hd.w >> 4) & 0x0f0f0f0fu) | ((hd.z >> 2) & 0x30303030u);
-          if (DN) {
-            // slopes for codes read as f16 denormals -- low nibbles, high nibbles -- and for minima read so
-            const half2v t = h2(hd.x) * h2(kq12);
-            k4w[nf][4] = u2(half2v{t.x, t.x} * half2v{(_Float16)4096.f, (_Float16)256.f});
-            k4w[nf][5] = u2(half2v{t.y, t.y} * half2v{(_Float16)-4096.f, (_Float16)-4096.f});
-          } else {
-            k4w[nf][4] = __builtin_amdgcn_perm(hd.x, hd.x, 0x01000100u);                 // (d, d)
-            k4w[nf][5] = __builtin_amdgcn_perm(hd.x, hd.x, 0x03020302u) ^ 0x80008000u;  // (-dmin, -dmin)
-          }
+          k4w[nf][4] = __builtin_amdgcn_perm(hd.x, hd.x, 0x01000100u);                 // (d, d)
+          k4w[nf][5] = __builtin_amdgcn_perm(hd.x, hd.x, 0x03020302u) ^ 0x80008000u;  // (-dmin, -dmin)
         }
         const uint32_t wsc = jj < 2 ? k4w[nf][0] : k4w[nf][1], wmn = jj < 2 ? k4w[nf][2] : k4w[nf][3];
         const half2v k1024 = half2v{(_Float16)1024.f, (_Float16)1024.f};
         const half2v sc = h2(__builtin_amdgcn_perm(0x64646464u, wsc, selb)) - k1024;
-        const half2v mn = DN ? h2(__builtin_amdgcn_perm(0u, wmn, selb)) : h2(__builtin_amdgcn_perm(0x64646464u, wmn, selb)) - k1024;
+        const half2v mn = h2(__builtin_amdgcn_perm(0x64646464u, wmn, selb)) - k1024;
         union { half2v h; uint32_t u; } a, b;
         a.h = sc * h2(k4w[nf][4]);
         b.h = mn * h2(k4w[nf][5]);
@@ -524,7 +514,7 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
       const uint32_t w8 = q == 0 ? cw8[nf].x : q == 1 ? cw8[nf].y : q == 2 ? cw8[nf].z : cw8[nf].w;
       const uint32_t ws = part >= 2 ? w8 : w;
       if ((part & 1) == 0) dst[nf].h[part] = h2(ws & 0x000f000fu) * as2[nf][0] + bs2[nf][0];
-      else dst[nf].h[part] = h2(ws & 0x00f000f0u) * (Q4K ? as2[nf][NS - 1] : as20[DN ? nf : 0]) + bs2[nf][Q4K ? NS - 1 : 0];
+      else dst[nf].h[part] = h2(ws & 0x00f000f0u) * as20[DN ? nf : 0] + bs2[nf][0];
     } else if (Q5) {
       // five-bit codes as bytes, the low nibbles' (parts 0, 2) and the high nibbles' (1, 3): parts 0 and 1 make them.  Bit
       // 2 jj / 2 jj + 1 of each byte of the qh word goes to bit 4
@@ -942,7 +932,7 @@ k_moe_gemm_q4cp(LutDev R, LutDev Sh, int n_experts, const __half* __restrict__ x
   const int e = shared ? 0 : tile.expert;
   // scaled dequantisation: the expert's power of two (requested here, used after the first loads have gone out)
   int pexp = MOE_PEXP_NONE;
-  if (!NAT && !Q5 && L.pexp) pexp = L.pexp[e];
+  if (!NAT && !Q4K && L.pexp) pexp = L.pexp[e];
   const int tid = threadIdx.x, lane = tid & 63;
 
   // the tile's row indices: requested before the codebook is looked at, so that the two round trips
@@ -996,10 +986,19 @@ k_moe_gemm_q4cp(LutDev R, LutDev Sh, int n_experts, const __half* __restrict__ x
 #define GEMM_GO(MF)                                                                                     \
   do {                                                                                                  \
     if constexpr (NAT) gemm_tile<UP, F16OUT, MF, false, false, 0, false, true>(GEMM_ARGS, GEMM_TAIL);      \
-    else if ((Q4K || GS == 2 || affine) && pexp != MOE_PEXP_NONE)                                       \
-      gemm_tile<UP, F16OUT, MF, true, Q4K, GS, Q5, false, !Q5, ROT>(GEMM_ARGS, pexp, npass, rot);       \
-    else if (Q4K || GS == 2 || affine) gemm_tile<UP, F16OUT, MF, true, Q4K, GS, Q5, false, false, ROT>(GEMM_ARGS, GEMM_TAIL, rot); \
-    else if constexpr (!Q4K && GS == 0) gemm_tile<UP, F16OUT, MF, false, false, GS, false>(GEMM_ARGS, GEMM_TAIL); \
+    else {                                                                                              \
+      bool scaled = false;                                                                              \
+      if constexpr (!Q4K) {                                                                             \
+        if ((GS == 2 || affine) && pexp != MOE_PEXP_NONE) {                                             \
+          gemm_tile<UP, F16OUT, MF, true, false, GS, false, false, true, ROT>(GEMM_ARGS, pexp, npass, rot); \
+          scaled = true;                                                                                \
+        }                                                                                               \
+      }                                                                                                 \
+      if (!scaled) {                                                                                    \
+        if (Q4K || GS == 2 || affine) gemm_tile<UP, F16OUT, MF, true, Q4K, GS, Q5, false, false, ROT>(GEMM_ARGS, GEMM_TAIL, rot); \
+        else if constexpr (!Q4K && GS == 0) gemm_tile<UP, F16OUT, MF, false, false, GS, false>(GEMM_ARGS, GEMM_TAIL); \
+      }                                                                                                 \
+    }                                                                                                   \
   } while (0)
   if (mfn <= 1) GEMM_GO(1);
   else if (mfn == 2) GEMM_GO(2);
@@ -1049,9 +1048,6 @@ namespace {
 // One block per expert: hi = exponent of |slope| * (largest |scale| of the expert), lo = exponent of |slope| * (the
 // smallest of the rows' largest scales; rows of zeros left out), as frexp gives them; hi = 127: the scaled
 // dequantisation does not apply (a scale or the slope not finite, slope zero); hi = -127: every scale is zero.
-// KQ (block bytes): the sub-blocks' d * sc of K-quants instead, with d and dmin by themselves counted into hi (the kernels
-// scale them before they multiply).
-template <int KQ>
 __global__ void __launch_bounds__(256) k_scale_span(const uint8_t* __restrict__ sc, const float* __restrict__ cb,
                                                     int sstride, int rows, int groups, int8_t* __restrict__ span) {
   __shared__ float s_hi[256], s_lo[256];
@@ -1061,28 +1057,12 @@ __global__ void __launch_bounds__(256) k_scale_span(const uint8_t* __restrict__ 
   float hi = 0.f, lo = INFINITY;
   int bad = 0;
   for (int r = tid; r < rows; r += 256) {
-    const uint8_t* row = base + (size_t)r * sstride;
+    const __half* row = (const __half*)(base + (size_t)r * sstride);
     float rm = 0.f;
     for (int g = 0; g < groups; g++) {
-      float v, m = 0.f;
-      if (KQ) {
-        const uint4 hd = *(const uint4*)(row + (size_t)g * KQ);
-        const uint32_t a = hd.y & 0x3f3f3f3fu, b = (hd.w & 0x0f0f0f0fu) | ((hd.y >> 2) & 0x30303030u);
-        uint32_t most = 0;
-        for (int i = 0; i < 4; i++) {
-          const uint32_t x = (a >> (8 * i)) & 63u, y = (b >> (8 * i)) & 63u;
-          most = most > x ? most : x;
-          most = most > y ? most : y;
-        }
-        m = fmaxf(fabsf((float)h2(hd.x).x), fabsf((float)h2(hd.x).y));
-        v = fabsf((float)h2(hd.x).x) * (float)most;
-        if (!(fabsf((float)h2(hd.x).x) <= 65504.f && fabsf((float)h2(hd.x).y) <= 65504.f)) bad = 1;
-      } else {
-        v = fabsf(__half2float(((const __half*)row)[g]));
-      }
-      if (!KQ && !(v <= 65504.f)) bad = 1;
+      const float v = fabsf(__half2float(row[g]));
+      if (!(v <= 65504.f)) bad = 1;
       rm = fmaxf(rm, v);
-      hi = fmaxf(hi, m);
     }
     hi = fmaxf(hi, rm);
     if (rm > 0.f) lo = fminf(lo, rm);
@@ -1098,7 +1078,7 @@ __global__ void __launch_bounds__(256) k_scale_span(const uint8_t* __restrict__ 
     __syncthreads();
   }
   if (tid == 0) {
-    const float a = KQ ? 1.f : fabsf(cb[1] - cb[0]);
+    const float a = fabsf(cb[1] - cb[0]);
     int h = 127, l = 127;
     if (!s_bad[0] && a > 0.f && a <= 3.0e38f) {
       if (s_hi[0] == 0.f) {
@@ -1116,17 +1096,16 @@ __global__ void __launch_bounds__(256) k_scale_span(const uint8_t* __restrict__ 
 }
 }  // namespace
 
-int moe_scale_span(const moe_lutw* w, int kq, int n_experts, int rows, int cols, int8_t* span_dev, hipStream_t st) {
+int moe_scale_span(const moe_lutw* w, int group, int n_experts, int rows, int cols, int8_t* span_dev, hipStream_t st) {
   if (!w || !span_dev || n_experts < 1 || rows < 1) return MOE_E_INVALID;
-  if (kq == 144) k_scale_span<144><<<n_experts, 256, 0, st>>>(w->w, nullptr, cols / 256 * 144, rows, cols / 256, span_dev);
-  else if (kq == 32 || kq == 128) k_scale_span<0><<<n_experts, 256, 0, st>>>(w->sc, w->cb, w->sstride, rows, cols / kq, span_dev);
-  else return MOE_E_INVALID;
+  if (group != 32 && group != 128) return MOE_E_INVALID;
+  k_scale_span<<<n_experts, 256, 0, st>>>(w->sc, w->cb, w->sstride, rows, cols / group, span_dev);
   MOE_LAUNCH_CHECK();
   return MOE_OK;
 }
 
 // hi_lo_b may be null (one tensor)
-int moe_pexp_from_span(const int8_t* a, const int8_t* b, bool kq) {
+int moe_pexp_from_span(const int8_t* a, const int8_t* b) {
   int hi = a[0], lo = a[1];
   if (hi == 127) return MOE_PEXP_NONE;
   if (b) {
@@ -1137,7 +1116,6 @@ int moe_pexp_from_span(const int8_t* a, const int8_t* b, bool kq) {
   if (hi == -127) return 0;          // nothing but zeros: any power will do
   if (hi - lo > 6) return MOE_PEXP_NONE;
   const int P = -8 - hi;             // |slope| * scale * 2^(24+P) < 2^16, rounded to f16 already (k_scale_span)
-  if (kq && (P < -26 || P > 3)) return MOE_PEXP_NONE;  // (2^(12+P) as an f16)
   return P < -100 || P > 100 ? MOE_PEXP_NONE : P;
 }
 

@@ -1,6 +1,6 @@
-"""The grouped GEMMs' scaled dequantisation (codes read as f16 denormals, a power of two per expert) of rotated and Q4_K experts:
-experts that have such a power and experts that do not, in one layer, on the few-pair and the 128-pair kernels, against the
-oracle.  Reference: src/gpu/parts/27_kernels_moe_lut.inc:16-29, 26_kernels_moe_gguf.inc:81-485."""
+"""The grouped GEMMs' scaled dequantisation (codes read as f16 denormals, a power of two per expert) of rotated experts: experts
+that have such a power and experts that do not, in one layer, on the few-pair and the 128-pair kernels, against the oracle; and
+Q4_K experts, whose arithmetic has no such form, at the same scales.  Reference: src/gpu/parts/27_kernels_moe_lut.inc:16-29, 26_kernels_moe_gguf.inc:81-485."""
 import numpy as np
 import pytest
 
