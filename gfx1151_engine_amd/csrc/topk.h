@@ -140,16 +140,85 @@ __device__ __forceinline__ void topk_select_lm(uint32_t (&key)[NPL], int lane, i
   }
 }
 
+// The n best of a wave's lane-major keys (n <= 63; key[j] of lane l = expert NPL*l + j, 0 = none) without a round per rank: lane
+// r < n gets the key and the expert of rank r.  A bound that at least n keys reach -- in each row of sixteen lanes the
+// ceil(n / 4)-th largest of the lanes' maxima, the least of the four rows' -- leaves a few dozen candidates; they are put
+// together through LDS, one to a lane, and each counts the candidates above it.  False (the same in every lane; the caller
+// selects by rounds): equal keys among the n best, more than 64 candidates, or fewer than n keys.  buf: 64 entries of LDS owned
+// by the wave.
+// (A round -- the wave's maximum, its owner, a pop -- is a chain of some 200 cycles and a token takes k + 1 of them after a sort of
+// each lane's keys.  us, by rounds and by counting: four layers of one token q4cp 91.0 89.6, table codebook 120.7 119.6, Q5_K / Q8_0
+// 116.7 114.4; two of three tokens Q5_K / Q8_0 118.2 116.8; rotated experts, 11 tokens 99.9 99.5.)
+template <int NPL>
+__device__ __forceinline__ bool topk_by_count(const uint32_t (&key)[NPL], int lane, int n, uint2* buf, uint32_t& mykey, int& myid) {
+  uint32_t cur = key[0];
+#pragma unroll
+  for (int j = 1; j < NPL; j++) cur = umax(cur, key[j]);
+  uint32_t rm = 0u;
+  for (int r = 0; r < (n + 3) >> 2; r++) {  // (equal maxima go together, which only lowers the bound)
+    rm = cur;
+    rm = umax(rm, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rm, 0xB1, 0xf, 0xf, true));
+    rm = umax(rm, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rm, 0x4E, 0xf, 0xf, true));
+    rm = umax(rm, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rm, 0x141, 0xf, 0xf, true));
+    rm = umax(rm, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rm, 0x140, 0xf, 0xf, true));
+    cur = cur == rm ? 0u : cur;
+  }
+  const uint32_t bound = umin(umin((uint32_t)__builtin_amdgcn_readlane((int)rm, 0), (uint32_t)__builtin_amdgcn_readlane((int)rm, 16)),
+                              umin((uint32_t)__builtin_amdgcn_readlane((int)rm, 32), (uint32_t)__builtin_amdgcn_readlane((int)rm, 48)));
+  if (bound == 0u) return false;
+  int total = 0;
+#pragma unroll
+  for (int j = 0; j < NPL; j++) {
+    const bool in = key[j] >= bound;
+    const unsigned long long b = __ballot(in);
+    const int pos = total + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
+    if (in && pos < 64) buf[pos] = make_uint2(key[j], (uint32_t)(NPL * lane + j));
+    total += __popcll(b);
+  }
+  if (total > 64) return false;
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wave's own LDS writes
+  __builtin_amdgcn_wave_barrier();
+  uint2 c = buf[lane];
+  c.x = lane < total ? c.x : 0u;
+  int rank = 0;
+  for (int i = 0; i < total; i += 4) {  // (lanes past the candidates hold 0, above which there is every key)
+#pragma unroll
+    for (int q = 0; q < 4; q++) rank += (uint32_t)__builtin_amdgcn_readlane((int)c.x, i + q) > c.x ? 1 : 0;
+  }
+  const int to = lane < total && rank < n ? rank : 63;
+  mykey = (uint32_t)__builtin_amdgcn_ds_permute(4 * to, (int)c.x);  // (0 where no lane sends)
+  myid = __builtin_amdgcn_ds_permute(4 * to, (int)c.y);
+  __builtin_amdgcn_wave_barrier();
+  return __all(lane >= n || mykey != 0u);
+}
+
 // Lane-major keys again, each lane's keys sorted first (descending, equal keys keep their index
 // order: an odd-even transposition sort with strict compares never lets equal keys pass each other).
 // A round is then the wave-wide maximum of the lanes' heads and a pop in the winning lane — the
 // per-lane scan over NPL registers, a chain of dependent compares and selects, leaves the
 // rounds.  The keys' original register indices travel in 4-bit fields of one word.
-// runner_up (optional): the expert ranked k + 1, or -1 when there is none, the same in every lane.
+// runner_up (optional): the expert ranked k + 1, or -1 when there is none, the same in every lane.  Where the keys allow it the ranks
+// are counted instead (topk_by_count; buf: its LDS).
 template <int NPL>
-__device__ __forceinline__ void topk_select_sorted(uint32_t (&key)[NPL], int lane, int k, int* ids_row,
-                                                   float* ws_row, int* runner_up = nullptr) {
+__device__ __forceinline__ void topk_select_sorted(uint32_t (&key)[NPL], int lane, int k, int* ids_row, float* ws_row,
+                                                   uint2* buf, int* runner_up = nullptr) {
   static_assert(NPL <= 8, "4-bit index fields in one 32-bit word");
+  {
+    uint32_t kr;
+    int id;
+    // (two more than k: equal keys across either border are for the rounds)
+    if (k <= 60 && topk_by_count<NPL>(key, lane, k + 2, buf, kr, id)) {
+      const float v = __uint_as_float(kr - 1u);
+      double sum = 0.0;
+      for (int r = 0; r < k; r++) sum += (double)__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), r));  // selection order
+      if (lane < k) {
+        ids_row[lane] = id;
+        ws_row[lane] = (float)((double)v / sum);
+      }
+      if (runner_up) *runner_up = __builtin_amdgcn_readlane(id, k);
+      return;
+    }
+  }
   uint32_t jj[NPL];
 #pragma unroll
   for (int j = 0; j < NPL; j++) jj[j] = (uint32_t)j;
@@ -276,7 +345,7 @@ __device__ __forceinline__ void topk_wave(const float* __restrict__ lg, int* __r
     const int e = NPL * lane + j;
     key[j] = e < E ? __float_as_uint((float)((double)p[j] / se)) + 1u : 0u;
   }
-  if constexpr (NPL <= 8) topk_select_sorted<NPL>(key, lane, k, ids_row, ws_row);
+  if constexpr (NPL <= 8) topk_select_sorted<NPL>(key, lane, k, ids_row, ws_row, (uint2*)pbuf);
   else topk_select_lm<NPL>(key, lane, k, ids_row, ws_row);
 }
 
@@ -293,7 +362,7 @@ template <int NPL, bool COH, int NT = 256, bool CHECK = false>
 __device__ float topk_block(const float* lg, int* ids_row, float* ws_row, int E, int k, float ulps = 4.8e-7f) {
   constexpr int NPT = (64 * NPL + NT - 1) / NT;  // values per thread
   constexpr int NW = NT / 64;
-  __shared__ float pb[64 * NPL];
+  __shared__ __attribute__((aligned(16))) float pb[64 * NPL];
   __shared__ uint32_t keys[64 * NPL];
   __shared__ double red[NW];
   __shared__ float redf[NW];
@@ -385,7 +454,7 @@ __device__ float topk_block(const float* lg, int* ids_row, float* ws_row, int E,
     for (int j = 0; j < NPL; j++) key[j] = keys[NPL * lane + j];
     if constexpr (NPL <= 8) {
       int ru = -1;
-      topk_select_sorted<NPL>(key, lane, k, ids_row, ws_row, CHECK ? &ru : nullptr);
+      topk_select_sorted<NPL>(key, lane, k, ids_row, ws_row, (uint2*)pb, CHECK ? &ru : nullptr);
       if constexpr (CHECK) {
         float sl = INFINITY;
         if (topk_fast_handled<NPL>(lg, E, k)) {
@@ -433,6 +502,7 @@ __device__ float topk_block(const float* lg, int* ids_row, float* ws_row, int E,
 template <int NPL>
 __device__ int topk_ids_by_logit(const float* lg, int* ids_row, int E, int k, float tol = 0.f, float ulps = 4.8e-7f) {
   __shared__ int fast_ok;
+  __shared__ uint2 cand[64];
   const int tid = threadIdx.x, lane = tid & 63;
   bool handled = false;
   handled = topk_fast_handled<NPL>(lg, E, k);
@@ -453,40 +523,44 @@ __device__ int topk_ids_by_logit(const float* lg, int* ids_row, int E, int k, fl
           key[4 * q + i] = idx < E ? o : 0u;
         }
       }
-#pragma unroll
-      for (int j = 0; j < 8; j++) jj[j] = (uint32_t)j;
-#pragma unroll
-      for (int pass = 0; pass < 8; pass++) {
-#pragma unroll
-        for (int i = pass & 1; i + 1 < 8; i += 2) {
-          const uint32_t ka = key[i], kb = key[i + 1], ia = jj[i], ib = jj[i + 1];
-          const bool sw = kb > ka;
-          key[i] = umax(ka, kb); key[i + 1] = umin(ka, kb);
-          jj[i] = sw ? ib : ia; jj[i + 1] = sw ? ia : ib;
-        }
-      }
-      uint32_t jw = 0;
-#pragma unroll
-      for (int j = 0; j < 8; j++) jw |= jj[j] << (4 * j);
       uint32_t mykey = 0;
       int myid = 0;
-      for (int r = 0; r <= k; r++) {  // k + 1 rounds: the runner-up is needed for the gap test
-        const uint32_t wm = wave_umax(key[0]);
-        const int wl = __builtin_ctzll(__ballot(key[0] == wm));
-        const int wj = __builtin_amdgcn_readlane((int)jw, wl) & 15;
-        if (lane == r) {
-          mykey = wm;
-          myid = 8 * wl + wj;
-        }
-        const bool me = lane == wl;
+      if (!topk_by_count<8>(key, lane, k + 1, cand, mykey, myid)) {
+        mykey = 0;
+        myid = 0;
 #pragma unroll
-        for (int j = 0; j + 1 < 8; j++) {
-          const uint32_t cur = key[j], nxt = key[j + 1];
-          key[j] = me ? nxt : cur;
+        for (int j = 0; j < 8; j++) jj[j] = (uint32_t)j;
+#pragma unroll
+        for (int pass = 0; pass < 8; pass++) {
+#pragma unroll
+          for (int i = pass & 1; i + 1 < 8; i += 2) {
+            const uint32_t ka = key[i], kb = key[i + 1], ia = jj[i], ib = jj[i + 1];
+            const bool sw = kb > ka;
+            key[i] = umax(ka, kb); key[i + 1] = umin(ka, kb);
+            jj[i] = sw ? ib : ia; jj[i + 1] = sw ? ia : ib;
+          }
         }
-        const uint32_t last = key[7], jsh = jw >> 4;
-        key[7] = me ? 0u : last;
-        jw = me ? jsh : jw;
+        uint32_t jw = 0;
+#pragma unroll
+        for (int j = 0; j < 8; j++) jw |= jj[j] << (4 * j);
+        for (int r = 0; r <= k; r++) {  // k + 1 rounds: the runner-up is needed for the gap test
+          const uint32_t wm = wave_umax(key[0]);
+          const int wl = __builtin_ctzll(__ballot(key[0] == wm));
+          const int wj = __builtin_amdgcn_readlane((int)jw, wl) & 15;
+          if (lane == r) {
+            mykey = wm;
+            myid = 8 * wl + wj;
+          }
+          const bool me = lane == wl;
+#pragma unroll
+          for (int j = 0; j + 1 < 8; j++) {
+            const uint32_t cur = key[j], nxt = key[j + 1];
+            key[j] = me ? nxt : cur;
+          }
+          const uint32_t last = key[7], jsh = jw >> 4;
+          key[7] = me ? 0u : last;
+          jw = me ? jsh : jw;
+        }
       }
       // lane r holds rank r: its logit against the next rank's (the subtraction of close floats is exact)
       const uint32_t nk = (uint32_t)__shfl_down((int)mykey, 1, 64);

@@ -135,6 +135,35 @@ def test_router_topk_ties_and_wide_range(capi, oracle):
     assert list(ids[0, :k]) == list(range(10))
 
 
+@pytest.mark.parametrize("E,k", [(512, 10), (512, 1), (512, 15), (500, 8), (260, 4), (64, 10), (17, 16), (16, 16)])
+def test_router_topk_by_counting(capi, oracle, E, k):
+    """Rows on either side of what the selection by counting settles: the best ones in one lane's or one row of lanes' experts, a
+    dozen to all experts above its bound, equal keys inside, across and behind the k-th place, fewer keys than places."""
+    rng = np.random.default_rng(E + k)
+    rows = [rng.standard_normal(E).astype(np.float32) for _ in range(40)]
+    for first, n in ((0, 8), (E // 2, 16), (0, 128), (max(E - 128, 0), 128)):  # the best are neighbours
+        r = rng.standard_normal(E).astype(np.float32)
+        r[first:first + n] += 5
+        rows.append(r)
+    for n in (3, 11, 12, 13, 60, 64, 65, 70, E):                               # n close to one another, the rest far below
+        r = rng.standard_normal(E).astype(np.float32) * 0.1 - 6
+        at = rng.permutation(E)[:n]
+        r[at] = 1 + 1e-3 * rng.permutation(len(at)).astype(np.float32)
+        rows.append(r)
+    for i in (0, k - 2, k - 1, k, k + 1):                                      # two equal logits at places i and i + 1
+        r = rng.standard_normal(E).astype(np.float32)
+        o = np.argsort(-r)
+        if 0 <= i and i + 1 < E:
+            r[o[i]] = r[o[i + 1]]
+        rows.append(r)
+    lg = np.stack(rows)
+    ids, ws = (a.cpu().numpy() for a in capi.router_topk(gpu(lg), k))
+    for t in range(len(lg)):
+        _, io, wo = oracle.softmax_topk(lg[t], k)
+        assert (ids[t, :k] == io).all(), t
+        assert same_bits(ws[t, :k], wo), t
+
+
 # ---------- permutation: exact ----------
 @pytest.mark.parametrize("P,E,k", [(1, 512, 10), (20, 512, 10), (32, 512, 10), (33, 512, 10), (32, 20, 16), (255, 512, 10), (257, 40, 6), (5000, 512, 10), (3, 7, 7)])
 def test_routing_exact(capi, oracle, P, E, k):
