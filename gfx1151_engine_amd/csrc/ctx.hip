@@ -1089,7 +1089,7 @@ static int forward_batch_impl(moe_ctx* c, MoeLayer& L, const float* x, int P, fl
   // middle sizes: tiles of few pairs, the weights streamed into registers
   const StreamKinds sk = stream_kinds(L, g);
   int cap = fused || sk.up < 0 || !c->stream_gemm ? 0 : moe_stream_tile_cap(P, g.topk, g.experts, sk.up, sk.dn, g.d, g.mid);
-  const int sxl = sk.up >= MOE_STREAM_Q4K ? 2 : sk.up == MOE_STREAM_TABLE ? 0 : 1;  // the order of activations it reads
+  const int sxl = q4k ? 2 : sk.up == MOE_STREAM_TABLE ? 0 : 1;  // the order of activations it reads
   if (c->x16_ext && sxl != batch_x16_layout(L, g)) cap = 0;
   // routed and shared experts in launches of their own
   bool split = shd || (q4k && !kd.uniform(L)) || (cap && L.has_shared && !sk.with_sh);

@@ -53,15 +53,15 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // F_Q4E, F_Q5E: Q4_K and Q5_K weights rounded to f16 once, from their exact values
 // F_I4D: i4r with the scaled dequantisation (3001 skewed tokens, gate/up 509 -> 459 us, down 284 -> 266; 130: 239 -> 227, 134 -> 129.
 // Q4_K gained half a per cent of a layer with it and Q5_K lost 15 at 1200 tokens, both short of registers.)
-enum { F_DN, F_AFF, F_TAB, F_I4D, F_I4R, F_Q4K, F_Q5K, F_Q80, F_Q4E, F_Q5E };
+enum { F_DN, F_AFF, F_TAB, F_I4R, F_Q4K, F_Q5K, F_Q80, F_Q4E, F_Q5E, F_I4D };
 constexpr bool q4(int FMT) { return FMT == F_Q4K || FMT == F_Q4E; }
 constexpr bool q5(int FMT) { return FMT == F_Q5K || FMT == F_Q5E; }
 constexpr bool i4(int FMT) { return FMT == F_I4D || FMT == F_I4R; }
 constexpr bool scaled(int FMT) { return FMT == F_DN || FMT == F_I4D; }
 constexpr bool once_rounded(int FMT) { return FMT == F_Q4E || FMT == F_Q5E; }
-constexpr bool scale_plane(int FMT) { return FMT <= F_I4R; }
+constexpr bool scale_plane(int FMT) { return FMT <= F_I4R || FMT == F_I4D; }
 // order of activations and hid (moe_f32_to_f16's layouts)
-constexpr int x_layout(int FMT) { return FMT == F_TAB ? 0 : FMT <= F_I4R ? 1 : 2; }
+constexpr int x_layout(int FMT) { return FMT == F_TAB ? 0 : scale_plane(FMT) ? 1 : 2; }
 
 constexpr int XROW = 512;  // bytes of a line of one pair row (256 f16)
 constexpr size_t LDS_MOST = 160 * 1024;  // of a CU
@@ -223,7 +223,7 @@ __device__ __forceinline__ void line_mma(const Line<FMT> (&q)[F], const uint32_t
           } else {
             const float s = (float)s2.x;
             as[f][0] = both(C.cb_a[f0 + f] * s);
-            bs[f][0] = bs[f][1] = both(C.cb_b[f0 + f] * s);
+            bs[f][0] = bs[f][1] = FMT == F_I4D ? as[f][0] * both(-0x1p-21f) : both(C.cb_b[f0 + f] * s);  // (i4r: -8; exact)
             as[f][1] = scaled(FMT) ? as[f][0] * both(0.0625f) : as[f][0];
           }
         }
@@ -440,6 +440,10 @@ __device__ __forceinline__ Consts make_consts(const SW& L, int pexp, const TabEn
       const float s24 = __builtin_ldexpf(1.f, 24 + pexp), sp = __builtin_ldexpf(1.f, pexp);
       C.cb_a[0] *= s24; C.cb_a[1] *= s24; C.cb_b[0] *= sp; C.cb_b[1] *= sp;
       oscale = __builtin_ldexpf(1.f, -pexp);
+      // (the same in every lane: as scalars they leave the down launches of 64 pairs their registers.  The layer, us: 2048 tokens q4cp 701
+      // 696, 3001 skewed i4r 882 871)
+      auto scalar = [](float& f) { f = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(f))); };
+      scalar(C.cb_a[0]); scalar(C.cb_a[1]); scalar(C.cb_b[0]); scalar(C.cb_b[1]); scalar(oscale);
     }
   } else if (FMT == F_TAB) {
     // TABC copies side by side: lanes that differ in their low bits never meet on a bank (with one copy the look-ups of a
@@ -887,9 +891,8 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
 constexpr int DN_ONE = 3;  // lines of the rows that a wave takes whole
 constexpr int up_waves(int FMT, int MFX) { return MFX == 4 || i4(FMT) ? 8 : 4; }
 // waves per SIMD asked for: what the registers of the lines in flight leave.  (Gate/up with Q5_K rounded once, 32 pairs: three; with
-// four 21 registers went to scratch inside the loop, 757 us for 702 at 1200 tokens of 2560 x 640.  A few kernels keep 1 .. 4
-// registers of their prologue in scratch until the epilogue, F_DN's down launch with 64 pairs an address once per pass:
-// gate/up F_Q5K with 32 pairs; down F_DN and F_TAB with 64.  F_Q5K with three waves has none and is no
+// four 21 registers went to scratch inside the loop, 757 us for 702 at 1200 tokens of 2560 x 640.  Two kernels keep 1 .. 4
+// registers of their prologue in scratch until the epilogue: gate/up F_Q5K with 32 pairs, down F_TAB with 64.  F_Q5K with three waves has none and is no
 // faster: 808 us for 799 at 515 tokens, 1159 for 1152 at 1700.)
 constexpr int simd_waves(int FMT, bool UP, int MFX, int NW) {
   if (UP) return FMT == F_Q5E && MFX == 2 ? 3 : 4;
@@ -1080,7 +1083,7 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
   // (down: groups of 32 rows, and a tile's hid rows in LDS)
   if (up && (uint64_t)x_rows * (uint64_t)k * 2 >= 1ull << 32) return MOE_E_UNSUPPORTED;  // (32-bit byte offsets into x)
   if (up ? k < 256 : k < 128 || m % 32 || smem_bytes(fmt, false, cap / 16, (k + 255) / 256, 1) > LDS_MOST) return MOE_E_UNSUPPORTED;
-  if (up && (m % 16 || (fmt >= F_Q4K && m % 64) || (i4(fmt) && m % 128))) return MOE_E_UNSUPPORTED;
+  if (up && (m % 16 || (!plane && m % 64) || (i4(fmt) && m % 128))) return MOE_E_UNSUPPORTED;
   if ((up && fmt == F_Q80) || (!up && (q5(fmt) || once_rounded(fmt))) || (cap > 32 && (q5(fmt) || fmt == F_Q80))) return MOE_E_UNSUPPORTED;
   if (i4(fmt) && up != (rot != nullptr)) return MOE_E_INVALID;
   if (rot && (!rot->svh_gu || !rot->suh_dn)) return MOE_E_INVALID;

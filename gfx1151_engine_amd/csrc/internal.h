@@ -78,8 +78,8 @@ int moe_launch_gemm_q4cp(bool up, const moe_lutw* routed, const moe_lutw* sh, in
                          bool q5k = false, bool nat = false, const int8_t* pexp_routed = nullptr,
                          const int8_t* pexp_sh = nullptr, const moe_rotv* rot = nullptr);
 // Grouped GEMM for tiles of few pairs, weights streamed into registers (gemm_stream.hip)
-enum { MOE_STREAM_SCALED, MOE_STREAM_AFFINE, MOE_STREAM_TABLE, MOE_STREAM_I4R_SCALED, MOE_STREAM_I4R, MOE_STREAM_Q4K, MOE_STREAM_Q5K, MOE_STREAM_Q8_0,
-       MOE_STREAM_Q4K_ONCE, MOE_STREAM_Q5K_ONCE };
+enum { MOE_STREAM_SCALED, MOE_STREAM_AFFINE, MOE_STREAM_TABLE, MOE_STREAM_I4R, MOE_STREAM_Q4K, MOE_STREAM_Q5K, MOE_STREAM_Q8_0,
+       MOE_STREAM_Q4K_ONCE, MOE_STREAM_Q5K_ONCE, MOE_STREAM_I4R_SCALED };
 int moe_stream_tile_cap(int P, int k, int experts, int fmt_up, int fmt_dn, int d, int mid);
 int moe_stream_tile_cap_least(int P, int k, int experts);
 int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const moe_lutw* sh, int n_experts, const __half* x, int x_rows,
