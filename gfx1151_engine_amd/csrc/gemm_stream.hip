@@ -13,11 +13,10 @@
 //     activations agree; a chunk is one scale group of 32 columns (q4cp), half of a 64-column run (Q4_K, Q5_K), a lane group's
 //     run (Q8_0).
 //   - gate/up keeps two lines per wave in flight, line by line; down requests a fragment's whole rows at once where they are
-//     three lines, else two lines at a time.  Rows start 64 bytes off the 128-byte cache lines (the codebook heads the tensor),
-//     so every line shares a cache line with the next one, and read a line at a time a third of the traffic is fetched twice
-//     (1.66 GB for 1.26, at 6.15 TB/s); whole rows brought down from 6.9 to 5.3 M cache lines (of 5.0).  For gate/up the same,
-//     pairs of lines with four in registers, fetched 1.51 GB and was no faster (270 us either way, three waves per SIMD for
-//     four).
+//     three lines, else two lines at a time.  q4cp rows start 64 bytes off the 128-byte cache lines (the codebook heads the
+//     tensor), and what one visit leaves of a cache line is gone from L2 before the next; so whole rows at once brought down
+//     from 6.9 to 5.3 M cache lines (of 5.0), and gate/up turns its lines by half a line, the last of a row ending with the row's
+//     first 64 bytes (up_rotates).
 //   - activations (16 pairs per MFMA, up to 64 per tile) go through LDS: gate/up one line at a time, double-buffered, one
 //     LDS-only barrier per line; down, where they are short, once per block, which then runs without barriers.
 //   - no branch stands around a load of the loops: the compiler counts outstanding loads exactly only along straight code
@@ -105,9 +104,10 @@ struct Line {
   uint4 hd[1], qh[1];             // K-quants: block header; Q5_K: this lane's fifth bits
   uint32_t last;                  // Q8_0: the 17th word
 };
-// b: wave-uniform address of the line's first row, o: this lane's row offset, half: the second half does not exist
+// b: wave-uniform address of the line's first row, o: this lane's row offset, half: the second half does not exist; second: where
+// the codes' second half lies behind the first, 64 bytes as a rule
 template <int FMT>
-__device__ __forceinline__ void load_line(Line<FMT>& q, const uint8_t* b, uint32_t o, int g, bool half) {
+__device__ __forceinline__ void load_line(Line<FMT>& q, const uint8_t* b, uint32_t o, int g, bool half, ptrdiff_t second = 64) {
   if constexpr (FMT == F_Q80) {
     // lane group g = columns 64 g .. of the line: two blocks, 68 bytes (4-byte aligned)
     const uint8_t* s = b + (o + 68u * (half ? (uint32_t)(g & 1) : (uint32_t)g));
@@ -122,7 +122,7 @@ __device__ __forceinline__ void load_line(Line<FMT>& q, const uint8_t* b, uint32
     if (q4(FMT) || q5(FMT)) q.hd[0] = *(const uint4*)(b + o);
     if (q5(FMT)) q.qh[0] = *(const uint4*)(b + (o + 16u + 16u * (uint32_t)(g & 1)));
     q.c[0] = *(const uint4*)(b + (o + C0 + 16u * (uint32_t)g));
-    const uint8_t* b1 = b + (half ? 0 : 64);
+    const uint8_t* b1 = b + (half ? 0 : second);
     q.c[1] = *(const uint4*)(b1 + (o + C0 + 16u * (uint32_t)g));
   }
 }
@@ -370,17 +370,23 @@ __device__ __forceinline__ void half_mma(const uint4 (&c)[F], const Deq<F>& D, c
 
 // Scales of four lines of a row (64 bytes, i4r: 16) from line `first` on: lane group i fetches line first + i's, the exchange
 // below then hands every lane one word per line with its own two scales.  (Past the row's end: one address for all lanes.)
+// ro: bytes of codes by which the lines are rotated (up_tile); last: the line whose second half is then the row's first 64 bytes
 template <int FMT>
 struct Raw { uint4 v; };
 template <int FMT>
-__device__ __forceinline__ Raw<FMT> load_scales(const uint8_t* b, uint32_t o, int first, int g, int sstride) {
+__device__ __forceinline__ Raw<FMT> load_scales(const uint8_t* b, uint32_t o, int first, int g, int sstride, uint32_t ro = 0, int last = -1) {
   Raw<FMT> r;
   if (i4(FMT)) {  // one word per line: both scales, the same for all lane groups
     const uint32_t p = 4u * (uint32_t)(first + g);
     r.v.x = *(const uint32_t*)(b + (p < (uint32_t)sstride ? o + p : 0u));
-  } else {
+  } else if (last < 0) {
     const uint32_t p = 16u * (uint32_t)(first + g);
     r.v = *(const uint4*)(b + (p < (uint32_t)sstride ? o + p : 0u));
+  } else {
+    const uint32_t p = 16u * (uint32_t)(first + g) + (ro >> 3), p1 = ro && first + g == last ? 0u : p + 8u;
+    const bool past = first + g > last;
+    const uint2 u = *(const uint2*)(b + (past ? 0u : o + p)), v = *(const uint2*)(b + (past ? 0u : o + p1));
+    r.v = make_uint4(u.x, u.y, v.x, v.y);
   }
   return r;
 }
@@ -484,12 +490,10 @@ __device__ __forceinline__ void x_addrs(int n, int g, uint32_t (&xa)[8]) {
 // ---- gate/up ----
 // HALVES (64 pairs of q4cp codes): the codes go through registers in half lines, the next line's activations in two parts, and
 // half_mma orders the rest.  Else whole lines, one ahead of the line worked on, in the compiler's order.  What either is
-// bound by is traffic first: 16.6 M cache lines for the 10.6 M that 2048 tokens' gate/up rows and scales have (q4cp; rows are
-// visited a line, their scales four lines at a time, and what a visit leaves of a cache line is gone from L2 before the
-// next), 345 us of 386 at the 6.15 TB/s that plain loads reach; half lines need 15.2 M.  us of the launch, whole lines and
+// bound by with 64 pairs is traffic first: 16.6 M cache lines for the 10.6 M that 2048 tokens' gate/up rows and scales have (q4cp; rows are
+// visited a line, their scales four lines at a time), 345 us of 386 at the 6.15 TB/s that plain loads reach; half lines need 15.2 M.  us of the launch, whole lines and
 // halves: 2048 tokens q4cp 386 371, table 483 432; but 515 q4cp (32 pairs) 312 320, 1500 Q4_K 404 425, 2048 i4r 401 406.
-// Tried beside it: lines that begin where the cache lines do (rows rotated by half a line: no fewer cache lines, +20 us),
-// a row's scales all at once (registers: spills at 64 pairs), non-temporal loads (21 M cache lines), 32 gate and 32 up rows to
+// Tried beside it: a row's scales all at once (registers: spills at 64 pairs), non-temporal loads (21 M cache lines), 32 gate and 32 up rows to
 // a wave with two waves per SIMD (half the LDS reads, +12 us), and x in registers with the waves of a block splitting K, which
 // reads 9.8 M cache lines for 9.75 M at 130 tokens but leaves two waves per SIMD whose arithmetic does not hide (280 us for 268).
 // (Straight code of two lines, where K is known to be whole pairs of lines, gave the compiler room to move loads and operands
@@ -501,6 +505,14 @@ constexpr bool up_halves(int FMT, int MFX) { return MFX == 4 && FMT <= F_TAB; }
 // 100 tokens (32 pairs) 128.3 126.6, 200 (64 pairs) 143.0 135.7, 256 146.4 140.7; 2560 x 640 200 123.5 116.2.  With one table there
 // is room, and reading again costs: 200 tokens without a shared expert 126.6 127.9
 constexpr size_t up_scales(int FMT, int tabs) { return FMT == F_TAB && tabs == 2 ? 0 : 256; }
+// Tiles of 16 and 32 pairs of q4cp codes: lines that begin where the cache lines do, where the rows of both tensors start in the
+// middle of one (up_tile's ro; activations and scales follow), and the scales of twelve (eight) lines requested together.
+// 130 tokens, gate/up: 13.3 M cache lines of 128 bytes for 9.8 M -> 9.9 M, 282 -> 265 us; the lines alone 262, of the scales alone 253.
+// us of the layer, before and after: q4cp 40 tokens 283 266, 130 457 429, 515 540 509, 800 585 560, 2560 x 640 200 362 330; table 40 313
+// 301, 515 588 562.  Not for tiles of 64, whose half lines come half a stage apart: 1200 tokens 623 -> 635, 2048 706 -> 711; nor
+// is there room for more scales (32 pairs, twelve lines' instead of eight: up to 9 registers in scratch, 515 tokens 512).
+constexpr bool up_rotates(int FMT, int MFX) { return FMT <= F_TAB && MFX < 4; }
+constexpr int up_scale_groups(int FMT, int MFX) { return FMT > F_TAB || MFX == 4 ? 1 : MFX == 2 ? 2 : 3; }
 template <int FMT, int MFX, int MF, bool ROT, int NW>
 __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const moe_tile tile, int nb, const __half* __restrict__ x,
                                         const int* __restrict__ tokidx, __half* __restrict__ out, int M, int K, int pexp,
@@ -529,6 +541,7 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
     sb[f] = scale_plane(FMT) ? (f ? L.sc_up : L.sc) + first * (size_t)L.sstride : nullptr;
   }
   const uint32_t wo = (uint32_t)r * RB, so = (uint32_t)r * (uint32_t)L.sstride;
+  const uint32_t ro = up_rotates(FMT, MFX) && (K & 255) == 0 && ((uintptr_t)wb[0] & 127) == 64 && ((uintptr_t)wb[1] & 127) == 64 ? 64u : 0u;
   Line<FMT> ln[HALVES ? 1 : DB][2];
   uint4 cd[HALVES ? DB : 1][2][2];  // line, half, fragment
   // (past the last line: one address for all lanes instead of a branch around the load)
@@ -536,12 +549,14 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
 #pragma unroll
     for (int f = 0; f < 2; f++) {
       const bool past = i >= nline;
-      load_line<FMT>(q[f], wb[f] + (past ? (size_t)0 : (size_t)i * LB), past ? 0u : wo, past ? 0 : g, tail && i >= nline - 1);
+      load_line<FMT>(q[f], wb[f] + (past ? (size_t)0 : (size_t)i * LB + ro), past ? 0u : wo, past ? 0 : g, tail && i >= nline - 1,
+                     ro && i == nline - 1 ? (ptrdiff_t)64 - (ptrdiff_t)RB : (ptrdiff_t)64);
     }
   };
   auto load_half = [&](uint4(&q)[2], int i, int E) {
     const bool past = i >= nline;
-    const size_t at = past ? (size_t)0 : (size_t)i * LB + (E && !(tail && i == nline - 1) ? 64 : 0);
+    const bool end = i == nline - 1;
+    const size_t at = past ? (size_t)0 : E && ro && end ? (size_t)0 : (size_t)i * LB + ro + (E && !(tail && end) ? 64 : 0);
 #pragma unroll
     for (int f = 0; f < 2; f++) q[f] = *(const uint4*)(wb[f] + at + (past ? 0u : wo + 16u * (uint32_t)g));
   };
@@ -566,11 +581,15 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
   }
   TabEntry te;
   if constexpr (MFX < 4) te = load_entry<FMT, true, NT, tab_copies(true, MFX)>(L, tid);
-  Raw<FMT> raw[2];
+  constexpr int SD = up_scale_groups(FMT, MFX);  // groups of four lines whose scales are in registers
+  Raw<FMT> raw[2][SD];
   uint32_t sq[2][4];
+  auto scales_of = [&](int f, int i) { return load_scales<FMT>(sb[f], so, i, g, L.sstride, ro, up_rotates(FMT, MFX) ? nline - 1 : -1); };
   if (scale_plane(FMT)) {
 #pragma unroll
-    for (int f = 0; f < 2; f++) raw[f] = load_scales<FMT>(sb[f], so, 0, g, L.sstride);
+    for (int f = 0; f < 2; f++)
+#pragma unroll
+      for (int k = 0; k < SD; k++) raw[f][k] = scales_of(f, 4 * k);
   }
 #pragma unroll
   for (int b = 0; b < DB; b++) {
@@ -596,13 +615,15 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
   auto fetch_x = [&](int i, auto part) {
     constexpr int h = XH * decltype(part)::value;
     i = i < nline ? i : nline - 1;
-    const bool half = tail && i == nline - 1;
-    const uint8_t* const xb = (const uint8_t*)x + 512 * (size_t)i;
-    const uint32_t back = half && xc >= 16 ? 256u : 0u;
-    if constexpr (h < XL) xv0 = *(const uint4*)(xb + (xr[h] - back));
-    if constexpr (XH > 1 && h + 1 < XL) xv1 = *(const uint4*)(xb + (xr[h + 1] - back));
-    if constexpr (XH > 2 && h + 2 < XL) xv2 = *(const uint4*)(xb + (xr[h + 2] - back));
-    if constexpr (XH > 3 && h + 3 < XL) xv3 = *(const uint4*)(xb + (xr[h + 3] - back));
+    // (the last line: half of it repeated where the row has none, the row's first columns where the lines are rotated)
+    const bool end = i == nline - 1 && xc >= 16;
+    const uint8_t* const xb = (const uint8_t*)x + (up_rotates(FMT, MFX) ? (size_t)0 : 512 * (size_t)i);
+    const uint32_t at = up_rotates(FMT, MFX) ? 512u * (uint32_t)i + 4u * ro - (!end ? 0u : tail ? 256u : ro ? 2u * (uint32_t)K : 0u)
+                                             : end && tail ? 0u - 256u : 0u;
+    if constexpr (h < XL) xv0 = *(const uint4*)(xb + (xr[h] + at));
+    if constexpr (XH > 1 && h + 1 < XL) xv1 = *(const uint4*)(xb + (xr[h + 1] + at));
+    if constexpr (XH > 2 && h + 2 < XL) xv2 = *(const uint4*)(xb + (xr[h + 2] + at));
+    if constexpr (XH > 3 && h + 3 < XL) xv3 = *(const uint4*)(xb + (xr[h + 3] + at));
   };
   auto put_x = [&](int buf, auto part) {
     constexpr int h = XH * decltype(part)::value;
@@ -644,7 +665,7 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
       __builtin_amdgcn_sched_barrier(0);
       if (V == 0) {
 #pragma unroll
-        for (int f = 0; f < 2; f++) take_scales<FMT>(raw[f], sq[f]);
+        for (int f = 0; f < 2; f++) take_scales<FMT>(raw[f][0], sq[f]);
       }
       const uint32_t sw[2] = {sq[0][V], sq[1][V]};
       half_mma<FMT, 2, MF, XROW, tab_copies(true, MFX), 0>(cd[S][0], make_deq<FMT, 2, 0>(sw, C), C, smem + B * XBUF, xa, acc);
@@ -660,7 +681,7 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
       load_half(cd[S][1], i + DB, 1);
       if (V == 2) {  // (the next four lines')
 #pragma unroll
-        for (int f = 0; f < 2; f++) raw[f] = load_scales<FMT>(sb[f], so, i + 2, g, L.sstride);
+        for (int f = 0; f < 2; f++) raw[f][0] = scales_of(f, i + 2);
       }
       __builtin_amdgcn_sched_barrier(0);
     } else {
@@ -674,8 +695,10 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
     if (scale_plane(FMT) && !HALVES) {
 #pragma unroll
       for (int f = 0; f < 2; f++) {
-        take_scales<FMT>(raw[f], sq[f]);
-        raw[f] = load_scales<FMT>(sb[f], so, i + 4, g, L.sstride);
+        take_scales<FMT>(raw[f][0], sq[f]);
+#pragma unroll
+        for (int k = 0; k + 1 < SD; k++) raw[f][k] = raw[f][k + 1];
+        raw[f][SD - 1] = scales_of(f, i + 4 * SD);
       }
     }
     stage(std::integral_constant<int, 0>{}, i);

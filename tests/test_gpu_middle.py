@@ -392,6 +392,41 @@ def test_few_pair_tiles_multiply_the_same_weights(capi, kind, kw, d, mid, T):
     assert (y1 == y0).all()
 
 
+# where the code planes lie against the cache lines (a blob's codes start 64 bytes behind it): the streaming GEMM turns its lines by half
+# a line where rows start in the middle of one -- in one tensor of a launch, in both, in none; rows of one line, of more
+# scales than are fetched at once (twelve lines) and of half a line more; tiles of 16, 32 and 64 pairs
+@pytest.mark.parametrize("kind", ["q4cp", "table"])
+@pytest.mark.parametrize("d,T", [(256, 33), (512, 64), (2560, 40), (3072, 64), (3328, 33), (640, 40), (3328, 70), (512, 130)])
+def test_lines_against_cache_lines(capi, oracle, kind, d, T):
+    import torch
+    rng = np.random.default_rng(d + T)
+    E, k, mid = 16, 4, 256
+    cb = None if kind == "q4cp" else np.sort(rng.standard_normal(16)).astype(np.float32)
+    hl = HostLayer(rng, d, mid, E, k, codebook=cb)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    yo, _, _ = oracle.moe_layer(hl.oracle_layer(), x)
+    m, dev = hl.to_gpu(max_tokens=T)
+
+    def at(name, offset):  # the blob moved by `offset` bytes inside an allocation
+        t = dev[name]
+        buf = torch.zeros(t.numel() + 256, dtype=torch.uint8, device="cuda")
+        buf[offset:offset + t.numel()] = t
+        dev[name + str(offset)] = buf
+        return buf[offset:offset + t.numel()]
+    ys = []
+    for experts, shared in ((0, 0), (64, 64), (64, 0), (0, 64), (16, 48)):
+        m.set_experts_q4cp(0, capi.wview(at("gate_up", experts), capi.Q4CP, E * 2 * mid, d),
+                           capi.wview(at("down", experts), capi.Q4CP, E * d, mid))
+        m.set_shared(0, capi.wview(at("shg", 0), capi.Q4CP, mid, d), capi.wview(at("shu", shared), capi.Q4CP, mid, d),
+                     capi.wview(at("shd", shared), capi.Q4CP, d, mid), capi.wview(dev["shsg"], capi.F32, 1, d))
+        ys.append(m.forward(0, gpu(x)).cpu().numpy())
+        assert m.last_path() == capi.PATH_BATCH
+        assert max_abs_rel(ys[-1], yo) <= 2e-3  # (as the other whole-layer tests of batches: f16 operands and intermediates)
+    m.close()
+    # against one another: the order of f32 sums of d terms, and f16 roundings of hid and pairs that it tips over (2^-11 each)
+    assert max(max_abs_rel(y, ys[0]) for y in ys[1:]) <= 2 * 2.0 ** -11
+
+
 # rows of hid of one line to eight, with and without a half line at the end; rows of d that are no whole blocks of sixteen waves
 STREAM_WIDTHS = [("q4cp", dict(fmt="q4cp"), 640, 256), ("q4cp", dict(fmt="q4cp"), 896, 384), ("q4cp", dict(fmt="q4cp"), 512, 1152),
                  ("q4cp", dict(fmt="q4cp"), 384, 2048), ("q4cp", dict(fmt="q4cp"), 256, 2560), ("q4cp-table", dict(fmt="q4cp", codebook=TABLE), 640, 512),
