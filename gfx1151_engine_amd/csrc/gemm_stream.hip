@@ -98,16 +98,19 @@ __device__ __forceinline__ int pos_elem(int wv, int i) {
 }
 
 // ---- one line of one weight fragment (16 rows) in registers ----
-template <int FMT>
+// SPLIT: a K-quant's header and fifth bits in parts (gather4)
+constexpr bool split_head(int MFX) { return MFX < 4; }
+template <int FMT, bool SPLIT>
 struct Line {
   uint4 c[FMT == F_Q80 ? 4 : 2];  // codes
-  uint4 hd[1], qh[1];             // K-quants: block header; Q5_K: this lane's fifth bits
+  typename std::conditional<SPLIT, uint32_t, uint4>::type hd;  // K-quants: word g of the block's header, or all of it
+  uint2 qh;                       // Q5_K: half of the fifth bits of lane groups g and g ^ 2
   uint32_t last;                  // Q8_0: the 17th word
 };
 // b: wave-uniform address of the line's first row, o: this lane's row offset, half: the second half does not exist; second: where
 // the codes' second half lies behind the first, 64 bytes as a rule
-template <int FMT>
-__device__ __forceinline__ void load_line(Line<FMT>& q, const uint8_t* b, uint32_t o, int g, bool half, ptrdiff_t second = 64) {
+template <int FMT, bool SPLIT>
+__device__ __forceinline__ void load_line(Line<FMT, SPLIT>& q, const uint8_t* b, uint32_t o, int g, bool half, ptrdiff_t second = 64) {
   if constexpr (FMT == F_Q80) {
     // lane group g = columns 64 g .. of the line: two blocks, 68 bytes (4-byte aligned)
     const uint8_t* s = b + (o + 68u * (half ? (uint32_t)(g & 1) : (uint32_t)g));
@@ -119,12 +122,28 @@ __device__ __forceinline__ void load_line(Line<FMT>& q, const uint8_t* b, uint32
     q.last = *(const uint32_t*)(s + 64);
   } else {
     constexpr uint32_t C0 = q4(FMT) ? 16 : q5(FMT) ? 48 : 0;
-    if (q4(FMT) || q5(FMT)) q.hd[0] = *(const uint4*)(b + o);
-    if (q5(FMT)) q.qh[0] = *(const uint4*)(b + (o + 16u + 16u * (uint32_t)(g & 1)));
+    if constexpr (q4(FMT) || q5(FMT)) q.hd = *(const decltype(q.hd)*)(b + (o + (SPLIT ? 4u * (uint32_t)g : 0u)));
+    if (q5(FMT)) q.qh = *(const uint2*)(b + (o + 16u + 16u * (uint32_t)(g & 1) + 8u * (uint32_t)(g >> 1)));
     q.c[0] = *(const uint4*)(b + (o + C0 + 16u * (uint32_t)g));
     const uint8_t* b1 = b + (half ? 0 : second);
     q.c[1] = *(const uint4*)(b1 + (o + C0 + 16u * (uint32_t)g));
   }
+}
+
+// A K-quant's header and fifth bits are the same for all (two) lane groups of a row, and a load costs the address unit 64 cycles
+// for 16 bytes of every lane, 16 for 4: each group fetches its part, and these hand the others' over.  us of the layer, whole and in
+// parts: Q4_K 130 tokens 490 487, 515 573.5 570; Q5_K / Q8_0 300 768 763, 800 844 830, 1300 954 937, 2560 x 640 3000 1147 1127.  (Tiles of
+// 64 pairs, Q4_K, where the vector port counts for more: 1300 tokens 694 698, 2500 898 901; they fetch it whole.)
+// word g of lane group g -> all four words
+__device__ __forceinline__ uint4 gather4(uint32_t v) {
+  const auto p = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  const auto a = __builtin_amdgcn_permlane32_swap(p[0], p[0], false, false), b = __builtin_amdgcn_permlane32_swap(p[1], p[1], false, false);
+  return make_uint4(a[0], b[0], a[1], b[1]);
+}
+// words 2 (g / 2), 2 (g / 2) + 1 of lane groups g and g ^ 2 -> all four
+__device__ __forceinline__ uint4 gather2(uint2 v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(v.x, v.x, false, false), b = __builtin_amdgcn_permlane32_swap(v.y, v.y, false, false);
+  return make_uint4(a[0], b[0], a[1], b[1]);
 }
 
 // What dequantisation needs beside the codes: per fragment the codebook's slope and offset or its pair table
@@ -139,8 +158,8 @@ struct Consts {
 // acc[f][mf] += line of fragment f x the line's activations.  f0: fragment 0's index into the constants; sw: this lane's two
 // scales of the line (scale planes); xb: the activations' line in LDS; xa: this lane's operand addresses of four steps
 // (Q8_0: eight)
-template <int FMT, int F, int MF, int XP, int TABC>
-__device__ __forceinline__ void line_mma(const Line<FMT> (&q)[F], const uint32_t (&sw)[F], const Consts& C, int f0,
+template <int FMT, int F, int MF, int XP, int TABC, bool SPLIT>
+__device__ __forceinline__ void line_mma(const Line<FMT, SPLIT> (&q)[F], const uint32_t (&sw)[F], const Consts& C, int f0,
                                          const uint8_t* xb, const uint32_t* xa, bool half, floatx4 (&acc)[F][MF]) {
   auto mma = [&](uint32_t xo, const H8 (&w)[F]) {
 #pragma unroll
@@ -187,6 +206,15 @@ __device__ __forceinline__ void line_mma(const Line<FMT> (&q)[F], const uint32_t
     }
     return;
   } else {
+    uint4 head[F], fifth[F];
+    if constexpr (q4(FMT) || q5(FMT)) {
+#pragma unroll
+      for (int f = 0; f < F; f++) {
+        if constexpr (SPLIT) head[f] = gather4(q[f].hd);
+        else head[f] = q[f].hd;
+        if (q5(FMT)) fifth[f] = gather2(q[f].qh);
+      }
+    }
     auto part = [&](auto ec) {
       constexpr int E_ = decltype(ec)::value;
       half2v as[F][2], bs[F][2];
@@ -196,7 +224,7 @@ __device__ __forceinline__ void line_mma(const Line<FMT> (&q)[F], const uint32_t
       for (int f = 0; f < F; f++) {
         if (q4(FMT) || q5(FMT)) {
           // 6-bit (scale, min) fields of sub-blocks 0-3 (E_ = 0) or 4-7 as bytes, gguf scale_min_k4
-          const uint4 hd = q[f].hd[0];
+          const uint4 hd = head[f];
           const uint32_t sc = E_ ? (hd.w & 0x0f0f0f0fu) | ((hd.y >> 2) & 0x30303030u) : hd.y & 0x3f3f3f3fu;
           const uint32_t mn = E_ ? ((hd.w >> 4) & 0x0f0f0f0fu) | ((hd.z >> 2) & 0x30303030u) : hd.z & 0x3f3f3f3fu;
           const half2v k1024 = both(1024.f);
@@ -253,7 +281,7 @@ __device__ __forceinline__ void line_mma(const Line<FMT> (&q)[F], const uint32_t
             uint32_t t2 = (w8 & 0x000f000fu) | 0x64006400u, t3 = (w8 & 0x00f000f0u) | 0x54005400u;
             if (q5(FMT)) {
               // fifth bits: bit 2 jj (low nibbles) and 2 jj + 1 (high) of the qh byte, jj = g / 2 + 2 E_
-              const uint4 qq = q[f].qh[0];
+              const uint4 qq = fifth[f];
               const uint32_t qw = s == 0 ? qq.x : s == 1 ? qq.y : s == 2 ? qq.z : qq.w;
               const uint32_t r = __builtin_amdgcn_alignbit(qw, qw, (uint32_t)((C.g & 2) + 4 * E_));
               t0 |= (r << 4) & 0x00100010u;
@@ -542,14 +570,15 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
   }
   const uint32_t wo = (uint32_t)r * RB, so = (uint32_t)r * (uint32_t)L.sstride;
   const uint32_t ro = up_rotates(FMT, MFX) && (K & 255) == 0 && ((uintptr_t)wb[0] & 127) == 64 && ((uintptr_t)wb[1] & 127) == 64 ? 64u : 0u;
-  Line<FMT> ln[HALVES ? 1 : DB][2];
+  typedef Line<FMT, split_head(MFX)> Ln;
+  Ln ln[HALVES ? 1 : DB][2];
   uint4 cd[HALVES ? DB : 1][2][2];  // line, half, fragment
   // (past the last line: one address for all lanes instead of a branch around the load)
-  auto load = [&](Line<FMT>(&q)[2], int i) {
+  auto load = [&](Ln(&q)[2], int i) {
 #pragma unroll
     for (int f = 0; f < 2; f++) {
       const bool past = i >= nline;
-      load_line<FMT>(q[f], wb[f] + (past ? (size_t)0 : (size_t)i * LB + ro), past ? 0u : wo, past ? 0 : g, tail && i >= nline - 1,
+      load_line(q[f], wb[f] + (past ? (size_t)0 : (size_t)i * LB + ro), past ? 0u : wo, past ? 0 : g, tail && i >= nline - 1,
                      ro && i == nline - 1 ? (ptrdiff_t)64 - (ptrdiff_t)RB : (ptrdiff_t)64);
     }
   };
@@ -807,7 +836,8 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
   const uint8_t* const wb = L.w + (size_t)e * L.e_rows * RB;
   const uint8_t* const sb = scale_plane(FMT) ? L.sc + (size_t)e * L.e_rows * (size_t)L.sstride : nullptr;
   // fragment f, MFMA row i = weight row 8 (i / 4) + 4 f + i % 4 of the wave's 32: a lane's eight results are neighbours
-  Line<FMT> ln[2][LN];
+  typedef Line<FMT, split_head(MFX)> Ln;
+  Ln ln[2][LN];
   Raw<FMT> raw[2];
   auto first_row = [&](int p) {
     const int r = (nb + p) * DNR + 32 * wv;
@@ -821,7 +851,7 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
 #pragma unroll
     for (int i = 0; i < LN; i++) {
       const int l = ONE || q * LN + i < nline ? q * LN + i : nline - 1;
-      load_line<FMT>(ln[f][i], wb + ((size_t)row0 * RB + l * LB), (uint32_t)r * RB, g, tail && l == nline - 1);
+      load_line(ln[f][i], wb + ((size_t)row0 * RB + l * LB), (uint32_t)r * RB, g, tail && l == nline - 1);
     }
   };
   TabEntry te;
@@ -862,7 +892,7 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
           for (int i = 0; i < LN; i++) {
             const int l = q * LN + i;
             if (!ONE && l >= nline) break;
-            const Line<FMT> q1[1] = {ln[f][i]};
+            const Ln q1[1] = {ln[f][i]};
             const uint32_t sw[1] = {sq[i]};
             line_mma<FMT, 1, MF, XP, tab_copies(false, MFX)>(q1, sw, C, 0, smem + l * XLINE, xa, tail && l == nline - 1, a1);
           }
@@ -881,7 +911,7 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
         for (int i = 0; i < LN; i++) {
           const int l = q * LN + i;
           if (!ONE && l >= nline) break;
-          const Line<FMT> q2[2] = {ln[0][i], ln[1][i]};
+          const Ln q2[2] = {ln[0][i], ln[1][i]};
           const uint32_t sw[2] = {sq[0][i], sq[1][i]};
           line_mma<FMT, 2, MF, XP, tab_copies(false, MFX)>(q2, sw, C, 0, smem + l * XLINE, xa, tail && l == nline - 1, acc);
         }
@@ -914,9 +944,9 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
 constexpr int DN_ONE = 3;  // lines of the rows that a wave takes whole
 constexpr int up_waves(int FMT, int MFX) { return MFX == 4 || i4(FMT) ? 8 : 4; }
 // waves per SIMD asked for: what the registers of the lines in flight leave.  (Gate/up with Q5_K rounded once, 32 pairs: three; with
-// four 21 registers went to scratch inside the loop, 757 us for 702 at 1200 tokens of 2560 x 640.  Two kernels keep 1 .. 4
-// registers of their prologue in scratch until the epilogue: gate/up F_Q5K with 32 pairs, down F_TAB with 64.  F_Q5K with three waves has none and is no
-// faster: 808 us for 799 at 515 tokens, 1159 for 1152 at 1700.)
+// four 21 registers went to scratch inside the loop, 757 us for 702 at 1200 tokens of 2560 x 640.  One kernel keeps four
+// registers of its prologue in scratch until the epilogue: down F_TAB with 64 pairs.  F_Q5K with 32 and three waves is no faster: 808 us
+// for 799 at 515 tokens, 1159 for 1152 at 1700.)
 constexpr int simd_waves(int FMT, bool UP, int MFX, int NW) {
   if (UP) return FMT == F_Q5E && MFX == 2 ? 3 : 4;
   return NW == 16 ? 4 : FMT == F_Q80 || FMT == F_Q4K ? 3 : 4;
