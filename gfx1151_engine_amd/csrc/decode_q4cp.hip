@@ -587,6 +587,165 @@ __global__ void __launch_bounds__(512) k_dec_dn(DnArgs2 A, const uint32_t* __res
   }
 }
 
+// The same for rows of 16, 20 or 24 groups, which leave lanes of a half-wave without one: a wave takes four slots, and its lanes the
+// 4 G (slot, group) units of a row one after the other -- the first 64, then the R = 4 G - 64 that are left, those of 64 / R rows
+// at a time (24 groups: two rows in three passes instead of four, 20: four rows in five instead of eight, 16: a row in one
+// instead of two).  A lane keeps the activations of its two units for all rows.  Units of a slot start at multiples of 8 (20
+// groups: 4) lanes, so a row's sums are taken over as many lanes in registers, the rest from LDS.
+// grid (d / ROWS, P), block 64 ceil(slots / 4).
+// What bounds the launch from a few tokens on is vector instructions: half-waves of 24, 20 or 16 busy lanes of 32 take 31 for a
+// row and slot, 24 groups packed 19.  Layers, us, half-waves and packed (rows of a block that are fastest): 3072 x 768 4 tokens (two
+// layers) 95.2 92.9, 12 102.8 100.9, 20 (local) 146.4 140.4, rotated experts 11 91.8 88.6; 2560 x 640 1 (four layers) 73.9 71.3, 20 124.1 118.7;
+// 3072 x 512 1 69.9 68.1, 20 119.3 106.1; table codebooks 3072 x 768 2 87.0 78.4, 5 78.1 67.8, 2560 x 640 3 96.9 83.8, 3072 x 512 5 68.2 51.7.
+// With 24 groups one token waits for latency, not instructions, and half as many waves are slower: one token 79.8 and 80 .. 82,
+// table 112.5 and 114 .. 119; three tokens 74.5 either way.  Rows: more share a lane's activations, fewer leave more blocks and waves
+// (20 tokens, 4, 8, 12, 16 and 24 rows of 24 groups: 152, 142, 140, 141 and 142; 20 groups 8 and 16: 122 and 119; one token 4 and 8: 71.3, 72.2).
+template <int G, int ROWS, int LUT>
+__global__ void __launch_bounds__(256) k_dec_dn_packed(DnArgs2 A, const uint32_t* __restrict__ hplanes, const float2* __restrict__ hmeta,
+                                                       const int* __restrict__ ids, const float* __restrict__ ws, int id_stride, int kpt,
+                                                       int d, float* __restrict__ out, uint64_t out_stride,
+                                                       const float* __restrict__ hid_f32) {
+  constexpr int R = 4 * G - 64, RS = R ? 64 / R : 1, NB = R ? ROWS / RS : 0;
+  static_assert(R >= 0 && R < 64 && (R == 0 || 64 % R == 0) && ROWS % RS == 0, "");
+  constexpr int PL = G % 8 ? 4 : 8, NPC = G / PL, PCP = NPC > 4 ? 8 : 4;  // lanes of a sum, sums of a row, floats of them in LDS
+  constexpr int SETS = R ? 2 : 1;
+  extern __shared__ float lutmem[];
+  __shared__ __attribute__((aligned(16))) float part[DN2_MAXSLOTS][ROWS][PCP];
+  __shared__ float wsm[DN2_MAXSLOTS];
+  const int tok = blockIdx.y, lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const bool has_shared = A.shd.codes != nullptr;
+  const int nslots = kpt + (has_shared ? 1 : 0), r0 = blockIdx.x * ROWS;
+  constexpr uint32_t rb = 16u * G;
+  const float* const tcb = has_shared ? A.shd.cb : A.dn.cb;
+  float c0 = 0.f, c1 = 0.f, c2 = 0.f, c3 = 0.f;
+  const int t2 = (int)(threadIdx.x + blockDim.x);
+  if (LUT == 1) {  // (a thread's first two pieces of each table)
+    c0 = A.dn.cb[threadIdx.x >> 4 & 15];
+    c1 = tcb[threadIdx.x >> 4 & 15];
+    c2 = A.dn.cb[t2 >> 4 & 15];
+    c3 = tcb[t2 >> 4 & 15];
+  }
+  float wmine = 0.f;
+  if ((int)threadIdx.x < nslots)
+    wmine = (int)threadIdx.x < kpt ? ws[(size_t)tok * id_stride + threadIdx.x] : A.sh_logit[tok];
+  // (branch-free loads, as above: a unit without a slot reads slot 0 and counts nothing)
+  int slot[SETS], grp[SETS];
+  float m[SETS], ca[SETS], cb[SETS], cbk[SETS];
+  const uint8_t *cp[SETS], *sp[SETS];
+  uint64_t wss[SETS];
+  uint32_t lt[SETS];
+  XG x[LUT ? 1 : SETS];
+  XF xh[LUT ? SETS : 1];
+  const uint32_t lut_r = LUT == 1 ? lut_at(lutmem) : 0u, lut_s = lut_r + LUT_BYTES;
+#pragma unroll
+  for (int i = 0; i < SETS; i++) {
+    const int u = i ? 64 + lane % (R ? R : 1) : lane;
+    grp[i] = u % G;
+    slot[i] = 4 * wv + u / G;
+    const bool live = slot[i] < nslots, shared = has_shared && slot[i] == nslots - 1;
+    const int s = live ? slot[i] : 0;
+    m[i] = live ? 1.f : 0.f;
+    const uint8_t* const codes = shared ? A.shd.codes : A.dn.codes;
+    const uint8_t* const scales = shared ? A.shd.scales : A.dn.scales;
+    const float* const wcb = shared ? A.shd.cb : A.dn.cb;
+    wss[i] = shared ? A.shd.ss : A.dn.ss;
+    const int gsh = shared ? A.shd.gsh : A.dn.gsh;
+    const int e_any = ids[tok * id_stride + (shared ? 0 : s)];
+    const uint32_t row0 = (shared ? 0u : (uint32_t)e_any) * (uint32_t)d + (uint32_t)(r0 + (i ? lane / (R ? R : 1) : 0));
+    if (LUT) load_xf(xh[LUT ? i : 0], hid_f32 + ((size_t)(tok * nslots + s) * G + grp[i]) * 32);
+    else load_xg(x[LUT ? 0 : i], hplanes, hmeta, (size_t)((tok * nslots + s) * G + grp[i]));
+    lt[i] = ((shared ? lut_s : lut_r) >> 8) * 0x01010101u;
+    ca[i] = wcb[1] - wcb[0];
+    cbk[i] = wcb[0];
+    cb[i] = fmaf(8.f, ca[i], wcb[0]);
+    cp[i] = codes + (uint64_t)row0 * rb + (uint32_t)grp[i] * 16;
+    sp[i] = scales + (uint64_t)row0 * (uint32_t)wss[i] + (uint32_t)(grp[i] >> gsh) * 2;
+  }
+  uint4 cw[ROWS], cwb[NB ? NB : 1];
+  __half sc[ROWS], scb[NB ? NB : 1];
+  {
+    const uint8_t *c = cp[0], *q = sp[0];
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+      cw[r] = *(const uint4*)c;
+      sc[r] = *(const __half*)q;
+      c += rb;
+      q += wss[0];
+    }
+  }
+  if constexpr (R > 0) {
+    const uint8_t *c = cp[1], *q = sp[1];
+#pragma unroll
+    for (int r = 0; r < NB; r++) {
+      cwb[r] = *(const uint4*)c;
+      scb[r] = *(const __half*)q;
+      c += RS * rb;
+      q += RS * wss[1];
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);  // every load is issued before the first dot product
+  if (LUT == 1) {
+    if (threadIdx.x < 256) {
+      lut_put(lut_r, threadIdx.x, c0);
+      lut_put(lut_s, threadIdx.x, c1);
+    }
+    if (t2 < 256) {
+      lut_put(lut_r, t2, c2);
+      lut_put(lut_s, t2, c3);
+    }
+    for (int i = t2 + (int)blockDim.x; i < 256; i += blockDim.x) {  // (one wave)
+      lut_put(lut_r, i, A.dn.cb[i >> 4]);
+      lut_put(lut_s, i, tcb[i >> 4]);
+    }
+    moe_lds_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  float sx[SETS];
+#pragma unroll
+  for (int i = 0; i < SETS; i++) sx[i] = LUT == 2 ? xf_sum(xh[LUT ? i : 0]) : 0.f;
+  auto dot = [&](int i, const uint4& c, __half s, int row) {
+    float v;
+    if (LUT) v = f32_dot<LUT>(c, xh[LUT ? i : 0], lt[i], ca[i], cbk[i], sx[i]);
+    else v = chunk_dot(c, x[LUT ? 0 : i], ca[i], cb[i]);
+    v *= __half2float(s) * m[i];
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));  // xor 1
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));  // xor 2
+    if (PL == 8) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true));  // mirror in 8
+    if (lane % PL == 0) part[slot[i]][row][grp[i] / PL] = v;
+  };
+#pragma unroll
+  for (int r = 0; r < ROWS; r++) {
+    dot(0, cw[r], sc[r], r);
+    if (r & 1) __builtin_amdgcn_sched_barrier(0);  // rows are consumed in arrival order
+  }
+  if constexpr (R > 0) {
+#pragma unroll
+    for (int r = 0; r < NB; r++) {
+      dot(1, cwb[r], scb[r], RS * r + lane / R);
+      if (r & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if ((int)threadIdx.x < nslots) wsm[threadIdx.x] = (int)threadIdx.x < kpt ? wmine : sigmoid_f(wmine);
+  __syncthreads();
+  if (threadIdx.x < ROWS) {
+    const int r = threadIdx.x;
+    auto total = [&](int s) {
+      float v = part[s][r][0];
+#pragma unroll
+      for (int i = 1; i < NPC; i++) v += part[s][r][i];
+      return v;
+    };
+    float y = 0.f;
+    for (int s = 0; s < kpt; s++) y += wsm[s] * total(s);
+    if (has_shared) {
+      const float shv = wsm[kpt] * total(kpt);
+      if (A.out_sh) A.out_sh[(size_t)tok * out_stride + r0 + r] = shv;
+      else y += shv;
+    }
+    out[(size_t)tok * out_stride + r0 + r] = y;
+  }
+}
+
 // Down projection of the unique-expert path: grid (d/DU_ROWS, tiles), block 256 = 8 half-waves of
 // DU_HW rows.  Lane g of a half-wave holds group g of its weight rows and walks the tile's pairs; the
 // unweighted row results go to pairs[pair][row] (f32) for the weighted combine that follows.
@@ -778,6 +937,23 @@ int moe_launch_dec_dn_lut(const moe_wview* dn, const moe_wview* sh_down, const f
 #define DEC_DN_F32(ROWS, MODE)                                                                                          \
   k_dec_dn<ROWS, MODE><<<dim3(d / ROWS, P), bs, MODE == 1 ? lds : 0, st>>>(A, nullptr, nullptr, ids, ws, id_stride, kpt, d, mid, \
                                                                            out, out_stride, hid_f32)
+  if (!affine) {
+    const int bs4 = 64 * ((nslots + 3) / 4);
+#define DEC_DN_PACKED(G, ROWS)                                                                                                       \
+  k_dec_dn_packed<G, ROWS, 1><<<dim3(d / ROWS, P), bs4, lds, st>>>(A, nullptr, nullptr, ids, ws, id_stride, kpt, d, out, out_stride, hid_f32)
+    bool taken = true;
+    if (mid == 768 && P > 1) DEC_DN_PACKED(24, 8);
+    else if (mid == 640 && P > 1) DEC_DN_PACKED(20, 8);
+    else if (mid == 640) DEC_DN_PACKED(20, 4);
+    else if (mid == 512 && P > 1) DEC_DN_PACKED(16, 8);
+    else if (mid == 512) DEC_DN_PACKED(16, 4);
+    else taken = false;
+#undef DEC_DN_PACKED
+    if (taken) {
+      MOE_LAUNCH_CHECK();
+      return MOE_OK;
+    }
+  }
   if (d % MOE_DN_ROWS == 0) {
     if (affine) DEC_DN_F32(MOE_DN_ROWS, 2);
     else DEC_DN_F32(MOE_DN_ROWS, 1);
@@ -833,6 +1009,23 @@ int moe_launch_dec_dn(const moe_wview* dn, const moe_wview* sh_down, const float
   if (!A.dn.cb) return MOE_E_STATE;
   if (dn->rows > 0xffffffffull) return MOE_E_UNSUPPORTED;  // (row numbers are 32-bit in the kernel)
   const int nslots = kpt + (sh_down ? 1 : 0), bs = 64 * ((nslots + 1) / 2);
+  const int bs4 = 64 * ((nslots + 3) / 4);
+#define DEC_DN_PACKED(G, ROWS)                                                                                                       \
+  k_dec_dn_packed<G, ROWS, 0><<<dim3(d / ROWS, P), bs4, 0, st>>>(A, hplanes, hmeta, ids, ws, id_stride, kpt, d, out, out_stride, nullptr)
+  bool taken = true;
+  if (mid == 768 && P > 3 && d % 12 == 0) DEC_DN_PACKED(24, 12);
+  else if (mid == 768 && P > 3) DEC_DN_PACKED(24, 8);
+  else if (mid == 640 && P == 1) DEC_DN_PACKED(20, 4);
+  else if (mid == 640 && P > 8 && d % 16 == 0) DEC_DN_PACKED(20, 16);
+  else if (mid == 640) DEC_DN_PACKED(20, 8);
+  else if (mid == 512 && P > 8 && d % 16 == 0) DEC_DN_PACKED(16, 16);
+  else if (mid == 512) DEC_DN_PACKED(16, 8);
+  else taken = false;
+#undef DEC_DN_PACKED
+  if (taken) {
+    MOE_LAUNCH_CHECK();
+    return MOE_OK;
+  }
   // MOE_DN_ROWS rows per block where that divides d (d = 3072: 512 blocks, two per CU), else 8
   if (d % MOE_DN_ROWS == 0)
     k_dec_dn<MOE_DN_ROWS, 0><<<dim3(d / MOE_DN_ROWS, P), bs, 0, st>>>(A, hplanes, hmeta, ids, ws, id_stride, kpt, d, mid, out, out_stride, nullptr);

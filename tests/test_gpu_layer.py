@@ -88,6 +88,23 @@ def test_small_batch_table_codebooks(oracle, T, kind):
     m.close()
 
 
+@pytest.mark.parametrize("T", [1, 3, 4, 5, 9])
+@pytest.mark.parametrize("d,mid", [(768, 768), (512, 768), (384, 640), (544, 640), (768, 512), (544, 512)])
+@pytest.mark.parametrize("kind,k,shared", [("q4cp", 1, False), ("q4cp", 10, True), ("q4cp", 15, True), ("table", 3, True), ("table", 10, True), ("table", 12, False)])
+def test_small_batch_rows_of_packed_groups(oracle, kind, k, shared, d, mid, T):
+    """Down rows of 16, 20 and 24 groups, which four slots to a wave share: one slot to sixteen (waves with slots left over), widths
+    that are and are not whole blocks of 12 and 16 rows, the shared expert with codebooks and scale strides of its own."""
+    rng = np.random.default_rng(d + mid + 10 * T + k)
+    cb = np.sort(rng.standard_normal(16)).astype(np.float32) if kind == "table" else None
+    scb = [np.sort(rng.standard_normal(16)).astype(np.float32) for _ in range(3)] if kind == "table" else None
+    hl = HostLayer(rng, d, mid, 20, k, codebook=cb, shared_codebooks=scb, shared=shared, scale_std=0.05)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    yo, io, wo = oracle.moe_layer(hl.oracle_layer(), x)
+    y, ids, ws = run_layer(hl, x)
+    assert (ids[:, :k] == io[:, :k]).all()
+    assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= (TOL_LUT if kind == "table" else TOL_INT_Q4CP)
+
+
 @pytest.mark.parametrize("limit", [0, 3, 32])
 @pytest.mark.parametrize("codebook", ["affine", "universal"])
 def test_f32_decode_token_limit(oracle, limit, codebook):
