@@ -656,51 +656,59 @@ struct DnGgArgs {
   int tdn, tsh;
 };
 
-// D4_ROWS output rows of one wave's slots: a row of 16 lanes = one slot
-template <int T>
-__device__ __forceinline__ void ggu_dn_rows(const uint8_t* base, int mid, int ul, float mlive, const XU& x, bool store,
-                                            float* part_s) {
-  constexpr int RB = ggu_batch<T>();
+// NR output rows of a wave's slots, row j at first + j step of `base`: U lanes of a slot, summed four at a time
+template <int T, int NR, class Store>
+__device__ __forceinline__ void ggu_dn_rows(const uint8_t* base, int mid, int first, int step, int ul, float mlive, const XU& x, Store&& store) {
+  constexpr int RB = NR < ggu_batch<T>() ? NR : ggu_batch<T>();
   const uint64_t rb = ggu_row_bytes(T, (uint64_t)mid);
   const int jj = ul & 3;
   GgU<T> u[RB];
+  auto fetch = [&](int j) {
+    const int r = first + j * step;
+    ggu_fetch<T>(base + (uint64_t)(r < D4_ROWS ? r : D4_ROWS - 1) * rb, ul, u[j % RB]);
+  };
 #pragma unroll
-  for (int r = 0; r < RB; r++) ggu_fetch<T>(base + (uint64_t)r * rb, ul, u[r]);
+  for (int j = 0; j < RB; j++) fetch(j);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int r = 0; r < D4_ROWS; r++) {
-    const float v = dpp_add_row(ggu_dot<T>(u[r % RB], jj, x) * mlive);
-    if (store) part_s[r] = v;
+  for (int j = 0; j < NR; j++) {
+    float v = ggu_dot<T>(u[j % RB], jj, x) * mlive;
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));  // xor 1
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));  // xor 2
+    store(first + j * step, v);
     __builtin_amdgcn_sched_barrier(0);
-    if (r + RB < D4_ROWS) ggu_fetch<T>(base + (uint64_t)(r + RB) * rb, ul, u[r % RB]);
+    if (j + RB < NR) fetch(j + RB);
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-// grid (d/D4_ROWS, P); block = 64 x (ceil(kpt/4) + 1 with a shared expert): waves 0.. hold four routed slots each (a row
-// of 16 lanes per slot), the last wave the shared expert alone, so that a wave's block type is uniform.
+// grid (d/D4_ROWS, P); block = 64 x (ceil(kpt/S) + 1 with a shared expert).  A slot is U = mid / 64 lanes (4, 8, 12 or 16) with a unit
+// each, S = 64 / U slots share a wave: waves 0.. hold the routed slots, the last wave the shared expert alone, whose S groups of
+// lanes take different rows, so that a wave's block type is uniform.  (Sixteen lanes to a slot whatever its units, and eight rows of the
+// shared expert in sixteen lanes of its wave, took four waves for ten slots of twelve units where this takes three, one of them a
+// quarter as long.  Q5_K / Q8_0 layers, 3072 x 768, us: 1 token (four layers) 115.0 -> 110.0, 3 (two) 117.6 116.6, 8 120.0 116.4, 20 252 242,
+// 32 379 363.  Q4_K layers' own kernel below 32 tokens is faster for them: 1 token 90.7 against 93.2, 20 tokens 175.9, 176.4.)
+template <int U>
 __global__ void __launch_bounds__(320) k_decgg_dn(DnGgArgs A, const uint32_t* __restrict__ hplanes,
                                                   const float2* __restrict__ hmeta, const int* __restrict__ ids,
-                                                  const float* __restrict__ ws, int id_stride, int kpt, int d, int mid,
+                                                  const float* __restrict__ ws, int id_stride, int kpt, int d,
                                                   float* __restrict__ out, uint64_t out_stride) {
-  __shared__ float part[D4_MAXSLOTS + 1][D4_ROWS];
+  constexpr int S = 64 / U, mid = 64 * U, NSH = (D4_ROWS + S - 1) / S;
+  __shared__ __attribute__((aligned(16))) float part[D4_MAXSLOTS + 1][D4_ROWS][4];  // a slot's row: the sums of its quads of lanes
   __shared__ float wsm[D4_MAXSLOTS + 1];
   const int tok = blockIdx.y;
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const bool has_shared = A.sh_down != nullptr;
-  const int nslots = kpt + (has_shared ? 1 : 0), rw = (kpt + 3) >> 2;  // rw: waves of routed slots
-  const int U = mid / 64, u_raw = lane & 15;
+  const int nslots = kpt + (has_shared ? 1 : 0), rw = (kpt + S - 1) / S;  // rw: waves of routed slots
   const int r0 = blockIdx.x * D4_ROWS;
   float wmine = 0.f;
   if ((int)threadIdx.x < nslots)
     wmine = (int)threadIdx.x < kpt ? ws[(size_t)tok * id_stride + threadIdx.x] : A.sh_logit[tok];
   {
-    const bool shw = wv >= rw;  // the shared expert's wave (its slot in lanes 0..15)
-    const int s_raw = shw ? kpt + (lane >> 4) * D4_MAXSLOTS : 4 * wv + (lane >> 4);  // lanes 16.. of that wave: no slot
-    const bool okslot = shw ? (lane >> 4) == 0 : s_raw < kpt;
-    const bool live = okslot && u_raw < U;
-    const int s = okslot ? s_raw : (shw ? kpt : 0);
-    const int ul = u_raw < U ? u_raw : (u_raw & 3);
+    const bool shw = wv >= rw;  // the shared expert's wave
+    const int group = lane / U, ul = lane % U, s_raw = shw ? kpt : S * wv + group;
+    const bool live = group < S && (shw || s_raw < kpt);
+    const int s = live ? s_raw : shw ? kpt : 0;
     const float mlive = live ? 1.f : 0.f;
     const int t = shw ? A.tsh : A.tdn;
     const uint64_t rb = ggu_row_bytes(t, (uint64_t)mid);
@@ -710,15 +718,25 @@ __global__ void __launch_bounds__(320) k_decgg_dn(DnGgArgs A, const uint32_t* __
     const uint8_t* base = (shw ? A.sh_down : A.down + (uint64_t)(e * (uint32_t)d) * rb) + (uint64_t)r0 * rb;
     XU x;
     load_xu(x, hplanes, hmeta, (((size_t)tok * nslots + s) * U + ul) * 2);
-    GGU_SWITCH(t, ggu_dn_rows<T>(base, mid, ul, mlive, x, u_raw == 0 && okslot, part[s]));
+    auto store = [&](int r, float v) {
+      if (live && r < D4_ROWS && (lane & 3) == 0) part[s][r][ul >> 2] = v;
+    };
+    if (shw) GGU_SWITCH(t, (ggu_dn_rows<T, NSH>(base, mid, group < S ? group : 0, S, ul, mlive, x, store)))
+    else GGU_SWITCH(t, (ggu_dn_rows<T, D4_ROWS>(base, mid, 0, 1, ul, mlive, x, store)))
   }
   if ((int)threadIdx.x < nslots) wsm[threadIdx.x] = (int)threadIdx.x < kpt ? wmine : sigmoid_f(wmine);
   __syncthreads();
   if (threadIdx.x < D4_ROWS) {
     const int r = threadIdx.x;
+    auto total = [&](int s) {
+      float v = part[s][r][0];
+#pragma unroll
+      for (int i = 1; i < U / 4; i++) v += part[s][r][i];
+      return v;
+    };
     float y = 0.f;
-    for (int i = 0; i < kpt; i++) y += wsm[i] * part[i][r];
-    if (has_shared) y += wsm[kpt] * part[kpt][r];
+    for (int i = 0; i < kpt; i++) y += wsm[i] * total(i);
+    if (has_shared) y += wsm[kpt] * total(kpt);
     out[(size_t)tok * out_stride + r0 + r] = y;
   }
 }
@@ -999,8 +1017,16 @@ int moe_launch_decgg_dn(int tdn, int tsh, const uint8_t* down, const uint8_t* sh
   if (!moe_aligned(down, ggu_align(tdn)) || (sh_down && !moe_aligned(sh_down, ggu_align(tsh)))) return MOE_E_INVALID;
   DnGgArgs A{down, sh_down, sh_logit, tdn, tsh};
   dim3 grid(d / D4_ROWS, P);
-  k_decgg_dn<<<grid, 64 * ((kpt + 3) / 4 + (sh_down ? 1 : 0)), 0, st>>>(A, hplanes, hmeta, ids, ws, id_stride, kpt, d, mid,
-                                                                        out, out_stride);
+#define DECGG_DN(U) \
+  k_decgg_dn<U><<<grid, 64 * ((kpt + 64 / U - 1) / (64 / U) + (sh_down ? 1 : 0)), 0, st>>>(A, hplanes, hmeta, ids, ws, id_stride, kpt, d, out, out_stride)
+  switch (mid / 64) {  // (moe_decgg_supported)
+    case 4: DECGG_DN(4); break;
+    case 8: DECGG_DN(8); break;
+    case 12: DECGG_DN(12); break;
+    case 16: DECGG_DN(16); break;
+    default: return MOE_E_UNSUPPORTED;
+  }
+#undef DECGG_DN
   MOE_LAUNCH_CHECK();
   return MOE_OK;
 }

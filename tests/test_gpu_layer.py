@@ -88,6 +88,22 @@ def test_small_batch_table_codebooks(oracle, T, kind):
     m.close()
 
 
+@pytest.mark.parametrize("T", [1, 3, 6])
+@pytest.mark.parametrize("mid", [256, 512, 768, 1024])
+@pytest.mark.parametrize("types,k,shared", [((13, 8, 8), 1, True), ((13, 8, 8), 10, True), ((12, 8, 12), 5, True), ((13, 13, 8), 15, True),
+                                            ((13, 8, 8), 6, False), ((8, 7, 12), 13, True)])
+def test_small_batch_gguf_rows_of_packed_units(oracle, types, k, shared, mid, T):
+    """Down rows of 4 to 16 units of 64 columns: one slot to fifteen, the last wave full and not, the shared expert's rows in its groups of
+    lanes, its type the routed experts' and another."""
+    rng = np.random.default_rng(mid + 10 * T + k)
+    hl = HostLayer(rng, 256, mid, 20, k, fmt="q4k", gg_types=types, shared=shared)
+    x = rng.standard_normal((T, 256), dtype=np.float32)
+    yo, io, wo = oracle.moe_layer(hl.oracle_layer(), x)
+    y, ids, ws = run_layer(hl, x)
+    assert (ids[:, :k] == io[:, :k]).all()
+    assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= TOL_INT_Q4K
+
+
 @pytest.mark.parametrize("T", [1, 3, 4, 5, 9])
 @pytest.mark.parametrize("d,mid", [(768, 768), (512, 768), (384, 640), (544, 640), (768, 512), (544, 512)])
 @pytest.mark.parametrize("kind,k,shared", [("q4cp", 1, False), ("q4cp", 10, True), ("q4cp", 15, True), ("table", 3, True), ("table", 10, True), ("table", 12, False)])
