@@ -219,12 +219,29 @@ __global__ void __launch_bounds__(256, 2) k_router_f16(const __half* __restrict_
 // past n repeat the last), columns c0 .. c1 - 1 of rows of ld (multiples of 64).  The wave keeps a panel of x in registers, four
 // columns of every 256 to a lane, widened once, and lets the rows go past it two at a time, the next two requested before
 // these are summed: a load covers 1 KB (bf16 512 bytes) of one row, no activation passes through LDS, and no more rows are
-// multiplied than there are candidates (one more where their number is odd).  A lane's sums wait in LDS between panels.
+// multiplied than there are candidates (one more where their number is odd).  A lane's sums wait in LDS between panels,
+// four rows' in a double of each lane: the launch runs beside the shared expert's GEMMs, which want the CUs' LDS (with a double of every
+// lane and row, 38 KB a block, it was as fast alone and the layer no faster for it at 4096 tokens).
 // What bounds it is widening the weights -- v_cvt_f64_f32 takes four times as long as an FMA -- next to the L2s' rate.  A float's
 // exponent and mantissa shifted into a double's places are the value times 2^-896, zeros and subnormals included, so the
 // weights are widened with shifts and x carries the 2^896 (|x| < 2^128: no overflow; infinities and NaNs never get here).
 // The order of the sums is fixed.
-constexpr int DR_ROWS = 16, DR_PITCH = 65;  // rows of a pass; doubles of a row's sums in LDS
+constexpr int DR_ROWS = 16;              // rows of a pass
+constexpr int DR_SUMS = DR_ROWS * 16;  // doubles of a wave's sums in LDS
+// lanes' a and b -> half as many lanes' sums of each (lanes 0 .. 31 a's, the others b's; by 16: in rows of 16 lanes a, b, a, b)
+template <bool BY32>
+__device__ __forceinline__ double swap_add(double a, double b) {
+  union U { double d; uint32_t i[2]; } x, y, p, q;
+  x.d = a;
+  y.d = b;
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const auto s = BY32 ? __builtin_amdgcn_permlane32_swap(x.i[i], y.i[i], false, false) : __builtin_amdgcn_permlane16_swap(x.i[i], y.i[i], false, false);
+    p.i[i] = s[0];
+    q.i[i] = s[1];
+  }
+  return p.d + q.d;
+}
 __device__ __forceinline__ double widen_m896(uint32_t u) {
   union { double d; uint32_t i[2]; } r;
   r.i[0] = u << 29;
@@ -237,7 +254,7 @@ __device__ __forceinline__ double widen_m896_hi(uint32_t u) {  // (a bf16 in the
   r.i[1] = (u & 0x80000000u) | ((u >> 3) & 0x0fffffffu);
   return r.d;
 }
-// sums: DR_ROWS x DR_PITCH doubles of LDS owned by the wave.  Returns row lane % 16's sum.  PP: pieces of 256 columns in a panel.
+// sums: DR_SUMS doubles of LDS owned by the wave.  Returns row lane % 16's sum.  PP: pieces of 256 columns in a panel.
 template <bool BF16, int PP>
 __device__ __forceinline__ double dot_rows(__amdgpu_buffer_rsrc_t W, const float* __restrict__ xrow, int ld, int c0, int c1, int ids, int n,
                                            int lane, double* sums) {
@@ -279,10 +296,8 @@ __device__ __forceinline__ double dot_rows(__amdgpu_buffer_rsrc_t W, const float
       for (int k = 0; k < 4; k++) x[i][k] = (double)f[k] * s;
     }
     const bool first = p0 == c0;
-    auto sum = [&](int r, const uint32_t(&q)[2][PP][WPL]) {
-      double a[2];
-#pragma unroll
-      for (int h = 0; h < 2; h++) a[h] = first ? 0.0 : mine[(r + h) * DR_PITCH];
+    auto sum = [&](const uint32_t(&q)[2][PP][WPL]) {
+      double a[2] = {0.0, 0.0};
 #pragma unroll
       for (int i = 0; i < PP; i++)
 #pragma unroll
@@ -294,29 +309,33 @@ __device__ __forceinline__ double dot_rows(__amdgpu_buffer_rsrc_t W, const float
             else wd = widen_m896(q[h][i][k]);
             a[h] = fma(wd, x[i][k], a[h]);
           }
-#pragma unroll
-      for (int h = 0; h < 2; h++) mine[(r + h) * DR_PITCH] = a[h];
+      return swap_add<true>(a[0], a[1]);
     };
+    // four rows' sums in the four rows of sixteen lanes: r, r + 2, r + 1, r + 3
 #pragma unroll 1
     for (int r = 0; r < n; r += 4) {
       load(r + 2, w[1]);
       __builtin_amdgcn_sched_barrier(0);
-      sum(r, w[0]);
+      const double lo = sum(w[0]);
       __builtin_amdgcn_sched_barrier(0);
       load(r + 4, w[0]);
       __builtin_amdgcn_sched_barrier(0);
-      if (r + 2 < n) sum(r + 2, w[1]);
+      double hi = 0.0;
+      if (r + 2 < n) hi = sum(w[1]);
       __builtin_amdgcn_sched_barrier(0);
+      const double v = swap_add<false>(lo, hi);
+      mine[16 * r] = first ? v : mine[16 * r] + v;
     }
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wave's own LDS writes
   __builtin_amdgcn_wave_barrier();
-  // lane group g adds sixteen lanes' sums of row lane % 16, two more steps add the groups'
-  const double* const q = sums + (lane & 15) * DR_PITCH + (lane >> 4) * 16;
+  // lane group g adds four of the sixteen lanes' sums of row lane % 16, two more steps add the groups'
+  const int row = lane & 15;
+  const double* const q = sums + 64 * (row >> 2) + 16 * (((row & 1) << 1) | (row >> 1 & 1)) + 4 * (lane >> 4);
   double v = 0.0;
   if (c1 > c0) {
 #pragma unroll
-    for (int i = 0; i < 16; i++) v += q[i];
+    for (int i = 0; i < 4; i++) v += q[i];
   }
   v += __shfl_xor(v, 16, 64);
   v += __shfl_xor(v, 32, 64);
@@ -328,7 +347,7 @@ __device__ __forceinline__ double dot_rows(__amdgpu_buffer_rsrc_t W, const float
 struct PickLds {
   __attribute__((aligned(16))) float lg[512];
   int cid[4][RC_SLOTS], sid[4][RC_SLOTS];
-  double sums[4][DR_ROWS * DR_PITCH], part[4][DR_ROWS];  // [wave]
+  double sums[4][DR_SUMS], part[4][DR_ROWS];  // [wave]
   float sval[4][RC_SLOTS], sel_ws[64];
   int sel_ids[64], zero[4], nzero;
 };
