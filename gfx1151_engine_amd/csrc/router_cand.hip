@@ -732,6 +732,7 @@ F16Shape f16_shape(int P, int E, int d) {
 bool moe_router_cand_supported(const moe_wview* W, int P, int k) {
   const int E = (int)W->rows, d = (int)W->cols;
   if (P < 1 || d % 64 || d < 64 || E > 512 || k + 1 > RC_SLOTS - 1 || k >= E) return false;
+  if ((uint64_t)E * (uint64_t)d * 4 >= 1ull << 31) return false;  // (32-bit byte offsets of the candidates' rows)
   return moe_aligned(W->data, 16);
 }
 
