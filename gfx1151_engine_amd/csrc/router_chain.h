@@ -4,9 +4,11 @@
 #include "internal.h"
 #include "topk.h"
 
-// One logit's fp64 sum as the reference's sequential chain (src/ref.cpp:70-77), by one wave: the lanes widen 256 columns
-// at a time into LDS (a single thread's 2 d quarter-rate conversions and its dependent loads took 110 us), then every lane
-// runs the same chain over them.  buf: 512 doubles of LDS owned by the wave.
+// One logit's fp64 sum as the reference's sequential chain (src/ref.cpp:70-77), by one wave: the lanes multiply 256 columns
+// at a time into LDS (a single thread's 2 d quarter-rate conversions and its dependent loads took 110 us) -- a product of two
+// floats is exact in fp64, so adding products is the chain of FMAs bit for bit --, then every lane adds them up in order.
+// buf: 512 doubles of LDS owned by the wave, two halves by turns.  (With both factors in LDS and an FMA each, a read of 16 bytes per column,
+// a batch that had such a token spent 34 us in its selecting launch at 48 tokens, 30 at 130; now 26 and 23.)
 __device__ __forceinline__ double exact_chain_wave(const moe_rfix& R, int t, int e, double* buf) {
   const int lane = threadIdx.x & 63;
   const float* xr = R.x + (size_t)t * R.d;
@@ -25,19 +27,22 @@ __device__ __forceinline__ double exact_chain_wave(const moe_rfix& R, int t, int
     }
   };
   load(4 * lane);
-  for (int c = 0; c < R.d; c += 256) {
-    double* const q = buf + 8 * lane;  // (w, x) pairs of this lane's four columns
-    q[0] = (double)w.x; q[1] = (double)xv.x; q[2] = (double)w.y; q[3] = (double)xv.y;
-    q[4] = (double)w.z; q[5] = (double)xv.z; q[6] = (double)w.w; q[7] = (double)xv.w;
+  for (int c = 0, half = 0; c < R.d; c += 256, half ^= 256) {
+    double2* const q = (double2*)(buf + half + 4 * lane);  // this lane's four columns
+    q[0] = double2{(double)w.x * (double)xv.x, (double)w.y * (double)xv.y};
+    q[1] = double2{(double)w.z * (double)xv.z, (double)w.w * (double)xv.w};
     load(c + 256 + 4 * lane);
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wave's own LDS writes
     __builtin_amdgcn_wave_barrier();
     const int n = R.d - c < 256 ? R.d - c : 256;  // (a multiple of 32)
-    for (int i = 0; i < n; i += 16) {
+    for (int i = 0; i < n; i += 32) {
+      double2 p[16];
+#pragma unroll
+      for (int j = 0; j < 16; j++) p[j] = *(const double2*)(buf + half + i + 2 * j);
 #pragma unroll
       for (int j = 0; j < 16; j++) {
-        const double2 p = *(const double2*)(buf + 2 * (i + j));
-        acc = fma(p.x, p.y, acc);
+        acc += p[j].x;
+        acc += p[j].y;
       }
     }
     __builtin_amdgcn_wave_barrier();
