@@ -31,9 +31,10 @@
 // Pairs per tile: 16, 32 or 64 by the batch's average (moe_stream_tile_cap): a block's work is the weights whatever the
 // tile holds, so tiles should hold an expert's pairs as a rule, and larger ones cost LDS and registers.
 // Measured (512 experts, top-10, 3072 x 768, gate/up + down, us; in brackets the 128-pair kernels):
-//   130 tokens q4cp 264 + 134 (354 + 178)      48 table 205 + 106 (298 + 170)    515 Q4_K 341 + 163 (431 + 234)
+//   130 tokens q4cp 240 + 135 (354 + 178)      48 table 175 + 102 (298 + 170)    515 Q4_K 337 + 167 (431 + 234)
 //   200 Q5_K / Q8_0 396 + 282 (487 + 357)     200 i4r 266 + 135 (369 + 191)      2048 q4cp 357 + 206 (444 + 239)
-// The layer at other widths, us (128-pair kernels in brackets), 48 / 515 / 1200 tokens, d = 3072: mid 256 q4cp 162 / 258 / 331 (207 / 307 /
+// The layer at other widths (with q4cp and table rows as they lie, see up_rotates: up to 515 tokens 4 .. 10 % more than now), us (128-pair
+// kernels in brackets), 48 / 515 / 1200 tokens, d = 3072: mid 256 q4cp 162 / 258 / 331 (207 / 307 /
 // 361), Q5_K / Q8_0 214 / 343 / 437 (261 / 409 / 461); 512 q4cp 245 / 401 / 474 (312 / 491 / 549), table 272 / 434 / 535 (392 / 610 / 639),
 // Q4_K 257 / 428 / 513 (339 / 544 / 602), i4r 245 / 378 / 467 (318 / 478 / 542); 1024 q4cp 429 / 719 / 827 (520 / 851 / 942), table 471 /
 // 781 / 930 (645 / 1074 / 1143); d = 2048: 1536 q4cp 419 / 759 / 891 (518 / 833 / 896), 2048 545 / 969 / 1083 (669 / 1083 / 1148).
