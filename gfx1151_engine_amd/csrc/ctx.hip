@@ -24,7 +24,7 @@ struct MoeLayer {
   int sh_dense = 0;  // != 0: gate/up/down of the shared expert are dense rows of this kind (dense.h), in launches of their own
   // every q4cp codebook of the layer is affine (cb[n] = a*n + b): the integer-dot decode kernels apply
   bool experts_affine = false, shared_affine = false;
-  // every expert of the tensor has a power of two for the scaled dequantisation (pexp below)
+  // every expert of the tensor has the scaled dequantisation (pexp below)
   bool scaled_gu = false, scaled_dn = false, scaled_sgu = false, scaled_sdn = false;
   // f16 range guard of the batch path: typical |hid| (and |pair|) per unit mean-square activation,
   // estimated from sampled weight rows when the weights are registered
@@ -140,7 +140,7 @@ struct moe_ctx {
 static int8_t* pexp_slot(moe_ctx* c, int layer, int slot0) {
   return c->pexp ? c->pexp + (size_t)layer * (2 * (size_t)c->cfg.experts + 2) + slot0 : nullptr;
 }
-// rows, cols: of one expert; group: columns of a scale.  *all: every expert has one.
+// rows, cols: of one expert; group: columns of a scale, 128 is i4r.  *all: every expert has one.
 static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_lutw* a, const moe_lutw* b, int group, int rows, int cols,
                          int n_experts, bool* all) {
   *all = false;
@@ -159,7 +159,7 @@ static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_lutw* a, co
     }
     *all = true;
     for (int e = 0; e < n_experts; e++) {
-      out[e] = (int8_t)moe_pexp_from_span(&sa[2 * e], b ? &sb[2 * e] : nullptr);
+      out[e] = (int8_t)(group == 128 ? moe_pexp_i4r(&sa[2 * e]) : moe_pexp_from_span(&sa[2 * e], b ? &sb[2 * e] : nullptr));
       *all = *all && out[e] != (int8_t)MOE_PEXP_NONE;
     }
   }

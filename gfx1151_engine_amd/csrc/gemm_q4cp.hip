@@ -141,14 +141,20 @@ __device__ __forceinline__ void g2l4(const void* g, uint8_t* lds_base) {
 // MF = live 32-row fragments of the tile (1 .. 4); AFFINE = codebook a*n+b.
 // NF = weight fragments (32 rows) per wave: the block's 16 fragments are split over NW = 16/NF
 // waves, each wave multiplying all MF pair fragments with its own NF weight fragments.
-// DN (affine q4cp codebooks and i4r, a power of two P known for the expert): two instructions per weight pair instead of three.
+// DN (affine q4cp codebooks, a power of two P known for the expert; i4r as below): two instructions per weight pair instead of three.
 // A masked code pair IS a pair of f16 denormals, n * 2^-24 (nibbles at bits 0-3) or n * 2^-20 (bits 4-7), so one packed
 // FMA with a = f16(cb_a * scale) * 2^(24+P) (or 2^(20+P)) and b = f16(cb_b * scale) * 2^P gives 2^P * f16(n*a' + b'):
 // the weights of the three-instruction form times 2^P, bit for bit wherever the scaled weight is a normal f16 (the
 // product is exact inside the FMA, one rounding).  P is chosen when the weights are registered, from the expert's
 // largest scale, so that the scaled slope stays below 2^15 (an f16 can hold it); the accumulators carry the factor
-// 2^P and the epilogue takes it out (exact).  v_pk_fma_f16 takes denormal operands at full rate on gfx950.  us, with three instructions
-// and two: i4r 8192 tokens (skewed) gate/up 1141 1098, down 558 531.  (Q4_K gained two per cent of a layer of 4096 tokens and more with it,
+// 2^P and the epilogue takes it out (exact).  v_pk_fma_f16 takes denormal operands at full rate on gfx950.
+// i4r (GS == 2), whose scales may lie far apart inside a row, takes the form without a power of two: all four nibbles of a half at
+// bits 4-7 (two more shifts for eight weights), a = scale * 2^20, b = -8 * scale, both exact while the expert's scales are below
+// 2^-4: the three-instruction form's weights bit for bit, subnormal ones included.  us, with three instructions and so: 8192 tokens
+// (skewed) gate/up 1016 975, down 493 482.  (With a power of two as q4cp's it was no faster, 3001
+// tokens 864 and 867 a layer, and weights below 2^-14 of the scaled units -- 1.5 % of them where a row's scales are normally distributed -- lost
+// bits that the plain units keep.)
+// (Q4_K gained two per cent of a layer of 4096 tokens and more with it,
 // d and dmin brought into the scaled units, but products of theirs that are subnormal as f16 were then rounded otherwise than
 // in the streaming GEMM; Q5_K's fifth bits leave no registers for it: 739 us without and 750 with it.)
 constexpr bool NH_OK = NF == 2;
@@ -167,13 +173,16 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
   constexpr bool WALK = !UP && F16OUT && !Q5 && AHEAD == 2;
   if (!WALK) npass = 1;
   static_assert(!DN || (AFFINE && !NAT && !Q4K), "scaled dequantisation: codes of four bits that stand for a * n + b");
-  if (DN) {  // the codebook in the scaled units
+  constexpr bool DN4 = DN && GS == 2;  // i4r: codes at bits 4-7, plain units
+  if (DN4) {
+    cb_a = cb_a_up = 0x1p20f;
+  } else if (DN) {  // the codebook in the scaled units
     const float s24 = __builtin_ldexpf(1.f, 24 + pexp);
     const float sp = __builtin_ldexpf(1.f, pexp);
     cb_a *= s24; cb_a_up *= s24;
     cb_b *= sp; cb_b_up *= sp;
   }
-  const float oscale = DN ? __builtin_ldexpf(1.f, -pexp) : 1.f;  // takes 2^P out of the accumulators
+  const float oscale = DN && !DN4 ? __builtin_ldexpf(1.f, -pexp) : 1.f;  // takes 2^P out of the accumulators
   constexpr int NH = NF / 2;  // gate/up: fragments per half
   static_assert(GS == 0 || (GS == 2 && !Q4K && NSB == 1), "one scale per 128 columns: q4cp-style planes, single scale buffer");
   static_assert(!Q5 || (Q4K && NSB == 1), "Q5_K: the Q4_K stages plus a fifth bit");
@@ -383,7 +392,7 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
   uint4 cw[NF], cw8[NF];  // code words of the stage and the same shifted right by 8 (parts 2, 3)
   constexpr int NS = Q4K ? 2 : 1;  // scale sets per stage (Q4_K: the two sub-blocks of the stage)
   half2v as2[NF][NS], bs2[NF][NS];
-  half2v as20[DN ? NF : 1];  // DN: the slope for code pairs at bits 4-7 (n * 2^-20): as2 / 16
+  half2v as20[DN && !DN4 ? NF : 1];  // DN: the slope for code pairs at bits 4-7 (n * 2^-20): as2 / 16
   float scf[NF];
   uint4 hdr[NF];
   uint4 qh4[Q5 ? NF : 1];  // Q5_K: this lane's 16 qh bytes of the current super-block (code bytes 16 h .. 16 h + 15)
@@ -501,7 +510,7 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
         const _Float16 as = (_Float16)((upf ? cb_a_up : cb_a) * scf[nf]), bs = (_Float16)((upf ? cb_b_up : cb_b) * scf[nf]);
         as2[nf][0] = half2v{as, as};
         bs2[nf][0] = half2v{bs, bs};
-        if (DN) as20[nf] = as2[nf][0] * half2v{(_Float16)0.0625f, (_Float16)0.0625f};  // (exact: a power of two, far from underflow)
+        if (DN && !DN4) as20[nf] = as2[nf][0] * half2v{(_Float16)0.0625f, (_Float16)0.0625f};  // (exact: a power of two, far from underflow)
       }
     }
   };
@@ -510,11 +519,15 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
   auto deq_unit = [&](int q, int u, H8* dst) {
     const int nf = u >> 2, part = u & 3;
     const uint32_t w = q == 0 ? cw[nf].x : q == 1 ? cw[nf].y : q == 2 ? cw[nf].z : cw[nf].w;
-    if (DN) {
+    if (DN4) {
+      const uint32_t w8 = q == 0 ? cw8[nf].x : q == 1 ? cw8[nf].y : q == 2 ? cw8[nf].z : cw8[nf].w;
+      const uint32_t ws = part == 0 ? w << 4 : part == 1 ? w : part == 2 ? w >> 4 : w8;
+      dst[nf].h[part] = h2(ws & 0x00f000f0u) * as2[nf][0] + bs2[nf][0];
+    } else if (DN) {
       const uint32_t w8 = q == 0 ? cw8[nf].x : q == 1 ? cw8[nf].y : q == 2 ? cw8[nf].z : cw8[nf].w;
       const uint32_t ws = part >= 2 ? w8 : w;
       if ((part & 1) == 0) dst[nf].h[part] = h2(ws & 0x000f000fu) * as2[nf][0] + bs2[nf][0];
-      else dst[nf].h[part] = h2(ws & 0x00f000f0u) * as20[DN ? nf : 0] + bs2[nf][0];
+      else dst[nf].h[part] = h2(ws & 0x00f000f0u) * as20[DN && !DN4 ? nf : 0] + bs2[nf][0];
     } else if (Q5) {
       // five-bit codes as bytes, the low nibbles' (parts 0, 2) and the high nibbles' (1, 3): parts 0 and 1 make them.  Bit
       // 2 jj / 2 jj + 1 of each byte of the qh word goes to bit 4
@@ -710,8 +723,8 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const LutDev& L, int e,
       for (int r = 0; r < 16; r++) {
         const int ml = 8 * (r >> 2) + 4 * h + (r & 3);
         uint8_t* prow = patch + (32 * mf + ml) * BP + (NC * wv + n) * 2;
-        *(__half*)prow = __float2half(DN ? acc[mf][0][r] * oscale : acc[mf][0][r]);
-        *(__half*)(prow + HALF * 2) = __float2half(DN ? acc[mf][1][r] * oscale : acc[mf][1][r]);
+        *(__half*)prow = __float2half(acc[mf][0][r]);
+        *(__half*)(prow + HALF * 2) = __float2half(acc[mf][1][r]);
       }
     }
     __syncthreads();
@@ -1118,6 +1131,8 @@ int moe_pexp_from_span(const int8_t* a, const int8_t* b) {
   const int P = -8 - hi;             // |slope| * scale * 2^(24+P) < 2^16, rounded to f16 already (k_scale_span)
   return P < -100 || P > 100 ? MOE_PEXP_NONE : P;
 }
+
+int moe_pexp_i4r(const int8_t* hi_lo) { return hi_lo[0] <= -4 ? 0 : MOE_PEXP_NONE; }
 
 bool moe_gemm_q5k_fits(uint64_t rows, uint64_t x_rows, int k) {
   const uint64_t lim = (1ull << 32) - (1ull << 16);

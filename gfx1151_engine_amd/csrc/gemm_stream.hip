@@ -51,13 +51,13 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // F_DN: affine q4cp codebooks whose experts all have a power of two for the scaled dequantisation (gemm_q4cp.hip, DN)
 // F_Q4E, F_Q5E: Q4_K and Q5_K weights rounded to f16 once, from their exact values
-// F_I4D: i4r with the scaled dequantisation (3001 skewed tokens, gate/up 509 -> 459 us, down 284 -> 266; 130: 239 -> 227, 134 -> 129.
+// F_I4D: i4r with codes read as denormals and no power of two (gemm_q4cp.hip, DN), layers whose experts all have scales below 2^-4
+// (3001 skewed tokens, gate/up 495 -> 474 us, down 271 -> 261; 130: 248 -> 236, 128 -> 124; the weights are F_I4R's bit for bit).
 // Q4_K gained half a per cent of a layer with it and Q5_K lost 15 at 1200 tokens, both short of registers.)
 enum { F_DN, F_AFF, F_TAB, F_I4R, F_Q4K, F_Q5K, F_Q80, F_Q4E, F_Q5E, F_I4D };
 constexpr bool q4(int FMT) { return FMT == F_Q4K || FMT == F_Q4E; }
 constexpr bool q5(int FMT) { return FMT == F_Q5K || FMT == F_Q5E; }
 constexpr bool i4(int FMT) { return FMT == F_I4D || FMT == F_I4R; }
-constexpr bool scaled(int FMT) { return FMT == F_DN || FMT == F_I4D; }
 constexpr bool once_rounded(int FMT) { return FMT == F_Q4E || FMT == F_Q5E; }
 constexpr bool scale_plane(int FMT) { return FMT <= F_I4R || FMT == F_I4D; }
 // order of activations and hid (moe_f32_to_f16's layouts)
@@ -252,8 +252,8 @@ __device__ __forceinline__ void line_mma(const Line<FMT, SPLIT> (&q)[F], const u
           } else {
             const float s = (float)s2.x;
             as[f][0] = both(C.cb_a[f0 + f] * s);
-            bs[f][0] = bs[f][1] = FMT == F_I4D ? as[f][0] * both(-0x1p-21f) : both(C.cb_b[f0 + f] * s);  // (i4r: -8; exact)
-            as[f][1] = scaled(FMT) ? as[f][0] * both(0.0625f) : as[f][0];
+            bs[f][0] = bs[f][1] = FMT == F_I4D ? as[f][0] * both(-0x1p-17f) : both(C.cb_b[f0 + f] * s);  // (i4r: -8 * s, exact)
+            as[f][1] = FMT == F_DN ? as[f][0] * both(0.0625f) : as[f][0];
           }
         }
       }
@@ -272,7 +272,12 @@ __device__ __forceinline__ void line_mma(const Line<FMT, SPLIT> (&q)[F], const u
             continue;
           }
           const uint32_t w8 = w >> 8;
-          if (scaled(FMT)) {  // codes read as f16 denormals
+          if (FMT == F_I4D) {  // codes read as f16 denormals, n * 2^-20
+            a[f].h[0] = h2((w << 4) & 0x00f000f0u) * as[f][0] + bs[f][0];
+            a[f].h[1] = h2(w & 0x00f000f0u) * as[f][0] + bs[f][0];
+            a[f].h[2] = h2((w >> 4) & 0x00f000f0u) * as[f][0] + bs[f][0];
+            a[f].h[3] = h2(w8 & 0x00f000f0u) * as[f][0] + bs[f][0];
+          } else if (FMT == F_DN) {  // n * 2^-24, n * 2^-20
             a[f].h[0] = h2(w & 0x000f000fu) * as[f][0] + bs[f][0];
             a[f].h[1] = h2(w & 0x00f000f0u) * as[f][1] + bs[f][0];
             a[f].h[2] = h2(w8 & 0x000f000fu) * as[f][0] + bs[f][0];
@@ -466,12 +471,12 @@ __device__ __forceinline__ Consts make_consts(const SW& L, int pexp, const TabEn
   C.tabs = tabs;
   C.tabo[0] = C.tabo[1] = 0u;
   oscale = 1.f;
-  if (FMT == F_AFF || scaled(FMT)) {
-    if (FMT != F_I4D) {
-      C.cb_a[0] = L.cb[1] - L.cb[0]; C.cb_b[0] = L.cb[0];
-      C.cb_a[1] = UP ? L.cb_up[1] - L.cb_up[0] : C.cb_a[0]; C.cb_b[1] = UP ? L.cb_up[0] : C.cb_b[0];
-    }
-    if (scaled(FMT)) {  // in units of 2^pexp; slopes for codes read as f16 denormals
+  if (FMT == F_I4D) {
+    C.cb_a[0] = C.cb_a[1] = 0x1p20f;
+  } else if (FMT == F_AFF || FMT == F_DN) {
+    C.cb_a[0] = L.cb[1] - L.cb[0]; C.cb_b[0] = L.cb[0];
+    C.cb_a[1] = UP ? L.cb_up[1] - L.cb_up[0] : C.cb_a[0]; C.cb_b[1] = UP ? L.cb_up[0] : C.cb_b[0];
+    if (FMT == F_DN) {  // in units of 2^pexp; slopes for codes read as f16 denormals
       const float s24 = __builtin_ldexpf(1.f, 24 + pexp), sp = __builtin_ldexpf(1.f, pexp);
       C.cb_a[0] *= s24; C.cb_a[1] *= s24; C.cb_b[0] *= sp; C.cb_b[1] *= sp;
       oscale = __builtin_ldexpf(1.f, -pexp);
@@ -755,7 +760,7 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
 #pragma unroll
         for (int r4 = 0; r4 < 4; r4++) {
           const int c = pos_elem<LAYOUT>(wv, 4 * g + r4);
-          *(__half*)(patch + (16 * mf + n) * BP + f * UPR * 2 + c * 2) = __float2half(acc[f][mf][r4] * oscale);
+          *(__half*)(patch + (16 * mf + n) * BP + f * UPR * 2 + c * 2) = __float2half(acc[f][mf][r4]);
         }
     __syncthreads();
     const int j = tid & 15, c = nb * UPR + 8 * j;
@@ -997,7 +1002,7 @@ k_moe_stream(SW R, SW Sh, int n_experts, const __half* __restrict__ x, const int
   L.up_off = shared ? Sh.up_off : R.up_off;
   L.pexp = shared ? Sh.pexp : R.pexp;
   const int e = shared ? 0 : tile.expert;
-  const int pexp = scaled(FMT) ? (int)L.pexp[e] : 0;
+  const int pexp = FMT == F_DN ? (int)L.pexp[e] : 0;
   const moe_cmag cmag = shared ? hs.c_shared : hs.c_routed;
   const int mfn = (tile.count + 15) >> 4;
   const bool two_tabs = R.cb != R.cb_up || Sh.cb != Sh.cb_up;  // (launch)
@@ -1141,7 +1146,7 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
   if ((up && fmt == F_Q80) || (!up && (q5(fmt) || once_rounded(fmt))) || (cap > 32 && (q5(fmt) || fmt == F_Q80))) return MOE_E_UNSUPPORTED;
   if (i4(fmt) && up != (rot != nullptr)) return MOE_E_INVALID;
   if (rot && (!rot->svh_gu || !rot->suh_dn)) return MOE_E_INVALID;
-  if (scaled(fmt) && (!pexp_routed || (sh && !pexp_sh))) return MOE_E_INVALID;
+  if (fmt == F_DN && (!pexp_routed || (sh && !pexp_sh))) return MOE_E_INVALID;
   if (!moe_aligned(x, 16) || !moe_aligned(out, 16)) return MOE_E_INVALID;
   if (max_tiles == 0) return MOE_OK;
   const SW R = to_dev(routed, nullptr, pexp_routed), S = to_dev(sh ? sh : routed, sh ? sh_cb_up : nullptr, sh ? pexp_sh : pexp_routed);

@@ -86,15 +86,17 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
                       const int* tokidx, const moe_tile* tiles, const int* ntiles, int max_tiles, __half* out, int m, int k,
                       moe_hscale hs, hipStream_t st, const float* sh_cb_up = nullptr, const int8_t* pexp_routed = nullptr,
                       const int8_t* pexp_sh = nullptr, const moe_rotv* rot = nullptr);
-// Scaled dequantisation of the grouped GEMMs (affine q4cp codebooks, i4r): per expert the power of two P with
+// Scaled dequantisation of the grouped GEMMs (affine q4cp codebooks): per expert the power of two P with
 // |cb slope| * (largest scale of the expert) * 2^(24+P) in [2^15, 2^16), or MOE_PEXP_NONE where the form does not apply
 // (a scale that is not finite, a zero slope, rows whose largest scale lies more than 2^6 below the expert's: their
 // weights would fall into the f16 denormals of the scaled units).  moe_scale_span fills one (hi, lo) pair of exponents per
-// expert for a tensor; moe_pexp_from_span combines the spans of the tensors one launch reads.
+// expert for a tensor; moe_pexp_from_span combines the spans of the tensors one launch reads.  i4r: moe_pexp_i4r, 0 where all of
+// the expert's scales are below 2^-4 (scale * 2^20 is an f16), else MOE_PEXP_NONE.
 constexpr int MOE_PEXP_NONE = -128;
 // group: columns per scale of the view's scale plane (32, 128)
 int moe_scale_span(const moe_lutw* w, int group, int n_experts, int rows, int cols, int8_t* span_dev, hipStream_t st);
 int moe_pexp_from_span(const int8_t* hi_lo_a, const int8_t* hi_lo_b);
+int moe_pexp_i4r(const int8_t* hi_lo);
 // The Q5_K form addresses weights and activations with 32-bit byte offsets: true when a tensor of `rows` rows of k
 // columns and an activation buffer of `x_rows` rows of k f16 values both stay below 4 GB (the caller of
 // moe_launch_gemm_q4cp(q5k = true) checks it; other layers take the general kernel)

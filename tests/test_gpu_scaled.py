@@ -1,6 +1,6 @@
-"""The grouped GEMMs' scaled dequantisation (codes read as f16 denormals, a power of two per expert) of rotated experts: experts
-that have such a power and experts that do not, in one layer, on the few-pair and the 128-pair kernels, against the oracle; and
-Q4_K experts, whose arithmetic has no such form, at the same scales.  Reference: src/gpu/parts/27_kernels_moe_lut.inc:16-29, 26_kernels_moe_gguf.inc:81-485."""
+"""The grouped GEMMs' dequantisation of codes that are read as f16 denormals (q4cp: with a power of two per expert): experts that
+have it and experts that do not, in one layer, on the few-pair and the 128-pair kernels, against the oracle; what the form
+does to the weights; and Q4_K experts, whose arithmetic has no such form, at the same scales.  Reference: src/gpu/parts/27_kernels_moe_lut.inc:16-29, 26_kernels_moe_gguf.inc:81-485."""
 import numpy as np
 import pytest
 
@@ -65,3 +65,43 @@ def test_experts_with_and_without_a_power_of_two(oracle, fmt, what, T):
     y = m.forward(0, torch.from_numpy(x).cuda())
     assert max_abs_rel(y.cpu().numpy(), yo) <= TOL_LAYER
     m.close()
+
+
+def run_both_kernels(hl, x, *options):
+    import torch
+    from gfx1151_engine_amd import capi
+    m, dev = hl.to_gpu(max_tokens=len(x))
+    ys = []
+    for o, v in options:
+        m.set_option(o, v)
+    for on in (1, 0):
+        m.set_option(capi.OPT_STREAM_GEMM, on)
+        ys.append(m.forward(0, torch.from_numpy(x).cuda()).cpu().numpy())
+        assert m.last_path() == capi.PATH_BATCH
+    m.close()
+    return ys
+
+
+@pytest.mark.parametrize("fused", [1, 0])
+@pytest.mark.parametrize("T", [40, 88, 152, 700])
+def test_rotated_experts_have_the_same_weights_in_either_form(T, fused):
+    """Every expert with one scale above the form's limit, in a group whose weights are all zero, which keeps it on the plain form;
+    and with that scale below it: the same results bit for bit, whatever the other groups' scales."""
+    from gfx1151_engine_amd import capi
+    d, mid, E = 768, 512, 16
+    x = np.random.default_rng(T).standard_normal((T, d), dtype=np.float32)
+    got = []
+    for s0 in (0.0624, 0.0625, 0.5):
+        hl = HostLayer(np.random.default_rng(5), d, mid, E, 4, fmt="i4r", bias=np.linspace(0, 0.5, E, dtype=np.float32))
+        for w, n, cols in ((hl.gate_up, 2 * mid, d), (hl.down, d, mid)):
+            codes = w[:E * n * cols // 2].reshape(E, n, cols // 128, 64)
+            sc = i4r_scales(w, E * n, cols).reshape(E, n, cols // 128)
+            sc[1, 8:40] *= np.float16(2.0 ** -6)   # rows and groups far below the expert's largest
+            sc[2:, :, 1] *= np.float16(2.0 ** -8)
+            sc[3, 9:20] = np.float16(2.0 ** -23)
+            codes[:, 5, 0] = 0x88
+            sc[:, 5, 0] = np.float16(s0)
+        got += run_both_kernels(hl, x, (capi.OPT_V2_FUSED_MIDDLE, fused))
+    assert np.isfinite(got[0]).all() and np.abs(got[0]).max() > 0
+    for i in (2, 3, 4, 5):
+        assert (got[i] == got[i & 1]).all()
