@@ -146,7 +146,7 @@ __device__ __forceinline__ void g2l4(const void* g, uint8_t* lds_base) {
 // FMA with a = f16(cb_a * scale) * 2^(24+P) (or 2^(20+P)) and b = f16(cb_b * scale) * 2^P gives 2^P * f16(n*a' + b'):
 // the weights of the three-instruction form times 2^P, bit for bit wherever the scaled weight is a normal f16 (the
 // product is exact inside the FMA, one rounding).  P is chosen when the weights are registered, from the expert's
-// largest scale, so that the scaled slope stays below 2^15 (an f16 can hold it); the accumulators carry the factor
+// largest scale, so that the scaled slope is a finite f16, 2^15 or more for the largest; the accumulators carry the factor
 // 2^P and the epilogue takes it out (exact).  v_pk_fma_f16 takes denormal operands at full rate on gfx950.
 // i4r (GS == 2), whose scales may lie far apart inside a row, takes the form without a power of two: all four nibbles of a half at
 // bits 4-7 (two more shifts for eight weights), a = scale * 2^20, b = -8 * scale, both exact while the expert's scales are below
@@ -1098,7 +1098,7 @@ __global__ void __launch_bounds__(256) k_scale_span(const uint8_t* __restrict__ 
         h = l = -127;
       } else if (s_lo[0] < INFINITY) {
         int eh, el;
-        if (frexpf(a * s_hi[0], &eh) >= 1.f - 0x1p-12f) eh++;  // (as rounded to f16)
+        if (frexpf(a * s_hi[0], &eh) >= 1.f - 0x1p-12f) eh++;  // (as an f16 that is a power of two)
         (void)frexpf(a * s_lo[0], &el);
         if (a * s_hi[0] <= 3.0e38f && a * s_lo[0] > 0.f && eh < 100 && el > -100) { h = eh; l = el; }
       }
@@ -1127,7 +1127,7 @@ int moe_pexp_from_span(const int8_t* a, const int8_t* b) {
     else if (b[0] != -127) { hi = b[0] > hi ? b[0] : hi; lo = b[1] < lo ? b[1] : lo; }
   }
   if (hi == -127) return 0;          // nothing but zeros: any power will do
-  if (hi - lo > 6) return MOE_PEXP_NONE;
+  if (hi - lo > 5) return MOE_PEXP_NONE;
   const int P = -8 - hi;             // |slope| * scale * 2^(24+P) < 2^16, rounded to f16 already (k_scale_span)
   return P < -100 || P > 100 ? MOE_PEXP_NONE : P;
 }

@@ -88,8 +88,8 @@ int moe_launch_stream(int fmt, bool up, int cap, const moe_lutw* routed, const m
                       const int8_t* pexp_sh = nullptr, const moe_rotv* rot = nullptr);
 // Scaled dequantisation of the grouped GEMMs (affine q4cp codebooks): per expert the power of two P with
 // |cb slope| * (largest scale of the expert) * 2^(24+P) in [2^15, 2^16), or MOE_PEXP_NONE where the form does not apply
-// (a scale that is not finite, a zero slope, rows whose largest scale lies more than 2^6 below the expert's: their
-// weights would fall into the f16 denormals of the scaled units).  moe_scale_span fills one (hi, lo) pair of exponents per
+// (a scale that is not finite, a zero slope, rows whose largest scale lies more than 2^5 below the expert's: their
+// weights would fall into the f16 denormals of the scaled units; up to there the row's largest slope is 2^-14 or more).  moe_scale_span fills one (hi, lo) pair of exponents per
 // expert for a tensor; moe_pexp_from_span combines the spans of the tensors one launch reads.  i4r: moe_pexp_i4r, 0 where all of
 // the expert's scales are below 2^-4 (scale * 2^20 is an f16), else MOE_PEXP_NONE.
 constexpr int MOE_PEXP_NONE = -128;

@@ -105,3 +105,33 @@ def test_rotated_experts_have_the_same_weights_in_either_form(T, fused):
     assert np.isfinite(got[0]).all() and np.abs(got[0]).max() > 0
     for i in (2, 3, 4, 5):
         assert (got[i] == got[i & 1]).all()
+
+
+def q4cp_scales(blob, rows, cols):
+    return blob[64 + rows * cols // 2:].view(np.float16).reshape(rows, -1)
+
+
+@pytest.mark.parametrize("T", [40, 88, 152, 700])
+@pytest.mark.parametrize("below", [5, 6, 7])
+def test_rows_far_below_an_experts_largest_scale(oracle, below, T):
+    """Rows whose largest scale lies 2^-5 below the expert's are the last that the scaled form takes; an expert with rows of 2^-6 has the
+    plain form's weights bit for bit, those of a layer whose every expert has another row, of zeros, further below."""
+    d, mid, E = 512, 640, 16
+    x = np.random.default_rng(T).standard_normal((T, d), dtype=np.float32)
+    got = []
+    for zeros in (below, 9):
+        hl = HostLayer(np.random.default_rng(9), d, mid, E, 4, shared=False, bias=np.linspace(0, 0.5, E, dtype=np.float32))
+        for w, n, cols in ((hl.gate_up, 2 * mid, d), (hl.down, d, mid)):
+            codes = w[64:64 + E * n * cols // 2].reshape(E, n, cols // 2)
+            sc = q4cp_scales(w, E * n, cols)[:, :cols // 32].reshape(E, n, cols // 32)
+            sc[:] = np.minimum(sc, np.float16(0.03))
+            sc[:, :, 0] = np.float16(0.03)
+            sc[:, 10:60] *= np.float16(2.0 ** -below)
+            codes[:, 5] = 0x88
+            sc[:, 5] = np.float16(0.03 * 2.0 ** -zeros)
+        got.append(run_both_kernels(hl, x))
+    yo, _, _ = oracle.moe_layer(hl.oracle_layer(), x)
+    for y in got[0]:
+        assert max_abs_rel(y, yo) <= TOL_LAYER
+    if below > 5:
+        assert (got[0][0] == got[1][0]).all() and (got[0][1] == got[1][1]).all()
