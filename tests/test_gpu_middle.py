@@ -353,9 +353,11 @@ STREAM_KINDS = [("q4cp", dict(fmt="q4cp"), 512, 640), ("q4cp-affine", dict(fmt="
                 ("q5k-q8_0", dict(fmt="q4k", gg_types=(13, 8, 8)), 512, 768), ("q4k-q8_0", dict(fmt="q4k", gg_types=(12, 8, 8)), 512, 768)]
 
 
-def both_kernels(capi, hl, x):
+def both_kernels(capi, hl, x, *options):
     m, dev = hl.to_gpu(max_tokens=len(x))
     ys = []
+    for o, v in options:
+        m.set_option(o, v)
     for on in (1, 0):
         m.set_option(capi.OPT_STREAM_GEMM, on)
         ys.append(m.forward(0, gpu(x)).cpu().numpy())
@@ -388,6 +390,36 @@ def test_few_pair_tiles_multiply_the_same_weights(capi, kind, kw, d, mid, T):
     x = np.zeros((T, d), np.float32)
     x[np.arange(T), rng.integers(0, d, T)] = rng.choice([-2.0, 1.0, 0.5], T) * 16
     y1, y0 = both_kernels(capi, hl, x)
+    assert np.abs(y0).max() > 0
+    assert (y1 == y0).all()
+
+
+@pytest.mark.parametrize("fused", [1, 0])
+@pytest.mark.parametrize("T", [40, 88, 152])
+@pytest.mark.parametrize("kind", ["i4r", "i4r-mixed"])
+def test_few_pair_tiles_multiply_the_same_rotated_weights(capi, kind, T, fused):
+    """Tokens that the rotation turns into one column, down_proj of one column: every sum over the weights has one term here too.
+    In a layer with one expert of larger scales the streaming launches give all experts the plain form, the 128-pair ones that expert."""
+    rng = np.random.default_rng(T)
+    d, mid, E, k = 512, 768, 16, 4
+    hl = HostLayer(rng, d, mid, E, k, fmt="i4r", shared=False, bias=np.linspace(0, 0.5, E, dtype=np.float32))
+    hl.planes = [np.ones_like(p) for p in hl.planes]
+    for w, n, cols in ((hl.gate_up, 2 * mid, d), (hl.down, d, mid)):
+        sc = w[E * n * cols // 2:].view(np.float16).reshape(E, n, cols // 128)
+        sc[:, :, 1] *= np.float16(2.0 ** -7)  # (weights that would be subnormal in units of an expert's largest scale)
+        if kind == "i4r-mixed":
+            sc[7, 3] = np.float16(0.25)
+    dn = hl.down[:E * d * mid // 2].reshape(E, d, mid // 2)
+    for e in range(E):
+        col = dn[e, :, 23 * e].copy()
+        dn[e] = 0x88
+        dn[e, :, 23 * e] = (col & 15) | 0x80
+    had = np.ones((1, 1), np.float32)
+    while len(had) < 128:
+        had = np.block([[had, had], [had, -had]])
+    x = np.zeros((T, d // 128, 128), np.float32)
+    x[np.arange(T), rng.integers(0, d // 128, T)] = had[rng.integers(0, 128, T)] * rng.choice([-2.0, 1.0, 0.5], (T, 1)).astype(np.float32)
+    y1, y0 = both_kernels(capi, hl, x.reshape(T, d), (capi.OPT_V2_FUSED_MIDDLE, fused))
     assert np.abs(y0).max() > 0
     assert (y1 == y0).all()
 
