@@ -28,7 +28,7 @@ def change(hl, what):
                 s[n + 3:n + 9] *= np.float16(2.0 ** -9)
             elif what == "zero":
                 s[n:2 * n] = 0
-            elif what == "edge":  # a largest scale that ends just under a power of two
+            elif what == "edge":  # a largest scale above the form's limit
                 s[n, 0] = np.float16(0.12494)
     else:
         for w, rows, cols in ((hl.gate, mid, d), (hl.up, mid, d), (hl.down, d, mid)):
@@ -109,6 +109,27 @@ def test_rotated_experts_have_the_same_weights_in_either_form(T, fused):
 
 def q4cp_scales(blob, rows, cols):
     return blob[64 + rows * cols // 2:].view(np.float16).reshape(rows, -1)
+
+
+# slope * largest scale as a mantissa in [0.5, 1): with 1.5 * 5461 / 8192 it rounds to 1 as an f16 (the power of two has to leave
+# that out, or the slope is infinite in the kernels), with 5459 / 8192 just not
+@pytest.mark.parametrize("T", [40, 88, 152, 700])
+@pytest.mark.parametrize("slope", [5461 / 8192, 5460 / 8192, 5459 / 8192, 1.0])
+def test_slopes_that_round_up_to_a_power_of_two(oracle, slope, T):
+    rng = np.random.default_rng(T)
+    d, mid, E = 512, 640, 16
+    cb = (np.arange(16) - 8).astype(np.float32) * np.float32(slope)
+    assert all(cb[n] == np.float32(n * (float(cb[1]) - float(cb[0])) + float(cb[0])) for n in range(16))
+    hl = HostLayer(rng, d, mid, E, 4, codebook=cb, bias=np.linspace(0, 0.5, E, dtype=np.float32))
+    top = np.float16(1.5 * 2.0 ** -6)
+    for w, n, cols in ((hl.gate_up, E * 2 * mid, d), (hl.down, E * d, mid), (hl.shared[0], mid, d), (hl.shared[1], mid, d), (hl.shared[2], d, mid)):
+        sc = q4cp_scales(w, n, cols)[:, :cols // 32]
+        sc[:] = np.minimum(sc, top)
+        sc[3::7, 1] = top
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    yo, _, _ = oracle.moe_layer(hl.oracle_layer(), x)
+    for y in run_both_kernels(hl, x):
+        assert np.isfinite(y).all() and max_abs_rel(y, yo) <= TOL_LAYER
 
 
 @pytest.mark.parametrize("T", [40, 88, 152, 700])
