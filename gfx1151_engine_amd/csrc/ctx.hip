@@ -46,8 +46,6 @@ static int codebook_affine(const moe_wview* w, bool* out) {
 }
 
 struct moe_ctx;
-static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_lutw* a, const moe_lutw* b, int group, int rows, int cols,
-                         int n_experts, bool* all);
 static int magnitude_constant(moe_ctx* c, int tgu, int tdn, const moe_wview* gate, uint64_t gate_stride,
                               const moe_wview* up, uint64_t up_first, const moe_wview* down, int n_experts,
                               moe_cmag* out);
@@ -134,19 +132,19 @@ struct moe_ctx {
   __half* v2_z16 = nullptr;      // [kT][2 mid]
 };
 
-// Scaled dequantisation of the grouped GEMM: the powers of two of the experts of tensor a (and, for a launch that reads
-// two tensors -- a shared expert's gate_proj and up_proj --, of a and b together) into slots slot0 .. of the layer's
-// table.  a == nullptr: the form is switched off for these slots.  Set-up work (a scan of the scale planes, a read-back).
 static int8_t* pexp_slot(moe_ctx* c, int layer, int slot0) {
   return c->pexp ? c->pexp + (size_t)layer * (2 * (size_t)c->cfg.experts + 2) + slot0 : nullptr;
 }
-// rows, cols: of one expert; group: columns of a scale, 128 is i4r.  *all: every expert has one.
-static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_lutw* a, const moe_lutw* b, int group, int rows, int cols,
-                         int n_experts, bool* all) {
-  *all = false;
-  int8_t* dst = pexp_slot(c, layer, slot0);
-  if (!dst) return MOE_OK;  // contexts for small batches only have no grouped GEMM
-  std::vector<int8_t> out((size_t)n_experts, (int8_t)MOE_PEXP_NONE);
+// Scaled dequantisation of the grouped GEMM: the powers of two of the experts of tensor a (and, for a launch that reads
+// two tensors -- a shared expert's gate_proj and up_proj --, of a and b together).  a == nullptr: none has the form.  rows,
+// cols: of one expert; group: columns of a scale, 128 is i4r.  Set-up work (a scan of the scale planes, a read-back).
+struct Pexp {
+  std::vector<int8_t> v;
+  bool all = false;  // every expert has the form
+};
+static int pexp_find(moe_ctx* c, const moe_lutw* a, const moe_lutw* b, int group, int rows, int cols, int n_experts, Pexp* out) {
+  if (!c->pexp) return MOE_OK;  // contexts for small batches only have no grouped GEMM
+  out->v.assign((size_t)n_experts, (int8_t)MOE_PEXP_NONE);
   if (a) {
     std::vector<int8_t> sa((size_t)2 * n_experts), sb;
     int rc = moe_scale_span(a, group, n_experts, rows, cols, c->span_tmp, nullptr);
@@ -157,14 +155,22 @@ static int pexp_register(moe_ctx* c, int layer, int slot0, const moe_lutw* a, co
       if ((rc = moe_scale_span(b, group, n_experts, rows, cols, c->span_tmp, nullptr))) return rc;
       MOE_HIP(hipMemcpy(sb.data(), c->span_tmp, sb.size(), hipMemcpyDeviceToHost));
     }
-    *all = true;
+    out->all = true;
     for (int e = 0; e < n_experts; e++) {
-      out[e] = (int8_t)(group == 128 ? moe_pexp_i4r(&sa[2 * e]) : moe_pexp_from_span(&sa[2 * e], b ? &sb[2 * e] : nullptr));
-      *all = *all && out[e] != (int8_t)MOE_PEXP_NONE;
+      out->v[e] = (int8_t)(group == 128 ? moe_pexp_i4r(&sa[2 * e]) : moe_pexp_from_span(&sa[2 * e], b ? &sb[2 * e] : nullptr));
+      out->all = out->all && out->v[e] != (int8_t)MOE_PEXP_NONE;
     }
   }
-  MOE_HIP(hipMemcpy(dst, out.data(), out.size(), hipMemcpyHostToDevice));
   return MOE_OK;
+}
+// ... into slots slot_a .. and slot_b .. of the layer's table, the last step of a registration that can fail: what the layer held
+// before would be multiplied with the new powers, so a failure clears it.
+static int pexp_write(moe_ctx* c, int layer, int slot_a, const Pexp& a, int slot_b, const Pexp& b) {
+  if (!c->pexp) return MOE_OK;
+  hipError_t e = hipMemcpy(pexp_slot(c, layer, slot_a), a.v.data(), a.v.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(pexp_slot(c, layer, slot_b), b.v.data(), b.v.size(), hipMemcpyHostToDevice);
+  if (e != hipSuccess) c->layers[layer] = MoeLayer();
+  return (int)e;
 }
 
 static void prof_mark(moe_ctx* c, int stage_done, hipStream_t st) {
@@ -317,15 +323,17 @@ MOE_API int moe_set_router(moe_ctx* c, int layer, const moe_wview* w, const floa
   if (!L || !w || !w->data) return MOE_E_INVALID;
   if (w->dtype != MOE_DT_F32 && w->dtype != MOE_DT_BF16) return MOE_E_UNSUPPORTED;
   if ((int)w->rows != c->cfg.experts || (int)w->cols != c->cfg.d) return MOE_E_INVALID;
-  const int rn = moe_router_row_norm_max(w, c->sample, &L->router_wmax);
+  float wmax = 0.f, bmax = 0.f;
+  const int rn = moe_router_row_norm_max(w, c->sample, &wmax);
   if (rn) return rn;
-  L->router_bmax = 0.f;
   if (bias) {
     std::vector<float> hb((size_t)w->rows);
     MOE_HIP(hipMemcpy(hb.data(), bias, hb.size() * 4, hipMemcpyDeviceToHost));
     for (float b : hb)
-      if (b != -INFINITY) L->router_bmax = fmaxf(L->router_bmax, fabsf(b));
+      if (b != -INFINITY) bmax = fmaxf(bmax, fabsf(b));
   }
+  L->router_wmax = wmax;
+  L->router_bmax = bmax;
   L->router = *w;
   L->router_bias = bias;
   L->has_router = true;
@@ -343,15 +351,20 @@ MOE_API int moe_set_experts_q4cp(moe_ctx* c, int layer, const moe_wview* gu, con
   bool a1 = false, a2 = false;
   int rc;
   if ((rc = codebook_affine(gu, &a1)) || (rc = codebook_affine(dn, &a2))) return rc;
-  L->experts_affine = a1 && a2;
-  if ((rc = magnitude_constant(c, 0, 0, gu, (uint64_t)2 * g.mid, gu, (uint64_t)g.mid, dn, g.experts, &L->c_routed)))
-    return rc;
+  moe_cmag cmag{0.f, 0.f};
+  if ((rc = magnitude_constant(c, 0, 0, gu, (uint64_t)2 * g.mid, gu, (uint64_t)g.mid, dn, g.experts, &cmag))) return rc;
   moe_lutw vg, vd;
   moe_lut_q4cp_view(gu->data, gu->rows, gu->cols, gu->scale_stride, 2 * g.mid, g.mid, &vg);
   moe_lut_q4cp_view(dn->data, dn->rows, dn->cols, dn->scale_stride, g.d, 0, &vd);
-  if ((rc = pexp_register(c, layer, 0, a1 ? &vg : nullptr, nullptr, 32, 2 * g.mid, g.d, g.experts, &L->scaled_gu)) ||
-      (rc = pexp_register(c, layer, g.experts, a2 ? &vd : nullptr, nullptr, 32, g.d, g.mid, g.experts, &L->scaled_dn)))
+  Pexp pg, pd;
+  if ((rc = pexp_find(c, a1 ? &vg : nullptr, nullptr, 32, 2 * g.mid, g.d, g.experts, &pg)) ||
+      (rc = pexp_find(c, a2 ? &vd : nullptr, nullptr, 32, g.d, g.mid, g.experts, &pd)) ||
+      (rc = pexp_write(c, layer, 0, pg, g.experts, pd)))
     return rc;
+  L->experts_affine = a1 && a2;
+  L->c_routed = cmag;
+  L->scaled_gu = pg.all;
+  L->scaled_dn = pd.all;
   L->gate_up = *gu;
   L->down = *dn;
   L->has_q4cp = true;
@@ -398,22 +411,25 @@ MOE_API int moe_set_experts_i4r(moe_ctx* c, int layer, const moe_wview* gu, cons
       return (int)e;
     }
   }
+  moe_cmag cmag{0.f, 0.f};
+  Pexp pg, pd;
   {
     moe_lutw vg, vd;
     int rc = moe_lut_i4r_view(gu->data, gu->rows, gu->cols, 2 * g.mid, g.mid, &vg);
     if (!rc) rc = moe_lut_i4r_view(dn->data, dn->rows, dn->cols, g.d, 0, &vd);
-    if (!rc) rc = pexp_register(c, layer, 0, &vg, nullptr, 128, 2 * g.mid, g.d, g.experts, &L->scaled_gu);
-    if (!rc) rc = pexp_register(c, layer, g.experts, &vd, nullptr, 128, g.d, g.mid, g.experts, &L->scaled_dn);
+    // (the batch path's f16 range guard; the small-batch kernels keep f32 between the projections)
+    if (!rc && c->v2_x16) rc = magnitude_constant_i4r(c, gu, dn, su, svh_gu, suh_dn, g.experts, &cmag);
+    if (!rc) rc = pexp_find(c, &vg, nullptr, 128, 2 * g.mid, g.d, g.experts, &pg);
+    if (!rc) rc = pexp_find(c, &vd, nullptr, 128, g.d, g.mid, g.experts, &pd);
+    if (!rc) rc = pexp_write(c, layer, 0, pg, g.experts, pd);
     if (rc) return rc;
   }
   L->gate_up = *gu;
   L->down = *dn;
   L->v2_su = su; L->v2_svh_gu = svh_gu; L->v2_suh_dn = suh_dn; L->v2_svh_dn = svh_dn;
-  L->c_routed = moe_cmag{0.f, 0.f};
-  if (c->v2_x16) {  // (the batch path's f16 range guard; the small-batch kernels keep f32 between the projections)
-    const int rm = magnitude_constant_i4r(c, gu, dn, su, svh_gu, suh_dn, g.experts, &L->c_routed);
-    if (rm) return rm;
-  }
+  L->c_routed = cmag;
+  L->scaled_gu = pg.all;
+  L->scaled_dn = pd.all;
   L->experts_affine = true;
   L->has_i4r = true;
   L->has_q4cp = false;
@@ -431,15 +447,16 @@ MOE_API int moe_set_experts_gguf(moe_ctx* c, int layer, const moe_gg_experts* gg
   MoeLayer* L = layer_of(c, layer);
   if (!L || !gg || !gg->gate || !gg->up || !gg->down) return MOE_E_INVALID;
   if (!moe_gg_types_supported(gg->tgu, gg->tdn, c->cfg.d, c->cfg.mid)) return MOE_E_UNSUPPORTED;
-  L->c_routed = moe_cmag{0.f, 0.f};
+  moe_cmag cmag{0.f, 0.f};
   {  // constant of the f16 range guard of the grouped GEMMs
     const moe_config& g = c->cfg;
     moe_wview gv{0, gg->gate, (uint64_t)g.experts * g.mid, (uint64_t)g.d, 0};
     moe_wview uv{0, gg->up, (uint64_t)g.experts * g.mid, (uint64_t)g.d, 0};
     moe_wview dv{0, gg->down, (uint64_t)g.experts * g.d, (uint64_t)g.mid, 0};
-    int rc = magnitude_constant(c, gg->tgu, gg->tdn, &gv, (uint64_t)g.mid, &uv, 0, &dv, g.experts, &L->c_routed);
+    int rc = magnitude_constant(c, gg->tgu, gg->tdn, &gv, (uint64_t)g.mid, &uv, 0, &dv, g.experts, &cmag);
     if (rc) return rc;
   }
+  L->c_routed = cmag;
   L->gg = *gg;
   L->has_gguf = true;
   L->has_q4cp = false;
@@ -466,31 +483,32 @@ MOE_API int moe_set_shared(moe_ctx* c, int layer, const moe_wview* g, const moe_
   } else if (!moe_gg_types_supported(sh_gguf_type, sh_gguf_type, cf.d, cf.mid)) {
     return MOE_E_UNSUPPORTED;
   }
-  L->shared_affine = false;
+  bool affine = false;
+  Pexp pu, pd;
+  int rc;
   if (sh_gguf_type == 0 && !dense) {
     bool a1 = false, a2 = false, a3 = false;
-    int rc;
     if ((rc = codebook_affine(g, &a1)) || (rc = codebook_affine(u, &a2)) || (rc = codebook_affine(dn, &a3))) return rc;
-    L->shared_affine = a1 && a2 && a3;
+    affine = a1 && a2 && a3;
     moe_lutw vg, vu, vd;
     moe_lut_q4cp_view(g->data, g->rows, g->cols, g->scale_stride, cf.mid, 0, &vg);
     moe_lut_q4cp_view(u->data, u->rows, u->cols, u->scale_stride, cf.mid, 0, &vu);
     moe_lut_q4cp_view(dn->data, dn->rows, dn->cols, dn->scale_stride, cf.d, 0, &vd);
-    if ((rc = pexp_register(c, layer, 2 * cf.experts, a1 && a2 ? &vg : nullptr, &vu, 32, cf.mid, cf.d, 1, &L->scaled_sgu)) ||
-        (rc = pexp_register(c, layer, 2 * cf.experts + 1, a3 ? &vd : nullptr, nullptr, 32, cf.d, cf.mid, 1, &L->scaled_sdn)))
+    if ((rc = pexp_find(c, a1 && a2 ? &vg : nullptr, &vu, 32, cf.mid, cf.d, 1, &pu)) ||
+        (rc = pexp_find(c, a3 ? &vd : nullptr, nullptr, 32, cf.d, cf.mid, 1, &pd)))
       return rc;
-  } else {
-    int rc;
-    if ((rc = pexp_register(c, layer, 2 * cf.experts, nullptr, nullptr, 32, cf.mid, cf.d, 1, &L->scaled_sgu)) ||
-        (rc = pexp_register(c, layer, 2 * cf.experts + 1, nullptr, nullptr, 32, cf.d, cf.mid, 1, &L->scaled_sdn)))
-      return rc;
+  } else if ((rc = pexp_find(c, nullptr, nullptr, 32, cf.mid, cf.d, 1, &pu)) || (rc = pexp_find(c, nullptr, nullptr, 32, cf.d, cf.mid, 1, &pd))) {
+    return rc;
   }
-  L->c_shared = moe_cmag{0.f, 0.f};
-  {
-    const int t = dense ? dense : sh_gguf_type;
-    int rc = magnitude_constant(c, t, t, g, (uint64_t)cf.mid, u, 0, dn, 1, &L->c_shared);
-    if (rc) return rc;
-  }
+  moe_cmag cmag{0.f, 0.f};
+  const int t = dense ? dense : sh_gguf_type;
+  if ((rc = magnitude_constant(c, t, t, g, (uint64_t)cf.mid, u, 0, dn, 1, &cmag)) ||
+      (rc = pexp_write(c, layer, 2 * cf.experts, pu, 2 * cf.experts + 1, pd)))
+    return rc;
+  L->shared_affine = affine;
+  L->c_shared = cmag;
+  L->scaled_sgu = pu.all;
+  L->scaled_sdn = pd.all;
   L->sh_dense = dense;
   L->sh_gate = *g;
   L->sh_up = *u;

@@ -238,7 +238,9 @@ int moe_destroy(moe_ctx* ctx);
  * tensors: rows*cols int8 codes then rows*cols/32 fp16 scales over the whole tensor, src/hgn.h:18,176-183); or, with
  * sh_gguf_type != 0, raw GGUF rows of that one ggml type.  shared_expert_gate: f32 or bf16.
  * MOE_E_UNSUPPORTED for other matrix dtypes.  A densely stored shared expert of a q4cp layer runs in launches of its
- * own next to the routed experts' kernels. */
+ * own next to the routed experts' kernels.
+ * A call that fails leaves the layer as it was; if the runtime fails in its last step (a hipError_t), the layer is cleared and
+ * moe_forward returns MOE_E_STATE until it is set again. */
 int moe_set_router(moe_ctx* ctx, int layer, const moe_wview* gate_w, const float* router_bias);
 int moe_set_experts_q4cp(moe_ctx* ctx, int layer, const moe_wview* gate_up, const moe_wview* down);
 int moe_set_experts_gguf(moe_ctx* ctx, int layer, const moe_gg_experts* gg);

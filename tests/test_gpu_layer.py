@@ -519,3 +519,37 @@ def test_look_up_blocks(oracle, d, mid, E, k, shared, T):
     m.close()
     assert (ids == io[:, :k]).all()
     assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= TOL_LUT
+
+
+@pytest.mark.parametrize("what", ["experts", "shared", "gguf"])
+def test_a_refused_registration_leaves_the_layer_as_it_was(what):
+    """Blobs off their alignment are refused after their codebooks have been looked at: the layer's own weights, of the other kind of
+    codebook, go on as before, in the integer-dot and the look-up decode kernels and in batches."""
+    import torch
+    from gfx1151_engine_amd import capi
+    rng = np.random.default_rng(3)
+    d, mid, E, k = 512, 256, 8, 2
+    cb = None if what == "shared" else np.sort(rng.standard_normal(16)).astype(np.float32)
+    hl = HostLayer(rng, d, mid, E, k, codebook=cb, scale_std=0.05)
+    m, dev = hl.to_gpu(max_tokens=64)
+    xs = [gpu(rng.standard_normal((T, d), dtype=np.float32)) for T in (1, 20, 64)]
+    before = [m.forward(0, x).cpu().numpy() for x in xs]
+
+    def off(a):
+        t = torch.zeros(a.nbytes + 16, dtype=torch.uint8, device="cuda")
+        t[2:2 + a.nbytes] = gpu(a.view(np.uint8).reshape(-1))
+        return t[2:2 + a.nbytes]
+    with pytest.raises(capi.MoeError):
+        if what == "experts":
+            a = HostLayer(rng, d, mid, E, k)
+            m.set_experts_q4cp(0, capi.wview(off(a.gate_up), capi.Q4CP, E * 2 * mid, d), capi.wview(off(a.down), capi.Q4CP, E * d, mid))
+        elif what == "shared":
+            sh = [off(S.make_gg(rng, 12, r, c)) for r, c in ((mid, d), (mid, d), (d, mid))]
+            m.set_shared(0, capi.wview(sh[0], 0, mid, d), capi.wview(sh[1], 0, mid, d), capi.wview(sh[2], 0, d, mid),
+                         capi.wview(dev["shsg"], capi.F32, 1, d), 12)
+        else:
+            a = HostLayer(rng, d, mid, E, k, fmt="q4k")
+            m.set_experts_gguf(0, off(a.gate), off(a.up), off(a.down), 12, 12)
+    for x, y in zip(xs, before):
+        assert (m.forward(0, x).cpu().numpy() == y).all()
+    m.close()
