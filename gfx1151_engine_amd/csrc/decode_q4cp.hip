@@ -600,7 +600,10 @@ __global__ void __launch_bounds__(512) k_dec_dn(DnArgs2 A, const uint32_t* __res
 // With 24 groups one token waits for latency, not instructions, and half as many waves are slower: one token 79.8 and 80 .. 82,
 // table 112.5 and 114 .. 119; three tokens 74.5 either way.  Rows: more share a lane's activations, fewer leave more blocks and waves
 // (20 tokens, 4, 8, 12, 16 and 24 rows of 24 groups: 152, 142, 140, 141 and 142; 20 groups 8 and 16: 122 and 119; one token 4 and 8: 71.3, 72.2).
-template <int G, int ROWS, int LUT>
+// 16, 20 and 24 groups are the widths that this dealing fits: what is left of four slots' units after 64 has to divide 64 (17 and 18
+// would too, but their sums are no whole quads of lanes; narrower rows would want more slots to a wave).  All other widths stay on
+// half-waves, with the lanes past their groups idle.
+template <int G, int ROWS, bool LUT>
 __global__ void __launch_bounds__(256) k_dec_dn_packed(DnArgs2 A, const uint32_t* __restrict__ hplanes, const float2* __restrict__ hmeta,
                                                        const int* __restrict__ ids, const float* __restrict__ ws, int id_stride, int kpt,
                                                        int d, float* __restrict__ out, uint64_t out_stride,
@@ -619,7 +622,7 @@ __global__ void __launch_bounds__(256) k_dec_dn_packed(DnArgs2 A, const uint32_t
   const float* const tcb = has_shared ? A.shd.cb : A.dn.cb;
   float c0 = 0.f, c1 = 0.f, c2 = 0.f, c3 = 0.f;
   const int t2 = (int)(threadIdx.x + blockDim.x);
-  if (LUT == 1) {  // (a thread's first two pieces of each table)
+  if (LUT) {  // (a thread's first two pieces of each table)
     c0 = A.dn.cb[threadIdx.x >> 4 & 15];
     c1 = tcb[threadIdx.x >> 4 & 15];
     c2 = A.dn.cb[t2 >> 4 & 15];
@@ -630,13 +633,13 @@ __global__ void __launch_bounds__(256) k_dec_dn_packed(DnArgs2 A, const uint32_t
     wmine = (int)threadIdx.x < kpt ? ws[(size_t)tok * id_stride + threadIdx.x] : A.sh_logit[tok];
   // (branch-free loads, as above: a unit without a slot reads slot 0 and counts nothing)
   int slot[SETS], grp[SETS];
-  float m[SETS], ca[SETS], cb[SETS], cbk[SETS];
+  float m[SETS], ca[SETS], cb[SETS];
   const uint8_t *cp[SETS], *sp[SETS];
   uint64_t wss[SETS];
   uint32_t lt[SETS];
   XG x[LUT ? 1 : SETS];
   XF xh[LUT ? SETS : 1];
-  const uint32_t lut_r = LUT == 1 ? lut_at(lutmem) : 0u, lut_s = lut_r + LUT_BYTES;
+  const uint32_t lut_r = LUT ? lut_at(lutmem) : 0u, lut_s = lut_r + LUT_BYTES;
 #pragma unroll
   for (int i = 0; i < SETS; i++) {
     const int u = i ? 64 + lane % (R ? R : 1) : lane;
@@ -656,7 +659,6 @@ __global__ void __launch_bounds__(256) k_dec_dn_packed(DnArgs2 A, const uint32_t
     else load_xg(x[LUT ? 0 : i], hplanes, hmeta, (size_t)((tok * nslots + s) * G + grp[i]));
     lt[i] = ((shared ? lut_s : lut_r) >> 8) * 0x01010101u;
     ca[i] = wcb[1] - wcb[0];
-    cbk[i] = wcb[0];
     cb[i] = fmaf(8.f, ca[i], wcb[0]);
     cp[i] = codes + (uint64_t)row0 * rb + (uint32_t)grp[i] * 16;
     sp[i] = scales + (uint64_t)row0 * (uint32_t)wss[i] + (uint32_t)(grp[i] >> gsh) * 2;
@@ -684,7 +686,7 @@ __global__ void __launch_bounds__(256) k_dec_dn_packed(DnArgs2 A, const uint32_t
     }
   }
   __builtin_amdgcn_sched_barrier(0);  // every load is issued before the first dot product
-  if (LUT == 1) {
+  if (LUT) {
     if (threadIdx.x < 256) {
       lut_put(lut_r, threadIdx.x, c0);
       lut_put(lut_s, threadIdx.x, c1);
@@ -700,12 +702,9 @@ __global__ void __launch_bounds__(256) k_dec_dn_packed(DnArgs2 A, const uint32_t
     moe_lds_barrier();
     __builtin_amdgcn_sched_barrier(0);
   }
-  float sx[SETS];
-#pragma unroll
-  for (int i = 0; i < SETS; i++) sx[i] = LUT == 2 ? xf_sum(xh[LUT ? i : 0]) : 0.f;
   auto dot = [&](int i, const uint4& c, __half s, int row) {
     float v;
-    if (LUT) v = f32_dot<LUT>(c, xh[LUT ? i : 0], lt[i], ca[i], cbk[i], sx[i]);
+    if (LUT) v = f32_dot<1>(c, xh[LUT ? i : 0], lt[i], 0.f, 0.f, 0.f);
     else v = chunk_dot(c, x[LUT ? 0 : i], ca[i], cb[i]);
     v *= __half2float(s) * m[i];
     v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));  // xor 1
@@ -940,7 +939,7 @@ int moe_launch_dec_dn_lut(const moe_wview* dn, const moe_wview* sh_down, const f
   if (!affine) {
     const int bs4 = 64 * ((nslots + 3) / 4);
 #define DEC_DN_PACKED(G, ROWS)                                                                                                       \
-  k_dec_dn_packed<G, ROWS, 1><<<dim3(d / ROWS, P), bs4, lds, st>>>(A, nullptr, nullptr, ids, ws, id_stride, kpt, d, out, out_stride, hid_f32)
+  k_dec_dn_packed<G, ROWS, true><<<dim3(d / ROWS, P), bs4, lds, st>>>(A, nullptr, nullptr, ids, ws, id_stride, kpt, d, out, out_stride, hid_f32)
     bool taken = true;
     if (mid == 768 && P > 1) DEC_DN_PACKED(24, 8);
     else if (mid == 640 && P > 1) DEC_DN_PACKED(20, 8);
@@ -1011,7 +1010,7 @@ int moe_launch_dec_dn(const moe_wview* dn, const moe_wview* sh_down, const float
   const int nslots = kpt + (sh_down ? 1 : 0), bs = 64 * ((nslots + 1) / 2);
   const int bs4 = 64 * ((nslots + 3) / 4);
 #define DEC_DN_PACKED(G, ROWS)                                                                                                       \
-  k_dec_dn_packed<G, ROWS, 0><<<dim3(d / ROWS, P), bs4, 0, st>>>(A, hplanes, hmeta, ids, ws, id_stride, kpt, d, out, out_stride, nullptr)
+  k_dec_dn_packed<G, ROWS, false><<<dim3(d / ROWS, P), bs4, 0, st>>>(A, hplanes, hmeta, ids, ws, id_stride, kpt, d, out, out_stride, nullptr)
   bool taken = true;
   if (mid == 768 && P > 3 && d % 12 == 0) DEC_DN_PACKED(24, 12);
   else if (mid == 768 && P > 3) DEC_DN_PACKED(24, 8);

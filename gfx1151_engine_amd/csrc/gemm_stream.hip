@@ -590,8 +590,7 @@ __device__ __forceinline__ void up_tile(uint8_t* smem, const SW& L, int e, const
   };
   auto load_half = [&](uint4(&q)[2], int i, int E) {
     const bool past = i >= nline;
-    const bool end = i == nline - 1;
-    const size_t at = past ? (size_t)0 : E && ro && end ? (size_t)0 : (size_t)i * LB + ro + (E && !(tail && end) ? 64 : 0);
+    const size_t at = past ? (size_t)0 : (size_t)i * LB + (E && !(tail && i == nline - 1) ? 64 : 0);
 #pragma unroll
     for (int f = 0; f < 2; f++) q[f] = *(const uint4*)(wb[f] + at + (past ? 0u : wo + 16u * (uint32_t)g));
   };
