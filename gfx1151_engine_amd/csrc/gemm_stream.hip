@@ -1065,11 +1065,12 @@ int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* 
 // and 22; 64-pair tiles at an average of 25 against 32-pair ones: 797 -> 779 us per layer (q4cp), 740 -> 738 (i4r).  Above, more
 // and more experts take a second tile and the 128-pair kernels draw level; the line lies where they do, for each kind of
 // layer with its own kernels, at even and at Zipf-skewed routing.  Layers, us, 128-pair kernels and these (3072 x 768):
-//   average pairs        51, even / skewed            59                         62, table 66           66, table 70
-//   q4cp                 907 833 / 935 855            949 896 / 999 922          984 948 / 1047 951     1015 1033 / 1070 981
+//   average pairs        51, even / skewed            56, table 60               62, table 66           66, table 70
+//   q4cp                 889 819 / 921 834            914 850 / 959 870          961 923 / 1013 927     996 1006 / 1050 953
 //   Q4_K                 966 927 / 1012 950           1005 995 / 1062 982 (55)   1043 1053 / 1115 1058
-//   i4r                  921 862 / 940 884            967 938 / 1016 967         1001 1000 / 1068 1005  1042 1088 / 1089 1038
-//   table                                             1183 1063 / 1247 1080 (60) 1232 1204              1265 1272 / 1348 1215
+//   i4r                  866 794 / 896 824            890 841 / 933 862          952 918 / 999 921      986 995 / 1032 951
+//   table                                             1142 1021 / 1193 1043      1194 1163 / 1262 1102  1239 1234 / 1300 1182
+// (i4r's line was found while its weights took an instruction more on either side, and lies a few pairs short of that.)
 // That is of layers whose weights are many.  With fewer the 128-pair kernels draw level earlier: a launch is then one or two rounds
 // of blocks, and a second tile of some experts is a round more.  d x mid x experts tells the layers apart better than either
 // width or the number of experts does.  q4cp, even / skewed, averages of 50, 56 and 62 (change against the 128-pair kernels, %):
@@ -1077,7 +1078,8 @@ int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* 
 //   4096 x 1024 of 128 (537 M) -6 / -9, -3, -1 / -4      2048 x 1024 of 256 (537 M) -3 / -4, -2, +2 / -3
 //   1024 x 512 of 1000 (524 M) -3 / -4, -3, 0 / -3       2048 x 768 of 256 (403 M)  0 / -4, 0, +2 / -4
 //   1024 x 768 of 512 (403 M)  0 / -5, +1, +3 / -1       3072 x 768 of 64 (151 M)   +9 / -1, +10, +15 / -3
-// (Q4_K and i4r 1 .. 2 % less throughout; table codebooks 2048 x 768 of 256 at 62 and 70 -3, 0, 3072 x 768 of 256 -3, +2.)  The
+// (i4r, even / skewed, 46, 50, 56 and 62: of 256 -8 / -6, -4 / -6, -3 / -5, 0 / -7; of 128 -6 / -8, -6 / -10, -5 / -10, +3 / -6.  Q4_K 1 .. 2 % less
+// throughout; table codebooks 2048 x 768 of 256 at 62 and 70 -3, 0, 3072 x 768 of 256 -3, +2.)  The
 // line between many and few lies between 403 and 524 M.
 constexpr int64_t MANY_WEIGHTS = (int64_t)7 << 26;
 // Q8_0 down rows beside Q4_K or Q5_K: the 128-pair kernels are k_moe_wide's, 32-pair tiles are the largest here.  Averages of 25, 28, 31
@@ -1088,8 +1090,11 @@ constexpr int64_t MANY_WEIGHTS = (int64_t)7 << 26;
 // +7 +10; 1024 x 512 of 128 (67 M) -1 -3 -2 +3 | +3 -1 +1 +6; 4096 x 1024 of 32 +1 +1 +1 +5 | +5 +4 +2 +5.  Below 34 M the two are
 // level at any average up to 38 (16 .. 64 experts of 512 x 256 .. 1024 x 768: 75 .. 95 us either way), and the line lies where
 // it did with slower 128-pair kernels.
-// Rows of more than four lines of hid (mid > 1024) leave no LDS for 64 pairs: 32-pair tiles as well, level earlier (2048 x 1536, even:
-// 23 q4cp 896 891, Q4_K 967 912; 29 q4cp 923 967, Q4_K 996 1038, table 1149 1139; 37 table 1248 1409).  Beside Q8_0, averages of 23,
+// Rows of more than four lines of hid (mid > 1024) leave no LDS for 64 pairs: 32-pair tiles as well, level earlier (2048 x 1536 of 512, even /
+// skewed: q4cp 23 882 869 / 920 909, 25 891 877 / 922 933, 27 899 908 / 940 962, 29 914 959 / 953 982; 2048 x 2048 of 256 25 608 587 / 636 623, 27
+// 613 594 / 643 639, 29 628 635 / 644 656; Q4_K 23 956 895 / 1010 986, 25 963 926 / 1012 1012, 27 978 963 / 1027 1047; table 29 1149 1054 / 1210
+// 1113, 33 1212 1188 / 1260 1207, 37 1263 1312 / 1280 1295: its line was found before tiles of 32 turned their lines (1149 1139 at 29, 1248 1409
+// at 37) and lies short of where both are level now).  Beside Q8_0, averages of 23,
 // 26, 29 and 32, Q4_K | Q5_K: 512 experts -5 -4 +2 +6 | -2 0 +6 +11; 128 0 +2 +9 +11 | +2 +5 +12 +16; 64 -4 -5 -3 +1 | -1 -1 +1 +9;
 // 16 -7 -4 +1 +5 | -8 -5 -4 +2.
 // (Q5_K with Q4_K down rows: 25, 28 and 31 3072 x 768 of 512 -7 -6 +1, of 256 -9 -5 0, 2048 x 768 of 256 -4 0 +8, 3072 x 768 of 64 -1 +1
