@@ -151,8 +151,8 @@ __device__ __forceinline__ void g2l4(const void* g, uint8_t* lds_base) {
 // i4r (GS == 2), whose scales may lie far apart inside a row, takes the form without a power of two: all four nibbles of a half at
 // bits 4-7 (two more shifts for eight weights), a = scale * 2^20, b = -8 * scale, both exact while the expert's scales are below
 // 2^-4: the three-instruction form's weights bit for bit, subnormal ones included.  us, with three instructions and so: 8192 tokens
-// (skewed) gate/up 1016 975, down 493 482.  (With a power of two as q4cp's it was no faster, 3001
-// tokens 864 and 867 a layer, and weights below 2^-14 of the scaled units -- 1.5 % of them where a row's scales are normally distributed -- lost
+// (skewed) gate/up 1016 975, down 493 482.  (With a power of two as q4cp's, 883 for 896 us
+// a layer of 3001 tokens, weights below 2^-14 of the scaled units -- 1.5 % of them where a row's scales are normally distributed -- lost
 // bits that the plain units keep.)
 // (Q4_K gained two per cent of a layer of 4096 tokens and more with it,
 // d and dmin brought into the scaled units, but products of theirs that are subnormal as f16 were then rounded otherwise than

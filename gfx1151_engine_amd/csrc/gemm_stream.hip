@@ -33,6 +33,7 @@
 // Measured (512 experts, top-10, 3072 x 768, gate/up + down, us; in brackets the 128-pair kernels):
 //   130 tokens q4cp 240 + 135 (354 + 178)      48 table 175 + 102 (298 + 170)    515 Q4_K 337 + 167 (431 + 234)
 //   200 Q5_K / Q8_0 396 + 282 (487 + 357)     200 i4r 266 + 135 (369 + 191)      2048 q4cp 357 + 206 (444 + 239)
+// (130 and 48 tokens behind a router launch with a redone logit, of which the chip comes back rested; else 253 + 138 and 195 + 107)
 // The layer at other widths (with q4cp and table rows as they lie, see up_rotates: up to 515 tokens 4 .. 10 % more than now), us (128-pair
 // kernels in brackets), 48 / 515 / 1200 tokens, d = 3072: mid 256 q4cp 162 / 258 / 331 (207 / 307 /
 // 361), Q5_K / Q8_0 214 / 343 / 437 (261 / 409 / 461); 512 q4cp 245 / 401 / 474 (312 / 491 / 549), table 272 / 434 / 535 (392 / 610 / 639),

@@ -338,7 +338,9 @@ int moe_forward_x16(moe_ctx* ctx, int layer, const float* x, const void* x16, in
 /* MOE_OPT_STREAM_GEMM (default 1): batches in which an expert has few pairs (33 tokens up to an average of 22 to 160 pairs,
  * by kind of layer) run the
  * routed experts' two GEMMs on tiles of 16 to 64 pairs with the weights streamed into registers; 0 = the 128-pair
- * kernels at every size.  The same f16 weights and f32 sums, in another order. */
+ * kernels at every size.  The same f16 weights and f32 sums, in another order.  On tiles of 16 and 32 pairs (averages up to 22) the
+ * order of a q4cp row's sums follows from where the code rows of the launch's tensors lie: 64 bytes behind a multiple of 128 (as behind
+ * the codebook of a blob that is a multiple itself), or elsewhere.  Copies of a layer at other offsets can differ in last bits. */
 enum { MOE_OPT_INT_DECODE = 1, MOE_OPT_UNIQUE_MIN_TOKENS = 2, MOE_OPT_FUSED_COMBINE = 3, MOE_OPT_SHARED_ASIDE = 4,
        MOE_OPT_TIMING_SKIP_STAGE = 5, MOE_OPT_ROUTER_CANDIDATES = 6, MOE_OPT_UNIQUE_GGUF = 7,
        MOE_OPT_GU_TOPK_MAX_TOKENS = 8, MOE_OPT_F32_DECODE_MAX_TOKENS = 9,
