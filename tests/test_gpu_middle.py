@@ -353,11 +353,9 @@ STREAM_KINDS = [("q4cp", dict(fmt="q4cp"), 512, 640), ("q4cp-affine", dict(fmt="
                 ("q5k-q8_0", dict(fmt="q4k", gg_types=(13, 8, 8)), 512, 768), ("q4k-q8_0", dict(fmt="q4k", gg_types=(12, 8, 8)), 512, 768)]
 
 
-def both_kernels(capi, hl, x, *options):
+def both_kernels(capi, hl, x):
     m, dev = hl.to_gpu(max_tokens=len(x))
     ys = []
-    for o, v in options:
-        m.set_option(o, v)
     for on in (1, 0):
         m.set_option(capi.OPT_STREAM_GEMM, on)
         ys.append(m.forward(0, gpu(x)).cpu().numpy())
@@ -419,9 +417,16 @@ def test_few_pair_tiles_multiply_the_same_rotated_weights(capi, kind, T, fused):
         had = np.block([[had, had], [had, -had]])
     x = np.zeros((T, d // 128, 128), np.float32)
     x[np.arange(T), rng.integers(0, d // 128, T)] = had[rng.integers(0, 128, T)] * rng.choice([-2.0, 1.0, 0.5], (T, 1)).astype(np.float32)
-    y1, y0 = both_kernels(capi, hl, x.reshape(T, d), (capi.OPT_V2_FUSED_MIDDLE, fused))
-    assert np.abs(y0).max() > 0
-    assert (y1 == y0).all()
+    m, dev = hl.to_gpu(max_tokens=T)
+    m.set_option(capi.OPT_V2_FUSED_MIDDLE, fused)
+    ys = []
+    for on in (1, 0):
+        m.set_option(capi.OPT_STREAM_GEMM, on)
+        ys.append(m.forward(0, gpu(x.reshape(T, d))).cpu().numpy())
+        assert m.last_path() == capi.PATH_BATCH
+    m.close()
+    assert np.abs(ys[1]).max() > 0
+    assert (ys[0] == ys[1]).all()
 
 
 # where the code planes lie against the cache lines (a blob's codes start 64 bytes behind it): the streaming GEMM turns its lines by half
