@@ -776,6 +776,9 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
   const bool use_intgg = L.has_gguf && c->int_decode && !use_int4k &&
                          moe_decgg_supported(L.gg.tgu, L.gg.tdn, L.sh_gguf_type, sh, g.d, g.mid, g.topk, g.experts) &&
                          (!sh || L.sh_gguf_type != 0);
+  // (Q4_K layers: the gate/up launch of the mixes where it deals its rows over all lanes)
+  const bool gu4k_dealt = use_int4k && moe_decgg_passes(g.d) > 0 &&
+                          moe_decgg_supported(L.gg.tgu, L.gg.tdn, L.sh_gguf_type, sh, g.d, g.mid, g.topk, g.experts);
   const bool use_uq = use_int && c->uq_min > 0 && P >= c->uq_min && moe_dec_uq_supported(g.d);
   // the same for GGUF layers on the integer-dot kernels (any mix of their four block types)
   const bool use_uq_gg = (use_int4k || use_intgg) && c->uq_gguf && c->uq_min > 0 && P >= c->uq_min && moe_decgg_uq_supported(g.d) &&
@@ -785,8 +788,11 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
   // latency-bound path than a top-k kernel, no last-block ticket in the logits launch)
   // -- as long as its blocks run in one round: each repeats the selection, 3 .. 4 us, where a launch of its own costs 7.
   // Two layers, us, in the gate/up launch and aside: look-up kernels 95.4 and 88.7 at 2 tokens; GGUF mixes 84.7 and 84.4 at 2,
-  // 122 and 119 at 3, 153 and 148 at 4; Q4_K 83.6 and 85.3 at 3, 113 and 108 at 4; q4cp 73.7 and 76.4 at 3, 100 and 97 at 4
-  const int topk_max = c->gu_topk_max >= 0 ? c->gu_topk_max : use_lut ? 1 : use_intgg ? 2 : use_f32a ? 4 : 3;
+  // 122 and 119 at 3, 153 and 148 at 4; Q4_K 83.6 and 85.3 at 3, 113 and 108 at 4; q4cp 73.7 and 76.4 at 3, 100 and 97 at 4; both kinds
+  // of GGUF layers with rows dealt over all lanes, whose rounds are shorter: mixes 104.5 and 106.4 at 3, 129.2 and 131.5 at 4, Q4_K 75.5
+  // and 82.7, 99.3 and 100.8 (above four the router launch leaves no bounds for the selection)
+  const bool gg_dealt = gu4k_dealt || (use_intgg && moe_decgg_passes(g.d) > 0);
+  const int topk_max = c->gu_topk_max >= 0 ? c->gu_topk_max : use_lut ? 1 : gg_dealt ? 4 : use_intgg ? 2 : use_f32a ? 4 : 3;
   const bool gu_topk = (((use_int && !use_uq) || ((use_int4k || use_intgg) && !use_uq_gg) || use_lut || use_f32a) && P <= topk_max) &&
                        moe_dec_gu_topk_supported(g.experts, g.topk);
   // (up to 4 tokens the router launch leaves each token's bound for the selection; larger batches: the selecting
@@ -932,6 +938,11 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
   }
   if (use_int4k) {
     if ((rc = stage(MOE_PROF_UP, [&]() -> int {
+           if (gu4k_dealt)
+             return gu_topk ? moe_launch_decgg_gu_topk(L.gg.tgu, L.sh_gguf_type, L.gg.gate, L.gg.up, rg, ru, c->xplanes, c->xmeta, c->logits,
+                                                       g.experts, c->ids, c->ws, g.id_stride, g.topk, P, g.d, g.mid, c->hplanes, c->hmeta, st, &rf)
+                            : moe_launch_decgg_gu(L.gg.tgu, L.sh_gguf_type, L.gg.gate, L.gg.up, rg, ru, c->xplanes, c->xmeta, c->ids,
+                                                  g.experts, g.id_stride, g.topk, P, g.d, g.mid, c->hplanes, c->hmeta, st);
            return gu_topk ? moe_launch_dec4k_gu_topk(L.gg.gate, L.gg.up, rg, ru, c->xplanes, c->xmeta, c->logits,
                                                      g.experts, c->ids, c->ws, g.id_stride, g.topk, P, g.d, g.mid,
                                                      c->hplanes, c->hmeta, st, &rf)
@@ -940,6 +951,11 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
          })))
       return rc;
     return stage(MOE_PROF_DOWN, [&]() -> int {
+      // (the mixes' down launch, three waves for ten slots instead of four, waits for less latency: Q4_K layers, 1 and 2 tokens, 82.6
+      // and 80.0 us, 61.2 60.0; at 3 81.4 82.7, 20 160.2 161.2)
+      if (gu4k_dealt && P <= 2)
+        return moe_launch_decgg_dn(L.gg.tdn, L.sh_gguf_type, L.gg.down, rd, c->sh_logit, c->hplanes, c->hmeta, c->ids, c->ws, g.id_stride,
+                                   g.topk, P, g.d, g.mid, y, (uint64_t)g.d, st);
       return moe_launch_dec4k_dn(L.gg.down, rd, c->sh_logit, c->hplanes, c->hmeta, c->ids, c->ws, g.id_stride, g.topk, P,
                                  g.d, g.mid, y, (uint64_t)g.d, st);
     });

@@ -4,7 +4,7 @@
 //   sum_k w_k x_k = d * (sc0 * qA * VA + sc1 * qB * VB) - dmin * (m0 * qA * SA + m1 * qB * SB)
 // with V = integer dot product of the codes with the activation group's two 8-bit digit planes
 // (natural element order) and q * S = the group's quantised sum.  A lane owns one unit of a row;
-// rows of 3072 are 48 units (lanes 48..63 idle: the kernels are bandwidth-bound), rows of 768 are
+// rows of 3072 are 48 units (gate/up deals several rows' units over a wave, ggu_gu_packed), rows of 768 are
 // 12 units (four slots per wave).
 // (reference: src/gpu/parts/26_kernels_moe_gguf.inc:527-568,693-756,893-939; src/gguf.h:328-336,408-441)
 #include "common.h"
@@ -115,7 +115,7 @@ struct Gu4kArgs {
 // rows of this block's 32; lane = unit (d/64 <= 64 units per row).  All 24 loads of a lane (8 rows x
 // two code halves + its dword of the header) are in flight together, in under 128 registers: two blocks fit
 // a CU, so the grid's 265 blocks are all resident at once (with one block per CU the last nine waited for a
-// second round).
+// second round).  For the widths that moe_decgg_passes leaves: k_decgg_gu deals the others' rows over all lanes.
 // NPL > 0 (E <= 64*NPL): only the logits are given; the blocks of the routed slots run the softmax /
 // top-k of their token themselves and block (0, 0, token) writes ids / weights out for the down
 // kernel (as in the q4cp gate/up kernel).
@@ -548,6 +548,69 @@ __device__ __forceinline__ void ggu_gu_rows(const uint8_t* gbase, const uint8_t*
   }
 }
 
+// The same eight rows with no lane idle, for rows of U = 8 NP units (NP 4 .. 7): a pass takes one row on lanes 0 .. U - 1, and the
+// other 64 - U lanes take the rows behind the first NP, unit by unit (rows follow one another in memory, and the first four are gate
+// rows, so what those lanes read is one run of the up tensor): 8 U units in NP passes instead of eight.  A sum of eight lanes lies
+// within a row on both sides; part[8 NP] = these sums in the order of the units.  xs: the token's activations in LDS, a unit's 128
+// + 16 bytes side by side (the pitch that 16-byte reads of neighbouring units want): lanes of the first kind read theirs once, the
+// others a unit's for each pass, which costs LDS a tenth of what the pass's vector instructions cost the SIMD.
+// What bounds the launch is those instructions (Q5_K: 145 a pass) from three tokens on, and the loads' latency below.  RB: passes in
+// flight; three (with the selection inside the launch, up to four tokens: 1 token, four layers, 100.3 -> 97.8 us; two and a ring of
+// five or six, which spills, are slower) or four (20 tokens 223.5, with three 224.1).
+// Layers, us, a lane per unit of a row and this (one token four layers, two and three two): 3072 x 768 Q5_K / Q8_0 1 token 109.9 96.5,
+// 2 79.6 71.2, 3 114.6 104.4, 4 141.7 129.2, 8 116.7 107.1, 20 244.8 223.6; Q4_K (k_dec4k_gu and this) 1 91.3 79.6, 2 65.6 59.0, 3 83.9 75.6,
+// 4 107.8 99.3, 8 82.0 77.2, 20 173.6 160.6; 1 and 20 tokens Q8_0 132 116, 296 278; Q5_1 / Q8_0 115 104, 244 232; IQ4_NL 116 98, 210 189;
+// IQ4_XS 118 101, 216 190; Q5_K / Q8_0 2048 wide 94 74, 201 161; 3584 125 114, 458 446; Q4_K 2560 wide 90 77, 159 143.
+constexpr int GXU_DW = 36;
+__device__ __forceinline__ void lds_xu(XU& x, const uint32_t* xs, int unit) {
+  const uint4* s = (const uint4*)(xs + unit * GXU_DW);
+#pragma unroll
+  for (int p = 0; p < 2; p++) {
+    const uint4 a0 = s[2 * p], a1 = s[2 * p + 1], b0 = s[4 + 2 * p], b1 = s[4 + 2 * p + 1];
+    x.a[p][0] = a0.x; x.a[p][1] = a0.y; x.a[p][2] = a0.z; x.a[p][3] = a0.w;
+    x.a[p][4] = a1.x; x.a[p][5] = a1.y; x.a[p][6] = a1.z; x.a[p][7] = a1.w;
+    x.b[p][0] = b0.x; x.b[p][1] = b0.y; x.b[p][2] = b0.z; x.b[p][3] = b0.w;
+    x.b[p][4] = b1.x; x.b[p][5] = b1.y; x.b[p][6] = b1.z; x.b[p][7] = b1.w;
+  }
+  const uint4 m = s[8];
+  x.qa = __uint_as_float(m.x); x.qsa = __uint_as_float(m.y); x.qb = __uint_as_float(m.z); x.qsb = __uint_as_float(m.w);
+}
+template <int T, int NP, int RB, class Stage>
+__device__ __forceinline__ void ggu_gu_packed(const uint8_t* gbase, const uint8_t* ubase, int r0, int lane, const uint32_t* xs, float* part,
+                                              Stage&& stage) {
+  constexpr int U = 8 * NP, L = 64 - U;
+  constexpr uint64_t rb = ggu_row_bytes(T, 64 * U);
+  const bool main_lane = lane < U;
+  const int u0 = main_lane ? lane : lane - U;
+  const uint8_t* const side = ubase + (uint64_t)(r0 + NP - 4) * rb;
+  GgU<T> u[RB];
+  auto fetch = [&](int p) {
+    const uint8_t* const row = (p < 4 ? gbase : ubase) + (uint64_t)(r0 + (p & 3)) * rb;
+    ggu_fetch<T>(main_lane ? row : side, main_lane ? u0 : u0 + p * L, u[p % RB]);
+  };
+#pragma unroll
+  for (int p = 0; p < RB; p++) fetch(p);
+  __builtin_amdgcn_sched_barrier(0);
+  stage();
+  XU x;
+  lds_xu(x, xs, u0);
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    if (p) {
+      const int un = u0 + p * L;
+      if (!main_lane) lds_xu(x, xs, un % U);
+    }
+    float v = ggu_dot<T>(u[p % RB], lane & 3, x);
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));   // xor 1
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));   // xor 2
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true));  // mirror in 8
+    if ((lane & 7) == 0) part[main_lane ? p * NP + (u0 >> 3) : NP * NP + ((u0 + p * L) >> 3)] = v;
+    __builtin_amdgcn_sched_barrier(0);  // passes are consumed in arrival order
+    if (p + RB < NP) fetch(p + RB);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 #define GGU_SWITCH(t, CALL)                                                       \
   switch (t) {                                                                    \
     case MOE_GGML_Q4_K: { constexpr int T = MOE_GGML_Q4_K; CALL; } break;          \
@@ -564,14 +627,18 @@ struct GuGgArgs {
 };
 
 // grid (mid/32, slots incl. shared + the exact top-k row, P); block 512: k_dec4k_gu<NPL> for any of the four types
-template <int NPL>
+// NP: rows of 8 NP units, dealt over all lanes (ggu_gu_packed); 0: a lane per unit of a row
+template <int NPL, int NP>
 __global__ void __launch_bounds__(512, 4) k_decgg_gu(GuGgArgs A, const uint32_t* __restrict__ xplanes,
                                                      const float2* __restrict__ xmeta, int id_stride, int kpt, int d,
                                                      int mid, uint32_t* __restrict__ hplanes,
                                                      float2* __restrict__ hmeta, const float* __restrict__ logits,
                                                      int n_experts, int* __restrict__ ids_out,
                                                      float* __restrict__ ws_out, const int* __restrict__ ids_in, moe_rfix RF) {
-  __shared__ float gs[G4_ROWS], us[G4_ROWS];
+  // a row's sums: of its eighths of 8 lanes, or of all of it; wave, row, part
+  constexpr int PARTS = NP ? NP : 1;
+  __shared__ float part[8 * 8 * PARTS];
+  __shared__ __attribute__((aligned(16))) uint32_t xs[NP ? 8 * NP * GXU_DW : 4];
   __shared__ uint32_t pk[QV_GROUP_DW];
   __shared__ int sel_ids[64];
   __shared__ float sel_ws[64];
@@ -587,7 +654,7 @@ __global__ void __launch_bounds__(512, 4) k_decgg_gu(GuGgArgs A, const uint32_t*
     }
     return;
   }
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = NP ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : (int)(threadIdx.x >> 6);
   const int U = d / 64;
   const bool shared = s >= kpt;
   int e = 0;
@@ -606,24 +673,42 @@ __global__ void __launch_bounds__(512, 4) k_decgg_gu(GuGgArgs A, const uint32_t*
   const uint8_t* gbase = shared ? A.sh_gate : A.gate + (uint64_t)e * mid * rb;
   const uint8_t* ubase = shared ? A.sh_up : A.up + (uint64_t)e * mid * rb;
   const int r0 = blockIdx.x * G4_ROWS + 4 * wv;
-  const bool live = lane < U;
-  const int ul = live ? lane : (lane & 3);
-  const float mlive = live ? 1.f : 0.f;
-  XU x;
-  load_xu(x, xplanes, xmeta, ((size_t)tok * U + ul) * 2);
-  float acc[8];
-  GGU_SWITCH(t, (ggu_gu_rows<T, (NPL > 0)>(gbase, ubase, r0, d, ul, mlive, x, acc)));
-  if (lane == 0) {
+  if constexpr (NP > 0) {
+    // (the activations, requested ahead of the weights, go to LDS behind the weights' requests)
+    const int t0 = (int)threadIdx.x;
+    const uint4 xp = ((const uint4*)xplanes)[(size_t)tok * (64 * NP) + (t0 < 64 * NP ? t0 : 0)];
+    const uint4 xm = ((const uint4*)xmeta)[(size_t)tok * (8 * NP) + (t0 < 8 * NP ? t0 : 0)];
+    __builtin_amdgcn_sched_barrier(0);
+    auto stage = [&]() {
+      if (t0 < 64 * NP) *(uint4*)(xs + (t0 >> 3) * GXU_DW + (t0 & 7) * 4) = xp;
+      if (t0 < 8 * NP) *(uint4*)(xs + t0 * GXU_DW + 32) = xm;
+      moe_lds_barrier();  // (the weights stay in flight)
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    GGU_SWITCH(t, (ggu_gu_packed<T, NP, (NPL > 0 ? 3 : 4)>(gbase, ubase, r0, lane, xs, part + 8 * NP * wv, stage)));
+  } else {
+    const bool live = lane < U;
+    const int ul = live ? lane : (lane & 3);
+    const float mlive = live ? 1.f : 0.f;
+    XU x;
+    load_xu(x, xplanes, xmeta, ((size_t)tok * U + ul) * 2);
+    float acc[8];
+    GGU_SWITCH(t, (ggu_gu_rows<T, (NPL > 0)>(gbase, ubase, r0, d, ul, mlive, x, acc)));
+    if (lane == 0) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      gs[4 * wv + i] = acc[i];
-      us[4 * wv + i] = acc[4 + i];
+      for (int i = 0; i < 8; i++) part[8 * wv + i] = acc[i];
     }
   }
   __syncthreads();
   if (wv == 0) {  // SwiGLU on the block's 32 rows = one activation group of the down projection; quantise it
     const int j = lane & 31;
-    const float g = gs[j], u = us[j];
+    const float* const pg = part + ((j >> 2) * 8 + (j & 3)) * PARTS;
+    float g = pg[0], u = pg[4 * PARTS];
+#pragma unroll
+    for (int i = 1; i < PARTS; i++) {
+      g += pg[i];
+      u += pg[4 * PARTS + i];
+    }
     const float hv = g / (1.f + expf(-g)) * u;
     float m = dpp_max_row(fabsf(hv));
     m = rows_half_max(m);
@@ -970,6 +1055,12 @@ bool moe_decgg_supported(int tgu, int tdn, int tsh, bool has_shared, int d, int 
          mid % G4_ROWS == 0 && d % D4_ROWS == 0 && ((kpt + 3) / 4 + 1) * 64 <= 320 && n_experts <= 1024 && kpt <= 64 &&
          kpt <= n_experts;
 }
+// Passes of the gate/up launch that deals its rows over all lanes, 0: rows that it does not take -- of 57 units and more, which leave
+// hardly a lane idle, of fewer than 32, whose spare lanes would reach into the gate rows, and those that are no whole eights of units,
+// whose sums would cross rows.
+int moe_decgg_passes(int d) {
+  return d % 512 == 0 && d >= 2048 && d <= 3584 ? d / 512 : 0;
+}
 static size_t ggu_align(int t) { return t == MOE_GGML_Q8_0 || t == MOE_GGML_IQ4_NL ? 4 : 16; }
 
 int moe_launch_decgg_gu_topk(int tgu, int tsh, const uint8_t* gate, const uint8_t* up, const uint8_t* sh_gate,
@@ -985,10 +1076,19 @@ int moe_launch_decgg_gu_topk(int tgu, int tsh, const uint8_t* gate, const uint8_
     return MOE_E_INVALID;
   GuGgArgs A{gate, up, sh_gate, sh_up, tgu, tsh};
   dim3 grid(mid / G4_ROWS, kpt + (sh_gate ? 1 : 0) + 1, P);
-  if (n_experts <= 512)
-    k_decgg_gu<8><<<grid, 512, 0, st>>>(A, xplanes, xmeta, id_stride, kpt, d, mid, hplanes, hmeta, logits, n_experts, ids, ws, nullptr, RFV);
-  else
-    k_decgg_gu<16><<<grid, 512, 0, st>>>(A, xplanes, xmeta, id_stride, kpt, d, mid, hplanes, hmeta, logits, n_experts, ids, ws, nullptr, RFV);
+#define DECGG_GU(NPL, NP) \
+  k_decgg_gu<NPL, NP><<<grid, 512, 0, st>>>(A, xplanes, xmeta, id_stride, kpt, d, mid, hplanes, hmeta, logits, n_experts, ids, ws, nullptr, RFV)
+#define DECGG_GU_NP(NPL)                                  \
+  switch (moe_decgg_passes(d)) {                          \
+    case 4: DECGG_GU(NPL, 4); break;                      \
+    case 5: DECGG_GU(NPL, 5); break;                      \
+    case 6: DECGG_GU(NPL, 6); break;                      \
+    case 7: DECGG_GU(NPL, 7); break;                      \
+    default: DECGG_GU(NPL, 0);                            \
+  }
+  if (n_experts <= 512) DECGG_GU_NP(8)
+  else DECGG_GU_NP(16)
+#undef DECGG_GU
   MOE_LAUNCH_CHECK();
   return MOE_OK;
 }
@@ -1004,8 +1104,11 @@ int moe_launch_decgg_gu(int tgu, int tsh, const uint8_t* gate, const uint8_t* up
     return MOE_E_INVALID;
   GuGgArgs A{gate, up, sh_gate, sh_up, tgu, tsh};
   dim3 grid(mid / G4_ROWS, kpt + (sh_gate ? 1 : 0), P);
-  k_decgg_gu<0><<<grid, 512, 0, st>>>(A, xplanes, xmeta, id_stride, kpt, d, mid, hplanes, hmeta, nullptr, n_experts, nullptr,
-                                      nullptr, ids, moe_rfix{});
+#define DECGG_GU(NPL, NP) \
+  k_decgg_gu<NPL, NP><<<grid, 512, 0, st>>>(A, xplanes, xmeta, id_stride, kpt, d, mid, hplanes, hmeta, nullptr, n_experts, nullptr, nullptr, ids, moe_rfix{})
+  DECGG_GU_NP(0)
+#undef DECGG_GU
+#undef DECGG_GU_NP
   MOE_LAUNCH_CHECK();
   return MOE_OK;
 }

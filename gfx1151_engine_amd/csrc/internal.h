@@ -194,6 +194,7 @@ int moe_launch_decgg_gu(int tgu, int tsh, const uint8_t* gate, const uint8_t* up
 int moe_launch_decgg_dn(int tdn, int tsh, const uint8_t* down, const uint8_t* sh_down, const float* sh_logit,
                         const uint32_t* hplanes, const float2* hmeta, const int* ids, const float* ws, int id_stride,
                         int kpt, int P, int d, int mid, float* out, uint64_t out_stride, hipStream_t st);
+int moe_decgg_passes(int d);
 bool moe_decgg_uq_supported(int d);
 int moe_decgg_uq_tile_cap();
 int moe_launch_decgg_gu_uq(int tgu, int tsh, const uint8_t* gate, const uint8_t* up, const uint8_t* sh_gate,

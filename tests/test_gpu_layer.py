@@ -296,6 +296,37 @@ def test_gguf_mixed_types(oracle, tgu, tdn, tsh, T):
     m.close()
 
 
+@pytest.mark.parametrize("T", [1, 2, 4, 5, 9])
+@pytest.mark.parametrize("types,d", [((12, 12, 12), 2048), ((12, 12, 12), 2560), ((12, 12, 12), 3072), ((12, 12, 12), 3584),
+                                     ((13, 8, 8), 2048), ((13, 8, 8), 2560), ((13, 8, 8), 3072), ((13, 8, 8), 3584), ((8, 8, 13), 2560),
+                                     ((7, 7, 12), 3072), ((20, 20, 23), 2560), ((23, 20, 20), 3584), ((13, 13, 7), 1792), ((12, 12, 12), 4096)])
+def test_small_batch_gguf_gate_up_rows_dealt_over_a_wave(oracle, types, d, T):
+    """Gate/up rows of 32, 40, 48 and 56 units, whose idle lanes take other rows (and of 28 and 64, which go a row at a time); the
+    selection inside the launch and ahead of it; the shared expert of the experts' type and of another."""
+    rng = np.random.default_rng(d + 10 * T + types[0])
+    hl = HostLayer(rng, d, 256, 10, 3, fmt="q4k", gg_types=types)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    yo, io, wo = oracle.moe_layer(hl.oracle_layer(), x)
+    y, ids, ws = run_layer(hl, x)
+    assert (ids[:, :3] == io[:, :3]).all()
+    assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= TOL_INT_Q4K
+
+
+@pytest.mark.parametrize("T", [1, 3])
+def test_gguf_gate_up_selects_among_more_than_512_experts(T):
+    """The selection inside the gate/up launch and the router's own give the same ids, and the rows' sums do not depend on it."""
+    import torch
+    from gfx1151_engine_amd import capi, workloads as W
+    L = W.DeviceLayer(1, 2048, 256, 520, 8, "q4k", gg_types=(13, 8, 8))
+    m = capi.Moe(2048, 256, 520, 8, layers=1, max_tokens=T)
+    L.register(m, 0)
+    x = torch.randn((T, 2048), device="cuda")
+    y = m.forward(0, x).clone()
+    m.set_option(capi.OPT_GU_TOPK_MAX_TOKENS, 0)
+    assert torch.equal(y, m.forward(0, x))
+    m.close()
+
+
 @pytest.mark.parametrize("tgu", [12, 13, 7, 8, 20, 23])
 def test_gguf_gate_up_rows_in_both_orders(oracle, tgu):
     """Every gate/up type (the shared expert's as well) in the launch that selects the experts itself, whose waves take their rows
