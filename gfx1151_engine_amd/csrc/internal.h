@@ -46,9 +46,10 @@ struct moe_rot_planes {
   uint32_t* planes;
   float2* meta;
 };
+enum { MOE_PLANES_QVEC4, MOE_PLANES_QVEC, MOE_PLANES_QVEC3 };  // (qvec.h)
 int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x,
                             int P, float* logits, float* out_x, uint32_t* planes, float2* meta,
-                            bool planes_natural, hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rot = nullptr,
+                            int planes_form, hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rot = nullptr,
                             float* tol_out = nullptr, float tol_scale = 0.f);
 // scratch of the column-split router launch (5..32 tokens): fp64 partial tiles of up to 8 splits x 32 tokens
 // for at most MOE_ROUTER_KSPLIT_ROWS rows, and one ticket counter (resting at 0) per 16 rows
@@ -184,16 +185,18 @@ int moe_launch_dec_dn_uq(const moe_wview* dn, const moe_wview* sh_down, const ui
 // the same for raw GGUF Q4_K rows (activation planes in natural order)
 bool moe_dec4k_supported(int d, int mid, int nslots);
 bool moe_decgg_supported(int tgu, int tdn, int tsh, bool has_shared, int d, int mid, int kpt, int n_experts);
+bool moe_decgg3_supported(int tgu, int tdn, int tsh, bool has_shared, int d, int mid, int kpt, int n_experts);
 int moe_launch_decgg_gu_topk(int tgu, int tsh, const uint8_t* gate, const uint8_t* up, const uint8_t* sh_gate,
                              const uint8_t* sh_up, const uint32_t* xplanes, const float2* xmeta, const float* logits,
                              int n_experts, int* ids, float* ws, int id_stride, int kpt, int P, int d, int mid,
-                             uint32_t* hplanes, float2* hmeta, hipStream_t st, const moe_rfix* rf = nullptr);
+                             uint32_t* hplanes, float2* hmeta, hipStream_t st, const moe_rfix* rf = nullptr, int planes = 2);
 int moe_launch_decgg_gu(int tgu, int tsh, const uint8_t* gate, const uint8_t* up, const uint8_t* sh_gate,
                         const uint8_t* sh_up, const uint32_t* xplanes, const float2* xmeta, const int* ids, int n_experts,
-                        int id_stride, int kpt, int P, int d, int mid, uint32_t* hplanes, float2* hmeta, hipStream_t st);
+                        int id_stride, int kpt, int P, int d, int mid, uint32_t* hplanes, float2* hmeta, hipStream_t st,
+                        int planes = 2);
 int moe_launch_decgg_dn(int tdn, int tsh, const uint8_t* down, const uint8_t* sh_down, const float* sh_logit,
                         const uint32_t* hplanes, const float2* hmeta, const int* ids, const float* ws, int id_stride,
-                        int kpt, int P, int d, int mid, float* out, uint64_t out_stride, hipStream_t st);
+                        int kpt, int P, int d, int mid, float* out, uint64_t out_stride, hipStream_t st, int planes = 2);
 int moe_decgg_passes(int d);
 bool moe_decgg_uq_supported(int d);
 int moe_decgg_uq_tile_cap();

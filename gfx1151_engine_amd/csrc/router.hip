@@ -167,13 +167,14 @@ __global__ void __launch_bounds__(256, 2) k_router_logits_seq(const void* __rest
 // q = index among these blocks, bs = block size.
 __device__ __forceinline__ void router_plane_blocks(int q, int bs, int tid, const float* __restrict__ x, int P, int d,
                                                     uint32_t* __restrict__ planes, float2* __restrict__ meta,
-                                                    bool planes_natural, const moe_rot_planes& R) {
+                                                    int planes_form, const moe_rot_planes& R) {
   const int G = d / 32, gb = (G + bs - 1) / bs;
   const int nq = planes ? P * gb : 0;
   if (q < nq) {
     const int t = q / gb, g = (q % gb) * bs + tid;
     if (t < P && g < G) {
-      if (planes_natural) qvec_group_from_f32(x, (uint64_t)d, G, t, g, planes, meta);  // Q4_K kernels
+      if (planes_form == MOE_PLANES_QVEC) qvec_group_from_f32<2>(x, (uint64_t)d, G, t, g, planes, meta);  // GGUF kernels
+      else if (planes_form == MOE_PLANES_QVEC3) qvec_group_from_f32<3>(x, (uint64_t)d, G, t, g, planes, meta);
       else qvec4_group_from_f32(x, (uint64_t)d, G, t, g, planes, meta);                       // q4cp kernels
     }
     return;
@@ -295,13 +296,13 @@ __global__ void __launch_bounds__(128) k_router_small(const void* __restrict__ W
                                                       const float* __restrict__ x, int E, int d,
                                                       float* __restrict__ logits, float* __restrict__ out_x,
                                                       int nrows, uint32_t* __restrict__ planes,
-                                                      float2* __restrict__ meta, bool planes_natural, moe_rot_planes rot,
+                                                      float2* __restrict__ meta, int planes_form, moe_rot_planes rot,
                                                       float* __restrict__ tol_out, float tol_scale) {
   // the wave index as a scalar: row, weight type and base address are then wave-uniform values
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int nrb = (nrows + 1) / 2;
   if ((int)blockIdx.x >= nrb) {
-    router_plane_blocks((int)blockIdx.x - nrb, (int)blockDim.x, (int)threadIdx.x, x, TT, d, planes, meta, planes_natural, rot);
+    router_plane_blocks((int)blockIdx.x - nrb, (int)blockDim.x, (int)threadIdx.x, x, TT, d, planes, meta, planes_form, rot);
     return;
   }
   const int row = blockIdx.x * 2 + wv;
@@ -343,12 +344,12 @@ __global__ void __launch_bounds__(256) k_router_mid(const void* __restrict__ W, 
                                                     const float* __restrict__ x, int P, int E, int d,
                                                     float* __restrict__ logits, float* __restrict__ out_x,
                                                     int nrows, uint32_t* __restrict__ planes,
-                                                    float2* __restrict__ meta, bool planes_natural, moe_rot_planes rot) {
+                                                    float2* __restrict__ meta, int planes_form, moe_rot_planes rot) {
   __shared__ __attribute__((aligned(16))) double Xd[2][PMAX][RM_C];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int nrb = (nrows + 3) >> 2;
   if ((int)blockIdx.x >= nrb) {
-    router_plane_blocks((int)blockIdx.x - nrb, 256, tid, x, P, d, planes, meta, planes_natural, rot);
+    router_plane_blocks((int)blockIdx.x - nrb, 256, tid, x, P, d, planes, meta, planes_form, rot);
     return;
   }
   // the wave's row as scalar values: the bf16 / f32 choice is then a scalar branch
@@ -513,14 +514,14 @@ __global__ void __launch_bounds__(512, 2) k_router_mfma(const void* __restrict__
                                                         const float* __restrict__ x, int P, int E, int d,
                                                         float* __restrict__ logits, float* __restrict__ out_x,
                                                         int nrows, uint32_t* __restrict__ planes,
-                                                        float2* __restrict__ meta, bool planes_natural, int KS,
+                                                        float2* __restrict__ meta, int planes_form, int KS,
                                                         double* gpart, unsigned* tickets, moe_rot_planes rot) {
   __shared__ double part[8][NTT][64][4];
   __shared__ int s_last;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nrt = (nrows + 15) >> 4;
   if ((int)blockIdx.x >= nrt * KS) {
-    router_plane_blocks((int)blockIdx.x - nrt * KS, 512, tid, x, P, d, planes, meta, planes_natural, rot);
+    router_plane_blocks((int)blockIdx.x - nrt * KS, 512, tid, x, P, d, planes, meta, planes_form, rot);
     return;
   }
   const int rg = (int)blockIdx.x % nrt, ks = (int)blockIdx.x / nrt;  // row group, column split
@@ -675,7 +676,7 @@ int moe_router_logits_seq(const moe_wview* W, const float* bias, const float* x,
 // planes of x for the integer-dot decode kernels) in the same launch.
 int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x,
                             int P, float* logits, float* out_x, uint32_t* planes, float2* meta,
-                            bool planes_natural, hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rotp,
+                            int planes_form, hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rotp,
                             float* tol_out, float tol_scale) {
   const int E = (int)W->rows, d = (int)W->cols;
   moe_rot_planes rot{nullptr, nullptr, nullptr};
@@ -702,8 +703,8 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
     // more than 24 tokens per block cost the kernel its second wave per SIMD (accumulators):
     // two launches of at most 16 tokens read the router matrix twice (L2 / MALL) and are faster
     const int P0 = 16, G = d / 32;
-    const size_t pdw = planes_natural ? QV_GROUP_DW : QV4_GROUP_DW;
-    int rc = moe_router_logits_small(W, bias, Wx, x, P0, logits, out_x, planes, meta, planes_natural, st, nullptr,
+    const size_t pdw = planes_form == MOE_PLANES_QVEC3 ? QV3_GROUP_DW : planes_form ? QV_GROUP_DW : QV4_GROUP_DW;
+    int rc = moe_router_logits_small(W, bias, Wx, x, P0, logits, out_x, planes, meta, planes_form, st, nullptr,
                                      nullptr, rotp);
     if (rc) return rc;
     moe_rot_planes rot2 = rot;
@@ -713,7 +714,7 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
     }
     return moe_router_logits_small(W, bias, Wx, x + (size_t)P0 * d, P - P0, logits + (size_t)P0 * E,
                                    out_x ? out_x + P0 : nullptr, planes ? planes + (size_t)P0 * G * pdw : nullptr,
-                                   meta ? meta + (size_t)P0 * G : nullptr, planes_natural, st, nullptr, nullptr,
+                                   meta ? meta + (size_t)P0 * G : nullptr, planes_form, st, nullptr, nullptr,
                                    rotp ? &rot2 : nullptr);
   }
   const bool bf = W->dtype == MOE_DT_BF16;
@@ -724,7 +725,7 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
   dim3 g((nrows + rpb - 1) / rpb + qblocks);
   const void* wx = Wx ? Wx->data : nullptr;
   if (P <= 4) {
-#define RSM_GO(BF, TT) k_router_small<BF, TT><<<g, bs, 0, st>>>(W->data, bias, wx, xbf, x, E, d, logits, out_x, nrows, planes, meta, planes_natural, rot, tol_out, tol_scale)
+#define RSM_GO(BF, TT) k_router_small<BF, TT><<<g, bs, 0, st>>>(W->data, bias, wx, xbf, x, E, d, logits, out_x, nrows, planes, meta, planes_form, rot, tol_out, tol_scale)
 #define RSM_T(TT) do { if (bf) RSM_GO(true, TT); else RSM_GO(false, TT); } while (0)
     if (P == 1) RSM_T(1);
     else if (P == 2) RSM_T(2);
@@ -737,7 +738,7 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
       // the f64 matrix pipe: 16 rows per block, columns split over KS blocks and their eight waves
       const int qb = (planes ? P * ((d / 32 + 511) / 512) : 0) + (rot.planes ? P * ((d / 8 + 511) / 512) : 0);
       dim3 gx((nrows + 15) / 16 * KS + qb);
-#define RX_GO(BF, NTT, RD) k_router_mfma<BF, NTT, RD><<<gx, 512, 0, st>>>(W->data, bias, wx, xbf, x, P, E, d, logits, out_x, nrows, planes, meta, planes_natural, KS, kpart, ktickets, rot)
+#define RX_GO(BF, NTT, RD) k_router_mfma<BF, NTT, RD><<<gx, 512, 0, st>>>(W->data, bias, wx, xbf, x, P, E, d, logits, out_x, nrows, planes, meta, planes_form, KS, kpart, ktickets, rot)
       const int nit = d / (8 * KS) / 16;  // ring steps a wave walks
       if (nit <= 3) {
         if (P <= 16) { if (bf) RX_GO(true, 1, 3); else RX_GO(false, 1, 3); }
@@ -750,7 +751,7 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
       MOE_LAUNCH_CHECK();
       return MOE_OK;
     }
-#define RMD_GO(BF, PM) k_router_mid<BF, PM><<<g, 256, 0, st>>>(W->data, bias, wx, xbf, x, P, E, d, logits, out_x, nrows, planes, meta, planes_natural, rot)
+#define RMD_GO(BF, PM) k_router_mid<BF, PM><<<g, 256, 0, st>>>(W->data, bias, wx, xbf, x, P, E, d, logits, out_x, nrows, planes, meta, planes_form, rot)
     if (P <= 8) { if (bf) RMD_GO(true, 8); else RMD_GO(false, 8); }
     else if (P <= 16) { if (bf) RMD_GO(true, 16); else RMD_GO(false, 16); }
     else { if (bf) RMD_GO(true, 24); else RMD_GO(false, 24); }  // P <= 24 (larger batches were split above)

@@ -312,6 +312,29 @@ def test_small_batch_gguf_gate_up_rows_dealt_over_a_wave(oracle, types, d, T):
     assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= TOL_INT_Q4K
 
 
+# Activations in three 8-bit digit planes: an element is rounded to 2^-24 of its group's largest, which is 2 .. 3 times their
+# root mean square, and up to 112 groups' sums are added in f32, in two projections one behind the other: 1e-6 of the largest output
+TOL_INT24 = 5e-6
+
+
+@pytest.mark.parametrize("T", [1, 4, 5, 9, 20, 32])
+@pytest.mark.parametrize("types,k,shared,d,mid", [((13, 8, 8), 3, True, 2560, 640), ((12, 8, 8), 10, True, 2560, 640), ((13, 7, 8), 6, True, 3072, 640),
+                                                  ((8, 8, 7), 7, True, 2048, 384), ((13, 8, 8), 15, True, 2048, 896), ((7, 8, 8), 1, False, 3584, 128),
+                                                  ((20, 7, 7), 5, False, 2560, 896), ((23, 8, 8), 2, True, 3072, 128)])
+def test_small_batch_gguf_down_rows_of_no_whole_super_blocks(oracle, types, k, shared, d, mid, T):
+    """Down rows of 2, 6, 10 and 14 units of 64 columns, one slot to fifteen, on activations of 24 bits a group: the error of f32
+    kernels, which is where such layers ran before."""
+    rng = np.random.default_rng(d + mid + 10 * T + k)
+    hl = HostLayer(rng, d, mid, 16, k, fmt="q4k", gg_types=types, shared=shared)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    x[0, 40:72] *= 1e-6  # (a group whose elements are of two sizes, and one that is small throughout)
+    x[T - 1] *= 1e4
+    yo, io, wo = oracle.moe_layer(hl.oracle_layer(), x)
+    y, ids, ws = run_layer(hl, x)
+    assert (ids[:, :k] == io[:, :k]).all()
+    assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= TOL_INT24
+
+
 @pytest.mark.parametrize("T", [1, 3])
 def test_gguf_gate_up_selects_among_more_than_512_experts(T):
     """The selection inside the gate/up launch and the router's own give the same ids, and the rows' sums do not depend on it."""
