@@ -737,6 +737,18 @@ static moe_rfix router_fix(const moe_ctx* c, const MoeLayer& L, const float* x, 
   return R;
 }
 
+// The selection of a small batch as a launch of its own: from the logits, or from the column shares that the router's launch left
+// (more than four tokens, where that launch splits the columns).
+static bool select_aside(const moe_ctx* c, const MoeLayer& L, int P, bool gu_topk) {
+  return !gu_topk && moe_router_split_supported(&L.router, P, c->cfg.topk);
+}
+static int select_small(moe_ctx* c, moe_rfix rf, int P, int parts, hipStream_t st) {
+  const moe_config& g = c->cfg;
+  if (!parts) return moe_launch_router_topk_small(c->logits, c->ids, c->ws, P, g.experts, g.topk, g.id_stride, &rf, st);
+  rf.tol = c->rtol;
+  return moe_launch_router_split_topk(c->kpart, parts, c->ids, c->ws, P, g.experts, g.topk, g.id_stride, rf, st);
+}
+
 // the router and the routed experts (and the shared expert where the kernels take it along as one more slot)
 static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, float* y, hipStream_t st) {
   const moe_config& g = c->cfg;
@@ -803,12 +815,12 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
   const moe_rfix rf = router_fix(c, L, x, P <= 4);
   if ((rc = stage(MOE_PROF_ROUTER, [&]() -> int {
          // (the selection runs in launches of its own here, so that it can be made certain: no top-k inside the logits launch)
+         int parts = 0;
          int e = moe_router_logits_small(&L.router, L.router_bias, L.has_shared ? &L.sh_sg : nullptr, x, P, c->logits,
                                          c->sh_logit, (use_int || use_int4k || use_intgg || use_intgg3) ? c->xplanes : nullptr, c->xmeta,
-                                         use_intgg3 ? MOE_PLANES_QVEC3 : use_int4k || use_intgg ? MOE_PLANES_QVEC : MOE_PLANES_QVEC4, st, c->kpart, c->ktickets, nullptr, P <= 4 && rf.W ? c->rtol : nullptr,
-                                         rf.tol_scale);
-         if (!e && !gu_topk)
-           e = moe_launch_router_topk_small(c->logits, c->ids, c->ws, P, g.experts, g.topk, g.id_stride, &rf, st);
+                                         use_intgg3 ? MOE_PLANES_QVEC3 : use_int4k || use_intgg ? MOE_PLANES_QVEC : MOE_PLANES_QVEC4, st, c->kpart, c->ktickets, nullptr, rf.W ? c->rtol : nullptr, rf.tol_scale,
+                                         select_aside(c, L, P, gu_topk) ? &parts : nullptr);
+         if (!e && !gu_topk) e = select_small(c, rf, P, parts, st);
          return e;
        })))
     return rc;
@@ -999,11 +1011,13 @@ static int forward_small_v2(moe_ctx* c, MoeLayer& L, const float* x, int P, floa
   const moe_rfix rf = router_fix(c, L, x, P <= 4);
   if ((rc = stage(MOE_PROF_ROUTER, [&]() -> int {
          // (the planes of rot_in(x, su) ride in the router launch's spare blocks)
+         int parts = 0;
          const moe_rot_planes rot{L.v2_su, c->v2_xplanes, c->v2_xmeta};
          int e = moe_router_logits_small(&L.router, L.router_bias, L.has_shared ? &L.sh_sg : nullptr, x, P, c->logits,
                                          c->sh_logit, sh ? c->xplanes : nullptr, c->xmeta, MOE_PLANES_QVEC4,
-                                         st, c->kpart, c->ktickets, &rot, P <= 4 && rf.W ? c->rtol : nullptr, rf.tol_scale);
-         if (!e && !gu_topk) e = moe_launch_router_topk_small(c->logits, c->ids, c->ws, P, g.experts, g.topk, g.id_stride, &rf, st);
+                                         st, c->kpart, c->ktickets, &rot, rf.W ? c->rtol : nullptr, rf.tol_scale,
+                                         select_aside(c, L, P, gu_topk) ? &parts : nullptr);
+         if (!e && !gu_topk) e = select_small(c, rf, P, parts, st);
          return e;
        })))
     return rc;

@@ -50,7 +50,9 @@ enum { MOE_PLANES_QVEC4, MOE_PLANES_QVEC, MOE_PLANES_QVEC3 };  // (qvec.h)
 int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x,
                             int P, float* logits, float* out_x, uint32_t* planes, float2* meta,
                             int planes_form, hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rot = nullptr,
-                            float* tol_out = nullptr, float tol_scale = 0.f);
+                            float* tol_out = nullptr, float tol_scale = 0.f, int* parts = nullptr);
+// (parts: where the launch can, it leaves the logits' column shares [*parts][P][E] in kpart for moe_launch_router_split_topk, and
+// tol_out; else *parts = 0)
 // scratch of the column-split router launch (5..32 tokens): fp64 partial tiles of up to 8 splits x 32 tokens
 // for at most MOE_ROUTER_KSPLIT_ROWS rows, and one ticket counter (resting at 0) per 16 rows
 constexpr int MOE_ROUTER_KSPLIT_ROWS = 1040;
@@ -131,6 +133,8 @@ struct moe_row_extras {
   float* out_x;      // [P] its logit
 };
 int moe_launch_row_extras(const float* x, int P, int d, const moe_row_extras& R, hipStream_t st);  // (reduce.hip)
+int moe_launch_router_split_topk(const double* gpart, int KS, int* ids, float* ws, int P, int E, int k, int id_stride, const moe_rfix& RF,
+                                 hipStream_t st);
 bool moe_router_split_supported(const moe_wview* W, int P, int k);
 size_t moe_router_split_scratch_bytes(int max_tokens, int experts, int d);
 int moe_router_batch_split(const moe_wview* W, const float* x, int P, int* ids, float* ws, int k,

@@ -503,34 +503,63 @@ void launch_seq(const void* W, bool bf, const float* bias, const float* x, int P
 // per lane (4 consecutive columns 4*(l/16)..+3 of its row / token) therefore feeds four MFMAs.
 // Every weight is read once, activations come from L2; loads run through a register ring of
 // RD 16-column steps.  Needs d % (128 * KS) == 0.  Blocks past the rows build the digit planes of x.
-// KS > 1 (needs gpart and tickets): the columns are split over KS blocks per row group as well, so that
+// KS > 1 (needs gpart): the columns are split over KS blocks per row group as well, so that
 // 16 rows x d columns, one block's work with KS = 1 and the whole time of the launch, become KS blocks on KS
-// CUs.  Each block leaves its fp64 partial tile in gpart and takes a ticket of its row group; the block that
+// CUs.  Each block leaves its fp64 partial tile in gpart.  Where the selection is a launch of its own, that one adds the KS shares
+// in share order (k_router_split_topk; no tickets).  With tickets (MOE_OPT_GU_TOPK_MAX_TOKENS above 4: the blocks of the gate/up launch
+// want logits) each block takes a ticket of its row group, and the block that
 // draws the last one adds the KS partial tiles in split order (fixed again) and writes the logits.  Partial
-// tiles go out and come back as device-scope accesses, the ticket counters rest at 0 between launches.
+// tiles go out and come back as device-scope accesses, the ticket counters rest at 0 between launches.  That hand-over is a
+// store's, a ticket's and a load's trip to memory one behind the other: the launch takes 2 us more, 20 tokens 14.3 for 12.2.
+// The shared expert's gate vector has a block per token, which leaves the selection's bound as well: as row 513 of 512 experts it made
+// 264 blocks, each a CU's work, for 256 CUs, and 20 tokens took 12.2 us for 7.4, eight 9.4 for 5.8.  The layer, us, with all of
+// this: 5 tokens q4cp 53.5 -> 48.8, 8 73.4 -> 67.7, 20 140.3 -> 133.8, rotated experts 11 89 -> 83.7; and a batch with a near tie, whose logits
+// the selecting launch redoes by waves now, 32 tokens 632 -> 243.
 template <bool BF16, int NTT, int RD>  // NTT = token tiles of 16 (1 or 2)
 __global__ void __launch_bounds__(512, 2) k_router_mfma(const void* __restrict__ W, const float* __restrict__ bias,
-                                                        const void* __restrict__ Wx, bool wx_bf16,
                                                         const float* __restrict__ x, int P, int E, int d,
-                                                        float* __restrict__ logits, float* __restrict__ out_x,
-                                                        int nrows, uint32_t* __restrict__ planes,
+                                                        float* __restrict__ logits, uint32_t* __restrict__ planes,
                                                         float2* __restrict__ meta, int planes_form, int KS,
-                                                        double* gpart, unsigned* tickets, moe_rot_planes rot) {
-  __shared__ double part[8][NTT][64][4];
+                                                        double* gpart, unsigned* tickets, moe_row_extras R, moe_rot_planes rot) {
+  __shared__ double part[8][NTT][4][64];
   __shared__ int s_last;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nrt = (nrows + 15) >> 4;
+  const int nrt = (E + 15) >> 4;
   if ((int)blockIdx.x >= nrt * KS) {
-    router_plane_blocks((int)blockIdx.x - nrt * KS, 512, tid, x, P, d, planes, meta, planes_form, rot);
+    const int nx = R.tol || R.wx ? P : 0, t = (int)blockIdx.x - nrt * KS;
+    if (t >= nx) {
+      router_plane_blocks(t - nx, 512, tid, x, P, d, planes, meta, planes_form, rot);
+      return;
+    }
+    // a block per token: |x| as the selection's bound, the shared expert's gate logit
+    double* const xp = &part[0][0][0][0];
+    float acc;
+    double gate;
+    row_extras_part(x, t, d, tid, 512, R, acc, gate);
+    acc = wave_sum(acc);
+    gate = wave_sum(gate);
+    if (lane == 0) {
+      xp[2 * wv] = (double)acc;
+      xp[2 * wv + 1] = gate;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      acc = 0.f;
+      gate = 0.0;
+#pragma unroll
+      for (int w = 0; w < 8; w++) {
+        acc += (float)xp[2 * w];
+        gate += xp[2 * w + 1];
+      }
+      row_extras_out(t, d, R, acc, gate);
+    }
     return;
   }
   const int rg = (int)blockIdx.x % nrt, ks = (int)blockIdx.x / nrt;  // row group, column split
   const int li = lane & 15, lg = lane >> 4;
   const int row = rg * 16 + li;
-  const bool rlive = row < nrows, extra = Wx != nullptr && row == E;
   // per-lane weight row (rows past the end read row 0 and are never stored); all loads unconditional
-  const bool wbf = extra ? wx_bf16 : BF16;
-  const uint8_t* wrow = extra ? (const uint8_t*)Wx : (const uint8_t*)W + (rlive ? (uint64_t)row : 0) * d * (BF16 ? 2 : 4);
+  const uint8_t* wrow = (const uint8_t*)W + (row < E ? (uint64_t)row : 0) * d * (BF16 ? 2 : 4);
   const float* xrow[NTT];
   float xm[NTT];
 #pragma unroll
@@ -545,9 +574,8 @@ __global__ void __launch_bounds__(512, 2) k_router_mfma(const void* __restrict__
   float4 xr[RD][NTT];
   auto fetch = [&](int j, int it) {
     const int c = k0 + 16 * (it < nit ? it : nit - 1);  // past the end: a repeat that is never used
-    // 16 bytes in either format (bf16: 8 bytes twice), so no branch surrounds the load
-    const uint8_t* p = wrow + (size_t)c * (wbf ? 2 : 4);
-    const gate_bf16x4 lo = *(const gate_bf16x4*)p, hi = *(const gate_bf16x4*)(p + (wbf ? 0 : 8));
+    const uint8_t* p = wrow + (size_t)c * (BF16 ? 2 : 4);
+    const gate_bf16x4 lo = *(const gate_bf16x4*)p, hi = *(const gate_bf16x4*)(p + (BF16 ? 0 : 8));
     wr[j] = make_uint4(lo.x, lo.y, hi.x, hi.y);
 #pragma unroll
     for (int tt = 0; tt < NTT; tt++) xr[j][tt] = *(const float4*)(xrow[tt] + c);
@@ -562,7 +590,7 @@ __global__ void __launch_bounds__(512, 2) k_router_mfma(const void* __restrict__
     for (int j = 0; j < RD; j++) {
       if (ib + j < nit) {  // block-uniform
         float w[4];
-        if (wbf) {
+        if (BF16) {
           w[0] = __uint_as_float(wr[j].x << 16); w[1] = __uint_as_float(wr[j].x & 0xffff0000u);
           w[2] = __uint_as_float(wr[j].y << 16); w[3] = __uint_as_float(wr[j].y & 0xffff0000u);
         } else {
@@ -588,31 +616,26 @@ __global__ void __launch_bounds__(512, 2) k_router_mfma(const void* __restrict__
 #pragma unroll
   for (int tt = 0; tt < NTT; tt++)
 #pragma unroll
-    for (int r = 0; r < 4; r++) part[wv][tt][lane][r] = acc[tt][r];
+    for (int r = 0; r < 4; r++) part[wv][tt][r][lane] = acc[tt][r];
   __syncthreads();
-  // D value r of lane l = [row 4r + l/16][token l%16]; one thread per (tile, lane, r) adds the eight partials
+  // D value r of lane l = [row 4r + l/16][token l%16]; thread i = (tile, row, token) adds the eight partials
   auto emit = [&](int i, double sum) {
-    const int tt = i >> 8, l = (i >> 2) & 63, r = i & 3;
-    const int orow = rg * 16 + 4 * r + (l >> 4), t = 16 * tt + (l & 15);
-    if (orow < nrows && t < P) {
-      float v = (float)sum;
-      if (orow == E) out_x[t] = v;
-      else {
-        if (bias) v += bias[orow];
-        logits[(size_t)t * E + orow] = v;
-      }
-    }
+    const int orow = rg * 16 + ((i >> 4) & 15), t = 16 * (i >> 8) + (i & 15);
+    if (orow < E && t < P) logits[(size_t)t * E + orow] = (float)sum + (bias ? bias[orow] : 0.f);
   };
   constexpr int NV = NTT * 256;
   for (int i = tid; i < NV; i += 512) {
-    const int tt = i >> 8, l = (i >> 2) & 63, r = i & 3;
-    double sum = part[0][tt][l][r];
+    const int tt = i >> 8, r = (i >> 6) & 3, l = i & 63;
+    double sum = part[0][tt][r][l];
 #pragma unroll
-    for (int w = 1; w < 8; w++) sum += part[w][tt][l][r];
+    for (int w = 1; w < 8; w++) sum += part[w][tt][r][l];
     if (KS == 1) emit(i, sum);
-    else __hip_atomic_store(&gpart[((size_t)ks * nrt + rg) * NV + i], sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else if (!tickets) {  // (the selecting launch adds the column shares)
+      const int orow = rg * 16 + ((i >> 4) & 15), t = 16 * tt + (i & 15);
+      if (orow < E && t < P) gpart[((size_t)ks * P + t) * E + orow] = sum;
+    } else __hip_atomic_store(&gpart[((size_t)ks * nrt + rg) * NV + i], sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  if (KS == 1) return;
+  if (KS == 1 || !tickets) return;
   // Hand-over of the partial tiles to the block that draws the row group's last ticket (possibly on another
   // XCD): the tiles are device-scope atomic stores, every storing thread waits until all of its stores have
   // been acknowledged (vmcnt = 0) before the barrier, thread 0 takes the device-scope ticket after the
@@ -677,8 +700,9 @@ int moe_router_logits_seq(const moe_wview* W, const float* bias, const float* x,
 int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x,
                             int P, float* logits, float* out_x, uint32_t* planes, float2* meta,
                             int planes_form, hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rotp,
-                            float* tol_out, float tol_scale) {
+                            float* tol_out, float tol_scale, int* parts) {
   const int E = (int)W->rows, d = (int)W->cols;
+  if (parts) *parts = 0;
   moe_rot_planes rot{nullptr, nullptr, nullptr};
   if (rotp) {  // hgn v2: the planes of rot_in(x, pre) in the same launch
     if (!rotp->pre || !rotp->planes || !rotp->meta || d % 128 || !moe_aligned(rotp->pre, 16) || !moe_aligned(x, 16)) return MOE_E_INVALID;
@@ -737,8 +761,15 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
     if (mfma_ok) {
       // the f64 matrix pipe: 16 rows per block, columns split over KS blocks and their eight waves
       const int qb = (planes ? P * ((d / 32 + 511) / 512) : 0) + (rot.planes ? P * ((d / 8 + 511) / 512) : 0);
-      dim3 gx((nrows + 15) / 16 * KS + qb);
-#define RX_GO(BF, NTT, RD) k_router_mfma<BF, NTT, RD><<<gx, 512, 0, st>>>(W->data, bias, wx, xbf, x, P, E, d, logits, out_x, nrows, planes, meta, planes_form, KS, kpart, ktickets, rot)
+      moe_row_extras ex{};
+      ex.wx = wx; ex.wx_bf16 = xbf; ex.out_x = out_x;
+      ex.tol = tol_out; ex.tol_scale = tol_scale;
+      dim3 gx((E + 15) / 16 * KS + (ex.wx || ex.tol ? P : 0) + qb);
+      if (parts && KS > 1) {
+        *parts = KS;
+        ktickets = nullptr;
+      }
+#define RX_GO(BF, NTT, RD) k_router_mfma<BF, NTT, RD><<<gx, 512, 0, st>>>(W->data, bias, x, P, E, d, logits, planes, meta, planes_form, KS, kpart, ktickets, ex, rot)
       const int nit = d / (8 * KS) / 16;  // ring steps a wave walks
       if (nit <= 3) {
         if (P <= 16) { if (bf) RX_GO(true, 1, 3); else RX_GO(false, 1, 3); }

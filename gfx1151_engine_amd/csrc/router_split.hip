@@ -144,7 +144,7 @@ __global__ void __launch_bounds__(512, 2) k_router_split(const void* __restrict_
   }
 }
 
-// The selecting block of a token: the column shares' sums in share order, + bias, softmax / top-k.
+// The selecting block of a token (also of 5 .. 32 tokens, behind k_router_mfma's shares): the column shares' sums in share order, + bias, softmax / top-k.
 // Its fp64 sums differ from the reference's sequential ones by at most tol; select_listed makes the ids certain.
 template <int NPL>
 __global__ void __launch_bounds__(256) k_router_split_topk(const double* __restrict__ gpart, int KS, int* __restrict__ ids,
@@ -228,6 +228,13 @@ int moe_router_batch_split(const moe_wview* W, const float* x, int P, int* ids, 
   else k_router_split<false><<<grid, 512, 0, st>>>(W->data, x, P, E, d, KS, nrg, ntg, gpart, R);
   MOE_LAUNCH_CHECK();
   if (after_rows) MOE_HIP(hipEventRecord(after_rows, st));
+  return moe_launch_router_split_topk(gpart, KS, ids, ws, P, E, k, id_stride, RF, st);
+}
+
+// (also behind k_router_mfma)
+int moe_launch_router_split_topk(const double* gpart, int KS, int* ids, float* ws, int P, int E, int k, int id_stride, const moe_rfix& RF,
+                                 hipStream_t st) {
+  if (KS < 1 || KS > MOE_ROUTER_SPLIT_KS || E > 1024 || !RF.W || !RF.tol) return MOE_E_INVALID;
   if (E <= 512) k_router_split_topk<8><<<P, 256, 0, st>>>(gpart, KS, ids, ws, P, E, k, id_stride, RF);
   else k_router_split_topk<16><<<P, 256, 0, st>>>(gpart, KS, ids, ws, P, E, k, id_stride, RF);
   MOE_LAUNCH_CHECK();

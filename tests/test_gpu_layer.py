@@ -335,6 +335,29 @@ def test_small_batch_gguf_down_rows_of_no_whole_super_blocks(oracle, types, k, s
     assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= TOL_INT24
 
 
+@pytest.mark.parametrize("T", [5, 16, 17, 25, 32])
+@pytest.mark.parametrize("E,d,router,shared", [(17, 1024, "f32", True), (32, 2048, "bf16", True), (513, 1024, "f32", False), (20, 768, "bf16", True),
+                                               (1000, 256, "f32", True), (16, 384, "f32", True)])
+def test_small_batch_router_in_column_shares(oracle, E, d, router, shared, T):
+    """5 .. 32 tokens: one and two tiles of tokens, row groups with rows left over, eight column shares, two and none; the shared expert's
+    gate logit and the selection's bound beside them.  One token's best logits are equal in pairs, another's are a tie in f32
+    only, so that the selection needs the bound."""
+    rng = np.random.default_rng(E + d + T)
+    hl = HostLayer(rng, d, 256, E, 6, router_dtype=router, shared=shared, scale_std=0.02)
+    if router == "f32":
+        hl.router[1] = hl.router[0]
+        hl.router[3] = hl.router[2]
+        hl.router[3, ::2] *= np.float32(1.0 + 2.0 ** -23)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    x[1] = 30 * hl.router[0].astype(np.float32) if router == "f32" else x[1]
+    x[2] = 30 * hl.router[2].astype(np.float32) if router == "f32" else x[2]
+    yo, io, wo = oracle.moe_layer(hl.oracle_layer(), x)
+    y, ids, ws = run_layer(hl, x)
+    assert (ids[:, :6] == io[:, :6]).all()
+    assert np.abs(ws[:, :6] - wo[:, :6]).max() <= 1e-6
+    assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= TOL_INT_Q4CP
+
+
 @pytest.mark.parametrize("T", [1, 3])
 def test_gguf_gate_up_selects_among_more_than_512_experts(T):
     """The selection inside the gate/up launch and the router's own give the same ids, and the rows' sums do not depend on it."""
