@@ -79,6 +79,17 @@ struct SW {
   const int8_t* pexp;
 };
 
+// (v & mask) | bits.  An instruction reads one scalar, and left to itself the compiler makes two instructions of this rather than keep
+// `bits` in a register: 64 of the 335 that a line of two Q4_K fragments took.  Layers, us: Q4_K 40 tokens 305.0 -> 300.7, 130 494 489,
+// 515 569.6 565.1, 1500 711.5 706.8, 2500 879 875; Q4_K / Q8_0 300 678.7 677.0, 2560 x 640 300 507.5 499.5.  (Not FUSED: down with 64 pairs, which
+// has no registers left.)
+template <bool FUSED>
+__device__ __forceinline__ uint32_t and_or(uint32_t v, uint32_t mask, uint32_t bits) {
+  if (!FUSED) return (v & mask) | bits;
+  uint32_t r;
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(mask), "v"(bits));
+  return r;
+}
 __device__ __forceinline__ half2v both(float f) { return half2v{(_Float16)f, (_Float16)f}; }
 
 template <int FMT>
@@ -160,7 +171,8 @@ struct Consts {
 // acc[f][mf] += line of fragment f x the line's activations.  f0: fragment 0's index into the constants; sw: this lane's two
 // scales of the line (scale planes); xb: the activations' line in LDS; xa: this lane's operand addresses of four steps
 // (Q8_0: eight)
-template <int FMT, int F, int MF, int XP, int TABC, bool SPLIT>
+// FUSED: and_or as one instruction
+template <int FMT, int F, int MF, int XP, int TABC, bool FUSED = true, bool SPLIT>
 __device__ __forceinline__ void line_mma(const Line<FMT, SPLIT> (&q)[F], const uint32_t (&sw)[F], const Consts& C, int f0,
                                          const uint8_t* xb, const uint32_t* xa, bool half, floatx4 (&acc)[F][MF]) {
   auto mma = [&](uint32_t xo, const H8 (&w)[F]) {
@@ -300,8 +312,8 @@ __device__ __forceinline__ void line_mma(const Line<FMT, SPLIT> (&q)[F], const u
               t2 = __builtin_amdgcn_perm(0x64646464u, lo, 0x04030401u);
               t3 = __builtin_amdgcn_perm(0x64646464u, hi, 0x04030401u);
             } else {
-              t0 = (w & 0x000f000fu) | 0x64006400u; t1 = (w & 0x00f000f0u) | 0x54005400u;
-              t2 = (w8 & 0x000f000fu) | 0x64006400u; t3 = (w8 & 0x00f000f0u) | 0x54005400u;
+              t0 = and_or<FUSED>(w, 0x000f000fu, 0x64006400u); t1 = and_or<FUSED>(w, 0x00f000f0u, 0x54005400u);
+              t2 = and_or<FUSED>(w8, 0x000f000fu, 0x64006400u); t3 = and_or<FUSED>(w8, 0x00f000f0u, 0x54005400u);
             }
             if (ONCE) {
               auto once = [&](uint32_t t, int i) {
@@ -381,7 +393,8 @@ __device__ __forceinline__ void half_mma(const uint4 (&c)[F], const Deq<F>& D, c
     } else {
       const uint32_t w = word(c[f], s), n = (b & 2 ? w >> 8 : w) & (i ? 0x00f000f0u : 0x000f000fu);
       if constexpr (FMT == F_DN) o.h[b] = h2(n) * D.as[f][i] + D.bs[f];
-      else o.h[b] = (h2(n | (i ? 0x54005400u : 0x64006400u)) - both(i ? 64.f : 1024.f)) * D.as[f][i] + D.bs[f];
+      else o.h[b] = (h2(and_or<true>(b & 2 ? w >> 8 : w, i ? 0x00f000f0u : 0x000f000fu, i ? 0x54005400u : 0x64006400u)) -
+                     both(i ? 64.f : 1024.f)) * D.as[f][i] + D.bs[f];
     }
   };
 #pragma unroll
@@ -926,7 +939,7 @@ __device__ __forceinline__ void dn_tile(uint8_t* smem, const SW& L, int e, const
           if (!ONE && l >= nline) break;
           const Ln q2[2] = {ln[0][i], ln[1][i]};
           const uint32_t sw[2] = {sq[0][i], sq[1][i]};
-          line_mma<FMT, 2, MF, XP, tab_copies(false, MFX)>(q2, sw, C, 0, smem + l * XLINE, xa, tail && l == nline - 1, acc);
+          line_mma<FMT, 2, MF, XP, tab_copies(false, MFX), false>(q2, sw, C, 0, smem + l * XLINE, xa, tail && l == nline - 1, acc);
         }
         load(0, pn, qn);
         load(1, pn, qn);
