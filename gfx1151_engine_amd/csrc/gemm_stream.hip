@@ -1065,12 +1065,15 @@ int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* 
     moe_dev_done(once, dev);
   }
   int nblk = UP ? (m + 16 * NW - 1) / (16 * NW) : (m + 32 * NW - 1) / (32 * NW), npass = 1;
-  // Down: a block walks several groups of rows behind one staging of the activations; the longest walk that leaves twelve
-  // blocks per CU (64 pairs: two.  Staging is most of a short walk there: 2048 tokens i4r 205 us, with six blocks 223, with
-  // twelve 300)
+  // Down: a block walks several groups of rows behind one staging of the activations; the longest walk that leaves ten blocks
+  // per CU, Q8_0 rows eight (64 pairs: two.  Staging is most of a short walk there: 2048 tokens i4r 205 us, with six blocks 223, with
+  // twelve 300).  With these instead of twelve throughout, us of the layer: Q5_K / Q8_0 48 tokens 467 -> 454, 100 630 618, 300 741 732,
+  // 800 818 803, 2560 x 640 60 399 382; q4cp 2560 x 640 60 233 229, 3072 x 768 300 477 475; Q4_K 300 539 537.  With eight for all, whose longer
+  // walks end raggedly where tiles are few: q4cp 48 294 288 but 36 255 258, 52 304 307, 300 474 480; Q4_K 48 332 327 but 40 299 304
+  constexpr int LEAVE = MFX == 4 ? 512 : FMT == F_Q80 ? 2048 : 2600;
   if (!UP)
     for (int c = 1; c <= nblk; c++)
-      if (nblk % c == 0 && (int64_t)max_tiles * (nblk / c) >= (MFX == 4 ? 512 : 3072)) npass = c;
+      if (nblk % c == 0 && (int64_t)max_tiles * (nblk / c) >= LEAVE) npass = c;
   nblk /= npass;
   const int per_xcd = (max_tiles + 7) / 8 + 1;
   k_moe_stream<FMT, UP, MFX, LN, NW><<<(unsigned)(per_xcd * nblk * 8), 64 * NW, lds, st>>>(
