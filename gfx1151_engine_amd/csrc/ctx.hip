@@ -802,12 +802,12 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
   // integer-dot kernels: the gate/up launch runs the softmax / top-k itself (one launch less on the
   // latency-bound path than a top-k kernel, no last-block ticket in the logits launch)
   // -- as long as its blocks run in one round: each repeats the selection, 3 .. 4 us, where a launch of its own costs 7.
-  // Two layers, us, in the gate/up launch and aside: look-up kernels 95.4 and 88.7 at 2 tokens; GGUF mixes 84.7 and 84.4 at 2,
+  // Two layers, us, in the gate/up launch and aside: look-up kernels 76.3 and 79.7 at 2 tokens, 101.5 and 98.3 at 3; GGUF mixes 84.7 and 84.4 at 2,
   // 122 and 119 at 3, 153 and 148 at 4; Q4_K 83.6 and 85.3 at 3, 113 and 108 at 4; q4cp 73.7 and 76.4 at 3, 100 and 97 at 4; both kinds
   // of GGUF layers with rows dealt over all lanes, whose rounds are shorter: mixes 104.5 and 106.4 at 3, 129.2 and 131.5 at 4, Q4_K 75.5
   // and 82.7, 99.3 and 100.8 (above four the router launch leaves no bounds for the selection)
   const bool gg_dealt = gu4k_dealt || use_intgg3 || (use_intgg && moe_decgg_passes(g.d) > 0);
-  const int topk_max = c->gu_topk_max >= 0 ? c->gu_topk_max : use_lut ? 1 : gg_dealt ? 4 : use_intgg ? 2 : use_f32a ? 4 : 3;
+  const int topk_max = c->gu_topk_max >= 0 ? c->gu_topk_max : use_lut ? 2 : gg_dealt ? 4 : use_intgg ? 2 : use_f32a ? 4 : 3;
   const bool gu_topk = (((use_int && !use_uq) || ((use_int4k || use_intgg) && !use_uq_gg) || use_intgg3 || use_lut || use_f32a) && P <= topk_max) &&
                        moe_dec_gu_topk_supported(g.experts, g.topk);
   // (up to 4 tokens the router launch leaves each token's bound for the selection; larger batches: the selecting

@@ -215,16 +215,20 @@ struct GuArgs2 {
 // ids and weights in every block; cheaper than a last-block ticket in the router launch plus a
 // dependent load of the ids here) and block (0, 0, token) writes ids / weights out for the down
 // kernel.  The shared expert's blocks skip it and have the CU to themselves meanwhile.
-// LUT = 1 (not with UQ): table look-up arithmetic (above) for any codebook; blocks of 16 rows and 256 threads; xf32 = the
+// LUT = 1 (not with UQ): table look-up arithmetic (above) for any codebook; blocks of 16 or 12 rows; xf32 = the
 // tokens' activations [P][d], dynamic LDS = the token's d activations and two tables (gate rows', up rows'), hid goes out as
 // f32 only.
 // LUT = 2: the same data flow with f32 arithmetic for codebooks a*n + b (no tables).
 constexpr int GU2_ROWS = 32;
 // (LUT = 1: four waves, 16 rows.  A block is tens of thousands of vector instructions there, and one token's 264 blocks of
-// eight waves leave the CUs that get a second one with twice the work: four layers 129 -> 119 us)
-constexpr int gu2_threads(int lut) { return lut == 1 ? 256 : 512; }
+// eight waves leave the CUs that get a second one with twice the work: four layers 129 -> 119 us.  With the selection inside, three
+// waves and 12 rows.  It is the selection that gains -- probably because a CU's waves go round its SIMDs: of blocks of four waves
+// the first ones, which select, would all share a SIMD.  us, 16 and 12 rows: 1 token (four layers) 3072 x 768 111.7 104.1, x 512 99.7 85.2, x 1024 127.5 113.5,
+// 2560 x 640 108.0 102.9; 2 tokens (two layers) 86.5 76.3 -- with the selection aside, where 16 rows are level or better (4 tokens
+// 117.9 120.3, 8 90.5 92.0), 79.7.  The last block's rows past mid are the last rows again and not stored.)
+constexpr int gu2_threads(int lut, int npl) { return lut == 1 ? (npl ? 192 : 256) : 512; }
 template <bool UQ, int NPL, int LUT>
-__global__ void __launch_bounds__(gu2_threads(LUT), 4) k_dec_gu(GuArgs2 A, const uint32_t* __restrict__ xplanes,
+__global__ void __launch_bounds__(gu2_threads(LUT, NPL), gu2_threads(LUT, NPL) < 256 ? 3 : 4) k_dec_gu(GuArgs2 A, const uint32_t* __restrict__ xplanes,
                                                 const float2* __restrict__ xmeta,
                                                 const int* __restrict__ ids, int id_stride, int kpt, int d,
                                                 int mid, uint32_t* __restrict__ hplanes,
@@ -233,7 +237,7 @@ __global__ void __launch_bounds__(gu2_threads(LUT), 4) k_dec_gu(GuArgs2 A, const
                                                 const int* __restrict__ tokidx, int n_experts,
                                                 const float* __restrict__ logits, int* __restrict__ ids_out,
                                                 float* __restrict__ ws_out, const float* __restrict__ xf32, moe_rfix RF) {
-  constexpr int NT = gu2_threads(LUT), ROWS = NT / 16;
+  constexpr int NT = gu2_threads(LUT, NPL), ROWS = NT / 16;
   extern __shared__ float lutmem[];
   __shared__ float gs[ROWS], us[ROWS];
   __shared__ uint32_t pk[QV4_GROUP_DW];
@@ -262,9 +266,9 @@ __global__ void __launch_bounds__(gu2_threads(LUT), 4) k_dec_gu(GuArgs2 A, const
   const float* const cbu = sh_blk ? A.shu.cb : A.gu.cb;
   const bool two_tabs = LUT == 1 && cbu != cbg;  // (block-uniform) the shared expert's up_proj is a tensor with a codebook of its own
   constexpr int XL = (96 * 8 + NT - 1) / NT;  // (d <= 3072)
-  static_assert(XL <= 3 && (LUT != 1 || NT == 256), "a thread stages at most three pieces of x and one of a table");
-  float4 x0, x1, x2;
-  float cg0 = 0.f, cu0 = 0.f;
+  static_assert(XL <= 4 && (LUT != 1 || (NT >= 128 && NT <= 256)), "a thread stages at most four pieces of x and two of a table");
+  float4 x0, x1, x2, x3;
+  float cg0 = 0.f, cu0 = 0.f, cg1 = 0.f, cu1 = 0.f;
   if (LUT) {
     const float4* xr = (const float4*)(xf32 + (size_t)blockIdx.z * d);
     auto ld = [&](int i) {
@@ -274,9 +278,14 @@ __global__ void __launch_bounds__(gu2_threads(LUT), 4) k_dec_gu(GuArgs2 A, const
     x0 = ld(0);
     x1 = ld(1);
     if (XL > 2) x2 = ld(2);
+    if (XL > 3) x3 = ld(3);
     if (LUT == 1) {
       cg0 = cbg[threadIdx.x >> 4];
       cu0 = cbu[threadIdx.x >> 4];
+      if (NT < 256) {
+        cg1 = cbg[(threadIdx.x + NT) >> 4 & 15];
+        cu1 = cbu[(threadIdx.x + NT) >> 4 & 15];
+      }
     }
   }
   bool shared;
@@ -310,7 +319,8 @@ __global__ void __launch_bounds__(gu2_threads(LUT), 4) k_dec_gu(GuArgs2 A, const
   const float* xs = lutmem;
   const uint64_t grow0 = shared ? 0 : (uint64_t)e * 2 * mid;
   const uint64_t urow0 = shared ? 0 : (uint64_t)e * 2 * mid + mid;
-  const int r0 = blockIdx.x * ROWS + 4 * wv;  // first of this wave's 4 gate rows
+  int r0 = blockIdx.x * ROWS + 4 * wv;  // first of this wave's 4 gate rows
+  if (NT < 256) r0 = r0 < mid ? r0 : mid - 4;
 
   // Branch-free loads: a lane whose group lies past the row reads group 0 instead and gets a zero
   // scale.  (Loads inside divergent branches make the compiler wait for each of them where it is
@@ -359,9 +369,14 @@ __global__ void __launch_bounds__(gu2_threads(LUT), 4) k_dec_gu(GuArgs2 A, const
     put(0, x0);
     put(1, x1);
     if (XL > 2) put(2, x2);
+    if (XL > 3) put(3, x3);
     if (LUT == 1) {
       lut_put(lut_g, threadIdx.x, cg0);
       if (two_tabs) lut_put(lut_u, threadIdx.x, cu0);
+      if (NT < 256 && threadIdx.x + NT < 256) {
+        lut_put(lut_g, threadIdx.x + NT, cg1);
+        if (two_tabs) lut_put(lut_u, threadIdx.x + NT, cu1);
+      }
     }
     moe_lds_barrier();  // (the weights stay in flight)
     __builtin_amdgcn_sched_barrier(0);
@@ -432,11 +447,11 @@ __global__ void __launch_bounds__(gu2_threads(LUT), 4) k_dec_gu(GuArgs2 A, const
   }
   // SwiGLU on the block's 32 rows = one group of the down projection's input; quantise it
   if (wv == 0) {
-    const int j = lane & (ROWS - 1);
+    const int j = (lane & 31) < ROWS ? lane & 31 : 0;
     const float g = gs[j], u = us[j];
     const float hv = g / (1.f + expf(-g)) * u;
     const size_t slot = UQ ? (size_t)(first + pi) : (size_t)tok * nslots + s;
-    if (hid_f32 && lane < ROWS) hid_f32[slot * mid + blockIdx.x * ROWS + j] = hv;
+    if (hid_f32 && lane < ROWS && (NT >= 256 || (int)blockIdx.x * ROWS + j < mid)) hid_f32[slot * mid + blockIdx.x * ROWS + j] = hv;
     if (LUT) return;  // (the down kernel of this arithmetic reads hid as f32)
     int p0, p1, p2, p3;
     float q, qsx;
@@ -902,8 +917,8 @@ int moe_launch_dec_gu_lut(const moe_wview* gu, const moe_wview* sh_gate, const m
   A.shg = decw(sh_gate);
   A.shu = decw(sh_up);
   if (d > 3072) return MOE_E_UNSUPPORTED;
-  const int nt = gu2_threads(affine ? 2 : 1);
-  dim3 grid(mid / (nt / 16), kpt + (sh_gate ? 1 : 0) + (logits ? 1 : 0), P);
+  const int nt = gu2_threads(affine ? 2 : 1, logits != nullptr);
+  dim3 grid((mid + nt / 16 - 1) / (nt / 16), kpt + (sh_gate ? 1 : 0) + (logits ? 1 : 0), P);
   const int lds = (affine ? 0 : 3 * LUT_BYTES) + d / 32 * XF_PITCH * 4;  // (a table's worth for the tables' alignment)
 #define DEC_GU_F32(NPL, MODE)                                                                                          \
   k_dec_gu<false, NPL, MODE><<<grid, nt, lds, st>>>(A, nullptr, nullptr, NPL ? nullptr : ids, id_stride, kpt, d, mid, nullptr, \

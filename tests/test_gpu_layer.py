@@ -88,6 +88,27 @@ def test_small_batch_table_codebooks(oracle, T, kind):
     m.close()
 
 
+@pytest.mark.parametrize("most", [0, 32])
+@pytest.mark.parametrize("T", [1, 2, 4])
+@pytest.mark.parametrize("d,mid,E", [(256, 32, 20), (512, 96, 20), (384, 160, 600), (768, 352, 20), (3072, 1024, 12)])
+def test_small_batch_table_gate_up_rows_of_a_block(oracle, d, mid, E, T, most):
+    """Gate/up blocks of twelve rows (the selection inside) and of sixteen (ids given): widths that are and are no multiples of
+    twelve, the last block with rows past mid, more than 512 experts."""
+    from gfx1151_engine_amd import capi
+    rng = np.random.default_rng(d + mid + T)
+    hl = HostLayer(rng, d, mid, E, 4, codebook=np.sort(rng.standard_normal(16)).astype(np.float32), scale_std=0.05,
+                   shared_codebooks=[np.sort(rng.standard_normal(16)).astype(np.float32) for _ in range(3)])
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    yo, io, wo = oracle.moe_layer(hl.oracle_layer(), x)
+    m, dev = hl.to_gpu(max_tokens=T)
+    m.set_option(capi.OPT_GU_TOPK_MAX_TOKENS, most)
+    y = m.forward(0, gpu(x)).cpu().numpy()
+    ids, _ = m.last_routing(T)
+    m.close()
+    assert (ids.cpu().numpy()[:, :4] == io[:, :4]).all()
+    assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= TOL_LUT
+
+
 @pytest.mark.parametrize("T", [1, 3, 6])
 @pytest.mark.parametrize("mid", [256, 512, 768, 1024])
 @pytest.mark.parametrize("types,k,shared", [((13, 8, 8), 1, True), ((13, 8, 8), 10, True), ((12, 8, 12), 5, True), ((13, 13, 8), 15, True),
