@@ -502,7 +502,7 @@ void launch_seq(const void* W, bool bf, const float* bias, const float* x, int P
 // v_mfma_f64_16x16x4_f64: lane l supplies A[row l%16][k l/16] and B[k l/16][token l%16]; a 16-byte load
 // per lane (4 consecutive columns 4*(l/16)..+3 of its row / token) therefore feeds four MFMAs.
 // Every weight is read once, activations come from L2; loads run through a register ring of
-// RD 16-column steps.  Needs d % (128 * KS) == 0.  Blocks past the rows build the digit planes of x.
+// RD 16-column steps.  Needs d % 128 == 0.  Blocks past the rows build the digit planes of x.
 // KS > 1 (needs gpart): the columns are split over KS blocks per row group as well, so that
 // 16 rows x d columns, one block's work with KS = 1 and the whole time of the launch, become KS blocks on KS
 // CUs.  Each block leaves its fp64 partial tile in gpart.  Where the selection is a launch of its own, that one adds the KS shares
@@ -568,8 +568,8 @@ __global__ void __launch_bounds__(512, 2) k_router_mfma(const void* __restrict__
     xrow[tt] = x + (size_t)(t < P ? t : 0) * d;
     xm[tt] = t < P ? 1.f : 0.f;
   }
-  const int kper = d / (8 * KS), k0 = (ks * 8 + wv) * kper + 4 * lg;  // this lane's first column
-  const int nit = kper / 16;
+  const int nst = d / 16, slot = ks * 8 + wv, s0 = slot * nst / (8 * KS);  // the wave's 16-column steps, one at least
+  const int k0 = 16 * s0 + 4 * lg, nit = (slot + 1) * nst / (8 * KS) - s0;  // this lane's first column
   uint4 wr[RD];
   float4 xr[RD][NTT];
   auto fetch = [&](int j, int it) {
@@ -715,13 +715,11 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
   // makes no difference to it: a lane loads its row in that row's own format.  With such a row, the router's
   // launches (logits, top-k) with k_router_mid and with this, us: 5 tokens 25 and 20, 11 tokens 32 and 22, 20 tokens 40 and
   // 25, 32 tokens 57 and 26.
+  // (as many shares as leave every wave a step of 16 columns, whether or not they are equal: 2560 columns in eight shares of two and three
+  // steps a wave instead of four of five: the launch 13.2 -> 7.5 us at 20 tokens; 2560 x 640 layers q4cp 5 tokens 49.0 -> 46.5, 20 118.2
+  // 112.4, table codebook 12 112.4 109.1; 2304 x 512 12 67.5 62.2)
   int KS = 1;
-  if (kpart && ktickets && P > 4 && E + 1 <= MOE_ROUTER_KSPLIT_ROWS)
-    for (int s = 8; s > 1; s >>= 1)
-      if (d % (128 * s) == 0) {
-        KS = s;
-        break;
-      }
+  if (kpart && ktickets && P > 4 && E + 1 <= MOE_ROUTER_KSPLIT_ROWS) KS = d < 256 ? 1 : d / 128 < 8 ? d / 128 : 8;
   const bool mfma_ok = (P > 24 || KS > 1) && d % 128 == 0;
   if (P > 24 && !mfma_ok) {
     // more than 24 tokens per block cost the kernel its second wave per SIMD (accumulators):
@@ -770,7 +768,7 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
         ktickets = nullptr;
       }
 #define RX_GO(BF, NTT, RD) k_router_mfma<BF, NTT, RD><<<gx, 512, 0, st>>>(W->data, bias, x, P, E, d, logits, planes, meta, planes_form, KS, kpart, ktickets, ex, rot)
-      const int nit = d / (8 * KS) / 16;  // ring steps a wave walks
+      const int nit = (d / 16 + 8 * KS - 1) / (8 * KS);  // ring steps a wave walks, at most
       if (nit <= 3) {
         if (P <= 16) { if (bf) RX_GO(true, 1, 3); else RX_GO(false, 1, 3); }
         else { if (bf) RX_GO(true, 2, 3); else RX_GO(false, 2, 3); }

@@ -358,9 +358,9 @@ def test_small_batch_gguf_down_rows_of_no_whole_super_blocks(oracle, types, k, s
 
 @pytest.mark.parametrize("T", [5, 16, 17, 25, 32])
 @pytest.mark.parametrize("E,d,router,shared", [(17, 1024, "f32", True), (32, 2048, "bf16", True), (513, 1024, "f32", False), (20, 768, "bf16", True),
-                                               (1000, 256, "f32", True), (16, 384, "f32", True)])
+                                               (1000, 256, "f32", True), (16, 384, "f32", True), (40, 640, "f32", True), (33, 2304, "bf16", True), (18, 128, "f32", False)])
 def test_small_batch_router_in_column_shares(oracle, E, d, router, shared, T):
-    """5 .. 32 tokens: one and two tiles of tokens, row groups with rows left over, eight column shares, two and none; the shared expert's
+    """5 .. 32 tokens: one and two tiles of tokens, row groups with rows left over, one to eight column shares, equal and not; the shared expert's
     gate logit and the selection's bound beside them.  One token's best logits are equal in pairs, another's are a tie in f32
     only, so that the selection needs the bound."""
     rng = np.random.default_rng(E + d + T)
