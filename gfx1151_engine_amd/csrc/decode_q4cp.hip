@@ -227,7 +227,11 @@ constexpr int GU2_ROWS = 32;
 // 2560 x 640 108.0 102.9; 2 tokens (two layers) 86.5 76.3 -- with the selection aside, where 16 rows are level or better (4 tokens
 // 117.9 120.3, 8 90.5 92.0), 79.7.  The last block's rows past mid are the last rows again and not stored.)
 constexpr int gu2_threads(int lut, int npl) { return lut == 1 ? (npl ? 192 : 256) : 512; }
-template <bool UQ, int NPL, int LUT>
+// TL: passes over the groups behind the first 64 of a row, of which a pass takes those of two rows (4 passes: up to 32 groups) or of four
+// (2 passes: up to 16), 0 where there are none.  us, four passes throughout and these, weights from HBM: table codebook
+// 2560 x 640 1 token 111 106, 3 91 87, 8 86 81, 20 169 158; 2048 x 768 8 90 78; q4cp 2048 x 768 1 81 74, 3 69 65, 8 59 56; q4cp 2560 x 640
+// 8 60 59, 20 112 110, and 1 token level at 79: an int kernel with the selection inside keeps four there.
+template <bool UQ, int NPL, int LUT, int TL = 4>
 __global__ void __launch_bounds__(gu2_threads(LUT, NPL), gu2_threads(LUT, NPL) < 256 ? 3 : 4) k_dec_gu(GuArgs2 A, const uint32_t* __restrict__ xplanes,
                                                 const float2* __restrict__ xmeta,
                                                 const int* __restrict__ ids, int id_stride, int kpt, int d,
@@ -325,8 +329,10 @@ __global__ void __launch_bounds__(gu2_threads(LUT, NPL), gu2_threads(LUT, NPL) <
   // Branch-free loads: a lane whose group lies past the row reads group 0 instead and gets a zero
   // scale.  (Loads inside divergent branches make the compiler wait for each of them where it is
   // issued; in straight-line code all of a wave's loads are in flight together.)
-  const bool vA = lane < G, vB = 64 + (lane & 31) < G;
-  const int gA = vA ? lane : 0, gB = vB ? 64 + (lane & 31) : 0;
+  constexpr int TLANES = TL == 2 ? 16 : 32, TROWS = TL == 2 ? 4 : 2;  // lanes of a row's tail, rows of a pass
+  const int tsub = lane / TLANES;            // which of the pass's rows
+  const bool vA = lane < G, vB = TL && 64 + (lane & (TLANES - 1)) < G;
+  const int gA = vA ? lane : 0, gB = vB ? 64 + (lane & (TLANES - 1)) : 0;
   const float mA = vA ? 1.f : 0.f, mB = vB ? 1.f : 0.f;
   const size_t rb = (size_t)d / 2;
   // the activation planes and codebook constants are requested first: loads return in order, so
@@ -338,25 +344,28 @@ __global__ void __launch_bounds__(gu2_threads(LUT, NPL), gu2_threads(LUT, NPL) <
     const uint32_t* xp = raw ? A.xplanes_rot : xplanes;
     const float2* xm = raw ? A.xmeta_rot : xmeta;
     load_xg(xa, xp, xm, xbase + gA);
-    load_xg(xb, xp, xm, xbase + gB);
+    if (TL) load_xg(xb, xp, xm, xbase + gB);
   }
   const float ga = Wg.cb[1] - Wg.cb[0], gb = fmaf(8.f, ga, Wg.cb[0]), ua = Wu.cb[1] - Wu.cb[0], ub = fmaf(8.f, ua, Wu.cb[0]);
   // pairs 0,1: gate rows (r0+2p, r0+2p+1); pairs 2,3: the up rows
-  uint4 ca[4], cb[4], ct[4];
-  __half sa[4], sb[4], st[4];
+  uint4 ca[4], cb[4], ct[TL ? TL : 1];
+  __half sa[4], sb[4], st[TL ? TL : 1];
 #pragma unroll
   for (int p = 0; p < 4; p++) {
     const DecW W = p >= 2 ? Wu : Wg;
     const uint64_t row = (p >= 2 ? urow0 : grow0) + r0 + 2 * (p & 1);
     const uint8_t* c0 = W.codes + row * rb;
     const uint8_t* s0 = W.scales + row * W.ss;
-    const uint64_t trow = lane < 32 ? 0 : 1;
     ca[p] = *(const uint4*)(c0 + (size_t)gA * 16);
     cb[p] = *(const uint4*)(c0 + rb + (size_t)gA * 16);
     sa[p] = *(const __half*)(s0 + (gA >> W.gsh) * 2);
     sb[p] = *(const __half*)(s0 + W.ss + (gA >> W.gsh) * 2);
-    ct[p] = *(const uint4*)(c0 + trow * rb + (size_t)gB * 16);
-    st[p] = *(const __half*)(s0 + trow * W.ss + (gB >> W.gsh) * 2);
+    if (TL == 4 || (TL == 2 && (p & 1))) {  // (two rows' tails, or those of four: the pair before this one and this)
+      const int t = TL == 4 ? p : p >> 1;
+      const uint8_t *const ct0 = TL == 4 ? c0 : c0 - 2 * rb, *const st0 = TL == 4 ? s0 : s0 - 2 * W.ss;
+      ct[t] = *(const uint4*)(ct0 + (uint64_t)tsub * rb + (size_t)gB * 16);
+      st[t] = *(const __half*)(st0 + (uint64_t)tsub * W.ss + (gB >> W.gsh) * 2);
+    }
   }
   __builtin_amdgcn_sched_barrier(0);  // every load above is issued before the first dot product
   if (LUT) {
@@ -403,27 +412,31 @@ __global__ void __launch_bounds__(gu2_threads(LUT, NPL), gu2_threads(LUT, NPL) <
       acc[2 * p] = __half2float(sa[p]) * mA * f32_dot<LUT>(ca[p], xf, lt, a, b0, sx);
       acc[2 * p + 1] = __half2float(sb[p]) * mA * f32_dot<LUT>(cb[p], xf, lt, a, b0, sx);
     }
-    load_xf(xf, xs + (size_t)gB * XF_PITCH);
+    if (TL) load_xf(xf, xs + (size_t)gB * XF_PITCH);
     sx = LUT == 2 ? xf_sum(xf) : 0.f;
 #pragma unroll
-    for (int p = 0; p < 4; p++) {
-      const float vt = __half2float(st[p]) * mB * f32_dot<LUT>(ct[p], xf, p >= 2 ? lutu : lutg, p >= 2 ? ua : ga, p >= 2 ? u0 : g0, sx);
-      if (lane < 32) acc[2 * p] += vt;
-      else acc[2 * p + 1] += vt;
+    for (int t = 0; t < TL; t++) {
+      const bool up = 2 * t >= TL;
+      const float vt = __half2float(st[t]) * mB * f32_dot<LUT>(ct[t], xf, up ? lutu : lutg, up ? ua : ga, up ? u0 : g0, sx);
+#pragma unroll
+      for (int i = 0; i < TROWS; i++)
+        if (tsub == i) acc[TROWS * t + i] += vt;
     }
   } else {
 #pragma unroll
   for (int p = 0; p < 4; p++) {
     const float a = p >= 2 ? ua : ga, b = p >= 2 ? ub : gb;
     // (a multiplication, not a select: a select lets the compiler move the load back under a branch)
-    const float fa = __half2float(sa[p]) * mA, fb = __half2float(sb[p]) * mA, ft = __half2float(st[p]) * mB;
-    float v0 = fa * chunk_dot(ca[p], xa, a, b);
-    float v1 = fb * chunk_dot(cb[p], xa, a, b);
-    const float vt = ft * chunk_dot(ct[p], xb, a, b);
-    if (lane < 32) v0 += vt;
-    else v1 += vt;
-    acc[2 * p] = v0;
-    acc[2 * p + 1] = v1;
+    const float fa = __half2float(sa[p]) * mA, fb = __half2float(sb[p]) * mA;
+    acc[2 * p] = fa * chunk_dot(ca[p], xa, a, b);
+    acc[2 * p + 1] = fb * chunk_dot(cb[p], xa, a, b);
+    if (TL == 4 || (TL == 2 && (p & 1))) {
+      const int t = TL == 4 ? p : p >> 1;
+      const float vt = __half2float(st[t]) * mB * chunk_dot(ct[t], xb, a, b);
+#pragma unroll
+      for (int i = 0; i < TROWS; i++)
+        if (tsub == i) acc[TROWS * t + i] += vt;
+    }
     __builtin_amdgcn_sched_barrier(0);  // row pair p is finished before the wait for pair p + 1
   }
   }
@@ -850,6 +863,13 @@ int moe_launch_qvec(const float* x, uint64_t x_stride, int P, int K, uint32_t* p
   return MOE_OK;
 }
 
+// (TL of k_dec_gu by the row's groups)
+#define DEC_GU_TAILS(GO)            \
+  do {                              \
+    if (d <= 64 * 32) GO(0);        \
+    else if (d <= 80 * 32) GO(2);   \
+    else GO(4);                     \
+  } while (0)
 int moe_launch_dec_gu(const moe_wview* gu, const moe_wview* sh_gate, const moe_wview* sh_up,
                       const uint32_t* xplanes, const float2* xmeta, const int* ids, int id_stride, int kpt,
                       int P, int d, int mid, uint32_t* hplanes, float2* hmeta, float* hid_f32,
@@ -866,8 +886,11 @@ int moe_launch_dec_gu(const moe_wview* gu, const moe_wview* sh_gate, const moe_w
   }
   if (!A.gu.cb) return MOE_E_STATE;
   dim3 grid(mid / GU2_ROWS, kpt + (sh_gate ? 1 : 0), P);
-  k_dec_gu<false, 0, 0><<<grid, 512, 0, st>>>(A, xplanes, xmeta, ids, id_stride, kpt, d, mid, hplanes, hmeta, hid_f32,
-                                                  nullptr, nullptr, nullptr, 0, nullptr, nullptr, nullptr, nullptr, moe_rfix{});
+#define DEC_GU(TL)                                                                                                                   \
+  k_dec_gu<false, 0, 0, TL><<<grid, 512, 0, st>>>(A, xplanes, xmeta, ids, id_stride, kpt, d, mid, hplanes, hmeta, hid_f32, nullptr, nullptr, \
+                                                  nullptr, 0, nullptr, nullptr, nullptr, nullptr, moe_rfix{})
+  DEC_GU_TAILS(DEC_GU);
+#undef DEC_GU
   MOE_LAUNCH_CHECK();
   return MOE_OK;
 }
@@ -893,9 +916,12 @@ int moe_launch_dec_gu_topk(const moe_wview* gu, const moe_wview* sh_gate, const 
   }
   if (!A.gu.cb) return MOE_E_STATE;
   dim3 grid(mid / GU2_ROWS, kpt + (sh_gate ? 1 : 0) + 1, P);  // + the row of the exact top-k block
-  if (n_experts <= 512)
-    k_dec_gu<false, 8, 0><<<grid, 512, 0, st>>>(A, xplanes, xmeta, nullptr, id_stride, kpt, d, mid, hplanes, hmeta,
-                                                    hid_f32, nullptr, nullptr, nullptr, n_experts, logits, ids, ws, nullptr, RFV);
+#define DEC_GU(TL)                                                                                                                      \
+  k_dec_gu<false, 8, 0, TL><<<grid, 512, 0, st>>>(A, xplanes, xmeta, nullptr, id_stride, kpt, d, mid, hplanes, hmeta, hid_f32, nullptr, nullptr, \
+                                                  nullptr, n_experts, logits, ids, ws, nullptr, RFV)
+  if (n_experts <= 512 && d <= 64 * 32) DEC_GU(0);
+  else if (n_experts <= 512) DEC_GU(4);
+#undef DEC_GU
   else
     k_dec_gu<false, 16, 0><<<grid, 512, 0, st>>>(A, xplanes, xmeta, nullptr, id_stride, kpt, d, mid, hplanes, hmeta,
                                                      hid_f32, nullptr, nullptr, nullptr, n_experts, logits, ids, ws, nullptr, RFV);
@@ -920,15 +946,19 @@ int moe_launch_dec_gu_lut(const moe_wview* gu, const moe_wview* sh_gate, const m
   const int nt = gu2_threads(affine ? 2 : 1, logits != nullptr);
   dim3 grid((mid + nt / 16 - 1) / (nt / 16), kpt + (sh_gate ? 1 : 0) + (logits ? 1 : 0), P);
   const int lds = (affine ? 0 : 3 * LUT_BYTES) + d / 32 * XF_PITCH * 4;  // (a table's worth for the tables' alignment)
-#define DEC_GU_F32(NPL, MODE)                                                                                          \
-  k_dec_gu<false, NPL, MODE><<<grid, nt, lds, st>>>(A, nullptr, nullptr, NPL ? nullptr : ids, id_stride, kpt, d, mid, nullptr, \
+#define DEC_GU_F32(NPL, MODE, ...)                                                                                     \
+  k_dec_gu<false, NPL, MODE, ##__VA_ARGS__><<<grid, nt, lds, st>>>(A, nullptr, nullptr, NPL ? nullptr : ids, id_stride, kpt, d, mid, nullptr, \
                                                      nullptr, hid_f32, nullptr, nullptr, nullptr, n_experts, logits, ids, ws, x, RFV)
   if (!logits) {
+#define DEC_GU(TL) DEC_GU_F32(0, 1, TL)
     if (affine) DEC_GU_F32(0, 2);
-    else DEC_GU_F32(0, 1);
+    else DEC_GU_TAILS(DEC_GU);
+#undef DEC_GU
   } else if (n_experts <= 512) {
+#define DEC_GU(TL) DEC_GU_F32(8, 1, TL)
     if (affine) DEC_GU_F32(8, 2);
-    else DEC_GU_F32(8, 1);
+    else DEC_GU_TAILS(DEC_GU);
+#undef DEC_GU
   } else {
     if (affine) DEC_GU_F32(16, 2);
     else DEC_GU_F32(16, 1);

@@ -88,6 +88,21 @@ def test_small_batch_table_codebooks(oracle, T, kind):
     m.close()
 
 
+@pytest.mark.parametrize("T", [1, 3, 6])
+@pytest.mark.parametrize("d", [2016, 2048, 2080, 2304, 2560, 2592, 3072])
+@pytest.mark.parametrize("kind", ["q4cp", "table"])
+def test_small_batch_gate_up_rows_of_64_groups_and_more(oracle, kind, d, T):
+    """Gate/up rows of 63 to 96 groups: none behind the first 64, up to 16 (four rows' to a pass) and more (two rows')."""
+    rng = np.random.default_rng(d + T)
+    cb = np.sort(rng.standard_normal(16)).astype(np.float32) if kind == "table" else None
+    hl = HostLayer(rng, d, 64, 12, 4, codebook=cb, scale_std=0.05)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    yo, io, wo = oracle.moe_layer(hl.oracle_layer(), x)
+    y, ids, ws = run_layer(hl, x)
+    assert (ids[:, :4] == io[:, :4]).all()
+    assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= (TOL_LUT if kind == "table" else TOL_INT_Q4CP)
+
+
 @pytest.mark.parametrize("most", [0, 32])
 @pytest.mark.parametrize("T", [1, 2, 4])
 @pytest.mark.parametrize("d,mid,E", [(256, 32, 20), (512, 96, 20), (384, 160, 600), (768, 352, 20), (3072, 1024, 12)])
