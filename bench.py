@@ -34,7 +34,7 @@ CPU_BUDGET_S = 12.0            # the cpu_baseline leg stops starting new work af
 PMC_TRAFFIC = {("prefill", "q4cp", 16384): ("prefill_q4cp_T16384_hbm_traffic.txt", "k_moe_gemm_q4cp<true", "max"),
                ("decode", "q4cp", 1): ("decode_q4cp_T1_hbm_traffic.txt", "k_dec_gu", "max"),
                ("verify", "q4cp", 20): ("verify_q4cp_T20_hbm_traffic.txt", "k_dec_gu", "max"),
-               ("decode", "q4k", 1): ("decode_q4k_T1_hbm_traffic.txt", "k_dec4k_gu", "max"),
+               ("decode", "q4k", 1): ("decode_q4k_T1_hbm_traffic.txt", "k_decgg_gu", "max"),
                ("prefill", "q4k", 8192): ("prefill_q4k_T8192_hbm_traffic.txt", "k_moe_gemm_q4cp<true", "max")}
 
 
