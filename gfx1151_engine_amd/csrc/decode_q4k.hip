@@ -738,8 +738,8 @@ __global__ void __launch_bounds__(512, 4) k_decgg_gu(GuGgArgs A, const uint32_t*
     const float hv = g / (1.f + expf(-g)) * u;
     float m = dpp_max_row(fabsf(hv));
     m = rows_half_max(m);
-    const float inv = m > 0.f ? qv_xmax<N>() / m : 0.f;
-    float q = m * (1.f / qv_xmax<N>());
+    float inv, q;
+    qv_factor<N>(m, inv, q);
     if (N == 3) q += rows_half_add(dpp_add_row(hv * 0.f));  // (NaN where a row is not finite)
     const int X = (int)rintf(hv * inv);
     int pd[N];

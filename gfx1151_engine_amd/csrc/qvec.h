@@ -66,6 +66,17 @@ __device__ __forceinline__ void qv_digits_n(int X, int (&p)[N]) {
 }
 template <int N>
 constexpr float qv_xmax() { return N == 3 ? QV3_XMAX : QV_XMAX; }
+// A group's factor and q, from its largest magnitude.  Three digits: a largest one below 2^-104 (5e-32, hid of x near 1e-16) would make
+// the factor infinite; the group keeps 2^126 and its elements fewer than 24 bits.
+template <int N>
+__device__ __forceinline__ void qv_factor(float m, float& inv, float& q) {
+  inv = m > 0.f ? qv_xmax<N>() / m : 0.f;
+  q = m * (1.f / qv_xmax<N>());
+  if (N == 3 && m < 0x1p-104f) {
+    inv = 0x1p126f;
+    q = 0x1p-126f;
+  }
+}
 
 // One thread quantises group g of token t into the qvec form (N = 2) or qvec3 (N = 3).
 template <int N>
@@ -81,8 +92,8 @@ __device__ __forceinline__ void qvec_group_from_f32(const float* __restrict__ x,
     v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
     m = fmaxf(m, fmaxf(fmaxf(fabsf(f.x), fabsf(f.y)), fmaxf(fabsf(f.z), fabsf(f.w))));
   }
-  const float inv = m > 0.f ? qv_xmax<N>() / m : 0.f;
-  float q = m * (1.f / qv_xmax<N>());
+  float inv, q;
+  qv_factor<N>(m, inv, q);
   if (N == 3) {
     float z = 0.f;  // (0, or NaN)
 #pragma unroll

@@ -371,6 +371,21 @@ def test_small_batch_gguf_down_rows_of_no_whole_super_blocks(oracle, types, k, s
     assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= TOL_INT24
 
 
+@pytest.mark.parametrize("T", [1, 3])
+@pytest.mark.parametrize("scale", [1e-17, 1e-18, 3e-19])
+def test_small_batch_gguf_hid_too_small_for_a_24_bit_factor(oracle, scale, T):
+    """hid above and below 2^-104 a group, whose factor would be infinite.  The smallest here keep 15 bits, and q times a block's scale is a
+    multiple of 2^-149 of 2^-136 or more: 2e-4 together."""
+    rng = np.random.default_rng(T)
+    hl = HostLayer(rng, 2560, 640, 16, 4, fmt="q4k", gg_types=(13, 8, 8))
+    x = rng.standard_normal((T, 2560), dtype=np.float32) * np.float32(scale)
+    yo, io, wo = oracle.moe_layer(hl.oracle_layer(), x)
+    assert np.abs(yo).max() > 1e-33
+    y, ids, ws = run_layer(hl, x)
+    assert (ids[:, :4] == io[:, :4]).all()
+    assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= 2e-4
+
+
 @pytest.mark.parametrize("T", [5, 16, 17, 25, 32])
 @pytest.mark.parametrize("E,d,router,shared", [(17, 1024, "f32", True), (32, 2048, "bf16", True), (513, 1024, "f32", False), (20, 768, "bf16", True),
                                                (1000, 256, "f32", True), (16, 384, "f32", True), (40, 640, "f32", True), (33, 2304, "bf16", True), (18, 128, "f32", False)])
