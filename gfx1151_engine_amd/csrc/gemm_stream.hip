@@ -81,8 +81,8 @@ struct SW {
 
 // (v & mask) | bits.  An instruction reads one scalar, and left to itself the compiler makes two instructions of this rather than keep
 // `bits` in a register: 64 of the 335 that a line of two Q4_K fragments took.  Layers, us: Q4_K 40 tokens 305.0 -> 300.7, 130 494 489,
-// 515 569.6 565.1, 1500 711.5 706.8, 2500 879 875; Q4_K / Q8_0 300 678.7 677.0, 2560 x 640 300 507.5 499.5.  (Not FUSED: down with 64 pairs, which
-// has no registers left.)
+// 515 569.6 565.1, 1500 711.5 706.8, 2500 879 875; Q4_K / Q8_0 300 678.7 677.0.  (Not FUSED: down with 64 pairs, which has no
+// registers left.)
 template <bool FUSED>
 __device__ __forceinline__ uint32_t and_or(uint32_t v, uint32_t mask, uint32_t bits) {
   if (!FUSED) return (v & mask) | bits;
@@ -245,12 +245,14 @@ __device__ __forceinline__ void line_mma(const Line<FMT, SPLIT> (&q)[F], const u
           const half2v s2 = h2(__builtin_amdgcn_perm(0x64646464u, sc, C.selb)) - k1024;
           const half2v m2 = h2(__builtin_amdgcn_perm(0x64646464u, mn, C.selb)) - k1024;
           if (ONCE) {
-            // d * sc and dmin * m are exact in f32, and so to 2^-14 of a step is what the codes' offsets (below) add
+            // (codes are read as denormals, below: n 2^-24, Q4_K's high ones n 2^-20.  d * sc, dmin * m and n times the slope are exact in
+            // f32, so that the addition alone rounds.  With codes as 1024 + n and 1024 times the slope in the constant 0.8 .. 1.6 % of the
+            // weights were not the nearest f16, and 2560 x 640 of Q5_K / Q8_0 took 1100 us at 3000 tokens, now 1072; level below 1000)
             const half2v dd = h2(hd.x);
-            ka[f][0] = (float)s2.x * (float)dd.x;
-            ka[f][1] = (float)s2.y * (float)dd.x;
-            kb[f][0] = -fmaf(1024.f, ka[f][0], (float)m2.x * (float)dd.y);
-            kb[f][1] = -fmaf(q5(FMT) ? 1024.f : 64.f, ka[f][1], (float)m2.y * (float)dd.y);
+            ka[f][0] = (float)s2.x * ((float)dd.x * 0x1p24f);
+            ka[f][1] = (float)s2.y * ((float)dd.x * (q5(FMT) ? 0x1p24f : 0x1p20f));
+            kb[f][0] = -((float)m2.x * (float)dd.y);
+            kb[f][1] = -((float)m2.y * (float)dd.y);
           } else {  // d * sc and dmin * m as packed f16 products of exact integers
             const half2v dd = h2(__builtin_amdgcn_perm(hd.x, hd.x, 0x01000100u));
             const half2v dm = h2(__builtin_amdgcn_perm(hd.x, hd.x, 0x03020302u) ^ 0x80008000u);
@@ -295,22 +297,26 @@ __device__ __forceinline__ void line_mma(const Line<FMT, SPLIT> (&q)[F], const u
             a[f].h[1] = h2(w & 0x00f000f0u) * as[f][1] + bs[f][0];
             a[f].h[2] = h2(w8 & 0x000f000fu) * as[f][0] + bs[f][0];
             a[f].h[3] = h2(w8 & 0x00f000f0u) * as[f][1] + bs[f][0];
-          } else {  // 0x6400 | n is the f16 1024 + n, 0x5400 | n << 4 is 64 + n
+          } else {  // 0x6400 | n is the f16 1024 + n, 0x5400 | n << 4 is 64 + n; ONCE: n by itself is the denormal n 2^-24
             constexpr float HI = q5(FMT) ? 1024.f : 64.f;
             uint32_t t0, t1, t2, t3;
             if (q5(FMT)) {
               // fifth bits: bit 2 jj (low nibbles) and 2 jj + 1 (high) of the qh byte, jj = g / 2 + 2 E_, rotated to bit 4 of the
               // codes' bytes; two bytes are a pair of 1024 + n: 19 operations for eight weights where bits put into the four pairs
               // of the other formats' form took 22.  Q5_K / Q8_0 layers, us: 40 tokens 422 -> 415, 130 693 -> 680, 300 754 -> 742, 1400
-              // 953 -> 941; 2560 x 640 300 559 -> 546, 3000 1134 -> 1112
+              // 953 -> 941
               const uint4 qq = fifth[f];
               const uint32_t qw = s == 0 ? qq.x : s == 1 ? qq.y : s == 2 ? qq.z : qq.w;
               const uint32_t lo = (w & 0x0f0f0f0fu) | (__builtin_amdgcn_alignbit(qw, qw, (uint32_t)((C.g & 2) + 4 * E_ + 28) & 31u) & 0x10101010u);
               const uint32_t hi = ((w >> 4) & 0x0f0f0f0fu) | (__builtin_amdgcn_alignbit(qw, qw, (uint32_t)((C.g & 2) + 4 * E_ + 29) & 31u) & 0x10101010u);
-              t0 = __builtin_amdgcn_perm(0x64646464u, lo, 0x04020400u);
-              t1 = __builtin_amdgcn_perm(0x64646464u, hi, 0x04020400u);
-              t2 = __builtin_amdgcn_perm(0x64646464u, lo, 0x04030401u);
-              t3 = __builtin_amdgcn_perm(0x64646464u, hi, 0x04030401u);
+              // (selector 0x0c is a byte of zeros)
+              t0 = __builtin_amdgcn_perm(0x64646464u, lo, ONCE ? 0x0c020c00u : 0x04020400u);
+              t1 = __builtin_amdgcn_perm(0x64646464u, hi, ONCE ? 0x0c020c00u : 0x04020400u);
+              t2 = __builtin_amdgcn_perm(0x64646464u, lo, ONCE ? 0x0c030c01u : 0x04030401u);
+              t3 = __builtin_amdgcn_perm(0x64646464u, hi, ONCE ? 0x0c030c01u : 0x04030401u);
+            } else if (ONCE) {
+              t0 = w & 0x000f000fu; t1 = w & 0x00f000f0u;
+              t2 = w8 & 0x000f000fu; t3 = w8 & 0x00f000f0u;
             } else {
               t0 = and_or<FUSED>(w, 0x000f000fu, 0x64006400u); t1 = and_or<FUSED>(w, 0x00f000f0u, 0x54005400u);
               t2 = and_or<FUSED>(w8, 0x000f000fu, 0x64006400u); t3 = and_or<FUSED>(w8, 0x00f000f0u, 0x54005400u);

@@ -493,6 +493,64 @@ def test_few_pair_tiles_are_no_less_exact(capi, oracle, kind, kw, d, mid, T):
     assert (y1 != y0).any() or (mid > 1024 and T > 100)  # (two kernels; longer rows leave them earlier)
 
 
+def k4_scale_bytes(sc, mn):
+    """The 12 bytes of eight 6-bit scales and minima."""
+    b = np.empty(sc.shape[:-1] + (12,), np.uint8)
+    b[..., 0:4] = sc[..., 0:4] | (sc[..., 4:8] >> 4) << 6
+    b[..., 4:8] = mn[..., 0:4] | (mn[..., 4:8] >> 4) << 6
+    b[..., 8:12] = (sc[..., 4:8] & 15) | (mn[..., 4:8] & 15) << 4
+    return b
+
+
+@pytest.mark.parametrize("ratio", [1.0, 0.125])
+@pytest.mark.parametrize("tgu", [12, 13])
+def test_few_pair_tiles_round_weights_beside_q8_0_rows_once(capi, tgu, ratio):
+    """Q4_K / Q5_K gate/up weights themselves: a token is one column of ones, gate rows are all 32 (silu(32) = 32 in f32), a down row picks one hid
+    column, one expert a token: y is 32 times a weight as the kernel has it.  It is the f16 nearest to d * sc * n - dmin * m, unless its
+    f32 value was rounded onto the middle between two, one of 2^13 places, from the other side: 2^-14 of the weights at most."""
+    rng = np.random.default_rng(tgu)
+    d, mid, E, T = 512, 640, 16, 512
+    hl = HostLayer(rng, d, mid, E, 1, fmt="q4k", gg_types=(tgu, 8, 8), shared=False)
+    nb, five = d // 256, tgu == 13
+    size, most = (176, 31) if five else (144, 15)
+
+    def rows(dd, dmin, sc, mn, n):  # n: codes [E, mid, nb, 4 pairs of sub-blocks, 2, 32]
+        b = np.zeros((E, mid, nb, size), np.uint8)
+        b[..., 0:2] = dd[..., None].view(np.uint8)
+        b[..., 2:4] = dmin[..., None].view(np.uint8)
+        b[..., 4:16] = k4_scale_bytes(sc, mn)
+        b[..., size - 128:] = ((n[..., 0, :] & 15) | (n[..., 1, :] & 15) << 4).reshape(E, mid, nb, 128)
+        if five:
+            for j in range(8):
+                b[..., 16:48] |= (n[..., j // 2, j % 2, :] >> 4) << j
+        return b.reshape(-1)
+    one = np.ones((E, mid, nb), np.float16)
+    full = lambda v: np.full((E, mid, nb, 8), v, np.uint8)
+    hl.gate = rows(one, 0 * one, full(32), full(0), np.ones((E, mid, nb, 4, 2, 32), np.uint8))
+    dd = (np.abs(rng.standard_normal((E, mid, nb))) * 0.01 + 0.002).astype(np.float16)
+    dmin = (dd.astype(np.float32) * ratio * rng.uniform(0.5, 2, dd.shape)).astype(np.float16)
+    sc, mn = (rng.integers(0, 64, (E, mid, nb, 8)).astype(np.uint8) for _ in range(2))
+    n = rng.integers(0, most + 1, (E, mid, nb, 4, 2, 32)).astype(np.uint8)
+    hl.up = rows(dd, dmin, sc, mn, n)
+    dn = np.zeros((E, d, mid // 32, 34), np.uint8)
+    dn[..., 0:2] = np.ones(1, np.float16).view(np.uint8)
+    pick = (5 * np.arange(d)[None] + np.arange(E)[:, None]) % mid
+    ee, rr = np.meshgrid(np.arange(E), np.arange(d), indexing="ij")
+    dn[ee, rr, pick // 32, 2 + pick % 32] = 1
+    hl.down = dn.reshape(-1)
+    w = (dd.astype(np.float64)[..., None] * sc)[..., None] * n.reshape(E, mid, nb, 8, 32)
+    w = (w - (dmin.astype(np.float64)[..., None] * mn)[..., None]).reshape(E, mid, d)
+    m, dev = hl.to_gpu(max_tokens=T)
+    y = m.forward(0, gpu(np.eye(T, d, dtype=np.float32))).cpu().numpy()
+    e = m.last_routing(T)[0].cpu().numpy()[:, 0]
+    m.close()
+    want = w[e[:, None], pick[e], np.arange(T)[:, None]].astype(np.float16)
+    far = np.abs(want) >= 0.03  # (32 of these are no f16 denormals, whatever the power of two that hid is kept at)
+    got = (y / 32).astype(np.float16)
+    assert far.mean() > 0.9 and np.abs(got[far].view(np.int16).astype(int) - want[far].view(np.int16)).max() <= 1
+    assert (got != want)[far].mean() <= 2.0 ** -14 + 4 * (2.0 ** -14 / far.sum()) ** 0.5
+
+
 @pytest.mark.parametrize("kind,kw,d,mid,last", [("q4cp", dict(fmt="q4cp"), 512, 640, 50), ("q4cp", dict(fmt="q4cp"), 384, 1152, 25),
                                                 ("table", dict(fmt="q4cp", codebook=TABLE), 512, 768, 60), ("i4r", dict(fmt="i4r"), 512, 768, 50),
                                                 ("table", dict(fmt="q4cp", codebook=TABLE), 384, 1152, 29), ("q4k", dict(fmt="q4k"), 512, 768, 50),
