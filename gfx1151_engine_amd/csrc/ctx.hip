@@ -766,6 +766,7 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
     return MOE_OK;
   };
   const bool sh = L.has_shared && !L.sh_dense;  // the shared expert rides in these kernels as one more slot
+  const uint8_t *rg = sh ? L.sh_gate.data : nullptr, *ru = sh ? L.sh_up.data : nullptr, *rd = sh ? L.sh_down.data : nullptr;
   const int nslots_d = g.topk + (sh ? 1 : 0);
   const bool use_int = L.has_q4cp && c->int_decode && L.experts_affine && (!sh || L.shared_affine) &&
                        (!sh || L.sh_gguf_type == 0) && moe_dec_supported(g.d, g.mid, nslots_d);
@@ -788,9 +789,10 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
   const bool use_intgg = L.has_gguf && c->int_decode && !use_int4k &&
                          moe_decgg_supported(L.gg.tgu, L.gg.tdn, L.sh_gguf_type, sh, g.d, g.mid, g.topk, g.experts) &&
                          (!sh || L.sh_gguf_type != 0);
-  // down rows that are no whole super-blocks: the same launches with 24-bit activations
+  // down rows that are no whole super-blocks: the same launches with 24-bit activations (tensors off their alignment: the general kernels)
   const bool use_intgg3 = L.has_gguf && c->int_decode && !use_int4k && !use_intgg && (!sh || L.sh_gguf_type != 0) &&
-                          moe_decgg3_supported(L.gg.tgu, L.gg.tdn, L.sh_gguf_type, sh, g.d, g.mid, g.topk, g.experts);
+                          moe_decgg3_supported(L.gg.tgu, L.gg.tdn, L.sh_gguf_type, sh, g.d, g.mid, g.topk, g.experts) &&
+                          moe_decgg_aligned(L.gg.tgu, L.gg.tdn, L.sh_gguf_type, L.gg.gate, L.gg.up, L.gg.down, rg, ru, rd);
   // (Q4_K layers: the gate/up launch of the mixes where it deals its rows over all lanes)
   const bool gu4k_dealt = use_int4k && moe_decgg_passes(g.d) > 0 &&
                           moe_decgg_supported(L.gg.tgu, L.gg.tdn, L.sh_gguf_type, sh, g.d, g.mid, g.topk, g.experts);
@@ -825,7 +827,6 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
        })))
     return rc;
   const moe_wview *shg = sh ? &L.sh_gate : nullptr, *shu = sh ? &L.sh_up : nullptr, *shd = sh ? &L.sh_down : nullptr;
-  const uint8_t *rg = sh ? L.sh_gate.data : nullptr, *ru = sh ? L.sh_up.data : nullptr, *rd = sh ? L.sh_down.data : nullptr;
   if (L.has_q4cp) {
     if (sh && L.sh_gguf_type != 0) return MOE_E_UNSUPPORTED;
     if (use_uq) {

@@ -1105,6 +1105,13 @@ bool moe_decgg3_supported(int tgu, int tdn, int tsh, bool has_shared, int d, int
          kpt + 1 <= D4_MAXSLOTS && n_experts <= 1024 && kpt <= n_experts;
 }
 static size_t ggu_align(int t) { return t == MOE_GGML_Q8_0 || t == MOE_GGML_IQ4_NL ? 4 : 16; }
+// Tensors that these launches can read.  The general f32 kernels ask for less (Q8_0 and IQ4_NL 2 bytes, Q5_1 and IQ4_XS 8).
+bool moe_decgg_aligned(int tgu, int tdn, int tsh, const uint8_t* gate, const uint8_t* up, const uint8_t* down, const uint8_t* sh_gate,
+                       const uint8_t* sh_up, const uint8_t* sh_down) {
+  const size_t gu = ggu_align(tgu), sh = ggu_align(tsh);
+  return moe_aligned(gate, gu) && moe_aligned(up, gu) && moe_aligned(down, ggu_align(tdn)) &&
+         (!sh_gate || (moe_aligned(sh_gate, sh) && moe_aligned(sh_up, sh) && moe_aligned(sh_down, sh)));
+}
 
 static bool decgg_gu_ok(int planes, int tgu, int tsh, bool sh, int d, int mid, int kpt, int n_experts) {
   return planes == 3 ? moe_decgg3_supported(tgu, MOE_GGML_Q8_0, tsh, sh, d, mid, kpt, n_experts)

@@ -190,6 +190,8 @@ int moe_launch_dec_dn_uq(const moe_wview* dn, const moe_wview* sh_down, const ui
 bool moe_dec4k_supported(int d, int mid, int nslots);
 bool moe_decgg_supported(int tgu, int tdn, int tsh, bool has_shared, int d, int mid, int kpt, int n_experts);
 bool moe_decgg3_supported(int tgu, int tdn, int tsh, bool has_shared, int d, int mid, int kpt, int n_experts);
+bool moe_decgg_aligned(int tgu, int tdn, int tsh, const uint8_t* gate, const uint8_t* up, const uint8_t* down, const uint8_t* sh_gate,
+                       const uint8_t* sh_up, const uint8_t* sh_down);
 int moe_launch_decgg_gu_topk(int tgu, int tsh, const uint8_t* gate, const uint8_t* up, const uint8_t* sh_gate,
                              const uint8_t* sh_up, const uint32_t* xplanes, const float2* xmeta, const float* logits,
                              int n_experts, int* ids, float* ws, int id_stride, int kpt, int P, int d, int mid,

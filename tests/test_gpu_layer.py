@@ -386,6 +386,37 @@ def test_small_batch_gguf_hid_too_small_for_a_24_bit_factor(oracle, scale, T):
     assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= 2e-4
 
 
+@pytest.mark.parametrize("T", [1, 4, 20, 40])
+@pytest.mark.parametrize("types,d,mid", [((13, 8, 8), 2560, 640), ((8, 7, 7), 2048, 128), ((20, 8, 7), 2048, 384), ((23, 7, 8), 2048, 128)])
+@pytest.mark.parametrize("moved", ["gate_up", "down", "shared"])
+def test_gguf_tensors_that_begin_where_their_blocks_may(oracle, types, d, mid, T, moved):
+    """Tensors two bytes (Q8_0, IQ4_NL) and eight bytes (Q5_1, IQ4_XS) off the alignment of the fastest kernels."""
+    import torch
+    from gfx1151_engine_amd import capi
+    rng = np.random.default_rng(d + mid + T)
+    hl = HostLayer(rng, d, mid, 6, 3, fmt="q4k", gg_types=types)
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    yo, io, wo = oracle.moe_layer(hl.oracle_layer(), x)
+    m, dev = hl.to_gpu(max_tokens=T)
+
+    def at(name, t, off):
+        n = {8: 2, 20: 2, 7: 8, 23: 8}.get(t, 0) if off else 0
+        buf = torch.zeros(dev[name].numel() + n, dtype=torch.uint8, device="cuda")
+        buf[n:] = dev[name].reshape(-1)
+        dev[name + "_moved"] = buf
+        return buf[n:]
+    m.set_experts_gguf(0, at("gate", types[0], moved == "gate_up"), at("up", types[0], moved == "gate_up"), at("down", types[1], moved == "down"),
+                       types[0], types[1])
+    sh = [at(n, types[2], moved == "shared") for n in ("shg", "shu", "shd")]
+    m.set_shared(0, capi.wview(sh[0], 0, mid, d), capi.wview(sh[1], 0, mid, d), capi.wview(sh[2], 0, d, mid), capi.wview(dev["shsg"], capi.F32, 1, d),
+                 types[2])
+    y = m.forward(0, gpu(x)).cpu().numpy()
+    ids = m.last_routing(T)[0].cpu().numpy()
+    m.close()
+    assert (ids[:, :3] == io[:, :3]).all()
+    assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= (TOL_GEMV if T <= 32 else TOL_LAYER)
+
+
 @pytest.mark.parametrize("T", [5, 16, 17, 25, 32])
 @pytest.mark.parametrize("E,d,router,shared", [(17, 1024, "f32", True), (32, 2048, "bf16", True), (513, 1024, "f32", False), (20, 768, "bf16", True),
                                                (1000, 256, "f32", True), (16, 384, "f32", True), (40, 640, "f32", True), (33, 2304, "bf16", True), (18, 128, "f32", False)])
