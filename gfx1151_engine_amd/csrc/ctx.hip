@@ -725,6 +725,8 @@ static int forward_small(moe_ctx* c, MoeLayer& L, const float* x, int P, float* 
 // What the selection of a small batch needs to be certain of its expert ids (topk.h, select_certain): the router
 // launch sums the products in a parallel order; |that fp64 sum - the reference's sequential one| <= 2 gamma_d |w||x|
 // for any row w (gamma_d = d u / (1 - d u), u = 2^-53), so tol_scale * |x| bounds it for every logit of a token.
+// Every block that selects for a token has to judge by the same bound: inside the gate/up launch, where most of them only rank, it is the
+// router launch's, and a launch that leaves none (tol_from_router; the selection's own block then takes |x| itself) selects aside.
 static moe_rfix router_fix(const moe_ctx* c, const MoeLayer& L, const float* x, bool tol_from_router) {
   moe_rfix R{};
   R.W = L.router.data;
@@ -742,10 +744,9 @@ static moe_rfix router_fix(const moe_ctx* c, const MoeLayer& L, const float* x, 
 static bool select_aside(const moe_ctx* c, const MoeLayer& L, int P, bool gu_topk) {
   return !gu_topk && moe_router_split_supported(&L.router, P, c->cfg.topk);
 }
-static int select_small(moe_ctx* c, moe_rfix rf, int P, int parts, hipStream_t st) {
+static int select_small(moe_ctx* c, const moe_rfix& rf, int P, int parts, hipStream_t st) {
   const moe_config& g = c->cfg;
   if (!parts) return moe_launch_router_topk_small(c->logits, c->ids, c->ws, P, g.experts, g.topk, g.id_stride, &rf, st);
-  rf.tol = c->rtol;
   return moe_launch_router_split_topk(c->kpart, parts, c->ids, c->ws, P, g.experts, g.topk, g.id_stride, rf, st);
 }
 
@@ -807,14 +808,12 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
   // Two layers, us, in the gate/up launch and aside: look-up kernels 76.3 and 79.7 at 2 tokens, 101.5 and 98.3 at 3; GGUF mixes 84.7 and 84.4 at 2,
   // 122 and 119 at 3, 153 and 148 at 4; Q4_K 83.6 and 85.3 at 3, 113 and 108 at 4; q4cp 73.7 and 76.4 at 3, 100 and 97 at 4; both kinds
   // of GGUF layers with rows dealt over all lanes, whose rounds are shorter: mixes 104.5 and 106.4 at 3, 129.2 and 131.5 at 4, Q4_K 75.5
-  // and 82.7, 99.3 and 100.8 (above four the router launch leaves no bounds for the selection)
+  // and 82.7, 99.3 and 100.8
   const bool gg_dealt = gu4k_dealt || use_intgg3 || (use_intgg && moe_decgg_passes(g.d) > 0);
   const int topk_max = c->gu_topk_max >= 0 ? c->gu_topk_max : use_lut ? 2 : gg_dealt ? 4 : use_intgg ? 2 : use_f32a ? 4 : 3;
   const bool gu_topk = (((use_int && !use_uq) || ((use_int4k || use_intgg) && !use_uq_gg) || use_intgg3 || use_lut || use_f32a) && P <= topk_max) &&
-                       moe_dec_gu_topk_supported(g.experts, g.topk);
-  // (up to 4 tokens the router launch leaves each token's bound for the selection; larger batches: the selecting
-  //  block takes the norm of x itself)
-  const moe_rfix rf = router_fix(c, L, x, P <= 4);
+                       moe_dec_gu_topk_supported(g.experts, g.topk) && moe_router_small_bounds(&L.router, P);
+  const moe_rfix rf = router_fix(c, L, x, moe_router_small_bounds(&L.router, P));
   if ((rc = stage(MOE_PROF_ROUTER, [&]() -> int {
          // (the selection runs in launches of its own here, so that it can be made certain: no top-k inside the logits launch)
          int parts = 0;
@@ -1008,8 +1007,8 @@ static int forward_small_v2(moe_ctx* c, MoeLayer& L, const float* x, int P, floa
   const bool sh = L.has_shared && !L.sh_dense;  // a q4cp shared expert rides in these kernels as one more slot
   if (sh && (L.sh_gguf_type != 0 || !L.shared_affine)) return MOE_E_UNSUPPORTED;
   const int nslots_d = g.topk + (sh ? 1 : 0);
-  const bool gu_topk = P <= (c->gu_topk_max >= 0 ? c->gu_topk_max : 4);  // (105 us either way at 4 tokens, two layers)
-  const moe_rfix rf = router_fix(c, L, x, P <= 4);
+  const bool gu_topk = P <= (c->gu_topk_max >= 0 ? c->gu_topk_max : 4) && moe_router_small_bounds(&L.router, P);  // (105 us either way at 4 tokens, two layers)
+  const moe_rfix rf = router_fix(c, L, x, moe_router_small_bounds(&L.router, P));
   if ((rc = stage(MOE_PROF_ROUTER, [&]() -> int {
          // (the planes of rot_in(x, su) ride in the router launch's spare blocks)
          int parts = 0;

@@ -904,6 +904,7 @@ int moe_launch_dec_gu_topk(const moe_wview* gu, const moe_wview* sh_gate, const 
                            uint32_t* hplanes, float2* hmeta, float* hid_f32, hipStream_t st, const moe_dec_v2* v2,
                            const moe_rfix* rf) {
   const moe_rfix RFV = rf ? *rf : moe_rfix{};
+  if (RFV.W && !RFV.tol) return MOE_E_INVALID;
   GuArgs2 A{};
   A.gu = decw(gu);
   A.shg = decw(sh_gate);
@@ -938,6 +939,7 @@ int moe_launch_dec_gu_lut(const moe_wview* gu, const moe_wview* sh_gate, const m
                           int mid, float* hid_f32, hipStream_t st, const moe_rfix* rf, bool affine) {
   if (!x || !hid_f32 || !ids || (logits && !moe_dec_gu_topk_supported(n_experts, kpt))) return MOE_E_INVALID;
   const moe_rfix RFV = rf ? *rf : moe_rfix{};
+  if (logits && RFV.W && !RFV.tol) return MOE_E_INVALID;
   GuArgs2 A{};
   A.gu = decw(gu);
   A.shg = decw(sh_gate);

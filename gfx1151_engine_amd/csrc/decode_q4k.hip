@@ -1046,6 +1046,7 @@ int moe_launch_dec4k_gu_topk(const uint8_t* gate, const uint8_t* up, const uint8
                              int* ids, float* ws, int id_stride, int kpt, int P, int d, int mid,
                              uint32_t* hplanes, float2* hmeta, hipStream_t st, const moe_rfix* rf) {
   const moe_rfix RFV = rf ? *rf : moe_rfix{};
+  if (RFV.W && !RFV.tol) return MOE_E_INVALID;
   if (!gate || !up || !xplanes || !xmeta || !logits || !ids || !ws || !hplanes || !hmeta || (!sh_gate != !sh_up))
     return MOE_E_INVALID;
   if (!moe_aligned(gate, 16) || !moe_aligned(up, 16) || (sh_gate && (!moe_aligned(sh_gate, 16) || !moe_aligned(sh_up, 16))))
@@ -1123,6 +1124,7 @@ int moe_launch_decgg_gu_topk(int tgu, int tsh, const uint8_t* gate, const uint8_
                              int n_experts, int* ids, float* ws, int id_stride, int kpt, int P, int d, int mid,
                              uint32_t* hplanes, float2* hmeta, hipStream_t st, const moe_rfix* rf, int planes) {
   const moe_rfix RFV = rf ? *rf : moe_rfix{};
+  if (RFV.W && !RFV.tol) return MOE_E_INVALID;
   if (!gate || !up || !xplanes || !xmeta || !logits || !ids || !ws || !hplanes || !hmeta || (!sh_gate != !sh_up))
     return MOE_E_INVALID;
   if (!decgg_gu_ok(planes, tgu, tsh, sh_gate != nullptr, d, mid, kpt, n_experts)) return MOE_E_UNSUPPORTED;

@@ -51,6 +51,8 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
                             int P, float* logits, float* out_x, uint32_t* planes, float2* meta,
                             int planes_form, hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rot = nullptr,
                             float* tol_out = nullptr, float tol_scale = 0.f, int* parts = nullptr);
+// Whether it leaves each token's bound in tol_out: not where its column shares do not apply (more than four tokens).
+bool moe_router_small_bounds(const moe_wview* W, int P);
 // (parts: where the launch can, it leaves the logits' column shares [*parts][P][E] in kpart for moe_launch_router_split_topk, and
 // tol_out; else *parts = 0)
 // scratch of the column-split router launch (5..32 tokens): fp64 partial tiles of up to 8 splits x 32 tokens

@@ -695,6 +695,16 @@ int moe_router_logits_seq(const moe_wview* W, const float* bias, const float* x,
   return MOE_OK;
 }
 
+static int column_shares(int P, int E, int d) {
+  if (P <= 4 || E + 1 > MOE_ROUTER_KSPLIT_ROWS || d < 256) return 1;
+  return d / 128 < 8 ? d / 128 : 8;
+}
+static bool on_matrix_pipe(int P, int d, int KS) { return P > 4 && (P > 24 || KS > 1) && d % 128 == 0; }
+bool moe_router_small_bounds(const moe_wview* W, int P) {
+  const int E = (int)W->rows, d = (int)W->cols;
+  return P <= 4 || on_matrix_pipe(P, d, column_shares(P, E, d));
+}
+
 // Internal: small-P logits plus the shared-expert gate row (and, if planes != nullptr, the digit
 // planes of x for the integer-dot decode kernels) in the same launch.
 int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x,
@@ -718,9 +728,8 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
   // (as many shares as leave every wave a step of 16 columns, whether or not they are equal: 2560 columns in eight shares of two and three
   // steps a wave instead of four of five: the launch 13.2 -> 7.5 us at 20 tokens; 2560 x 640 layers q4cp 5 tokens 49.0 -> 46.5, 20 118.2
   // 112.4, table codebook 12 112.4 109.1; 2304 x 512 12 67.5 62.2)
-  int KS = 1;
-  if (kpart && ktickets && P > 4 && E + 1 <= MOE_ROUTER_KSPLIT_ROWS) KS = d < 256 ? 1 : d / 128 < 8 ? d / 128 : 8;
-  const bool mfma_ok = (P > 24 || KS > 1) && d % 128 == 0;
+  const int KS = kpart && ktickets ? column_shares(P, E, d) : 1;
+  const bool mfma_ok = on_matrix_pipe(P, d, KS);
   if (P > 24 && !mfma_ok) {
     // more than 24 tokens per block cost the kernel its second wave per SIMD (accumulators):
     // two launches of at most 16 tokens read the router matrix twice (L2 / MALL) and are faster

@@ -690,7 +690,7 @@ __device__ bool select_certain(const float* lg, const moe_rfix& R, int tok, int*
   __shared__ float xsq[NT / 64];
   float tol = 0.f;
   if (!want_ws) {
-    tol = R.W && R.tol ? R.tol[tok] : 0.f;  // (blocks that only rank take the bound from the router launch)
+    tol = R.W ? R.tol[tok] : 0.f;  // (blocks that only rank take the bound from the router launch)
     const int r = topk_ids_by_logit<NPL>(lg, sel_ids, E, k, tol);
     if (r == 1) return true;
     if (r != 0 || !R.W) {  // rows the ranking does not handle, or no router operands: the logits as they stand

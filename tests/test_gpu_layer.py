@@ -659,6 +659,66 @@ def test_small_batch_ids_when_summation_orders_disagree(oracle, fmt, T, int_deco
     m.close()
 
 
+@pytest.mark.parametrize("T", [3, 7, 20, 32])
+@pytest.mark.parametrize("fmt,d", [("q4cp", 1024), ("q4cp", 1056), ("table", 640), ("q4k", 2304), ("q4k", 2560), ("ggmix", 1024), ("ggmix", 3072), ("i4r", 1024)])
+def test_all_blocks_of_a_launch_select_by_one_bound(oracle, fmt, d, T):
+    """The ladder of test_small_batch_ids_when_summation_orders_disagree with MOE_OPT_GU_TOPK_MAX_TOKENS = 32: the blocks that only rank must judge
+    a token's gaps by the bound of the block that writes the ids, or a slot's gate/up rows and its down rows are two experts'.  The
+    selection aside gives the same result but for the last bits of the weights, whose normaliser has terms of logits that are not redone:
+    two steps of 2^-23, of weights below 1.  (1056 columns: the router launch leaves no bounds above four tokens.)"""
+    import torch
+    from gfx1151_engine_amd import capi
+    rng = np.random.default_rng(d + T)
+    mid, E, k = 256, 64, 8
+    bias = np.full(E, -30.0, np.float32)
+    cb = np.sort(rng.standard_normal(16)).astype(np.float32) if fmt == "table" else None
+    hl = HostLayer(rng, d, mid, E, k, fmt={"table": "q4cp", "ggmix": "q4k"}.get(fmt, fmt), bias=bias, codebook=cb, scale_std=0.05,
+                   gg_types=(13, 8, 8) if fmt == "ggmix" else (12, 12, 12))
+    hl.router[:] = 0.0
+    A = 61
+    hl.router[A] = rng.standard_normal(d).astype(np.float32) * np.float32(0.05)
+    hl.router[A, [0, d - 1]] = 1.0
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    x[:, 0], x[:, d - 1] = 2.0 ** 36, -2.0 ** 36
+    bias[A] = 0.0
+    lgA = oracle.router(hl.oracle_layer().router, x, k, bias=bias)[0][:, A]
+    for j in range(40):
+        bias[j] = np.float32(np.float64(lgA[0]) + (3.5 - j) * 1e-5)
+    hl.bias = bias
+    io = oracle.router(hl.oracle_layer().router, x, k, bias=bias)[1]
+    m, dev = hl.to_gpu(max_tokens=T)
+    ys = []
+    for most in (32, 0):
+        m.set_option(capi.OPT_GU_TOPK_MAX_TOKENS, most)
+        ys.append(m.forward(0, gpu(x)).cpu().numpy())
+        assert (m.last_routing(T)[0].cpu().numpy()[:, :k] == io[:, :k]).all()
+    m.close()
+    assert np.isfinite(ys[0]).all()
+    assert max(max_abs_rel(ys[0][t], ys[1][t]) for t in range(T)) <= 1e-6
+
+
+@pytest.mark.parametrize("T", [5, 17, 32])
+@pytest.mark.parametrize("E,d,router", [(40, 640, "f32"), (40, 2304, "bf16"), (24, 2560, "f32"), (100, 384, "f32"), (18, 128, "f32"), (20, 1024, "bf16")])
+def test_small_batch_router_shares_added_by_the_last_block(oracle, E, d, router, T):
+    """The selection inside the gate/up launch at more than four tokens: the column shares are handed over by tickets.  One and two tiles of
+    tokens, several row groups, one with rows left over, equal and unequal shares."""
+    from gfx1151_engine_amd import capi
+    rng = np.random.default_rng(E + d + T)
+    hl = HostLayer(rng, d, 256, E, 6, router_dtype=router, scale_std=0.02)
+    if router == "f32":
+        hl.router[1] = hl.router[0]
+    x = rng.standard_normal((T, d), dtype=np.float32)
+    yo, io, wo = oracle.moe_layer(hl.oracle_layer(), x)
+    m, dev = hl.to_gpu(max_tokens=T)
+    m.set_option(capi.OPT_GU_TOPK_MAX_TOKENS, 32)
+    for _ in range(3):  # (the tickets rest at 0 between launches)
+        y = m.forward(0, gpu(x)).cpu().numpy()
+        ids, ws = (a.cpu().numpy()[:, :6] for a in m.last_routing(T))
+        assert (ids == io[:, :6]).all() and np.abs(ws - wo[:, :6]).max() <= 1e-6
+        assert max(max_abs_rel(y[t], yo[t]) for t in range(T)) <= TOL_INT_Q4CP
+    m.close()
+
+
 # ---------- few tokens, codebooks by look-up: where its blocks, tables and selection end ----------
 # (one slot: a down block of a single wave fills the tables in four turns; 1000 experts: the selection keeps twice the LDS;
 # a gate codebook and an up codebook of the shared expert: two tables; groups past the lanes of a row: d = 3072)
