@@ -790,9 +790,9 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
   const bool use_intgg = L.has_gguf && c->int_decode && !use_int4k &&
                          moe_decgg_supported(L.gg.tgu, L.gg.tdn, L.sh_gguf_type, sh, g.d, g.mid, g.topk, g.experts) &&
                          (!sh || L.sh_gguf_type != 0);
-  // down rows that are no whole super-blocks: the same launches with 24-bit activations (tensors off their alignment: the general kernels)
-  const bool use_intgg3 = L.has_gguf && c->int_decode && !use_int4k && !use_intgg && (!sh || L.sh_gguf_type != 0) &&
-                          moe_decgg3_supported(L.gg.tgu, L.gg.tdn, L.sh_gguf_type, sh, g.d, g.mid, g.topk, g.experts) &&
+  // down rows that are no whole super-blocks: the same launches on activations in f32 (tensors off their alignment: the general kernels)
+  const bool use_ggf32 = L.has_gguf && c->int_decode && !use_int4k && !use_intgg && (!sh || L.sh_gguf_type != 0) &&
+                          moe_decgg_f32_supported(L.gg.tgu, L.gg.tdn, L.sh_gguf_type, sh, g.d, g.mid, g.topk, g.experts) &&
                           moe_decgg_aligned(L.gg.tgu, L.gg.tdn, L.sh_gguf_type, L.gg.gate, L.gg.up, L.gg.down, rg, ru, rd);
   // (Q4_K layers: the gate/up launch of the mixes where it deals its rows over all lanes)
   const bool gu4k_dealt = use_int4k && moe_decgg_passes(g.d) > 0 &&
@@ -809,17 +809,17 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
   // 122 and 119 at 3, 153 and 148 at 4; Q4_K 83.6 and 85.3 at 3, 113 and 108 at 4; q4cp 73.7 and 76.4 at 3, 100 and 97 at 4; both kinds
   // of GGUF layers with rows dealt over all lanes, whose rounds are shorter: mixes 104.5 and 106.4 at 3, 129.2 and 131.5 at 4, Q4_K 75.5
   // and 82.7, 99.3 and 100.8
-  const bool gg_dealt = gu4k_dealt || use_intgg3 || (use_intgg && moe_decgg_passes(g.d) > 0);
+  const bool gg_dealt = gu4k_dealt || use_ggf32 || (use_intgg && moe_decgg_passes(g.d) > 0);
   const int topk_max = c->gu_topk_max >= 0 ? c->gu_topk_max : use_lut ? 2 : gg_dealt ? 4 : use_intgg ? 2 : use_f32a ? 4 : 3;
-  const bool gu_topk = (((use_int && !use_uq) || ((use_int4k || use_intgg) && !use_uq_gg) || use_intgg3 || use_lut || use_f32a) && P <= topk_max) &&
+  const bool gu_topk = (((use_int && !use_uq) || ((use_int4k || use_intgg) && !use_uq_gg) || use_ggf32 || use_lut || use_f32a) && P <= topk_max) &&
                        moe_dec_gu_topk_supported(g.experts, g.topk) && moe_router_small_bounds(&L.router, P);
   const moe_rfix rf = router_fix(c, L, x, moe_router_small_bounds(&L.router, P));
   if ((rc = stage(MOE_PROF_ROUTER, [&]() -> int {
          // (the selection runs in launches of its own here, so that it can be made certain: no top-k inside the logits launch)
          int parts = 0;
          int e = moe_router_logits_small(&L.router, L.router_bias, L.has_shared ? &L.sh_sg : nullptr, x, P, c->logits,
-                                         c->sh_logit, (use_int || use_int4k || use_intgg || use_intgg3) ? c->xplanes : nullptr, c->xmeta,
-                                         use_intgg3 ? MOE_PLANES_QVEC3 : use_int4k || use_intgg ? MOE_PLANES_QVEC : MOE_PLANES_QVEC4, st, c->kpart, c->ktickets, nullptr, rf.W ? c->rtol : nullptr, rf.tol_scale,
+                                         c->sh_logit, (use_int || use_int4k || use_intgg) ? c->xplanes : nullptr, c->xmeta,
+                                         use_int4k || use_intgg, st, c->kpart, c->ktickets, nullptr, rf.W ? c->rtol : nullptr, rf.tol_scale,
                                          select_aside(c, L, P, gu_topk) ? &parts : nullptr);
          if (!e && !gu_topk) e = select_small(c, rf, P, parts, st);
          return e;
@@ -925,20 +925,20 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
                                g.d, g.topk, moe_hscale{nullptr, 0.f, 0.f}, st, nullptr);
     });
   }
-  if (use_intgg || use_intgg3) {
-    const int planes = use_intgg3 ? 3 : 2;
+  if (use_intgg || use_ggf32) {
+    const moe_dec_f32 f32 = use_ggf32 ? moe_dec_f32{x, c->hid32} : moe_dec_f32{};
     if ((rc = stage(MOE_PROF_UP, [&]() -> int {
            return gu_topk ? moe_launch_decgg_gu_topk(L.gg.tgu, L.sh_gguf_type, L.gg.gate, L.gg.up, rg, ru, c->xplanes,
                                                      c->xmeta, c->logits, g.experts, c->ids, c->ws, g.id_stride, g.topk,
-                                                     P, g.d, g.mid, c->hplanes, c->hmeta, st, &rf, planes)
+                                                     P, g.d, g.mid, c->hplanes, c->hmeta, st, &rf, f32)
                           : moe_launch_decgg_gu(L.gg.tgu, L.sh_gguf_type, L.gg.gate, L.gg.up, rg, ru, c->xplanes, c->xmeta,
                                                 c->ids, g.experts, g.id_stride, g.topk, P, g.d, g.mid, c->hplanes, c->hmeta,
-                                                st, planes);
+                                                st, f32);
          })))
       return rc;
     return stage(MOE_PROF_DOWN, [&]() -> int {
       return moe_launch_decgg_dn(L.gg.tdn, L.sh_gguf_type, L.gg.down, rd, c->sh_logit, c->hplanes, c->hmeta, c->ids, c->ws,
-                                 g.id_stride, g.topk, P, g.d, g.mid, y, (uint64_t)g.d, st, planes);
+                                 g.id_stride, g.topk, P, g.d, g.mid, y, (uint64_t)g.d, st, f32.hid);
     });
   }
   if (L.gg.tgu != MOE_GGML_Q4_K || L.gg.tdn != MOE_GGML_Q4_K || (sh && L.sh_gguf_type != MOE_GGML_Q4_K)) {
@@ -1014,7 +1014,7 @@ static int forward_small_v2(moe_ctx* c, MoeLayer& L, const float* x, int P, floa
          int parts = 0;
          const moe_rot_planes rot{L.v2_su, c->v2_xplanes, c->v2_xmeta};
          int e = moe_router_logits_small(&L.router, L.router_bias, L.has_shared ? &L.sh_sg : nullptr, x, P, c->logits,
-                                         c->sh_logit, sh ? c->xplanes : nullptr, c->xmeta, MOE_PLANES_QVEC4,
+                                         c->sh_logit, sh ? c->xplanes : nullptr, c->xmeta, false,
                                          st, c->kpart, c->ktickets, &rot, rf.W ? c->rtol : nullptr, rf.tol_scale,
                                          select_aside(c, L, P, gu_topk) ? &parts : nullptr);
          if (!e && !gu_topk) e = select_small(c, rf, P, parts, st);

@@ -843,7 +843,7 @@ DecW decw(const moe_wview* w) {
 
 }  // namespace
 
-size_t moe_qvec_plane_bytes(int K) { return (size_t)(K / 32) * QV3_GROUP_DW * 4; }  // (the largest form)
+size_t moe_qvec_plane_bytes(int K) { return (size_t)(K / 32) * QV_GROUP_DW * 4; }
 size_t moe_qvec_meta_bytes(int K) { return (size_t)(K / 32) * sizeof(float2); }
 
 // Supported shapes of the integer-dot decode kernels (otherwise the caller uses the f32 kernels).

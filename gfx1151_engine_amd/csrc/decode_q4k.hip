@@ -7,6 +7,8 @@
 // rows of 3072 are 48 units (gate/up deals several rows' units over a wave, ggu_gu_packed), rows of 768 are
 // 12 units (four slots per wave).
 // (reference: src/gpu/parts/26_kernels_moe_gguf.inc:527-568,693-756,893-939; src/gguf.h:328-336,408-441)
+#include <type_traits>
+
 #include "common.h"
 #include "internal.h"
 #include "iq4.h"
@@ -33,27 +35,23 @@ __device__ __forceinline__ float sum64(float v) {
   return rows_total_add(dpp_add_row(v));
 }
 
-// activation planes of one unit: two groups (A = low nibbles, B = high nibbles), N planes (qvec, qvec3)
-template <int N>
-struct XUn {
-  uint32_t a[N][8], b[N][8];
+// activation planes of one unit: two groups (A = low nibbles, B = high nibbles)
+struct XU {
+  uint32_t a[2][8], b[2][8];
   float qa, qsa, qb, qsb;
 };
-typedef XUn<2> XU;
-template <int N>
-__device__ __forceinline__ void take_planes(XUn<N>& x, const uint4* s) {
+__device__ __forceinline__ void take_planes(XU& x, const uint4* s) {
 #pragma unroll
-  for (int p = 0; p < N; p++) {
-    const uint4 a0 = s[2 * p], a1 = s[2 * p + 1], b0 = s[2 * N + 2 * p], b1 = s[2 * N + 2 * p + 1];
+  for (int p = 0; p < 2; p++) {
+    const uint4 a0 = s[2 * p], a1 = s[2 * p + 1], b0 = s[4 + 2 * p], b1 = s[4 + 2 * p + 1];
     x.a[p][0] = a0.x; x.a[p][1] = a0.y; x.a[p][2] = a0.z; x.a[p][3] = a0.w;
     x.a[p][4] = a1.x; x.a[p][5] = a1.y; x.a[p][6] = a1.z; x.a[p][7] = a1.w;
     x.b[p][0] = b0.x; x.b[p][1] = b0.y; x.b[p][2] = b0.z; x.b[p][3] = b0.w;
     x.b[p][4] = b1.x; x.b[p][5] = b1.y; x.b[p][6] = b1.z; x.b[p][7] = b1.w;
   }
 }
-template <int N>
-__device__ __forceinline__ void load_xu(XUn<N>& x, const uint32_t* planes, const float2* meta, size_t g0) {
-  take_planes(x, (const uint4*)(planes + g0 * (8 * N)));
+__device__ __forceinline__ void load_xu(XU& x, const uint32_t* planes, const float2* meta, size_t g0) {
+  take_planes(x, (const uint4*)(planes + g0 * QV_GROUP_DW));
   const float2 ma = meta[g0], mb = meta[g0 + 1];
   x.qa = ma.x; x.qsa = ma.y; x.qb = mb.x; x.qsb = mb.y;
 }
@@ -383,36 +381,73 @@ __device__ __forceinline__ void ggu_fetch(const uint8_t* row, int ul, GgU<T>& o)
   }
 }
 
-// integer sums of a group against its digit planes -> float (together they can exceed 2^24 for 5- and 8-bit codes: exact
-// conversions and a rounded fma for each plane but one instead of an integer combine)
-template <int N>
-__device__ __forceinline__ float planes_val(const int (&v)[N]) {
-  float r = (float)v[N - 1];
-  if (N == 3) r = fmaf((float)v[1], 256.f, r);
-  return fmaf((float)v[0], N == 3 ? 65536.f : 256.f, r);
-}
-// v[p] += four codes x four digits of plane p
-template <int N>
-__device__ __forceinline__ void planes_dot(int (&v)[N], int codes, const uint32_t (&pl)[N][8], int i) {
+// A unit's activations as they are (layers whose activations stay in f32, moe_decgg_f32_supported): its 64 values and their sums by group.
+struct XF {
+  float a[32], b[32], sa, sb;
+};
+__device__ __forceinline__ void take_f32(XF& x, const float4* s) {
 #pragma unroll
-  for (int p = 0; p < N; p++) v[p] = __builtin_amdgcn_sdot4(codes, (int)pl[p][i], v[p], false);
+  for (int i = 0; i < 8; i++) {
+    const float4 a = s[i], b = s[8 + i];
+    x.a[4 * i] = a.x; x.a[4 * i + 1] = a.y; x.a[4 * i + 2] = a.z; x.a[4 * i + 3] = a.w;
+    x.b[4 * i] = b.x; x.b[4 * i + 1] = b.y; x.b[4 * i + 2] = b.z; x.b[4 * i + 3] = b.w;
+  }
+}
+__device__ __forceinline__ void sum_f32(XF& x) {
+  float a[4] = {}, b[4] = {};
+#pragma unroll
+  for (int i = 0; i < 32; i++) {
+    a[i & 3] += x.a[i];
+    b[i & 3] += x.b[i];
+  }
+  x.sa = (a[0] + a[1]) + (a[2] + a[3]);
+  x.sb = (b[0] + b[1]) + (b[2] + b[3]);
 }
 
-template <int T, int N>
-__device__ __forceinline__ float ggu_dot(const GgU<T>& o, int jj, const XUn<N>& x) {
-  if constexpr (T == MOE_GGML_Q4_K && N == 2) {
+// The sum over a group of codes times activations, group A or B (GB) of a unit; codes come four to a word as signed (S) or unsigned bytes.
+template <class X> struct Acc;
+template <> struct Acc<XU> { int hi = 0, lo = 0; };
+template <> struct Acc<XF> { float v = 0.f; };
+template <bool GB, bool S>
+__device__ __forceinline__ void dot4(Acc<XU>& c, int codes, const XU& x, int i) {
+  c.hi = __builtin_amdgcn_sdot4(codes, (int)(GB ? x.b : x.a)[0][i], c.hi, false);
+  c.lo = __builtin_amdgcn_sdot4(codes, (int)(GB ? x.b : x.a)[1][i], c.lo, false);
+}
+template <bool GB, bool S>
+__device__ __forceinline__ void dot4(Acc<XF>& c, int codes, const XF& x, int i) {
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const float n = S ? (float)(int8_t)(codes >> (8 * j)) : (float)(((uint32_t)codes >> (8 * j)) & 0xffu);
+    c.v = fmaf(n, (GB ? x.b : x.a)[4 * i + j], c.v);
+  }
+}
+// s times that sum.  (digit planes: the integer sums can exceed 2^24 for 5- and 8-bit codes: two exact conversions and one rounded fma
+// instead of an integer combine)
+template <bool GB>
+__device__ __forceinline__ float times(float s, const Acc<XU>& c, const XU& x) { return s * (GB ? x.qb : x.qa) * fmaf((float)c.hi, 256.f, (float)c.lo); }
+template <bool GB>
+__device__ __forceinline__ float times(float s, const Acc<XF>& c, const XF& x) { return s * c.v; }
+// the group's activations, summed
+template <bool GB>
+__device__ __forceinline__ float total(const XU& x) { return GB ? x.qsb : x.qsa; }
+template <bool GB>
+__device__ __forceinline__ float total(const XF& x) { return GB ? x.sb : x.sa; }
+
+template <int T, class X>
+__device__ __forceinline__ float ggu_dot(const GgU<T>& o, int jj, const X& x) {
+  Acc<X> va, vb;
+  if constexpr (T == MOE_GGML_Q4_K && std::is_same<X, XU>::value) {
     return unit_dot(o.c0, o.c1, quad_header(o.hw), jj, x);
   } else if constexpr (T == MOE_GGML_Q4_K) {
     const uint32_t w[8] = {o.c0.x, o.c0.y, o.c0.z, o.c0.w, o.c1.x, o.c1.y, o.c1.z, o.c1.w};
-    int va[N] = {}, vb[N] = {};
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      planes_dot(va, (int)(w[i] & 0x0f0f0f0fu), x.a, i);
-      planes_dot(vb, (int)((w[i] >> 4) & 0x0f0f0f0fu), x.b, i);
+      dot4<false, false>(va, (int)(w[i] & 0x0f0f0f0fu), x, i);
+      dot4<true, false>(vb, (int)((w[i] >> 4) & 0x0f0f0f0fu), x, i);
     }
     float sa, ma, sb, mb;
     k4_pair(quad_header(o.hw), jj, sa, ma, sb, mb);
-    return (sa * x.qa * planes_val(va) + sb * x.qb * planes_val(vb)) - (ma * x.qsa + mb * x.qsb);
+    return (times<false>(sa, va, x) + times<true>(sb, vb, x)) - (ma * total<false>(x) + mb * total<true>(x));
   } else if constexpr (T == MOE_GGML_Q5_K) {
     const uint4 hd = quad_header(o.hw);
     const uint32_t w[8] = {o.c0.x, o.c0.y, o.c0.z, o.c0.w, o.c1.x, o.c1.y, o.c1.z, o.c1.w};
@@ -427,31 +462,29 @@ __device__ __forceinline__ float ggu_dot(const GgU<T>& o, int jj, const XUn<N>& 
     qh[5] = (uint32_t)__builtin_amdgcn_mov_dpp((int)o.qh.y, 0xAA, 0xf, 0xf, true);
     qh[6] = (uint32_t)__builtin_amdgcn_mov_dpp((int)o.qh.x, 0xFF, 0xf, 0xf, true);
     qh[7] = (uint32_t)__builtin_amdgcn_mov_dpp((int)o.qh.y, 0xFF, 0xf, 0xf, true);
-    int va[N] = {}, vb[N] = {};
 #pragma unroll
     for (int i = 0; i < 8; i++) {
       // (the unit's two bits rotated to bit 4 of each byte: 2 operations of 20 per word less)
       const int lo = (int)((w[i] & 0x0f0f0f0fu) | (__builtin_amdgcn_alignbit(qh[i], qh[i], to4) & 0x10101010u));
       const int hi = (int)(((w[i] >> 4) & 0x0f0f0f0fu) | (__builtin_amdgcn_alignbit(qh[i], qh[i], to4h) & 0x10101010u));
-      planes_dot(va, lo, x.a, i);
-      planes_dot(vb, hi, x.b, i);
+      dot4<false, false>(va, lo, x, i);
+      dot4<true, false>(vb, hi, x, i);
     }
     float sa, ma, sb, mb;
     k4_pair(hd, jj, sa, ma, sb, mb);
-    return (sa * x.qa * planes_val(va) + sb * x.qb * planes_val(vb)) - (ma * x.qsa + mb * x.qsb);
+    return (times<false>(sa, va, x) + times<true>(sb, vb, x)) - (ma * total<false>(x) + mb * total<true>(x));
   } else if constexpr (T == MOE_GGML_Q8_0) {
-    int va[N] = {}, vb[N] = {};
 #pragma unroll
     for (int i = 0; i < 8; i++) {
       const int ca = (int)__builtin_amdgcn_alignbit(o.w[i + 1], o.w[i], 16);  // the first block's codes: 2 bytes off the dword grid
       const int cb = (int)o.w[9 + i];
-      planes_dot(va, ca, x.a, i);
-      planes_dot(vb, cb, x.b, i);
+      dot4<false, true>(va, ca, x, i);
+      dot4<true, true>(vb, cb, x, i);
     }
     union { uint16_t u; __half h; } d0, d1;
     d0.u = (uint16_t)(o.w[0] & 0xffffu);
     d1.u = (uint16_t)(o.w[8] >> 16);
-    return __half2float(d0.h) * x.qa * planes_val(va) + __half2float(d1.h) * x.qb * planes_val(vb);
+    return times<false>(__half2float(d0.h), va, x) + times<true>(__half2float(d1.h), vb, x);
   } else if constexpr (T == MOE_GGML_IQ4_NL || T == MOE_GGML_IQ4_XS) {
     uint32_t qa[4], qb[4];  // the 16 code bytes of the unit's two 32-element blocks
     float da, db;           // their scales
@@ -479,39 +512,35 @@ __device__ __forceinline__ float ggu_dot(const GgU<T>& o, int jj, const XUn<N>& 
       da = dd * (float)la;
       db = dd * (float)lb;
     }
-    int va[N] = {}, vb[N] = {};
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int al = iq4_lookup4(qa[i], 0), ah = iq4_lookup4(qa[i], 4);
       const int bl = iq4_lookup4(qb[i], 0), bh = iq4_lookup4(qb[i], 4);
-      planes_dot(va, al, x.a, i);
-      planes_dot(va, ah, x.a, 4 + i);
-      planes_dot(vb, bl, x.b, i);
-      planes_dot(vb, bh, x.b, 4 + i);
+      dot4<false, true>(va, al, x, i);
+      dot4<false, true>(va, ah, x, 4 + i);
+      dot4<true, true>(vb, bl, x, i);
+      dot4<true, true>(vb, bh, x, 4 + i);
     }
-    return da * x.qa * planes_val(va) + db * x.qb * planes_val(vb);
+    return times<false>(da, va, x) + times<true>(db, vb, x);
   } else {  // Q5_1
     const uint32_t dw[12] = {o.a.x, o.a.y, o.a.z, o.a.w, o.b.x, o.b.y, o.b.z, o.b.w, o.c.x, o.c.y, o.c.z, o.c.w};
-    float r = 0.f;
-#pragma unroll
-    for (int blk = 0; blk < 2; blk++) {
-      const uint32_t dm = dw[6 * blk], qh = dw[6 * blk + 1];
-      int v[N] = {};
+    auto block = [&](auto gb, Acc<X>& v) {
+      constexpr bool GB = decltype(gb)::value;
+      const uint32_t dm = dw[6 * GB], qh = dw[6 * GB + 1];
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const uint32_t q = dw[6 * blk + 2 + i];
-        // four bits of qh -> bit 4 of four bytes
+        const uint32_t q = dw[6 * GB + 2 + i];
+        // four fifth bits (elements 4i.. / 16 + 4i..) to bit 4 of the four bytes
         const uint32_t hl = ((((qh >> (4 * i)) & 0xFu) * 0x00204081u) & 0x01010101u) << 4;
         const uint32_t hh = ((((qh >> (16 + 4 * i)) & 0xFu) * 0x00204081u) & 0x01010101u) << 4;
-        const int lo = (int)((q & 0x0f0f0f0fu) | hl), hi = (int)(((q >> 4) & 0x0f0f0f0fu) | hh);
-        planes_dot(v, lo, blk ? x.b : x.a, i);
-        planes_dot(v, hi, blk ? x.b : x.a, 4 + i);
+        dot4<GB, false>(v, (int)((q & 0x0f0f0f0fu) | hl), x, i);
+        dot4<GB, false>(v, (int)(((q >> 4) & 0x0f0f0f0fu) | hh), x, 4 + i);
       }
       union { uint32_t u; __half2 h; } cv;
       cv.u = dm;
-      r += __low2float(cv.h) * (blk ? x.qb : x.qa) * planes_val(v) + __high2float(cv.h) * (blk ? x.qsb : x.qsa);
-    }
-    return r;
+      return times<GB>(__low2float(cv.h), v, x) + __high2float(cv.h) * total<GB>(x);
+    };
+    return block(std::false_type{}, va) + block(std::true_type{}, vb);
   }
 }
 
@@ -569,7 +598,7 @@ __device__ __forceinline__ void ggu_gu_rows(const uint8_t* gbase, const uint8_t*
 // rows, so what those lanes read is one run of the up tensor): 8 U units in NP passes instead of eight.  A sum of eight lanes lies
 // within a row on both sides; part[8 NP] = these sums in the order of the units.  xs: the token's activations in LDS, a unit's 128
 // + 16 bytes side by side (the pitch that 16-byte reads of neighbouring units want): lanes of the first kind read theirs once, the
-// others a unit's for each pass, which costs LDS a tenth of what the pass's vector instructions cost the SIMD.  (N: digit planes.)
+// others a unit's for each pass, which costs LDS a tenth of what the pass's vector instructions cost the SIMD.
 // What bounds the launch is those instructions (Q5_K: 145 a pass) from three tokens on, and the loads' latency below.  RB: passes in
 // flight; three (with the selection inside the launch, up to four tokens: 1 token, four layers, 100.3 -> 97.8 us; two and a ring of
 // five or six, which spills, are slower) or four (20 tokens 223.5, with three 224.1).
@@ -577,17 +606,27 @@ __device__ __forceinline__ void ggu_gu_rows(const uint8_t* gbase, const uint8_t*
 // 2 79.6 71.2, 3 114.6 104.4, 4 141.7 129.2, 8 116.7 107.1, 20 244.8 223.6; Q4_K (k_dec4k_gu and this) 1 91.3 79.6, 2 65.6 59.0, 3 83.9 75.6,
 // 4 107.8 99.3, 8 82.0 77.2, 20 173.6 160.6; 1 and 20 tokens Q8_0 132 116, 296 278; Q5_1 / Q8_0 115 104, 244 232; IQ4_NL 116 98, 210 189;
 // IQ4_XS 118 101, 216 190; Q5_K / Q8_0 2048 wide 94 74, 201 161; 3584 125 114, 458 446; Q4_K 2560 wide 90 77, 159 143.
-constexpr int gxu_dw(int N) { return 16 * N + 4; }
-template <int N>
-__device__ __forceinline__ void lds_xu(XUn<N>& x, const uint32_t* xs, int unit) {
-  const uint4* s = (const uint4*)(xs + unit * gxu_dw(N));
+constexpr int gx_dw(bool f32) { return f32 ? 68 : 36; }  // dwords of a unit in LDS
+__device__ __forceinline__ void lds_x(XU& x, const uint32_t* xs, int unit) {
+  const uint4* s = (const uint4*)(xs + unit * gx_dw(false));
   take_planes(x, s);
-  const uint4 m = s[4 * N];
+  const uint4 m = s[8];
   x.qa = __uint_as_float(m.x); x.qsa = __uint_as_float(m.y); x.qb = __uint_as_float(m.z); x.qsb = __uint_as_float(m.w);
 }
-// (three planes leave registers for a pass less, two where a unit is Q8_0's 17 words or a kernel's addresses are many)
-constexpr int ggu_ring(int t, int npl, int np, int n) { return n == 3 ? (np >= 6 || t == MOE_GGML_Q8_0 ? 2 : 3) : npl > 0 ? 3 : 4; }
-template <int T, int NP, int RB, int N, class Stage>
+__device__ __forceinline__ void lds_x(XF& x, const uint32_t* xs, int unit) {
+  const float* s = (const float*)(xs + unit * gx_dw(true));
+  take_f32(x, (const float4*)s);
+  x.sa = s[64];
+  x.sb = s[65];
+}
+// (f32 activations, 66 registers, leave room for two passes)
+constexpr int ggu_ring(int npl, bool f32) { return f32 ? 2 : npl > 0 ? 3 : 4; }
+__device__ __forceinline__ float sum8(float v) {  // over the eight lanes of an eighth of a wave
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));          // xor 1
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));          // xor 2
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true));  // mirror in 8
+}
+template <int T, int NP, int RB, class X, class Stage>
 __device__ __forceinline__ void ggu_gu_packed(const uint8_t* gbase, const uint8_t* ubase, int r0, int lane, const uint32_t* xs, float* part,
                                               Stage&& stage) {
   constexpr int U = 8 * NP, L = 64 - U;
@@ -604,18 +643,16 @@ __device__ __forceinline__ void ggu_gu_packed(const uint8_t* gbase, const uint8_
   for (int p = 0; p < RB; p++) fetch(p);
   __builtin_amdgcn_sched_barrier(0);
   stage();
-  XUn<N> x;
-  lds_xu(x, xs, u0);
+  X x;
+  lds_x(x, xs, u0);
 #pragma unroll
   for (int p = 0; p < NP; p++) {
     if (p) {
       const int un = u0 + p * L;
-      if (!main_lane) lds_xu(x, xs, un % U);
+      if (!main_lane) lds_x(x, xs, un % U);
     }
     float v = ggu_dot<T>(u[p % RB], lane & 3, x);
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));   // xor 1
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));   // xor 2
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true));  // mirror in 8
+    v = sum8(v);
     if ((lane & 7) == 0) part[main_lane ? p * NP + (u0 >> 3) : NP * NP + ((u0 + p * L) >> 3)] = v;
     __builtin_amdgcn_sched_barrier(0);  // passes are consumed in arrival order
     if (p + RB < NP) fetch(p + RB);
@@ -633,8 +670,8 @@ __device__ __forceinline__ void ggu_gu_packed(const uint8_t* gbase, const uint8_
     default: { constexpr int T = MOE_GGML_Q5_1; CALL; } break;                    \
   }
 
-// (moe_decgg3_supported's down rows)
-#define GGU_SWITCH3(t, CALL)                                                      \
+// (moe_decgg_f32_supported's down rows)
+#define GGU_SWITCH_F32(t, CALL)                                                      \
   switch (t) {                                                                    \
     case MOE_GGML_Q8_0: { constexpr int T = MOE_GGML_Q8_0; CALL; } break;          \
     default: { constexpr int T = MOE_GGML_Q5_1; CALL; } break;                    \
@@ -646,19 +683,22 @@ struct GuGgArgs {
 };
 
 // grid (mid/32, slots incl. shared + the exact top-k row, P); block 512: k_dec4k_gu<NPL> for any of the four types
-// NP: rows of 8 NP units, dealt over all lanes (ggu_gu_packed); 0: a lane per unit of a row.  N: digit planes of x and hid
-template <int NPL, int NP, int N = 2>
+// NP: rows of 8 NP units, dealt over all lanes (ggu_gu_packed); 0: a lane per unit of a row.
+// F32 (with NP): x and hid as they are, x32 and hid32, instead of digit planes
+template <int NPL, int NP, bool F32 = false>
 __global__ void __launch_bounds__(512, 4) k_decgg_gu(GuGgArgs A, const uint32_t* __restrict__ xplanes,
                                                      const float2* __restrict__ xmeta, int id_stride, int kpt, int d,
                                                      int mid, uint32_t* __restrict__ hplanes,
                                                      float2* __restrict__ hmeta, const float* __restrict__ logits,
                                                      int n_experts, int* __restrict__ ids_out,
-                                                     float* __restrict__ ws_out, const int* __restrict__ ids_in, moe_rfix RF) {
+                                                     float* __restrict__ ws_out, const int* __restrict__ ids_in, moe_rfix RF,
+                                                     const float* __restrict__ x32, float* __restrict__ hid32) {
+  static_assert(!F32 || NP, "rows dealt over all lanes");
   // a row's sums: of its eighths of 8 lanes, or of all of it; wave, row, part
   constexpr int PARTS = NP ? NP : 1;
   __shared__ float part[8 * 8 * PARTS];
-  __shared__ __attribute__((aligned(16))) uint32_t xs[NP ? 8 * NP * gxu_dw(N) : 4];
-  __shared__ uint32_t pk[8 * N];
+  __shared__ __attribute__((aligned(16))) uint32_t xs[NP ? 8 * NP * gx_dw(F32) : 4];
+  __shared__ uint32_t pk[QV_GROUP_DW];
   __shared__ int sel_ids[64];
   __shared__ float sel_ws[64];
   const int s = blockIdx.y, tok = blockIdx.z, nslots = gridDim.y - (NPL > 0 ? 1 : 0);
@@ -695,23 +735,31 @@ __global__ void __launch_bounds__(512, 4) k_decgg_gu(GuGgArgs A, const uint32_t*
   if constexpr (NP > 0) {
     // (the activations, requested ahead of the weights, go to LDS behind the weights' requests)
     const int t0 = (int)threadIdx.x;
-    constexpr int XP = 8 * NP * 4 * N;  // 16-byte pieces of the planes
-    static_assert(XP <= 1024, "two to a thread");
-    const uint4* const xg = (const uint4*)xplanes + (size_t)tok * XP;
+    constexpr int XP = 8 * NP * (F32 ? 16 : 8);  // 16-byte pieces of the activations
+    static_assert(XP <= 1024 && XP % 64 == 0, "two to a thread, whole waves");
+    const uint4* const xg = (F32 ? (const uint4*)x32 : (const uint4*)xplanes) + (size_t)tok * XP;
     const uint4 xp = xg[t0 < XP ? t0 : 0], xp2 = XP > 512 ? xg[t0 + 512 < XP ? t0 + 512 : 0] : xp;
-    const uint4 xm = ((const uint4*)xmeta)[(size_t)tok * (8 * NP) + (t0 < 8 * NP ? t0 : 0)];
+    const uint4 xm = F32 ? xp : ((const uint4*)xmeta)[(size_t)tok * (8 * NP) + (t0 < 8 * NP ? t0 : 0)];
     __builtin_amdgcn_sched_barrier(0);
     auto stage = [&]() {
       auto put = [&](int i, const uint4& v) {
-        if (i < XP) *(uint4*)(xs + i / (4 * N) * gxu_dw(N) + i % (4 * N) * 4) = v;
+        constexpr int PU = F32 ? 16 : 8;  // pieces of a unit
+        uint32_t* const u = xs + i / PU * gx_dw(F32);
+        if (i < XP) *(uint4*)(u + i % PU * 4) = v;
+        if (F32) {  // (a group is the pieces of eight neighbouring lanes)
+          float g = (__uint_as_float(v.x) + __uint_as_float(v.y)) + (__uint_as_float(v.z) + __uint_as_float(v.w));
+          g = sum8(g);
+          if (i < XP && (i & 7) == 0) u[64 + ((i >> 3) & 1)] = __float_as_uint(g);
+        }
       };
       put(t0, xp);
       if (XP > 512) put(t0 + 512, xp2);
-      if (t0 < 8 * NP) *(uint4*)(xs + t0 * gxu_dw(N) + 16 * N) = xm;
+      if (!F32 && t0 < 8 * NP) *(uint4*)(xs + t0 * gx_dw(false) + 32) = xm;
       moe_lds_barrier();  // (the weights stay in flight)
       __builtin_amdgcn_sched_barrier(0);
     };
-    GGU_SWITCH(t, (ggu_gu_packed<T, NP, ggu_ring(T, NPL, NP, N), N>(gbase, ubase, r0, lane, xs, part + 8 * NP * wv, stage)));
+    typedef typename std::conditional<F32, XF, XU>::type X;
+    GGU_SWITCH(t, (ggu_gu_packed<T, NP, ggu_ring(NPL, F32), X>(gbase, ubase, r0, lane, xs, part + 8 * NP * wv, stage)));
   } else {
     const bool live = lane < U;
     const int ul = live ? lane : (lane & 3);
@@ -736,28 +784,31 @@ __global__ void __launch_bounds__(512, 4) k_decgg_gu(GuGgArgs A, const uint32_t*
       u += pg[4 * PARTS + i];
     }
     const float hv = g / (1.f + expf(-g)) * u;
+    if (F32) {
+      if (lane < 32) hid32[((size_t)tok * nslots + s) * mid + blockIdx.x * G4_ROWS + j] = hv;
+      return;
+    }
     float m = dpp_max_row(fabsf(hv));
     m = rows_half_max(m);
-    float inv, q;
-    qv_factor<N>(m, inv, q);
-    if (N == 3) q += rows_half_add(dpp_add_row(hv * 0.f));  // (NaN where a row is not finite)
+    const float inv = m > 0.f ? QV_XMAX / m : 0.f;
+    const float q = m * (1.f / QV_XMAX);
     const int X = (int)rintf(hv * inv);
-    int pd[N];
-    qv_digits_n<N>(X, pd);
+    int p0, p1;
+    qv_digits(X, p0, p1);
     float sx = dpp_add_row((float)X);
     sx = rows_half_add(sx);
-    if (lane < 8 * N) pk[lane] = 0;
+    if (lane < QV_GROUP_DW) pk[lane] = 0;
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
     __builtin_amdgcn_wave_barrier();
     if (lane < 32) {
       const int dw = j >> 2, sh = 8 * (j & 3);
-#pragma unroll
-      for (int p = 0; p < N; p++) atomicOr(&pk[8 * p + dw], (uint32_t)(pd[p] & 0xff) << sh);
+      atomicOr(&pk[dw], (uint32_t)(p0 & 0xff) << sh);
+      atomicOr(&pk[8 + dw], (uint32_t)(p1 & 0xff) << sh);
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);
     __builtin_amdgcn_wave_barrier();
     const size_t gi = ((size_t)tok * nslots + s) * (mid / 32) + blockIdx.x;
-    if (lane < 8 * N) hplanes[gi * (8 * N) + lane] = pk[lane];
+    if (lane < QV_GROUP_DW) hplanes[gi * QV_GROUP_DW + lane] = pk[lane];
     if (lane == 0) hmeta[gi] = make_float2(q, q * sx);
   }
 }
@@ -769,8 +820,8 @@ struct DnGgArgs {
 };
 
 // NR output rows of a wave's slots, row j at first + j step of `base`: U lanes of a slot, summed four (QUADS) or two at a time
-template <int T, int NR, bool QUADS, int N, class Store>
-__device__ __forceinline__ void ggu_dn_rows(const uint8_t* base, int mid, int first, int step, int ul, float mlive, const XUn<N>& x, Store&& store) {
+template <int T, int NR, bool QUADS, class X, class Store>
+__device__ __forceinline__ void ggu_dn_rows(const uint8_t* base, int mid, int first, int step, int ul, float mlive, const X& x, Store&& store) {
   constexpr int RB = NR < ggu_batch<T>() ? NR : ggu_batch<T>();
   const uint64_t rb = ggu_row_bytes(T, (uint64_t)mid);
   const int jj = ul & 3;
@@ -800,13 +851,14 @@ __device__ __forceinline__ void ggu_dn_rows(const uint8_t* base, int mid, int fi
 // shared expert in sixteen lanes of its wave, took four waves for ten slots of twelve units where this takes three, one of them a
 // quarter as long.  Q5_K / Q8_0 layers, 3072 x 768, us: 1 token (four layers) 115.0 -> 110.0, 3 (two) 117.6 116.6, 8 120.0 116.4, 20 252 242,
 // 32 379 363.  Q4_K layers' own kernel below 32 tokens is faster for them: 1 token 90.7 against 93.2, 20 tokens 175.9, 176.4.)
-// N = 3: hid in three planes, U = 2, 6, 10 or 14 (moe_decgg3_supported).
-template <int U, int N = 2>
+// U = 2, 6, 10 or 14 (moe_decgg_f32_supported): hid as it is, hid32, instead of digit planes.
+template <int U>
 __global__ void __launch_bounds__(320) k_decgg_dn(DnGgArgs A, const uint32_t* __restrict__ hplanes,
                                                   const float2* __restrict__ hmeta, const int* __restrict__ ids,
                                                   const float* __restrict__ ws, int id_stride, int kpt, int d,
-                                                  float* __restrict__ out, uint64_t out_stride) {
+                                                  float* __restrict__ out, uint64_t out_stride, const float* __restrict__ hid32) {
   constexpr int S = 64 / U, mid = 64 * U, NSH = (D4_ROWS + S - 1) / S, PL = U % 4 ? 2 : 4, NPC = U / PL;
+  constexpr bool F32 = PL == 2;
   __shared__ __attribute__((aligned(16))) float part[D4_MAXSLOTS + 1][D4_ROWS][NPC > 4 ? 8 : 4];  // a slot's row: the sums of its quads (pairs) of lanes
   __shared__ float wsm[D4_MAXSLOTS + 1];
   const int tok = blockIdx.y;
@@ -829,17 +881,19 @@ __global__ void __launch_bounds__(320) k_decgg_dn(DnGgArgs A, const uint32_t* __
     const int e_any = ids[tok * id_stride + (shw ? 0 : s)];
     const uint32_t e = shw ? 0u : (uint32_t)e_any;
     const uint8_t* base = (shw ? A.sh_down : A.down + (uint64_t)(e * (uint32_t)d) * rb) + (uint64_t)r0 * rb;
-    XUn<N> x;
-    load_xu(x, hplanes, hmeta, (((size_t)tok * nslots + s) * U + ul) * 2);
+    typename std::conditional<F32, XF, XU>::type x;
+    if constexpr (F32) take_f32(x, (const float4*)(hid32 + (((size_t)tok * nslots + s) * U + ul) * 64));
+    else load_xu(x, hplanes, hmeta, (((size_t)tok * nslots + s) * U + ul) * 2);
     auto store = [&](int r, float v) {
       if (live && r < D4_ROWS && ul % PL == 0) part[s][r][ul / PL] = v;
     };
-    if constexpr (PL == 4) {
+    if constexpr (!F32) {
       if (shw) GGU_SWITCH(t, (ggu_dn_rows<T, NSH, true>(base, mid, group < S ? group : 0, S, ul, mlive, x, store)))
       else GGU_SWITCH(t, (ggu_dn_rows<T, D4_ROWS, true>(base, mid, 0, 1, ul, mlive, x, store)))
     } else {
-      if (shw) GGU_SWITCH3(t, (ggu_dn_rows<T, NSH, false>(base, mid, group < S ? group : 0, S, ul, mlive, x, store)))
-      else GGU_SWITCH3(t, (ggu_dn_rows<T, D4_ROWS, false>(base, mid, 0, 1, ul, mlive, x, store)))
+      sum_f32(x);
+      if (shw) GGU_SWITCH_F32(t, (ggu_dn_rows<T, NSH, false>(base, mid, group < S ? group : 0, S, ul, mlive, x, store)))
+      else GGU_SWITCH_F32(t, (ggu_dn_rows<T, D4_ROWS, false>(base, mid, 0, 1, ul, mlive, x, store)))
     }
   }
   if ((int)threadIdx.x < nslots) wsm[threadIdx.x] = (int)threadIdx.x < kpt ? wmine : sigmoid_f(wmine);
@@ -1095,12 +1149,13 @@ bool moe_decgg_supported(int tgu, int tdn, int tsh, bool has_shared, int d, int 
 int moe_decgg_passes(int d) {
   return d % 512 == 0 && d >= 2048 && d <= 3584 ? d / 512 : 0;
 }
-// Down rows that are no whole super-blocks (2560 x 640): activations in three planes.  Such layers ran on f32 activations, and 24 bits of
-// a group's largest element keep their error where it was: relative to fp64, 1 .. 20 tokens, on the f32 kernels and here, Q5_K / Q8_0
-// 3.1e-7 .. 1.0e-6, 2.8e-7 .. 3.5e-7; Q4_K / Q8_0 3.2 .. 8.8e-7, 2.6 .. 3.8e-7; Q8_0 4.7 .. 6.6e-7, 3.0 .. 3.2e-7; Q5_K / Q5_1 3.0 ..
-// 5.2e-7, 2.8 .. 4.2e-7.  Not IQ4_NL down rows: 1.3 .. 2.3e-7, 1.6 .. 3.8e-7.  2560 x 640 Q5_K / Q8_0, us, f32 kernels and here: 1 token
-// (four layers) 201 84.5, 2 (two) 147 56, 4 267 104, 8 237 84, 20 557 180, 32 874 265.
-bool moe_decgg3_supported(int tgu, int tdn, int tsh, bool has_shared, int d, int mid, int kpt, int n_experts) {
+// Down rows that are no whole super-blocks (2560 x 640): x and hid stay in f32, as on the general kernels (gguf_types.hip), where such layers
+// ran before and where tensors that are not aligned for these still do.  (As 24 bits of the group's largest, three digit planes, an
+// element 2^16 below it kept 8; that took 14 % less time.)  Error against fp64 in the 2-norm at 1, 5 and 20 tokens, on the general kernels and here,
+// 1e-7: Q5_K / Q8_0 3.4 8.2 5.7, 2.4 2.0 2.2; Q4_K / Q8_0 4.3 4.6 6.6, 2.5 2.3 2.1; Q8_0 3.9 4.8 4.9, 2.1 2.2 2.3; Q5_1 / Q8_0 6.5 4.7 5.2, 2.4 2.4
+// 2.4; IQ4_NL / Q8_0 5.0 5.1 4.9, 2.1 2.2 2.2; IQ4_XS / Q8_0 5.2 6.0 4.9, 2.2 2.3 2.3; Q5_K / Q5_1 3.7 3.4 3.6, 3.2 3.2 3.3.  2560 x 640 Q5_K / Q8_0, us, general
+// kernels and here: 1 token (four layers) 201 97.8, 2 (two) 147 64.5, 4 267 116, 8 237 91, 20 557 192, 32 874 294.
+bool moe_decgg_f32_supported(int tgu, int tdn, int tsh, bool has_shared, int d, int mid, int kpt, int n_experts) {
   auto down = [](int t) { return t == MOE_GGML_Q8_0 || t == MOE_GGML_Q5_1; };
   return ggu_type(tgu) && down(tdn) && (!has_shared || down(tsh)) && moe_decgg_passes(d) && mid % 128 == 0 && mid % 256 && mid <= 896 &&
          kpt + 1 <= D4_MAXSLOTS && n_experts <= 1024 && kpt <= n_experts;
@@ -1114,39 +1169,40 @@ bool moe_decgg_aligned(int tgu, int tdn, int tsh, const uint8_t* gate, const uin
          (!sh_gate || (moe_aligned(sh_gate, sh) && moe_aligned(sh_up, sh) && moe_aligned(sh_down, sh)));
 }
 
-static bool decgg_gu_ok(int planes, int tgu, int tsh, bool sh, int d, int mid, int kpt, int n_experts) {
-  return planes == 3 ? moe_decgg3_supported(tgu, MOE_GGML_Q8_0, tsh, sh, d, mid, kpt, n_experts)
-                     : moe_decgg_supported(tgu, tgu, tsh, sh, d, mid, kpt, n_experts);
+static bool decgg_gu_ok(bool f32, int tgu, int tsh, bool sh, int d, int mid, int kpt, int n_experts) {
+  return f32 ? moe_decgg_f32_supported(tgu, MOE_GGML_Q8_0, tsh, sh, d, mid, kpt, n_experts)
+             : moe_decgg_supported(tgu, tgu, tsh, sh, d, mid, kpt, n_experts);
 }
 
 int moe_launch_decgg_gu_topk(int tgu, int tsh, const uint8_t* gate, const uint8_t* up, const uint8_t* sh_gate,
                              const uint8_t* sh_up, const uint32_t* xplanes, const float2* xmeta, const float* logits,
                              int n_experts, int* ids, float* ws, int id_stride, int kpt, int P, int d, int mid,
-                             uint32_t* hplanes, float2* hmeta, hipStream_t st, const moe_rfix* rf, int planes) {
+                             uint32_t* hplanes, float2* hmeta, hipStream_t st, const moe_rfix* rf, const moe_dec_f32& f) {
   const moe_rfix RFV = rf ? *rf : moe_rfix{};
   if (RFV.W && !RFV.tol) return MOE_E_INVALID;
-  if (!gate || !up || !xplanes || !xmeta || !logits || !ids || !ws || !hplanes || !hmeta || (!sh_gate != !sh_up))
+  const bool f32 = f.x != nullptr;
+  if (!gate || !up || !logits || !ids || !ws || (!sh_gate != !sh_up) || (f32 ? !f.hid || !moe_aligned(f.x, 16) : !xplanes || !xmeta || !hplanes || !hmeta))
     return MOE_E_INVALID;
-  if (!decgg_gu_ok(planes, tgu, tsh, sh_gate != nullptr, d, mid, kpt, n_experts)) return MOE_E_UNSUPPORTED;
+  if (!decgg_gu_ok(f32, tgu, tsh, sh_gate != nullptr, d, mid, kpt, n_experts)) return MOE_E_UNSUPPORTED;
   if (!moe_aligned(gate, ggu_align(tgu)) || !moe_aligned(up, ggu_align(tgu)) ||
       (sh_gate && (!moe_aligned(sh_gate, ggu_align(tsh)) || !moe_aligned(sh_up, ggu_align(tsh)))))
     return MOE_E_INVALID;
   GuGgArgs A{gate, up, sh_gate, sh_up, tgu, tsh};
   dim3 grid(mid / G4_ROWS, kpt + (sh_gate ? 1 : 0) + 1, P);
-#define DECGG_GU(NPL, NP, N) \
-  k_decgg_gu<NPL, NP, N><<<grid, 512, 0, st>>>(A, xplanes, xmeta, id_stride, kpt, d, mid, hplanes, hmeta, logits, n_experts, ids, ws, nullptr, RFV)
-#define DECGG_GU_NP(NPL, N)                                  \
+#define DECGG_GU(NPL, NP, F32) \
+  k_decgg_gu<NPL, NP, F32><<<grid, 512, 0, st>>>(A, xplanes, xmeta, id_stride, kpt, d, mid, hplanes, hmeta, logits, n_experts, ids, ws, nullptr, RFV, f.x, f.hid)
+#define DECGG_GU_NP(NPL, F32)                                \
   switch (moe_decgg_passes(d)) {                             \
-    case 4: DECGG_GU(NPL, 4, N); break;                      \
-    case 5: DECGG_GU(NPL, 5, N); break;                      \
-    case 6: DECGG_GU(NPL, 6, N); break;                      \
-    case 7: DECGG_GU(NPL, 7, N); break;                      \
-    default: DECGG_GU(NPL, 0, 2);                            \
+    case 4: DECGG_GU(NPL, 4, F32); break;                    \
+    case 5: DECGG_GU(NPL, 5, F32); break;                    \
+    case 6: DECGG_GU(NPL, 6, F32); break;                    \
+    case 7: DECGG_GU(NPL, 7, F32); break;                    \
+    default: DECGG_GU(NPL, 0, false);                        \
   }
-  if (planes == 3 && n_experts <= 512) DECGG_GU_NP(8, 3)
-  else if (planes == 3) DECGG_GU_NP(16, 3)
-  else if (n_experts <= 512) DECGG_GU_NP(8, 2)
-  else DECGG_GU_NP(16, 2)
+  if (f32 && n_experts <= 512) DECGG_GU_NP(8, true)
+  else if (f32) DECGG_GU_NP(16, true)
+  else if (n_experts <= 512) DECGG_GU_NP(8, false)
+  else DECGG_GU_NP(16, false)
 #undef DECGG_GU
   MOE_LAUNCH_CHECK();
   return MOE_OK;
@@ -1155,18 +1211,22 @@ int moe_launch_decgg_gu_topk(int tgu, int tsh, const uint8_t* gate, const uint8_
 // the same with the ids already there (the router's launches made them)
 int moe_launch_decgg_gu(int tgu, int tsh, const uint8_t* gate, const uint8_t* up, const uint8_t* sh_gate,
                         const uint8_t* sh_up, const uint32_t* xplanes, const float2* xmeta, const int* ids, int n_experts,
-                        int id_stride, int kpt, int P, int d, int mid, uint32_t* hplanes, float2* hmeta, hipStream_t st, int planes) {
-  if (!gate || !up || !xplanes || !xmeta || !ids || !hplanes || !hmeta || (!sh_gate != !sh_up)) return MOE_E_INVALID;
-  if (!decgg_gu_ok(planes, tgu, tsh, sh_gate != nullptr, d, mid, kpt, n_experts)) return MOE_E_UNSUPPORTED;
+                        int id_stride, int kpt, int P, int d, int mid, uint32_t* hplanes, float2* hmeta, hipStream_t st,
+                        const moe_dec_f32& f) {
+  const bool f32 = f.x != nullptr;
+  if (!gate || !up || !ids || (!sh_gate != !sh_up) || (f32 ? !f.hid || !moe_aligned(f.x, 16) : !xplanes || !xmeta || !hplanes || !hmeta))
+    return MOE_E_INVALID;
+  if (!decgg_gu_ok(f32, tgu, tsh, sh_gate != nullptr, d, mid, kpt, n_experts)) return MOE_E_UNSUPPORTED;
   if (!moe_aligned(gate, ggu_align(tgu)) || !moe_aligned(up, ggu_align(tgu)) ||
       (sh_gate && (!moe_aligned(sh_gate, ggu_align(tsh)) || !moe_aligned(sh_up, ggu_align(tsh)))))
     return MOE_E_INVALID;
   GuGgArgs A{gate, up, sh_gate, sh_up, tgu, tsh};
   dim3 grid(mid / G4_ROWS, kpt + (sh_gate ? 1 : 0), P);
-#define DECGG_GU(NPL, NP, N) \
-  k_decgg_gu<NPL, NP, N><<<grid, 512, 0, st>>>(A, xplanes, xmeta, id_stride, kpt, d, mid, hplanes, hmeta, nullptr, n_experts, nullptr, nullptr, ids, moe_rfix{})
-  if (planes == 3) DECGG_GU_NP(0, 3)
-  else DECGG_GU_NP(0, 2)
+#define DECGG_GU(NPL, NP, F32)                                                                                                                \
+  k_decgg_gu<NPL, NP, F32><<<grid, 512, 0, st>>>(A, xplanes, xmeta, id_stride, kpt, d, mid, hplanes, hmeta, nullptr, n_experts, nullptr, nullptr, ids, \
+                                                 moe_rfix{}, f.x, f.hid)
+  if (f32) DECGG_GU_NP(0, true)
+  else DECGG_GU_NP(0, false)
 #undef DECGG_GU
 #undef DECGG_GU_NP
   MOE_LAUNCH_CHECK();
@@ -1175,23 +1235,23 @@ int moe_launch_decgg_gu(int tgu, int tsh, const uint8_t* gate, const uint8_t* up
 
 int moe_launch_decgg_dn(int tdn, int tsh, const uint8_t* down, const uint8_t* sh_down, const float* sh_logit,
                         const uint32_t* hplanes, const float2* hmeta, const int* ids, const float* ws, int id_stride,
-                        int kpt, int P, int d, int mid, float* out, uint64_t out_stride, hipStream_t st, int planes) {
-  if (!down || !hplanes || !hmeta || !ids || !ws || !out || (sh_down && !sh_logit)) return MOE_E_INVALID;
+                        int kpt, int P, int d, int mid, float* out, uint64_t out_stride, hipStream_t st, const float* hid32) {
+  if (!down || (hid32 ? !moe_aligned(hid32, 16) : !hplanes || !hmeta) || !ids || !ws || !out || (sh_down && !sh_logit)) return MOE_E_INVALID;
   if (!moe_aligned(down, ggu_align(tdn)) || (sh_down && !moe_aligned(sh_down, ggu_align(tsh)))) return MOE_E_INVALID;
   DnGgArgs A{down, sh_down, sh_logit, tdn, tsh};
   dim3 grid(d / D4_ROWS, P);
-#define DECGG_DN(U, N) \
-  k_decgg_dn<U, N><<<grid, 64 * ((kpt + 64 / U - 1) / (64 / U) + (sh_down ? 1 : 0)), 0, st>>>(A, hplanes, hmeta, ids, ws, id_stride, kpt, d, out, out_stride)
-  if (mid % 64 || (mid % 256 != 0) != (planes == 3)) return MOE_E_UNSUPPORTED;
-  switch (mid / 64) {  // (moe_decgg_supported, moe_decgg3_supported)
-    case 4: DECGG_DN(4, 2); break;
-    case 8: DECGG_DN(8, 2); break;
-    case 12: DECGG_DN(12, 2); break;
-    case 16: DECGG_DN(16, 2); break;
-    case 2: DECGG_DN(2, 3); break;
-    case 6: DECGG_DN(6, 3); break;
-    case 10: DECGG_DN(10, 3); break;
-    case 14: DECGG_DN(14, 3); break;
+#define DECGG_DN(U) \
+  k_decgg_dn<U><<<grid, 64 * ((kpt + 64 / U - 1) / (64 / U) + (sh_down ? 1 : 0)), 0, st>>>(A, hplanes, hmeta, ids, ws, id_stride, kpt, d, out, out_stride, hid32)
+  if (mid % 64 || (mid % 256 != 0) != (hid32 != nullptr)) return MOE_E_UNSUPPORTED;
+  switch (mid / 64) {  // (moe_decgg_supported, moe_decgg_f32_supported)
+    case 4: DECGG_DN(4); break;
+    case 8: DECGG_DN(8); break;
+    case 12: DECGG_DN(12); break;
+    case 16: DECGG_DN(16); break;
+    case 2: DECGG_DN(2); break;
+    case 6: DECGG_DN(6); break;
+    case 10: DECGG_DN(10); break;
+    case 14: DECGG_DN(14); break;
     default: return MOE_E_UNSUPPORTED;
   }
 #undef DECGG_DN

@@ -46,10 +46,9 @@ struct moe_rot_planes {
   uint32_t* planes;
   float2* meta;
 };
-enum { MOE_PLANES_QVEC4, MOE_PLANES_QVEC, MOE_PLANES_QVEC3 };  // (qvec.h)
 int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x,
                             int P, float* logits, float* out_x, uint32_t* planes, float2* meta,
-                            int planes_form, hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rot = nullptr,
+                            bool planes_natural, hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rot = nullptr,
                             float* tol_out = nullptr, float tol_scale = 0.f, int* parts = nullptr);
 // Whether it leaves each token's bound in tol_out: not where its column shares do not apply (more than four tokens).
 bool moe_router_small_bounds(const moe_wview* W, int P);
@@ -191,20 +190,27 @@ int moe_launch_dec_dn_uq(const moe_wview* dn, const moe_wview* sh_down, const ui
 // the same for raw GGUF Q4_K rows (activation planes in natural order)
 bool moe_dec4k_supported(int d, int mid, int nslots);
 bool moe_decgg_supported(int tgu, int tdn, int tsh, bool has_shared, int d, int mid, int kpt, int n_experts);
-bool moe_decgg3_supported(int tgu, int tdn, int tsh, bool has_shared, int d, int mid, int kpt, int n_experts);
+bool moe_decgg_f32_supported(int tgu, int tdn, int tsh, bool has_shared, int d, int mid, int kpt, int n_experts);
 bool moe_decgg_aligned(int tgu, int tdn, int tsh, const uint8_t* gate, const uint8_t* up, const uint8_t* down, const uint8_t* sh_gate,
                        const uint8_t* sh_up, const uint8_t* sh_down);
+// Activations that stay in f32 (moe_decgg_f32_supported): x [P][d] instead of its planes, hid [P][slots][mid] out.
+struct moe_dec_f32 {
+  const float* x = nullptr;
+  float* hid = nullptr;
+};
 int moe_launch_decgg_gu_topk(int tgu, int tsh, const uint8_t* gate, const uint8_t* up, const uint8_t* sh_gate,
                              const uint8_t* sh_up, const uint32_t* xplanes, const float2* xmeta, const float* logits,
                              int n_experts, int* ids, float* ws, int id_stride, int kpt, int P, int d, int mid,
-                             uint32_t* hplanes, float2* hmeta, hipStream_t st, const moe_rfix* rf = nullptr, int planes = 2);
+                             uint32_t* hplanes, float2* hmeta, hipStream_t st, const moe_rfix* rf = nullptr,
+                             const moe_dec_f32& f = {});
 int moe_launch_decgg_gu(int tgu, int tsh, const uint8_t* gate, const uint8_t* up, const uint8_t* sh_gate,
                         const uint8_t* sh_up, const uint32_t* xplanes, const float2* xmeta, const int* ids, int n_experts,
                         int id_stride, int kpt, int P, int d, int mid, uint32_t* hplanes, float2* hmeta, hipStream_t st,
-                        int planes = 2);
+                        const moe_dec_f32& f = {});
 int moe_launch_decgg_dn(int tdn, int tsh, const uint8_t* down, const uint8_t* sh_down, const float* sh_logit,
                         const uint32_t* hplanes, const float2* hmeta, const int* ids, const float* ws, int id_stride,
-                        int kpt, int P, int d, int mid, float* out, uint64_t out_stride, hipStream_t st, int planes = 2);
+                        int kpt, int P, int d, int mid, float* out, uint64_t out_stride, hipStream_t st,
+                        const float* hid32 = nullptr);
 int moe_decgg_passes(int d);
 bool moe_decgg_uq_supported(int d);
 int moe_decgg_uq_tile_cap();

@@ -15,17 +15,12 @@
 //           32-element sub-block and the high nibbles the next, so `w & 0x0f0f0f0f` and
 //           `(w >> 4) & 0x0f0f0f0f` deliver four consecutive codes of one sub-block each)
 //   meta:   float2 (q, q * sum of the quantised elements)
-//
-// qvec3 (GGUF layers whose activations are kept at 32 bits): the same with 3 x 8 dwords, x ~= q * (65536 p0 + 256 p1 + p2),
-//   |X| <= 8355585 (23.99 bits); q is NaN where an element is not finite.
 #pragma once
 #include "common.h"
 
 constexpr int QV_GROUP_DW = 16;
 constexpr int QV4_GROUP_DW = 16;
 constexpr float QV_XMAX = 32639.f;   // 0x7f7f: both balanced digits at +127
-constexpr int QV3_GROUP_DW = 24;
-constexpr float QV3_XMAX = 8355584.f;  // 0x7f7f00: 127 short of three digits of +127, since the factor and the product are rounded to 24 bits
 constexpr float QV4_XMAX = 30583.f;  // 0x7777: every balanced digit at +7
 
 // Cross-row steps of the wave reductions of the decode kernels.  v holds its row's (16 lanes) result
@@ -55,31 +50,7 @@ __device__ __forceinline__ void qv_digits(int X, int& p0, int& p1) {
   p0 = (X - p1) >> 8;
 }
 
-// N digits, 2 or 3
-template <int N>
-__device__ __forceinline__ void qv_digits_n(int X, int (&p)[N]) {
-  if constexpr (N == 3) {
-    p[2] = ((X + 128) & 255) - 128;
-    X = (X - p[2]) >> 8;
-  }
-  qv_digits(X, p[0], p[1]);
-}
-template <int N>
-constexpr float qv_xmax() { return N == 3 ? QV3_XMAX : QV_XMAX; }
-// A group's factor and q, from its largest magnitude.  Three digits: a largest one below 2^-104 (5e-32, hid of x near 1e-16) would make
-// the factor infinite; the group keeps 2^126 and its elements fewer than 24 bits.
-template <int N>
-__device__ __forceinline__ void qv_factor(float m, float& inv, float& q) {
-  inv = m > 0.f ? qv_xmax<N>() / m : 0.f;
-  q = m * (1.f / qv_xmax<N>());
-  if (N == 3 && m < 0x1p-104f) {
-    inv = 0x1p126f;
-    q = 0x1p-126f;
-  }
-}
-
-// One thread quantises group g of token t into the qvec form (N = 2) or qvec3 (N = 3).
-template <int N>
+// One thread quantises group g of token t into the qvec form.
 __device__ __forceinline__ void qvec_group_from_f32(const float* __restrict__ x, uint64_t x_stride, int G, int t,
                                                     int g, uint32_t* __restrict__ planes,
                                                     float2* __restrict__ meta) {
@@ -92,17 +63,11 @@ __device__ __forceinline__ void qvec_group_from_f32(const float* __restrict__ x,
     v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
     m = fmaxf(m, fmaxf(fmaxf(fabsf(f.x), fabsf(f.y)), fmaxf(fabsf(f.z), fabsf(f.w))));
   }
-  float inv, q;
-  qv_factor<N>(m, inv, q);
-  if (N == 3) {
-    float z = 0.f;  // (0, or NaN)
+  const float inv = m > 0.f ? QV_XMAX / m : 0.f;
+  const float q = m * (1.f / QV_XMAX);
+  uint32_t pl[2][8];
 #pragma unroll
-    for (int j = 0; j < 32; j++) z = fmaf(v[j], 0.f, z);
-    q += z;
-  }
-  uint32_t pl[N][8];
-#pragma unroll
-  for (int p = 0; p < N; p++)
+  for (int p = 0; p < 2; p++)
 #pragma unroll
     for (int i = 0; i < 8; i++) pl[p][i] = 0;
   int sx = 0;
@@ -110,15 +75,15 @@ __device__ __forceinline__ void qvec_group_from_f32(const float* __restrict__ x,
   for (int j = 0; j < 32; j++) {
     const int X = (int)rintf(v[j] * inv);
     sx += X;
-    int p[N];
-    qv_digits_n<N>(X, p);
+    int p0, p1;
+    qv_digits(X, p0, p1);
     const int dw = j >> 2, sh = 8 * (j & 3);
-#pragma unroll
-    for (int i = 0; i < N; i++) pl[i][dw] |= (uint32_t)(p[i] & 0xff) << sh;
+    pl[0][dw] |= (uint32_t)(p0 & 0xff) << sh;
+    pl[1][dw] |= (uint32_t)(p1 & 0xff) << sh;
   }
-  uint4* dst = (uint4*)(planes + ((size_t)t * G + g) * (8 * N));
+  uint4* dst = (uint4*)(planes + ((size_t)t * G + g) * QV_GROUP_DW);
 #pragma unroll
-  for (int p = 0; p < N; p++) {
+  for (int p = 0; p < 2; p++) {
     dst[2 * p] = make_uint4(pl[p][0], pl[p][1], pl[p][2], pl[p][3]);
     dst[2 * p + 1] = make_uint4(pl[p][4], pl[p][5], pl[p][6], pl[p][7]);
   }

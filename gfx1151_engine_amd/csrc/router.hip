@@ -167,14 +167,13 @@ __global__ void __launch_bounds__(256, 2) k_router_logits_seq(const void* __rest
 // q = index among these blocks, bs = block size.
 __device__ __forceinline__ void router_plane_blocks(int q, int bs, int tid, const float* __restrict__ x, int P, int d,
                                                     uint32_t* __restrict__ planes, float2* __restrict__ meta,
-                                                    int planes_form, const moe_rot_planes& R) {
+                                                    bool planes_natural, const moe_rot_planes& R) {
   const int G = d / 32, gb = (G + bs - 1) / bs;
   const int nq = planes ? P * gb : 0;
   if (q < nq) {
     const int t = q / gb, g = (q % gb) * bs + tid;
     if (t < P && g < G) {
-      if (planes_form == MOE_PLANES_QVEC) qvec_group_from_f32<2>(x, (uint64_t)d, G, t, g, planes, meta);  // GGUF kernels
-      else if (planes_form == MOE_PLANES_QVEC3) qvec_group_from_f32<3>(x, (uint64_t)d, G, t, g, planes, meta);
+      if (planes_natural) qvec_group_from_f32(x, (uint64_t)d, G, t, g, planes, meta);  // GGUF kernels
       else qvec4_group_from_f32(x, (uint64_t)d, G, t, g, planes, meta);                       // q4cp kernels
     }
     return;
@@ -296,13 +295,13 @@ __global__ void __launch_bounds__(128) k_router_small(const void* __restrict__ W
                                                       const float* __restrict__ x, int E, int d,
                                                       float* __restrict__ logits, float* __restrict__ out_x,
                                                       int nrows, uint32_t* __restrict__ planes,
-                                                      float2* __restrict__ meta, int planes_form, moe_rot_planes rot,
+                                                      float2* __restrict__ meta, bool planes_natural, moe_rot_planes rot,
                                                       float* __restrict__ tol_out, float tol_scale) {
   // the wave index as a scalar: row, weight type and base address are then wave-uniform values
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int nrb = (nrows + 1) / 2;
   if ((int)blockIdx.x >= nrb) {
-    router_plane_blocks((int)blockIdx.x - nrb, (int)blockDim.x, (int)threadIdx.x, x, TT, d, planes, meta, planes_form, rot);
+    router_plane_blocks((int)blockIdx.x - nrb, (int)blockDim.x, (int)threadIdx.x, x, TT, d, planes, meta, planes_natural, rot);
     return;
   }
   const int row = blockIdx.x * 2 + wv;
@@ -344,12 +343,12 @@ __global__ void __launch_bounds__(256) k_router_mid(const void* __restrict__ W, 
                                                     const float* __restrict__ x, int P, int E, int d,
                                                     float* __restrict__ logits, float* __restrict__ out_x,
                                                     int nrows, uint32_t* __restrict__ planes,
-                                                    float2* __restrict__ meta, int planes_form, moe_rot_planes rot) {
+                                                    float2* __restrict__ meta, bool planes_natural, moe_rot_planes rot) {
   __shared__ __attribute__((aligned(16))) double Xd[2][PMAX][RM_C];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int nrb = (nrows + 3) >> 2;
   if ((int)blockIdx.x >= nrb) {
-    router_plane_blocks((int)blockIdx.x - nrb, 256, tid, x, P, d, planes, meta, planes_form, rot);
+    router_plane_blocks((int)blockIdx.x - nrb, 256, tid, x, P, d, planes, meta, planes_natural, rot);
     return;
   }
   // the wave's row as scalar values: the bf16 / f32 choice is then a scalar branch
@@ -519,7 +518,7 @@ template <bool BF16, int NTT, int RD>  // NTT = token tiles of 16 (1 or 2)
 __global__ void __launch_bounds__(512, 2) k_router_mfma(const void* __restrict__ W, const float* __restrict__ bias,
                                                         const float* __restrict__ x, int P, int E, int d,
                                                         float* __restrict__ logits, uint32_t* __restrict__ planes,
-                                                        float2* __restrict__ meta, int planes_form, int KS,
+                                                        float2* __restrict__ meta, bool planes_natural, int KS,
                                                         double* gpart, unsigned* tickets, moe_row_extras R, moe_rot_planes rot) {
   __shared__ double part[8][NTT][4][64];
   __shared__ int s_last;
@@ -528,7 +527,7 @@ __global__ void __launch_bounds__(512, 2) k_router_mfma(const void* __restrict__
   if ((int)blockIdx.x >= nrt * KS) {
     const int nx = R.tol || R.wx ? P : 0, t = (int)blockIdx.x - nrt * KS;
     if (t >= nx) {
-      router_plane_blocks(t - nx, 512, tid, x, P, d, planes, meta, planes_form, rot);
+      router_plane_blocks(t - nx, 512, tid, x, P, d, planes, meta, planes_natural, rot);
       return;
     }
     // a block per token: |x| as the selection's bound, the shared expert's gate logit
@@ -709,7 +708,7 @@ bool moe_router_small_bounds(const moe_wview* W, int P) {
 // planes of x for the integer-dot decode kernels) in the same launch.
 int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wview* Wx, const float* x,
                             int P, float* logits, float* out_x, uint32_t* planes, float2* meta,
-                            int planes_form, hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rotp,
+                            bool planes_natural, hipStream_t st, double* kpart, unsigned* ktickets, const moe_rot_planes* rotp,
                             float* tol_out, float tol_scale, int* parts) {
   const int E = (int)W->rows, d = (int)W->cols;
   if (parts) *parts = 0;
@@ -734,8 +733,8 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
     // more than 24 tokens per block cost the kernel its second wave per SIMD (accumulators):
     // two launches of at most 16 tokens read the router matrix twice (L2 / MALL) and are faster
     const int P0 = 16, G = d / 32;
-    const size_t pdw = planes_form == MOE_PLANES_QVEC3 ? QV3_GROUP_DW : planes_form ? QV_GROUP_DW : QV4_GROUP_DW;
-    int rc = moe_router_logits_small(W, bias, Wx, x, P0, logits, out_x, planes, meta, planes_form, st, nullptr,
+    const size_t pdw = planes_natural ? QV_GROUP_DW : QV4_GROUP_DW;
+    int rc = moe_router_logits_small(W, bias, Wx, x, P0, logits, out_x, planes, meta, planes_natural, st, nullptr,
                                      nullptr, rotp);
     if (rc) return rc;
     moe_rot_planes rot2 = rot;
@@ -745,7 +744,7 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
     }
     return moe_router_logits_small(W, bias, Wx, x + (size_t)P0 * d, P - P0, logits + (size_t)P0 * E,
                                    out_x ? out_x + P0 : nullptr, planes ? planes + (size_t)P0 * G * pdw : nullptr,
-                                   meta ? meta + (size_t)P0 * G : nullptr, planes_form, st, nullptr, nullptr,
+                                   meta ? meta + (size_t)P0 * G : nullptr, planes_natural, st, nullptr, nullptr,
                                    rotp ? &rot2 : nullptr);
   }
   const bool bf = W->dtype == MOE_DT_BF16;
@@ -756,7 +755,7 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
   dim3 g((nrows + rpb - 1) / rpb + qblocks);
   const void* wx = Wx ? Wx->data : nullptr;
   if (P <= 4) {
-#define RSM_GO(BF, TT) k_router_small<BF, TT><<<g, bs, 0, st>>>(W->data, bias, wx, xbf, x, E, d, logits, out_x, nrows, planes, meta, planes_form, rot, tol_out, tol_scale)
+#define RSM_GO(BF, TT) k_router_small<BF, TT><<<g, bs, 0, st>>>(W->data, bias, wx, xbf, x, E, d, logits, out_x, nrows, planes, meta, planes_natural, rot, tol_out, tol_scale)
 #define RSM_T(TT) do { if (bf) RSM_GO(true, TT); else RSM_GO(false, TT); } while (0)
     if (P == 1) RSM_T(1);
     else if (P == 2) RSM_T(2);
@@ -776,7 +775,7 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
         *parts = KS;
         ktickets = nullptr;
       }
-#define RX_GO(BF, NTT, RD) k_router_mfma<BF, NTT, RD><<<gx, 512, 0, st>>>(W->data, bias, x, P, E, d, logits, planes, meta, planes_form, KS, kpart, ktickets, ex, rot)
+#define RX_GO(BF, NTT, RD) k_router_mfma<BF, NTT, RD><<<gx, 512, 0, st>>>(W->data, bias, x, P, E, d, logits, planes, meta, planes_natural, KS, kpart, ktickets, ex, rot)
       const int nit = (d / 16 + 8 * KS - 1) / (8 * KS);  // ring steps a wave walks, at most
       if (nit <= 3) {
         if (P <= 16) { if (bf) RX_GO(true, 1, 3); else RX_GO(false, 1, 3); }
@@ -789,7 +788,7 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
       MOE_LAUNCH_CHECK();
       return MOE_OK;
     }
-#define RMD_GO(BF, PM) k_router_mid<BF, PM><<<g, 256, 0, st>>>(W->data, bias, wx, xbf, x, P, E, d, logits, out_x, nrows, planes, meta, planes_form, rot)
+#define RMD_GO(BF, PM) k_router_mid<BF, PM><<<g, 256, 0, st>>>(W->data, bias, wx, xbf, x, P, E, d, logits, out_x, nrows, planes, meta, planes_natural, rot)
     if (P <= 8) { if (bf) RMD_GO(true, 8); else RMD_GO(false, 8); }
     else if (P <= 16) { if (bf) RMD_GO(true, 16); else RMD_GO(false, 16); }
     else { if (bf) RMD_GO(true, 24); else RMD_GO(false, 24); }  // P <= 24 (larger batches were split above)

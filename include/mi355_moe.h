@@ -284,7 +284,9 @@ int moe_forward_x16(moe_ctx* ctx, int layer, const float* x, const void* x16, in
 /* Switches in the spirit of the reference's QWENOX_* opt-outs (src/gpu/parts/40_model.inc:1959-1996):
  * every fast path is on by default and can be turned off to fall back to the plainer kernel.
  * MOE_OPT_INT_DECODE (default 1): small batches use the integer-dot GEMV kernels (activations as
- * digit planes per 32-group, 16 significant bits relative to the group maximum) instead of the f32 FMA kernels. */
+ * digit planes per 32-group, 16 significant bits relative to the group maximum) instead of the f32 FMA kernels.
+ * q4cp layers with a table codebook and GGUF layers whose down rows are no multiple of 256 keep f32 activations either way
+ * (in other kernels). */
 /* MOE_OPT_UNIQUE_MIN_TOKENS (default 24; 0 = off): q4cp batches of at least this many tokens (and at most 32)
  * walk the expert-sorted pair lists, so that an expert shared by several tokens is read once
  * (the reference's _uq decode kernels, src/gpu/parts/26_kernels_moe_gguf.inc:758-877).  One extra launch
