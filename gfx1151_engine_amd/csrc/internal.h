@@ -165,6 +165,8 @@ struct moe_dec_v2 {
   const float2* xmeta_rot;
 };
 bool moe_dec_gu_topk_supported(int n_experts, int kpt);
+// rows whose experts a block can rank by logit, without the softmax (topk.h)
+constexpr bool moe_topk_ranked(int E, int k) { return E % 4 == 0 && E >= 4 && E <= 512 && k < E && k < 63; }
 int moe_launch_dec_gu_topk(const moe_wview* gu, const moe_wview* sh_gate, const moe_wview* sh_up,
                            const uint32_t* xplanes, const float2* xmeta, const float* logits, int n_experts,
                            int* ids, float* ws, int id_stride, int kpt, int P, int d, int mid,

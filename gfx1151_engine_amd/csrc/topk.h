@@ -283,7 +283,7 @@ __device__ __forceinline__ float topk_gap_needed(float la, float lb, float tol, 
 // rows that the ranking by logit handles (block-uniform)
 template <int NPL>
 __device__ __forceinline__ bool topk_fast_handled(const float* lg, int E, int k) {
-  if constexpr (NPL == 8) return E % 4 == 0 && E >= 4 && k < E && k < 63 && ((uintptr_t)lg & 15) == 0;
+  if constexpr (NPL == 8) return moe_topk_ranked(E, k) && ((uintptr_t)lg & 15) == 0;
   return false;
 }
 

@@ -124,3 +124,39 @@ def test_listed_tokens_under_graph_capture(oracle):
             torch.cuda.synchronize()
             assert torch.equal(y.nan_to_num(), eager[(i + 1) % 3][0].nan_to_num())
     m.close()
+
+
+def launches(m, x, y):
+    """Nodes of a captured call."""
+    import ctypes as C
+    import torch
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        m.forward(0, x, y)
+    n = C.c_size_t(0)
+    assert C.CDLL("libamdhip64.so").hipGraphGetNodes(C.c_void_p(g.raw_cuda_graph()), None, C.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("E", [64, 62, 520])
+@pytest.mark.parametrize("variant,ranked", [("q4cp", 3), ("table", 2), ("q4k", 4), ("ggmix", 4), ("i4r", 4)])
+def test_up_to_how_many_tokens_the_gate_up_launch_selects(variant, ranked, E):
+    """Router, gate/up and down launch, and the selection as a fourth from one token more on (rotated experts: two launches more).  Rows that cannot
+    be ranked by logit -- more than 512 experts, or a number that is no multiple of four -- leave the launch earlier: with table codebooks
+    at two tokens, else at three."""
+    import torch
+    from gfx1151_engine_amd import synth as S
+    d, mid, k = 2048, 256, 4
+    hl = HostLayer(np.random.default_rng(E), d, mid, E, k, fmt={"table": "q4cp", "ggmix": "q4k"}.get(variant, variant),
+                   codebook=S.UNIVERSAL_CODEBOOK if variant == "table" else None, gg_types=(13, 8, 8) if variant == "ggmix" else (12, 12, 12))
+    m, dev = hl.to_gpu(max_tokens=8)
+    most = ranked if E == 64 else 1 if variant == "table" else 2
+    count = {}
+    for T in (1, most, most + 1):
+        x = torch.randn((T, d), device="cuda")
+        y = torch.empty_like(x)
+        m.forward(0, x, y)
+        count[T] = launches(m, x, y)
+    m.close()
+    assert count[1] == (5 if variant == "i4r" else 3)
+    assert count[most] == count[1] and count[most + 1] == count[1] + 1, count
