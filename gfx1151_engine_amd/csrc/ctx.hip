@@ -811,10 +811,15 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
   // and 82.7, 99.3 and 100.8
   const bool gg_dealt = gu4k_dealt || use_ggf32 || (use_intgg && moe_decgg_passes(g.d) > 0);
   // Rows that cannot be ranked by logit (more than 512 experts, or a number that is no multiple of four) cost every block the softmax and k
-  // rounds: one layer of 1000 / 510 experts, 2560 x 640, in the launch and aside, 2 tokens mixes 38.7 42.1 / 34.9 37.6, q4cp 26.8 29.9 / 23.7 26.3, f32
-  // arithmetic 38.0 38.8 / 34.6 35.2, look-up 45.7 37.8 / 38.3 33.9; 3 tokens 56.3 53.6 / 50.7 50.4, 40.2 37.6 / 34.0 33.3, 57.1 49.6 / 50.3 44.7; look-up kernels
-  // at 1 29.6 29.5 / 27.3 26.2, 3072 x 768 29.9 33.1 / 28.2 29.4
-  const int topk_most = !moe_topk_ranked(g.experts, g.topk) ? (use_lut ? 1 : 2) : use_lut ? 2 : gg_dealt ? 4 : use_intgg ? 2 : use_f32a ? 4 : 3;
+  // rounds.  One layer of 1000 / 510 experts, in the launch and aside: 3072 x 768 2 tokens mixes 45.1 43.9 / 40.7 40.9, q4cp 37.4 35.7 / 31.0 31.5, f32
+  // arithmetic 49.9 45.7 / 42.3 40.6, 3 tokens 62.2 57.3 / 56.7 55.1, 52.0 47.0 / 44.8 42.7; 2560 x 640 2 tokens 40.9 43.6 / 35.3 37.7, 28.5 30.3 / 24.5 26.4, 40.2
+  // 40.2 / 35.3 35.3; look-up kernels 1 token 32.5 33.2 / 29.3 29.4, 2560 x 640 32.0 30.1 / 28.2 26.0
+  const int topk_most = !moe_topk_ranked(g.experts, g.topk) ? (use_lut ? 0 : use_f32a ? 1 : 2)
+                        : use_lut                           ? 2
+                        : gg_dealt                          ? 4
+                        : use_intgg                         ? 2
+                        : use_f32a                          ? 4
+                                                            : 3;
   const int topk_max = c->gu_topk_max >= 0 ? c->gu_topk_max : topk_most;
   const bool gu_topk = (((use_int && !use_uq) || ((use_int4k || use_intgg) && !use_uq_gg) || use_ggf32 || use_lut || use_f32a) && P <= topk_max) &&
                        moe_dec_gu_topk_supported(g.experts, g.topk) && moe_router_small_bounds(&L.router, P);
@@ -1012,8 +1017,8 @@ static int forward_small_v2(moe_ctx* c, MoeLayer& L, const float* x, int P, floa
   const bool sh = L.has_shared && !L.sh_dense;  // a q4cp shared expert rides in these kernels as one more slot
   if (sh && (L.sh_gguf_type != 0 || !L.shared_affine)) return MOE_E_UNSUPPORTED;
   const int nslots_d = g.topk + (sh ? 1 : 0);
-  // (512 experts: 105 us either way at 4 tokens, two layers.  Rows that cannot be ranked by logit, 1000 experts, one layer, in the launch and aside: 2
-  // tokens 40.0 40.8, 3 53.2 51.7, 4 63.6 59.5)
+  // (512 experts: 105 us either way at 4 tokens, two layers.  Rows that cannot be ranked by logit, 1000 / 510 experts, one layer, in the launch
+  // and aside: 2 tokens 43.4 41.6 / 36.3 37.4, 3 56.7 52.6 / 49.5 48.1)
   const int topk_most = moe_topk_ranked(g.experts, g.topk) ? 4 : 2;
   const bool gu_topk = P <= (c->gu_topk_max >= 0 ? c->gu_topk_max : topk_most) && moe_router_small_bounds(&L.router, P);
   const moe_rfix rf = router_fix(c, L, x, moe_router_small_bounds(&L.router, P));

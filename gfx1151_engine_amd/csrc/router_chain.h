@@ -70,7 +70,7 @@ __device__ __forceinline__ void select_listed(float* lg, const int* list, int nl
   float slack = INFINITY;
   if (nlist) slack = topk_block<NPL, false, 256, true>(lg, sel_ids, sel_ws, E, k);
   else (void)topk_block<NPL, false, 256>(lg, sel_ids, sel_ws, E, k);
-  if (nlist && (!(slack > 2.f * tol) || !topk_fast_handled<NPL>(lg, E, k))) {
+  if (nlist && !(slack > 2.f * tol)) {
     for (int i = threadIdx.x >> 6; i < nlist; i += 4) {
       const int e = list[i];
       const float v = (float)exact_chain_wave(RF, t, e, chain[threadIdx.x >> 6]) + (RF.bias ? RF.bias[e] : 0.f);

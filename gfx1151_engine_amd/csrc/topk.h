@@ -108,11 +108,11 @@ __device__ __forceinline__ void topk_select(uint32_t (&key)[NPL], int lane, int 
 // the lowest expert is then in the lowest lane, so the second wave-wide reduction becomes a ballot
 // and a find-first-one, and the winner's register index is one lane read.
 template <int NPL>
-__device__ __forceinline__ void topk_select_lm(uint32_t (&key)[NPL], int lane, int k, int* ids_row, float* ws_row) {
+__device__ __forceinline__ void topk_select_lm(uint32_t (&key)[NPL], int lane, int k, int* ids_row, float* ws_row, int* runner_up = nullptr) {
   double wsum = 0.0;
   float mine = 0.f;
   int myid = 0;
-  for (int r = 0; r < k; r++) {
+  for (int r = 0;; r++) {
     uint32_t m = key[0];
     int jm = 0;
 #pragma unroll
@@ -124,6 +124,10 @@ __device__ __forceinline__ void topk_select_lm(uint32_t (&key)[NPL], int lane, i
     const uint32_t wm = wave_umax(m);
     const int wl = __builtin_ctzll(__ballot(m == wm));          // lowest lane holding the maximum
     const int wj = __builtin_amdgcn_readlane(jm, wl);           // its register
+    if (r == k) {
+      if (runner_up) *runner_up = wm != 0u ? NPL * wl + wj : -1;
+      break;
+    }
     const float bv = __uint_as_float(wm - 1u);
     wsum += (double)bv;  // selection order, as the reference's loop over idx[0..k)
     if (lane == r) {
@@ -356,8 +360,7 @@ __device__ __forceinline__ void topk_wave(const float* __restrict__ lg, int* __r
 // CHECK: also returns (to every thread; one more barrier) the slack of the k + 1 best logits: the smallest gap between
 // neighbours minus what topk_gap_needed asks for at tol = 0 (-inf: a logit range in which probabilities underflow, or
 // NaNs).  The selection is certain when the slack exceeds 2 tol -- the verdict of topk_ids_by_logit below on the same
-// row, so that blocks which rank by logit and a block which runs this function agree on when to fall back.  Rows
-// that ranking does not handle return +inf (taken as they are).
+// row, so that blocks which rank by logit and a block which runs this function agree on when to fall back.
 template <int NPL, bool COH, int NT = 256, bool CHECK = false>
 __device__ float topk_block(const float* lg, int* ids_row, float* ws_row, int E, int k, float ulps = 4.8e-7f) {
   constexpr int NPT = (64 * NPL + NT - 1) / NT;  // values per thread
@@ -452,30 +455,23 @@ __device__ float topk_block(const float* lg, int* ids_row, float* ws_row, int E,
     uint32_t key[NPL];
 #pragma unroll
     for (int j = 0; j < NPL; j++) key[j] = keys[NPL * lane + j];
-    if constexpr (NPL <= 8) {
-      int ru = -1;
-      topk_select_sorted<NPL>(key, lane, k, ids_row, ws_row, (uint2*)pb, CHECK ? &ru : nullptr);
-      if constexpr (CHECK) {
-        float sl = INFINITY;
-        if (topk_fast_handled<NPL>(lg, E, k)) {
-          // lane r < k: the expert of rank r (its own write), lane k: the runner-up; each against the next rank
-          const int idr = lane < k ? ids_row[lane] : lane == k ? ru : -1;
-          const float la = idr >= 0 ? lgs[idr] : -INFINITY;
-          const float lb = __shfl_down(la, 1, 64);
-          const float lmax = __shfl(la, 0, 64);
-          float mine = INFINITY;
-          if (lane < k) {
-            const bool fine = idr >= 0 && lb > -INFINITY && lmax - lb < 70.f;  // false for NaNs
-            mine = fine ? (la - lb) - topk_gap_needed(la, lb, 0.f, ulps) : -INFINITY;
-            if (!(mine == mine)) mine = -INFINITY;
-          }
-          sl = -wave_fmax_dpp(-mine);
-        }
-        if (lane == 0) slack = sl;
+    int ru = -1;
+    if constexpr (NPL <= 8) topk_select_sorted<NPL>(key, lane, k, ids_row, ws_row, (uint2*)pb, CHECK ? &ru : nullptr);
+    else topk_select_lm<NPL>(key, lane, k, ids_row, ws_row, CHECK ? &ru : nullptr);
+    if constexpr (CHECK) {
+      // lane r: the expert of rank r (its own write) against the next rank, the last one against the best that was not selected
+      const int idr = lane < k ? ids_row[lane] : -1;
+      const float la = idr >= 0 ? lgs[idr] : -INFINITY, lru = ru >= 0 ? lgs[ru] : -INFINITY;
+      const float lnext = __shfl_down(la, 1, 64), lmax = __shfl(la, 0, 64);
+      const float lb = lane == k - 1 ? lru : lnext;
+      float mine = INFINITY;
+      if (lane < k && (lane < k - 1 || k < E)) {  // (nothing behind the last where all are selected)
+        const bool fine = idr >= 0 && lb > -INFINITY && lmax - lb < 70.f;  // false for NaNs
+        mine = fine ? (la - lb) - topk_gap_needed(la, lb, 0.f, ulps) : -INFINITY;
+        if (!(mine == mine)) mine = -INFINITY;
       }
-    } else {
-      topk_select_lm<NPL>(key, lane, k, ids_row, ws_row);
-      if (CHECK && lane == 0) slack = INFINITY;
+      const float sl = -wave_fmax_dpp(-mine);
+      if (lane == 0) slack = sl;
     }
   }
   if constexpr (CHECK) {
@@ -688,20 +684,18 @@ __device__ bool select_certain(const float* lg, const moe_rfix& R, int tok, int*
                                bool want_ws) {
   __shared__ __attribute__((aligned(16))) float lgfix[64 * NPL];
   __shared__ float xsq[NT / 64];
+  const bool ranked = topk_fast_handled<NPL>(lg, E, k);
+  const bool ranks = !want_ws && ranked;
+  if (!R.W) {  // (no router operands: the logits as they stand)
+    if (ranks && topk_ids_by_logit<NPL>(lg, sel_ids, E, k) == 1) return true;
+    topk_block<NPL, false, NT>(lg, sel_ids, sel_ws, E, k);
+    return false;
+  }
   float tol = 0.f;
-  if (!want_ws) {
-    tol = R.W ? R.tol[tok] : 0.f;  // (blocks that only rank take the bound from the router launch)
-    const int r = topk_ids_by_logit<NPL>(lg, sel_ids, E, k, tol);
-    if (r == 1) return true;
-    if (r != 0 || !R.W) {  // rows the ranking does not handle, or no router operands: the logits as they stand
-      topk_block<NPL, false, NT>(lg, sel_ids, sel_ws, E, k);
-      return false;
-    }
+  if (ranks) {
+    tol = R.tol[tok];  // (blocks that only rank take the bound from the router launch)
+    if (topk_ids_by_logit<NPL>(lg, sel_ids, E, k, tol) == 1) return true;
   } else {
-    if (!R.W) {
-      topk_block<NPL, false, NT>(lg, sel_ids, sel_ws, E, k);
-      return false;
-    }
     // The exact selection on the logits as they stand, with the slack of the k + 1 best on the side.  Without a
     // bound from the router launch the block takes |x| itself: the loads go out first and are summed after the
     // selection, whose own loads and barriers they then overlap.
@@ -751,7 +745,7 @@ __device__ bool select_certain(const float* lg, const moe_rfix& R, int tok, int*
       lgfix[e] = v >= lk - margin ? exact_logit(R, tok, e) : v;  // (NaNs stay as they are)
     }
     __syncthreads();
-    if (!want_ws) {
+    if (ranks) {
       if (topk_ids_by_logit<NPL>(lgfix, sel_ids, E, k, 0.f, 0.f) == 1) return true;
       full = true;
     } else {

@@ -317,10 +317,11 @@ int moe_forward_x16(moe_ctx* ctx, int layer, const float* x, const void* x16, in
  * tokens has run on the context.  The difference between the times of a loop of calls without and with the skip is
  * that stage's cost inside the pipelined stream, without the dispatch latency that an event pair around a 10 us
  * kernel adds. */
-/* MOE_OPT_GU_TOPK_MAX_TOKENS (default: the measured crossover of the kernels a layer takes, 1 .. 4): batches of at most this many tokens run the softmax / top-k inside the gate/up launch
+/* MOE_OPT_GU_TOPK_MAX_TOKENS (default: the measured crossover of the kernels a layer takes, 2 .. 4, and 0 .. 2 with more than 512 experts or a
+ * number of them that is no multiple of four): batches of at most this many tokens run the softmax / top-k inside the gate/up launch
  * (every block of a routed slot selects its token's experts itself: one launch less on the latency-bound path);
  * larger batches of the integer-dot kernels take the ids from the router's launches, so that the thousands of blocks
- * of such a launch do not each repeat the selection. */
+ * of such a launch do not each repeat the selection.  Above four tokens it applies to d that is a multiple of 128 (256 and more). */
 /* MOE_OPT_F32_DECODE_MAX_TOKENS (default 5; 0 .. 32): q4cp layers that do not run on the integer-dot kernels (a codebook
  * that is not a*n + b, or MOE_OPT_INT_DECODE = 0) use f32 kernels in which a lane keeps its group's activations in
  * registers over a block's rows (a look-up per weight for table codebooks, a conversion and an FMA for a*n + b); for

@@ -716,20 +716,23 @@ def test_small_batch_ids_when_summation_orders_disagree(oracle, fmt, T, int_deco
     m.close()
 
 
-@pytest.mark.parametrize("T", [3, 7, 20, 32])
-@pytest.mark.parametrize("fmt,d", [("q4cp", 1024), ("q4cp", 1056), ("table", 640), ("q4k", 2304), ("q4k", 2560), ("ggmix", 1024), ("ggmix", 3072), ("i4r", 1024)])
-def test_all_blocks_of_a_launch_select_by_one_bound(oracle, fmt, d, T):
+@pytest.mark.parametrize("T", [1, 3, 7, 20, 32])
+@pytest.mark.parametrize("fmt,d,E", [("q4cp", 1024, 64), ("q4cp", 1056, 64), ("table", 640, 64), ("q4k", 2304, 64), ("q4k", 2560, 64), ("ggmix", 1024, 64),
+                                     ("ggmix", 3072, 64), ("i4r", 1024, 64), ("q4cp", 1024, 62), ("q4cp", 1056, 520), ("table", 640, 520), ("q4k", 512, 513),
+                                     ("q4k", 2048, 63), ("ggmix", 2560, 62), ("i4r", 512, 520), ("f32", 640, 520), ("q4k", 512, 62)])
+def test_all_blocks_of_a_launch_select_by_one_bound(oracle, fmt, d, E, T):
     """The ladder of test_small_batch_ids_when_summation_orders_disagree with MOE_OPT_GU_TOPK_MAX_TOKENS = 32: the blocks that only rank must judge
     a token's gaps by the bound of the block that writes the ids, or a slot's gate/up rows and its down rows are two experts'.  The
     selection aside gives the same result but for the last bits of the weights, whose normaliser has terms of logits that are not redone:
-    two steps of 2^-23, of weights below 1.  (1056 columns: the router launch leaves no bounds above four tokens.)"""
+    two steps of 2^-23 of experts' outputs that are up to some hundred times their sum; another expert's output is of its size.  (1056 columns: the router launch leaves no bounds above four tokens; 62, 63 and more than 512
+    experts: rows that cannot be ranked by logit.)"""
     import torch
     from gfx1151_engine_amd import capi
     rng = np.random.default_rng(d + T)
-    mid, E, k = 256, 64, 8
+    mid, k = 256, 8
     bias = np.full(E, -30.0, np.float32)
     cb = np.sort(rng.standard_normal(16)).astype(np.float32) if fmt == "table" else None
-    hl = HostLayer(rng, d, mid, E, k, fmt={"table": "q4cp", "ggmix": "q4k"}.get(fmt, fmt), bias=bias, codebook=cb, scale_std=0.05,
+    hl = HostLayer(rng, d, mid, E, k, fmt={"table": "q4cp", "ggmix": "q4k", "f32": "q4cp"}.get(fmt, fmt), bias=bias, codebook=cb, scale_std=0.05,
                    gg_types=(13, 8, 8) if fmt == "ggmix" else (12, 12, 12))
     hl.router[:] = 0.0
     A = 61
@@ -744,6 +747,7 @@ def test_all_blocks_of_a_launch_select_by_one_bound(oracle, fmt, d, T):
     hl.bias = bias
     io = oracle.router(hl.oracle_layer().router, x, k, bias=bias)[1]
     m, dev = hl.to_gpu(max_tokens=T)
+    m.set_option(capi.OPT_INT_DECODE, fmt != "f32")
     ys = []
     for most in (32, 0):
         m.set_option(capi.OPT_GU_TOPK_MAX_TOKENS, most)
@@ -751,7 +755,7 @@ def test_all_blocks_of_a_launch_select_by_one_bound(oracle, fmt, d, T):
         assert (m.last_routing(T)[0].cpu().numpy()[:, :k] == io[:, :k]).all()
     m.close()
     assert np.isfinite(ys[0]).all()
-    assert max(max_abs_rel(ys[0][t], ys[1][t]) for t in range(T)) <= 1e-6
+    assert max(max_abs_rel(ys[0][t], ys[1][t]) for t in range(T)) <= 1e-4
 
 
 @pytest.mark.parametrize("T", [5, 17, 32])
