@@ -1073,10 +1073,15 @@ int launch(const SW& R, const SW& S, int n_experts, const __half* x, const int* 
   int nblk = UP ? (m + 16 * NW - 1) / (16 * NW) : (m + 32 * NW - 1) / (32 * NW), npass = 1;
   // Down: a block walks several groups of rows behind one staging of the activations; the longest walk that leaves ten blocks
   // per CU, Q8_0 rows eight (64 pairs: two.  Staging is most of a short walk there: 2048 tokens i4r 205 us, with six blocks 223, with
-  // twelve 300).  With these instead of twelve throughout, us of the layer: Q5_K / Q8_0 48 tokens 467 -> 454, 100 630 618, 300 741 732,
-  // 800 818 803, 2560 x 640 60 399 382; q4cp 2560 x 640 60 233 229, 3072 x 768 300 477 475; Q4_K 300 539 537.  With eight for all, whose longer
-  // walks end raggedly where tiles are few: q4cp 48 294 288 but 36 255 258, 52 304 307, 300 474 480; Q4_K 48 332 327 but 40 299 304
-  constexpr int LEAVE = MFX == 4 ? 512 : FMT == F_Q80 ? 2048 : 2600;
+  // twelve 300).  That is of the tile list's places, all that the host knows: it has one for every expert, so that with a pair to an
+  // expert a third of them, and of the ten blocks, have nothing to do, and with half a pair three in five.  With these instead of twelve
+  // throughout, us of the layer: 512 experts Q5_K / Q8_0 48 tokens 452 -> 441, 100 615 602, 300 743 737, 800 818 805, 2560 x 640 60 399 377; q4cp
+  // 2560 x 640 60 239 235, 3072 x 768 300 486 486; Q4_K 300 543 540.  192 experts Q5_K / Q8_0 62 353 314, 2560 x 640 (four slots) 273 280 256, q4cp (eight
+  // slots) 49 193 180; 256 experts table 2048 x 768 (eight) 464 281 259, Q4_K / Q8_0 2048 x 768 87 298 264; 128 experts q4cp 128 168 155, Q4_K 250
+  // 214 200; with 16 to 64 experts a block has one group of rows either way.  With eight for all, whose longer walks end raggedly where tiles
+  // are few, from ten: 512 experts q4cp 48 282 280 but 36 247 248, 52 295 298, 300 486 491; Q4_K 48 317 315 but 40 290 292; 1000 experts q4cp and Q4_K 33
+  // 270 276, 303 312
+  constexpr int LEAVE = MFX == 4 ? 512 : FMT == F_Q80 ? 2048 : 2560;
   if (!UP)
     for (int c = 1; c <= nblk; c++)
       if (nblk % c == 0 && (int64_t)max_tiles * (nblk / c) >= LEAVE) npass = c;
