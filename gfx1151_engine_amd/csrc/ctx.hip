@@ -805,15 +805,17 @@ static int forward_small_routed(moe_ctx* c, MoeLayer& L, const float* x, int P, 
   // integer-dot kernels: the gate/up launch runs the softmax / top-k itself (one launch less on the
   // latency-bound path than a top-k kernel, no last-block ticket in the logits launch)
   // -- as long as its blocks run in one round: each repeats the selection, 3 .. 4 us, where a launch of its own costs 7.
-  // Two layers, us, in the gate/up launch and aside: look-up kernels 76.3 and 79.7 at 2 tokens, 101.5 and 98.3 at 3; GGUF mixes 84.7 and 84.4 at 2,
-  // 122 and 119 at 3, 153 and 148 at 4; Q4_K 83.6 and 85.3 at 3, 113 and 108 at 4; q4cp 73.7 and 76.4 at 3, 100 and 97 at 4; both kinds
-  // of GGUF layers with rows dealt over all lanes, whose rounds are shorter: mixes 104.5 and 106.4 at 3, 129.2 and 131.5 at 4, Q4_K 75.5
-  // and 82.7, 99.3 and 100.8
+  // Layers of 512 experts, us, in the gate/up launch and aside, weights from HBM (2 tokens four layers, 3 and 4 three): q4cp 3 tokens 121 127, 4 148
+  // 147; look-up kernels 2 165 172, 4 195 185; GGUF layers with rows dealt over all lanes, mixes 3 155 159, 4 188 191, Q4_K 122 131, 152 155; mixes of
+  // 4096 x 768, not dealt, 2 203 210, 4 255 256.  At 3 tokens look-up kernels and mixes that are not dealt gain 2 % in the launch from
+  // HBM, 159 162 and 202 207, and lose 3 % out of the last-level cache.  f32 arithmetic (MOE_OPT_INT_DECODE = 0): its line of 4 was drawn on
+  // earlier kernels; 1 107 130, 2 180 173, 3 179 168, 4 221 199 now
   const bool gg_dealt = gu4k_dealt || use_ggf32 || (use_intgg && moe_decgg_passes(g.d) > 0);
   // Rows that cannot be ranked by logit (more than 512 experts, or a number that is no multiple of four) cost every block the softmax and k
-  // rounds.  One layer of 1000 / 510 experts, in the launch and aside: 3072 x 768 2 tokens mixes 45.1 43.9 / 40.7 40.9, q4cp 37.4 35.7 / 31.0 31.5, f32
-  // arithmetic 49.9 45.7 / 42.3 40.6, 3 tokens 62.2 57.3 / 56.7 55.1, 52.0 47.0 / 44.8 42.7; 2560 x 640 2 tokens 40.9 43.6 / 35.3 37.7, 28.5 30.3 / 24.5 26.4, 40.2
-  // 40.2 / 35.3 35.3; look-up kernels 1 token 32.5 33.2 / 29.3 29.4, 2560 x 640 32.0 30.1 / 28.2 26.0
+  // rounds.  1000 / 510 experts, in the launch and aside, weights from HBM (1 and 2 tokens four layers, 3 three): 3072 x 768 2 tokens mixes 180 178 / 164
+  // 164, Q4_K 161 158 / 135 139, q4cp 155 151 / 130 135, f32 arithmetic 204 188 / 178 171; 3 tokens mixes 187 173 / 164 159, q4cp 154 140 / 131 126;
+  // narrower layers gain at 2 tokens also with 1000 experts (q4cp 2304 x 512 117 123, mixes 2560 x 640 166 176); look-up kernels 1 token 136 138 / 124
+  // 124, 2560 x 640 134 126 / 119 112
   const int topk_most = !moe_topk_ranked(g.experts, g.topk) ? (use_lut ? 0 : use_f32a ? 1 : 2)
                         : use_lut                           ? 2
                         : gg_dealt                          ? 4
@@ -1017,8 +1019,8 @@ static int forward_small_v2(moe_ctx* c, MoeLayer& L, const float* x, int P, floa
   const bool sh = L.has_shared && !L.sh_dense;  // a q4cp shared expert rides in these kernels as one more slot
   if (sh && (L.sh_gguf_type != 0 || !L.shared_affine)) return MOE_E_UNSUPPORTED;
   const int nslots_d = g.topk + (sh ? 1 : 0);
-  // (512 experts: 105 us either way at 4 tokens, two layers.  Rows that cannot be ranked by logit, 1000 / 510 experts, one layer, in the launch
-  // and aside: 2 tokens 43.4 41.6 / 36.3 37.4, 3 56.7 52.6 / 49.5 48.1)
+  // (us, in the launch and aside, weights from HBM: 512 experts 4 tokens, three layers, 159 162.  Rows that cannot be ranked by logit, 1000 / 510
+  // experts: 2 tokens, four layers, 179 176 / 153 158, 3, three layers, 170 157 / 146 143)
   const int topk_most = moe_topk_ranked(g.experts, g.topk) ? 4 : 2;
   const bool gu_topk = P <= (c->gu_topk_max >= 0 ? c->gu_topk_max : topk_most) && moe_router_small_bounds(&L.router, P);
   const moe_rfix rf = router_fix(c, L, x, moe_router_small_bounds(&L.router, P));

@@ -223,7 +223,7 @@ constexpr int GU2_ROWS = 32;
 // (LUT = 1: four waves, 16 rows.  A block is tens of thousands of vector instructions there, and one token's 264 blocks of
 // eight waves leave the CUs that get a second one with twice the work: four layers 129 -> 119 us.  With the selection inside, three
 // waves and 12 rows.  It is the selection that gains -- probably because a CU's waves go round its SIMDs: of blocks of four waves
-// the first ones, which select, would all share a SIMD.  us, 16 and 12 rows: 1 token (four layers) 3072 x 768 111.7 104.1, x 512 99.7 85.2, x 1024 127.5 113.5,
+// the first ones, which select, would all share a SIMD.  us, out of the last-level cache (from HBM, 3072 x 768, 1 token 117.7 108.1), 16 and 12 rows: 1 token (four layers) 3072 x 768 111.7 104.1, x 512 99.7 85.2, x 1024 127.5 113.5,
 // 2560 x 640 108.0 102.9; 2 tokens (two layers) 86.5 76.3 -- with the selection aside, where 16 rows are level or better (4 tokens
 // 117.9 120.3, 8 90.5 92.0), 79.7.  The last block's rows past mid are the last rows again and not stored.)
 constexpr int gu2_threads(int lut, int npl) { return lut == 1 ? (npl ? 192 : 256) : 512; }

@@ -602,10 +602,11 @@ __device__ __forceinline__ void ggu_gu_rows(const uint8_t* gbase, const uint8_t*
 // What bounds the launch is those instructions (Q5_K: 145 a pass) from three tokens on, and the loads' latency below.  RB: passes in
 // flight; three (with the selection inside the launch, up to four tokens: 1 token, four layers, 100.3 -> 97.8 us; two and a ring of
 // five or six, which spills, are slower) or four (20 tokens 223.5, with three 224.1).
-// Layers, us, a lane per unit of a row and this (one token four layers, two and three two): 3072 x 768 Q5_K / Q8_0 1 token 109.9 96.5,
-// 2 79.6 71.2, 3 114.6 104.4, 4 141.7 129.2, 8 116.7 107.1, 20 244.8 223.6; Q4_K (k_dec4k_gu and this) 1 91.3 79.6, 2 65.6 59.0, 3 83.9 75.6,
-// 4 107.8 99.3, 8 82.0 77.2, 20 173.6 160.6; 1 and 20 tokens Q8_0 132 116, 296 278; Q5_1 / Q8_0 115 104, 244 232; IQ4_NL 116 98, 210 189;
-// IQ4_XS 118 101, 216 190; Q5_K / Q8_0 2048 wide 94 74, 201 161; 3584 125 114, 458 446; Q4_K 2560 wide 90 77, 159 143.
+// Layers, us, a lane per unit of a row and this (weights from HBM, other inputs each call; four layers, at 20 tokens two): 3072 x 768
+// Q5_K / Q8_0 1 token 115 104, 2 168 156, 3 228 208, 4 277 251, 5 318 295, 8 441 402, 20 467 421; Q4_K (k_dec4k_gu, at 1 and 2 tokens with its
+// down launch, and this) 1 95.0 85.7, 2 142 127, 3 180 164, 4 225 203, 5 240 224, 8 324 303, 20 330 301; 1 and 20 tokens Q8_0 130 115, 562 529; Q5_1 / Q8_0
+// 114 104, 462 439; IQ4_NL 120 105, 410 366; IQ4_XS 124 106, 412 370; Q5_K / Q8_0 2048 wide 99 81, 383 304; 3584 129 119, 530 502; Q4_K 2560
+// wide 94 83, 298 268.
 constexpr int gx_dw(bool f32) { return f32 ? 68 : 36; }  // dwords of a unit in LDS
 __device__ __forceinline__ void lds_x(XU& x, const uint32_t* xs, int unit) {
   const uint4* s = (const uint4*)(xs + unit * gx_dw(false));
@@ -1151,10 +1152,10 @@ int moe_decgg_passes(int d) {
 }
 // Down rows that are no whole super-blocks (2560 x 640): x and hid stay in f32, as on the general kernels (gguf_types.hip), where such layers
 // ran before and where tensors that are not aligned for these still do.  (As 24 bits of the group's largest, three digit planes, an
-// element 2^16 below it kept 8; that took 14 % less time.)  Error against fp64 in the 2-norm at 1, 5 and 20 tokens, on the general kernels and here,
+// element 2^16 below it kept 8; that took 10 .. 15 % less time.)  Error against fp64 in the 2-norm at 1, 5 and 20 tokens, on the general kernels and here,
 // 1e-7: Q5_K / Q8_0 3.4 8.2 5.7, 2.4 2.0 2.2; Q4_K / Q8_0 4.3 4.6 6.6, 2.5 2.3 2.1; Q8_0 3.9 4.8 4.9, 2.1 2.2 2.3; Q5_1 / Q8_0 6.5 4.7 5.2, 2.4 2.4
 // 2.4; IQ4_NL / Q8_0 5.0 5.1 4.9, 2.1 2.2 2.2; IQ4_XS / Q8_0 5.2 6.0 4.9, 2.2 2.3 2.3; Q5_K / Q5_1 3.7 3.4 3.6, 3.2 3.2 3.3.  2560 x 640 Q5_K / Q8_0, us, general
-// kernels and here: 1 token (four layers) 201 97.8, 2 (two) 147 64.5, 4 267 116, 8 237 91, 20 557 192, 32 874 294.
+// kernels and here (weights from HBM, other inputs each call): four layers 1 token 221 102, 2 338 143, 4 542 240, 8 990 373; two 20 1126 401, 32 1751 594.
 bool moe_decgg_f32_supported(int tgu, int tdn, int tsh, bool has_shared, int d, int mid, int kpt, int n_experts) {
   auto down = [](int t) { return t == MOE_GGML_Q8_0 || t == MOE_GGML_Q5_1; };
   return ggu_type(tgu) && down(tdn) && (!has_shared || down(tsh)) && moe_decgg_passes(d) && mid % 128 == 0 && mid % 256 && mid <= 896 &&

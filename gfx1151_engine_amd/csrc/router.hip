@@ -511,8 +511,8 @@ void launch_seq(const void* W, bool bf, const float* bias, const float* x, int P
 // tiles go out and come back as device-scope accesses, the ticket counters rest at 0 between launches.  That hand-over is a
 // store's, a ticket's and a load's trip to memory one behind the other: the launch takes 2 us more, 20 tokens 14.3 for 12.2.
 // The shared expert's gate vector has a block per token, which leaves the selection's bound as well: as row 513 of 512 experts it made
-// 264 blocks, each a CU's work, for 256 CUs, and 20 tokens took 12.2 us for 7.4, eight 9.4 for 5.8.  The layer, us, with all of
-// this: 5 tokens q4cp 53.5 -> 48.8, 8 73.4 -> 67.7, 20 140.3 -> 133.8, rotated experts 11 89 -> 83.7; and a batch with a near tie, whose logits
+// 264 blocks, each a CU's work, for 256 CUs, and 20 tokens took 12.2 us for 7.4, eight 9.4 for 5.8.  Layers, us, with all of
+// this, weights from HBM: q4cp 5 tokens (four) 238 -> 216, 8 315 -> 293, 20 (two) 306 -> 292, rotated experts 11 (two) 198 -> 187; and a batch with a near tie, whose logits
 // the selecting launch redoes by waves now, 32 tokens 632 -> 243.
 template <bool BF16, int NTT, int RD>  // NTT = token tiles of 16 (1 or 2)
 __global__ void __launch_bounds__(512, 2) k_router_mfma(const void* __restrict__ W, const float* __restrict__ bias,
@@ -587,7 +587,7 @@ __global__ void __launch_bounds__(512, 2) k_router_mfma(const void* __restrict__
   for (int ib = 0; ib < nit; ib += RD) {
 #pragma unroll
     for (int j = 0; j < RD; j++) {
-      if (ib + j < nit) {  // block-uniform
+      if (ib + j < nit) {  // wave-uniform (a wave's steps may be one fewer than another's)
         float w[4];
         if (BF16) {
           w[0] = __uint_as_float(wr[j].x << 16); w[1] = __uint_as_float(wr[j].x & 0xffff0000u);
@@ -721,12 +721,11 @@ int moe_router_logits_small(const moe_wview* W, const float* bias, const moe_wvi
   // partial tiles the columns are split over up to eight blocks per 16 rows and it serves 5..32 tokens;
   // without it one block per 16 rows leaves most CUs idle (38 us at 32 tokens), which only beats
   // k_router_mid above 24 tokens.  A shared-expert gate row in the other format (checkpoints: a bf16 matrix, an f32 row)
-  // makes no difference to it: a lane loads its row in that row's own format.  With such a row, the router's
-  // launches (logits, top-k) with k_router_mid and with this, us: 5 tokens 25 and 20, 11 tokens 32 and 22, 20 tokens 40 and
-  // 25, 32 tokens 57 and 26.
+  // makes no difference to it: that row is read by a block per token, in its own format.
   // (as many shares as leave every wave a step of 16 columns, whether or not they are equal: 2560 columns in eight shares of two and three
-  // steps a wave instead of four of five: the launch 13.2 -> 7.5 us at 20 tokens; 2560 x 640 layers q4cp 5 tokens 49.0 -> 46.5, 20 118.2
-  // 112.4, table codebook 12 112.4 109.1; 2304 x 512 12 67.5 62.2)
+  // steps a wave instead of four of five: the launch 13.2 -> 7.5 us at 20 tokens; one layer of 2560 x 640 again and again
+  // (up to 12 tokens wholly or mostly out of the last-level cache), q4cp 5 tokens 49.0 -> 46.5, 20 118.2 112.4, table codebook 12 112.4 109.1; 2304 x 512 12
+  // 67.5 62.2)
   const int KS = kpart && ktickets ? column_shares(P, E, d) : 1;
   const bool mfma_ok = on_matrix_pipe(P, d, KS);
   if (P > 24 && !mfma_ok) {

@@ -62,7 +62,7 @@ __device__ __forceinline__ bool logit_doubtful(double sum, float tol) {
 // Block of 256 threads: softmax / top-k of token t's logits lg (LDS), of which list[0 .. nlist) are doubtful.  None (two tokens
 // in three): the selection is the reference's as it stands.  Otherwise the k + 1 best must be further apart than the doubt
 // (topk.h), and where they are not, the doubtful logits alone are redone as the reference's chains -- which leaves none in
-// doubt.  (Redoing all 512 logits of such a token, as the launches for up to 32 tokens do, takes 70 us; one batch of 515
+// doubt.  (Redoing all 512 logits of such a token, as select_certain does with a true near tie, takes 70 us; one batch of 515
 // tokens in ten has one.)  Block-uniform arguments; a barrier stands behind the caller's writes and behind the results.
 template <int NPL>
 __device__ __forceinline__ void select_listed(float* lg, const int* list, int nlist, float tol, const moe_rfix& RF, int t, int E, int k,
